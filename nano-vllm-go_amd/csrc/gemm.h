@@ -27,6 +27,7 @@
 // the tight-tolerance parity mode, not a performance path.
 #pragma once
 #include <stdexcept>
+#include <algorithm>
 #include <type_traits>
 #include "common.h"
 
@@ -110,6 +111,10 @@ struct GemmArgs {
     // The kernel boundary is the synchronisation: no fences, no atomics, fixed summation order.
     float* sk_part;
     int sk_slices;
+    // K split inside a launch: partial tiles and, zero between launches, the tiles' arrival counters (split_finish); NULL: no such split
+    float* split_ws;
+    int* split_cnt;
+    int splits;             // workgroups per tile (set by the launcher)
     // Deferred RMSNorm (decode; RMSNorm + SwiGLU, sequential block): the residual projection that completes x also
     // emits the NEXT projection's operand un-normalised, xn_raw = bf16(x * w_norm) (fragment-major), plus the sums of
     // x^2 over its 16 columns, rs_out[tile][m]; the consumer scales its accumulators by
@@ -343,6 +348,7 @@ __device__ __forceinline__ void epilogue_qkv_head(const GemmArgs& p, int m, int 
 // across the barrier (never vmcnt(0) in the steady state of the 3-stage instance).
 // ------------------------------------------------------------------------------------------
 constexpr int G_BK = 64;
+__device__ __forceinline__ int cdiv_dev(int a, int b) { return (a + b - 1) / b; }
 
 // XCD-aware block remap (bijective for any grid size): blocks b and b+8 share an XCD, so give
 // each XCD a contiguous run of tiles -> neighbouring tiles (same A row panel) hit one L2.
@@ -528,6 +534,71 @@ void gemm_bf16_kernel(GemmArgs p) {
 }
 
 // ------------------------------------------------------------------------------------------
+// K split inside one launch.  `parts` workgroups share an output tile; each leaves its fp32 accumulators in split_ws, draws a number
+// from the tile's counter, and the one that draws the last adds the parts up in part order (always the same sum) and runs the
+// epilogue.  Nobody waits for anybody.  The workgroups may sit on different XCDs, whose L2s are not coherent: the parts are
+// written through and read past the L2 (sc0 sc1) instead of fencing, which would write back everything that XCD has dirty
+// (4096 x 2048 x 6144 in two parts: 85 us so, 156 us with __threadfence, 94 us unsplit).
+// ------------------------------------------------------------------------------------------
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+constexpr int64_t SPLIT_WS_BYTES = 64ll << 20;      // 256 parts of 256 x 256 fp32, or 512 of 128 x 128
+constexpr int SPLIT_MAX_TILES = 512;
+constexpr int SPLIT_COHERENT = 0x11;      // buffer cache policy: sc0 | sc1
+
+// acc: this wave's F fragments; a part takes `bytes` of split_ws (waves one after the other, 1 KiB a fragment).  True in the workgroup
+// that holds the sum.  Whole workgroups call it; `flag`: one int of LDS that nothing else uses.
+template <int F>
+__device__ __forceinline__ bool split_finish(const GemmArgs& p, int tile, int part, int parts, int bytes, int wave, f32x4* acc, int* flag, bool holds = true) {
+    const int lane = threadIdx.x & 63, voff = wave * (F * 1024) + lane * 16;
+    int* cnt = p.split_cnt + tile;
+    char* ws = (char*)p.split_ws + (int64_t)tile * parts * bytes;
+    {
+        const auto rs = __builtin_amdgcn_make_buffer_rsrc(ws + (int64_t)part * bytes, 0, bytes, 0x00020000);
+        if (holds) {
+#pragma unroll
+            for (int f = 0; f < F; f++) {
+                union { f32x4 v; u32x4 u; } t; t.v = acc[f];
+                __builtin_amdgcn_raw_buffer_store_b128(t.u, rs, voff, f * 1024, SPLIT_COHERENT);
+            }
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this wave's stores have reached memory
+        __syncthreads();
+        if (threadIdx.x == 0) *flag = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (*flag != parts - 1) return false;
+    }
+    if (threadIdx.x == 0) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!holds) return true;
+    constexpr int B = F > 16 ? 4 : F % 8 == 0 ? 8 : F;      // fragments at a time, of four parts: their loads travel together
+    static_assert(B <= 8 && F % B == 0, "registers of the loads in flight");
+#pragma unroll
+    for (int f0 = 0; f0 < F; f0 += B) {
+        f32x4 sum[B];
+#pragma unroll
+        for (int f = 0; f < B; f++) sum[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int c0 = 0; c0 < parts; c0 += 4) {
+            union { f32x4 v; u32x4 u; } t[4][B];
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                if (c0 + c >= parts || c0 + c == part) continue;
+                const auto rs = __builtin_amdgcn_make_buffer_rsrc(ws + (int64_t)(c0 + c) * bytes, 0, bytes, 0x00020000);
+#pragma unroll
+                for (int f = 0; f < B; f++) t[c][f].u = __builtin_amdgcn_raw_buffer_load_b128(rs, voff, (f0 + f) * 1024, SPLIT_COHERENT);
+            }
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                if (c0 + c >= parts) break;
+#pragma unroll
+                for (int f = 0; f < B; f++) sum[f] += c0 + c == part ? acc[f0 + f] : t[c][f].v;
+            }
+        }
+#pragma unroll
+        for (int f = 0; f < B; f++) acc[f0 + f] = sum[f];
+    }
+    return true;
+}
+
+// ------------------------------------------------------------------------------------------
 // bf16 MFMA kernel, ping-pong form (prefill, tuning option 5): 256x256 tile, 8 waves as two groups of four (one wave
 // of each group per SIMD), K in 32-wide stages through a STAGES-slot LDS ring (4 slots = 128 KiB by default).  A stage is one PHASE for a wave:
 //   L: 12 fragment ds_reads of stage s, LDS-DMA issue of stage s+STAGES-1, lgkmcnt(0), counted vmcnt (stage s+1 landed)
@@ -701,6 +772,182 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_pp_kernel(GemmArgs p) {
 template <bool KEEP>
 __device__ __forceinline__ bf16x8 weight_load(const bf16x8* p) {
     if constexpr (KEEP) return *p;
+// ------------------------------------------------------------------------------------------
+// bf16 kernel for 65 .. 512 rows (large decode batches, short prompts): weights still come from HBM once, but the 64-row groups of the
+// decode form pull every activation row through every CU for 16 weight rows each (FFN-down of Llama-3.2-1B at 96 rows: 128 workgroups x
+// 2 x 1.3 MB, 25 us for 34 MB of weights).  Here a workgroup owns MT x 16 rows by CT x 32 columns, both operands staged through an
+// LDS ring by global_load_lds, so an activation row is fetched once per CT x 32 weight rows and the ring keeps a
+// fixed amount of weights in flight per CU; K is split over workgroups (split_finish) until the launch fills the chip.
+// Eight waves: 2 x 2 over the tile (a wave reads MT / 2 + CT fragments for MT / 2 x CT products) times two halves of every
+// 128-wide K stage, added through LDS at the end.
+// ------------------------------------------------------------------------------------------
+template <int MT, int CT> constexpr int mid_stage_bytes() { return (MT + 2 * CT) * 4096; }
+template <int MT, int CT> constexpr int mid_stages() { return 163328 / mid_stage_bytes<MT, CT>() > 5 ? 5 : 163328 / mid_stage_bytes<MT, CT>(); }
+template <int MT, int CT> constexpr int mid_lds_bytes() { return mid_stages<MT, CT>() * mid_stage_bytes<MT, CT>() + 16; }
+constexpr int MID_MAX_ROWS = 512;
+
+// one pair of rotated quads (EPI_QKV): x1 at column d of the head, x2 at d + hd / 2
+__device__ __forceinline__ void epilogue_qkv_pair(const GemmArgs& p, int m, int head, int d, f32x4 x1, f32x4 x2) {
+    if (m >= p.M) return;
+    const QkvEpi& q = p.qkv;
+    const int HD = q.hd, half = HD >> 1;
+    if (p.bias) { x1 += *(const f32x4*)(p.bias + head * HD + d); x2 += *(const f32x4*)(p.bias + head * HD + d + half); }
+    const int pos = q.tok_pos[m];
+    if (head < q.nH + q.nKV && q.cos_t) {
+        const f32x4 c = *(const f32x4*)(q.cos_t + (int64_t)pos * HD + d), s = *(const f32x4*)(q.sin_t + (int64_t)pos * HD + d);
+        const f32x4 a = x1, b = x2;
+        x1 = a * c + (-b) * s;          // rope.go:196-202
+        x2 = b * c + a * s;
+    }
+    int blk = 0, row = 0;
+    if (head >= q.nH) kv_locate(q.blk_table, q.tok_tbl[m], pos, q.Tmax, blk, row);
+    bf16_t* dst;
+    if (head < q.nH) dst = q.q_out + (int64_t)m * (q.nH * HD) + head * HD + d;
+    else if (head < q.nH + q.nKV) dst = q.kcache + (int64_t)blk * q.slot_stride + ((int64_t)(head - q.nH) * q.Tmax + row) * HD + d;
+    else dst = q.vcache + (int64_t)blk * q.slot_stride + ((int64_t)(head - q.nH - q.nKV) * q.Tmax + row) * HD + d;
+    bf16x4 o1, o2;
+#pragma unroll
+    for (int r = 0; r < 4; r++) { o1[r] = (bf16_t)x1[r]; o2[r] = (bf16_t)x2[r]; }
+    *(bf16x4*)dst = o1;
+    *(bf16x4*)(dst + half) = o2;
+}
+
+template <int MT, int CT, int EPI, typename OutT>
+__global__ __launch_bounds__(512, 1) void gemm_mid_bf16_kernel(GemmArgs p) {
+    constexpr int NST = mid_stages<MT, CT>(), SB = mid_stage_bytes<MT, CT>(), NA = 4 * MT, PW = (MT + 2 * CT) / 2, TM = MT / 2;
+    static_assert(MT % 2 == 0 && NST >= 3 && PW * (NST - 2) < 64, "two waves share the rows; vmcnt counts to 63");
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int lane = threadIdx.x & 63, fr = lane & 15, fg = lane >> 4;
+    const int wave8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave = wave8 & 3, kh = wave8 >> 2, wm = wave >> 1, wn = wave & 1;
+    // ids 8 apart share an XCD: the row groups and parts of a column block follow each other there, so its weights cross HBM once
+    const int groups = cdiv_dev(p.M, 16 * MT), per = groups * p.splits, nb = cdiv_dev(p.N, 32 * CT);
+    const int q = blockIdx.x >> 3, cb = (q / per) * 8 + (blockIdx.x & 7), item = q % per;
+    if (cb >= nb) return;
+    const int part = item % p.splits, m0 = item / p.splits * (16 * MT), n0 = cb * (32 * CT);
+    const int stages = (p.K + 127) >> 7;
+    const int k0 = (int)((int64_t)part * stages / p.splits), n = (int)((int64_t)(part + 1) * stages / p.splits) - k0;
+    const bool ragged = (p.K & 64) && k0 + n == stages;          // K % 128 == 64: the last stage has its first half only
+
+    // 1-KiB blocks (row tile, k-step) of a stage, PW for each wave: rows first, then columns
+    const bf16_t* src[PW];
+#pragma unroll
+    for (int i = 0; i < PW; i++) {
+        const int blk = wave8 * PW + i, rt = (blk < NA ? blk : blk - NA) >> 2, ks = blk & 3;
+        if (blk < NA) {
+            int am = m0 + rt * 16 + fr;
+            if (am > p.M - 1) am = p.M - 1;                     // rows >= M are never stored
+            src[i] = (const bf16_t*)p.A + ((((int64_t)(am >> 4) * (p.K >> 5) + ks) * 64) + (am & 15) + 16 * fg) * 8;
+        } else src[i] = (const bf16_t*)p.W + (((int64_t)((n0 >> 4) + rt) * (p.K >> 5) + ks) * 64 + lane) * 8;
+        src[i] += (int64_t)k0 * 2048;
+    }
+    auto stage = [&](int buf, int s) {
+        char* base = smem + buf * SB + wave8 * (PW * 1024);
+        const bool cut = ragged && s == n - 1;
+#pragma unroll
+        for (int i = 0; i < PW; i++) {
+            if (cut && ((wave8 * PW + i) & 2)) continue;        // (k-steps 2 and 3; waited for with vmcnt(0))
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] + (int64_t)s * 2048),
+                                             (__attribute__((address_space(3))) void*)(base + i * 1024), 16, 0, 0);
+        }
+    };
+    // a wave's column tiles: neighbours for gate | up pairs, else two apart (a head's rotated halves then lie in one wave)
+    constexpr bool PAIRS = epi_glu(EPI);
+    int ct[CT];
+#pragma unroll
+    for (int j = 0; j < CT; j++) ct[j] = PAIRS ? CT * wn + j : wn + 2 * j;
+    // (the row tiles this wave finishes, below: the scales of a deferred RMSNorm are fetched beside the first operands)
+    constexpr bool QKV = EPI == EPI_QKV, BOTH = TM % 2 == 0 || !(PAIRS || QKV), RSTD = PAIRS || EPI == EPI_STORE;
+    constexpr int F = TM * CT, H = BOTH ? F / 2 : F, NR = (H - 1) / CT + 1 + (H % CT ? 1 : 0);
+    const int i0 = BOTH ? kh * H / CT : 0;
+    f32x4 acc[F];
+#pragma unroll
+    for (int i = 0; i < F; i++) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < NST - 1; s++)
+        if (s < n) stage(s, s);
+    float rstd[NR];
+#pragma unroll
+    for (int r = 0; r < NR; r++) rstd[r] = RSTD && p.rs_in && (BOTH || kh == 0) ? deferred_rstd(p, min(m0 + (wm * TM + i0 + r) * 16 + fr, p.M - 1)) : 1.0f;
+    int buf = 0;
+    for (int t = 0; t < n; t++) {
+        // my pieces of stage t landed; the ring's younger stages stay in flight (a cut stage only ever is the youngest)
+        if (n - 1 - t > NST - 2 || (n - 1 - t == NST - 2 && !ragged)) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PW * (NST - 2)) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();           // everybody's pieces landed, and everybody is done with the slot that is filled next
+        __builtin_amdgcn_sched_barrier(0);
+        if (t + NST - 1 < n) stage(buf == 0 ? NST - 1 : buf - 1, t + NST - 1);
+        const char* sb = smem + buf * SB + kh * 2048 + lane * 16;
+        if (!(kh == 1 && ragged && t == n - 1)) {
+            bf16x8 af[2][TM], wf[2][CT];
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++) {
+#pragma unroll
+                for (int j = 0; j < CT; j++) wf[ks][j] = *(const bf16x8*)(sb + NA * 1024 + ct[j] * 4096 + ks * 1024);
+#pragma unroll
+                for (int i = 0; i < TM; i++) af[ks][i] = *(const bf16x8*)(sb + (wm * TM + i) * 4096 + ks * 1024);
+            }
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+                for (int i = 0; i < TM; i++)
+#pragma unroll
+                    for (int j = 0; j < CT; j++)
+                        acc[i * CT + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[ks][j], af[ks][i], acc[i * CT + j], 0, 0, 0);
+        }
+        buf = buf + 1 == NST ? 0 : buf + 1;
+        __builtin_amdgcn_s_waitcnt(0xC07F);     // fragment reads retired before the barrier that lets their slot be filled
+    }
+    // add the K halves: each of the two waves keeps half of the fragments (all of them the first one, where pairs would be cut)
+    __syncthreads();
+    f32x4* red = (f32x4*)smem + lane;
+    f32x4 mine[H];
+    if constexpr (BOTH) {
+#pragma unroll
+        for (int e = 0; e < H; e++) red[(wave8 * H + e) * 64] = kh ? acc[e] : acc[H + e];
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < H; e++) mine[e] = (kh ? acc[H + e] : acc[e]) + red[((wave8 ^ 4) * H + e) * 64];
+    } else {
+        if (kh == 1)
+#pragma unroll
+            for (int e = 0; e < H; e++) red[(wave * H + e) * 64] = acc[e];
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < H; e++) mine[e] = acc[e] + red[(wave * H + e) * 64];
+    }
+    if (p.splits > 1 && !split_finish<H>(p, cb * groups + item / p.splits, part, p.splits, (BOTH ? 8 : 4) * H * 1024, BOTH ? wave8 : wave, mine, (int*)(smem + NST * SB), BOTH || kh == 0)) return;
+    if (!BOTH && kh == 1) return;
+
+#pragma unroll
+    for (int e = 0; e < H; e += (PAIRS || (QKV && CT == 2) ? 2 : 1)) {
+        const int idx = (BOTH ? kh * H : 0) + e, i = idx / CT, j = idx - i * CT;
+        const int m = m0 + (wm * TM + i) * 16 + fr, ctile = PAIRS ? CT * wn + j : wn + 2 * j;
+        const int nn = n0 + ctile * 16 + 4 * fg;
+        const float rs = !RSTD ? 1.0f : BOTH && kh ? rstd[(H + e) / CT - H / CT] : rstd[e / CT];
+        if constexpr (QKV) {
+            if (CT == 4 && (e & 2)) continue;                        // (pairs are CT / 2 fragments apart)
+            epilogue_qkv_pair(p, m, n0 / (32 * CT), 16 * ctile + 4 * fg, mine[e], mine[e + CT / 2]);      // the workgroup's columns are one head
+        } else if constexpr (PAIRS) {
+            epilogue_glu4<EPI, OutT>(p, m, ((n0 >> 4) + ctile) / 2 * 16 + 4 * fg, mine[e], mine[e + 1], rs);
+        } else if (EPI == EPI_RESID && p.rs_out) {                   // deferred RMSNorm producer: as in the decode kernel (N % 16 == 0)
+            f32x4 v = mine[e];
+            float ss = 0.f;
+            if (m < p.M && nn < p.N) {
+                if (p.bias) v += *(const f32x4*)(p.bias + nn);
+                float* x = (float*)p.C + (int64_t)m * p.ldc + nn;
+                const f32x4 o = *(f32x4*)x + p.alpha * v;
+                *(f32x4*)x = o;
+                act_store4<bf16_t>(p.nrm_xn, m, nn, p.N, o * *(const f32x4*)(p.nrm_w + nn));
+                ss = o[0] * o[0] + o[1] * o[1] + o[2] * o[2] + o[3] * o[3];
+            }
+            ss += __shfl_xor(ss, 16, 64);
+            ss += __shfl_xor(ss, 32, 64);
+            if (fg == 0 && m < p.M && nn < p.N) p.rs_out[(int64_t)m * (p.N >> 4) + (nn >> 4)] = ss;
+        } else epilogue4<EPI, OutT>(p, m, nn, mine[e], rs);
+    }
+}
+
     else return __builtin_nontemporal_load(p);
 }
 
@@ -1487,10 +1734,53 @@ void launch_gemm_bf16(hipStream_t st, const GemmArgs& a) {
     if (tile == 3) launch_gemm_tile<256, 256, 2, 4, 2, EPI, OutT>(st, a);
     else if (tile == 2) launch_gemm_tile<256, 128, 4, 2, 3, EPI, OutT>(st, a);
     else launch_gemm_tile<128, 128, 2, 2, 2, EPI, OutT>(st, a);
+// 65 .. MID_MAX_ROWS rows: returns false where gemm_mid_bf16_kernel does not apply
+inline int g_mid = 1;               // nvl_set_tuning key 38: 0 never
+inline int g_mid_splits = 0;        // nvl_set_tuning key 39: parts of K (0: from the grid)
+template <int MT, int CT, int EPI, typename OutT>
+static inline void launch_gemm_mid_rows(hipStream_t st, const GemmArgs& a0) {
+    GemmArgs a = a0;
+    const int nb = cdiv(a.N, 32 * CT), groups = cdiv(a.M, 16 * MT);
+    a.splits = 1;
+    if (a.split_ws) {
+        // four stages and more a part (2048 x 2048 at 96 rows: 15.8 / 12.3 / 10.6 / 11.3 us in 1 / 2 / 4 / 8 parts; 2048 x 8192: 47.7 / 29.3 / 19.6 / 17.8)
+        while (nb * groups * a.splits * 2 <= 256 && (a.K >> 7) / (a.splits * 2) >= 4 && a.splits < 8) a.splits *= 2;
+        if (g_mid_splits) a.splits = std::min(g_mid_splits, std::max(1, a.K >> 7));
+        while (a.splits > 1 && (nb * groups > SPLIT_MAX_TILES || (int64_t)nb * groups * a.splits * MT * CT * 2048 > SPLIT_WS_BYTES)) a.splits--;
+    }
+    NVL_LDS_ATTR((gemm_mid_bf16_kernel<MT, CT, EPI, OutT>), (mid_lds_bytes<MT, CT>()));
+    hipLaunchKernelGGL((gemm_mid_bf16_kernel<MT, CT, EPI, OutT>), dim3(cdiv(nb, 8) * 8 * groups * a.splits), dim3(512), (mid_lds_bytes<MT, CT>()), st, a);
+}
+template <int EPI, typename OutT>
+static inline bool launch_gemm_mid(hipStream_t st, const GemmArgs& a) {
+    if (!g_mid || a.M <= 64 || a.M > MID_MAX_ROWS || a.M > g_chunk_max_m || a.K % 64 != 0 || a.a_rows || a.seg || a.tile_map || a.sk_part || a.moe_gate || a.c_row0 || g_force_tile) return false;
+    // (GPT-2's 768-wide projections at 96 rows: 12.7 / 12.0 / 11.1 us here, 8.8 / 10.1 / 9.3 in the decode form)
+    if ((EPI != EPI_QKV && a.K < 2048) || (EPI == EPI_RESID && a.rs_in)) return false;
+    const int groups = cdiv(a.M, 128), rows = cdiv(cdiv(a.M, groups), 32) * 2;      // 16-row tiles of a group: 4, 6 or 8
+    if constexpr (EPI == EPI_QKV) {
+        if (a.qkv.hd == 128) {
+            if (cdiv(a.N, 128) * cdiv(a.M, 64) > 512) return false;
+            launch_gemm_mid_rows<4, 4, EPI, OutT>(st, a);      // (a head of 128 columns per workgroup: 64 rows leave room for three stages)
+            return true;
+        }
+        if (a.qkv.hd != 64) return false;
+    }
+    // One row group reads the weights once at any width up to a few rounds of workgroups (a workgroup per CU: each round has its own
+    // ramp; LM head at 128 rows 168 us against 152 on the tiles, 28672 x 4096 72 against 74).  Several groups pay while one round holds
+    // them (3072 x 2048: 192 rows 12.5 against 17.4 us, 512 rows 18.3 against 29; 16384 x 2048 at 512 rows 68 against 43).
+    const int wgs = cdiv(a.N, 64) * groups;
+    if (wgs > (groups == 1 ? 512 : 256)) return false;
+    if (rows <= 4) launch_gemm_mid_rows<4, 2, EPI, OutT>(st, a);
+    else if (rows <= 6) launch_gemm_mid_rows<6, 2, EPI, OutT>(st, a);
+    else launch_gemm_mid_rows<8, 2, EPI, OutT>(st, a);
+    return true;
+}
+
 }
 
 template <int EPI, typename OutT>
 void launch_gemm_f32(hipStream_t st, const GemmArgs& a) {
+    if (launch_gemm_mid<EPI, OutT>(st, a)) return;
     const int tiles = cdiv(a.M, 64) * cdiv(a.N, 64);
     hipLaunchKernelGGL((gemm_f32_kernel<EPI, OutT>), dim3(tiles), dim3(256), 0, st, a);
 }

@@ -806,6 +806,7 @@ void layered_finalize(nvl_model* m) {
     m->argmax_pidx = dmalloc<int32_t>(std::max<int64_t>(S, Mmax) * cdiv(m->V, ARGMAX_CHUNK));
     m->sk_rows = (int)std::min<int64_t>(std::max<int64_t>(Mmax, 64), SK_TILE_MAX_M);
     if (!m->f32) m->sk_part = dmalloc<float>((int64_t)std::max(m->sk_max_slices, SK_TILE_MAX_SLICES) * m->sk_rows * H);
+    init_split(m);
     m->key_rows.assign(m->masks.size(), 0); m->key_max.assign(m->masks.size(), 0);
     init_slots(m);
     init_meta(m);

@@ -178,6 +178,7 @@ void gemm(nvl_model* m, int epi, bool out_f32, GemmArgs a, double flops = -1.0) 
         : ((double)a.N * a.K + (double)a.M * a.K) * (double)m->wsize + (double)a.M * a.N * (out_f32 || epi == EPI_RESID ? 4.0 : (double)m->wsize);
     KScope ks(m, KC_GEMM, flops >= 0 ? flops : 2.0 * (double)a.M * (double)a.N * (double)a.K, -1, gbytes);
     hipStream_t st = m->stream;
+    a.split_ws = m->split_ws; a.split_cnt = m->split_cnt; a.splits = 1;
     if (m->f32) {
         switch (epi) {
             case EPI_STORE: launch_gemm_f32<EPI_STORE, float>(st, a); break;
@@ -375,7 +376,7 @@ extern "C" void nvl_destroy(nvl_model* m) {
     dfree(m->x); dfree(m->xn); dfree(m->qkv); dfree(m->q); dfree(m->attn_out); dfree(m->attn_part); dfree(m->attn_part_cnt); dfree(m->hbuf); dfree(m->h2);
     dfree(m->xn_last); dfree(m->logits); dfree(m->argmax_dev); dfree(m->argmax_pval); dfree(m->argmax_pidx); dfree(m->router_logits); dfree(m->expert_ids);
     dfree(m->expert_w); dfree(m->seg_start); dfree(m->moe_counts); dfree(m->moe_cursor); dfree(m->moe_tile_map); dfree(m->moe_n_mtiles); dfree(m->perm_token); dfree(m->slot_of); dfree(m->moe_eo); dfree(m->moe_xg);
-    dfree(m->meta_dev); dfree(m->hidden); dfree(m->sk_part); dfree(m->tp_part); dfree(m->ring); dfree(m->rs_part);
+    dfree(m->meta_dev); dfree(m->hidden); dfree(m->sk_part); dfree(m->split_ws); dfree(m->split_cnt); dfree(m->tp_part); dfree(m->ring); dfree(m->rs_part);
     for (int r = 0; r < 8; r++) if (m->p2p_peer[r] && m->p2p_peer[r] != m->p2p_buf) (void)hipIpcCloseMemHandle(m->p2p_peer[r]);
     p2p_give_back(m->p2p_buf, m->p2p_bytes);
     dfree(m->moe_gate); dfree(m->moe_hall); dfree(m->moe_part);
@@ -665,6 +666,13 @@ std::vector<int32_t> swiglu_interleave(int64_t F, int64_t src_base) {
     return idx;
 }
 
+// gemm.h split_finish: launches on m->stream only, one at a time, so one workspace serves all of them
+void init_split(nvl_model* m) {
+    if (m->f32) return;
+    m->split_ws = (float*)dmalloc_bytes(SPLIT_WS_BYTES);
+    m->split_cnt = dmalloc<int32_t>(SPLIT_MAX_TILES);
+    NVL_HIP(hipMemsetAsync(m->split_cnt, 0, SPLIT_MAX_TILES * 4, m->stream));
+}
 void init_slots(nvl_model* m) {
     m->slot_len.assign((size_t)m->opts.max_seqs, 0);
     m->slot_tick.assign((size_t)m->opts.max_seqs, 0);
@@ -899,6 +907,7 @@ extern "C" int nvl_finalize(nvl_model* m) {
     m->sk_rows = (int)std::min<int64_t>(std::max<int64_t>(Mmax, 64), SK_TILE_MAX_M);
     if (!m->f32) m->sk_part = dmalloc<float>((int64_t)std::max(m->sk_max_slices, SK_TILE_MAX_SLICES) * m->sk_rows * H);
     if (!m->f32) m->rs_part = dmalloc<float>((int64_t)cdiv(H, 8) * DEFER_MAX_M);      // x^2 partials per 16 (half tiles: 8) columns
+    init_split(m);
     if (m->tp > 1 || m->tp_force) m->tp_part = dmalloc<float>(Mmax * H);
     init_meta(m);
     NVL_HIP(hipStreamSynchronize(m->stream));   // every memset/copy above ran on the model's own (non-blocking) stream
@@ -1343,7 +1352,7 @@ GemmArgs mk(const void* A, int lda, const void* W, void* C, int ldc, const float
     a.M = M; a.N = N; a.K = K; a.seg = nullptr; a.c_row0 = 0;
     a.qkv = QkvEpi{};
     a.tile_map = nullptr; a.n_mtiles = nullptr; a.w_expert_stride = 0;
-    a.sk_part = nullptr; a.sk_slices = 1; a.m_split = 0; a.rs_half = 0; a.grid_y = 1; a.nrm_w = nullptr; a.nrm_xn = nullptr; a.rs_out = nullptr; a.rs_in = nullptr; a.rs_tiles = 0; a.rs_inv_h = 0.f; a.rs_eps = 0.f;
+    a.sk_part = nullptr; a.sk_slices = 1; a.split_ws = nullptr; a.split_cnt = nullptr; a.splits = 1; a.m_split = 0; a.rs_half = 0; a.grid_y = 1; a.nrm_w = nullptr; a.nrm_xn = nullptr; a.rs_out = nullptr; a.rs_in = nullptr; a.rs_tiles = 0; a.rs_inv_h = 0.f; a.rs_eps = 0.f;
     return a;
 }
 
@@ -1431,7 +1440,7 @@ void tp_p2p_allreduce_resid(nvl_model* m, const float* part, int M, int N, float
 // Prefill and the fp32 mode fuse the add into the GEMM epilogue.  Decode-sized batches split K over
 // `slices` workgroups per column block so that all 256 CUs stream weights (a 2048-column projection has
 // only 128 column blocks), and leave the add to the norm kernel that always follows (PendingResid).
-static int g_qkv_store_max_m = 256;   // nvl_set_tuning key 18: largest prefill batch whose QKV projection runs as decode-form groups + rope_kv_kernel
+static int g_qkv_store_max_m = 64;   // nvl_set_tuning key 18: largest prefill batch whose QKV projection runs as decode-form groups + rope_kv_kernel
 static int g_moe_dense = 1;    // nvl_set_tuning key 22: decode MoE as two dense-masked projections (gemm.h moe_gate); 0 = sort + grouped GEMMs
 static int g_moe_deep = 1;     // nvl_set_tuning key 19: four-stage grouped GEMM for decode-sized MoE batches (0 = two stages)
 static int g_moe_bm = 0;       // nvl_set_tuning key 17: prefill MoE grouped GEMMs: 0 = 256-row tiles on the ping-pong kernel, 128 / 256 = the lock-step tile kernels
@@ -1447,6 +1456,7 @@ static int g_mamba_ssd = 1;    // nvl_set_tuning key 30: chunked (SSD) Mamba2 sc
 static int g_decode_seam = 1;  // nvl_set_tuning key 7: decode_seam_kernel in nvl_decode_greedy (0 = separate kernels)
 static int g_defer_norm = 1;   // nvl_set_tuning key 3: deferred RMSNorm between O-proj and FFN-up in decode (0 = off)
 static int g_sk_slices = 0;    // tuning override (nvl_set_tuning key 1): 0 automatic, 1 = never split
+static int g_mid_resid_rows = 256;   // nvl_set_tuning key 40: up to here the 65..512-row kernel completes a residual projection (gemm_mid_bf16_kernel)
 // consumer side of the deferred RMSNorm: the projection reads xn_raw and scales its accumulators (gemm.h)
 void set_deferred_in(nvl_model* m, GemmArgs& a) {
     a.rs_in = m->rs_part; a.rs_tiles = defer_half(m, a.M) ? m->H / 8 : m->H / 16; a.rs_inv_h = 1.0f / (float)m->H; a.rs_eps = m->cfg.norm_eps;
@@ -1488,7 +1498,7 @@ void resid_gemm(nvl_model* m, const void* A, int lda, const void* W, const float
     // form pull every activation row through every CU (1.3 GB of ingest for that projection: 85 us).  K split over
     // gridDim.y workgroups per tile instead, the slices summed by the norm that follows (which must be the row kernel).
     const bool norm_ok = (M <= 512 && m->H <= 1024 * NORM_ROW_MAXCH) || (m->H % 32 == 0 && m->H <= 2048 && g_norm_t16);   // launch_norm
-    if (g_sk_tile && !m->f32 && M > 64 && M <= m->sk_rows && !m->keep_hidden && m->sk_part && m->pending_slices == 0 &&
+    if (g_sk_tile && !m->f32 && M > (g_mid && K >= 2048 ? std::max(64, std::min(g_mid_resid_rows, g_chunk_max_m)) : 64) && M <= m->sk_rows && !m->keep_hidden && m->sk_part && m->pending_slices == 0 &&
         N % 128 == 0 && K % 64 == 0 && norm_ok && N == m->H && g_force_tile == 0 && m->n_mamba == 0) {
         const int tiles = cdiv(M, 128) * (N / 128);
         while (slices < SK_TILE_MAX_SLICES && tiles * slices < 512 && K / (slices * 2) >= 512) slices *= 2;

@@ -16,10 +16,12 @@ struct OpCtx {   // a model-less nvl_model carrying just a stream and the fields
         m.f32 = precision == NVL_PRECISION_F32;
         m.wsize = m.f32 ? 4 : 2;
         NVL_HIP(hipStreamCreateWithFlags(&m.stream, hipStreamNonBlocking));
+        init_split(&m);
     }
     ~OpCtx() {
         if (m.stream) { (void)hipStreamSynchronize(m.stream); (void)hipStreamDestroy(m.stream); }
         for (void* p : bufs) dfree(p);
+        dfree(m.split_ws); dfree(m.split_cnt);
     }
     void* alloc(int64_t bytes) { void* p = dmalloc_bytes(bytes); bufs.push_back(p); return p; }
     float* up_f32(const float* h, int64_t n) {
@@ -358,10 +360,10 @@ extern "C" int nvl_bench_gemm(int device, int M, int N, int K, int epi, int forc
     for (auto& v : hw) { v = rnd(); if (s & 0x80000000u) v |= 0x8000u; }
     void* A = cx.alloc((int64_t)ha.size() * 2);
     NVL_HIP(hipMemcpy(A, ha.data(), ha.size() * 2, hipMemcpyHostToDevice));
-    // decode shapes (M <= 64) are weight-streaming: rotate through enough copies of W (> 512 MiB in all) that every
+    // decode shapes (M <= 512) are weight-streaming: rotate through enough copies of W (> 512 MiB in all) that every
     // launch reads its weights cold from HBM, as in the model, not from the 256 MiB Infinity Cache
     const int64_t wbytes = (int64_t)hw.size() * 2;
-    const int copies = M <= 64 ? (int)std::min<int64_t>(64, std::max<int64_t>(1, (640ll << 20) / wbytes + 1)) : 1;
+    const int copies = M <= 512 ? (int)std::min<int64_t>(64, std::max<int64_t>(1, (640ll << 20) / wbytes + 1)) : 1;
     std::vector<void*> Ws((size_t)copies);
     for (int cidx = 0; cidx < copies; cidx++) {
         Ws[(size_t)cidx] = cx.alloc(wbytes);
@@ -428,5 +430,8 @@ extern "C" int nvl_set_tuning(int key, int value) {
     if (key == 35) { const int old = g_attn_kv_nt; g_attn_kv_nt = value; return old; }
     if (key == 37) { const int old = g_grouped_split; g_grouped_split = value < 0 || value > GROUPED_SPLITS ? 0 : value; return old; }
     if (key == 36) { const int old = g_wide_ntb; g_wide_ntb = value; return old; }
+    if (key == 38) { const int old = g_mid; g_mid = value; return old; }
+    if (key == 40) { const int old = g_mid_resid_rows; g_mid_resid_rows = value; return old; }
+    if (key == 39) { const int old = g_mid_splits; g_mid_splits = value; return old; }
     return -1;
 }

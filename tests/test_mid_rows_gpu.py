@@ -1,0 +1,57 @@
+"""Projections of 65 .. 512 rows (gemm.h gemm_mid_bf16_kernel: K split over workgroups, split_finish), at the sizes where they can go wrong."""
+import numpy as np
+import pytest
+
+from conftest import rel_err
+
+pytestmark = pytest.mark.gpu
+TOL = 1.5e-2
+
+
+@pytest.mark.parametrize("parts", [0, 1, 2, 5, 8])                 # K split over workgroups; 0: the launcher's choice
+@pytest.mark.parametrize("m,k,n", [(65, 2048, 64), (66, 2112, 200), (96, 2048, 130), (97, 4160, 2048), (128, 2048, 1003), (129, 2048, 256),
+                                   (255, 2176, 320), (257, 2048, 2049), (512, 2048, 192)])
+def test_matmul_is_exact_on_integers(gpu, parts, m, k, n):
+    """Ragged rows, columns and K (a last stage of 64, K parts of unequal length); the sums are exact in fp32 in any order, twice in a
+    row (the counters of a split are zero again)."""
+    a = (np.arange(m * k).reshape(m, k) % 7).astype(np.float32) - 1.0
+    b = (np.arange(k * n).reshape(k, n) % 5).astype(np.float32) - 2.0        # |sums| < 2^24
+    old = gpu.lib().nvl_set_tuning(39, parts)
+    try:
+        got = [gpu.ops.mat_mul(a, b, precision="bf16") for _ in range(2)]
+    finally:
+        gpu.lib().nvl_set_tuning(39, old)
+    want = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32)
+    assert np.array_equal(got[0], want) and np.array_equal(got[1], want)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("n", [65, 97, 128, 130])                  # 130: past the deferred norm
+def test_decode_and_prompt_batches(gpu, hd, n):
+    """Every epilogue of the kernel in a model: decode batches (deferred norms, gate | up pairs) and short prompts (rotated heads, cache rows)
+    against the fp32 mode, and the greedy loop (graph replays) against single steps."""
+    cfg = gpu.synth.tiny_config("llama", hidden=2048, num_heads=2048 // hd, num_kv_heads=512 // hd, head_dim=hd, ffn_dim=2048, max_seq_len=64)
+    w = gpu.synth.make_weights(cfg, seed=4, scale=0.02)
+    r = np.random.default_rng(n)
+    prompts = [r.integers(0, cfg["vocab_size"], 1 + i % 3).tolist() for i in range(n)]
+    ids, got = list(range(n)), {}
+    for precision in ("bf16", "f32"):
+        m = gpu.HipTransformerModel(cfg, w, precision=precision, max_seqs=n, max_batch_tokens=512)
+        for i in ids:
+            m.seq_reset(i)
+        first, _ = m.forward_batch(ids, prompts, [0] * n)
+        step, am = m.forward_batch(ids, [[7]] * n, [len(p) for p in prompts])
+        got[precision] = first, step
+        if precision == "bf16":
+            pos = [len(p) + 1 for p in prompts]
+            one = []
+            for j in range(3):
+                _, am = m.forward_batch(ids, [[int(t)] for t in am], [p + j for p in pos], want_logits=False)
+                one.append(am)
+            for i in ids:
+                m.seq_reset(i)
+            m.forward_batch(ids, prompts, [0] * n, want_logits=False)
+            _, am = m.forward_batch(ids, [[7]] * n, [len(p) for p in prompts], want_logits=False)
+            assert np.array_equal(m.decode_greedy(ids, am, 3), np.stack(one))
+        m.close()
+    assert rel_err(got["bf16"][0], got["f32"][0]) <= TOL and rel_err(got["bf16"][1], got["f32"][1]) <= TOL
