@@ -754,25 +754,6 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_pp_kernel(GemmArgs p) {
 }
 
 // ------------------------------------------------------------------------------------------
-// bf16 skinny kernel (decode: M <= 64 rows).  The projection is then a weight-streaming problem
-// (HBM-bound: every weight byte is read once, activations are a few hundred KB in L2), so the
-// shape of the kernel is set by memory-level parallelism, not by MFMA:
-//   * one workgroup owns NTW 16-row weight tiles (16*NTW output columns) over ALL of K;
-//   * it runs NTW*KSPLIT waves; wave w streams tile w/KSPLIT over K slice w%KSPLIT straight
-//     HBM -> VGPR with non-temporal 16-byte loads — one contiguous KiB per instruction thanks to the
-//     fragment-major layout; no LDS round trip, nothing is shared between waves; two register sets
-//     keep the next block of k-steps in flight behind the current block's MFMAs;
-//   * activations (<= 64 x K bf16, fragment-major too) are read as MFMA fragments from L2;
-//   * the K slices are reduced through LDS in fixed wave order (deterministic, no atomics) and the
-//     fused epilogue (bias / residual / SwiGLU / GELU) runs once per output element.  For SwiGLU
-//     NTW = 2: tile 0 is the gate block, tile 1 the up block of the same 16 features.
-// ------------------------------------------------------------------------------------------
-// weight fragments are read once per launch: non-temporal.  In the 64-row-group launches the groups of a weight block
-// read them side by side, so there they take the regular path and stay in L2 for the other groups.
-template <bool KEEP>
-__device__ __forceinline__ bf16x8 weight_load(const bf16x8* p) {
-    if constexpr (KEEP) return *p;
-// ------------------------------------------------------------------------------------------
 // bf16 kernel for 65 .. 512 rows (large decode batches, short prompts): weights still come from HBM once, but the 64-row groups of the
 // decode form pull every activation row through every CU for 16 weight rows each (FFN-down of Llama-3.2-1B at 96 rows: 128 workgroups x
 // 2 x 1.3 MB, 25 us for 34 MB of weights).  Here a workgroup owns MT x 16 rows by CT x 32 columns, both operands staged through an
@@ -948,6 +929,25 @@ __global__ __launch_bounds__(512, 1) void gemm_mid_bf16_kernel(GemmArgs p) {
     }
 }
 
+// ------------------------------------------------------------------------------------------
+// bf16 skinny kernel (decode: M <= 64 rows).  The projection is then a weight-streaming problem
+// (HBM-bound: every weight byte is read once, activations are a few hundred KB in L2), so the
+// shape of the kernel is set by memory-level parallelism, not by MFMA:
+//   * one workgroup owns NTW 16-row weight tiles (16*NTW output columns) over ALL of K;
+//   * it runs NTW*KSPLIT waves; wave w streams tile w/KSPLIT over K slice w%KSPLIT straight
+//     HBM -> VGPR with non-temporal 16-byte loads — one contiguous KiB per instruction thanks to the
+//     fragment-major layout; no LDS round trip, nothing is shared between waves; two register sets
+//     keep the next block of k-steps in flight behind the current block's MFMAs;
+//   * activations (<= 64 x K bf16, fragment-major too) are read as MFMA fragments from L2;
+//   * the K slices are reduced through LDS in fixed wave order (deterministic, no atomics) and the
+//     fused epilogue (bias / residual / SwiGLU / GELU) runs once per output element.  For SwiGLU
+//     NTW = 2: tile 0 is the gate block, tile 1 the up block of the same 16 features.
+// ------------------------------------------------------------------------------------------
+// weight fragments are read once per launch: non-temporal.  In the 64-row-group launches the groups of a weight block
+// read them side by side, so there they take the regular path and stay in L2 for the other groups.
+template <bool KEEP>
+__device__ __forceinline__ bf16x8 weight_load(const bf16x8* p) {
+    if constexpr (KEEP) return *p;
     else return __builtin_nontemporal_load(p);
 }
 
@@ -1678,10 +1678,53 @@ static inline void launch_gemm_grouped(hipStream_t st, const GemmArgs& a, int ma
                        lds, st, a);
 }
 
+// 65 .. MID_MAX_ROWS rows: returns false where gemm_mid_bf16_kernel does not apply
+inline int g_mid = 1;               // nvl_set_tuning key 38: 0 never
+inline int g_mid_splits = 0;        // nvl_set_tuning key 39: parts of K (0: from the grid)
+template <int MT, int CT, int EPI, typename OutT>
+static inline void launch_gemm_mid_rows(hipStream_t st, const GemmArgs& a0) {
+    GemmArgs a = a0;
+    const int nb = cdiv(a.N, 32 * CT), groups = cdiv(a.M, 16 * MT);
+    a.splits = 1;
+    if (a.split_ws) {
+        // four stages and more a part (2048 x 2048 at 96 rows: 15.8 / 12.3 / 10.6 / 11.3 us in 1 / 2 / 4 / 8 parts; 2048 x 8192: 47.7 / 29.3 / 19.6 / 17.8)
+        while (nb * groups * a.splits * 2 <= 256 && (a.K >> 7) / (a.splits * 2) >= 4 && a.splits < 8) a.splits *= 2;
+        if (g_mid_splits) a.splits = std::min(g_mid_splits, std::max(1, a.K >> 7));
+        while (a.splits > 1 && (nb * groups > SPLIT_MAX_TILES || (int64_t)nb * groups * a.splits * MT * CT * 2048 > SPLIT_WS_BYTES)) a.splits--;
+    }
+    NVL_LDS_ATTR((gemm_mid_bf16_kernel<MT, CT, EPI, OutT>), (mid_lds_bytes<MT, CT>()));
+    hipLaunchKernelGGL((gemm_mid_bf16_kernel<MT, CT, EPI, OutT>), dim3(cdiv(nb, 8) * 8 * groups * a.splits), dim3(512), (mid_lds_bytes<MT, CT>()), st, a);
+}
+template <int EPI, typename OutT>
+static inline bool launch_gemm_mid(hipStream_t st, const GemmArgs& a) {
+    if (!g_mid || a.M <= 64 || a.M > MID_MAX_ROWS || a.M > g_chunk_max_m || a.K % 64 != 0 || a.a_rows || a.seg || a.tile_map || a.sk_part || a.moe_gate || a.c_row0 || g_force_tile) return false;
+    // (GPT-2's 768-wide projections at 96 rows: 12.7 / 12.0 / 11.1 us here, 8.8 / 10.1 / 9.3 in the decode form)
+    if ((EPI != EPI_QKV && a.K < 2048) || (EPI == EPI_RESID && a.rs_in)) return false;
+    const int groups = cdiv(a.M, 128), rows = cdiv(cdiv(a.M, groups), 32) * 2;      // 16-row tiles of a group: 4, 6 or 8
+    if constexpr (EPI == EPI_QKV) {
+        if (a.qkv.hd == 128) {
+            if (cdiv(a.N, 128) * cdiv(a.M, 64) > 512) return false;
+            launch_gemm_mid_rows<4, 4, EPI, OutT>(st, a);      // (a head of 128 columns per workgroup: 64 rows leave room for three stages)
+            return true;
+        }
+        if (a.qkv.hd != 64) return false;
+    }
+    // One row group reads the weights once at any width up to a few rounds of workgroups (a workgroup per CU: each round has its own
+    // ramp; LM head at 128 rows 168 us against 152 on the tiles, 28672 x 4096 72 against 74).  Several groups pay while one round holds
+    // them (3072 x 2048: 192 rows 12.5 against 17.4 us, 512 rows 18.3 against 29; 16384 x 2048 at 512 rows 68 against 43).
+    const int wgs = cdiv(a.N, 64) * groups;
+    if (wgs > (groups == 1 ? 512 : 256)) return false;
+    if (rows <= 4) launch_gemm_mid_rows<4, 2, EPI, OutT>(st, a);
+    else if (rows <= 6) launch_gemm_mid_rows<6, 2, EPI, OutT>(st, a);
+    else launch_gemm_mid_rows<8, 2, EPI, OutT>(st, a);
+    return true;
+}
+
 template <int EPI, typename OutT>
 void launch_gemm_bf16(hipStream_t st, const GemmArgs& a) {
     if (a.tile_map) { launch_gemm_grouped<EPI, OutT>(st, a, a.M); return; }   // a.M carries the m-tile bound
     if (launch_gemm_skinny_bf16<EPI, OutT>(st, a)) return;
+    if (launch_gemm_mid<EPI, OutT>(st, a)) return;
     if constexpr (EPI != EPI_QKV) {
         // 64 < M <= g_chunk_max_m (large decode batches): the tile kernels would launch only N/128 * M/128 workgroups, far
         // too few to stream the weights at HBM rate.  Run the decode form over ceil(M/64) groups of 64 activation rows
@@ -1734,53 +1777,10 @@ void launch_gemm_bf16(hipStream_t st, const GemmArgs& a) {
     if (tile == 3) launch_gemm_tile<256, 256, 2, 4, 2, EPI, OutT>(st, a);
     else if (tile == 2) launch_gemm_tile<256, 128, 4, 2, 3, EPI, OutT>(st, a);
     else launch_gemm_tile<128, 128, 2, 2, 2, EPI, OutT>(st, a);
-// 65 .. MID_MAX_ROWS rows: returns false where gemm_mid_bf16_kernel does not apply
-inline int g_mid = 1;               // nvl_set_tuning key 38: 0 never
-inline int g_mid_splits = 0;        // nvl_set_tuning key 39: parts of K (0: from the grid)
-template <int MT, int CT, int EPI, typename OutT>
-static inline void launch_gemm_mid_rows(hipStream_t st, const GemmArgs& a0) {
-    GemmArgs a = a0;
-    const int nb = cdiv(a.N, 32 * CT), groups = cdiv(a.M, 16 * MT);
-    a.splits = 1;
-    if (a.split_ws) {
-        // four stages and more a part (2048 x 2048 at 96 rows: 15.8 / 12.3 / 10.6 / 11.3 us in 1 / 2 / 4 / 8 parts; 2048 x 8192: 47.7 / 29.3 / 19.6 / 17.8)
-        while (nb * groups * a.splits * 2 <= 256 && (a.K >> 7) / (a.splits * 2) >= 4 && a.splits < 8) a.splits *= 2;
-        if (g_mid_splits) a.splits = std::min(g_mid_splits, std::max(1, a.K >> 7));
-        while (a.splits > 1 && (nb * groups > SPLIT_MAX_TILES || (int64_t)nb * groups * a.splits * MT * CT * 2048 > SPLIT_WS_BYTES)) a.splits--;
-    }
-    NVL_LDS_ATTR((gemm_mid_bf16_kernel<MT, CT, EPI, OutT>), (mid_lds_bytes<MT, CT>()));
-    hipLaunchKernelGGL((gemm_mid_bf16_kernel<MT, CT, EPI, OutT>), dim3(cdiv(nb, 8) * 8 * groups * a.splits), dim3(512), (mid_lds_bytes<MT, CT>()), st, a);
-}
-template <int EPI, typename OutT>
-static inline bool launch_gemm_mid(hipStream_t st, const GemmArgs& a) {
-    if (!g_mid || a.M <= 64 || a.M > MID_MAX_ROWS || a.M > g_chunk_max_m || a.K % 64 != 0 || a.a_rows || a.seg || a.tile_map || a.sk_part || a.moe_gate || a.c_row0 || g_force_tile) return false;
-    // (GPT-2's 768-wide projections at 96 rows: 12.7 / 12.0 / 11.1 us here, 8.8 / 10.1 / 9.3 in the decode form)
-    if ((EPI != EPI_QKV && a.K < 2048) || (EPI == EPI_RESID && a.rs_in)) return false;
-    const int groups = cdiv(a.M, 128), rows = cdiv(cdiv(a.M, groups), 32) * 2;      // 16-row tiles of a group: 4, 6 or 8
-    if constexpr (EPI == EPI_QKV) {
-        if (a.qkv.hd == 128) {
-            if (cdiv(a.N, 128) * cdiv(a.M, 64) > 512) return false;
-            launch_gemm_mid_rows<4, 4, EPI, OutT>(st, a);      // (a head of 128 columns per workgroup: 64 rows leave room for three stages)
-            return true;
-        }
-        if (a.qkv.hd != 64) return false;
-    }
-    // One row group reads the weights once at any width up to a few rounds of workgroups (a workgroup per CU: each round has its own
-    // ramp; LM head at 128 rows 168 us against 152 on the tiles, 28672 x 4096 72 against 74).  Several groups pay while one round holds
-    // them (3072 x 2048: 192 rows 12.5 against 17.4 us, 512 rows 18.3 against 29; 16384 x 2048 at 512 rows 68 against 43).
-    const int wgs = cdiv(a.N, 64) * groups;
-    if (wgs > (groups == 1 ? 512 : 256)) return false;
-    if (rows <= 4) launch_gemm_mid_rows<4, 2, EPI, OutT>(st, a);
-    else if (rows <= 6) launch_gemm_mid_rows<6, 2, EPI, OutT>(st, a);
-    else launch_gemm_mid_rows<8, 2, EPI, OutT>(st, a);
-    return true;
-}
-
 }
 
 template <int EPI, typename OutT>
 void launch_gemm_f32(hipStream_t st, const GemmArgs& a) {
-    if (launch_gemm_mid<EPI, OutT>(st, a)) return;
     const int tiles = cdiv(a.M, 64) * cdiv(a.N, 64);
     hipLaunchKernelGGL((gemm_f32_kernel<EPI, OutT>), dim3(tiles), dim3(256), 0, st, a);
 }
