@@ -1002,7 +1002,7 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
     // (MT = 4 — batches above 32 and the 64-row groups of larger ones — has no registers to hold it across the stream:
     // 34-54 spilled there, QKV at 128 rows 7.2 -> 10.8 us; those launches are long enough to fetch it in the epilogue)
     constexpr bool RSTD_PRE = MT <= 2;
-    const float rstd_pre = (RSTD_PRE && (EPI == EPI_STORE || epi_glu(EPI)) && wave < NTW * MT) ? deferred_rstd(p, 16 * i_pre + fr) : 1.0f;   // (only the waves that run an epilogue element)
+    const float rstd_pre = (RSTD_PRE && (EPI == EPI_STORE || EPI == EPI_RESID || epi_glu(EPI)) && wave < NTW * MT) ? deferred_rstd(p, 16 * (i_pre + i_off) + fr) : 1.0f;   // (only the waves that run an epilogue element)
     // (grid_y: gridDim.y as an explicit argument — the built-in lives in the hidden part of the kernarg block and costs a
     // dependent scalar round trip of its own before the first weight load)
     const int nslices = p.m_split ? 1 : p.grid_y, slice = p.m_split ? 0 : blockIdx.y;
@@ -1155,6 +1155,7 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
             const int t = e / MT, i = e - t * MT;
             const int m = 16 * (i + i_off) + fr, n = (nt0 + t) * 16 + 4 * fg;      // N % 16 == 0 (hidden width)
             f32x4 v = ksum(t, i);
+            if (p.rs_in) v *= RSTD_PRE && i == i_pre ? rstd_pre : deferred_rstd(p, m);
             float ss = 0.f;
             if (m < p.M && n < p.N && (!HALF || (fg >> 1) == half)) {
                 if (p.bias) v += *(const f32x4*)(p.bias + n);

@@ -384,7 +384,7 @@ extern "C" void nvl_destroy(nvl_model* m) {
     if (m->am_host) (void)hipHostFree(m->am_host);
     dfree(m->ring_pos0);
     dfree(m->conv_tail); dfree(m->stamp_buf); dfree(m->ssd_z); dfree(m->ssd_decay);
-    dfree(m->ssm_state); dfree(m->mproj); dfree(m->mxbc); dfree(m->mdelta); dfree(m->my); dfree(m->myn);
+    dfree(m->ssm_state); dfree(m->mproj); dfree(m->mxbc); dfree(m->mdelta); dfree(m->mrs); dfree(m->my); dfree(m->myn);
     free_sample_bufs(m->samp);
     dfree(m->samp_hist); dfree(m->samp_hist_len); dfree(m->samp_u_steps);
     if (m->tp_comm) (void)ncclCommDestroy((ncclComm_t)m->tp_comm);
@@ -899,6 +899,7 @@ extern "C" int nvl_finalize(nvl_model* m) {
         m->mproj = dmalloc<float>(Mmax * m->mP);
         m->mxbc = dmalloc<float>(Mmax * m->mConv);
         m->mdelta = dmalloc<float>(Mmax * m->m_nh);
+        m->mrs = dmalloc<float>(64 * (int64_t)m->m_nh);
         m->my = dmalloc<float>(Mmax * m->mEH);
         m->myn = dmalloc_bytes(Mp * m->mEH * (int64_t)m->wsize);
         NVL_HIP(hipMemsetAsync(m->myn, 0, (size_t)(Mp * m->mEH) * m->wsize, m->stream));
@@ -1461,8 +1462,10 @@ static int g_sk_slices = 0;    // tuning override (nvl_set_tuning key 1): 0 auto
 void set_deferred_in(nvl_model* m, GemmArgs& a) {
     a.rs_in = m->rs_part; a.rs_tiles = defer_half(m, a.M) ? m->H / 8 : m->H / 16; a.rs_inv_h = 1.0f / (float)m->H; a.rs_eps = m->cfg.norm_eps;
 }
+// the rows of A still have to be multiplied by 1 / sqrt(sum(part[row][tiles]) / width + eps) (with a deferred norm only)
+struct RowScale { const float* part; int tiles, width; float eps; };
 void resid_gemm(nvl_model* m, const void* A, int lda, const void* W, const float* bias, float alpha, int M, int N, int K,
-                const float* defer_norm_w = nullptr) {
+                const float* defer_norm_w = nullptr, const RowScale* scale = nullptr) {
     if (m->tp > 1 || m->tp_force) {
         // row-parallel projection: this rank holds a K slice -> fp32 partial [M][N] (the bias lives on rank 0 only),
         // all-reduce over the tensor-parallel group, then the residual add (folded into the next norm for decode)
@@ -1484,6 +1487,7 @@ void resid_gemm(nvl_model* m, const void* A, int lda, const void* W, const float
     if (defer_norm_w) {     // deferred RMSNorm: x complete in this launch (no K split over workgroups) + xn_raw + x^2 partials
         a.nrm_w = defer_norm_w; a.nrm_xn = (bf16_t*)m->xn; a.rs_out = m->rs_part; a.m_split = g_defer_norm >= 2 ? 0 : 1;
         a.rs_half = a.m_split && N == m->H && defer_half(m, M) ? 1 : 0;
+        if (scale) { a.rs_in = scale->part; a.rs_tiles = scale->tiles; a.rs_inv_h = 1.0f / (float)scale->width; a.rs_eps = scale->eps; }
         gemm(m, EPI_RESID, true, a);
         return;
     }
@@ -1810,7 +1814,7 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
     const bool tp_defer = tp_on && m->p2p_ready && M <= g_p2p_oneshot_rows && M <= 64;
     const bool defer_ok = g_defer_norm && !m->f32 && (M <= 64 || (M <= DEFER_MAX_M && big_decode && g_defer_norm == 1 && !tp_on)) && !c.use_moe && (!tp_on || tp_defer) && !m->keep_hidden &&
                           c.block_style == NVL_BLOCK_SEQUENTIAL && c.norm_type == NVL_NORM_RMS &&
-                          c.activation_type == NVL_ACT_SWIGLU && H % 256 == 0 && m->rs_part && m->n_mamba == 0;
+                          c.activation_type == NVL_ACT_SWIGLU && H % 256 == 0 && m->rs_part && (m->n_mamba == 0 || M <= 64);
     // MoE layers (decode form): only the O projection carries a norm (the FFN norm); the expert-down projection leaves
     // K-slice partials that the next attention norm sums
     const bool defer_moe_ok = g_defer_norm && c.use_moe && M <= 64 && m->tp == 1 && !m->tp_force && c.block_style == NVL_BLOCK_SEQUENTIAL &&
@@ -1821,9 +1825,13 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
         const LayerW& l = m->layers[li];
         if (l.mamba) {
             // forwardMamba2 (generic_model.go:160-202): norm, Mamba2Layer.Forward (mamba2.go:74-181), residual; norm, shared MLP, residual
-            norm(m, m->x, nullptr, l.t[NVL_T_ATTN_NORM_W], l.t[NVL_T_ATTN_NORM_B], m->xn, M);
+            const bool in_deferred = xn_deferred;
+            if (!xn_deferred && !(li == 0 && (seam & 1))) norm(m, m->x, nullptr, l.t[NVL_T_ATTN_NORM_W], l.t[NVL_T_ATTN_NORM_B], m->xn, M);
+            xn_deferred = false;
             m->site = KS_MAMBA_IN;
-            gemm(m, EPI_STORE, true, mk(m->xn, H, l.t[NVL_T_MAMBA_IN_PROJ].p, m->mproj, m->mP, nullptr, 1.f, M, m->mP, H));
+            GemmArgs ai = mk(m->xn, H, l.t[NVL_T_MAMBA_IN_PROJ].p, m->mproj, m->mP, nullptr, 1.f, M, m->mP, H);
+            if (in_deferred) set_deferred_in(m, ai);
+            gemm(m, EPI_STORE, true, ai);
             MambaArgs a{};
             a.proj = m->mproj; a.P = m->mP; a.EH = m->mEH; a.conv_dim = m->mConv; a.nh = m->m_nh; a.hd = m->m_hd; a.ss = m->m_ss;
             a.ng = m->m_ng; a.K = m->m_K;
@@ -1837,78 +1845,97 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
             a.chain = m->conv_tail ? m->conv_chain : 0;
             a.tail = m->conv_tail ? m->conv_tail + (int64_t)l.mamba_idx * m->conv_tail_layer_stride : nullptr;
             a.tail_slot_stride = m->conv_tail_slot_stride;
-            {
-                KScope ks(m, KC_OTHER, 0, KS_MAMBA_CONV, (double)M * (m->mP + m->mConv + m->m_nh) * 4.0);
-                hipLaunchKernelGGL(mamba_conv_kernel, dim3(M), dim3(256), 0, m->stream, a);
-                if (a.chain) hipLaunchKernelGGL(mamba_tail_kernel, dim3(n_seqs), dim3(256), 0, m->stream, a);
-                NVL_HIP(hipGetLastError());
-            }
-            {
+            // both norms of the layer and the next one's can be carried by the projections in front of them (see below)
+            const bool defer = defer_ok && m->pending_slices == 0 && !l.t[NVL_T_FFN_NORM_B].present();
+            const int per_thread = m->m_ss / (256 / m->m_hd);
+            const bool step = defer && max_len == 1 && !a.chain && m->m_nh % 16 == 0 && m->mEH % 32 == 0 && m->m_hd <= 64 && m->m_ss <= 256 && per_thread >= 4;
+            if (step) {
                 KScope ks(m, KC_OTHER, 2.0 * 3.0 * (double)M * m->mEH * m->m_ss, KS_MAMBA_SCAN,
-                          (double)M * (m->mConv + m->m_nh + m->mEH) * 4.0 + 2.0 * n_seqs * (double)m->ssm_layer_stride * 4.0);
-                const int per = m->m_ss / (256 / m->m_hd);
-                dim3 grid(m->m_nh, n_seqs);
-                // prefill-sized calls, bf16 mode: the chunked (SSD) form on MFMA — 64 tokens per step instead of one
-                const bool ssd = g_mamba_ssd && !m->f32 && max_len >= 16 && (m->m_hd == 32 || m->m_hd == 64) &&
-                                 (m->m_ss == 32 || m->m_ss == 64 || m->m_ss == 128) && m->mConv % 4 == 0 && m->mEH % 4 == 0;
-                // (sequence, head) pairs for fewer than half the CUs and several chunks: the chunks of a sequence in parallel (state
-                // contributions, a short recurrence over the chunks, outputs: three launches; 1 x 2048: 318 -> 90 us per layer) —
-                // with a workgroup per CU already (8 x 512) the extra state traffic loses (86 -> 174 us); scratch capped at 256 MB
-                const int max_chunks = cdiv(max_len, 64);
-                const int64_t z_floats = (int64_t)n_seqs * max_chunks * m->m_nh * m->m_hd * m->m_ss;
-                const bool par = ssd && g_mamba_ssd >= 1 && g_mamba_ssd != 2 && max_chunks >= 4 && m->m_nh * n_seqs < 128 && z_floats * 4 <= (256ll << 20);
-                if (par && z_floats > m->ssd_z_floats) {
-                    NVL_HIP(hipStreamSynchronize(m->stream));
-                    dfree(m->ssd_z); dfree(m->ssd_decay);
-                    m->ssd_z = dmalloc<float>(z_floats); m->ssd_z_floats = z_floats;
-                    m->ssd_decay = dmalloc<float>((int64_t)n_seqs * max_chunks * m->m_nh + 1024);
-                    m->ssd_decay_floats = (int64_t)n_seqs * max_chunks * m->m_nh + 1024;
+                          (double)M * (m->mP * 4.0 + m->mEH * 2.0) + 2.0 * n_seqs * (double)m->ssm_layer_stride * 4.0);
+                const dim3 grid(m->m_nh, n_seqs);
+#define NVL_STEP(PERv) hipLaunchKernelGGL(mamba_step_kernel<PERv>, grid, dim3(256), 0, m->stream, a, (bf16_t*)m->myn, m->mrs)
+                if (per_thread <= 4) NVL_STEP(4); else if (per_thread <= 8) NVL_STEP(8); else if (per_thread <= 16) NVL_STEP(16); else NVL_STEP(32);
+#undef NVL_STEP
+                NVL_HIP(hipGetLastError());
+            } else {
+                {
+                    KScope ks(m, KC_OTHER, 0, KS_MAMBA_CONV, (double)M * (m->mP + m->mConv + m->m_nh) * 4.0);
+                    hipLaunchKernelGGL(mamba_conv_kernel, dim3(M), dim3(256), 0, m->stream, a);
+                    if (a.chain) hipLaunchKernelGGL(mamba_tail_kernel, dim3(n_seqs), dim3(256), 0, m->stream, a);
+                    NVL_HIP(hipGetLastError());
                 }
-                if (par && (int64_t)n_seqs * max_chunks * m->m_nh > m->ssd_decay_floats) {
-                    NVL_HIP(hipStreamSynchronize(m->stream));
-                    dfree(m->ssd_decay);
-                    m->ssd_decay_floats = (int64_t)n_seqs * max_chunks * m->m_nh + 1024;
-                    m->ssd_decay = dmalloc<float>(m->ssd_decay_floats);
-                }
-                a.ssd_z = m->ssd_z; a.ssd_decay = m->ssd_decay;
+                {
+                    KScope ks(m, KC_OTHER, 2.0 * 3.0 * (double)M * m->mEH * m->m_ss, KS_MAMBA_SCAN,
+                              (double)M * (m->mConv + m->m_nh + m->mEH) * 4.0 + 2.0 * n_seqs * (double)m->ssm_layer_stride * 4.0);
+                    const int per = m->m_ss / (256 / m->m_hd);
+                    dim3 grid(m->m_nh, n_seqs);
+                    // prefill-sized calls, bf16 mode: the chunked (SSD) form on MFMA — 64 tokens per step instead of one
+                    const bool ssd = g_mamba_ssd && !m->f32 && max_len >= 16 && (m->m_hd == 32 || m->m_hd == 64) &&
+                                     (m->m_ss == 32 || m->m_ss == 64 || m->m_ss == 128) && m->mConv % 4 == 0 && m->mEH % 4 == 0;
+                    // (sequence, head) pairs for fewer than half the CUs and several chunks: the chunks of a sequence in parallel (state
+                    // contributions, a short recurrence over the chunks, outputs: three launches; 1 x 2048: 318 -> 90 us per layer) —
+                    // with a workgroup per CU already (8 x 512) the extra state traffic loses (86 -> 174 us); scratch capped at 256 MB
+                    const int max_chunks = cdiv(max_len, 64);
+                    const int64_t z_floats = (int64_t)n_seqs * max_chunks * m->m_nh * m->m_hd * m->m_ss;
+                    const bool par = ssd && g_mamba_ssd >= 1 && g_mamba_ssd != 2 && max_chunks >= 4 && m->m_nh * n_seqs < 128 && z_floats * 4 <= (256ll << 20);
+                    if (par && z_floats > m->ssd_z_floats) {
+                        NVL_HIP(hipStreamSynchronize(m->stream));
+                        dfree(m->ssd_z); dfree(m->ssd_decay);
+                        m->ssd_z = dmalloc<float>(z_floats); m->ssd_z_floats = z_floats;
+                        m->ssd_decay = dmalloc<float>((int64_t)n_seqs * max_chunks * m->m_nh + 1024);
+                        m->ssd_decay_floats = (int64_t)n_seqs * max_chunks * m->m_nh + 1024;
+                    }
+                    if (par && (int64_t)n_seqs * max_chunks * m->m_nh > m->ssd_decay_floats) {
+                        NVL_HIP(hipStreamSynchronize(m->stream));
+                        dfree(m->ssd_decay);
+                        m->ssd_decay_floats = (int64_t)n_seqs * max_chunks * m->m_nh + 1024;
+                        m->ssd_decay = dmalloc<float>(m->ssd_decay_floats);
+                    }
+                    a.ssd_z = m->ssd_z; a.ssd_decay = m->ssd_decay;
 #define NVL_SSD(HDv, SSv)                                                                                              \
-                do {                                                                                                   \
-                    constexpr int lds_ = mamba_ssd_lds_bytes<HDv, SSv>();                                              \
-                    if (par) {                                                                                         \
-                        dim3 g3(m->m_nh, n_seqs, max_chunks);                                                          \
-                        NVL_LDS_ATTR((mamba_ssd_kernel<HDv, SSv, 1>), lds_);                                           \
-                        NVL_LDS_ATTR((mamba_ssd_kernel<HDv, SSv, 2>), lds_);                                           \
-                        hipLaunchKernelGGL((mamba_ssd_kernel<HDv, SSv, 1>), g3, dim3(256), lds_, m->stream, a);        \
-                        hipLaunchKernelGGL(mamba_ssd_prefix_kernel, dim3(m->m_nh, n_seqs, cdiv(HDv * SSv, 1024)), dim3(256), 0, m->stream, a, max_chunks, HDv * SSv); \
-                        hipLaunchKernelGGL((mamba_ssd_kernel<HDv, SSv, 2>), g3, dim3(256), lds_, m->stream, a);        \
-                    } else {                                                                                           \
-                        NVL_LDS_ATTR((mamba_ssd_kernel<HDv, SSv, 0>), lds_);                                           \
-                        hipLaunchKernelGGL((mamba_ssd_kernel<HDv, SSv, 0>), grid, dim3(256), lds_, m->stream, a);      \
-                    }                                                                                                  \
-                } while (0)
-                if (ssd) {
-                    if (m->m_hd == 64) { if (m->m_ss == 128) NVL_SSD(64, 128); else if (m->m_ss == 64) NVL_SSD(64, 64); else NVL_SSD(64, 32); }
-                    else { if (m->m_ss == 128) NVL_SSD(32, 128); else if (m->m_ss == 64) NVL_SSD(32, 64); else NVL_SSD(32, 32); }
-                } else
+                    do {                                                                                                   \
+                        constexpr int lds_ = mamba_ssd_lds_bytes<HDv, SSv>();                                              \
+                        if (par) {                                                                                         \
+                            dim3 g3(m->m_nh, n_seqs, max_chunks);                                                          \
+                            NVL_LDS_ATTR((mamba_ssd_kernel<HDv, SSv, 1>), lds_);                                           \
+                            NVL_LDS_ATTR((mamba_ssd_kernel<HDv, SSv, 2>), lds_);                                           \
+                            hipLaunchKernelGGL((mamba_ssd_kernel<HDv, SSv, 1>), g3, dim3(256), lds_, m->stream, a);        \
+                            hipLaunchKernelGGL(mamba_ssd_prefix_kernel, dim3(m->m_nh, n_seqs, cdiv(HDv * SSv, 1024)), dim3(256), 0, m->stream, a, max_chunks, HDv * SSv); \
+                            hipLaunchKernelGGL((mamba_ssd_kernel<HDv, SSv, 2>), g3, dim3(256), lds_, m->stream, a);        \
+                        } else {                                                                                           \
+                            NVL_LDS_ATTR((mamba_ssd_kernel<HDv, SSv, 0>), lds_);                                           \
+                            hipLaunchKernelGGL((mamba_ssd_kernel<HDv, SSv, 0>), grid, dim3(256), lds_, m->stream, a);      \
+                        }                                                                                                  \
+                    } while (0)
+                    if (ssd) {
+                        if (m->m_hd == 64) { if (m->m_ss == 128) NVL_SSD(64, 128); else if (m->m_ss == 64) NVL_SSD(64, 64); else NVL_SSD(64, 32); }
+                        else { if (m->m_ss == 128) NVL_SSD(32, 128); else if (m->m_ss == 64) NVL_SSD(32, 64); else NVL_SSD(32, 32); }
+                    } else
 #undef NVL_SSD
-                if (per <= 4) hipLaunchKernelGGL(mamba_scan_kernel<4>, grid, dim3(256), 0, m->stream, a);
-                else if (per <= 8) hipLaunchKernelGGL(mamba_scan_kernel<8>, grid, dim3(256), 0, m->stream, a);
-                else if (per <= 16) hipLaunchKernelGGL(mamba_scan_kernel<16>, grid, dim3(256), 0, m->stream, a);
-                else hipLaunchKernelGGL(mamba_scan_kernel<32>, grid, dim3(256), 0, m->stream, a);
-                NVL_HIP(hipGetLastError());
+                    if (per <= 4) hipLaunchKernelGGL(mamba_scan_kernel<4>, grid, dim3(256), 0, m->stream, a);
+                    else if (per <= 8) hipLaunchKernelGGL(mamba_scan_kernel<8>, grid, dim3(256), 0, m->stream, a);
+                    else if (per <= 16) hipLaunchKernelGGL(mamba_scan_kernel<16>, grid, dim3(256), 0, m->stream, a);
+                    else hipLaunchKernelGGL(mamba_scan_kernel<32>, grid, dim3(256), 0, m->stream, a);
+                    NVL_HIP(hipGetLastError());
+                }
+                {
+                    KScope ks(m, KC_OTHER, 0, KS_MAMBA_GATE, (double)M * m->mEH * (8.0 + (double)m->wsize));
+                    if (m->f32) hipLaunchKernelGGL((mamba_gate_norm_kernel<float>), dim3(M), dim3(256), 0, m->stream, a, (float*)m->myn);
+                    else hipLaunchKernelGGL((mamba_gate_norm_kernel<bf16_t>), dim3(M), dim3(256), 0, m->stream, a, (bf16_t*)m->myn);
+                    NVL_HIP(hipGetLastError());
+                }
             }
-            {
-                KScope ks(m, KC_OTHER, 0, KS_MAMBA_GATE, (double)M * m->mEH * (8.0 + (double)m->wsize));
-                if (m->f32) hipLaunchKernelGGL((mamba_gate_norm_kernel<float>), dim3(M), dim3(256), 0, m->stream, a, (float*)m->myn);
-                else hipLaunchKernelGGL((mamba_gate_norm_kernel<bf16_t>), dim3(M), dim3(256), 0, m->stream, a, (bf16_t*)m->myn);
-                NVL_HIP(hipGetLastError());
-            }
+            const RowScale gate_rms{m->mrs, m->m_nh, m->mEH, 1e-5f};
             m->site = KS_MAMBA_OUT;
-            resid_gemm(m, m->myn, m->mEH, l.t[NVL_T_MAMBA_OUT_PROJ].p, nullptr, m->resid_alpha, M, H, m->mEH);
-            norm(m, m->x, nullptr, l.t[NVL_T_FFN_NORM_W], l.t[NVL_T_FFN_NORM_B], m->xn, M);
-            ffn_up(m, l, M);
+            resid_gemm(m, m->myn, m->mEH, l.t[NVL_T_MAMBA_OUT_PROJ].p, nullptr, m->resid_alpha, M, H, m->mEH,
+                       defer ? (const float*)l.t[NVL_T_FFN_NORM_W].p : nullptr, step ? &gate_rms : nullptr);
+            if (!defer) norm(m, m->x, nullptr, l.t[NVL_T_FFN_NORM_W], l.t[NVL_T_FFN_NORM_B], m->xn, M);
+            ffn_up(m, l, M, defer);
+            const DevTensor& nxt_w = li + 1 < m->L ? m->layers[li + 1].t[NVL_T_ATTN_NORM_W] : m->g[NVL_T_FINAL_NORM_W];
+            const DevTensor& nxt_b = li + 1 < m->L ? m->layers[li + 1].t[NVL_T_ATTN_NORM_B] : m->g[NVL_T_FINAL_NORM_B];
+            xn_deferred = defer && g_defer_norm != 3 && m->pending_slices == 0 && !nxt_b.present() && (li + 1 < m->L || (!all_rows && M == n_seqs && M <= 64));
             m->site = KS_FFN_DOWN;
-            resid_gemm(m, m->hbuf, m->F, l.t[NVL_T_W2].p, (const float*)l.t[NVL_T_B2].p, m->resid_alpha, M, H, m->F);
+            resid_gemm(m, m->hbuf, m->F, l.t[NVL_T_W2].p, (const float*)l.t[NVL_T_B2].p, m->resid_alpha, M, H, m->F, xn_deferred ? (const float*)nxt_w.p : nullptr);
             tap_layer(m, li, M);
             continue;
         }

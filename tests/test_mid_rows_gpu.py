@@ -1,4 +1,5 @@
-"""Projections of 65 .. 512 rows (gemm.h gemm_mid_bf16_kernel: K split over workgroups, split_finish), at the sizes where they can go wrong."""
+"""Projections of 65 .. 512 rows (gemm.h gemm_mid_bf16_kernel: K split over workgroups, split_finish) and the single-launch Mamba-2 decode
+step (mamba.h mamba_step_kernel), at the sizes where they can go wrong."""
 import numpy as np
 import pytest
 
@@ -55,3 +56,35 @@ def test_decode_and_prompt_batches(gpu, hd, n):
             assert np.array_equal(m.decode_greedy(ids, am, 3), np.stack(one))
         m.close()
     assert rel_err(got["bf16"][0], got["f32"][0]) <= TOL and rel_err(got["bf16"][1], got["f32"][1]) <= TOL
+
+
+@pytest.mark.parametrize("hidden,heads,hd,state,groups", [(512, 16, 64, 128, 2), (256, 16, 32, 32, 1), (256, 16, 32, 256, 4), (512, 32, 32, 64, 32)])
+@pytest.mark.parametrize("n", [1, 16, 17, 64])
+def test_mamba_decode_step(gpu, oracle, hidden, heads, hd, state, groups, n):
+    """One launch from the input projection's rows to the output projection's operand, the gated norm deferred: logits and states of a
+    few steps against the fp32 mode and, for one sequence, the oracle."""
+    cfg = gpu.synth.tiny_config("granite_hybrid", hidden=hidden, num_heads=hidden // 64, num_kv_heads=hidden // 128, mamba_num_heads=heads, mamba_head_dim=hd,
+                                mamba_state_size=state, mamba_n_groups=groups)
+    w = gpu.synth.make_weights(cfg, seed=23, scale=0.05)
+    r = np.random.default_rng(n)
+    prompts = [r.integers(0, cfg["vocab_size"], 1 + i % 4).tolist() for i in range(n)]
+    steps = r.integers(0, cfg["vocab_size"], (3, n)).tolist()
+    ids, got = list(range(n)), {}
+    for precision in ("bf16", "f32"):
+        m = gpu.HipTransformerModel(cfg, w, precision=precision, max_seqs=n, max_batch_tokens=256)
+        for i in ids:
+            m.seq_reset(i)
+        m.forward_batch(ids, prompts, [0] * n, want_logits=False)
+        lg = [m.forward_batch(ids, [[t] for t in s], [len(p) + j for p in prompts])[0] for j, s in enumerate(steps)]
+        got[precision] = lg, m.get_mamba_state(n - 1, 0), m.get_mamba_state(0, 3)
+        m.close()
+    for j in range(3):
+        assert rel_err(got["bf16"][0][j], got["f32"][0][j]) <= TOL
+    assert rel_err(got["bf16"][1], got["f32"][1]) <= TOL and rel_err(got["bf16"][2], got["f32"][2]) <= TOL
+    om = oracle.OracleModel(cfg, w)
+    kv = om.new_cache()
+    om.forward_with_cache(prompts[0], kv, 0)
+    if len(prompts[0]) == 1:              # (a one-token call does not reset the oracle's state: it starts at zero here)
+        for j, s in enumerate(steps):
+            want = om.forward_with_cache([s[0]], kv, 1 + j)[-1]
+            assert rel_err(got["bf16"][0][j][0], want) <= TOL
