@@ -973,7 +973,8 @@ __device__ __forceinline__ void skinny_pass_remap(GemmArgs& p, int& bx) {
 // others pulled 256 KB each through one CU).  The other 8 lanes of every 16-lane row group feed zeros (their loads are
 // predicated off: 4 x 128-byte lines per k-step instead of 8); only the owned rows are stored; the x^2 partials are per
 // 8 columns (rs_tiles = N / 8).
-template <int MT, int NTW, int U, int EPI, typename OutT, bool PASSES = false, bool MOE = false, bool HALF = false>
+// SCALED: a residual projection whose input rows carry a deferred scale of their own (rs_in; its own instance: the others lose 1 % beside it).
+template <int MT, int NTW, int U, int EPI, typename OutT, bool PASSES = false, bool MOE = false, bool HALF = false, bool SCALED = false>
 __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     f32x4* red = (f32x4*)smem;                       // [NTW][ksplit][MT][64]
@@ -1002,7 +1003,7 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
     // (MT = 4 — batches above 32 and the 64-row groups of larger ones — has no registers to hold it across the stream:
     // 34-54 spilled there, QKV at 128 rows 7.2 -> 10.8 us; those launches are long enough to fetch it in the epilogue)
     constexpr bool RSTD_PRE = MT <= 2;
-    const float rstd_pre = (RSTD_PRE && (EPI == EPI_STORE || EPI == EPI_RESID || epi_glu(EPI)) && wave < NTW * MT) ? deferred_rstd(p, 16 * (i_pre + i_off) + fr) : 1.0f;   // (only the waves that run an epilogue element)
+    const float rstd_pre = (RSTD_PRE && (EPI == EPI_STORE || SCALED || epi_glu(EPI)) && wave < NTW * MT) ? deferred_rstd(p, 16 * (i_pre + (SCALED ? i_off : 0)) + fr) : 1.0f;   // (only the waves that run an epilogue element)
     // (grid_y: gridDim.y as an explicit argument — the built-in lives in the hidden part of the kernarg block and costs a
     // dependent scalar round trip of its own before the first weight load)
     const int nslices = p.m_split ? 1 : p.grid_y, slice = p.m_split ? 0 : blockIdx.y;
@@ -1155,7 +1156,7 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
             const int t = e / MT, i = e - t * MT;
             const int m = 16 * (i + i_off) + fr, n = (nt0 + t) * 16 + 4 * fg;      // N % 16 == 0 (hidden width)
             f32x4 v = ksum(t, i);
-            if (p.rs_in) v *= RSTD_PRE && i == i_pre ? rstd_pre : deferred_rstd(p, m);
+            if constexpr (SCALED) v *= rstd_pre;      // (MT = 1: one row tile)
             float ss = 0.f;
             if (m < p.M && n < p.N && (!HALF || (fg >> 1) == half)) {
                 if (p.bias) v += *(const f32x4*)(p.bias + n);
@@ -1521,6 +1522,17 @@ static inline bool launch_gemm_skinny_ntw(hipStream_t st, const GemmArgs& a) {
                                        (size_t)NTW * ks * 64 * 16, st, a);
                 } else {
                     hipLaunchKernelGGL((gemm_skinny_bf16_kernel<1, NTW, 4, EPI, OutT, false, true>), dim3(nblocks, cdiv(a.M, 16)), dim3(NTW * ks * 64),
+                                       (size_t)NTW * ks * 64 * 16, st, a);
+                }
+                return true;
+            }
+            if (a.rs_in) {        // (the output projection of a Mamba-2 step)
+                if (a.rs_half) {
+                    if (a.M > 16) return false;
+                    hipLaunchKernelGGL((gemm_skinny_bf16_kernel<1, NTW, 4, EPI, OutT, false, false, true, true>), dim3(2 * nblocks, 1), dim3(NTW * ks * 64),
+                                       (size_t)NTW * ks * 64 * 16, st, a);
+                } else {
+                    hipLaunchKernelGGL((gemm_skinny_bf16_kernel<1, NTW, 4, EPI, OutT, false, false, false, true>), dim3(nblocks, cdiv(a.M, 16)), dim3(NTW * ks * 64),
                                        (size_t)NTW * ks * 64 * 16, st, a);
                 }
                 return true;
