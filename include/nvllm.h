@@ -581,6 +581,7 @@ int nvl_bench_gemm(int device, int M, int N, int K, int epi, int force_bnt, int 
  * key 36: weight tiles per wave of the wide decode projections (FFN-up, LM head): 0 (default) 2 for 17..32 rows and N < 65536, else 4;
  * 2 / 4 forced.
  * key 37: workgroups the keys of a row tile are split over in the short grouped attention (lists of layers): 0 (default) from the context.
+ * key 41: parts of K for the 256x256 tiles of the last, partly filled round (0, default: from the grid; 1 never).
  * key 33: MoE decode: the experts' down projection carries the next RMSNorm (no K slices, no norm launch before the next QKV);
  * 0 (default): measured slower.
  * The settings are PROCESS-GLOBAL and unsynchronised (every model in the process sees them): set them from one thread

@@ -609,7 +609,8 @@ __device__ __forceinline__ bool split_finish(const GemmArgs& p, int tile, int pa
 // after its last readers retired their ds_reads before the barrier that ended L(s-1) of the LATE group (WAR);
 // stage s+1 is waited for at the end of L(s) by every wave, one barrier before the early group reads it (RAW).
 // ------------------------------------------------------------------------------------------
-template <int EPI, typename OutT, int STAGES = 4, int PRIO = 0, int WAVES_N = 4, int BN = 256>
+// SPLIT: its own instance, the unsplit loop loses 3 % beside the code of the sum
+template <int EPI, typename OutT, int STAGES = 4, int PRIO = 0, int WAVES_N = 4, int BN = 256, bool SPLIT = false>
 __global__ __launch_bounds__(512, 1) void gemm_bf16_pp_kernel(GemmArgs p) {
     // BN 256: WAVES_N = 4 -> wave tile 128x64 (a head of 64 per wave), WAVES_N = 2 -> 64x128 (a head of 128 per wave);
     // BN 128 (mid-size M: twice the tiles): WAVES_N = 2 -> wave tile 64x64
@@ -623,7 +624,7 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_pp_kernel(GemmArgs p) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int tiles_n = (p.N + BN - 1) / BN;
     int tm, tn;
-    int row_base = 0;
+    int row_base = 0, part = 0, split_tile = -1;
     if (p.tile_map) {
         // grouped launch (MoE prefill): m-tile ti = (expert, 256-row segment of its rows in the expert-ordered buffer).
         // After xcd_remap an XCD owns a contiguous range of (ti, tn): whole experts, so an expert's weights and each
@@ -637,6 +638,20 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_pp_kernel(GemmArgs p) {
         p.c_row0 = row_base;
         p.W = (const bf16_t*)p.W + (int64_t)p.tile_map[4 * ti] * p.w_expert_stride;
         tm = 0;
+    } else if (SPLIT) {
+        // Each XCD has a contiguous run of tiles, 32 at a time; those of its last, partly filled round are cut along K into p.splits parts
+        // (the launcher says when).  All workgroups of the round walk the same K ranges in step, so the panels they share
+        // stay in the XCD's L2.
+        const int tiles_m = cdiv_dev(p.M, BM), T = tiles_m * tiles_n, xcd = blockIdx.x & 7, k = blockIdx.x >> 3;
+        const int first = xcd * (T >> 3) + min(xcd, T & 7), n = (T >> 3) + (xcd < (T & 7) ? 1 : 0), whole = n & ~31, rest = n - whole;
+        int i = k;
+        if (k >= whole) {
+            if (k - whole >= rest * p.splits) return;
+            part = (k - whole) / rest;
+            i = whole + (k - whole) - part * rest;
+            split_tile = xcd * (32 / p.splits) + i - whole;      // (rest * splits <= 32)
+        }
+        tile_coords(first + i, tiles_m, tiles_n, 4, tm, tn);
     } else {
         tile_coords(xcd_remap(blockIdx.x, gridDim.x), gridDim.x / tiles_n, tiles_n, 4, tm, tn);
     }
@@ -646,6 +661,9 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_pp_kernel(GemmArgs p) {
     const int fr = lane & 15, fg = lane >> 4;
     if (m0 >= p.M) return;
 
+    // K-steps of this workgroup
+    const int k_all = p.K >> 5, k0 = !SPLIT || split_tile < 0 ? 0 : (int)((int64_t)part * k_all / p.splits);
+    const int nt = !SPLIT || split_tile < 0 ? k_all : (int)((int64_t)(part + 1) * k_all / p.splits) - k0;            // stages
     const bf16_t* src[PW];
 #pragma unroll
     for (int i = 0; i < PW; i++) {
@@ -658,6 +676,7 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_pp_kernel(GemmArgs p) {
         } else {
             src[i] = (const bf16_t*)p.W + ((int64_t)((n0 >> 4) + blk - NA) * (p.K >> 5) * 64 + lane) * 8;
         }
+        src[i] += (int64_t)k0 * 512;
     }
     auto stage = [&](int buf, int ks) {
         char* base = smem + buf * STAGE_BYTES + wave * (PW * 1024);
@@ -674,7 +693,6 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_pp_kernel(GemmArgs p) {
 #pragma unroll
         for (int j = 0; j < TN; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    const int nt = p.K >> 5;            // stages
 #pragma unroll
     for (int s = 0; s < STAGES - 1; s++)
         if (s < nt) stage(s, s);
@@ -732,6 +750,7 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_pp_kernel(GemmArgs p) {
         buf = buf + 1 == STAGES ? 0 : buf + 1;
     }
     if (grp == 0) __builtin_amdgcn_s_barrier();         // pairs with the late group's last barrier
+    if (SPLIT && split_tile >= 0 && !split_finish<TM * TN>(p, split_tile, part, p.splits, BM * BN * 4, wave, &acc[0][0], (int*)(smem + STAGES * STAGE_BYTES))) return;
 
 #pragma unroll
     for (int i = 0; i < TM; i++) {
@@ -1658,17 +1677,53 @@ static inline void launch_gemm_tile(hipStream_t st, const GemmArgs& a) {
                        dim3(tiles, (EPI == EPI_RESID && a.sk_part) ? a.sk_slices : 1), dim3(WAVES_M * WAVES_N * 64), lds, st, a);
 }
 
-// how well `tiles` workgroups (one per CU at a time for the big tiles) fill 256 CUs
-static inline double cu_fill(int tiles, int per_cu) {
-    const int slots = 256 * per_cu;
-    return (double)tiles / (double)(cdiv(tiles, slots) * slots);
+// What a projection takes on the two prefill forms, in microseconds: fitted to launches of 10 .. 600 us between 480 and 8500 rows, good to
+// 15 %.  Ping-pong 256x256 tiles: a K-step is 0.46 us while power does not bind (up to half of the CUs busy) and 0.69 with all of
+// them; the last round's tiles (`rest` of 32 per XCD) may be cut into parts, which costs 10 + 2.5 us a part.
+constexpr int PP_LDS = 4 * 32 * 1024 + 16;
+inline int g_pp_split = 0;          // nvl_set_tuning key 41: 0 from the grid, 1 never, n parts
+static inline double gemm_epilogue_us(int M, int N, int bytes) { return (double)M * N * bytes / 4.5e6; }
+static inline double pp_cost(int M, int N, int K, int out_bytes, bool can_split, int& parts) {
+    const int T = cdiv(M, 256) * cdiv(N, 256), n = cdiv(T, 8), rest = n & 31, stages = K >> 5;
+    parts = 1;
+    double best = 0;
+    for (int c = 1; c <= 8 && rest * c <= 32; c++) {
+        if (c > 1 && (!can_split || !rest || T < 8 || stages / c < 12 || (g_pp_split && c != g_pp_split))) continue;
+        const double fill = rest * c / 32.0, t = rest ? (stages / c) * (0.46 + (fill > 0.45 ? 0.42 * (fill - 0.45) : 0.0)) + (c > 1 ? 10.0 + 2.5 * c : 0.0) : 0.0;
+        if (c == 1 || t < 0.92 * best || g_pp_split == c) { best = t; parts = c; }
+    }
+    return (n >> 5) * (stages * 0.69 + 4.0) + best + gemm_epilogue_us(M, N, out_bytes) + 6.0;
+}
+// 128x128 tiles, two workgroups a CU; K in `slices` whose sums somebody else adds up
+static inline double tile128_cost(int M, int N, int K, int out_bytes, int slices) {
+    const double wgs = (double)cdiv(M, 128) * cdiv(N, 128) * slices, per = 9.7 * wgs / 256.0 + 1.5;
+    return K / 1024.0 / slices * (per > 10.2 ? per : 10.2) + 4.0 + (slices > 1 ? gemm_epilogue_us(M, N, 8 * slices) : 0.5 * gemm_epilogue_us(M, N, out_bytes));
+}
+// is the ping-pong form the faster one?  (its parts in a.splits)
+template <int EPI, typename OutT>
+static inline bool pp_wins(GemmArgs& a) {
+    a.splits = 1;
+    if (a.seg || a.a_rows || a.tile_map || a.sk_part || a.K < 160) return false;
+    const int bytes = EPI == EPI_RESID ? 8 : EPI == EPI_GROUPED_RAW ? 4 : epi_glu(EPI) ? (int)sizeof(OutT) / 2 : (int)sizeof(OutT);
+    return pp_cost(a.M, a.N, a.K, bytes, a.split_ws != nullptr, a.splits) < 0.93 * tile128_cost(a.M, a.N, a.K, bytes, 1);
+}
+template <int EPI, typename OutT, int WAVES_N>
+static inline void launch_pp(hipStream_t st, const GemmArgs& a) {
+    const int T = cdiv(a.M, 256) * cdiv(a.N, 256), n = cdiv(T, 8);
+    if (a.splits > 1) {
+        NVL_LDS_ATTR((gemm_bf16_pp_kernel<EPI, OutT, 4, 0, WAVES_N, 256, true>), PP_LDS);
+        hipLaunchKernelGGL((gemm_bf16_pp_kernel<EPI, OutT, 4, 0, WAVES_N, 256, true>), dim3(8 * ((n & ~31) + (n & 31) * a.splits)), dim3(512), PP_LDS, st, a);
+    } else {
+        NVL_LDS_ATTR((gemm_bf16_pp_kernel<EPI, OutT, 4, 0, WAVES_N>), PP_LDS);
+        hipLaunchKernelGGL((gemm_bf16_pp_kernel<EPI, OutT, 4, 0, WAVES_N>), dim3(T), dim3(512), PP_LDS, st, a);
+    }
 }
 
 template <int EPI, typename OutT>
 static inline void launch_gemm_grouped(hipStream_t st, const GemmArgs& a, int max_mtiles) {
     if (a.grp_bm == 512) {      // prefill MoE, the default: 256-row m-tiles on the ping-pong kernel
-        NVL_LDS_ATTR((gemm_bf16_pp_kernel<EPI, OutT, 4, 0>), 4 * 32 * 1024);
-        hipLaunchKernelGGL((gemm_bf16_pp_kernel<EPI, OutT, 4, 0>), dim3(cdiv(a.N, 256) * max_mtiles), dim3(512), 4 * 32 * 1024, st, a);
+        NVL_LDS_ATTR((gemm_bf16_pp_kernel<EPI, OutT, 4, 0>), PP_LDS);
+        hipLaunchKernelGGL((gemm_bf16_pp_kernel<EPI, OutT, 4, 0>), dim3(cdiv(a.N, 256) * max_mtiles), dim3(512), PP_LDS, st, a);
         return;
     }
     if (a.grp_bm == 256) {      // prefill MoE with long expert segments: 256-row m-tiles, three stages
@@ -1757,10 +1812,10 @@ void launch_gemm_bf16(hipStream_t st, const GemmArgs& a) {
     if (a.rs_in || a.rs_out) throw std::runtime_error("gemm: a deferred-RMSNorm projection did not fit the decode kernels");
     if constexpr (EPI == EPI_QKV) {
         if (a.qkv.hd == 128) {     // a wave must own a whole 128-column head: 256x256 tile as 4x2 waves of 64x128
-            const int t3 = cdiv(a.M, 256) * cdiv(a.N, 256);
-            if (g_force_tile == 0 && t3 >= 192 && cu_fill(t3, 1) >= 0.74 && a.K >= 160 && !a.seg && !a.a_rows) {
-                NVL_LDS_ATTR((gemm_bf16_pp_kernel<EPI, OutT, 4, 0, 2>), 4 * 32 * 1024);     // the ping-pong form, wave tile 64x128
-                hipLaunchKernelGGL((gemm_bf16_pp_kernel<EPI, OutT, 4, 0, 2>), dim3(t3), dim3(512), 4 * 32 * 1024, st, a);
+            if (g_force_tile == 0 && a.K >= 160 && !a.seg && !a.a_rows) {
+                GemmArgs as = a;
+                pp_wins<EPI, OutT>(as);                   // (for its parts: the lock-step form below is never the faster one)
+                launch_pp<EPI, OutT, 2>(st, as);                  // wave tile 64x128
                 return;
             }
             launch_gemm_tile<256, 256, 4, 2, 2, EPI, OutT>(st, a);
@@ -1768,25 +1823,13 @@ void launch_gemm_bf16(hipStream_t st, const GemmArgs& a) {
         }
     }
     int tile = g_force_tile;
-    if (tile == 0) {
-        tile = 1;
-        if (!a.seg && a.K >= 128) {
-            // r01 sweeps (profiles/r01e_gemm_sweep_mid.txt): the ping-pong 256x256 form wins as soon as its tiles cover
-            // 3/4 of the CUs; below that the 128x128 form (2 workgroups per CU) does; the lock-step 256-wide forms and a
-            // ping-pong 256x128 variant (wave tile 64x64: 8 fragment reads per 16 MFMAs) never do
-            const int t3 = cdiv(a.M, 256) * cdiv(a.N, 256);
-            if (t3 >= 192 && cu_fill(t3, 1) >= 0.74) tile = (!a.seg && !a.a_rows && a.K >= 160) ? 5 : 3;   // 5: ping-pong form
-        }
-    }
-#define NVL_PP(TILE, ST, PR)                                                                                          \
-    if (tile == TILE && !a.seg && !a.a_rows) {                                                                         \
-        NVL_LDS_ATTR((gemm_bf16_pp_kernel<EPI, OutT, ST, PR>), ST * 32 * 1024);                                        \
-        hipLaunchKernelGGL((gemm_bf16_pp_kernel<EPI, OutT, ST, PR>), dim3(cdiv(a.M, 256) * cdiv(a.N, 256)), dim3(512), \
-                           ST * 32 * 1024, st, a);                                                                     \
-        return;                                                                                                        \
-    }
-    NVL_PP(5, 4, 0)      // the default large-M form: 4-slot ring (5 slots: -3 %, 3 slots: -3 %, r01 sweep)
-#undef NVL_PP
+    GemmArgs as = a;
+    as.splits = 1;
+    // 5: the ping-pong form; else 128x128 tiles (the lock-step 256-wide forms and a ping-pong 256x128 variant with wave tiles of 64x64
+    // never win, profiles/r01e_gemm_sweep_mid.txt)
+    if (tile == 0) tile = pp_wins<EPI, OutT>(as) ? 5 : 1;
+    else if (tile == 5) pp_wins<EPI, OutT>(as);
+    if (tile == 5 && !a.seg && !a.a_rows) { launch_pp<EPI, OutT, 4>(st, as); return; }      // (4-slot ring: 5 slots -3 %, 3 slots -3 %, r01 sweep)
     if (tile == 3) launch_gemm_tile<256, 256, 2, 4, 2, EPI, OutT>(st, a);
     else if (tile == 2) launch_gemm_tile<256, 128, 4, 2, 3, EPI, OutT>(st, a);
     else launch_gemm_tile<128, 128, 2, 2, 2, EPI, OutT>(st, a);

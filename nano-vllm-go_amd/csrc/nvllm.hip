@@ -1509,6 +1509,9 @@ void resid_gemm(nvl_model* m, const void* A, int lda, const void* W, const float
         // (fewer than 64 workgroups even so — GPT-2's 768 columns below 512 rows —: the decode form's 64-row groups stream
         // better, profiles/r03_gpt2_large_decode_batches.txt: B = 128 147.5 K -> 159.0 K, B = 256 224.8 K -> 237.2 K tok/s)
         if (tiles * slices < 64) slices = 1;
+        // ... unless large tiles whose K is cut inside the launch are faster (1024 x 4096 x 14336: 118 us, and no slices for the norm)
+        int parts;
+        if (slices > 1 && M > 256 && pp_cost(M, N, K, 8, m->split_ws != nullptr, parts) < 0.72 * tile128_cost(M, N, K, 8, slices)) slices = 1;
     }
     if (slices > 1) {
         a.sk_part = m->sk_part; a.sk_slices = slices;

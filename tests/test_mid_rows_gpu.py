@@ -88,3 +88,20 @@ def test_mamba_decode_step(gpu, oracle, hidden, heads, hd, state, groups, n):
         for j, s in enumerate(steps):
             want = om.forward_with_cache([s[0]], kv, 1 + j)[-1]
             assert rel_err(got["bf16"][0][j][0], want) <= TOL
+
+
+@pytest.mark.parametrize("parts", [2, 3, 5])
+@pytest.mark.parametrize("m,k,n", [(520, 2048, 1300), (2100, 2112, 2056), (256, 1984, 256 * 9), (1025, 2048, 256 * 53)])     # tiles: 18, 81, 9, 265
+def test_large_tiles_of_the_last_round_in_parts(gpu, parts, m, k, n):
+    """The ping-pong kernel with its last round cut along K, uneven parts, XCDs with one tile less than others or none: exact on integers,
+    twice in a row."""
+    a = (np.arange(m * k).reshape(m, k) % 7).astype(np.float32) - 1.0
+    b = (np.arange(k * n).reshape(k, n) % 5).astype(np.float32) - 2.0
+    old = [(key, gpu.lib().nvl_set_tuning(key, v)) for key, v in ((0, 5), (41, parts))]
+    try:
+        got = [gpu.ops.mat_mul(a, b, precision="bf16") for _ in range(2)]
+    finally:
+        for key, v in old:
+            gpu.lib().nvl_set_tuning(key, v)
+    want = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32)
+    assert np.array_equal(got[0], want) and np.array_equal(got[1], want)
