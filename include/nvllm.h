@@ -561,8 +561,9 @@ int nvl_bench_gemm(int device, int M, int N, int K, int epi, int force_bnt, int 
  * key 19: decode-sized MoE batches run the grouped GEMMs on the four-stage 128x128 instance (1, default) or two stages (0).
  * key 18: largest prefill batch (tokens) whose QKV projection runs as decode-form groups + rope_kv_kernel instead of a
  * fused-epilogue kernel (default 64: never beyond the decode form's own rows).
- * key 38: projections of 65..512 rows (as far as key 11 goes) on their own kernel, K split over workgroups (1, default; 0 never);
- * key 39: the parts of K there (0, default: from the grid); key 40: rows up to which it completes residual projections (default 256).
+ * key 38: projections of up to 512 rows (beyond 64 as far as key 11 goes) on their own kernel, K split over workgroups (1, default,
+ * by cost; 0 never; 2 wherever it applies);
+ * key 39: the parts of K there (0, default: by cost); key 40: rows up to which it completes residual projections (default 256).
  * key 21: hipGraph replay of decode passes (1, default; 0 = every launch eager).  key 22: decode MoE as two dense-masked
  * weight-streaming projections (1, default) or sort + grouped GEMMs (0).  key 23: largest payload (rows of the residual
  * stream) the tensor-parallel P2P all-reduce sends one-shot; above it reduce-scatter + all-gather (default 64).

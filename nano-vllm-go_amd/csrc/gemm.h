@@ -28,6 +28,7 @@
 #pragma once
 #include <stdexcept>
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 #include "common.h"
 
@@ -773,7 +774,7 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_pp_kernel(GemmArgs p) {
 }
 
 // ------------------------------------------------------------------------------------------
-// bf16 kernel for 65 .. 512 rows (large decode batches, short prompts): weights still come from HBM once, but the 64-row groups of the
+// bf16 kernel for up to 512 rows (decode batches, short prompts; mid_wins says where): weights still come from HBM once, but the 64-row groups of the
 // decode form pull every activation row through every CU for 16 weight rows each (FFN-down of Llama-3.2-1B at 96 rows: 128 workgroups x
 // 2 x 1.3 MB, 25 us for 34 MB of weights).  Here a workgroup owns MT x 16 rows by CT x 32 columns, both operands staged through an
 // LDS ring by global_load_lds, so an activation row is fetched once per CT x 32 weight rows and the ring keeps a
@@ -782,8 +783,8 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_pp_kernel(GemmArgs p) {
 // 128-wide K stage, added through LDS at the end.
 // ------------------------------------------------------------------------------------------
 template <int MT, int CT> constexpr int mid_stage_bytes() { return (MT + 2 * CT) * 4096; }
-template <int MT, int CT> constexpr int mid_stages() { return 163328 / mid_stage_bytes<MT, CT>() > 5 ? 5 : 163328 / mid_stage_bytes<MT, CT>(); }
-template <int MT, int CT> constexpr int mid_lds_bytes() { return mid_stages<MT, CT>() * mid_stage_bytes<MT, CT>() + 16; }
+template <int MT, int CT> constexpr int mid_stages() { return 163200 / mid_stage_bytes<MT, CT>() > 5 ? 5 : 163200 / mid_stage_bytes<MT, CT>(); }
+template <int MT, int CT> constexpr int mid_lds_bytes() { return mid_stages<MT, CT>() * mid_stage_bytes<MT, CT>() + 16 + MT * 64; }
 constexpr int MID_MAX_ROWS = 512;
 
 // one pair of rotated quads (EPI_QKV): x1 at column d of the head, x2 at d + hd / 2
@@ -855,19 +856,21 @@ __global__ __launch_bounds__(512, 1) void gemm_mid_bf16_kernel(GemmArgs p) {
     int ct[CT];
 #pragma unroll
     for (int j = 0; j < CT; j++) ct[j] = PAIRS ? CT * wn + j : wn + 2 * j;
-    // (the row tiles this wave finishes, below: the scales of a deferred RMSNorm are fetched beside the first operands)
     constexpr bool QKV = EPI == EPI_QKV, BOTH = TM % 2 == 0 || !(PAIRS || QKV), RSTD = PAIRS || EPI == EPI_STORE;
-    constexpr int F = TM * CT, H = BOTH ? F / 2 : F, NR = (H - 1) / CT + 1 + (H % CT ? 1 : 0);
-    const int i0 = BOTH ? kh * H / CT : 0;
+    constexpr int F = TM * CT, H = BOTH ? F / 2 : F;
     f32x4 acc[F];
 #pragma unroll
     for (int i = 0; i < F; i++) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < NST - 1; s++)
         if (s < n) stage(s, s);
-    float rstd[NR];
-#pragma unroll
-    for (int r = 0; r < NR; r++) rstd[r] = RSTD && p.rs_in && (BOTH || kh == 0) ? deferred_rstd(p, min(m0 + (wm * TM + i0 + r) * 16 + fr, p.M - 1)) : 1.0f;
+    // the rows' scales of a deferred RMSNorm, once per workgroup and beside the first operands (by every wave for the rows it
+    // finishes they were 64 .. 128 KiB of loads: 3 us of a 14 us launch)
+    float* rstd = (float*)(smem + NST * SB + 16);
+    if (RSTD && p.rs_in && wave8 < MT) {
+        const float r = deferred_rstd(p, min(m0 + wave8 * 16 + fr, p.M - 1));
+        if (fg == 0) rstd[wave8 * 16 + fr] = r;
+    }
     int buf = 0;
     for (int t = 0; t < n; t++) {
         // my pieces of stage t landed; the ring's younger stages stay in flight (a cut stage only ever is the youngest)
@@ -924,7 +927,7 @@ __global__ __launch_bounds__(512, 1) void gemm_mid_bf16_kernel(GemmArgs p) {
         const int idx = (BOTH ? kh * H : 0) + e, i = idx / CT, j = idx - i * CT;
         const int m = m0 + (wm * TM + i) * 16 + fr, ctile = PAIRS ? CT * wn + j : wn + 2 * j;
         const int nn = n0 + ctile * 16 + 4 * fg;
-        const float rs = !RSTD ? 1.0f : BOTH && kh ? rstd[(H + e) / CT - H / CT] : rstd[e / CT];
+        const float rs = RSTD && p.rs_in ? rstd[(wm * TM + i) * 16 + fr] : 1.0f;
         if constexpr (QKV) {
             if (CT == 4 && (e & 2)) continue;                        // (pairs are CT / 2 fragments apart)
             epilogue_qkv_pair(p, m, n0 / (32 * CT), 16 * ctile + 4 * fg, mine[e], mine[e + CT / 2]);      // the workgroup's columns are one head
@@ -1746,44 +1749,82 @@ static inline void launch_gemm_grouped(hipStream_t st, const GemmArgs& a, int ma
                        lds, st, a);
 }
 
-// 65 .. MID_MAX_ROWS rows: returns false where gemm_mid_bf16_kernel does not apply
-inline int g_mid = 1;               // nvl_set_tuning key 38: 0 never
-inline int g_mid_splits = 0;        // nvl_set_tuning key 39: parts of K (0: from the grid)
+// What a projection of up to MID_MAX_ROWS rows takes on gemm_mid_bf16_kernel, in microseconds, and into how many parts its K goes (fitted to 8 .. 512
+// rows of 2048 .. 4544-wide models, good to 15 %): a stage of a CU moves at some 56 GB/s, all weights together at 6.6 TB/s; a part
+// more costs the hand-over 0.45 us and every round of workgroups beyond the first its ramp.
+constexpr int MID_MAX_PARTS = 8;
+static inline int mid_row_tiles(int M) { return cdiv(cdiv(M, cdiv(M, 128)), 32) * 2; }      // 16-row tiles of a row group: 2, 4, 6 or 8
+static inline double mid_cost(int M, int N, int K, int mt, int ct, bool can_split, int& parts) {
+    const int tiles = cdiv(N, 32 * ct) * cdiv(M, 16 * mt), stages = cdiv(K, 128);
+    const double stage_us = 0.0178 * 4.0 * (mt + 2 * ct), hbm_us = 2e-6 * N * K / 6.6;
+    double best = 0;
+    parts = 1;
+    for (int c = 1; c <= MID_MAX_PARTS; c++) {
+        if (c > 1 && (!can_split || tiles * c > 256 || stages / c < 2)) break;
+        const double rounds = cdiv(tiles * c, 256), t = std::max(rounds * cdiv(stages, c) * stage_us, hbm_us) + (c > 1 ? 2.5 + 0.45 * c : 0.0) + 2.0 * (rounds - 1);
+        if (c == 1 || t < best) { best = t; parts = c; }
+    }
+    return best + 4.0;
+}
+// ... and on the narrow decode form (M <= 64): every 16-row tile of the activations comes beside the weights, at 11.5 TB/s with all CUs at work.
+// `blocks`: workgroups of one row tile; tile_split: each row tile has its own workgroups (GemmArgs::m_split)
+static inline double narrow_cost(int M, int N, int K, int blocks, int waves, bool tile_split) {
+    const double mb = 2e-6 * N * K, rows = M < 16 ? M / 16.0 : cdiv(M, 16), wgs = tile_split ? blocks * cdiv(M, 16) : blocks;
+    const double rate = 11.5 * std::min(1.0, wgs / 256.0) * (waves >= 2048 ? 1.0 : pow(waves / 2048.0, 0.6)) * (!tile_split && rows > 2 ? 1.25 : 1.0);
+    return std::max(mb / 5.9, mb * (tile_split ? 2.0 * cdiv(M, 16) : 1.0 + rows) / rate) + 2.5;
+}
+inline int g_mid = 1;               // nvl_set_tuning key 38: 0 never, 2 wherever it applies
+inline int g_mid_splits = 0;        // nvl_set_tuning key 39: parts of K (0: from the cost)
 template <int MT, int CT, int EPI, typename OutT>
 static inline void launch_gemm_mid_rows(hipStream_t st, const GemmArgs& a0) {
     GemmArgs a = a0;
     const int nb = cdiv(a.N, 32 * CT), groups = cdiv(a.M, 16 * MT);
-    a.splits = 1;
-    if (a.split_ws) {
-        // four stages and more a part (2048 x 2048 at 96 rows: 15.8 / 12.3 / 10.6 / 11.3 us in 1 / 2 / 4 / 8 parts; 2048 x 8192: 47.7 / 29.3 / 19.6 / 17.8)
-        while (nb * groups * a.splits * 2 <= 256 && (a.K >> 7) / (a.splits * 2) >= 4 && a.splits < 8) a.splits *= 2;
-        if (g_mid_splits) a.splits = std::min(g_mid_splits, std::max(1, a.K >> 7));
-        while (a.splits > 1 && (nb * groups > SPLIT_MAX_TILES || (int64_t)nb * groups * a.splits * MT * CT * 2048 > SPLIT_WS_BYTES)) a.splits--;
-    }
+    mid_cost(a.M, a.N, a.K, MT, CT, a.split_ws != nullptr, a.splits);
+    if (a.split_ws && g_mid_splits) a.splits = std::min(g_mid_splits, std::max(1, a.K >> 7));
+    while (a.splits > 1 && (nb * groups > SPLIT_MAX_TILES || (int64_t)nb * groups * a.splits * MT * CT * 2048 > SPLIT_WS_BYTES)) a.splits--;
     NVL_LDS_ATTR((gemm_mid_bf16_kernel<MT, CT, EPI, OutT>), (mid_lds_bytes<MT, CT>()));
     hipLaunchKernelGGL((gemm_mid_bf16_kernel<MT, CT, EPI, OutT>), dim3(cdiv(nb, 8) * 8 * groups * a.splits), dim3(512), (mid_lds_bytes<MT, CT>()), st, a);
 }
+// does the kernel take this projection, and is it the one to take it?
 template <int EPI, typename OutT>
-static inline bool launch_gemm_mid(hipStream_t st, const GemmArgs& a) {
-    if (!g_mid || a.M <= 64 || a.M > MID_MAX_ROWS || a.M > g_chunk_max_m || a.K % 64 != 0 || a.a_rows || a.seg || a.tile_map || a.sk_part || a.moe_gate || a.c_row0 || g_force_tile) return false;
-    // (GPT-2's 768-wide projections at 96 rows: 12.7 / 12.0 / 11.1 us here, 8.8 / 10.1 / 9.3 in the decode form)
-    if ((EPI != EPI_QKV && a.K < 2048) || (EPI == EPI_RESID && a.rs_in)) return false;
-    const int groups = cdiv(a.M, 128), rows = cdiv(cdiv(a.M, groups), 32) * 2;      // 16-row tiles of a group: 4, 6 or 8
-    if constexpr (EPI == EPI_QKV) {
-        if (a.qkv.hd == 128) {
-            if (cdiv(a.N, 128) * cdiv(a.M, 64) > 512) return false;
-            launch_gemm_mid_rows<4, 4, EPI, OutT>(st, a);      // (a head of 128 columns per workgroup: 64 rows leave room for three stages)
-            return true;
-        }
-        if (a.qkv.hd != 64) return false;
+static inline bool mid_wins(const GemmArgs& a) {
+    if (!g_mid || a.M > MID_MAX_ROWS || a.M > std::max(64, g_chunk_max_m) || a.K % 64 != 0 || a.a_rows || a.seg || a.tile_map || a.sk_part || a.moe_gate || a.c_row0 || g_force_tile ||
+        g_force_ntw || a.rs_half || (EPI == EPI_RESID && a.rs_in)) return false;
+    if (EPI == EPI_QKV && a.qkv.hd == 128) return a.M > 64 && cdiv(a.N, 128) * cdiv(a.M, 64) <= 512;
+    if (EPI == EPI_QKV && a.qkv.hd != 64) return false;
+    if (g_mid == 2) return true;
+    if (a.M <= 64) {
+        // (pairs and wide projections: the decode forms; below some 16 MB of weights, or with few rows of a short K, a launch is all ramp:
+        // 5120 x 2048 at 19 rows 12.0 us there, 13.9 here; 8512 x 2048 at 24 13.1 and 15.6, at 48 19.0 and 17.4)
+        if (EPI == EPI_QKV || epi_glu(EPI) || cdiv(a.N, 64) >= 256 || (int64_t)a.N * a.K < (8 << 20) || (a.M <= 32 && a.K < 4096)) return false;
+        const bool split = EPI == EPI_RESID && a.m_split && a.rs_out;
+        const int blocks = cdiv(a.N, 16);
+        int ks = split ? 8 : 16, mid_parts;                       // (waves of a workgroup: launch_gemm_skinny_ntw)
+        if (!split) while (ks > 1 && blocks * ks > g_narrow_waves) ks >>= 1;
+        // a step in favour of the form that is there: 8 % is half the error of the two costs.  At 24 / 32 / 64 rows, decode form -> here:
+        // 4096 x 14336 43 -> 28.6, 55 -> 29.9, 85.7 -> 32.6 us; 4544 x 18176 at 16 rows 48.7 -> 34.9; 2048 x 8192 stays at 15.3 up to 32 rows, 23.1 -> 18.4 at 64
+        return mid_cost(a.M, a.N, a.K, mid_row_tiles(a.M), 2, a.split_ws != nullptr, mid_parts) < 0.92 * narrow_cost(a.M, a.N, a.K, blocks, blocks * ks * (split ? cdiv(a.M, 16) : 1), split);
     }
+    // (GPT-2's 768-wide projections at 96 rows: 12.7 / 12.0 / 11.1 us here, 8.8 / 10.1 / 9.3 in groups of the decode form)
+    if (EPI != EPI_QKV && a.K < 2048) return false;
     // One row group reads the weights once at any width up to a few rounds of workgroups (a workgroup per CU: each round has its own
     // ramp; LM head at 128 rows 168 us against 152 on the tiles, 28672 x 4096 72 against 74).  Several groups pay while one round holds
     // them (3072 x 2048: 192 rows 12.5 against 17.4 us, 512 rows 18.3 against 29; 16384 x 2048 at 512 rows 68 against 43).
-    const int wgs = cdiv(a.N, 64) * groups;
-    if (wgs > (groups == 1 ? 512 : 256)) return false;
-    if (rows <= 4) launch_gemm_mid_rows<4, 2, EPI, OutT>(st, a);
-    else if (rows <= 6) launch_gemm_mid_rows<6, 2, EPI, OutT>(st, a);
+    return cdiv(a.N, 64) * cdiv(a.M, 128) <= (a.M <= 128 ? 512 : 256);
+}
+template <int EPI, typename OutT>
+static inline bool launch_gemm_mid(hipStream_t st, const GemmArgs& a) {
+    if (!mid_wins<EPI, OutT>(a)) return false;
+    const int mt = mid_row_tiles(a.M);
+    if constexpr (EPI == EPI_QKV) {
+        if (a.qkv.hd == 128) {
+            launch_gemm_mid_rows<4, 4, EPI, OutT>(st, a);      // (a head of 128 columns per workgroup: 64 rows leave room for three stages)
+            return true;
+        }
+    }
+    if (mt <= 2) launch_gemm_mid_rows<2, 2, EPI, OutT>(st, a);
+    else if (mt <= 4) launch_gemm_mid_rows<4, 2, EPI, OutT>(st, a);
+    else if (mt <= 6) launch_gemm_mid_rows<6, 2, EPI, OutT>(st, a);
     else launch_gemm_mid_rows<8, 2, EPI, OutT>(st, a);
     return true;
 }
@@ -1791,8 +1832,8 @@ static inline bool launch_gemm_mid(hipStream_t st, const GemmArgs& a) {
 template <int EPI, typename OutT>
 void launch_gemm_bf16(hipStream_t st, const GemmArgs& a) {
     if (a.tile_map) { launch_gemm_grouped<EPI, OutT>(st, a, a.M); return; }   // a.M carries the m-tile bound
-    if (launch_gemm_skinny_bf16<EPI, OutT>(st, a)) return;
     if (launch_gemm_mid<EPI, OutT>(st, a)) return;
+    if (launch_gemm_skinny_bf16<EPI, OutT>(st, a)) return;
     if constexpr (EPI != EPI_QKV) {
         // 64 < M <= g_chunk_max_m (large decode batches): the tile kernels would launch only N/128 * M/128 workgroups, far
         // too few to stream the weights at HBM rate.  Run the decode form over ceil(M/64) groups of 64 activation rows

@@ -1456,7 +1456,7 @@ static int g_mamba_ssd = 1;    // nvl_set_tuning key 30: chunked (SSD) Mamba2 sc
                                // 2 = chunk after chunk only, never the chunk-parallel three-launch form)
 static int g_decode_seam = 1;  // nvl_set_tuning key 7: decode_seam_kernel in nvl_decode_greedy (0 = separate kernels)
 static int g_defer_norm = 1;   // nvl_set_tuning key 3: deferred RMSNorm between O-proj and FFN-up in decode (0 = off)
-static int g_mid_resid_rows = 256;   // nvl_set_tuning key 40: up to here the 65..512-row kernel completes a residual projection (gemm_mid_bf16_kernel)
+static int g_mid_resid_rows = 256;   // nvl_set_tuning key 40: up to here one launch completes a residual projection of a decode batch or short prompt (gemm_mid_bf16_kernel)
 static int g_sk_slices = 0;    // tuning override (nvl_set_tuning key 1): 0 automatic, 1 = never split
 // consumer side of the deferred RMSNorm: the projection reads xn_raw and scales its accumulators (gemm.h)
 void set_deferred_in(nvl_model* m, GemmArgs& a) {

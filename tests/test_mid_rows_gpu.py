@@ -1,4 +1,4 @@
-"""Projections of 65 .. 512 rows (gemm.h gemm_mid_bf16_kernel: K split over workgroups, split_finish) and the single-launch Mamba-2 decode
+"""Projections of up to 512 rows (gemm.h gemm_mid_bf16_kernel: K split over workgroups, split_finish) and the single-launch Mamba-2 decode
 step (mamba.h mamba_step_kernel), at the sizes where they can go wrong."""
 import numpy as np
 import pytest
@@ -11,24 +11,25 @@ TOL = 1.5e-2
 
 @pytest.mark.parametrize("parts", [0, 1, 2, 5, 8])                 # K split over workgroups; 0: the launcher's choice
 @pytest.mark.parametrize("m,k,n", [(65, 2048, 64), (66, 2112, 200), (96, 2048, 130), (97, 4160, 2048), (128, 2048, 1003), (129, 2048, 256),
-                                   (255, 2176, 320), (257, 2048, 2049), (512, 2048, 192)])
+                                   (255, 2176, 320), (257, 2048, 2049), (512, 2048, 192), (1, 4096, 64), (33, 1984, 2049), (64, 64, 33)])
 def test_matmul_is_exact_on_integers(gpu, parts, m, k, n):
     """Ragged rows, columns and K (a last stage of 64, K parts of unequal length); the sums are exact in fp32 in any order, twice in a
     row (the counters of a split are zero again)."""
     a = (np.arange(m * k).reshape(m, k) % 7).astype(np.float32) - 1.0
     b = (np.arange(k * n).reshape(k, n) % 5).astype(np.float32) - 2.0        # |sums| < 2^24
-    old = gpu.lib().nvl_set_tuning(39, parts)
+    old = [(key, gpu.lib().nvl_set_tuning(key, v)) for key, v in ((39, parts), (38, 2 if m <= 64 else 1))]
     try:
         got = [gpu.ops.mat_mul(a, b, precision="bf16") for _ in range(2)]
     finally:
-        gpu.lib().nvl_set_tuning(39, old)
+        for key, v in old:
+            gpu.lib().nvl_set_tuning(key, v)
     want = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32)
     assert np.array_equal(got[0], want) and np.array_equal(got[1], want)
 
 
 @pytest.mark.parametrize("hd", [64, 128])
-@pytest.mark.parametrize("n", [65, 97, 128, 130])                  # 130: past the deferred norm
-def test_decode_and_prompt_batches(gpu, hd, n):
+@pytest.mark.parametrize("n,mid", [(5, 2), (33, 2), (64, 1), (64, 2), (65, 1), (97, 1), (128, 1), (130, 1)])      # 130: past the deferred norm
+def test_decode_and_prompt_batches(gpu, hd, n, mid):
     """Every epilogue of the kernel in a model: decode batches (deferred norms, gate | up pairs) and short prompts (rotated heads, cache rows)
     against the fp32 mode, and the greedy loop (graph replays) against single steps."""
     cfg = gpu.synth.tiny_config("llama", hidden=2048, num_heads=2048 // hd, num_kv_heads=512 // hd, head_dim=hd, ffn_dim=2048, max_seq_len=64)
@@ -36,6 +37,7 @@ def test_decode_and_prompt_batches(gpu, hd, n):
     r = np.random.default_rng(n)
     prompts = [r.integers(0, cfg["vocab_size"], 1 + i % 3).tolist() for i in range(n)]
     ids, got = list(range(n)), {}
+    old = gpu.lib().nvl_set_tuning(38, mid)
     for precision in ("bf16", "f32"):
         m = gpu.HipTransformerModel(cfg, w, precision=precision, max_seqs=n, max_batch_tokens=512)
         for i in ids:
@@ -55,6 +57,7 @@ def test_decode_and_prompt_batches(gpu, hd, n):
             _, am = m.forward_batch(ids, [[7]] * n, [len(p) for p in prompts], want_logits=False)
             assert np.array_equal(m.decode_greedy(ids, am, 3), np.stack(one))
         m.close()
+    gpu.lib().nvl_set_tuning(38, old)
     assert rel_err(got["bf16"][0], got["f32"][0]) <= TOL and rel_err(got["bf16"][1], got["f32"][1]) <= TOL
 
 
