@@ -973,6 +973,51 @@ __device__ __forceinline__ bf16x8 weight_load(const bf16x8* p) {
     else return __builtin_nontemporal_load(p);
 }
 
+// split_finish for one 16 x 16 tile held by one wave (a lane: four columns of a row): its parts are 1 KiB each, [part][tiles] in sk_part.
+__device__ __forceinline__ bool split_finish_wave(const GemmArgs& p, int tile, int tiles, int part, int parts, f32x4& v) {
+    const int lane = threadIdx.x & 63, voff = lane * 16;
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc((char*)p.sk_part, 0, parts * tiles * 1024, 0x00020000);
+    union { f32x4 v; u32x4 u; } mine; mine.v = v;
+    __builtin_amdgcn_raw_buffer_store_b128(mine.u, rs, voff, __builtin_amdgcn_readfirstlane((part * tiles + tile) * 1024), SPLIT_COHERENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the part has reached memory
+    int before = 0;
+    if (lane == 0) before = __hip_atomic_fetch_add(p.split_cnt + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__builtin_amdgcn_readfirstlane(before) != parts - 1) return false;
+    asm volatile("" ::: "memory");
+    if (lane == 0) __hip_atomic_store(p.split_cnt + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int c0 = 0; c0 < parts; c0 += 4) {
+        union { f32x4 v; u32x4 u; } got[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+            if (c0 + c < parts) got[c].u = __builtin_amdgcn_raw_buffer_load_b128(rs, voff, __builtin_amdgcn_readfirstlane(((c0 + c) * tiles + tile) * 1024), SPLIT_COHERENT);
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+            if (c0 + c < parts) sum += got[c].v;
+    }
+    v = sum;
+    return true;
+}
+// x += alpha * v for four columns of row m, with the operand and the x^2 partials of the deferred norm that follows
+__device__ __forceinline__ void resid_norm_tile(const GemmArgs& p, int m, int n, f32x4 v, const f32x4* x_pre) {
+    const int fg = (threadIdx.x >> 4) & 3;
+    float ss = 0.f;
+    if (m < p.M) {
+        float* x = (float*)p.C + (int64_t)m * p.ldc + n;
+        const f32x4 o = (x_pre ? *x_pre : *(f32x4*)x) + p.alpha * v;
+        *(f32x4*)x = o;
+        act_store4<bf16_t>(p.nrm_xn, m, n, p.N, o * *(const f32x4*)(p.nrm_w + n));
+        ss = o[0] * o[0] + o[1] * o[1] + o[2] * o[2] + o[3] * o[3];
+    }
+    ss += __shfl_xor(ss, 16, 64);
+    if (p.rs_half) {      // (partials per 8 columns)
+        if (m < p.M && (fg & 1) == 0) p.rs_out[(int64_t)m * (p.N >> 3) + (n >> 3)] = ss;
+        return;
+    }
+    ss += __shfl_xor(ss, 32, 64);
+    if (m < p.M && fg == 0) p.rs_out[(int64_t)m * (p.N >> 4) + (n >> 4)] = ss;
+}
+
 // m_passes > 1: block id -> (weight block, 64-row activation group).  Ids that differ by 8 share an XCD and are
 // dispatched back to back: the groups of one weight block stream the same weights at the same time.
 __device__ __forceinline__ void skinny_pass_remap(GemmArgs& p, int& bx) {
@@ -1034,8 +1079,7 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
     int my_steps = q + (part < rr ? 1 : 0);
     const int ks0 = part * q + (part < rr ? part : rr);   // first k-step of this wave
     // MoE decode (its own instantiation): stream only the experts some token of the batch picked.  Up: a workgroup's rows
-    // belong to one expert.  Down: a wave's K range covers up to four experts (one with the K split over workgroups, two
-    // to four in the deferred-norm form, which keeps all of K in one workgroup); blk_live bit b = block b (U k-steps,
+    // belong to one expert.  Down: a wave's K range covers up to four experts (one: launch_gemm_skinny_ntw); blk_live bit b = block b (U k-steps,
     // inside one expert: the launcher checks the divisibility) of this wave's range is to be streamed.
     uint32_t blk_live = 0xffffffffu;
     bool tail_live = true;                 // the ragged tail (fewer than U k-steps; it lies inside the range's last expert)
@@ -1167,6 +1211,14 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
         for (int e = wave; e < NTW * MT; e += NTW * ksplit) {
             const int t = e / MT, i = e - t * MT;
             const int m = 16 * i + fr, n = (nt0 + t) * 16 + 4 * fg;
+            if constexpr (MOE) {
+                if (p.rs_out) {
+                    f32x4 v = ksum(t, i);
+                    const int n16 = p.N >> 4;
+                    if (nt0 + t < n16 && split_finish_wave(p, i * n16 + nt0 + t, n16 * MT, slice, nslices, v)) resid_norm_tile(p, m, n, v, e == wave ? &x_pre : nullptr);
+                    continue;
+                }
+            }
             if (m >= p.M || n >= p.N) continue;
             f32x4 v = ksum(t, i);
             if (p.bias && slice == 0) v += *(const f32x4*)(p.bias + n);    // N % 4 == 0 for residual widths
@@ -1209,12 +1261,16 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
 // ------------------------------------------------------------------------------------------
 // MoE decode routing in ONE launch (moe.go:57-103): router logits of a 16-row activation tile (E <= 64 experts, all of K),
 // softmax, top-k, renormalised weights as the dense gate matrix GemmArgs::moe_gate of the expert projections.  Before:
-// the router as a skinny GEMM launch (4.6 us) + moe_gate_kernel (4.5 us).  grid = 16-row tiles of the batch, 1024
+// the router as a skinny GEMM launch (4.6 us) + moe_gate_kernel (4.5 us).  grid = 16-row tiles of the batch x ROUTE_ROWS of their rows (the
+// logits of a tile are cheap, 96 KiB from L2; the ranking is serial: at 16 rows all of them in one workgroup 8.4 us, eight 7.2, four 7.0; at 6 rows two
+// workgroups lose 0.3), 1024
 // threads: wave w takes expert tile w % ET over K slice w / ET (fragments straight from L2 / HBM, as the skinny kernel),
-// the K slices are summed through LDS in wave order, then wave r routes row r of the tile with a lane per expert.
+// the K slices are summed through LDS in wave order, then wave r routes the workgroup's row r with a lane per expert.
 // p: A (fragment-major operand, possibly the deferred-norm raw form with rs_in), W (router, fragment-major), bias, M, N = E, K.
 // The gate's columns E .. E + n_always - 1 are one (experts every token takes), those up to gate_ld zero.
 // ------------------------------------------------------------------------------------------
+constexpr int ROUTE_ROWS = 8;
+static inline dim3 router_gate_grid(int M) { return dim3(cdiv(M, 16), cdiv(M < 16 ? M : 16, ROUTE_ROWS)); }
 static __global__ __launch_bounds__(1024) void moe_router_gate_kernel(GemmArgs p, int top_k, float* __restrict__ gate, float* __restrict__ logits_out, int ld_logits,
                                                                       int gate_ld, int n_always) {
     __shared__ f32x4 red[16][64];
@@ -1245,10 +1301,12 @@ static __global__ __launch_bounds__(1024) void moe_router_gate_kernel(GemmArgs p
     }
     for (; s < my_steps; s++)
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(wp + (int64_t)s * 512), x_live ? *(const bf16x8*)(xp + (int64_t)s * 512) : zero, acc, 0, 0, 0);
-    // deferred RMSNorm: wave r owns row r of the tile — its x^2 partials, a lane per 16-byte chunk
+    // deferred RMSNorm: wave r owns the workgroup's row r — its x^2 partials, a lane per 16-byte chunk
+    const int row = blockIdx.y * ROUTE_ROWS + wave, m = row0 + row;
+    const bool routes = wave < ROUTE_ROWS && m < p.M;
     float ssq = 0.f;
-    if (p.rs_in && row0 + wave < p.M) {
-        const f32x4* src = (const f32x4*)(p.rs_in + (int64_t)(row0 + wave) * p.rs_tiles);
+    if (p.rs_in && routes) {
+        const f32x4* src = (const f32x4*)(p.rs_in + (int64_t)m * p.rs_tiles);
         f32x4 a4 = f32x4{0.f, 0.f, 0.f, 0.f};
         for (int c = lane; c < (p.rs_tiles >> 2); c += 64) a4 += src[c];
         ssq = (a4[0] + a4[1]) + (a4[2] + a4[3]);
@@ -1264,10 +1322,9 @@ static __global__ __launch_bounds__(1024) void moe_router_gate_kernel(GemmArgs p
         for (int r = 0; r < 4; r++) lg[fr][16 * wave + 4 * fg + r] = v[r];
     }
     __syncthreads();
-    const int m = row0 + wave;
-    if (m >= p.M) return;
+    if (!routes) return;
     const float rstd = p.rs_in ? 1.0f / sqrtf(ssq * p.rs_inv_h + p.rs_eps) : 1.0f;
-    const float v = (lane < E) ? lg[wave][lane] * rstd + (p.bias ? p.bias[lane] : 0.f) : -INFINITY;
+    const float v = (lane < E) ? lg[row][lane] * rstd + (p.bias ? p.bias[lane] : 0.f) : -INFINITY;
     if (logits_out && lane < E) logits_out[(int64_t)m * ld_logits + lane] = v;
     float mx = v;
 #pragma unroll
@@ -1534,20 +1591,6 @@ static inline bool launch_gemm_skinny_ntw(hipStream_t st, const GemmArgs& a) {
         while (ks > 1 && (a.K >> 5) / ks < 4) ks >>= 1;
         if (a.K % 32 != 0) return false;
         if constexpr (EPI == EPI_RESID) {
-            if (a.moe_gate) {     // MoE down as the deferred-norm producer: all experts in one workgroup's K range, 16 waves
-                ks = 16;
-                const int nks = a.K >> 5, spe = a.moe_I >> 5;
-                if (nks % (ks * 4) != 0 || spe % 4 != 0 || nks / ks > 4 * spe || nks / ks / 4 > 32) return false;
-                if (a.rs_half) {
-                    if (a.M > 16) return false;
-                    hipLaunchKernelGGL((gemm_skinny_bf16_kernel<1, NTW, 4, EPI, OutT, false, true, true>), dim3(2 * nblocks, 1), dim3(NTW * ks * 64),
-                                       (size_t)NTW * ks * 64 * 16, st, a);
-                } else {
-                    hipLaunchKernelGGL((gemm_skinny_bf16_kernel<1, NTW, 4, EPI, OutT, false, true>), dim3(nblocks, cdiv(a.M, 16)), dim3(NTW * ks * 64),
-                                       (size_t)NTW * ks * 64 * 16, st, a);
-                }
-                return true;
-            }
             if (a.rs_in) {        // (the output projection of a Mamba-2 step)
                 if (a.rs_half) {
                     if (a.M > 16) return false;

@@ -1459,7 +1459,7 @@ SubOut expert_ffn(nvl_model* m, const LayerRun& r, const MixerW& w, int M, Exper
     if (dense && E <= 64 && c.route_softmax) {
         GemmArgs a = mk(m->xn, m->H, w.router, nullptr, E, w.route_bias, 1.f, M, E, m->H);
         KScope ks(m, KC_OTHER, 2.0 * M * E * m->Hn, KS_MOE_ROUTER, ((double)E * m->Hn + (double)M * m->Hn) * (double)m->wsize + (double)M * E * 4.0);
-        hipLaunchKernelGGL(moe_router_gate_kernel, dim3(cdiv(M, 16)), dim3(1024), 0, m->stream, a, k, m->moe_gate, (float*)nullptr, 0, r.Ep, parts);
+        hipLaunchKernelGGL(moe_router_gate_kernel, router_gate_grid(M), dim3(1024), 0, m->stream, a, k, m->moe_gate, (float*)nullptr, 0, r.Ep, parts);
         NVL_HIP(hipGetLastError());
     } else {
         m->site = KS_MOE_ROUTER;

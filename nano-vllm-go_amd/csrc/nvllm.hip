@@ -1446,10 +1446,8 @@ static int g_moe_dense = 1;    // nvl_set_tuning key 22: decode MoE as two dense
 static int g_moe_deep = 1;     // nvl_set_tuning key 19: four-stage grouped GEMM for decode-sized MoE batches (0 = two stages)
 static int g_moe_bm = 0;       // nvl_set_tuning key 17: prefill MoE grouped GEMMs: 0 = 256-row tiles on the ping-pong kernel, 128 / 256 = the lock-step tile kernels
 static int g_moe_gather = 1;   // nvl_set_tuning key 16: prefill MoE gathers the token rows into expert order before the grouped GEMM (0 = per-lane gather inside it)
-static int g_moe_defer_down = 0;    // nvl_set_tuning key 33: MoE decode: the down projection carries the next norm (deferred RMSNorm producer: all of
-                                    // K in one workgroup, one launch less per layer) instead of K slices + a norm launch.  Off: with 128 workgroups of
-                                    // 16 waves each wave walks 8 blocks (two experts) instead of 4 — Granite-1B B=8 down projection 8.9 -> 14.5 us, more
-                                    // than the norm launch it saves: 6.48 K -> 6.26 K decode tok/s (profiles/r03_moe_decode_experiments.txt)
+static int g_moe_defer_down = 1;    // nvl_set_tuning key 33: MoE decode: the last of the K slices' workgroups completes the residual and carries the next norm
+                                    // (deferred RMSNorm producer, gemm.h split_finish_wave); 0: slices left to a norm launch
 static int g_moe_fused_route = 1;   // nvl_set_tuning key 31: MoE decode routing (router GEMM + softmax / top-k / gate matrix) as one launch (0 = two)
 static int g_moe_small = 1;    // nvl_set_tuning key 8: fused MoE planning launch + combine folded into the next norm (0 = off)
 static int g_mamba_ssd = 1;    // nvl_set_tuning key 30: chunked (SSD) Mamba2 scan on MFMA for prefill-sized bf16 calls (0 = the sequential scan,
@@ -1627,8 +1625,7 @@ bool moe_dense_ok(const nvl_model* m, const LayerW& l, int M) {
 // deferred_norm: m->xn holds xn_raw = bf16(x * w_norm) and m->rs_part the x^2 partials (the O projection carried the FFN
 // norm): the router and the expert-up projection scale their accumulators by rstd[m] instead of reading a normed operand
 // next_norm_w (decode, dense-masked form only): the down projection carries the NEXT norm (the following layer's attention
-// norm / the final norm) as the deferred-RMSNorm producer — all of K in one workgroup per (weight half-tile, row tile), no
-// slices left for a norm launch to sum; returns true when it did (m->xn / m->rs_part then hold that norm's operand).
+// norm / the final norm) as the deferred-RMSNorm producer, no slices left for a norm launch to sum; returns true when it did (m->xn / m->rs_part then hold that norm's operand).
 bool moe(nvl_model* m, const LayerW& l, int M, bool deferred_norm = false, const float* next_norm_w = nullptr) {
     const nvl_model_config& c = m->cfg;
     const int E = c.num_experts, k = c.num_experts_per_tok, I = m->F, H = m->H;
@@ -1644,7 +1641,7 @@ bool moe(nvl_model* m, const LayerW& l, int M, bool deferred_norm = false, const
         if (deferred_norm) set_deferred_in(m, ar);
         if (fused_route) {
             KScope ks(m, KC_GEMM, 2.0 * (double)M * E * H, -1, ((double)E * H + (double)M * H) * (double)m->wsize + (double)M * E * 8.0);
-            hipLaunchKernelGGL(moe_router_gate_kernel, dim3(cdiv(M, 16)), dim3(1024), 0, m->stream, ar, k, m->moe_gate, m->router_logits, 128, E, 0);
+            hipLaunchKernelGGL(moe_router_gate_kernel, router_gate_grid(M), dim3(1024), 0, m->stream, ar, k, m->moe_gate, m->router_logits, 128, E, 0);
             NVL_HIP(hipGetLastError());
         } else {
             gemm(m, EPI_STORE, true, ar);
@@ -1666,22 +1663,15 @@ bool moe(nvl_model* m, const LayerW& l, int M, bool deferred_norm = false, const
         if (deferred_norm) set_deferred_in(m, a);
         m->site = KS_MOE_UP; m->site_bytes = (e_touch * 2 * I * H + (double)M * H + e_touch * M * I) * (double)m->wsize;
         gemm(m, EPI_SWIGLU, false, a, 2.0 * pairs * 2 * I * H);
-        const int nks = (E * I) >> 5, spe = I >> 5;
-        if (next_norm_w && g_moe_defer_down && nks % 64 == 0 && spe % 4 == 0 && nks / 16 <= 4 * spe && nks / 64 <= 32) {
-            // (the launcher's conditions: 16 waves, whole blocks of 4 k-steps inside one expert, <= 4 experts per wave)
-            GemmArgs d = mk(m->moe_hall, E * I, l.moe_out_cat, m->x, H, nullptr, m->resid_alpha, M, H, E * I);
-            d.moe_gate = m->moe_gate; d.moe_E = E; d.moe_I = I;
-            d.nrm_w = next_norm_w; d.nrm_xn = (bf16_t*)m->xn; d.rs_out = m->rs_part; d.m_split = 1;
-            d.rs_half = defer_half(m, M) ? 1 : 0;
-            m->site = KS_MOE_DOWN; m->site_bytes = (e_touch * H * I + e_touch * M * I) * (double)m->wsize + (double)M * H * 10.0;
-            gemm(m, EPI_RESID, true, d, 2.0 * pairs * H * I);
-            return true;
-        }
-        GemmArgs d = mk(m->moe_hall, E * I, l.moe_out_cat, m->x, H, nullptr, 1.f, M, H, E * I);
+        GemmArgs d = mk(m->moe_hall, E * I, l.moe_out_cat, m->x, H, nullptr, m->resid_alpha, M, H, E * I);
         const int nsl = moe_down_slices(E);
         d.moe_gate = m->moe_gate; d.moe_E = E; d.moe_I = I; d.sk_part = m->moe_part; d.sk_slices = nsl;
+        // (a counter per 16 x 16 tile)
+        const bool carry = next_norm_w && g_moe_defer_down && nsl > 1 && m->split_cnt && H % 16 == 0 && (H / 16) * (M <= 16 ? 1 : M <= 32 ? 2 : 4) <= SPLIT_MAX_TILES;
+        if (carry) { d.split_cnt = m->split_cnt; d.nrm_w = next_norm_w; d.nrm_xn = (bf16_t*)m->xn; d.rs_out = m->rs_part; d.rs_half = defer_half(m, M) ? 1 : 0; }
         m->site = KS_MOE_DOWN; m->site_bytes = (e_touch * H * I + e_touch * M * I) * (double)m->wsize + (double)nsl * M * H * 4.0;
         gemm(m, EPI_RESID, true, d, 2.0 * pairs * H * I);
+        if (carry) return true;
         m->pending_part = m->moe_part; m->pending_slices = nsl; m->pending_rows = M; m->pending_alpha = m->resid_alpha;
         return false;
     }
@@ -1818,8 +1808,7 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
     const bool defer_ok = g_defer_norm && !m->f32 && (M <= 64 || (M <= DEFER_MAX_M && big_decode && g_defer_norm == 1 && !tp_on)) && !c.use_moe && (!tp_on || tp_defer) && !m->keep_hidden &&
                           c.block_style == NVL_BLOCK_SEQUENTIAL && c.norm_type == NVL_NORM_RMS &&
                           c.activation_type == NVL_ACT_SWIGLU && H % 256 == 0 && m->rs_part && (m->n_mamba == 0 || M <= 64);
-    // MoE layers (decode form): only the O projection carries a norm (the FFN norm); the expert-down projection leaves
-    // K-slice partials that the next attention norm sums
+    // MoE layers (decode form): the O projection carries the FFN norm, the experts' down projection the next attention norm
     const bool defer_moe_ok = g_defer_norm && c.use_moe && M <= 64 && m->tp == 1 && !m->tp_force && c.block_style == NVL_BLOCK_SEQUENTIAL &&
                               c.norm_type == NVL_NORM_RMS && H % 256 == 0 && m->rs_part && m->n_mamba == 0;
     const bool all_rows = (flags & NVL_FWD_ALL_LOGITS) != 0;

@@ -108,3 +108,37 @@ def test_large_tiles_of_the_last_round_in_parts(gpu, parts, m, k, n):
             gpu.lib().nvl_set_tuning(key, v)
     want = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32)
     assert np.array_equal(got[0], want) and np.array_equal(got[1], want)
+
+
+@pytest.mark.parametrize("n", [1, 16, 17, 40, 64])
+def test_moe_down_completes_its_slices(gpu, n):
+    """The experts' down projection of a decode batch: the last of a tile's K slices adds them up and carries the next norm (gemm.h
+    split_finish_wave), against slices left to a norm launch; graph replays against single steps (every counter back at zero)."""
+    import torch
+    from bench import gen_weights_on_device
+    cfg = dict(gpu.synth.FULL_CONFIGS["granite-3.0-1b-a400m"], num_layers=2, vocab_size=1000)
+    m = gpu.HipTransformerModel(cfg, None, precision="bf16", max_seqs=n, max_batch_tokens=256)
+    gen_weights_on_device(gpu, cfg, m, torch, torch.device("cuda", 0), keep_host=False)
+    m.finalize()
+    ids, prompts, got = list(range(n)), [[3 + i % 900, 5] for i in range(n)], {}
+
+    def prompt():
+        for i in ids:
+            m.seq_reset(i)
+        m.forward_batch(ids, prompts, [0] * n, want_logits=False)
+
+    for form in (0, 1):
+        old = gpu.lib().nvl_set_tuning(33, form)
+        prompt()
+        got[form], am = m.forward_batch(ids, [[7]] * n, [2] * n)
+        one = []
+        for j in range(4):
+            _, am = m.forward_batch(ids, [[int(t)] for t in am], [3 + j] * n, want_logits=False)
+            one.append(am)
+        prompt()
+        _, am = m.forward_batch(ids, [[7]] * n, [2] * n, want_logits=False)
+        assert np.array_equal(m.decode_greedy(ids, am, 4), np.stack(one)), form
+        gpu.lib().nvl_set_tuning(33, old)
+    m.close()
+    # the norm's factor multiplies the bf16 operand in one form, the fp32 products in the other: one bf16 rounding (2^-9) a layer
+    assert rel_err(got[1], got[0]) <= 2e-2
