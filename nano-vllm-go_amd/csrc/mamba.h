@@ -78,6 +78,58 @@ __global__ __launch_bounds__(256) void mamba_conv_kernel(MambaArgs p) {
     }
 }
 
+// The same for four taps on 16-byte rows: a thread convolves four channels over MAMBA_CONV_RUN tokens, each row fetched once per run (a
+// workgroup per token re-read the three rows before it from another XCD's memory: 2326 x 4352 took 81 us, 25 here).  The last
+// column of workgroups has the dt values.
+constexpr int MAMBA_CONV_RUN = 8;
+static inline bool mamba_conv_run_ok(const MambaArgs& p) { return p.K == 4 && p.P % 4 == 0 && p.EH % 4 == 0 && p.conv_dim % 4 == 0 && p.tail_slot_stride % 4 == 0; }
+__global__ __launch_bounds__(256) void mamba_conv_run_kernel(MambaArgs p, int tokens) {
+    constexpr int T = MAMBA_CONV_RUN;
+    const int t0 = blockIdx.x * T, n = min(T, tokens - t0);
+    if (blockIdx.y == gridDim.y - 1) {
+        for (int i = threadIdx.x; i < n * p.nh; i += 256) {
+            const int h = i % p.nh;
+            const int64_t t = t0 + i / p.nh;
+            float v = p.proj[t * p.P + p.EH + p.conv_dim + h];
+            if (p.dt_bias) v += p.dt_bias[h];
+            p.delta[t * p.nh + h] = softplus_ref(v);
+        }
+        return;
+    }
+    const int c = (blockIdx.y * 256 + threadIdx.x) * 4;
+    if (c >= p.conv_dim) return;
+    const float* col = p.proj + p.EH + c;
+    f32x4 x[T + 3], w[4];
+#pragma unroll
+    for (int i = 0; i < T + 3; i++) {
+        const int t = t0 + i - 3;
+        x[i] = t >= 0 && t < tokens ? *(const f32x4*)(col + (int64_t)t * p.P) : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) w[r] = *(const f32x4*)(p.conv_w + (int64_t)(c + r) * 4);
+    const f32x4 b = p.conv_b ? *(const f32x4*)(p.conv_b + c) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < T; i++) {
+        if (i >= n) break;
+        const int t = t0 + i, seq = p.tok_seq[t], j = p.tok_pos[t] - p.seq_pos[seq];
+        f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int back = 3 - k;
+            f32x4 v;
+            if (back <= j) v = x[i + k];
+            else if (p.chain == 2) v = *(const f32x4*)(p.tail + (int64_t)p.seq_slot[seq] * p.tail_slot_stride + (int64_t)(3 - (back - j)) * p.conv_dim + c);
+            else continue;
+#pragma unroll
+            for (int r = 0; r < 4; r++) sum[r] = fmaf(v[r], w[r][k], sum[r]);
+        }
+        if (p.conv_b) sum += b;
+#pragma unroll
+        for (int r = 0; r < 4; r++) sum[r] = silu_ref(sum[r]);
+        *(f32x4*)(p.xbc + (int64_t)t * p.conv_dim + c) = sum;
+    }
+}
+
 // grid (sequences), 256 threads over channels: after the convolution of a chunk of a chained prefill (chain >= 1), keep the
 // raw xBC rows of the sequence's last K-1 tokens for the next chunk (a chunk shorter than K-1 keeps the newest old rows).
 __global__ __launch_bounds__(256) void mamba_tail_kernel(MambaArgs p) {
@@ -456,6 +508,62 @@ __global__ __launch_bounds__(256) void mamba_gate_norm_kernel(MambaArgs p, ActT*
         if (p.norm_w) v *= *(const f32x4*)(p.norm_w + c);
         act_store4<ActT>(out, t, c, p.EH, v);
     }
+}
+
+// Prefill-sized bf16 batches, EH <= 4096: a wave holds a row in registers (y is read once and not written back), eight rows a workgroup, so
+// that the operand leaves in whole 128-byte lines (row by row each lane's 8 bytes were a line of their own: 2326 x 4096 48 us, 34
+// here).  Below some 128 rows too few workgroups.
+constexpr int MAMBA_GATE_TILE_ROWS = 128;
+static inline constexpr int mamba_gate_tile_lds_bytes(int EH) { return 8 * (EH + 8) * 2; }
+static __global__ __launch_bounds__(512) void mamba_gate_norm_tile_kernel(MambaArgs p, bf16_t* __restrict__ out, int tokens) {
+    constexpr int CH = 16;
+    extern __shared__ __attribute__((aligned(16))) char smem_g[];
+    bf16_t* tile = (bf16_t*)smem_g;                       // [8][EH + 8]
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, LT = p.EH + 8;
+    const int64_t t = (int64_t)blockIdx.x * 8 + wave;
+    if (t < tokens) {
+        const float *gate = p.proj + t * p.P, *yr = p.y + t * p.EH;
+        f32x4 v[CH];
+        float ss = 0.f;
+#pragma unroll
+        for (int c0 = 0; c0 < CH; c0 += 8) {
+            f32x4 g[8];
+#pragma unroll
+            for (int c = 0; c < 8; c++) {
+                const int j = (lane + (c0 + c) * 64) * 4;
+                const bool in = j < p.EH;
+                v[c0 + c] = in ? *(const f32x4*)(yr + j) : f32x4{0.f, 0.f, 0.f, 0.f};
+                g[c] = in ? *(const f32x4*)(gate + j) : f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+#pragma unroll
+            for (int c = 0; c < 8; c++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const float a = v[c0 + c][r] * silu_ref(g[c][r]);
+                    v[c0 + c][r] = a;
+                    ss = fmaf(a, a, ss);
+                }
+        }
+        const float rms = 1.0f / sqrtf(wave_sum(ss) / (float)p.EH + 1e-5f);
+#pragma unroll
+        for (int c = 0; c < CH; c++) {
+            const int j = (lane + c * 64) * 4;
+            if (j >= p.EH) continue;
+            f32x4 a = v[c] * rms;
+            if (p.norm_w) a *= *(const f32x4*)(p.norm_w + j);
+            bf16x4 o;
+#pragma unroll
+            for (int r = 0; r < 4; r++) o[r] = (bf16_t)a[r];
+            *(bf16x4*)(tile + wave * LT + j) = o;
+        }
+    }
+    __syncthreads();
+    // 32 columns of eight rows: lane (row, 8 columns) of half an operand block, two blocks a wave
+    const int nkb = p.EH >> 5, row = lane & 7, q = (lane >> 3) & 3;
+    const int64_t r0 = (int64_t)blockIdx.x * 8;
+    if (r0 + row < tokens)
+        for (int kb = 2 * wave + (lane >> 5); kb < nkb; kb += 16)
+            *(bf16x8*)(out + fm_index(r0 + row, kb * 32 + 8 * q, p.EH)) = *(const bf16x8*)(tile + row * LT + kb * 32 + 8 * q);
 }
 
 }  // namespace nvl

@@ -1852,7 +1852,9 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
             } else {
                 {
                     KScope ks(m, KC_OTHER, 0, KS_MAMBA_CONV, (double)M * (m->mP + m->mConv + m->m_nh) * 4.0);
-                    hipLaunchKernelGGL(mamba_conv_kernel, dim3(M), dim3(256), 0, m->stream, a);
+                    if (mamba_conv_run_ok(a))
+                        hipLaunchKernelGGL(mamba_conv_run_kernel, dim3(cdiv(M, MAMBA_CONV_RUN), cdiv(a.conv_dim, 1024) + 1), dim3(256), 0, m->stream, a, M);
+                    else hipLaunchKernelGGL(mamba_conv_kernel, dim3(M), dim3(256), 0, m->stream, a);
                     if (a.chain) hipLaunchKernelGGL(mamba_tail_kernel, dim3(n_seqs), dim3(256), 0, m->stream, a);
                     NVL_HIP(hipGetLastError());
                 }
@@ -1912,7 +1914,11 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
                 }
                 {
                     KScope ks(m, KC_OTHER, 0, KS_MAMBA_GATE, (double)M * m->mEH * (8.0 + (double)m->wsize));
-                    if (m->f32) hipLaunchKernelGGL((mamba_gate_norm_kernel<float>), dim3(M), dim3(256), 0, m->stream, a, (float*)m->myn);
+                    if (!m->f32 && M >= MAMBA_GATE_TILE_ROWS && m->mP % 4 == 0 && m->mEH % 32 == 0 && m->mEH <= 4096) {
+                        const int lds = mamba_gate_tile_lds_bytes(m->mEH);
+                        NVL_LDS_ATTR((mamba_gate_norm_tile_kernel), mamba_gate_tile_lds_bytes(4096));
+                        hipLaunchKernelGGL(mamba_gate_norm_tile_kernel, dim3(cdiv(M, 8)), dim3(512), lds, m->stream, a, (bf16_t*)m->myn, M);
+                    } else if (m->f32) hipLaunchKernelGGL((mamba_gate_norm_kernel<float>), dim3(M), dim3(256), 0, m->stream, a, (float*)m->myn);
                     else hipLaunchKernelGGL((mamba_gate_norm_kernel<bf16_t>), dim3(M), dim3(256), 0, m->stream, a, (bf16_t*)m->myn);
                     NVL_HIP(hipGetLastError());
                 }

@@ -142,3 +142,28 @@ def test_moe_down_completes_its_slices(gpu, n):
     m.close()
     # the norm's factor multiplies the bf16 operand in one form, the fp32 products in the other: one bf16 rounding (2^-9) a layer
     assert rel_err(got[1], got[0]) <= 2e-2
+
+
+@pytest.mark.parametrize("heads,hd,groups", [(16, 64, 2), (8, 32, 1), (10, 64, 1)])      # 10 heads: rows that are no multiple of 16 bytes
+@pytest.mark.parametrize("lens", [[1, 2, 3, 4, 117], [128], [5, 7, 9, 130, 1, 8, 23]])
+def test_mamba_prompts(gpu, heads, hd, groups, lens):
+    """The convolution over runs of tokens (sequences that begin anywhere in a run) and the gated norm of eight rows: a batch against each
+    prompt alone in the fp32 mode (the same sums), and the bf16 mode against it."""
+    cfg = gpu.synth.tiny_config("granite_hybrid", hidden=heads * hd // 2, num_heads=heads * hd // 128, num_kv_heads=1, mamba_num_heads=heads, mamba_head_dim=hd, mamba_state_size=32,
+                                mamba_n_groups=groups, max_seq_len=256)
+    w = gpu.synth.make_weights(cfg, seed=29, scale=0.05)
+    r = np.random.default_rng(len(lens))
+    prompts = [r.integers(0, cfg["vocab_size"], n).tolist() for n in lens]
+    ids, got = list(range(len(lens))), {}
+    for precision in ("bf16", "f32"):
+        m = gpu.HipTransformerModel(cfg, w, precision=precision, max_seqs=len(lens), max_batch_tokens=256)
+        for i in ids:
+            m.seq_reset(i)
+        got[precision] = m.forward_batch(ids, prompts, [0] * len(ids))[0]
+        if precision == "f32":
+            for i in ids:
+                m.seq_reset(i)
+                alone = m.forward_batch([i], [prompts[i]], [0])[0]
+                assert rel_err(alone[0], got["f32"][i]) <= 1e-5, lens[i]
+        m.close()
+    assert rel_err(got["bf16"], got["f32"]) <= TOL
