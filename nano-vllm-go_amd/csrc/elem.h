@@ -118,12 +118,16 @@ struct PendingResid {
 // normalises one row held in registers (same arithmetic as norm_kernel) into LDS; the workgroup then writes the tile's
 // 1-KiB operand blocks with full-line stores (norm_kernel's lanes each write 8 bytes of a block: 16-byte fragments at a
 // 256-byte stride).  H <= 64 * 4 * MAXCH (instances for 8 and 16 chunks per lane: H <= 2048 / 4096).
+// bf16 row pitch of such a tile in LDS: 16 bytes beyond a multiple of 64, or the 16 rows of a fragment read would share their banks
+__host__ __device__ __forceinline__ int tile16_pitch(int H) { return H + 8; }
 template <int MAXCH, bool PENDING = false>
 __global__ __launch_bounds__(1024) void norm_tile16_kernel(float* __restrict__ x, const int32_t* __restrict__ rows_idx,
                                                            const float* __restrict__ w, const float* __restrict__ b,
-                                                           float eps, bf16_t* __restrict__ y, int rows, int H, PendingResid pr) {
+                                                           float eps, bf16_t* __restrict__ y, int rows, int H, PendingResid pr,
+                                                           bf16_t* __restrict__ y_rows) {      // not NULL: the result a second time, row-major
     extern __shared__ __attribute__((aligned(16))) char smem_n[];
-    bf16_t* tile = (bf16_t*)smem_n;                       // [16][H]
+    bf16_t* tile = (bf16_t*)smem_n;                       // [16][LT]
+    const int LT = tile16_pitch(H);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r = blockIdx.x * 16 + wave;
     const int H4 = H >> 2;
@@ -197,7 +201,8 @@ __global__ __launch_bounds__(1024) void norm_tile16_kernel(float* __restrict__ x
 #pragma unroll
                     for (int k = 0; k < 4; k++) o[k] = (bf16_t)(((v[c][k] - mean) / inv) * ww[k] + bb[k]);
                 }
-                *(bf16x4*)(tile + wave * H + j * 4) = o;
+                *(bf16x4*)(tile + wave * LT + j * 4) = o;
+                if (y_rows) *(bf16x4*)(y_rows + (int64_t)r * H + j * 4) = o;
             }
         }
     }
@@ -207,7 +212,7 @@ __global__ __launch_bounds__(1024) void norm_tile16_kernel(float* __restrict__ x
     const int lr = lane & 15, lc = lane >> 4;
     if (blockIdx.x * 16 + lr < rows)
         for (int kb = wave; kb < nkb; kb += 16) {
-            const bf16x8 f = *(const bf16x8*)(tile + lr * H + kb * 32 + lc * 8);
+            const bf16x8 f = *(const bf16x8*)(tile + lr * LT + kb * 32 + lc * 8);
             *(bf16x8*)(y + (((int64_t)blockIdx.x * nkb + kb) * 64 + lane) * 8) = f;
         }
 }
@@ -468,7 +473,8 @@ __global__ __launch_bounds__(256) void sandwich_row_kernel(SandwichArgs p, ActT*
 template <int MAXCH, bool EXT = false>
 __global__ __launch_bounds__(1024) void sandwich_tile16_kernel(SandwichArgs p, bf16_t* __restrict__ xn) {
     extern __shared__ __attribute__((aligned(16))) char smem_n[];
-    bf16_t* tile = (bf16_t*)smem_n;                       // [16][H]
+    bf16_t* tile = (bf16_t*)smem_n;                       // [16][LT]
+    const int LT = tile16_pitch(p.H);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r = blockIdx.x * 16 + wave, H4 = p.H >> 2;
     if (r < p.rows) {
@@ -540,7 +546,7 @@ __global__ __launch_bounds__(1024) void sandwich_tile16_kernel(SandwichArgs p, b
                 bf16x4 o;
 #pragma unroll
                 for (int k = 0; k < 4; k++) o[k] = (bf16_t)x[c][k];
-                if (j < H4) *(bf16x4*)(tile + wave * p.H + j * 4) = o;
+                if (j < H4) *(bf16x4*)(tile + wave * LT + j * 4) = o;
             }
         }
         if (EXT && p.w_next && p.b_next) {
@@ -557,7 +563,7 @@ __global__ __launch_bounds__(1024) void sandwich_tile16_kernel(SandwichArgs p, b
                     bf16x4 o;
 #pragma unroll
                     for (int k = 0; k < 4; k++) o[k] = (bf16_t)(((x[c][k] - mean) / sd) * w[k] + b[k]);
-                    *(bf16x4*)(tile + wave * p.H + j * 4) = o;
+                    *(bf16x4*)(tile + wave * LT + j * 4) = o;
                 }
             }
         } else if (p.w_next) {
@@ -573,7 +579,7 @@ __global__ __launch_bounds__(1024) void sandwich_tile16_kernel(SandwichArgs p, b
                     bf16x4 o;
 #pragma unroll
                     for (int k = 0; k < 4; k++) o[k] = (bf16_t)((x[c][k] / rms) * w[k]);
-                    *(bf16x4*)(tile + wave * p.H + j * 4) = o;
+                    *(bf16x4*)(tile + wave * LT + j * 4) = o;
                 }
             }
         }
@@ -583,7 +589,7 @@ __global__ __launch_bounds__(1024) void sandwich_tile16_kernel(SandwichArgs p, b
     const int nkb = p.H >> 5, lr = lane & 15, lc = lane >> 4;
     if (blockIdx.x * 16 + lr < p.rows)
         for (int kb = wave; kb < nkb; kb += 16)
-            *(bf16x8*)(xn + (((int64_t)blockIdx.x * nkb + kb) * 64 + lane) * 8) = *(const bf16x8*)(tile + lr * p.H + kb * 32 + lc * 8);
+            *(bf16x8*)(xn + (((int64_t)blockIdx.x * nkb + kb) * 64 + lane) * 8) = *(const bf16x8*)(tile + lr * LT + kb * 32 + lc * 8);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1204,19 +1210,27 @@ __global__ __launch_bounds__(256) void moe_route_grouped_kernel(GroupRouteArgs p
 
 // out[t] (+)= resid_mult * sum_rank w[t][rank] * eo[slot_of(t,rank)]   in rank order
 // (moe.go:117-119 accumulates in expert-rank order; generic_model.go:383-389 adds the residual)
-__global__ void moe_combine_kernel(const float* __restrict__ eo, const int32_t* __restrict__ slot_of,
+// One workgroup per token, 16 bytes a lane, the rows of eight ranks on their way together (6867 tokens x 8 x 1024: one column a lane
+// and one rank after the other moved 281 MB at 2.7 TB/s, 102 us; now 45).  H % 4 == 0.
+__global__ __launch_bounds__(256) void moe_combine_kernel(const float* __restrict__ eo, const int32_t* __restrict__ slot_of,
                                    const float* __restrict__ w, int top_k, float resid_mult,
                                    float* __restrict__ x, int H, int accumulate_into_x) {
-    const int t = blockIdx.x;
-    for (int j = threadIdx.x; j < H; j += blockDim.x) {
-        float acc = 0.f;
-        for (int k = 0; k < top_k; k++) {
-            const int sl = slot_of[(int64_t)t * top_k + k];
-            acc += w[(int64_t)t * top_k + k] * eo[(int64_t)sl * H + j];
+    const int64_t t = blockIdx.x;
+    const int32_t* slots = slot_of + t * top_k;
+    const float* wt = w + t * top_k;
+    for (int j = threadIdx.x * 4; j < H; j += 1024) {
+        float* xp = x + t * H + j;
+        f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f}, old = acc;
+        if (accumulate_into_x) old = *(const f32x4*)xp;
+        for (int k0 = 0; k0 < top_k; k0 += 8) {
+            f32x4 e[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) if (k0 + k < top_k) e[k] = *(const f32x4*)(eo + (int64_t)slots[k0 + k] * H + j);
+#pragma unroll
+            for (int k = 0; k < 8; k++) if (k0 + k < top_k) acc += wt[k0 + k] * e[k];
         }
-        float* xp = x + (int64_t)t * H + j;
-        if (accumulate_into_x) *xp = *xp + (resid_mult != 0.f ? resid_mult * acc : acc);
-        else *xp = acc;
+        if (accumulate_into_x) acc = old + (resid_mult != 0.f ? resid_mult * acc : acc);
+        *(f32x4*)xp = acc;
     }
 }
 
@@ -1242,8 +1256,10 @@ __global__ __launch_bounds__(256) void moe_hist_kernel(const int32_t* __restrict
     __syncthreads();
     if (lc[threadIdx.x]) atomicAdd(&counts[threadIdx.x], lc[threadIdx.x]);
 }
-// prefill: rows of the fragment-major activation matrix copied into expert order (dst row i = src row perm[i]), one
-// workgroup per 16 destination rows; a wave moves whole 1-KiB operand blocks (coalesced stores, 16-byte gathers)
+// prefill: rows of the activation matrix copied into expert order (dst row i = src row perm[i], fragment-major), one workgroup per 16
+// destination rows; a wave moves two 1-KiB operand blocks at a time: whole lines of a row-major source.  From a fragment-major source
+// (ROWS false) every 16 bytes are a line of their own: 54936 x 1024 61 us, from rows 34.
+template <bool ROWS>
 __global__ __launch_bounds__(256) void moe_gather_fm_kernel(const bf16_t* __restrict__ src, const int32_t* __restrict__ perm,
                                                             bf16_t* __restrict__ dst, int n_rows, int K) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1251,10 +1267,14 @@ __global__ __launch_bounds__(256) void moe_gather_fm_kernel(const bf16_t* __rest
     const int nks = K >> 5;
     if (r >= n_rows) return;                       // rows past the end of the last tile are never stored by the GEMM
     const int tok = perm[r];
-    const bf16_t* s = src + ((int64_t)(tok >> 4) * nks * 64 + (tok & 15) + 16 * fg) * 8;
+    const bf16_t* s = ROWS ? src + (int64_t)tok * K + fg * 8 : src + ((int64_t)(tok >> 4) * nks * 64 + (tok & 15) + 16 * fg) * 8;
     bf16_t* d = dst + ((int64_t)blockIdx.x * nks * 64 + lane) * 8;
-    for (int ks = wave; ks < nks; ks += 4)
-        *(bf16x8*)(d + (int64_t)ks * 512) = *(const bf16x8*)(s + (int64_t)ks * 512);
+    constexpr int STEP = ROWS ? 32 : 512;
+    for (int ks = 2 * wave; ks < nks; ks += 8) {   // (K % 64 == 0)
+        const bf16x8 x = *(const bf16x8*)(s + (int64_t)ks * STEP), y = *(const bf16x8*)(s + (int64_t)(ks + 1) * STEP);
+        *(bf16x8*)(d + (int64_t)ks * 512) = x;
+        *(bf16x8*)(d + (int64_t)(ks + 1) * 512) = y;
+    }
 }
 __global__ __launch_bounds__(64) void moe_scan_kernel(const int32_t* __restrict__ counts, int E, int BM,
                                                       int32_t* __restrict__ seg_start, int32_t* __restrict__ cursor,

@@ -1271,8 +1271,11 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
 // ------------------------------------------------------------------------------------------
 constexpr int ROUTE_ROWS = 8;
 static inline dim3 router_gate_grid(int M) { return dim3(cdiv(M, 16), cdiv(M < 16 ? M : 16, ROUTE_ROWS)); }
-static __global__ __launch_bounds__(1024) void moe_router_gate_kernel(GemmArgs p, int top_k, float* __restrict__ gate, float* __restrict__ logits_out, int ld_logits,
+// prefill: ids / weights [row][top_k] in rank order instead of the gate matrix, all 16 rows of a tile in a workgroup (enough workgroups without)
+struct RouteOut { float* gate; int32_t* ids; float* w; };
+static __global__ __launch_bounds__(1024) void moe_router_gate_kernel(GemmArgs p, int top_k, RouteOut out, float* __restrict__ logits_out, int ld_logits,
                                                                       int gate_ld, int n_always) {
+    float* gate = out.gate;
     __shared__ f32x4 red[16][64];
     __shared__ float lg[16][64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1302,8 +1305,8 @@ static __global__ __launch_bounds__(1024) void moe_router_gate_kernel(GemmArgs p
     for (; s < my_steps; s++)
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(wp + (int64_t)s * 512), x_live ? *(const bf16x8*)(xp + (int64_t)s * 512) : zero, acc, 0, 0, 0);
     // deferred RMSNorm: wave r owns the workgroup's row r — its x^2 partials, a lane per 16-byte chunk
-    const int row = blockIdx.y * ROUTE_ROWS + wave, m = row0 + row;
-    const bool routes = wave < ROUTE_ROWS && m < p.M;
+    const int rows = out.ids ? 16 : ROUTE_ROWS, row = blockIdx.y * rows + wave, m = row0 + row;
+    const bool routes = wave < rows && m < p.M;
     float ssq = 0.f;
     if (p.rs_in && routes) {
         const f32x4* src = (const f32x4*)(p.rs_in + (int64_t)m * p.rs_tiles);
@@ -1345,6 +1348,10 @@ static __global__ __launch_bounds__(1024) void moe_router_gate_kernel(GemmArgs p
     for (int k = 0; k < top_k; k++) {               // moe.go:89-92: fp32 sum in rank order
         const int src = __ffsll((unsigned long long)__ballot(rank == k)) - 1;
         wsum += __builtin_bit_cast(float, __builtin_amdgcn_readlane(pbits, src));
+    }
+    if (out.ids) {
+        if (lane < E && rank < top_k) { out.ids[(int64_t)m * top_k + rank] = lane; out.w[(int64_t)m * top_k + rank] = prob / wsum; }
+        return;
     }
     if (lane < E) gate[(int64_t)m * gate_ld + lane] = rank < top_k ? prob / wsum : 0.f;      // moe.go:103
     for (int e = E + lane; e < gate_ld; e += 64) gate[(int64_t)m * gate_ld + e] = e < E + n_always ? 1.0f : 0.f;

@@ -902,7 +902,7 @@ void sandwich(nvl_model* m, SubOut y, const float* w_post, NextNorm next, void* 
     if (sh.mu) { a.shift = sh.mu; a.before = sh.state; a.before_stride = m->rec_slot_stride; a.seq_slot = sh.md->seq_slot; a.seq_pos = sh.md->seq_pos; }
     const bool ext = (y.y && !w_post) || next.b || a.sum_scale != 0.f || sh.mu;
     if (!m->f32 && rows > 512 && !sh.mu && m->H <= 4096 && y.slices <= 1) {
-        const size_t lds = (size_t)16 * m->H * 2;
+        const size_t lds = (size_t)16 * tile16_pitch(m->H) * 2;
 #define NVL_SW16E(CH, EXT)                                                                                                  \
         do {                                                                                                                \
             NVL_LDS_ATTR((sandwich_tile16_kernel<CH, EXT>), 160 * 1024);                                                    \
@@ -1459,7 +1459,7 @@ SubOut expert_ffn(nvl_model* m, const LayerRun& r, const MixerW& w, int M, Exper
     if (dense && E <= 64 && c.route_softmax) {
         GemmArgs a = mk(m->xn, m->H, w.router, nullptr, E, w.route_bias, 1.f, M, E, m->H);
         KScope ks(m, KC_OTHER, 2.0 * M * E * m->Hn, KS_MOE_ROUTER, ((double)E * m->Hn + (double)M * m->Hn) * (double)m->wsize + (double)M * E * 4.0);
-        hipLaunchKernelGGL(moe_router_gate_kernel, router_gate_grid(M), dim3(1024), 0, m->stream, a, k, m->moe_gate, (float*)nullptr, 0, r.Ep, parts);
+        hipLaunchKernelGGL(moe_router_gate_kernel, router_gate_grid(M), dim3(1024), 0, m->stream, a, k, RouteOut{m->moe_gate, nullptr, nullptr}, (float*)nullptr, 0, r.Ep, parts);
         NVL_HIP(hipGetLastError());
     } else {
         m->site = KS_MOE_ROUTER;

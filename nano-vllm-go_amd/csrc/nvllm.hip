@@ -1186,7 +1186,7 @@ void bind_slot(const nvl_model* m, const Meta& hm, int i, int slot) {
 static int g_norm_t16 = 1;     // nvl_set_tuning key 9: norm_tile16_kernel for prefill-sized bf16 norms (0 = norm_kernel)
 template <typename ActT>
 void launch_norm(nvl_model* m, float* x, const int32_t* rows_idx, const float* w, const float* b,
-                 void* y, int rows) {
+                 void* y, int rows, bf16_t* y_rows = nullptr) {
     KScope ks(m, KC_OTHER, 0, KS_NORM, (double)rows * m->H * (4.0 + (double)m->wsize));
     PendingResid pr{nullptr, 0, 0, 0.f, nullptr, nullptr};
     if (m->pending_slices > 0) {            // complete the residual add the previous decode GEMM left as split-K slices
@@ -1201,12 +1201,12 @@ void launch_norm(nvl_model* m, float* x, const int32_t* rows_idx, const float* w
         hipLaunchKernelGGL((norm_row_kernel<ActT>), dim3(rows), dim3(256), 0, m->stream, x, rows_idx, w, b,
                            m->cfg.norm_eps, (ActT*)y, m->H, pr);
     else if (sizeof(ActT) == 2 && m->H % 32 == 0 && m->H <= 4096 && g_norm_t16) {   // (wider rows would spill: norm_kernel)
-        // 16 rows x H bf16 of LDS (up to 160 KiB); the row sits in registers: instance by chunks per lane
+        // 16 rows x H bf16 of LDS (up to 129 KiB); the row sits in registers: instance by chunks per lane
 #define NVL_NT16(CH, PEND)                                                                                             \
         do {                                                                                                           \
             NVL_LDS_ATTR((norm_tile16_kernel<CH, PEND>), 160 * 1024);                                                  \
-            hipLaunchKernelGGL((norm_tile16_kernel<CH, PEND>), dim3(cdiv(rows, 16)), dim3(1024), (size_t)16 * m->H * 2, m->stream, x, \
-                               rows_idx, w, b, m->cfg.norm_eps, (bf16_t*)y, rows, m->H, pr);                            \
+            hipLaunchKernelGGL((norm_tile16_kernel<CH, PEND>), dim3(cdiv(rows, 16)), dim3(1024), (size_t)16 * tile16_pitch(m->H) * 2, m->stream, x, \
+                               rows_idx, w, b, m->cfg.norm_eps, (bf16_t*)y, rows, m->H, pr, y_rows);                    \
         } while (0)
         if (pr.part) NVL_NT16(8, true);        // (H <= 2048: checked above)
         else { if (m->H <= 2048) NVL_NT16(8, false); else NVL_NT16(16, false); }
@@ -1215,9 +1215,11 @@ void launch_norm(nvl_model* m, float* x, const int32_t* rows_idx, const float* w
         hipLaunchKernelGGL((norm_kernel<ActT>), dim3(cdiv(rows, 4)), dim3(256), 0, m->stream, x, rows_idx, w, b,
                            m->cfg.norm_eps, (ActT*)y, rows, m->H);
 }
-void norm(nvl_model* m, float* x, const int32_t* rows_idx, const DevTensor& w, const DevTensor& b, void* y, int rows) {
+// does the norm of so many rows leave a row-major copy of its result (y_rows) too?
+bool norm_copies_rows(const nvl_model* m, int rows) { return !m->f32 && rows > 512 && m->H <= 4096 && g_norm_t16; }
+void norm(nvl_model* m, float* x, const int32_t* rows_idx, const DevTensor& w, const DevTensor& b, void* y, int rows, bf16_t* y_rows = nullptr) {
     if (m->f32) launch_norm<float>(m, x, rows_idx, (const float*)w.p, (const float*)b.p, y, rows);
-    else launch_norm<bf16_t>(m, x, rows_idx, (const float*)w.p, (const float*)b.p, y, rows);
+    else launch_norm<bf16_t>(m, x, rows_idx, (const float*)w.p, (const float*)b.p, y, rows, y_rows);
     NVL_HIP(hipGetLastError());
 }
 
@@ -1569,7 +1571,8 @@ void moe_sort(nvl_model* m, int E, int k, int M, int BM) {
     NVL_HIP(hipGetLastError());
 }
 // the experts' feed-forwards over the sorted pairs: rows of m->xn -> m->moe_eo (pair order of m->slot_of)
-void moe_expert_gemms(nvl_model* m, const MoeW& w, int M, int BM, bool pp, bool small) {
+// xn_rows: a row-major copy of m->xn, or NULL
+void moe_expert_gemms(nvl_model* m, const MoeW& w, int M, int BM, bool pp, bool small, const bf16_t* xn_rows = nullptr) {
     const int E = w.E, k = w.k, I = w.I, H = m->H, pairs = M * k;
     const double e_touch = (double)std::min(E, pairs);
     const int max_mtiles = cdiv(pairs, BM) + E;      // every expert may end on a partial tile
@@ -1603,8 +1606,8 @@ void moe_expert_gemms(nvl_model* m, const MoeW& w, int M, int BM, bool pp, bool 
         // (64 cache lines per load instruction); copy them into expert order once, then the GEMM streams whole
         // 1-KiB operand blocks (Granite-1B, 16384 tokens: expert-up 1119 -> ? us per layer)
         KScope ks(m, KC_OTHER);
-        hipLaunchKernelGGL(moe_gather_fm_kernel, dim3(cdiv(pairs, 16)), dim3(256), 0, m->stream, (const bf16_t*)m->xn,
-                           m->perm_token, (bf16_t*)m->moe_xg, pairs, H);
+        if (xn_rows) hipLaunchKernelGGL((moe_gather_fm_kernel<true>), dim3(cdiv(pairs, 16)), dim3(256), 0, m->stream, xn_rows, m->perm_token, (bf16_t*)m->moe_xg, pairs, H);
+        else hipLaunchKernelGGL((moe_gather_fm_kernel<false>), dim3(cdiv(pairs, 16)), dim3(256), 0, m->stream, (const bf16_t*)m->xn, m->perm_token, (bf16_t*)m->moe_xg, pairs, H);
         NVL_HIP(hipGetLastError());
         a.A = m->moe_xg; a.a_rows = nullptr;
     }
@@ -1626,7 +1629,8 @@ bool moe_dense_ok(const nvl_model* m, const LayerW& l, int M) {
 // norm): the router and the expert-up projection scale their accumulators by rstd[m] instead of reading a normed operand
 // next_norm_w (decode, dense-masked form only): the down projection carries the NEXT norm (the following layer's attention
 // norm / the final norm) as the deferred-RMSNorm producer, no slices left for a norm launch to sum; returns true when it did (m->xn / m->rs_part then hold that norm's operand).
-bool moe(nvl_model* m, const LayerW& l, int M, bool deferred_norm = false, const float* next_norm_w = nullptr) {
+// xn_rows: a row-major copy of m->xn, or NULL (it may lie in m->moe_eo, which the experts' products replace)
+bool moe(nvl_model* m, const LayerW& l, int M, bool deferred_norm = false, const float* next_norm_w = nullptr, const bf16_t* xn_rows = nullptr) {
     const nvl_model_config& c = m->cfg;
     const int E = c.num_experts, k = c.num_experts_per_tok, I = m->F, H = m->H;
     const int pairs = M * k;
@@ -1636,12 +1640,21 @@ bool moe(nvl_model* m, const LayerW& l, int M, bool deferred_norm = false, const
     const bool dense = moe_dense_ok(m, l, M) && m->pending_slices == 0;
     // decode: router logits, softmax, top-k and the dense gate matrix in one launch (gemm.h moe_router_gate_kernel)
     const bool fused_route = dense && g_moe_fused_route && E <= 64 && H % 32 == 0;
+    // decode-sized batches: one planning launch, and the weighted combine rides on the norm that follows
+    const bool small = !m->f32 && M <= 64 && pairs <= MOE_PLAN_MAX_PAIRS && E <= MOE_PLAN_MAX_E && g_moe_small;
+    // prefill: the same launch, leaving the chosen experts (6867 rows of 1024, 32 experts: 20 us on 54 tiles of 128 x 128 and 9 us of
+    // routing before, 12.7 now)
+    const bool route_ids = !m->f32 && !dense && !small && !deferred_norm && g_moe_fused_route && E <= 64 && H % 32 == 0 && g_force_tile == 0;
     {
         GemmArgs ar = mk(m->xn, H, l.t[NVL_T_ROUTER].p, m->router_logits, 128, nullptr, 1.f, M, E, H);
         if (deferred_norm) set_deferred_in(m, ar);
         if (fused_route) {
             KScope ks(m, KC_GEMM, 2.0 * (double)M * E * H, -1, ((double)E * H + (double)M * H) * (double)m->wsize + (double)M * E * 8.0);
-            hipLaunchKernelGGL(moe_router_gate_kernel, router_gate_grid(M), dim3(1024), 0, m->stream, ar, k, m->moe_gate, m->router_logits, 128, E, 0);
+            hipLaunchKernelGGL(moe_router_gate_kernel, router_gate_grid(M), dim3(1024), 0, m->stream, ar, k, RouteOut{m->moe_gate, nullptr, nullptr}, m->router_logits, 128, E, 0);
+            NVL_HIP(hipGetLastError());
+        } else if (route_ids) {
+            KScope ks(m, KC_GEMM, 2.0 * (double)M * E * H, -1, ((double)E * H + (double)M * H) * (double)m->wsize + (double)pairs * 8.0);
+            hipLaunchKernelGGL(moe_router_gate_kernel, dim3(cdiv(M, 16)), dim3(1024), 0, m->stream, ar, k, RouteOut{nullptr, m->expert_ids, m->expert_w}, (float*)nullptr, 0, 0, 0);
             NVL_HIP(hipGetLastError());
         } else {
             gemm(m, EPI_STORE, true, ar);
@@ -1675,8 +1688,6 @@ bool moe(nvl_model* m, const LayerW& l, int M, bool deferred_norm = false, const
         m->pending_part = m->moe_part; m->pending_slices = nsl; m->pending_rows = M; m->pending_alpha = m->resid_alpha;
         return false;
     }
-    // decode-sized batches: one planning launch, and the weighted combine rides on the norm that follows
-    const bool small = !m->f32 && M <= 64 && pairs <= MOE_PLAN_MAX_PAIRS && E <= MOE_PLAN_MAX_E && g_moe_small;
     // m-tile height of the grouped GEMMs: 128 rows; the 256x128 three-stage instance stays a tuning option (Granite-1B,
     // 4096 rows per expert: 441 K vs 450 K prefill tok/s)
     const bool pp = moe_pp_ok(m, I, small);
@@ -1687,7 +1698,7 @@ bool moe(nvl_model* m, const LayerW& l, int M, bool deferred_norm = false, const
                            m->expert_w, m->seg_start, m->moe_tile_map, m->moe_n_mtiles, m->perm_token, m->slot_of);
         NVL_HIP(hipGetLastError());
     } else {
-        {
+        if (!route_ids) {
             KScope ks(m, KC_OTHER, 0, KS_MOE_PLAN);
             hipLaunchKernelGGL(moe_route_kernel, dim3(cdiv(M, 4)), dim3(256), 0, m->stream, m->router_logits, 128, M, E, k,
                                m->expert_ids, m->expert_w);
@@ -1695,7 +1706,7 @@ bool moe(nvl_model* m, const LayerW& l, int M, bool deferred_norm = false, const
         }
         moe_sort(m, E, k, M, BM);
     }
-    moe_expert_gemms(m, MoeW{E, k, I, l.moe_in, l.t[NVL_T_MOE_OUT].p}, M, BM, pp, small);
+    moe_expert_gemms(m, MoeW{E, k, I, l.moe_in, l.t[NVL_T_MOE_OUT].p}, M, BM, pp, small, xn_rows);
     if (small && !m->keep_hidden && m->pending_slices == 0 && H % 4 == 0 && H <= 1024 * NORM_ROW_MAXCH) {
         // x += rm * sum_k w[t][k] * eo[slot[t][k]] is completed by the next norm's read of x (PendingResid)
         m->pending_part = m->moe_eo; m->pending_slices = k; m->pending_rows = M; m->pending_alpha = c.residual_multiplier;
@@ -1980,11 +1991,12 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
             // decode, RMSNorm + SwiGLU: the O-projection carries the FFN norm (deferred RMSNorm, gemm.h) — one launch less
             const bool defer = (defer_ok || (defer_moe_ok && moe_dense_ok(m, l, M))) && m->pending_slices == 0 && !l.t[NVL_T_FFN_NORM_B].present();
             m->site = KS_OPROJ;
+            bf16_t* xn_rows = c.use_moe && !defer && norm_copies_rows(m, M) ? (bf16_t*)m->moe_eo : nullptr;      // (for the copy into expert order)
             if (defer) {
                 resid_gemm(m, m->attn_out, qw, l.t[NVL_T_WO].p, bo, m->resid_alpha, M, H, qw, (const float*)l.t[NVL_T_FFN_NORM_W].p);
             } else {
                 resid_gemm(m, m->attn_out, qw, l.t[NVL_T_WO].p, bo, m->resid_alpha, M, H, qw);
-                norm(m, m->x, nullptr, l.t[NVL_T_FFN_NORM_W], l.t[NVL_T_FFN_NORM_B], m->xn, M);
+                norm(m, m->x, nullptr, l.t[NVL_T_FFN_NORM_W], l.t[NVL_T_FFN_NORM_B], m->xn, M, xn_rows);
             }
             // the FFN-down projection carries the NEXT layer's attention norm, or the final norm when every row is
             // a last row (decode)
@@ -1993,7 +2005,7 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
             if (c.use_moe) {
                 const bool defer2 = defer && defer_moe_ok && g_defer_norm != 3 && !nxt_b->present() &&
                                     (li + 1 < m->L || (!all_rows && M == n_seqs && M <= 64));
-                xn_deferred = moe(m, l, M, defer, defer2 ? (const float*)nxt_w->p : nullptr);
+                xn_deferred = moe(m, l, M, defer, defer2 ? (const float*)nxt_w->p : nullptr, xn_rows);
             } else {
                 ffn_up(m, l, M, defer);
                 const bool defer2 = defer_ok && g_defer_norm != 3 && m->pending_slices == 0 && !nxt_b->present() &&

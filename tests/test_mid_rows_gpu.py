@@ -167,3 +167,26 @@ def test_mamba_prompts(gpu, heads, hd, groups, lens):
                 assert rel_err(alone[0], got["f32"][i]) <= 1e-5, lens[i]
         m.close()
     assert rel_err(got["bf16"], got["f32"]) <= TOL
+
+
+@pytest.mark.parametrize("n", [65, 513, 530, 1040])
+def test_moe_prompt_forms(gpu, n):
+    """Routing in the router's launch, expert-ordered rows copied from the norm's row-major result (beyond 512 tokens): against the separate
+    launches and the fragment-major source."""
+    import torch
+    from bench import gen_weights_on_device
+    cfg = dict(gpu.synth.FULL_CONFIGS["granite-3.0-1b-a400m"], num_layers=1, vocab_size=1000)
+    m = gpu.HipTransformerModel(cfg, None, precision="bf16", max_seqs=1, max_batch_tokens=1088)
+    gen_weights_on_device(gpu, cfg, m, torch, torch.device("cuda", 0), keep_host=False)
+    m.finalize()
+    tokens, got = np.random.default_rng(n).integers(0, 1000, n).tolist(), []
+    for forms in ((1, 1), (0, 0)):
+        old = [(key, gpu.lib().nvl_set_tuning(key, v)) for key, v in zip((9, 31), forms)]
+        m.seq_reset(0)
+        got.append(m.forward_batch([0], [tokens], [0], all_logits=True)[0])
+        for key, v in old:
+            gpu.lib().nvl_set_tuning(key, v)
+    m.close()
+    # the same bf16 operands; logits of the router that differ in the order of their fp32 sums may swap two experts of equal weight: few rows
+    err = np.abs(got[0] - got[1]).max(-1) / np.abs(got[1]).max()
+    assert np.mean(err > 5e-3) <= 0.01
