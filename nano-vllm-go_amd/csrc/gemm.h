@@ -1070,7 +1070,7 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
     // (MT = 4 — batches above 32 and the 64-row groups of larger ones — has no registers to hold it across the stream:
     // 34-54 spilled there, QKV at 128 rows 7.2 -> 10.8 us; those launches are long enough to fetch it in the epilogue)
     constexpr bool RSTD_PRE = MT <= 2;
-    const float rstd_pre = (RSTD_PRE && (EPI == EPI_STORE || SCALED || epi_glu(EPI)) && wave < NTW * MT) ? deferred_rstd(p, 16 * (i_pre + (SCALED ? i_off : 0)) + fr) : 1.0f;   // (only the waves that run an epilogue element)
+    const float rstd_pre = (RSTD_PRE && (EPI == EPI_STORE || EPI == EPI_QKV || SCALED || epi_glu(EPI)) && wave < NTW * MT) ? deferred_rstd(p, 16 * (i_pre + (SCALED ? i_off : 0)) + fr) : 1.0f;   // (only the waves that run an epilogue element)
     // (grid_y: gridDim.y as an explicit argument — the built-in lives in the hidden part of the kernarg block and costs a
     // dependent scalar round trip of its own before the first weight load)
     const int nslices = p.m_split ? 1 : p.grid_y, slice = p.m_split ? 0 : blockIdx.y;
@@ -1102,7 +1102,10 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
         }
     }
 
-    const bf16_t* wp = (const bf16_t*)p.W + (((int64_t)(nt0 + tile) * (p.K >> 5) + ks0) * 64 + lane) * 8;
+    // EPI_QKV: the workgroup's two tiles are half a head apart (they rotate together)
+    const int q_half = EPI == EPI_QKV ? p.qkv.hd >> 5 : 0, q_head = EPI == EPI_QKV ? bx / q_half : 0, q_tile = bx - q_head * q_half;
+    const int wt = EPI == EPI_QKV ? q_head * 2 * q_half + q_tile + tile * q_half : nt0 + tile;
+    const bf16_t* wp = (const bf16_t*)p.W + (((int64_t)wt * (p.K >> 5) + ks0) * 64 + lane) * 8;
     const bf16_t* xp[MT];
 #pragma unroll
     for (int i = 0; i < MT; i++)   // rows >= M of the last 16-row tile exist (padded allocation) and are never stored
@@ -1204,6 +1207,11 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
             const int f = (nt0 >> 1) * 16 + 4 * fg;    // NTW == 2: tiles [gate 16 | up 16] of features 8*nt0..
             epilogue_glu4<EPI, OutT, MOE>(p, 16 * i + fr, f, ksum(0, i), ksum(NTW - 1, i),
                                         RSTD_PRE && i == i_pre ? rstd_pre : deferred_rstd(p, 16 * i + fr));
+        }
+    } else if constexpr (EPI == EPI_QKV) {
+        for (int i = wave; i < MT; i += NTW * ksplit) {
+            const float rs = RSTD_PRE && i == i_pre ? rstd_pre : deferred_rstd(p, 16 * i + fr);
+            epilogue_qkv_pair(p, 16 * i + fr, q_head, q_tile * 16 + 4 * fg, ksum(0, i) * rs, ksum(NTW - 1, i) * rs);
         }
     } else if (EPI == EPI_RESID && nslices > 1) {
         // split-K across workgroups: publish the partial tile (slice 0 carries the bias); the following norm
@@ -1706,7 +1714,7 @@ static inline bool launch_gemm_skinny_wide(hipStream_t st, const GemmArgs& a) {
 }
 template <int EPI, typename OutT>
 static inline bool launch_gemm_skinny_bf16(hipStream_t st, const GemmArgs& a0) {
-    if (EPI == EPI_QKV) return false;               // prefill-only epilogue (a decode workgroup owns 16 columns, not a head)
+    if (EPI == EPI_QKV && (a0.qkv.hd % 32 != 0 || a0.m_passes > 1)) return false;
     if (skinny_rows(a0) > 64 || a0.a_rows || a0.seg || a0.tile_map) return false;
     GemmArgs a = a0;
     a.x_mask = (g_x_mask && a0.M % 16 != 0) ? 1 : 0;     // padded rows of the last 16-row activation tile are not fetched
@@ -1715,7 +1723,7 @@ static inline bool launch_gemm_skinny_bf16(hipStream_t st, const GemmArgs& a0) {
         const bool wide_ok = skinny_rows(a) > 16 && cdiv(a.N, 64) >= 256 && !a.sk_part;   // M <= 16: the narrow form streams as fast
         if (g_force_ntw == 8 || (g_force_ntw == 0 && wide_ok)) { if (launch_gemm_skinny_wide<EPI, OutT>(st, a)) return true; }
     }
-    if (epi_glu(EPI)) return launch_gemm_skinny_ntw<2, EPI, OutT>(st, a);
+    if constexpr (epi_glu(EPI) || EPI == EPI_QKV) return launch_gemm_skinny_ntw<2, EPI, OutT>(st, a);      // (pairs: gate | up, the halves of a head)
     if (g_force_ntw == 2) return launch_gemm_skinny_ntw<2, EPI, OutT>(st, a);
     if (g_force_ntw == 4) return launch_gemm_skinny_ntw<4, EPI, OutT>(st, a);
     return launch_gemm_skinny_ntw<1, EPI, OutT>(st, a);
@@ -1839,7 +1847,7 @@ static inline void launch_gemm_mid_rows(hipStream_t st, const GemmArgs& a0) {
 template <int EPI, typename OutT>
 static inline bool mid_wins(const GemmArgs& a) {
     if (!g_mid || a.M > MID_MAX_ROWS || a.M > std::max(64, g_chunk_max_m) || a.K % 64 != 0 || a.a_rows || a.seg || a.tile_map || a.sk_part || a.moe_gate || a.c_row0 || g_force_tile ||
-        g_force_ntw || a.rs_half || (EPI == EPI_RESID && a.rs_in)) return false;
+        g_force_ntw || a.rs_half || ((EPI == EPI_RESID || EPI == EPI_QKV) && a.rs_in)) return false;
     if (EPI == EPI_QKV && a.qkv.hd == 128) return a.M > 64 && cdiv(a.N, 128) * cdiv(a.M, 64) <= 512;
     if (EPI == EPI_QKV && a.qkv.hd != 64) return false;
     if (g_mid == 2) return true;

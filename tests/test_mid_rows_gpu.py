@@ -190,3 +190,24 @@ def test_moe_prompt_forms(gpu, n):
     # the same bf16 operands; logits of the router that differ in the order of their fp32 sums may swap two experts of equal weight: few rows
     err = np.abs(got[0] - got[1]).max(-1) / np.abs(got[1]).max()
     assert np.mean(err > 5e-3) <= 0.01
+
+
+@pytest.mark.parametrize("family,hd", [("gpt2", 64), ("llama", 64), ("llama", 128), ("falcon", 64)])
+@pytest.mark.parametrize("lens", [[2], [16], [1, 15, 1], [33], [20, 44], [31, 1, 1]])
+def test_short_prompts_place_their_heads(gpu, family, hd, lens):
+    """Up to 64 tokens: the QKV projection rotates and places its heads itself (key 18 = 64: fp32 rows and a launch of their own).  The same
+    fp32 sums and one rounding each way, so only the order of the K slices differs; the cache by a decode step that reads it."""
+    cfg = gpu.synth.tiny_config(family, hidden=256, num_heads=256 // hd, head_dim=hd, num_kv_heads=1 if family == "falcon" else 256 // hd, max_seq_len=64)
+    m = gpu.HipTransformerModel(cfg, gpu.synth.make_weights(cfg, seed=3, scale=0.05), precision="bf16", max_seqs=len(lens), max_batch_tokens=128)
+    r = np.random.default_rng(sum(lens))
+    prompts = [r.integers(0, cfg["vocab_size"], n).tolist() for n in lens]
+    ids, got = list(range(len(lens))), []
+    for rows in (0, 64):
+        old = gpu.lib().nvl_set_tuning(18, rows)
+        for i in ids:
+            m.seq_reset(i)
+        first = m.forward_batch(ids, prompts, [0] * len(ids))[0]
+        got.append((first, m.forward_batch(ids, [[9]] * len(ids), lens)[0]))
+        gpu.lib().nvl_set_tuning(18, old)
+    m.close()
+    assert rel_err(got[0][0], got[1][0]) <= TOL and rel_err(got[0][1], got[1][1]) <= TOL
