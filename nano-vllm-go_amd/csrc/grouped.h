@@ -21,6 +21,7 @@
 #include "attn.h"
 #include "common.h"
 #include "latent.h"
+#include "linrec.h"
 
 namespace nvl {
 
@@ -51,6 +52,8 @@ struct GroupedArgs {
     void* out; int64_t out_ld;                    // operand of W_o: [token][out_ld], head h at column h * vp
     int table;                                    // grouped_prefill_kernel: the distance bias comes from a table in LDS (it has room for it)
     float* part; int32_t* part_cnt;               // keys split over workgroups: partial results, arrival tickets (zero between launches)
+    int row_wgs;                                  // grouped_short_kernel: workgroups of the rows of a sequence and key split
+    GatedNormArgs gn; void* gn_out;               // ... QK: what one more workgroup per sequence does, the gated norm of its token's row (gn_out NULL: none)
 };
 
 // ---- fp32 mode: keys and values of the batch's tokens into the cache (bf16: gemm.h EPI_GROUPED): grid (32-token units of a sequence's new positions, sequences, G) ----
@@ -614,11 +617,54 @@ __device__ __forceinline__ f32x4 grouped_part_load(const float* p) {
     grouped_part_load2(p, a, b); grouped_part_load2(p + 2, c, d);
     return f32x4{a, b, c, d};
 }
-template <int KS, int DT, int NW>
+// One wave's head row (grouped_qk_row_kernel's fast case: four channels a lane, dim = dp <= 256, rot 0 or dim), split so that the first key
+// tile's loads can leave between its loads and its arithmetic.
+struct GroupedTurnRow {
+    f32x4 v, w, cs[2];
+    __device__ __forceinline__ void load(const GroupedArgs& p, const float* row, int h, const float* wt, int pos, int lane) {
+        const int c = lane * 4, half = p.rot >> 1;
+        v = w = cs[0] = cs[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (c >= p.dp) return;
+        v = *(const f32x4*)(row + (int64_t)h * p.dp + c);
+        if (p.qk_norm) w = *(const f32x4*)(wt + (p.qk_norm == 2 ? (int64_t)h * p.dim : 0) + c);
+        if (p.rot) {
+            const f32x2* t = p.turn + (int64_t)pos * half + (c < half ? c : c - half);
+            cs[0] = *(const f32x4*)t; cs[1] = *(const f32x4*)(t + 2);
+        }
+    }
+    // ss: the sum of squares of the whole projection (qk_norm 2) of `heads` heads
+    __device__ __forceinline__ void finish(const GroupedArgs& p, float ss, int heads, int lane, bf16_t* dst) {
+        const int c = lane * 4, half = p.rot >> 1;
+        if (p.qk_norm) {
+            if (p.qk_norm == 1) ss = wave_sum(v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3]);
+            v *= 1.0f / sqrtf(ss / ((float)p.dim * (p.qk_norm == 2 ? heads : 1)) + p.eps) * w;
+        }
+        const int other = c < half ? lane + (half >> 2) : lane - (half >> 2);
+        bf16x4 y;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const float u = __shfl(v[r], other & 63, 64), cc = cs[r >> 1][2 * (r & 1)], s = cs[r >> 1][2 * (r & 1) + 1];
+            y[r] = (bf16_t)(!p.rot ? v[r] : c < half ? v[r] * cc - u * s : v[r] * cc + u * s);
+        }
+        if (c < p.dp) *(bf16x4*)(dst + c) = y;
+    }
+};
+// QK (one token per sequence): queries and the new key come from the fp32 rows of proj, normed and rotated here, a head a wave, under the
+// first key tile's loads; the wave with the last key tile puts the new key in its operand and appends it to the cache.  Besides, the
+// launch may carry the gated norm of a second mixer's rows.  (As launches of their own those two took 6.4 and 6.3 us.)
+template <int KS, int DT, int NW, bool QK>
 __global__ __launch_bounds__(NW * 64) void grouped_short_kernel(GroupedArgs p) {
     extern __shared__ __attribute__((aligned(16))) char grp_sm[];       // [NW][DT][64] f32x4
     __shared__ float red_m[NW][16], red_l[NW][16];
     __shared__ int ticket;
+    constexpr int QLD = KS * 32 + 8;
+    __shared__ __attribute__((aligned(16))) bf16_t qsm[QK ? 17 : 1][QLD];      // QK: the row tile's queries, the new key
+    if constexpr (QK) {
+        if ((int)blockIdx.x == p.row_wgs) {
+            if (blockIdx.z == 0) gated_norm_row<NW * 64>(p.gn, p.seq_tok_start[blockIdx.y], (bf16_t*)p.gn_out, &red_m[0][0]);
+            return;
+        }
+    }
     const int kvh = blockIdx.x % p.G, rt = blockIdx.x / p.G, seq = blockIdx.y;
     const int R = p.seq_len[seq] * p.group;
     if (R > p.short_rows || rt * 16 >= R) return;
@@ -634,19 +680,44 @@ __global__ __launch_bounds__(NW * 64) void grouped_short_kernel(GroupedArgs p) {
     const int full_lo = p.mask.lo(last), full_hi = first;
     const int64_t tok = tok0 + si;
     bf16x8 qf[KS], kf[4][KS], vf[DT][2];
+    // (a barrier for LDS only: the tile's loads stay in flight)
+    auto lds_barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); __builtin_amdgcn_s_barrier(); asm volatile("" ::: "memory"); };
+    const int it_last = n_tiles - 1 - (blockIdx.z * NW + wave);
+    const bool appends = QK && it_last >= 0 && it_last % (NW * (int)gridDim.z) == 0;      // (this wave walks the tile of the new key)
+    const int nq = min(16, R - rt * 16);
+    GroupedTurnRow turn;
+    auto turn_load = [&](int r) {
+        const float* pr = p.proj + (int64_t)tok0 * p.proj_ld;
+        if (r < nq) turn.load(p, pr, kvh * p.group + rt * 16 + r, p.q_norm, pos0, lane);
+        else turn.load(p, pr + p.qk_koff, kvh, p.k_norm, pos0, lane);
+    };
+    // a norm over the projection: the workgroup's threads have four columns each on their way
+    const float *rq = p.proj + (int64_t)tok0 * p.proj_ld, *rk = rq + p.qk_koff;
+    f32x4 uq = f32x4{0.f, 0.f, 0.f, 0.f}, uk = uq;
+    const int nqc = p.H * p.dp, nkc = p.G * p.dp;
+    if constexpr (QK) {
+        if (wave <= nq) turn_load(wave);
+        if (p.qk_norm == 2) {
+            if (tid * 4 < nqc) uq = *(const f32x4*)(rq + tid * 4);
+            if (tid * 4 < nkc) uk = *(const f32x4*)(rk + tid * 4);
+        }
+    } else {
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) qf[ks] = grouped_load_q(p, tok, head, ks, fg);
+        for (int ks = 0; ks < KS; ks++) qf[ks] = grouped_load_q(p, tok, head, ks, fg);
+    }
     const GroupedScore f(p, head);
     f32x4 o[DT];
 #pragma unroll
     for (int d = 0; d < DT; d++) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m = -1e30f, l = 0.f;
     const int64_t v_ld = p.bs >> 5;
-    for (int it = blockIdx.z * NW + wave; it < n_tiles; it += NW * gridDim.z) {
-        const int kt = it < n_pre ? it : t0 + it - n_pre;
-        const int bi = kt * 64 / p.bs, r0 = kt * 64 - bi * p.bs;
+    const bf16_t* kp = nullptr;
+    int kt = 0, bi = 0, r0 = 0;
+    auto load_tile = [&](int it) {
+        kt = it < n_pre ? it : t0 + it - n_pre;
+        bi = kt * 64 / p.bs; r0 = kt * 64 - bi * p.bs;
         const bf16_t* base = (const bf16_t*)p.cache + (int64_t)__builtin_amdgcn_readfirstlane(tbl[bi]) * p.block_stride + lane * 8;
-        const bf16_t* kp = base + ((int64_t)kvh * p.bs + r0) * p.dp;
+        kp = base + ((int64_t)kvh * p.bs + r0) * p.dp;
         const bf16_t* vp = base + (int64_t)p.G * p.bs * p.dp + (int64_t)kvh * p.bs * p.vp + (r0 >> 5) * 512;
 #pragma unroll
         for (int t = 0; t < 4; t++)
@@ -656,6 +727,19 @@ __global__ __launch_bounds__(NW * 64) void grouped_short_kernel(GroupedArgs p) {
         for (int d = 0; d < DT; d++)
 #pragma unroll
             for (int u = 0; u < 2; u++) vf[d][u] = *(const bf16x8*)(vp + (d * v_ld + u) * 512);
+    };
+    auto do_tile = [&](int it) __attribute__((always_inline)) {
+        if (QK && appends && it == n_tiles - 1) {
+            const int kr = grouped_k_row(last - bi * p.bs);
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int ks = 0; ks < KS; ks++)
+                    if (kr - r0 == 16 * t + fq) {
+                        kf[t][ks] = *(const bf16x8*)(qsm[16] + ks * 32 + fg * 8);
+                        *(bf16x8*)((bf16_t*)kp + (t * KS + ks) * 512) = kf[t][ks];      // (this lane's place in the block it has read)
+                    }
+        }
         f32x4 s[4];
 #pragma unroll
         for (int t = 0; t < 4; t++) {
@@ -685,6 +769,34 @@ __global__ __launch_bounds__(NW * 64) void grouped_short_kernel(GroupedArgs p) {
             o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[d][0], p0, o[d], 0, 0, 0);
             o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[d][1], p1, o[d], 0, 0, 0);
         }
+    };
+    const int it0 = blockIdx.z * NW + wave;
+    if (it0 < n_tiles) load_tile(it0);
+    if constexpr (QK) {
+        float sq = 0.f, sk = 0.f;
+        if (p.qk_norm == 2) {
+            auto sum4 = [](f32x4 u) { return (u[0] * u[0] + u[1] * u[1]) + (u[2] * u[2] + u[3] * u[3]); };
+            float aq = sum4(uq), ak = sum4(uk);
+            for (int i = tid * 4 + NW * 256; i < nqc; i += NW * 256) aq += sum4(*(const f32x4*)(rq + i));
+            for (int i = tid * 4 + NW * 256; i < nkc; i += NW * 256) ak += sum4(*(const f32x4*)(rk + i));
+            aq = wave_sum(aq); ak = wave_sum(ak);
+            if (lane == 0) { red_m[wave][0] = aq; red_l[wave][0] = ak; }
+            lds_barrier();
+#pragma unroll
+            for (int i = 0; i < NW; i++) { sq += red_m[i][0]; sk += red_l[i][0]; }
+        }
+        for (int r = wave; r <= nq; r += NW) {
+            if (r != wave) turn_load(r);
+            turn.finish(p, r < nq ? sq : sk, r < nq ? p.H : p.G, lane, qsm[r < nq ? r : 16]);
+        }
+        lds_barrier();
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) qf[ks] = *(const bf16x8*)(qsm[min(fq, nq - 1)] + ks * 32 + fg * 8);
+    }
+    if (it0 < n_tiles) do_tile(it0);
+    for (int it = it0 + NW * gridDim.z; it < n_tiles; it += NW * gridDim.z) {
+        load_tile(it);
+        do_tile(it);
     }
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
@@ -698,7 +810,7 @@ __global__ __launch_bounds__(NW * 64) void grouped_short_kernel(GroupedArgs p) {
     for (int w = 1; w < NW; w++) ms = fmaxf(ms, red_m[w][fq]);
 #pragma unroll
     for (int w = 0; w < NW; w++) { sc[w] = __builtin_amdgcn_exp2f(red_m[w][fq] - ms); L += red_l[w][fq] * sc[w]; }      // (a wave without a tile: l = 0, O = 0)
-    const int nz = gridDim.z, pair = seq * gridDim.x + blockIdx.x;
+    const int nz = gridDim.z, pair = seq * p.row_wgs + blockIdx.x;
     const float sink = grouped_sink(p, head);
     if (nz == 1 && p.sink) L += __builtin_amdgcn_exp2f(sink - ms);       // (a sink far above every score: inf, and the row is zero)
     float* rec = p.part + ((int64_t)pair * nz + blockIdx.z) * grouped_part_floats<DT>();

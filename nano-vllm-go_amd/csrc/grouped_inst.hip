@@ -35,8 +35,15 @@ void grouped_prefill_launch(hipStream_t st, const GroupedArgs& p, dim3 grid, siz
 template <int KS, int DT>
 static void run_short(hipStream_t st, const GroupedArgs& p, dim3 grid) {
     constexpr int nw = DT <= 8 ? 8 : 4;
-    NVL_LDS_ATTR((grouped_short_kernel<KS, DT, nw>), nw * DT * 1024);
-    hipLaunchKernelGGL((grouped_short_kernel<KS, DT, nw>), grid, dim3(nw * 64), nw * DT * 1024, st, p);
+    if constexpr (KS == 2 || KS == 4) {
+        if (p.qk_koff >= 0) {
+            NVL_LDS_ATTR((grouped_short_kernel<KS, DT, nw, true>), nw * DT * 1024);
+            hipLaunchKernelGGL((grouped_short_kernel<KS, DT, nw, true>), dim3(grid.x + (p.gn_out ? 1 : 0), grid.y, grid.z), dim3(nw * 64), nw * DT * 1024, st, p);
+            return;
+        }
+    }
+    NVL_LDS_ATTR((grouped_short_kernel<KS, DT, nw, false>), nw * DT * 1024);
+    hipLaunchKernelGGL((grouped_short_kernel<KS, DT, nw, false>), grid, dim3(nw * 64), nw * DT * 1024, st, p);
 }
 template <int KS>
 static void run_short_ks(hipStream_t st, const GroupedArgs& p, dim3 grid) {

@@ -23,6 +23,7 @@
 //     query rows; recurrences go token by token up to REC_STEP_MAX.
 #pragma once
 
+static int g_grouped_qk = 1;         // nvl_set_tuning key 42: decode: queries and keys normed and rotated by the attention launch (0 = by one of their own)
 static int g_grouped_split = 0;      // nvl_set_tuning key 37: key splits of the short grouped attention (1 .. 16); 0 = automatic
 
 namespace {
@@ -1109,9 +1110,10 @@ void linrec(nvl_model* m, LinRecArgs a, int n_seqs, int M, int max_len, bool fus
     NVL_HIP(hipGetLastError());
 }
 
+bool gated_norm_v4(const GatedNormArgs& a) { return a.part % 4 == 0 && a.y_ld % 4 == 0 && a.gate_ld % 4 == 0 && (((uintptr_t)a.y | (uintptr_t)a.gate) & 15) == 0; }
 template <typename ActT, bool GATE_FIRST>
 void gated_norm_launch(nvl_model* m, GatedNormArgs a, int col) {
-    const bool v4 = a.part % 4 == 0 && a.y_ld % 4 == 0 && a.gate_ld % 4 == 0 && (((uintptr_t)a.y | (uintptr_t)a.gate) & 15) == 0;
+    const bool v4 = gated_norm_v4(a);
     const bool wide = a.part > 1024;
     a.lanes = 4;
     while (a.lanes < 64 && a.lanes * (v4 ? 4 : 1) < a.part) a.lanes *= 2;
@@ -1271,7 +1273,8 @@ void mix_delta(nvl_model* m, const LayerRun& r, const MixerW& w, const Meta& md,
 void tap_layer(nvl_model* m, int li, int M);
 
 // ---- lightning attention beside another mixer: columns of the joint input projection -> m->lmix columns [ko, ko + ko2) ----
-void mix_lightning(nvl_model* m, const LayerRun& r, const MixerW& w, const Meta& md, int n_seqs, int M, int max_len) {
+// carry: not NULL: the gated norm of its rows is left to another launch (gn, gn_out) where that can do it
+void mix_lightning(nvl_model* m, const LayerRun& r, const MixerW& w, const Meta& md, int n_seqs, int M, int max_len, GroupedArgs* carry) {
     const nvl_layer_config& c = r.c;
     LinRecArgs a = linrec_args(m, r, md);
     a.H = c.heads2; a.DK = c.dim2; a.DV = c.vdim2; a.DVp = (int)round_up(c.vdim2, 4); a.kdiv = 1; a.q_scale = 1.f;
@@ -1279,7 +1282,8 @@ void mix_lightning(nvl_model* m, const LayerRun& r, const MixerW& w, const Meta&
     a.decay = w.decay; a.log2_decay = w.log2_decay;
     linrec<false>(m, a, n_seqs, M, max_len, false, KS_LIN_SCAN);
     GatedNormArgs g{m->lo, m->lo_ld, m->lproj + r.lg_off, m->lproj_ld, w.lin_norm, M, 1, c.heads2 * c.vdim2, m->cfg.norm_eps, r.kd, 0, 1};
-    gated_norm<false>(m, g, KS_LIN_GATE, r.ko);
+    if (carry && gated_norm_v4(g) && ((uintptr_t)g.w & 15) == 0) { carry->gn = g; carry->gn_out = (bf16_t*)m->lmix + (int64_t)(r.ko >> 5) * 512; }
+    else gated_norm<false>(m, g, KS_LIN_GATE, r.ko);
 }
 
 // ---- grouped-query attention: m->xn -> m->lmix columns [0, ko) ----
@@ -1314,16 +1318,24 @@ void mix_grouped(nvl_model* m, const LayerRun& r, const MixerW& w, const Meta& m
         m->site = KS_MIX_IN;
         gemm(m, r.raw ? EPI_GROUPED_RAW : EPI_GROUPED, false, g);
     }
-    if (c.mixer2) mix_lightning(m, r, w, md, n_seqs, M, max_len);
+    const bool plain = m->f32 || r.dp > 256 || r.vp > 256;
+    a.short_rows = GROUPED_SHORT_ROWS;
+    // one token per sequence: the attention launch norms and rotates them itself, and carries the second mixer's gated norm
+    const bool in_attn = g_grouped_qk && r.raw && !plain && max_len == 1 && M == n_seqs && a.group <= a.short_rows && c.ungated && c.dim == r.dp && (r.dp == 64 || r.dp == 128) &&
+                         (c.rot_dim == 0 || c.rot_dim == c.dim) && (((uintptr_t)w.q_norm | (uintptr_t)w.k_norm | (uintptr_t)r.turn) & 15) == 0;
+    a.qk_koff = -1;
+    if (c.mixer2) mix_lightning(m, r, w, md, n_seqs, M, max_len, in_attn ? &a : nullptr);
     if (r.raw) {          // norms and rotation of the fp32 queries and keys
         a.proj = m->lproj; a.proj_ld = m->lproj_ld; a.qk_koff = r.k_off; a.qk_norm = c.qk_norm; a.q_norm = w.q_norm; a.k_norm = w.k_norm; a.eps = m->cfg.norm_eps;
         a.rot = c.rot_dim; a.turn = r.turn; a.tok_pos = md.tok_pos; a.tok_tbl = md.tok_tbl; a.rows = M;
         a.q = a.q_out = m->lqg; a.q_ld = (int64_t)a.H * r.dp;
-        KScope ks(m, KC_OTHER, 0, KS_QK_TURN, (double)M * (a.H + a.G) * c.dim * (4.0 + ws));
-        grouped_qk_launch(m->stream, a, m->f32);
-        NVL_HIP(hipGetLastError());
+        if (!in_attn) {
+            KScope ks(m, KC_OTHER, 0, KS_QK_TURN, (double)M * (a.H + a.G) * c.dim * (4.0 + ws));
+            grouped_qk_launch(m->stream, a, m->f32);
+            NVL_HIP(hipGetLastError());
+            a.qk_koff = -1;
+        }
     }
-    const bool plain = m->f32 || r.dp > 256 || r.vp > 256;
     const int ctx = m->ctx_hint > 0 ? m->ctx_hint : m->cfg.max_seq_len;
     int tiles = cdiv(ctx, 64) + 1;                              // most key tiles a 256-row workgroup walks
     const int span = a.mask.span();
@@ -1333,7 +1345,6 @@ void mix_grouped(nvl_model* m, const LayerRun& r, const MixerW& w, const Meta& m
     // the distance biases of a workgroup's rows as a table in LDS, where they leave as many workgroups per CU as the ring does
     const size_t tab = lds + (size_t)grouped_tab_span(std::min(ctx, span > 0 ? span : ctx)) * a.group * 4;
     if (w.r1 && !a.mask.keep && tab <= (size_t)(r.dp <= 64 && r.vp <= 64 ? 80 : 160) * 1024) { a.table = tiles; lds = tab; }
-    a.short_rows = GROUPED_SHORT_ROWS;
     if ((r.dp == 256 && r.vp == 256) || lds > 160 * 1024) a.short_rows = 1 << 30;      // (three slots would not fit LDS)
     const bool any_short = m->min_len * a.group <= a.short_rows, any_long = max_len * a.group > a.short_rows;
     auto scope = [&](int several) {
@@ -1366,6 +1377,7 @@ void mix_grouped(nvl_model* m, const LayerRun& r, const MixerW& w, const Meta& m
         while (z < GROUPED_SPLITS && wgs * n_seqs * z * 2 <= 256 && z * 2 * 2 * nw <= key_tiles) z *= 2;
         if (g_grouped_split) z = (int)std::min<int64_t>(g_grouped_split, std::max<int64_t>(1, m->grp_cap / (wgs * n_seqs)));
         a.part = m->grp_part; a.part_cnt = m->grp_cnt;
+        a.row_wgs = (int)wgs;
         const dim3 grid((unsigned)wgs, n_seqs, z);
         grouped_short_launch(m->stream, a, grid);
         NVL_HIP(hipGetLastError());

@@ -700,6 +700,27 @@ __global__ __launch_bounds__(256) void gated_norm_kernel(GatedNormArgs p, ActT* 
     for (int c = (l + KEEP * nt) * E; c < part; c += nt * E) put(c, load(c));
 }
 
+// the same for one bf16 row by one workgroup of NT threads (a single part; 16-byte rows): part of another launch.  red: NT / 64 floats of LDS
+template <int NT>
+__device__ __forceinline__ void gated_norm_row(const GatedNormArgs& p, int64_t t, bf16_t* __restrict__ out, float* red) {
+    const float *y = p.y + t * p.y_ld, *g = p.gate + t * p.gate_ld;
+    float ss = 0.f;
+    for (int c = threadIdx.x * 4; c < p.part; c += NT * 4) { const f32x4 v = *(const f32x4*)(y + c); ss += (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]); }
+    ss = wave_sum(ss);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    ss = 0.f;
+    for (int w = 0; w < NT / 64; w++) ss += red[w];
+    const float inv = 1.0f / sqrtf(ss / (float)p.part + p.eps);
+    for (int c = threadIdx.x * 4; c < p.part; c += NT * 4) {
+        f32x4 v = *(const f32x4*)(y + c);
+        const f32x4 s = *(const f32x4*)(g + c), w = *(const f32x4*)(p.w + c);
+#pragma unroll
+        for (int r = 0; r < 4; r++) v[r] *= inv * w[r] * (p.sig ? lr_sigmoid(s[r]) : lr_silu(s[r]));
+        act_store4<bf16_t>(out, t, c, p.out_ld, v);
+    }
+}
+
 // launches (linrec_inst.hip).  ch: a decay per key channel; nk, nw: template arguments of the chunk kernel; par: pieces in parallel
 void linrec_step_launch(hipStream_t st, const LinRecArgs& p, int n_seqs, bool ch, bool fused, bool f32);
 void linrec_chunk_launch(hipStream_t st, const LinRecArgs& p, int n_seqs, bool ch, int nk, int nw, bool par);

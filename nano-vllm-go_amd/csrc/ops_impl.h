@@ -430,6 +430,7 @@ extern "C" int nvl_set_tuning(int key, int value) {
     if (key == 41) { const int old = g_pp_split; g_pp_split = value; return old; }
     if (key == 35) { const int old = g_attn_kv_nt; g_attn_kv_nt = value; return old; }
     if (key == 37) { const int old = g_grouped_split; g_grouped_split = value < 0 || value > GROUPED_SPLITS ? 0 : value; return old; }
+    if (key == 42) { const int old = g_grouped_qk; g_grouped_qk = value; return old; }
     if (key == 38) { const int old = g_mid; g_mid = value; return old; }
     if (key == 40) { const int old = g_mid_resid_rows; g_mid_resid_rows = value; return old; }
     if (key == 39) { const int old = g_mid_splits; g_mid_splits = value; return old; }
