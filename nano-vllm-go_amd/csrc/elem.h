@@ -332,12 +332,22 @@ struct SandwichArgs {
     const float* y2;          // a second source, added as it is: [slices2][.][H], or with slot_of the rows slot_of[r * slices2 + k], weighted by gate_w
     int slices2; int64_t stride2;
     const int32_t* slot_of; const float* gate_w;
+    bf16_t* xn_rows;          // tile kernel: not NULL: xn a second time, row-major
 };
 // four columns of everything that joins row r (EXT)
 __device__ __forceinline__ f32x4 sandwich_more(const SandwichArgs& p, int r, int col) {
     f32x4 a = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (p.slot_of) for (int k = 0; k < p.slices2; k++) a += p.gate_w[(int64_t)r * p.slices2 + k] * *(const f32x4*)(p.y2 + (int64_t)p.slot_of[(int64_t)r * p.slices2 + k] * p.H + col);
-    else for (int k = 0; k < p.slices2; k++) a += *(const f32x4*)(p.y2 + k * p.stride2 + (int64_t)r * p.H + col);
+    if (p.slot_of) {
+        const int32_t* slots = p.slot_of + (int64_t)r * p.slices2;
+        const float* w = p.gate_w + (int64_t)r * p.slices2;
+        for (int k0 = 0; k0 < p.slices2; k0 += 8) {      // (eight experts' rows on their way together)
+            f32x4 e[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) if (k0 + k < p.slices2) e[k] = *(const f32x4*)(p.y2 + (int64_t)slots[k0 + k] * p.H + col);
+#pragma unroll
+            for (int k = 0; k < 8; k++) if (k0 + k < p.slices2) a += w[k0 + k] * e[k];
+        }
+    } else for (int k = 0; k < p.slices2; k++) a += *(const f32x4*)(p.y2 + k * p.stride2 + (int64_t)r * p.H + col);
     return a;
 }
 // sum over the row's data columns of (x - mean)^2 held by this thread: chunk c is columns (first + c * step) * 4 ..
@@ -475,7 +485,7 @@ __global__ __launch_bounds__(1024) void sandwich_tile16_kernel(SandwichArgs p, b
     extern __shared__ __attribute__((aligned(16))) char smem_n[];
     bf16_t* tile = (bf16_t*)smem_n;                       // [16][LT]
     const int LT = tile16_pitch(p.H);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);      // (a row's slots and weights by scalar loads)
     const int r = blockIdx.x * 16 + wave, H4 = p.H >> 2;
     if (r < p.rows) {
         const int src = p.rows_idx ? p.rows_idx[r] : r;
@@ -585,6 +595,8 @@ __global__ __launch_bounds__(1024) void sandwich_tile16_kernel(SandwichArgs p, b
         }
     }
     if (!p.w_next && !p.raw_next) return;
+    if (p.xn_rows && r < p.rows)
+        for (int j = lane * 8; j < p.H; j += 512) *(bf16x8*)(p.xn_rows + (int64_t)r * p.H + j) = *(const bf16x8*)(tile + wave * LT + j);      // (its own row: no barrier)
     __syncthreads();
     const int nkb = p.H >> 5, lr = lane & 15, lc = lane >> 4;
     if (blockIdx.x * 16 + lr < p.rows)
@@ -1269,9 +1281,12 @@ __global__ __launch_bounds__(256) void moe_gather_fm_kernel(const bf16_t* __rest
     const int tok = perm[r];
     const bf16_t* s = ROWS ? src + (int64_t)tok * K + fg * 8 : src + ((int64_t)(tok >> 4) * nks * 64 + (tok & 15) + 16 * fg) * 8;
     bf16_t* d = dst + ((int64_t)blockIdx.x * nks * 64 + lane) * 8;
-    constexpr int STEP = ROWS ? 32 : 512;
+    if constexpr (!ROWS) {
+        for (int ks = wave; ks < nks; ks += 4) *(bf16x8*)(d + (int64_t)ks * 512) = *(const bf16x8*)(s + (int64_t)ks * 512);
+        return;
+    }
     for (int ks = 2 * wave; ks < nks; ks += 8) {   // (K % 64 == 0)
-        const bf16x8 x = *(const bf16x8*)(s + (int64_t)ks * STEP), y = *(const bf16x8*)(s + (int64_t)(ks + 1) * STEP);
+        const bf16x8 x = *(const bf16x8*)(s + ks * 32), y = *(const bf16x8*)(s + (ks + 1) * 32);
         *(bf16x8*)(d + (int64_t)ks * 512) = x;
         *(bf16x8*)(d + (int64_t)(ks + 1) * 512) = y;
     }

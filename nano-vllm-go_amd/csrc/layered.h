@@ -891,9 +891,11 @@ struct ExpertOut { const float* y = nullptr; int slices = 0; int64_t stride = 0;
 // token shift of the next mixer's input: its weights, the rows kept in the slots (one token per sequence: done by the same launch)
 struct ShiftOut { const float* mu = nullptr; float* state = nullptr; const Meta* md = nullptr; };
 
+// does it leave a row-major copy of xn (xn_rows) too?
+bool sandwich_copies_rows(const nvl_model* m, SubOut y, int rows) { return !m->f32 && rows > 512 && m->H <= 4096 && y.slices <= 1; }
 // x += rms(y) * w_post (w_post NULL: x += y + experts; NVL_BLOCK_SUM_NORM: x = rms(stream_scale x + y + experts) * w_post) and / or
 // xn = next(x) (elem.h SandwichArgs)
-void sandwich(nvl_model* m, SubOut y, const float* w_post, NextNorm next, void* xn, int rows, const int32_t* rows_idx = nullptr, ExpertOut ex = {}, ShiftOut sh = {}) {
+void sandwich(nvl_model* m, SubOut y, const float* w_post, NextNorm next, void* xn, int rows, const int32_t* rows_idx = nullptr, ExpertOut ex = {}, ShiftOut sh = {}, bf16_t* xn_rows = nullptr) {
     KScope ks(m, KC_OTHER, 0, KS_SANDWICH, (double)rows * m->Hn * ((y.y ? 8.0 + 4.0 * (std::max(y.slices, 1) + ex.slices) : 4.0) + (next.w || next.raw ? (double)m->wsize : 0.0)));
     SandwichArgs a{};
     a.x = m->x; a.y = y.y; a.slices = y.slices; a.slice_stride = y.stride; a.w_post = w_post; a.w_next = next.w; a.b_next = next.b; a.rows_idx = rows_idx;
@@ -902,7 +904,8 @@ void sandwich(nvl_model* m, SubOut y, const float* w_post, NextNorm next, void* 
     if (m->cfg.block_style == NVL_BLOCK_SUM_NORM && w_post) a.sum_scale = m->cfg.stream_scale;
     if (sh.mu) { a.shift = sh.mu; a.before = sh.state; a.before_stride = m->rec_slot_stride; a.seq_slot = sh.md->seq_slot; a.seq_pos = sh.md->seq_pos; }
     const bool ext = (y.y && !w_post) || next.b || a.sum_scale != 0.f || sh.mu;
-    if (!m->f32 && rows > 512 && !sh.mu && m->H <= 4096 && y.slices <= 1) {
+    a.xn_rows = xn_rows;
+    if (sandwich_copies_rows(m, y, rows) && !sh.mu) {
         const size_t lds = (size_t)16 * tile16_pitch(m->H) * 2;
 #define NVL_SW16E(CH, EXT)                                                                                                  \
         do {                                                                                                                \
@@ -1457,7 +1460,8 @@ void glu_up(nvl_model* m, const void* W, int M, int Fp, int act, float limit) {
     gemm(m, act == NVL_ACT_CLAMPED_GLU ? EPI_CLAMP_GLU : act == NVL_ACT_REGLU ? EPI_REGLU : EPI_GEGLU, false, up);
 }
 // ---- experts that read m->xn by themselves, and their shared expert: returns what is added, the rest of it in `ex` ----
-SubOut expert_ffn(nvl_model* m, const LayerRun& r, const MixerW& w, int M, ExpertOut& ex) {
+// xn_rows: a row-major copy of m->xn, or NULL (it may lie in m->moe_eo)
+SubOut expert_ffn(nvl_model* m, const LayerRun& r, const MixerW& w, int M, ExpertOut& ex, const bf16_t* xn_rows) {
     const nvl_layer_config& c = r.c;
     const int E = c.experts, k = c.top_k, pairs = M * k;
     const bool dense = !m->f32 && M <= 64 && r.Ip <= 2048;          // decode: masked projections over all experts (gemm.h GemmArgs::moe_gate)
@@ -1502,7 +1506,7 @@ SubOut expert_ffn(nvl_model* m, const LayerRun& r, const MixerW& w, int M, Exper
     const bool pp = moe_pp_ok(m, r.Ip, false);
     const int BM = pp ? 256 : ((!m->f32 && g_moe_bm == 256) ? 256 : 128);
     moe_sort(m, E, k, M, BM);
-    moe_expert_gemms(m, MoeW{E, k, r.Ip, w.moe_up, w.moe_down, c.expert_limit}, M, BM, pp, false);
+    moe_expert_gemms(m, MoeW{E, k, r.Ip, w.moe_up, w.moe_down, c.expert_limit}, M, BM, pp, false, xn_rows);
     ex = {m->moe_eo, k, 0, m->slot_of, m->expert_w};
     if (c.ffn_dim) shared();
     else {               // nothing but the experts joins
@@ -1595,10 +1599,11 @@ bool layered_stack(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len,
         if (sum || shift) {
             const bool apart = shift && !ones && li + 1 < m->L, ff = r.c.ffn_dim || r.c.experts;      // apart: the next mixer's input comes from shift_rows
             const NextNorm own{nullptr, nullptr, true}, close = apart ? NextNorm{nullptr, nullptr, false} : after;
-            sandwich(m, y, w.norm1b, ff ? own : close, m->xn, M, nullptr, {}, ff ? ShiftOut{} : shift_out(li + 1));
+            bf16_t* xn_rows = r.c.experts && sandwich_copies_rows(m, y, M) ? (bf16_t*)m->moe_eo : nullptr;      // (for the copy into expert order)
+            sandwich(m, y, w.norm1b, ff ? own : close, m->xn, M, nullptr, {}, ff ? ShiftOut{} : shift_out(li + 1), xn_rows);
             if (ff) {
                 ExpertOut ex;
-                if (r.c.experts) y = expert_ffn(m, r, w, M, ex);
+                if (r.c.experts) y = expert_ffn(m, r, w, M, ex, xn_rows);
                 else { glu_up(m, w.w1, M, r.Fp, r.act, r.c.ffn_limit); y = sub_out(m, KS_FFN_DOWN, m->hbuf, w.w2, M, r.Fp); }
                 sandwich(m, y, w.norm2b, close, m->xn, M, nullptr, ex, shift_out(li + 1));
             }
