@@ -550,8 +550,8 @@ int nvl_bench_gemm(int device, int M, int N, int K, int epi, int force_bnt, int 
  * 8 = wide-N form (4 weight tiles per wave).
  * key 3: deferred RMSNorm in decode (0 off, 1 on, 2 on without the activation-tile split, 3 only the O-proj -> FFN-up seam).
  * keys 4-6 (sweeps): K split of the wide form, waves per narrow-form launch, K split of the deferred-norm residual
- * projections.  key 7: decode seam kernel, 8: MoE small-batch fusion, 9: 16-row norm kernel, 10: prefill attention
- * with 128 query rows per workgroup (0 never, 1 automatic, 2 always).  keys 11-14: decode batches of 65..512 rows (key 11, default 512; 64 = off) run the
+ * projections.  key 7: decode seam kernel, 8: MoE small-batch fusion, 9: 16-row norm kernel, 10: query rows per
+ * workgroup of the prefill attention (0: 256, 1 from their number, 2: 128, 3: 64).  keys 11-14: decode batches of 65..512 rows (key 11, default 512; 64 = off) run the
  * projections whose 128x128 tile grid has fewer than key 12 (160) workgroups as ceil(M/64) groups of 64 rows of the
  * decode GEMM form, in one launch interleaved over the weight blocks (key 13 = 1) or one launch per group (0); up to
  * key 14 rows (64) every projection does.  key 15: waves per decode-attention workgroup (0 = from context length and

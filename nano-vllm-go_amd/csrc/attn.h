@@ -127,19 +127,19 @@ __device__ __forceinline__ float rows_max(float x) {
 }
 
 // ------------------------------------------------------------------------------------------
-// bf16 prefill kernel.  One workgroup = 8 waves = 256 query rows of one (sequence, kv head); each wave owns 32 rows as
-// two 16-row sub-tiles, so every K / V fragment read from LDS feeds two MFMAs.  K and V tiles (64 keys) stream
+// bf16 prefill kernel.  One workgroup = NW waves of TQ 16-row sub-tiles = 256, 128 or 64 query rows of one (sequence, kv head) (which:
+// attn_prefill_rows); with two sub-tiles every K / V fragment read from LDS feeds two MFMAs.  K and V tiles (64 keys) stream
 // HBM -> LDS by LDS-DMA through a 3-slot ring, two tiles ahead of the compute, with ONE barrier per tile:
 //     wait (my pieces of tile kt landed)  |  barrier  |  issue tile kt+2 into the slot tile kt-1 used  |  compute tile kt
 // (a slot is re-filled only after every wave passed the barrier that follows its last read; LDS-DMA is ordered by the
 // issuing wave's vmcnt + that barrier).  hd 64: four waves per SIMD (two workgroups per CU), so one wave's softmax VALU
 // runs beside another's MFMAs; hd 128: two.
 // ------------------------------------------------------------------------------------------
-template <int HD>
-__global__ __launch_bounds__(512, HD == 64 ? 4 : 2) void attn_prefill_bf16_kernel(AttnArgs p) {
-    constexpr int KS = HD / 32, DT = HD / 16, CPR = HD / 8, TQ = 2;
-    constexpr int TILE_BYTES = 64 * HD * 2, PIECES = TILE_BYTES / 1024, PW = 2 * PIECES / 8, NBUF = 3;
-    constexpr int QROWS = 256;
+template <int HD, int TQ, int NW>
+__global__ __launch_bounds__(NW * 64, HD == 64 ? 4 : 2) void attn_prefill_bf16_kernel(AttnArgs p) {
+    constexpr int KS = HD / 32, DT = HD / 16, CPR = HD / 8;
+    constexpr int TILE_BYTES = 64 * HD * 2, PIECES = TILE_BYTES / 1024, PW = 2 * PIECES / NW, NBUF = 3;
+    constexpr int QROWS = NW * TQ * 16;
     extern __shared__ __attribute__((aligned(16))) char smem[];     // NBUF x [K image | V image]
     __shared__ int32_t sblk[128];          // this sequence's block table (<= 128 blocks: host-checked)
 
@@ -189,8 +189,8 @@ __global__ __launch_bounds__(512, HD == 64 ? 4 : 2) void attn_prefill_bf16_kerne
     if (last_row > R - 1) last_row = R - 1;
     const int n_kt = (pos0 + last_row / p.group) / 64 + 1;
     // key tiles this WAVE needs: up to its last valid row's causal limit (none when the wave has no valid row)
-    const int w_row0 = qt * QROWS + wave * 32;
-    int w_last = w_row0 + 31;
+    const int w_row0 = qt * QROWS + wave * (TQ * 16);
+    int w_last = w_row0 + TQ * 16 - 1;
     if (w_last > R - 1) w_last = R - 1;
     const int wave_n_kt = w_row0 < R ? (pos0 + w_last / p.group) / 64 + 1 : 0;
     const int wave_first_limit = pos0 + w_row0 / p.group;     // tiles wholly below it need no masking
@@ -246,7 +246,9 @@ __global__ __launch_bounds__(512, HD == 64 ? 4 : 2) void attn_prefill_bf16_kerne
         // my pieces of tile kt have landed (tile kt+1's may stay in flight)
         if (kt + 1 < n_kt) {
             if (PW == 2) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
-            else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+            else if (PW == 4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+            else asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+            static_assert(PW == 2 || PW == 4 || PW == 8, "pieces of a tile per wave");
         } else {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }

@@ -1227,7 +1227,7 @@ static int g_p2p_oneshot_rows = 64;   // nvl_set_tuning key 23: payloads of up t
 static int g_use_graphs = 1;   // nvl_set_tuning key 21: hipGraph replay of decode passes (0 = every launch eager)
 static int g_tune_epoch = 0;   // bumped by every nvl_set_tuning: captured graphs bake the tuning in (part of their key)
 static int g_attn_nw = 0;      // nvl_set_tuning key 15: waves per decode-attention workgroup (0 = from the context length, 2, 4, 8)
-static int g_attn_tq2 = 1;     // nvl_set_tuning key 10: unused since round 2 (the prefill kernel always keeps two sub-tiles per wave)
+static int g_attn_rows = 1;    // nvl_set_tuning key 10: query rows per workgroup of the prefill attention (0: 256, 1: from their number, 2: 128, 3: 64)
 static int g_attn_kv_nt = 1;   // nvl_set_tuning key 35: non-temporal K/V loads in the decode attention (0 never, 1 automatic, 2 always)
 static int g_attn_split = 1;   // nvl_set_tuning key 25: split a decode attention's keys over up to 8 workgroups per (sequence, kv head) (0 = never)
 // Launch shape of the decode attention for the batch being enqueued (also part of a captured graph's key): waves per
@@ -1254,7 +1254,18 @@ int decode_attn_cfg(const nvl_model* m, int n_seqs) {
 }
 int layered_decode_key(const nvl_model* m);
 int decode_attn_waves(const nvl_model* m, int n_seqs) { return m->layered ? layered_decode_key(m) : decode_attn_cfg(m, n_seqs); }   // (graph keys: the whole shape)
-void attention(nvl_model* m, int li, const Meta& md, int n_seqs, int max_len, double flops, bool fused_qkv = false) {
+// Query rows per workgroup of the prefill attention.  A workgroup walks its key tiles one after the other, so that short calls are a serial
+// chain on a part of the chip: fewer rows a wave shorten each tile, fewer waves a workgroup spread them.  256 / 128 / 64 rows, us:
+//   heads of 64:  487 x 32 heads 17.7 / 13.2 / 11.4, 1900 x 32 52 / 36 / 32, 4 x 487 x 32 20.3 / 16.4 / 16.9, 12 x 487 x 32 34.7 / 30.8 / 35.3,
+//                 4 x 1900 x 32 90.8 / 89.1 / 100.7, 32 x 512 x 32 75.0 / 77.4 / 93.1
+//   heads of 128 (one workgroup a CU): worth it while one round holds them all: 487 x 32 23.7 / 20.3 / 17.1, 2 x 1400 x 32 59.7 / 72.3 / 102.9
+int attn_prefill_rows(const nvl_model* m, int n_seqs, int M) {
+    if (g_attn_rows != 1) return g_attn_rows == 0 ? 256 : g_attn_rows == 2 ? 128 : 64;
+    const int64_t rows = (int64_t)M * m->group * m->nKV, ragged = (int64_t)n_seqs * m->nKV;
+    if (m->hd == 64) return rows < 65536 ? 64 : rows < 262144 ? 128 : 256;
+    return rows / 64 + ragged <= 256 ? 64 : rows / 128 + ragged <= 256 ? 128 : 256;
+}
+void attention(nvl_model* m, int li, const Meta& md, int n_seqs, int M, int max_len, double flops, bool fused_qkv = false) {
     AttnArgs a{};
     a.q = m->q; a.q_stride = m->nH * m->hd;
     a.out = m->attn_out; a.out_stride = m->nH * m->hd;
@@ -1311,16 +1322,23 @@ void attention(nvl_model* m, int li, const Meta& md, int n_seqs, int max_len, do
 #undef NVL_DEC
 #undef NVL_DEC_LEAD
     } else {
-        // 256 query rows (position x head-in-group, position-major) per workgroup of 8 waves; K/V tiles by LDS-DMA
+        // query rows (position x head-in-group, position-major) in workgroups of 4 or 8 waves; K/V tiles by LDS-DMA
         const int64_t qrows = (int64_t)max_len * m->group;
         if (m->blocks_per_seq > 128) throw std::runtime_error("attention: more than 128 KV blocks per sequence");
-        dim3 grid(m->nKV, n_seqs, cdiv(qrows, 256));      // (kv head fastest, query tile slowest: attn.h)
-        if (m->hd == 64) {
-            hipLaunchKernelGGL((attn_prefill_bf16_kernel<64>), grid, dim3(512), attn_prefill_lds_bytes<64>(), m->stream, a);
-        } else {
-            NVL_LDS_ATTR(attn_prefill_bf16_kernel<128>, attn_prefill_lds_bytes<128>());
-            hipLaunchKernelGGL((attn_prefill_bf16_kernel<128>), grid, dim3(512), attn_prefill_lds_bytes<128>(), m->stream, a);
-        }
+        const int rows = attn_prefill_rows(m, n_seqs, M);
+        dim3 grid(m->nKV, n_seqs, cdiv(qrows, rows));      // (kv head fastest, query tile slowest: attn.h)
+#define NVL_PRE(HDv)                                                                                                   \
+        do {                                                                                                           \
+            constexpr int lds = attn_prefill_lds_bytes<HDv>();                                                         \
+            NVL_LDS_ATTR((attn_prefill_bf16_kernel<HDv, 2, 8>), lds);                                                  \
+            NVL_LDS_ATTR((attn_prefill_bf16_kernel<HDv, 1, 8>), lds);                                                  \
+            NVL_LDS_ATTR((attn_prefill_bf16_kernel<HDv, 1, 4>), lds);                                                  \
+            if (rows == 256) hipLaunchKernelGGL((attn_prefill_bf16_kernel<HDv, 2, 8>), grid, dim3(512), lds, m->stream, a);      \
+            else if (rows == 128) hipLaunchKernelGGL((attn_prefill_bf16_kernel<HDv, 1, 8>), grid, dim3(512), lds, m->stream, a); \
+            else hipLaunchKernelGGL((attn_prefill_bf16_kernel<HDv, 1, 4>), grid, dim3(256), lds, m->stream, a);                  \
+        } while (0)
+        if (m->hd == 64) NVL_PRE(64); else NVL_PRE(128);
+#undef NVL_PRE
     }
     NVL_HIP(hipGetLastError());
 }
@@ -1976,7 +1994,7 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
             fused_dec = !m->f32 && max_len == 1;     // decode: RoPE + KV append live in the attention kernel
             if (!fused_dec) rope_kv(m, li, md, M);
         }
-        attention(m, li, md, n_seqs, max_len, attn_flops, fused_dec);
+        attention(m, li, md, n_seqs, M, max_len, attn_flops, fused_dec);
         const float* bo = (const float*)l.t[NVL_T_BO].p;
         if (parallel) {
             // generic_model.go:395-418: r + [am*]attn + [rm*]ffn, both branches read the same normed x

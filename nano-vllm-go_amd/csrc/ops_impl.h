@@ -202,7 +202,7 @@ extern "C" int nvl_op_attention(int device, int precision, const float* q, const
     Meta md{};
     md.seq_tok_start = dmeta; md.seq_len = dmeta + 1; md.seq_pos = dmeta + 2; md.seq_tbl = dmeta + 3; md.blk_table = dmeta + 4;
     m.blocks_per_seq = 1;
-    attention(&m, 0, md, 1, S, 0.0);
+    attention(&m, 0, md, 1, S, S, 0.0);
     // back to fp32 [nH, S, hd]
     std::vector<float> ot((size_t)S * nH * hd);
     if (m.f32) {
@@ -413,7 +413,7 @@ extern "C" int nvl_set_tuning(int key, int value) {
     if (key == 13) { const int old = g_pass_interleave; g_pass_interleave = value; return old; }
     if (key == 12) { const int old = g_chunk_min_tiles; g_chunk_min_tiles = value; return old; }
     if (key == 11) { const int old = g_chunk_max_m; g_chunk_max_m = value; return old; }
-    if (key == 10) { const int old = g_attn_tq2; g_attn_tq2 = value; return old; }
+    if (key == 10) { const int old = g_attn_rows; g_attn_rows = value; return old; }
     if (key == 9) { const int old = g_norm_t16; g_norm_t16 = value; return old; }
     if (key == 8) { const int old = g_moe_small; g_moe_small = value; return old; }
     if (key == 7) { const int old = g_decode_seam; g_decode_seam = value; return old; }

@@ -211,3 +211,17 @@ def test_short_prompts_place_their_heads(gpu, family, hd, lens):
         gpu.lib().nvl_set_tuning(18, old)
     m.close()
     assert rel_err(got[0][0], got[1][0]) <= TOL and rel_err(got[0][1], got[1][1]) <= TOL
+
+
+@pytest.mark.parametrize("rows", [0, 2, 3])                          # 256, 128, 64 query rows per workgroup
+@pytest.mark.parametrize("nH,nKV,S,T,hd", [(4, 2, 5, 5, 64), (2, 2, 33, 100, 64), (3, 1, 7, 64, 128), (71, 1, 2, 130, 64), (8, 2, 130, 130, 128),
+                                           (4, 2, 300, 1400, 64), (4, 2, 65, 257, 128), (1, 1, 64, 64, 64), (1, 1, 129, 200, 128)])
+def test_prefill_attention_rows(gpu, oracle, rows, nH, nKV, S, T, hd):
+    """Ragged row counts, waves without a row, diagonal and whole key tiles, more of them than the LDS ring holds; the same products whatever
+    the workgroup's rows: only the last tiles of the other rows differ, and those are masked."""
+    r = np.random.default_rng(nH * 10 + T)
+    q, k, v = (r.standard_normal(s, dtype=np.float32) for s in ((nH, S, hd), (nKV, T, hd), (nKV, T, hd)))
+    old = gpu.lib().nvl_set_tuning(10, rows)
+    got = gpu.ops.attention(q, k, v, precision="bf16")
+    gpu.lib().nvl_set_tuning(10, old)
+    assert rel_err(got, oracle.gqa_core(q, k, v)) <= TOL
