@@ -47,14 +47,17 @@ struct AttnArgs {
     int qkv_stride;
     const float* cos_t;   // [max_seq][HD] or NULL
     const float* sin_t;
-    // decode kernel with gridDim.z > 1 (keys split over workgroups): workgroup z leaves its partial result here —
-    // [(seq * gridDim.x + blockIdx.x) * gridDim.z + z] records of {O^T [HD/16][64 lanes] f32x4 (unnormalised), m[16], l[16]} — and
-    // takes a ticket from part_cnt[seq * gridDim.x + blockIdx.x]; the workgroup that draws the last one combines them in z order.
+    // decode kernel, keys split over workgroups: a sequence of n key tiles is dealt over min(split_max, ceil(n / split_tiles)) of the
+    // split_max = gridDim.z workgroups of its (kv head, query tile), the others return.  Of several, workgroup z leaves its partial result in
+    // [(seq * gridDim.x + blockIdx.x) * split_max + z] records of {O^T [HD/16][64 lanes] f32x4 (unnormalised), m[16], l[16]} and
+    // takes a ticket from part_cnt[seq * gridDim.x + blockIdx.x]; the one that draws the last combines them in z order.
+    int split_max, split_tiles;
     float* part;
     int32_t* part_cnt;    // zero between launches
     unsigned long long* stamps;   // diagnostic runs: per-workgroup time stamps (common.h nvl_stamp), else NULL
     int kv_nt;                    // decode: non-temporal K/V loads (set by the host: attention() in nvllm.hip)
 };
+constexpr int ATTN_SPLIT_MAX = 8;      // most workgroups the keys of a (sequence, kv head) are split over
 template <int HD> constexpr int attn_part_floats() { return (HD / 16) * 64 * 4 + 32; }
 
 // index of the KV block that holds key `key`
@@ -417,27 +420,45 @@ __device__ __forceinline__ void rope_math8(const RopeRaw& r, bool rot, bf16x8& l
     }
 }
 
+// partial results go past the L2 of this XCD and are read past the reader's (sc0 sc1): no cache has to be written back or invalidated
+__device__ __forceinline__ void part_store(float* base, int64_t floats, f32x4 v) {
+    union { f32x4 f; u32x4 u; } t; t.f = v;
+    __builtin_amdgcn_raw_buffer_store_b128(t.u, __builtin_amdgcn_make_buffer_rsrc(base, 0, 1 << 30, 0x00020000), (int)(floats * 4), 0, 0x11);
+}
+__device__ __forceinline__ f32x4 part_load(const float* base, int64_t floats) {
+    union { f32x4 f; u32x4 u; } t;
+    t.u = __builtin_amdgcn_raw_buffer_load_b128(__builtin_amdgcn_make_buffer_rsrc((void*)base, 0, 1 << 30, 0x00020000), (int)(floats * 4), 0, 0x11);
+    return t.f;
+}
 // combine of a split decode launch: the nsplit partial results of one (sequence, kv head, query tile), in workgroup order
 // whichever workgroup runs it.  One wave, the lanes of real heads; lane (fq, fg) as in the kernel's own combine.
 template <int HD>
 __device__ __forceinline__ void attn_decode_merge(const AttnArgs& p, int pair, int tok, int head, int nsplit, int lane) {
     constexpr int DT = HD / 16;
     const int fq = lane & 15, fg = lane >> 4;
-    const float* rec0 = p.part + (int64_t)pair * nsplit * attn_part_floats<HD>();
-    float mstar = -INFINITY;
-    for (int z = 0; z < nsplit; z++) mstar = fmaxf(mstar, rec0[(int64_t)z * attn_part_floats<HD>() + DT * 256 + fq]);
-    float L = 0.f;
+    // (a record ends in m | l of its 16 rows, four rows a lane group: (m, l) of row fq by two loads of four)
+    const float* rec0 = p.part + (int64_t)pair * p.split_max * attn_part_floats<HD>();
+    float mz[ATTN_SPLIT_MAX], lz[ATTN_SPLIT_MAX], mstar = -INFINITY, L = 0.f;
+#pragma unroll
+    for (int z = 0; z < ATTN_SPLIT_MAX; z++) {
+        if (z >= nsplit) break;
+        const int at = z * attn_part_floats<HD>() + DT * 256 + (fq & ~3);
+        const f32x4 m4 = part_load(rec0, at), l4 = part_load(rec0, at + 16);
+        mz[z] = fq & 2 ? (fq & 1 ? m4[3] : m4[2]) : (fq & 1 ? m4[1] : m4[0]);
+        lz[z] = fq & 2 ? (fq & 1 ? l4[3] : l4[2]) : (fq & 1 ? l4[1] : l4[0]);
+    }
     f32x4 O[DT];
 #pragma unroll
     for (int d = 0; d < DT; d++) O[d] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int z = 0; z < nsplit; z++) {
-        const float* rec = rec0 + (int64_t)z * attn_part_floats<HD>();
-        const float mz = rec[DT * 256 + fq];
-        if (mz == -INFINITY) continue;                 // that workgroup had no tile
-        const float sc = __builtin_amdgcn_exp2f(mz - mstar);
-        L += rec[DT * 256 + 16 + fq] * sc;
 #pragma unroll
-        for (int d = 0; d < DT; d++) O[d] += ((const f32x4*)rec)[d * 64 + lane] * sc;
+    for (int z = 0; z < ATTN_SPLIT_MAX; z++) if (z < nsplit) mstar = fmaxf(mstar, mz[z]);
+#pragma unroll
+    for (int z = 0; z < ATTN_SPLIT_MAX; z++) {
+        if (z >= nsplit) break;
+        const float sc = __builtin_amdgcn_exp2f(mz[z] - mstar);      // (no tile: m = -inf, O = l = 0)
+        L += lz[z] * sc;
+#pragma unroll
+        for (int d = 0; d < DT; d++) O[d] += part_load(rec0, z * attn_part_floats<HD>() + (d * 64 + lane) * 4) * sc;
     }
     const float inv = 1.0f / L;
 #pragma unroll
@@ -472,13 +493,12 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t
     // wave's first tiles (which do not depend on the position).  Left to itself the compiler sinks the block-id loads behind
     // the position's wait and the tile-count branch (two more dependent scalar round trips before the first vector load:
     // +0.7 us per launch at B = 1).
-    constexpr int NT2_ = HD <= 64 ? 2 : 1;
-    const int vw_ = blockIdx.z * NW + wave, nvw_ = NW * gridDim.z;
+    const int vw = blockIdx.z * (NW * NT2) + wave;          // this wave's first tile; the others of its round are NW apart
     const int tok = seq, pos0 = a_seq_pos[seq];              // (decode launches carry one token per sequence, in sequence order)
-    int first_blk[NT2_];
+    int first_blk[NT2];
 #pragma unroll
-    for (int h = 0; h < NT2_; h++) {
-        const int key = (vw_ + h * nvw_) * 64;
+    for (int h = 0; h < NT2; h++) {
+        const int key = (vw + h * NW) * 64;
         const int bi = a_bs_shift >= 0 ? (key >> a_bs_shift) : key / a_Tmax;
         first_blk[h] = tbl[min(bi, a_tbl_stride - 1)];
     }
@@ -489,10 +509,10 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t
     char* vimg = smem + wave * TILE_BYTES;
     bf16x8 qf[KS];
     const int n_kt = pos0 / 64 + 1;
-    // key tiles are dealt round-robin over "virtual waves": the NW waves of each of the gridDim.z workgroups of this
-    // (sequence, kv head).  gridDim.z > 1 (long contexts in small batches: one workgroup would pull the whole K/V of its
-    // head through one CU, ~50 GB/s) leaves partial results for attn_decode_merge_kernel.
-    const int vw = blockIdx.z * NW + wave, nvw = NW * gridDim.z;
+    // rounds of NW x NT2 key tiles are dealt over the nz workgroups of this (sequence, kv head) in turn (one workgroup pulls all K/V of its
+    // head through one CU, ~50 GB/s, one round after the other)
+    const int nz = p.split_max == 1 ? 1 : min(p.split_max, (n_kt + p.split_tiles - 1) / p.split_tiles), stride = NW * NT2 * nz;
+    if ((int)blockIdx.z >= nz) return;
     // (FUSED: the new token's q / k / v are fetched and rotated AFTER the first round's K/V loads are issued: below)
     bf16x8 knew[KS];
     bf16x8 vnew8;
@@ -520,7 +540,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t
         constexpr bool NT = decltype(nt_tag)::value;
 #pragma unroll
         for (int h = 0; h < NT2; h++) {
-            const int kt = kt0 + h * nvw;
+            const int kt = kt0 + h * NW;
             if (kt >= n_kt) continue;
             const int bi = kv_block_index(p, kt * 64), krow0 = kt * 64 - bi * p.Tmax;     // the KV block holding this tile
             const int blk = kt0 == vw ? first_blk[h] : tbl[bi];
@@ -613,7 +633,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t
         float tmax = -INFINITY;
 #pragma unroll
         for (int h = 0; h < NT2; h++) {
-            const int kt = kt0 + h * nvw;
+            const int kt = kt0 + h * NW;
             if (kt >= n_kt) {
 #pragma unroll
                 for (int t = 0; t < 4; t++) s[h][t] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
@@ -671,7 +691,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t
         // MFMA operand (ds_read_b64_tr_b16); a wave's LDS accesses execute in order, so no barrier ----
 #pragma unroll
         for (int h = 0; h < NT2; h++) {
-            if (kt0 + h * nvw >= n_kt) continue;
+            if (kt0 + h * NW >= n_kt) continue;
 #pragma unroll
             for (int i = 0; i < NVL; i++) *(bf16x8*)(vimg + w_base[i & 1] + i * (16 * KPI * CPR)) = vch[h][i];
 #pragma unroll
@@ -692,7 +712,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t
         }
     };
     if (vw < n_kt) do_round(vw);
-    for (int kt0 = vw + NT2 * nvw; kt0 < n_kt; kt0 += NT2 * nvw) {
+    for (int kt0 = vw + stride; kt0 < n_kt; kt0 += stride) {
         issue_round(kt0);
         do_round(kt0);
     }
@@ -719,7 +739,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t
     for (int d = 0; d < DT; d++) my_o[d * 64 + lane] = o[d];
     __syncthreads();
     stamps.mark(4);                     // every wave's tiles done
-    if (gridDim.z == 1 && NW >= DT) {
+    if (nz == 1 && NW >= DT) {
         // whole (sequence, kv head) in this workgroup: wave d combines output block d (same sums, same order as below;
         // one wave doing all DT blocks: B = 32 33.55 K -> 33.80 K decode tok/s, B = 8 +0.9 %, same-box A/B)
         if (wave >= DT || !row_ok) return;
@@ -755,23 +775,26 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t
             for (int d = 0; d < DT; d++) O[d] += wo[d * 64 + lane] * sc;
         }
     }
-    if (gridDim.z > 1) {
+    if (nz > 1) {
         const int pair = seq * gridDim.x + blockIdx.x;               // (sequence, kv head, query tile)
-        float* rec = p.part + ((int64_t)pair * gridDim.z + blockIdx.z) * attn_part_floats<HD>();
+        float* rec = p.part + ((int64_t)pair * p.split_max + blockIdx.z) * attn_part_floats<HD>();
 #pragma unroll
-        for (int d = 0; d < DT; d++) ((f32x4*)rec)[d * 64 + lane] = O[d];
-        if (fg == 0) { rec[DT * 256 + fq] = mstar; rec[DT * 256 + 16 + fq] = L; }
-        // Last arriver combines (no second launch: a merge kernel cost 5-7 us of the 8-11 the split saves).  Release my
-        // record device-wide (the workgroups of a pair may sit on different XCDs, whose L2s are not coherent), draw a
-        // ticket, and if it is the last one acquire the others' records.  The order of the sum is z order regardless.
-        __threadfence();
+        for (int d = 0; d < DT; d++) part_store(rec, (d * 64 + lane) * 4, O[d]);
+        // (m and l of four rows by the lane of the first: 16-byte stores)
+        f32x4 m4, l4;
+#pragma unroll
+        for (int r = 0; r < 4; r++) { m4[r] = __shfl(mstar, (lane & ~3) + r, 64); l4[r] = __shfl(L, (lane & ~3) + r, 64); }
+        if (fg == 0 && (fq & 3) == 0) { part_store(rec, DT * 256 + fq, m4); part_store(rec, DT * 256 + 16 + fq, l4); }
+        // Last arriver combines (no second launch: a merge kernel cost 5-7 us of the 8-11 the split saves); the order of the sum is z
+        // order regardless.
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // the record has reached memory
         int ticket = 0;
         int32_t* cnt = p.part_cnt + pair;
         if (lane == 0) ticket = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         ticket = __builtin_amdgcn_readfirstlane(ticket);
-        if (ticket != (int)gridDim.z - 1) return;
-        __threadfence();
-        attn_decode_merge<HD>(p, pair, tok, head, gridDim.z, lane);
+        if (ticket != nz - 1) return;
+        asm volatile("" ::: "memory");
+        attn_decode_merge<HD>(p, pair, tok, head, nz, lane);
         if (lane == 0) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);    // for the next launch
         return;
     }

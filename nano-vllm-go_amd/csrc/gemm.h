@@ -541,7 +541,6 @@ void gemm_bf16_kernel(GemmArgs p) {
 // written through and read past the L2 (sc0 sc1) instead of fencing, which would write back everything that XCD has dirty
 // (4096 x 2048 x 6144 in two parts: 85 us so, 156 us with __threadfence, 94 us unsplit).
 // ------------------------------------------------------------------------------------------
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 constexpr int64_t SPLIT_WS_BYTES = 64ll << 20;      // 256 parts of 256 x 256 fp32, or 512 of 128 x 128
 constexpr int SPLIT_MAX_TILES = 512;
 constexpr int SPLIT_COHERENT = 0x11;      // buffer cache policy: sc0 | sc1

@@ -17,7 +17,7 @@
 using namespace nvl;
 
 static thread_local std::string g_create_err;
-constexpr int ATTN_SPLIT_MAX_PAIRS = 32, ATTN_SPLIT_MAX = 8;     // split decode attention: (sequence, kv head) pairs a launch may have; most workgroups per pair
+constexpr int ATTN_SPLIT_RECORDS = 4096;      // split decode attention: most partial results of a launch (17 / 34 MB)
 constexpr int SK_TILE_MAX_M = 2048, SK_TILE_MAX_SLICES = 8;      // split-K of the tile kernel for mid-size residual projections (resid_gemm)
 static int g_sk_tile = 1;            // nvl_set_tuning key 26: that split (0 = off)
 constexpr int MOE_DOWN_SLICES = 4;    // at most this many K slices (workgroups per column tile) in the dense-masked MoE down projection
@@ -848,9 +848,9 @@ extern "C" int nvl_finalize(nvl_model* m) {
     m->q = dmalloc_bytes(Mmax * qw * (int64_t)m->wsize);
     m->attn_out = dmalloc_bytes(Mp * qw * (int64_t)m->wsize);
     if (!m->f32 && (m->hd == 64 || m->hd == 128)) {     // partial results of a split decode attention (attn.h)
-        m->attn_part = dmalloc<float>((int64_t)ATTN_SPLIT_MAX_PAIRS * ATTN_SPLIT_MAX * (m->hd == 64 ? attn_part_floats<64>() : attn_part_floats<128>()));
-        m->attn_part_cnt = dmalloc<int32_t>(ATTN_SPLIT_MAX_PAIRS);
-        NVL_HIP(hipMemset(m->attn_part_cnt, 0, ATTN_SPLIT_MAX_PAIRS * sizeof(int32_t)));
+        m->attn_part = dmalloc<float>((int64_t)ATTN_SPLIT_RECORDS * (m->hd == 64 ? attn_part_floats<64>() : attn_part_floats<128>()));
+        m->attn_part_cnt = dmalloc<int32_t>(ATTN_SPLIT_RECORDS);
+        NVL_HIP(hipMemset(m->attn_part_cnt, 0, ATTN_SPLIT_RECORDS * sizeof(int32_t)));
     }
     const int64_t k = c.use_moe ? c.num_experts_per_tok : 1;
     m->hbuf = dmalloc_bytes(round_up(Mmax * k, 64) * m->F * (int64_t)m->wsize);
@@ -1229,28 +1229,32 @@ static int g_tune_epoch = 0;   // bumped by every nvl_set_tuning: captured graph
 static int g_attn_nw = 0;      // nvl_set_tuning key 15: waves per decode-attention workgroup (0 = from the context length, 2, 4, 8)
 static int g_attn_rows = 1;    // nvl_set_tuning key 10: query rows per workgroup of the prefill attention (0: 256, 1: from their number, 2: 128, 3: 64)
 static int g_attn_kv_nt = 1;   // nvl_set_tuning key 35: non-temporal K/V loads in the decode attention (0 never, 1 automatic, 2 always)
-static int g_attn_split = 1;   // nvl_set_tuning key 25: split a decode attention's keys over up to 8 workgroups per (sequence, kv head) (0 = never)
+static int g_attn_split = 1;   // nvl_set_tuning key 25: split a decode attention's keys over up to 8 workgroups per (sequence, kv head) (0 never, 1 automatic, 1 + n: n rounds each)
 // Launch shape of the decode attention for the batch being enqueued (also part of a captured graph's key): waves per
-// workgroup | workgroups per (sequence, kv head) << 8.
-// Split: a workgroup pulls all K/V of its (sequence, kv head) through ONE CU; with a few sequences and a long context
-// (B = 1 at 2048 keys: 8 workgroups x 512 KB) that, not HBM, is the time.  Then the key tiles are dealt over up to 8
-// workgroups of 2 waves each; the last of them to finish combines the partial results (attn.h).  Every workgroup of a
-// split launch pays a device-scope release fence, so the launch stays within 128 workgroups.  Measured (decode ms/step,
-// Llama-3.2-1B, 2048 / 1024 keys): B=1 0.891 -> 0.811 / 0.808 -> 0.780, B=2 0.893 -> 0.834 / 0.869 -> 0.792, B=4 (4
-// workgroups per pair) 0.924 -> 0.883 / 0.812 -> 0.817 (hence from 2048 keys on above 16 pairs); B=8 loses either way
-// (2 workgroups per pair 0.96 -> 0.99, 8 per pair -> 1.13).
+// workgroup | most workgroups per (sequence, kv head) << 8 | key tiles a workgroup has at least << 12.
+// Split: a workgroup pulls all K/V of its (sequence, kv head) through ONE CU, one round of tiles after the other; with few of
+// them and a long context that, not HBM, is the time.  A sequence is then dealt over workgroups of one round each (attn.h), and the
+// last of them combines the parts: about 2 us, so that contexts of one round stay whole.  Beyond 128 pairs the launch fills the
+// chip and a split only adds traffic.  us per launch whole / split, Llama-3.2-1B (8 kv heads of 64): 1 x 700 keys 11.6 / 10.6,
+// 4 x 1800 16.9 / 12.8, 8 x 1800 20.1 / 15.6, 8 x 300..1800 17.9 / 13.1, 16 x 200..1000 13.5 / 12.8, but 12 x 600 10.7 / 12.0,
+// 32 x 1500 23.2 / 27.0; Llama-3-8B (8 of 128): 1 x 700 15.2 / 13.0, 8 x 1500 27.0 / 20.1, 16 x 300..1200 22.2 / 25.3.
 int decode_attn_cfg(const nvl_model* m, int n_seqs) {
     const int n_kt = m->ctx_hint > 0 ? (m->ctx_hint - 1) / 64 + 1 : 1 << 20;
     const int per_wave = m->hd == 64 ? 2 : 1;
     const int wgs = m->nKV * cdiv(m->group, 16) * n_seqs;
-    if (g_attn_split && !g_attn_nw && m->attn_part && m->ctx_hint > 0 && wgs <= ATTN_SPLIT_MAX_PAIRS && n_kt >= 16) {
-        const int want = cdiv(n_kt, 2 * per_wave);                       // workgroups of 2 waves that get a full round each
-        const int ns = (wgs > 16 && n_kt < 32) ? 1 : std::min(std::min(want, ATTN_SPLIT_MAX), 128 / wgs);
-        if (ns >= 2) return 2 | (ns << 8);
-    }
     const int cap = wgs >= 512 ? 2 : (wgs >= 320 ? 4 : 8);
-    const int nw = n_kt <= 2 * per_wave ? 2 : (n_kt <= 4 * per_wave ? 4 : 8);
-    return (g_attn_nw ? g_attn_nw : std::min(nw, cap)) | (1 << 8);
+    int nw = n_kt <= 2 * per_wave ? 2 : (n_kt <= 4 * per_wave ? 4 : 8);
+    nw = g_attn_nw ? g_attn_nw : std::min(nw, cap);
+    auto cfg = [&](int waves, int most, int tiles) { return waves | most << 8 | tiles << 12; };
+    const int most = m->attn_part && m->ctx_hint > 0 ? std::min(ATTN_SPLIT_MAX, ATTN_SPLIT_RECORDS / wgs) : 1;
+    if (g_attn_split >= 2) { const int tiles = (g_attn_split - 1) * nw * per_wave; return cfg(nw, std::max(1, std::min(most, cdiv(n_kt, tiles))), tiles); }
+    if (g_attn_split && !g_attn_nw && most > 1) {
+        int waves = 0;
+        if (m->hd == 64) waves = wgs <= 48 ? (n_kt > 16 ? 4 : n_kt > 8 ? 2 : 0) : wgs <= 128 && n_kt > 12 ? 4 : 0;
+        else waves = wgs <= 32 ? (n_kt > 16 ? 4 : n_kt > 5 ? 2 : 0) : wgs <= 96 && n_kt > 8 ? 8 : 0;
+        if (waves) return cfg(waves, std::min(most, cdiv(n_kt, waves * per_wave)), waves * per_wave);
+    }
+    return cfg(nw, 1, 1 << 16);
 }
 int layered_decode_key(const nvl_model* m);
 int decode_attn_waves(const nvl_model* m, int n_seqs) { return m->layered ? layered_decode_key(m) : decode_attn_cfg(m, n_seqs); }   // (graph keys: the whole shape)
@@ -1282,7 +1286,8 @@ void attention(nvl_model* m, int li, const Meta& md, int n_seqs, int M, int max_
         const size_t lds = (size_t)m->Tmax * 4;
         hipLaunchKernelGGL(attn_f32_kernel, dim3(max_len, m->nH, n_seqs), dim3(256), lds, m->stream, a, m->hd);
     } else if (max_len == 1) {
-        const int cfg = decode_attn_cfg(m, n_seqs), nsplit = cfg >> 8;
+        const int cfg = decode_attn_cfg(m, n_seqs), nsplit = cfg >> 8 & 15;
+        a.split_max = nsplit; a.split_tiles = cfg >> 12;
         dim3 grid(m->nKV * cdiv(m->group, 16), n_seqs, nsplit);      // (kv head x 16-head query tile, sequence, key split)
         a.part = m->attn_part; a.part_cnt = m->attn_part_cnt;
         // waves per workgroup: each wave takes NT2 key tiles per round trip (2 for hd 64, 1 for hd 128).  Short contexts

@@ -225,3 +225,39 @@ def test_prefill_attention_rows(gpu, oracle, rows, nH, nKV, S, T, hd):
     got = gpu.ops.attention(q, k, v, precision="bf16")
     gpu.lib().nvl_set_tuning(10, old)
     assert rel_err(got, oracle.gqa_core(q, k, v)) <= TOL
+
+
+@pytest.mark.parametrize("hd,kv", [(64, 1), (64, 4), (128, 2)])
+@pytest.mark.parametrize("waves", [0, 2, 4, 8])                       # 0: the launcher's form
+@pytest.mark.parametrize("rounds", [1, 2])
+def test_decode_attention_in_parts(gpu, hd, kv, waves, rounds):
+    """Each sequence dealt over as many workgroups as its own length asks for (one, some, the most; a last part of one key): a step against the
+    whole form and the greedy loop (graph replays: the tickets are zero again) against single steps."""
+    cfg = gpu.synth.tiny_config("llama", hidden=256, num_heads=256 // hd, head_dim=hd, num_kv_heads=min(kv, 256 // hd), max_seq_len=1536)
+    m = gpu.HipTransformerModel(cfg, gpu.synth.make_weights(cfg, seed=5, scale=0.05), precision="bf16", max_seqs=5, max_batch_tokens=1536)
+    r = np.random.default_rng(8)
+    lens = [1400, 1, 256, 511, 700]
+    prompts = [r.integers(0, cfg["vocab_size"], n).tolist() for n in lens]
+    ids, got = list(range(5)), []
+
+    def prompt():
+        for i in ids:
+            m.seq_reset(i)
+            m.forward_batch([i], [prompts[i]], [0], want_logits=False)
+
+    for form in (0, 1 + rounds if waves else 1):
+        old = [(key, gpu.lib().nvl_set_tuning(key, v)) for key, v in ((25, form), (15, waves if form else 0))]
+        prompt()
+        first, am = m.forward_batch(ids, [[7]] * 5, lens)
+        one = []
+        for j in range(3):
+            _, am = m.forward_batch(ids, [[int(t)] for t in am], [n + 1 + j for n in lens], want_logits=False)
+            one.append(am)
+        prompt()
+        _, am = m.forward_batch(ids, [[7]] * 5, lens, want_logits=False)
+        assert np.array_equal(m.decode_greedy(ids, am, 3), np.stack(one))
+        got.append(first)
+        for key, v in old:
+            gpu.lib().nvl_set_tuning(key, v)
+    m.close()
+    assert rel_err(got[1], got[0]) <= TOL
