@@ -471,7 +471,8 @@ __device__ __forceinline__ void attn_decode_merge(const AttnArgs& p, int pair, i
 // sequence's position, the block id of its first tile) leave at once — with everything inside the struct the compiler
 // fetched the argument block in two dependent pieces first (in-kernel stamps: 2.4 us from entry to the first vector load
 // at B = 1, against 0.4 us in the projection kernels).
-template <int HD, int NW, bool FUSED, bool STAMP = false>
+// SPLIT: its own instance — the arguments and the branch that deal a sequence over workgroups cost an unsplit launch 0.6 us (GPT-2, 104 rows)
+template <int HD, int NW, bool FUSED, bool SPLIT, bool STAMP = false>
 __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t* __restrict__ a_seq_pos, const int32_t* __restrict__ a_blk_table,
                                                                    int a_tbl_stride, int a_bs_shift, int a_Tmax, int a_group, AttnArgs p) {
     constexpr int KS = HD / 32, DT = HD / 16, HALF = HD / 2, CPR = HD / 8, KPI = 64 / CPR, NVL = 64 / KPI;
@@ -482,7 +483,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t
     __shared__ float red_l[NW][16];
     // grid.x = kv head x query tile: a workgroup takes 16 of the group's query heads (GQA / MHA: one tile; Falcon's MQA:
     // 71 heads = 5 tiles that stream the same K/V — it is tiny next to the weights — from L2)
-    const int swg = (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+    const int swg = ((SPLIT ? blockIdx.z * gridDim.y : 0) + blockIdx.y) * gridDim.x + blockIdx.x;
     NvlStampsT<STAMP> stamps(p.stamps, swg);          // (diagnostic instantiation only: see common.h)
     const int QT = (a_group + 15) >> 4;
     const int seq = blockIdx.y, kvh = blockIdx.x / QT, qt = blockIdx.x - kvh * QT;
@@ -493,7 +494,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t
     // wave's first tiles (which do not depend on the position).  Left to itself the compiler sinks the block-id loads behind
     // the position's wait and the tile-count branch (two more dependent scalar round trips before the first vector load:
     // +0.7 us per launch at B = 1).
-    const int vw = blockIdx.z * (NW * NT2) + wave;          // this wave's first tile; the others of its round are NW apart
+    const int vw = (SPLIT ? blockIdx.z * (NW * NT2) : 0) + wave;          // this wave's first tile; the others of its round are NW apart
     const int tok = seq, pos0 = a_seq_pos[seq];              // (decode launches carry one token per sequence, in sequence order)
     int first_blk[NT2];
 #pragma unroll
@@ -511,8 +512,8 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t
     const int n_kt = pos0 / 64 + 1;
     // rounds of NW x NT2 key tiles are dealt over the nz workgroups of this (sequence, kv head) in turn (one workgroup pulls all K/V of its
     // head through one CU, ~50 GB/s, one round after the other)
-    const int nz = p.split_max == 1 ? 1 : min(p.split_max, (n_kt + p.split_tiles - 1) / p.split_tiles), stride = NW * NT2 * nz;
-    if ((int)blockIdx.z >= nz) return;
+    const int nz = SPLIT ? min(p.split_max, (n_kt + p.split_tiles - 1) / p.split_tiles) : 1, stride = NW * NT2 * nz, z = SPLIT ? blockIdx.z : 0;
+    if (SPLIT && z >= nz) return;
     // (FUSED: the new token's q / k / v are fetched and rotated AFTER the first round's K/V loads are issued: below)
     bf16x8 knew[KS];
     bf16x8 vnew8;
@@ -716,7 +717,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t
         issue_round(kt0);
         do_round(kt0);
     }
-    if (FUSED && blockIdx.z == 0 && qt == 0) {
+    if (FUSED && z == 0 && qt == 0) {
         // append the new key/value to the slabs for the following steps — after every load of this step (which used
         // the register copies), so the loads above are not ordered behind these stores
         int nblk, nrow;
@@ -765,7 +766,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t
     f32x4 O[DT];
 #pragma unroll
     for (int d = 0; d < DT; d++) O[d] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (mstar > -INFINITY) {       // (a workgroup of a split launch may have had no tile at all)
+    if (!SPLIT || mstar > -INFINITY) {       // (a workgroup of a split launch may have had no tile at all)
 #pragma unroll
         for (int w = 0; w < NW; w++) {
             const float sc = __builtin_amdgcn_exp2f(red_m[w][fq] - mstar);   // idle waves: exp2(-inf) = 0
@@ -775,9 +776,9 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t
             for (int d = 0; d < DT; d++) O[d] += wo[d * 64 + lane] * sc;
         }
     }
-    if (nz > 1) {
+    if (SPLIT && nz > 1) {
         const int pair = seq * gridDim.x + blockIdx.x;               // (sequence, kv head, query tile)
-        float* rec = p.part + ((int64_t)pair * p.split_max + blockIdx.z) * attn_part_floats<HD>();
+        float* rec = p.part + ((int64_t)pair * p.split_max + z) * attn_part_floats<HD>();
 #pragma unroll
         for (int d = 0; d < DT; d++) part_store(rec, (d * 64 + lane) * 4, O[d]);
         // (m and l of four rows by the lane of the first: 16-byte stores)

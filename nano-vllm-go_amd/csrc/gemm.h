@@ -1862,8 +1862,8 @@ static inline bool mid_wins(const GemmArgs& a) {
         // 4096 x 14336 43 -> 28.6, 55 -> 29.9, 85.7 -> 32.6 us; 4544 x 18176 at 16 rows 48.7 -> 34.9; 2048 x 8192 stays at 15.3 up to 32 rows, 23.1 -> 18.4 at 64
         return mid_cost(a.M, a.N, a.K, mid_row_tiles(a.M), 2, a.split_ws != nullptr, mid_parts) < 0.92 * narrow_cost(a.M, a.N, a.K, blocks, blocks * ks * (split ? cdiv(a.M, 16) : 1), split);
     }
-    // (GPT-2's 768-wide projections at 96 rows: 12.7 / 12.0 / 11.1 us here, 8.8 / 10.1 / 9.3 in groups of the decode form)
-    if (EPI != EPI_QKV && a.K < 2048) return false;
+    // (GPT-2's projections at 96 .. 104 rows: 768 x 768 12.7 us here and 8.8 in groups of the decode form, 768 x 3072 14.7 and 13.6)
+    if (EPI != EPI_QKV && (a.K < 2048 || (int64_t)a.N * a.K < (4 << 20))) return false;
     // One row group reads the weights once at any width up to a few rounds of workgroups (a workgroup per CU: each round has its own
     // ramp; LM head at 128 rows 168 us against 152 on the tiles, 28672 x 4096 72 against 74).  Several groups pay while one round holds
     // them (3072 x 2048: 192 rows 12.5 against 17.4 us, 512 rows 18.3 against 29; 16384 x 2048 at 512 rows 68 against 43).

@@ -1304,26 +1304,22 @@ void attention(nvl_model* m, int li, const Meta& md, int n_seqs, int M, int max_
             a.qkv = m->qkv; a.qkv_stride = m->n_qkv; a.cos_t = m->rope_cos; a.sin_t = m->rope_sin;
         }
 #define NVL_DEC_LEAD a.seq_pos, a.blk_table, a.tbl_stride, a.bs_shift, a.Tmax, a.group      /* the preloaded leading arguments (attn.h) */
-#define NVL_DEC(HDv, FUSEDv)                                                                                           \
+#define NVL_DECN(HDv, NWv, FUSEDv, SPLITv, STv)                                                                         \
         do {                                                                                                           \
-            constexpr int tile_bytes = 64 * HDv * 2;                                                                   \
-            if (nw == 2) hipLaunchKernelGGL((attn_decode_bf16_kernel<HDv, 2, FUSEDv>), grid, dim3(128), 2 * tile_bytes, m->stream, NVL_DEC_LEAD, a);      \
-            else if (nw == 4) hipLaunchKernelGGL((attn_decode_bf16_kernel<HDv, 4, FUSEDv>), grid, dim3(256), 4 * tile_bytes, m->stream, NVL_DEC_LEAD, a); \
-            else {                                                                                                     \
-                NVL_LDS_ATTR((attn_decode_bf16_kernel<HDv, 8, FUSEDv>), 8 * tile_bytes);                               \
-                hipLaunchKernelGGL((attn_decode_bf16_kernel<HDv, 8, FUSEDv>), grid, dim3(512), 8 * tile_bytes, m->stream, NVL_DEC_LEAD, a);               \
-            }                                                                                                          \
+            NVL_LDS_ATTR((attn_decode_bf16_kernel<HDv, NWv, FUSEDv, SPLITv, STv>), NWv * 64 * HDv * 2);                \
+            hipLaunchKernelGGL((attn_decode_bf16_kernel<HDv, NWv, FUSEDv, SPLITv, STv>), grid, dim3(NWv * 64), NWv * 64 * HDv * 2, m->stream, NVL_DEC_LEAD, a); \
         } while (0)
-        if (a.stamps && fused_qkv && m->hd == 64) {     // diagnostic instantiation with the in-kernel stamps compiled in
-            constexpr int tb = 64 * 64 * 2;
-            if (nw == 2) hipLaunchKernelGGL((attn_decode_bf16_kernel<64, 2, true, true>), grid, dim3(128), 2 * tb, m->stream, NVL_DEC_LEAD, a);
-            else if (nw == 4) hipLaunchKernelGGL((attn_decode_bf16_kernel<64, 4, true, true>), grid, dim3(256), 4 * tb, m->stream, NVL_DEC_LEAD, a);
-            else {
-                NVL_LDS_ATTR((attn_decode_bf16_kernel<64, 8, true, true>), 8 * tb);
-                hipLaunchKernelGGL((attn_decode_bf16_kernel<64, 8, true, true>), grid, dim3(512), 8 * tb, m->stream, NVL_DEC_LEAD, a);
-            }
-        } else if (fused_qkv) { if (m->hd == 64) NVL_DEC(64, true); else NVL_DEC(128, true); }
-        else { if (m->hd == 64) NVL_DEC(64, false); else NVL_DEC(128, false); }
+#define NVL_DEC(HDv, FUSEDv, SPLITv, STv)                                                                               \
+        do {                                                                                                           \
+            if (nw == 2) NVL_DECN(HDv, 2, FUSEDv, SPLITv, STv); else if (nw == 4) NVL_DECN(HDv, 4, FUSEDv, SPLITv, STv); \
+            else NVL_DECN(HDv, 8, FUSEDv, SPLITv, STv);                                                                \
+        } while (0)
+        if (a.stamps && fused_qkv && m->hd == 64 && nsplit == 1) NVL_DEC(64, true, false, true);      // diagnostic instantiation with the in-kernel stamps compiled in
+        else if (fused_qkv && nsplit > 1) { if (m->hd == 64) NVL_DEC(64, true, true, false); else NVL_DEC(128, true, true, false); }
+        else if (fused_qkv) { if (m->hd == 64) NVL_DEC(64, true, false, false); else NVL_DEC(128, true, false, false); }
+        else if (nsplit > 1) { if (m->hd == 64) NVL_DEC(64, false, true, false); else NVL_DEC(128, false, true, false); }
+        else { if (m->hd == 64) NVL_DEC(64, false, false, false); else NVL_DEC(128, false, false, false); }
+#undef NVL_DECN
 #undef NVL_DEC
 #undef NVL_DEC_LEAD
     } else {
