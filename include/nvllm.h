@@ -582,7 +582,7 @@ int nvl_bench_gemm(int device, int M, int N, int K, int epi, int force_bnt, int 
  * key 36: weight tiles per wave of the wide decode projections (FFN-up, LM head): 0 (default) 2 for 17..32 rows and N < 65536, else 4;
  * 2 / 4 forced.
  * key 37: workgroups the keys of a row tile are split over in the short grouped attention (lists of layers): 0 (default) from the context.
- * key 41: parts of K for the 256x256 tiles of the last, partly filled round (0, default: from the grid; 1 never).
+ * key 41: parts of K for the 256x256 tiles of the last, partly filled round (0, default: from the grid; 1 never; up to 512 rows only with key 11 above them).
  * key 42: lists of layers, decode: the grouped attention launch norms and rotates queries and keys and carries a second mixer's gated
  * norm (1, default; 0 = launches of their own).
  * key 33: MoE decode: the experts' down projection completes the residual and carries the next RMSNorm (1, default; 0: K slices that a

@@ -1765,7 +1765,8 @@ static inline bool pp_wins(GemmArgs& a) {
     a.splits = 1;
     if (a.seg || a.a_rows || a.tile_map || a.sk_part || a.K < 160) return false;
     const int bytes = EPI == EPI_RESID ? 8 : EPI == EPI_GROUPED_RAW ? 4 : epi_glu(EPI) ? (int)sizeof(OutT) / 2 : (int)sizeof(OutT);
-    return pp_cost(a.M, a.N, a.K, bytes, a.split_ws != nullptr, a.splits) < 0.93 * tile128_cost(a.M, a.N, a.K, bytes, 1);
+    const bool parts = a.split_ws && (a.M > MID_MAX_ROWS || a.M <= std::max(64, g_chunk_max_m));      // (key 11 = 64: sums in one order whatever the rows, up to 512)
+    return pp_cost(a.M, a.N, a.K, bytes, parts, a.splits) < 0.93 * tile128_cost(a.M, a.N, a.K, bytes, 1);
 }
 template <int EPI, typename OutT, int WAVES_N>
 static inline void launch_pp(hipStream_t st, const GemmArgs& a) {
