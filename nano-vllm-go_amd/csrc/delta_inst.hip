@@ -1,4 +1,5 @@
 // delta_inst.hip — the instances of the channel-wise delta rule's kernels (delta.h) and their launches.
+#include <algorithm>
 #include "delta.h"
 
 namespace nvl {
@@ -37,16 +38,30 @@ static void scan(hipStream_t st, const DeltaArgs& p, int n_seqs) {
     NVL_LDS_ATTR((delta_scan_kernel<NK, NW, KSP>), lds);
     hipLaunchKernelGGL((delta_scan_kernel<NK, NW, KSP>), dim3(p.H, n_seqs, cdiv(p.DV, 16 * NW / KSP)), dim3(NW * 64), lds, st, p);
 }
-// columns per workgroup, and with few of them the key channels split over the waves too
-template <int NK, int LOW>
-static void scan_shape(hipStream_t st, const DeltaArgs& p, int n_seqs) {
-    const int pairs = p.H * n_seqs;
-    if (pairs * cdiv(p.DV, 64) < 128) scan<NK, 4, LOW>(st, p, n_seqs);
-    else if (p.DV <= 64 || pairs * cdiv(p.DV, 128) < 256) scan<NK, 4, 1>(st, p, n_seqs);
-    else scan<NK, 8, 1>(st, p, n_seqs);
+// Columns per workgroup (64 or 128) and parts of the key channels (KSP): more parts shorten the chain of a sequence's chunks, whose fp32
+// products bound a wave, and cost each of them an exchange.  us, fitted to 1 .. 64 sequences of 100 .. 1900 tokens x 16 heads of 128,
+// good to 20 %: the longest sequence's chain, all chunks at the chip's rate, the larger of them and a third of the other.
+// 5 x 300..1900 x 16 heads: 297 with whole channels, 237 in two parts; 1 x 1900 271 / 194 / 155 in one / two / four; 16 x 900 237 / 314 / 553.
+static double scan_cost(const DeltaArgs& p, int n_seqs, int nk, int nw, int ksp, int max_len, int tokens) {
+    const double size = nk / 8.0, heads = p.H * cdiv(p.DV, 64) / 2.0;
+    const double chain = cdiv(max_len, DELTA_C) * (1.95 + size * 2.55 * (nw / 4) / ksp);
+    const double all = heads * ((double)tokens / DELTA_C + 0.5 * n_seqs) * (size * 0.0225 + 0.0105 * ksp + (nw == 8 ? 0.0025 : 0.0));
+    return std::max(chain, all) + 0.35 * std::min(chain, all);
 }
-void delta_scan_launch(hipStream_t st, const DeltaArgs& p, int n_seqs, int nk) {
+template <int NK, int... PARTS>
+static void scan_shape(hipStream_t st, const DeltaArgs& p, int n_seqs, int max_len, int tokens) {
+    int best = 1;
+    double t = scan_cost(p, n_seqs, NK, 4, 1, max_len, tokens);
+    auto consider = [&](int ksp) { const double c = scan_cost(p, n_seqs, NK, 4, ksp, max_len, tokens); if (c < 0.95 * t) { t = c; best = ksp; } };
+    (consider(PARTS), ...);
+    if (p.DV > 64 && scan_cost(p, n_seqs, NK, 8, 1, max_len, tokens) < t) { scan<NK, 8, 1>(st, p, n_seqs); return; }
+    if (best == 1) { scan<NK, 4, 1>(st, p, n_seqs); return; }
+    ((best == PARTS ? scan<NK, 4, PARTS>(st, p, n_seqs) : void()), ...);
+}
+void delta_scan_launch(hipStream_t st, const DeltaArgs& p, int n_seqs, int nk, int max_len, int tokens) {
     if (nk == 2) scan<2, 4, 1>(st, p, n_seqs);
-    else if (nk == 4) scan_shape<4, 2>(st, p, n_seqs); else if (nk == 8) scan_shape<8, 4>(st, p, n_seqs); else scan_shape<16, 4>(st, p, n_seqs);
+    else if (nk == 4) scan_shape<4, 2>(st, p, n_seqs, max_len, tokens);
+    else if (nk == 8) scan_shape<8, 2, 4>(st, p, n_seqs, max_len, tokens);
+    else scan_shape<16, 2, 4>(st, p, n_seqs, max_len, tokens);
 }
 }  // namespace nvl

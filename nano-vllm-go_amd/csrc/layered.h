@@ -1265,7 +1265,7 @@ void mix_delta(nvl_model* m, const LayerRun& r, const MixerW& w, const Meta& md,
         }
         {
             KScope ks(m, KC_OTHER, 6.0 * M * elems, KS_DELTA_SCAN, scratch + 2.0 * n_seqs * elems * 4.0);
-            delta_scan_launch(m->stream, a, n_seqs, nk);
+            delta_scan_launch(m->stream, a, n_seqs, nk, max_len, M);
             NVL_HIP(hipGetLastError());
         }
     }
