@@ -270,7 +270,7 @@ __global__ __launch_bounds__(256) void mamba_step_kernel(MambaArgs p, bf16_t* __
 // ------------------------------------------------------------------------------------------
 template <int HD, int SS>
 constexpr int mamba_ssd_lds_bytes() {
-    return 2 * ((64 * (SS + 8)) * 2 + SS * (64 + 8) + 2 * HD * (64 + 8) + 64 * (64 + 8) + HD * (SS + 8)) + 64 * 4 * 3;
+    return 2 * ((64 * (SS + 8)) * 2 + SS * (64 + 8) + 2 * HD * (64 + 8) + 64 * (64 + 8) + HD * (SS + 8)) + 64 * 4 * 2;
 }
 // MODE 0: one workgroup per (sequence, head) walks the chunks in order (the state stays in its accumulators).
 // With few (sequence, head) pairs and long prompts that leaves most of the chip idle, so the chunks can run in parallel:
@@ -295,7 +295,6 @@ __global__ __launch_bounds__(256) void mamba_ssd_kernel(MambaArgs p) {
     bf16_t* Sb = Ms + Q * LQ;                     // [HD][LC]   bf16 copy of the state entering the chunk
     float* s_cum = (float*)(Sb + HD * LC);        // [Q] inclusive prefix sums of a_j
     float* s_dt = s_cum + Q;                      // [Q] dt_j
-    float* s_w = s_dt + Q;                        // [Q] exp(s_Q - s_j) dt_j
     const int h = blockIdx.x, seq = blockIdx.y;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int fr = lane & 15, fg = lane >> 4;
@@ -320,19 +319,47 @@ __global__ __launch_bounds__(256) void mamba_ssd_kernel(MambaArgs p) {
             sacc[j][r] = MODE == 1 ? 0.f : (MODE == 2 ? zs[o] : (fresh ? 0.f : st[o]));
         }
 
-    for (int c0 = MODE == 0 ? 0 : (int)blockIdx.z * Q; c0 < (MODE == 0 ? n : (int)blockIdx.z * Q + 1); c0 += Q) {
+    // A chunk's operands travel in registers while the chunk before it is worked on (98 KiB of LDS leave one workgroup a CU: nothing else hides
+    // them).  A thread has four tokens of four columns: the transposed copies go to LDS four tokens at a time, in whole rows of banks
+    // (token by token they were 2-byte stores, eight to a bank).  2326 tokens x 64 heads, longest 600: 133 us before, 103 now.
+    constexpr int BI = 16 * (SS / 4), NBI = (BI + 255) / 256, UI = 16 * (HD / 4);      // (UI <= 256)
+    f32x4 rb[NBI][4], rc[NBI][4], ru[4];
+    float rdt = 0.f;
+    auto fetch = [&](int c0) {
+        const int nv = min(Q, n - c0);
+        const float* x0 = p.xbc + (int64_t)(t0 + c0) * p.conv_dim;
+        rdt = lane < nv ? p.delta[(int64_t)(t0 + c0 + lane) * p.nh + h] : 0.f;
+#pragma unroll
+        for (int k = 0; k < NBI; k++) {
+            const int i = tid + 256 * k, t = 4 * (i & 15), q4 = (i >> 4) * 4;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                rb[k][e] = rc[k][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+                if (i < BI && t + e < nv) {
+                    const float* xr = x0 + (int64_t)(t + e) * p.conv_dim + p.EH + g * SS + q4;
+                    rb[k][e] = *(const f32x4*)xr;
+                    if (MODE != 1) rc[k][e] = *(const f32x4*)(xr + p.ng * SS);
+                }
+            }
+        }
+        const int t = 4 * (tid & 15), d4 = (tid >> 4) * 4;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            ru[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (tid < UI && t + e < nv) ru[e] = *(const f32x4*)(x0 + (int64_t)(t + e) * p.conv_dim + h * HD + d4);
+        }
+    };
+    const int c_first = MODE == 0 ? 0 : (int)blockIdx.z * Q, c_end = MODE == 0 ? n : c_first + 1;
+    fetch(c_first);
+    for (int c0 = c_first; c0 < c_end; c0 += Q) {
         const int nv = min(Q, n - c0);                          // valid tokens of this chunk
         __syncthreads();                                        // the previous chunk's LDS readers are done
-        // ---- decay bookkeeping: wave 0 scans a_j = A dt_j ----
-        if (wave == 0) {
-            const float dt = lane < nv ? p.delta[(int64_t)(t0 + c0 + lane) * p.nh + h] : 0.f;
-            float s = A * dt;
+        // ---- decay bookkeeping: every wave scans a_j = A dt_j (lane j), wave 0 leaves it in LDS ----
+        float s = A * rdt;
 #pragma unroll
-            for (int o = 1; o < 64; o <<= 1) { const float v = __shfl_up(s, o, 64); if (lane >= o) s += v; }
-            s_cum[lane] = s; s_dt[lane] = dt;
-            const float sq = __shfl(s, 63, 64);
-            s_w[lane] = __expf(sq - s) * dt;
-        }
+        for (int o = 1; o < 64; o <<= 1) { const float v = __shfl_up(s, o, 64); if (lane >= o) s += v; }
+        const float wj = __expf(__shfl(s, 63, 64) - s) * rdt;
+        if (wave == 0) { s_cum[lane] = s; s_dt[lane] = rdt; }
         // ---- the state entering the chunk, as the bf16 operand of Y_inter ----
         if (MODE != 1) {
 #pragma unroll
@@ -340,32 +367,49 @@ __global__ __launch_bounds__(256) void mamba_ssd_kernel(MambaArgs p) {
 #pragma unroll
                 for (int r = 0; r < 4; r++) Sb[(16 * sd + 4 * fg + r) * LC + 16 * (sn0 + j) + fr] = (bf16_t)sacc[j][r];
         }
-        __syncthreads();
-        // ---- stage u, B, C of the chunk (fp32 rows of xbc -> bf16, K-contiguous; B and u also transposed) ----
-        for (int i = tid; i < Q * (SS / 4); i += 256) {
-            const int t = i / (SS / 4), q4 = (i - t * (SS / 4)) * 4;
-            f32x4 b = f32x4{0.f, 0.f, 0.f, 0.f}, c = b;
-            if (t < nv) {
-                const float* xr = p.xbc + (int64_t)(t0 + c0 + t) * p.conv_dim + p.EH + g * SS + q4;
-                b = *(const f32x4*)xr;
-                if (MODE != 1) c = *(const f32x4*)(xr + p.ng * SS);
-            }
-            bf16x4 bb, cc;
+        // ---- u, B, C of the chunk as bf16, K-contiguous; B and u also transposed ----
 #pragma unroll
-            for (int r = 0; r < 4; r++) { bb[r] = (bf16_t)b[r]; cc[r] = (bf16_t)c[r]; if (MODE != 2) Bt[(q4 + r) * LQ + t] = (bf16_t)b[r]; }
-            if (MODE != 1) { *(bf16x4*)(Bs + t * LC + q4) = bb; *(bf16x4*)(Cs + t * LC + q4) = cc; }
+        for (int k = 0; k < NBI; k++) {
+            const int i = tid + 256 * k, t = 4 * (i & 15), q4 = (i >> 4) * 4;
+            if (i < BI) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    bf16x4 bb, cc, bt;
+#pragma unroll
+                    for (int r = 0; r < 4; r++) { bb[r] = (bf16_t)rb[k][e][r]; cc[r] = (bf16_t)rc[k][e][r]; bt[r] = (bf16_t)rb[k][r][e]; }
+                    if (MODE != 1) { *(bf16x4*)(Bs + (t + e) * LC + q4) = bb; *(bf16x4*)(Cs + (t + e) * LC + q4) = cc; }
+                    if (MODE != 2) *(bf16x4*)(Bt + (q4 + e) * LQ + t) = bt;
+                }
+            }
         }
-        for (int i = tid; i < Q * (HD / 4); i += 256) {
-            const int t = i / (HD / 4), d4 = (i - t * (HD / 4)) * 4;
-            f32x4 u = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (t < nv) u = *(const f32x4*)(p.xbc + (int64_t)(t0 + c0 + t) * p.conv_dim + h * HD + d4);
-            const float w = s_w[t];
+        {
+            const int t = 4 * (tid & 15), d4 = (tid >> 4) * 4;
+            float w[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) w[r] = __shfl(wj, 4 * (lane & 15) + r, 64);
+            if (tid < UI) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    bf16x4 ut, uw;
+#pragma unroll
+                    for (int r = 0; r < 4; r++) { ut[r] = (bf16_t)ru[r][e]; uw[r] = (bf16_t)(ru[r][e] * w[r]); }
+                    if (MODE != 1) *(bf16x4*)(Ut + (d4 + e) * LQ + t) = ut;
+                    if (MODE != 2) *(bf16x4*)(Uw + (d4 + e) * LQ + t) = uw;
+                }
+            }
+        }
+        // D u of this wave's rows, then the next chunk (loads return in order)
+        float du[4][DT];
+        if (MODE != 1) {
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                if (MODE != 1) Ut[(d4 + r) * LQ + t] = (bf16_t)u[r];
-                if (MODE != 2) Uw[(d4 + r) * LQ + t] = (bf16_t)(u[r] * w);
+                const int t = min(16 * wave + 4 * fg + r, nv - 1);
+                const float* ur = p.xbc + (int64_t)(t0 + c0 + t) * p.conv_dim + h * HD;
+#pragma unroll
+                for (int d = 0; d < DT; d++) du[r][d] = ur[16 * d + fr];
             }
         }
+        if (MODE == 0 && c0 + Q < n) fetch(c0 + Q);
         __syncthreads();
         if (MODE != 1) {
             // ---- G = C B^T for this wave's 16 tokens (row tile `wave`), causal column tiles only; M = G o L -> LDS ----
@@ -425,10 +469,9 @@ __global__ __launch_bounds__(256) void mamba_ssd_kernel(MambaArgs p) {
                     const int t = 16 * tt + 4 * fg + r;
                     if (t >= nv) continue;
                     const float es = __expf(s_cum[t]);
-                    const float* ur = p.xbc + (int64_t)(t0 + c0 + t) * p.conv_dim + h * HD;
                     float* yr = p.y + (int64_t)(t0 + c0 + t) * p.EH + h * HD;
 #pragma unroll
-                    for (int d = 0; d < DT; d++) yr[16 * d + fr] = yi[d][r] + es * ye[d][r] + Dh * ur[16 * d + fr];
+                    for (int d = 0; d < DT; d++) yr[16 * d + fr] = yi[d][r] + es * ye[d][r] + Dh * du[r][d];
                 }
             }
         }
