@@ -1250,7 +1250,7 @@ int decode_attn_cfg(const nvl_model* m, int n_seqs) {
     if (g_attn_split >= 2) { const int tiles = (g_attn_split - 1) * nw * per_wave; return cfg(nw, std::max(1, std::min(most, cdiv(n_kt, tiles))), tiles); }
     if (g_attn_split && !g_attn_nw && most > 1) {
         int waves = 0;
-        if (m->hd == 64) waves = wgs <= 48 ? (n_kt > 16 ? 4 : n_kt > 8 ? 2 : 0) : wgs <= 128 && n_kt > 12 ? 4 : 0;
+        if (m->hd == 64) waves = wgs <= 48 ? (n_kt > 20 ? 4 : n_kt > 8 ? 2 : 0) : wgs <= 128 && n_kt > 12 ? 4 : 0;
         else waves = wgs <= 32 ? (n_kt > 16 ? 4 : n_kt > 5 ? 2 : 0) : wgs <= 96 && n_kt > 8 ? 8 : 0;
         if (waves) return cfg(waves, std::min(most, cdiv(n_kt, waves * per_wave)), waves * per_wave);
     }
