@@ -114,22 +114,26 @@ struct PendingResid {
     const int32_t* slot_of;
     const float* gate_w;
 };
-// Prefill-sized batches, bf16 output: one 1024-thread workgroup per 16 output rows (one fragment-major row tile).  A wave
-// normalises one row held in registers (same arithmetic as norm_kernel) into LDS; the workgroup then writes the tile's
-// 1-KiB operand blocks with full-line stores (norm_kernel's lanes each write 8 bytes of a block: 16-byte fragments at a
-// 256-byte stride).  H <= 64 * 4 * MAXCH (instances for 8 and 16 chunks per lane: H <= 2048 / 4096).
+// Prefill-sized batches, bf16 output: one 512-thread workgroup per 8 output rows (half a fragment-major row tile).  A wave
+// normalises one row held in registers (same arithmetic as norm_kernel) into LDS; the workgroup then writes its halves of the
+// operand blocks, 128-byte lines of 8 rows x 16 bytes (norm_kernel's lanes each write 8 bytes of a block: 16-byte fragments at a
+// 256-byte stride).  Bound by HBM.  Eight rows and not sixteen: sixteen of 4096 columns fill a CU's LDS, and their few workgroups
+// leave CUs idle.  Sixteen -> eight rows, event times: 16384 x 2048 45.7 -> 38.4 us, 4170 x 4096 36.8 -> 30.7, 6867 x 1024
+// 14.4 -> 13.5, 2326 x 2048 11.5 -> 11.9; 1200 x 4544, on norm_kernel before, 21.4 -> 17.6.
+// H <= 64 * 4 * MAXCH (instances for 8, 16 and 18 chunks per lane: H <= 2048 / 4096 / 4608).
 // bf16 row pitch of such a tile in LDS: 16 bytes beyond a multiple of 64, or the 16 rows of a fragment read would share their banks
 __host__ __device__ __forceinline__ int tile16_pitch(int H) { return H + 8; }
+constexpr int NORM_TILE_ROWS = 8;
 template <int MAXCH, bool PENDING = false>
-__global__ __launch_bounds__(1024) void norm_tile16_kernel(float* __restrict__ x, const int32_t* __restrict__ rows_idx,
-                                                           const float* __restrict__ w, const float* __restrict__ b,
-                                                           float eps, bf16_t* __restrict__ y, int rows, int H, PendingResid pr,
-                                                           bf16_t* __restrict__ y_rows) {      // not NULL: the result a second time, row-major
+__global__ __launch_bounds__(64 * NORM_TILE_ROWS) void norm_tile_kernel(float* __restrict__ x, const int32_t* __restrict__ rows_idx,
+                                                                      const float* __restrict__ w, const float* __restrict__ b,
+                                                                      float eps, bf16_t* __restrict__ y, int rows, int H, PendingResid pr,
+                                                                      bf16_t* __restrict__ y_rows) {      // not NULL: the result a second time, row-major
     extern __shared__ __attribute__((aligned(16))) char smem_n[];
-    bf16_t* tile = (bf16_t*)smem_n;                       // [16][LT]
+    bf16_t* tile = (bf16_t*)smem_n;                       // [NORM_TILE_ROWS][LT]
     const int LT = tile16_pitch(H);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int r = blockIdx.x * 16 + wave;
+    const int r = blockIdx.x * NORM_TILE_ROWS + wave;
     const int H4 = H >> 2;
     if (r < rows) {
         const int src = rows_idx ? rows_idx[r] : r;
@@ -207,13 +211,15 @@ __global__ __launch_bounds__(1024) void norm_tile16_kernel(float* __restrict__ x
         }
     }
     __syncthreads();
-    // operand blocks of this row tile: block kb holds k = 32kb .. 32kb+31 of the 16 rows, lane l = row (l & 15), 8 k's (l >> 4)
-    const int nkb = H >> 5;
-    const int lr = lane & 15, lc = lane >> 4;
-    if (blockIdx.x * 16 + lr < rows)
-        for (int kb = wave; kb < nkb; kb += 16) {
+    // operand blocks of this row tile: block kb holds k = 32kb .. 32kb+31 of 16 rows, 8 k's of a row in 16 bytes, rows adjacent.  Lanes
+    // 0-7 take 8 rows of one block, lanes 8-15 of the block two further: the 128 bytes of rows and the 128 between the blocks keep the
+    // sixteen reads of a phase on different banks.
+    const int nkb = H >> 5, half = blockIdx.x & 1;
+    const int lr = lane & 7, lc = lane >> 4;
+    if (blockIdx.x * NORM_TILE_ROWS + lr < rows)
+        for (int kb = 4 * (wave >> 1) + (wave & 1) + ((lane >> 2) & 2); kb < nkb; kb += 2 * NORM_TILE_ROWS) {
             const bf16x8 f = *(const bf16x8*)(tile + lr * LT + kb * 32 + lc * 8);
-            *(bf16x8*)(y + (((int64_t)blockIdx.x * nkb + kb) * 64 + lane) * 8) = f;
+            *(bf16x8*)(y + (((int64_t)(blockIdx.x >> 1) * nkb + kb) * 64 + lc * 16 + half * 8 + lr) * 8) = f;
         }
 }
 

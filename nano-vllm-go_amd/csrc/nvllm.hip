@@ -1183,7 +1183,7 @@ void bind_slot(const nvl_model* m, const Meta& hm, int i, int slot) {
     }
 }
 
-static int g_norm_t16 = 1;     // nvl_set_tuning key 9: norm_tile16_kernel for prefill-sized bf16 norms (0 = norm_kernel)
+static int g_norm_t16 = 1;     // nvl_set_tuning key 9: norm_tile_kernel for prefill-sized bf16 norms (0 = norm_kernel)
 template <typename ActT>
 void launch_norm(nvl_model* m, float* x, const int32_t* rows_idx, const float* w, const float* b,
                  void* y, int rows, bf16_t* y_rows = nullptr) {
@@ -1200,23 +1200,24 @@ void launch_norm(nvl_model* m, float* x, const int32_t* rows_idx, const float* w
     if (rows <= 512 && m->H <= 1024 * NORM_ROW_MAXCH)
         hipLaunchKernelGGL((norm_row_kernel<ActT>), dim3(rows), dim3(256), 0, m->stream, x, rows_idx, w, b,
                            m->cfg.norm_eps, (ActT*)y, m->H, pr);
-    else if (sizeof(ActT) == 2 && m->H % 32 == 0 && m->H <= 4096 && g_norm_t16) {   // (wider rows would spill: norm_kernel)
-        // 16 rows x H bf16 of LDS (up to 129 KiB); the row sits in registers: instance by chunks per lane
-#define NVL_NT16(CH, PEND)                                                                                             \
+    else if (sizeof(ActT) == 2 && m->H % 32 == 0 && m->H <= 4608 && g_norm_t16) {   // (two workgroups' tiles of wider rows would not fit the LDS of a CU: norm_kernel)
+        // 8 rows x H bf16 of LDS (up to 73 KiB); the row sits in registers: instance by chunks per lane
+#define NVL_NT(CH, PEND)                                                                                             \
         do {                                                                                                           \
-            NVL_LDS_ATTR((norm_tile16_kernel<CH, PEND>), 160 * 1024);                                                  \
-            hipLaunchKernelGGL((norm_tile16_kernel<CH, PEND>), dim3(cdiv(rows, 16)), dim3(1024), (size_t)16 * tile16_pitch(m->H) * 2, m->stream, x, \
-                               rows_idx, w, b, m->cfg.norm_eps, (bf16_t*)y, rows, m->H, pr, y_rows);                    \
+            NVL_LDS_ATTR((norm_tile_kernel<CH, PEND>), 80 * 1024);                                                     \
+            hipLaunchKernelGGL((norm_tile_kernel<CH, PEND>), dim3(cdiv(rows, NORM_TILE_ROWS)), dim3(64 * NORM_TILE_ROWS),  \
+                               (size_t)NORM_TILE_ROWS * tile16_pitch(m->H) * 2, m->stream, x,                          \
+                               rows_idx, w, b, m->cfg.norm_eps, (bf16_t*)y, rows, m->H, pr, y_rows);                   \
         } while (0)
-        if (pr.part) NVL_NT16(8, true);        // (H <= 2048: checked above)
-        else { if (m->H <= 2048) NVL_NT16(8, false); else NVL_NT16(16, false); }
-#undef NVL_NT16
+        if (pr.part) NVL_NT(8, true);        // (H <= 2048: checked above)
+        else { if (m->H <= 2048) NVL_NT(8, false); else if (m->H <= 4096) NVL_NT(16, false); else NVL_NT(18, false); }
+#undef NVL_NT
     } else
         hipLaunchKernelGGL((norm_kernel<ActT>), dim3(cdiv(rows, 4)), dim3(256), 0, m->stream, x, rows_idx, w, b,
                            m->cfg.norm_eps, (ActT*)y, rows, m->H);
 }
 // does the norm of so many rows leave a row-major copy of its result (y_rows) too?
-bool norm_copies_rows(const nvl_model* m, int rows) { return !m->f32 && rows > 512 && m->H <= 4096 && g_norm_t16; }
+bool norm_copies_rows(const nvl_model* m, int rows) { return !m->f32 && rows > 512 && m->H % 32 == 0 && m->H <= 4608 && g_norm_t16; }
 void norm(nvl_model* m, float* x, const int32_t* rows_idx, const DevTensor& w, const DevTensor& b, void* y, int rows, bf16_t* y_rows = nullptr) {
     if (m->f32) launch_norm<float>(m, x, rows_idx, (const float*)w.p, (const float*)b.p, y, rows);
     else launch_norm<bf16_t>(m, x, rows_idx, (const float*)w.p, (const float*)b.p, y, rows, y_rows);

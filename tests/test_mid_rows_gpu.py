@@ -261,3 +261,29 @@ def test_decode_attention_in_parts(gpu, hd, kv, waves, rounds):
             gpu.lib().nvl_set_tuning(key, v)
     m.close()
     assert rel_err(got[1], got[0]) <= TOL
+
+
+@pytest.mark.parametrize("family,hidden,heads", [("llama", 192, 3), ("llama", 2048, 16), ("falcon", 2112, 33), ("llama", 4096, 32), ("falcon", 4544, 71),
+                                                 ("llama", 4608, 36), ("llama", 4672, 73)])       # up to 2048 / 4096 / 4608 columns, and beyond
+@pytest.mark.parametrize("lens", [[513], [300, 220], [521], [519, 9]])      # 513, 520, 521, 528 rows: remainders of 8 and of 16, whole halves
+def test_norm_tiles(gpu, family, hidden, heads, lens):
+    """The prompt's norms in tiles of eight rows (also with a residual add left as slices) against one wave per row: an operand may round
+    the other way, one bf16 step of 2^-8."""
+    kv = 1 if family == "falcon" else heads
+    cfg = gpu.synth.tiny_config(family, hidden=hidden, num_heads=heads, num_kv_heads=kv, head_dim=hidden // heads,
+                                ffn_dim=512, num_layers=1, max_seq_len=600)
+    w = gpu.synth.make_weights(cfg, seed=6, scale=0.02)
+    r = np.random.default_rng(hidden)
+    prompts = [r.integers(0, cfg["vocab_size"], t).tolist() for t in lens]
+    got = []
+    for tiles in (1, 0):
+        old = gpu.lib().nvl_set_tuning(9, tiles)
+        m = gpu.HipTransformerModel(cfg, w, precision="bf16", max_seqs=len(lens), max_batch_tokens=1024)
+        try:
+            for i in range(len(lens)):
+                m.seq_reset(i)
+            got.append(m.forward_batch(list(range(len(lens))), prompts, [0] * len(lens), want_logits=True)[0])
+        finally:
+            gpu.lib().nvl_set_tuning(9, old)
+            m.close()
+    assert np.isfinite(got[0]).all() and rel_err(got[0], got[1]) < 2.0 ** -8
