@@ -124,6 +124,18 @@ struct PendingResid {
 // bf16 row pitch of such a tile in LDS: 16 bytes beyond a multiple of 64, or the 16 rows of a fragment read would share their banks
 __host__ __device__ __forceinline__ int tile16_pitch(int H) { return H + 8; }
 constexpr int NORM_TILE_ROWS = 8;
+// Operand blocks of a workgroup's rows: block kb holds k = 32kb .. 32kb+31 of 16 rows, 8 k's of a row in 16 bytes, rows adjacent.  Lanes
+// 0-7 take 8 rows of one block, lanes 8-15 of the block two further: the 128 bytes of rows and the 128 between the blocks keep the
+// sixteen reads of a phase on different banks.
+__device__ __forceinline__ void store_norm_tile(const bf16_t* tile, bf16_t* __restrict__ y, int rows, int H, int lane, int wave) {
+    const int nkb = H >> 5, half = blockIdx.x & 1, LT = tile16_pitch(H);
+    const int lr = lane & 7, lc = lane >> 4;
+    if (blockIdx.x * NORM_TILE_ROWS + lr < rows)
+        for (int kb = 4 * (wave >> 1) + (wave & 1) + ((lane >> 2) & 2); kb < nkb; kb += 2 * NORM_TILE_ROWS) {
+            const bf16x8 f = *(const bf16x8*)(tile + lr * LT + kb * 32 + lc * 8);
+            *(bf16x8*)(y + (((int64_t)(blockIdx.x >> 1) * nkb + kb) * 64 + lc * 16 + half * 8 + lr) * 8) = f;
+        }
+}
 template <int MAXCH, bool PENDING = false>
 __global__ __launch_bounds__(64 * NORM_TILE_ROWS) void norm_tile_kernel(float* __restrict__ x, const int32_t* __restrict__ rows_idx,
                                                                       const float* __restrict__ w, const float* __restrict__ b,
@@ -211,16 +223,7 @@ __global__ __launch_bounds__(64 * NORM_TILE_ROWS) void norm_tile_kernel(float* _
         }
     }
     __syncthreads();
-    // operand blocks of this row tile: block kb holds k = 32kb .. 32kb+31 of 16 rows, 8 k's of a row in 16 bytes, rows adjacent.  Lanes
-    // 0-7 take 8 rows of one block, lanes 8-15 of the block two further: the 128 bytes of rows and the 128 between the blocks keep the
-    // sixteen reads of a phase on different banks.
-    const int nkb = H >> 5, half = blockIdx.x & 1;
-    const int lr = lane & 7, lc = lane >> 4;
-    if (blockIdx.x * NORM_TILE_ROWS + lr < rows)
-        for (int kb = 4 * (wave >> 1) + (wave & 1) + ((lane >> 2) & 2); kb < nkb; kb += 2 * NORM_TILE_ROWS) {
-            const bf16x8 f = *(const bf16x8*)(tile + lr * LT + kb * 32 + lc * 8);
-            *(bf16x8*)(y + (((int64_t)(blockIdx.x >> 1) * nkb + kb) * 64 + lc * 16 + half * 8 + lr) * 8) = f;
-        }
+    store_norm_tile(tile, y, rows, H, lane, wave);
 }
 
 // the arithmetic of one row once it sits in registers (shared by norm_row_kernel and decode_seam_kernel)
@@ -318,7 +321,8 @@ __global__ __launch_bounds__(256) void norm_row_kernel(float* __restrict__ x,
 // second; w_next == NULL: only the first, or with `raw_next` xn = x, for blocks without a norm in front).  Rows are H floats apart, the mean runs over `width` <= H columns (the padding
 // columns of x, y and the weights are zero).  y may be split over `slices` partial sums (a K split of the projection).
 //   sandwich_row_kernel    : one 256-thread workgroup per row, the row in registers (decode, short batches, wide rows)
-//   sandwich_tile16_kernel : one wave per row, 16 rows per workgroup, operand blocks written whole (prefill, bf16)
+//   sandwich_tile_kernel : one wave per row, 8 rows per workgroup as in norm_tile_kernel (prefill, bf16; sixteen -> eight rows, event
+//                          times: 5471 x 2048 31.9 -> 28.5 us, 4096 x 4096 107 -> 105, where 16 chunks a lane now fit the registers)
 // ---------------------------------------------------------------------------------------
 struct SandwichArgs {
     float* x;                 // residual stream [rows][H]
@@ -487,12 +491,12 @@ __global__ __launch_bounds__(256) void sandwich_row_kernel(SandwichArgs p, ActT*
     }
 }
 template <int MAXCH, bool EXT = false>
-__global__ __launch_bounds__(1024) void sandwich_tile16_kernel(SandwichArgs p, bf16_t* __restrict__ xn) {
+__global__ __launch_bounds__(64 * NORM_TILE_ROWS, MAXCH <= 8 ? 4 : 2) void sandwich_tile_kernel(SandwichArgs p, bf16_t* __restrict__ xn) {
     extern __shared__ __attribute__((aligned(16))) char smem_n[];
-    bf16_t* tile = (bf16_t*)smem_n;                       // [16][LT]
+    bf16_t* tile = (bf16_t*)smem_n;                       // [NORM_TILE_ROWS][LT]
     const int LT = tile16_pitch(p.H);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);      // (a row's slots and weights by scalar loads)
-    const int r = blockIdx.x * 16 + wave, H4 = p.H >> 2;
+    const int r = blockIdx.x * NORM_TILE_ROWS + wave, H4 = p.H >> 2;
     if (r < p.rows) {
         const int src = p.rows_idx ? p.rows_idx[r] : r;
         float* xr = p.x + (int64_t)src * p.H;
@@ -604,10 +608,7 @@ __global__ __launch_bounds__(1024) void sandwich_tile16_kernel(SandwichArgs p, b
     if (p.xn_rows && r < p.rows)
         for (int j = lane * 8; j < p.H; j += 512) *(bf16x8*)(p.xn_rows + (int64_t)r * p.H + j) = *(const bf16x8*)(tile + wave * LT + j);      // (its own row: no barrier)
     __syncthreads();
-    const int nkb = p.H >> 5, lr = lane & 15, lc = lane >> 4;
-    if (blockIdx.x * 16 + lr < p.rows)
-        for (int kb = wave; kb < nkb; kb += 16)
-            *(bf16x8*)(xn + (((int64_t)blockIdx.x * nkb + kb) * 64 + lane) * 8) = *(const bf16x8*)(tile + lr * LT + kb * 32 + lc * 8);
+    store_norm_tile(tile, xn, p.rows, p.H, lane, wave);
 }
 
 // ---------------------------------------------------------------------------------------

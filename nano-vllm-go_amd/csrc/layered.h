@@ -906,16 +906,16 @@ void sandwich(nvl_model* m, SubOut y, const float* w_post, NextNorm next, void* 
     const bool ext = (y.y && !w_post) || next.b || a.sum_scale != 0.f || sh.mu;
     a.xn_rows = xn_rows;
     if (sandwich_copies_rows(m, y, rows) && !sh.mu) {
-        const size_t lds = (size_t)16 * tile16_pitch(m->H) * 2;
-#define NVL_SW16E(CH, EXT)                                                                                                  \
+        const size_t lds = (size_t)NORM_TILE_ROWS * tile16_pitch(m->H) * 2;
+#define NVL_SWTE(CH, EXT)                                                                                                  \
         do {                                                                                                                \
-            NVL_LDS_ATTR((sandwich_tile16_kernel<CH, EXT>), 160 * 1024);                                                    \
-            hipLaunchKernelGGL((sandwich_tile16_kernel<CH, EXT>), dim3(cdiv(rows, 16)), dim3(1024), lds, m->stream, a, (bf16_t*)xn); \
+            NVL_LDS_ATTR((sandwich_tile_kernel<CH, EXT>), 80 * 1024);                                                       \
+            hipLaunchKernelGGL((sandwich_tile_kernel<CH, EXT>), dim3(cdiv(rows, NORM_TILE_ROWS)), dim3(64 * NORM_TILE_ROWS), lds, m->stream, a, (bf16_t*)xn); \
         } while (0)
-#define NVL_SW16(CH) do { if (ext) NVL_SW16E(CH, true); else NVL_SW16E(CH, false); } while (0)
-        if (m->H <= 1024) NVL_SW16(4); else if (m->H <= 2048) NVL_SW16(8); else NVL_SW16(16);
-#undef NVL_SW16
-#undef NVL_SW16E
+#define NVL_SWT(CH) do { if (ext) NVL_SWTE(CH, true); else NVL_SWTE(CH, false); } while (0)
+        if (m->H <= 1024) NVL_SWT(4); else if (m->H <= 2048) NVL_SWT(8); else NVL_SWT(16);
+#undef NVL_SWT
+#undef NVL_SWTE
     } else {
 #define NVL_SWR(CH)                                                                                                          \
         do {                                                                                                                \

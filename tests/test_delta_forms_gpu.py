@@ -9,6 +9,7 @@ from layered_helpers import build, err
 
 pytestmark = pytest.mark.gpu
 F32_LAYER = 1e-4        # a single fp32 layer against the plain restatement, as in the other tests of these models
+BF16_LAYER = 0.03       # a single bf16 layer, as there
 
 
 @pytest.mark.parametrize("heads,dim,vdim", [(2, 40, 24), (4, 100, 72), (16, 128, 128), (3, 200, 72), (40, 128, 40), (20, 250, 130)])
@@ -27,3 +28,25 @@ def test_scan_parts(gpu, tmp_path, heads, dim, vdim):
         got = m.forward_batch(ids, tok[:n], [0] * n, all_logits=True)[0]
         assert err(np.asarray(got)[:330], want, "f32") < F32_LAYER, n
     m.close()
+
+
+@pytest.mark.parametrize("width", [64, 1056, 2080, 4096])             # 4 / 8 / 16 chunks of a row per lane
+@pytest.mark.parametrize("lens", [[513], [519, 9]])                    # 513 and 528 rows: remainders of 8 and of 16, whole halves
+def test_sandwich_tiles(gpu, tmp_path, width, lens):
+    """The prompt's sandwich norms in tiles of eight rows against portions of up to 300 rows, a row per workgroup: two bf16 runs whose
+    operands may round apart, each within the bf16 bound of a layer."""
+    cfg = LM.config([LM.delta(heads=2, kv_heads=2, dim=32, vdim=32)], width=width, vocab=60)
+    w = LM.weights(cfg, 17)
+    g = np.random.default_rng(width)
+    tok = [g.integers(0, 60, n).tolist() for n in lens]
+    m = build(gpu, tmp_path, cfg, w, "bf16", max_seqs=4, max_batch_tokens=1024)
+    ids = list(range(len(lens)))
+    for i in range(4):
+        m.seq_reset(i)
+    whole = np.asarray(m.forward_batch(ids, tok, [0] * len(ids), all_logits=True)[0])
+    parts = []
+    for i, t in enumerate(tok):
+        for a in range(0, len(t), 300):
+            parts.append(np.asarray(m.forward_batch([2 + i], [t[a:a + 300]], [a], all_logits=True)[0]))
+    m.close()
+    assert err(whole, np.concatenate(parts), "bf16") < 2 * BF16_LAYER
