@@ -1184,6 +1184,12 @@ void bind_slot(const nvl_model* m, const Meta& hm, int i, int slot) {
 }
 
 static int g_norm_t16 = 1;     // nvl_set_tuning key 9: norm_tile_kernel for prefill-sized bf16 norms (0 = norm_kernel)
+// A workgroup per row up to here, tiles of eight rows above: fewer tiles than CUs wait for one another's loads.  Row / tile, event us:
+//   2048 columns with slices to add: 520 11.0 / 23.7, 700 12.4 / 23.5, 1000 13.4 / 20.0, 1500 19.8 / 21.4, 2000 18.5 / 19.0
+//   768: 520 6.8 / 8.9, 1000 7.9 / 9.3, 1500 9.9 / 9.5, 2000 10.9 / 9.6        4096: 1000 15.3 / 17.0, 2000 20.1 / 17.3
+//   4544: 520 11.3 / 15.7, 1000 14.9 / 17.0, 1500 20.0 / 18.5
+// (a row-major copy is the tiles' alone: with one, and where there are no tiles, the line is 512 rows)
+constexpr int NORM_ROW_KERNEL_ROWS = 1024;
 template <typename ActT>
 void launch_norm(nvl_model* m, float* x, const int32_t* rows_idx, const float* w, const float* b,
                  void* y, int rows, bf16_t* y_rows = nullptr) {
@@ -1197,10 +1203,11 @@ void launch_norm(nvl_model* m, float* x, const int32_t* rows_idx, const float* w
         const bool tile_kernel = sizeof(ActT) == 2 && m->H % 32 == 0 && m->H <= 2048 && g_norm_t16 && !pr.slot_of;   // (the 16-chunk instance would spill)
         if (!row_kernel && !tile_kernel) throw std::runtime_error("norm: no kernel for this pending residual");
     }
-    if (rows <= 512 && m->H <= 1024 * NORM_ROW_MAXCH)
+    const bool tiles = sizeof(ActT) == 2 && m->H % 32 == 0 && m->H <= 4608 && g_norm_t16 && !pr.slot_of && (!pr.part || m->H <= 2048);
+    if (rows <= (tiles && !y_rows ? NORM_ROW_KERNEL_ROWS : 512) && m->H <= 1024 * NORM_ROW_MAXCH)
         hipLaunchKernelGGL((norm_row_kernel<ActT>), dim3(rows), dim3(256), 0, m->stream, x, rows_idx, w, b,
                            m->cfg.norm_eps, (ActT*)y, m->H, pr);
-    else if (sizeof(ActT) == 2 && m->H % 32 == 0 && m->H <= 4608 && g_norm_t16) {   // (two workgroups' tiles of wider rows would not fit the LDS of a CU: norm_kernel)
+    else if (tiles) {   // (two workgroups' tiles of wider rows would not fit the LDS of a CU: norm_kernel)
         // 8 rows x H bf16 of LDS (up to 73 KiB); the row sits in registers: instance by chunks per lane
 #define NVL_NT(CH, PEND)                                                                                             \
         do {                                                                                                           \

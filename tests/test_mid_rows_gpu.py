@@ -265,20 +265,21 @@ def test_decode_attention_in_parts(gpu, hd, kv, waves, rounds):
 
 @pytest.mark.parametrize("family,hidden,heads", [("llama", 192, 3), ("llama", 2048, 16), ("falcon", 2112, 33), ("llama", 4096, 32), ("falcon", 4544, 71),
                                                  ("llama", 4608, 36), ("llama", 4672, 73)])       # up to 2048 / 4096 / 4608 columns, and beyond
-@pytest.mark.parametrize("lens", [[513], [300, 220], [521], [519, 9]])      # 513, 520, 521, 528 rows: remainders of 8 and of 16, whole halves
+@pytest.mark.parametrize("lens", [[513], [1025], [600, 440], [1033]])      # a row per workgroup up to 1024 rows; tiles: remainders of 8 and of 16
 def test_norm_tiles(gpu, family, hidden, heads, lens):
-    """The prompt's norms in tiles of eight rows (also with a residual add left as slices) against one wave per row: an operand may round
-    the other way, one bf16 step of 2^-8."""
+    """The prompt's norms in tiles of eight rows (also with a residual add left as slices) or a row per workgroup against one wave per row.
+    The sums differ in order, so an operand may round the other way, one bf16 step of 2^-8; three norms lie on the way to the logits
+    (before attention, before the FFN, before the head): 3 * 2^-8."""
     kv = 1 if family == "falcon" else heads
     cfg = gpu.synth.tiny_config(family, hidden=hidden, num_heads=heads, num_kv_heads=kv, head_dim=hidden // heads,
-                                ffn_dim=512, num_layers=1, max_seq_len=600)
+                                ffn_dim=512, num_layers=1, max_seq_len=1100)
     w = gpu.synth.make_weights(cfg, seed=6, scale=0.02)
     r = np.random.default_rng(hidden)
     prompts = [r.integers(0, cfg["vocab_size"], t).tolist() for t in lens]
     got = []
     for tiles in (1, 0):
         old = gpu.lib().nvl_set_tuning(9, tiles)
-        m = gpu.HipTransformerModel(cfg, w, precision="bf16", max_seqs=len(lens), max_batch_tokens=1024)
+        m = gpu.HipTransformerModel(cfg, w, precision="bf16", max_seqs=len(lens), max_batch_tokens=2048)
         try:
             for i in range(len(lens)):
                 m.seq_reset(i)
@@ -286,4 +287,4 @@ def test_norm_tiles(gpu, family, hidden, heads, lens):
         finally:
             gpu.lib().nvl_set_tuning(9, old)
             m.close()
-    assert np.isfinite(got[0]).all() and rel_err(got[0], got[1]) < 2.0 ** -8
+    assert np.isfinite(got[0]).all() and rel_err(got[0], got[1]) < 3 * 2.0 ** -8
