@@ -1427,11 +1427,16 @@ void tp_allreduce(nvl_model* m, float* buf, int64_t count) {
     }
 }
 
+static int g_defer_norm = 1;   // nvl_set_tuning key 3: deferred RMSNorm between O-proj and FFN-up in decode (0 = off)
+// Does a residual projection that carries a norm run a workgroup per (column tile, 16-row tile), all of K each (gemm.h GemmArgs::m_split)?  Not under
+// key 3 = 2 / 3, nor with several weight tiles per workgroup forced (key 2): those take the plain narrow form.
+bool defer_tiles() { return g_defer_norm == 1 && g_force_ntw != 2 && g_force_ntw != 4; }
 static int g_half_tiles = 1;   // nvl_set_tuning key 27: deferred-norm residual projections of <= 16 rows on 8-row half tiles (gemm.h HALF)
 // (producer and consumer agree through M alone: every projection of a pass has the same row count)
 // (only while the 16-row tiles leave CUs idle: at H = 4096 — 256 tiles — the halves doubled the x^2 partials every consumer
 // sums and the workgroups that each fetch the activations: Llama-3-8B B = 16 FFN-down 23.7 -> 34.2 us, O 9.3 -> 12.4 us)
-bool defer_half(const nvl_model* m, int M) { return g_half_tiles && M <= 16 && m->H % 128 == 0 && m->H / 16 < 256; }
+// (and only in the form that has half tiles: producer and consumer would disagree about the partials otherwise)
+bool defer_half(const nvl_model* m, int M) { return defer_tiles() && g_half_tiles && M <= 16 && m->H % 128 == 0 && m->H / 16 < 256; }
 // after a forward's stream sync: did a P2P wait give up?  (a peer died or never called: the residual stream is garbage)
 void p2p_check(nvl_model* m) {
     if (!m->p2p_ready) return;
@@ -1482,7 +1487,6 @@ static int g_moe_small = 1;    // nvl_set_tuning key 8: fused MoE planning launc
 static int g_mamba_ssd = 1;    // nvl_set_tuning key 30: chunked (SSD) Mamba2 scan on MFMA for prefill-sized bf16 calls (0 = the sequential scan,
                                // 2 = chunk after chunk only, never the chunk-parallel three-launch form)
 static int g_decode_seam = 1;  // nvl_set_tuning key 7: decode_seam_kernel in nvl_decode_greedy (0 = separate kernels)
-static int g_defer_norm = 1;   // nvl_set_tuning key 3: deferred RMSNorm between O-proj and FFN-up in decode (0 = off)
 static int g_mid_resid_rows = 256;   // nvl_set_tuning key 40: up to here one launch completes a residual projection of a decode batch or short prompt (gemm_mid_bf16_kernel)
 static int g_sk_slices = 0;    // tuning override (nvl_set_tuning key 1): 0 automatic, 1 = never split
 // consumer side of the deferred RMSNorm: the projection reads xn_raw and scales its accumulators (gemm.h)
@@ -1512,7 +1516,7 @@ void resid_gemm(nvl_model* m, const void* A, int lda, const void* W, const float
     }
     GemmArgs a = mk(A, lda, W, m->x, N, bias, alpha, M, N, K);
     if (defer_norm_w) {     // deferred RMSNorm: x complete in this launch (no K split over workgroups) + xn_raw + x^2 partials
-        a.nrm_w = defer_norm_w; a.nrm_xn = (bf16_t*)m->xn; a.rs_out = m->rs_part; a.m_split = g_defer_norm >= 2 ? 0 : 1;
+        a.nrm_w = defer_norm_w; a.nrm_xn = (bf16_t*)m->xn; a.rs_out = m->rs_part; a.m_split = defer_tiles() ? 1 : 0;
         a.rs_half = a.m_split && N == m->H && defer_half(m, M) ? 1 : 0;
         if (scale) { a.rs_in = scale->part; a.rs_tiles = scale->tiles; a.rs_inv_h = 1.0f / (float)scale->width; a.rs_eps = scale->eps; }
         gemm(m, EPI_RESID, true, a);

@@ -1,0 +1,46 @@
+"""Decode steps under the documented settings that change which projections a deferred norm rides on (nvl_set_tuning keys 2, 3, 27): the same
+numbers as the fp32 mode whatever the form."""
+import numpy as np
+import pytest
+
+from conftest import rel_err
+
+pytestmark = pytest.mark.gpu
+TOL = 1.5e-2
+
+CONFIGS = {
+    "llama": ("llama", dict(num_layers=3)),
+    "moe": ("granite_moe", dict(num_layers=3, embedding_multiplier=1.0, residual_multiplier=1.0, num_experts_per_tok=8)),      # all eight: no near tie between experts
+}
+
+
+@pytest.mark.parametrize("name", list(CONFIGS))
+@pytest.mark.parametrize("n", [1, 16, 17, 40])                  # half tiles of 8 columns up to 16 rows, whole tiles above
+def test_settings_keep_the_numbers(gpu, name, n):
+    family, over = CONFIGS[name]
+    cfg = gpu.synth.tiny_config(family, **over)
+    w = gpu.synth.make_weights(cfg, seed=31, scale=0.05)
+    r = np.random.default_rng(n)
+    prompts = [r.integers(0, cfg["vocab_size"], 2 + i % 3).tolist() for i in range(n)]
+    steps = r.integers(0, cfg["vocab_size"], (2, n)).tolist()
+    ids = list(range(n))
+
+    def logits(m):
+        for i in ids:
+            m.seq_reset(i)
+        m.forward_batch(ids, prompts, [0] * n, want_logits=False)
+        return np.stack([m.forward_batch(ids, [[t] for t in s], [len(p) + j for p in prompts])[0] for j, s in enumerate(steps)])
+
+    m = gpu.HipTransformerModel(cfg, w, precision="f32", max_seqs=n, max_batch_tokens=256)
+    want = logits(m)
+    m.close()
+    m = gpu.HipTransformerModel(cfg, w, precision="bf16", max_seqs=n, max_batch_tokens=256)
+    errs = {}
+    for key, value in ((3, 1), (3, 0), (3, 2), (3, 3), (2, 1), (2, 2), (2, 4), (27, 0)):
+        old = gpu.lib().nvl_set_tuning(key, value)
+        try:
+            errs[key, value] = rel_err(logits(m), want)
+        finally:
+            gpu.lib().nvl_set_tuning(key, old)
+    m.close()
+    assert max(errs.values()) <= TOL, errs
