@@ -1627,7 +1627,7 @@ static inline bool launch_gemm_skinny_ntw(hipStream_t st, const GemmArgs& a) {
                            (size_t)NTW * ks * 64 * 16, st, a);
         return true;
     }
-    if (EPI == EPI_RESID && a.rs_half && !a.moe_gate) return false;      // (half tiles: the form above alone)
+    if (EPI == EPI_RESID && !a.moe_gate && (a.rs_half || a.rs_in)) return false;      // (half tiles, scaled rows: the form above alone)
     // waves per launch: enough to cover HBM latency on every CU (~2-4 thousand), not more — extra K slices only
     // shorten each wave's stream below the depth of its two-block pipeline (r01 sweeps: LM head, W1)
     int ksplit = 16;

@@ -1497,6 +1497,7 @@ void set_deferred_in(nvl_model* m, GemmArgs& a) {
 struct RowScale { const float* part; int tiles, width; float eps; };
 void resid_gemm(nvl_model* m, const void* A, int lda, const void* W, const float* bias, float alpha, int M, int N, int K,
                 const float* defer_norm_w = nullptr, const RowScale* scale = nullptr) {
+    if (scale && (!defer_norm_w || m->tp > 1 || m->tp_force)) throw std::runtime_error("resid_gemm: a row scale needs the projection that carries the next norm");
     if (m->tp > 1 || m->tp_force) {
         // row-parallel projection: this rank holds a K slice -> fp32 partial [M][N] (the bias lives on rank 0 only),
         // all-reduce over the tensor-parallel group, then the residual add (folded into the next norm for decode)
@@ -1881,8 +1882,9 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
             a.tail_slot_stride = m->conv_tail_slot_stride;
             // both norms of the layer and the next one's can be carried by the projections in front of them (see below)
             const bool defer = defer_ok && m->pending_slices == 0 && !l.t[NVL_T_FFN_NORM_B].present();
+            // (step: the output projection scales its rows by the gated norm, which only that form of it does)
             const int per_thread = m->m_ss / (256 / m->m_hd);
-            const bool step = defer && max_len == 1 && !a.chain && m->m_nh % 16 == 0 && m->mEH % 32 == 0 && m->m_hd <= 64 && m->m_ss <= 256 && per_thread >= 4;
+            const bool step = defer && defer_tiles() && !tp_on && max_len == 1 && !a.chain && m->m_nh % 16 == 0 && m->mEH % 32 == 0 && m->m_hd <= 64 && m->m_ss <= 256 && per_thread >= 4;
             if (step) {
                 KScope ks(m, KC_OTHER, 2.0 * 3.0 * (double)M * m->mEH * m->m_ss, KS_MAMBA_SCAN,
                           (double)M * (m->mP * 4.0 + m->mEH * 2.0) + 2.0 * n_seqs * (double)m->ssm_layer_stride * 4.0);

@@ -11,6 +11,7 @@ TOL = 1.5e-2
 CONFIGS = {
     "llama": ("llama", dict(num_layers=3)),
     "moe": ("granite_moe", dict(num_layers=3, embedding_multiplier=1.0, residual_multiplier=1.0, num_experts_per_tok=8)),      # all eight: no near tie between experts
+    "hybrid": ("granite_hybrid", dict(hidden=256, mamba_num_heads=16, mamba_head_dim=32, embedding_multiplier=1.0, residual_multiplier=1.0)),      # 16 heads: the one-launch Mamba-2 step
 }
 
 
