@@ -45,3 +45,22 @@ def test_settings_keep_the_numbers(gpu, name, n):
             gpu.lib().nvl_set_tuning(key, old)
     m.close()
     assert max(errs.values()) <= TOL, errs
+
+
+@pytest.mark.parametrize("n,ffn", [(8, 4096), (8, 8256), (40, 2048), (40, 4160)])      # up to and beyond 32 blocks of an expert's k-steps a wave
+def test_wide_experts(gpu, n, ffn):
+    """The experts' down projection of a decode batch, an expert of any width a wave, against experts sorted into grouped products (key 22 = 0)."""
+    cfg = gpu.synth.tiny_config("granite_moe", ffn_dim=ffn, num_experts=4, num_layers=2)
+    m = gpu.HipTransformerModel(cfg, gpu.synth.make_weights(cfg, seed=7, scale=0.05), precision="bf16", max_seqs=n, max_batch_tokens=128)
+    ids, got = list(range(n)), []
+    for dense in (1, 0):
+        old = gpu.lib().nvl_set_tuning(22, dense)
+        try:
+            for i in ids:
+                m.seq_reset(i)
+            m.forward_batch(ids, [[3 + i] for i in ids], [0] * n, want_logits=False)
+            got.append(m.forward_batch(ids, [[9 + i] for i in ids], [1] * n)[0])
+        finally:
+            gpu.lib().nvl_set_tuning(22, old)
+    m.close()
+    assert rel_err(got[0], got[1]) <= TOL
