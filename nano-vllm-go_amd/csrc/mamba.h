@@ -153,7 +153,7 @@ __global__ __launch_bounds__(256) void mamba_tail_kernel(MambaArgs p) {
 template <int PER>
 __global__ __launch_bounds__(256) void mamba_scan_kernel(MambaArgs p) {
     const int h = blockIdx.x, seq = blockIdx.y;
-    const int SG = 256 / p.hd;                       // host guarantees hd | 256, SG a power of two <= 64, SG * PER == ss
+    const int SG = 256 / p.hd;                       // host: hd | 256, SG a power of two <= 64, SG * PER == ss (nvllm.hip mamba_states)
     const int d = threadIdx.x / SG, sg = threadIdx.x % SG;
     const int t0 = p.seq_tok_start[seq], n = p.seq_len[seq];
     float* st = p.state + (int64_t)p.seq_slot[seq] * p.state_slot_stride + ((int64_t)h * p.hd + d) * p.ss + sg * PER;
@@ -201,7 +201,7 @@ template <int PER>
 __global__ __launch_bounds__(256) void mamba_step_kernel(MambaArgs p, bf16_t* __restrict__ yn, float* __restrict__ rs) {
     __shared__ __attribute__((aligned(16))) float bc[512], yv[64];
     const int h = blockIdx.x, seq = blockIdx.y, t = p.seq_tok_start[seq];
-    const int SG = 256 / p.hd, d = threadIdx.x / SG, sg = threadIdx.x % SG;      // (host: hd | 256, SG * PER == ss <= 256, hd <= 64)
+    const int SG = 256 / p.hd, d = threadIdx.x / SG, sg = threadIdx.x % SG;      // (host: hd | 256, SG * PER == ss <= 256, hd <= 64: nvllm.hip mamba_states)
     f32x4* st = (f32x4*)(p.state + (int64_t)p.seq_slot[seq] * p.state_slot_stride + ((int64_t)h * p.hd + d) * p.ss) + sg;
     f32x4 s[PER / 4];
     if (p.seq_pos[seq] == 0) {

@@ -1805,6 +1805,14 @@ void tap_layer(nvl_model* m, int li, int M) {
     NVL_HIP(hipGetLastError());
 }
 
+// states a thread of mamba_scan_kernel / mamba_step_kernel holds: 4, 8 .. 32 (nvl_create), an instance for each
+template <int PER = 4, typename F>
+void mamba_states(int per, F&& launch) {
+    if constexpr (PER > 32) throw std::runtime_error("mamba: no kernel for these states per thread");
+    else if (per == PER) launch(std::integral_constant<int, PER>{});
+    else mamba_states<PER + 4>(per, launch);
+}
+
 // Enqueue ONE forward pass (embedding ... argmax) on the model's stream for the batch described by the device
 // metadata `md` — no host synchronisation.  Returns the number of logits rows produced.
 // seam: 0 = whole pass; bit 0 = x and layer 0's normed operand are already in place (skip embed + first norm);
@@ -1889,9 +1897,7 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
                 KScope ks(m, KC_OTHER, 2.0 * 3.0 * (double)M * m->mEH * m->m_ss, KS_MAMBA_SCAN,
                           (double)M * (m->mP * 4.0 + m->mEH * 2.0) + 2.0 * n_seqs * (double)m->ssm_layer_stride * 4.0);
                 const dim3 grid(m->m_nh, n_seqs);
-#define NVL_STEP(PERv) hipLaunchKernelGGL(mamba_step_kernel<PERv>, grid, dim3(256), 0, m->stream, a, (bf16_t*)m->myn, m->mrs)
-                if (per_thread <= 4) NVL_STEP(4); else if (per_thread <= 8) NVL_STEP(8); else if (per_thread <= 16) NVL_STEP(16); else NVL_STEP(32);
-#undef NVL_STEP
+                mamba_states(per_thread, [&](auto n) { hipLaunchKernelGGL(mamba_step_kernel<decltype(n)::value>, grid, dim3(256), 0, m->stream, a, (bf16_t*)m->myn, m->mrs); });
                 NVL_HIP(hipGetLastError());
             } else {
                 {
@@ -1950,10 +1956,7 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
                         else { if (m->m_ss == 128) NVL_SSD(32, 128); else if (m->m_ss == 64) NVL_SSD(32, 64); else NVL_SSD(32, 32); }
                     } else
 #undef NVL_SSD
-                    if (per <= 4) hipLaunchKernelGGL(mamba_scan_kernel<4>, grid, dim3(256), 0, m->stream, a);
-                    else if (per <= 8) hipLaunchKernelGGL(mamba_scan_kernel<8>, grid, dim3(256), 0, m->stream, a);
-                    else if (per <= 16) hipLaunchKernelGGL(mamba_scan_kernel<16>, grid, dim3(256), 0, m->stream, a);
-                    else hipLaunchKernelGGL(mamba_scan_kernel<32>, grid, dim3(256), 0, m->stream, a);
+                    mamba_states(per, [&](auto n) { hipLaunchKernelGGL(mamba_scan_kernel<decltype(n)::value>, grid, dim3(256), 0, m->stream, a); });
                     NVL_HIP(hipGetLastError());
                 }
                 {

@@ -219,3 +219,30 @@ def test_hybrid_is_refused_where_it_cannot_work(gpu):
     bad = dict(cfg, mamba_num_heads=3)                      # heads x head_dim != expand x hidden
     with pytest.raises(gpu.NvlError):
         gpu.HipTransformerModel(bad, None)
+
+
+@pytest.mark.parametrize("precision", ["f32", "bf16"])
+@pytest.mark.parametrize("head_dim,per", [(64, 12), (32, 20), (32, 24), (16, 12), (16, 28), (64, 32), (32, 4)])      # states a thread of the kernels holds
+def test_states_per_thread(gpu, oracle, precision, head_dim, per):
+    """Every number of states that nvl_create accepts, prompt and decode steps (16 or 32 heads: the one-launch step) of two sequences side by side:
+    no channel touches its neighbour's states."""
+    heads = 16 if head_dim >= 32 else 32
+    hidden, state = heads * head_dim // 2, 256 // head_dim * per
+    cfg, w, hm = build(gpu, oracle, precision, hidden=hidden, num_heads=2, num_kv_heads=1, mamba_num_heads=heads, mamba_head_dim=head_dim, mamba_state_size=state)
+    r = np.random.default_rng(per)
+    prompts = [r.integers(0, cfg["vocab_size"], n).tolist() for n in (7, 19)]
+    oms = [oracle.OracleModel(cfg, w) for _ in prompts]
+    kvs = [om.new_cache() for om in oms]
+    tokens = r.integers(0, cfg["vocab_size"], (3, 2)).tolist()
+    for i in range(2):
+        hm.seq_reset(i)
+    got = [hm.forward_batch([0, 1], prompts, [0, 0])[0]]
+    got += [hm.forward_batch([0, 1], [[t] for t in s], [len(p) + j for p in prompts])[0] for j, s in enumerate(tokens)]
+    for i, p in enumerate(prompts):
+        want = [oms[i].forward_with_cache(p, kvs[i], 0)[-1]] + [oms[i].forward_with_cache([s[i]], kvs[i], len(p) + j)[-1] for j, s in enumerate(tokens)]
+        for a, b in zip(got, want):
+            assert rel_err(a[i], b) <= TOL[precision]
+        for li, kind in enumerate(cfg["hybrid_layers"]):
+            if kind == "mamba":
+                assert rel_err(hm.get_mamba_state(i, li), oms[i].mamba_state(li)) <= TOL[precision]
+    hm.close()
