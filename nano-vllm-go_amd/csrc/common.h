@@ -90,6 +90,14 @@ struct KeyMask {
     bool operator==(const KeyMask& o) const { return window == o.window && chunk == o.chunk && keep == o.keep; }
 };
 
+// Routing scores as integers in the same order, every NaN above all numbers and equal to the others (and -0 equal to 0): ranks by these, ties by
+// index, name each place once whatever the scores are.  Ranks by the floats gave all experts of a NaN row the first place and left the
+// other places of its list unwritten, and what lay there was taken for expert numbers.
+__device__ __forceinline__ int score_key(float x) {
+    const int b = __builtin_bit_cast(int, x + 0.0f);
+    return x != x ? 0x7fffffff : b >= 0 ? b : b ^ 0x7fffffff;
+}
+
 __device__ __forceinline__ float gelu_tanh_f(float x) {
     // tensor.go:181-190: 0.5 x (1 + tanh(sqrt(2/pi) (x + 0.044715 x^3))), the tanh in float64 there.
     // tanh(u) = 1 - 2 / (exp(2u) + 1) on the hardware exp2 / rcp (both ~1 ulp): ABSOLUTE error ~1e-7, and only the absolute

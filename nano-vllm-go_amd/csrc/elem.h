@@ -1001,11 +1001,11 @@ __device__ __forceinline__ void moe_route_row(const float* __restrict__ logits_r
     // rank of this lane's probability: larger first, ties to the lower index — the order the reference's repeated
     // argmax visits them (moe.go:75-92).  64 register broadcasts instead of top_k dependent butterfly reductions.
     int rank = 0;
-    const int pbits = __builtin_bit_cast(int, prob);
+    const int pbits = __builtin_bit_cast(int, prob), key = score_key(prob);
 #pragma unroll 8
     for (int j = 0; j < E; j++) {       // (lanes >= E hold -1: they never outrank an expert)
-        const float pj = __builtin_bit_cast(float, __builtin_amdgcn_readlane(pbits, j));
-        rank += (pj > prob || (pj == prob && j < lane)) ? 1 : 0;
+        const int kj = __builtin_amdgcn_readlane(key, j);
+        rank += (kj > key || (kj == key && j < lane)) ? 1 : 0;
     }
     float wsum = 0.f;
     for (int k = 0; k < top_k; k++) {     // moe.go:89-92: fp32 sum in rank order
@@ -1041,11 +1041,11 @@ __global__ __launch_bounds__(256) void moe_gate_kernel(const float* __restrict__
     const float s = wave_sum(e);
     const float prob = (lane < E) ? e / s : -1.f;
     int rank = 0;                                   // as moe_route_row: larger first, ties to the lower index
-    const int pbits = __builtin_bit_cast(int, prob);
+    const int pbits = __builtin_bit_cast(int, prob), key = score_key(prob);
 #pragma unroll 8
     for (int j = 0; j < E; j++) {       // (lanes >= E hold -1: they never outrank an expert)
-        const float pj = __builtin_bit_cast(float, __builtin_amdgcn_readlane(pbits, j));
-        rank += (pj > prob || (pj == prob && j < lane)) ? 1 : 0;
+        const int kj = __builtin_amdgcn_readlane(key, j);
+        rank += (kj > key || (kj == key && j < lane)) ? 1 : 0;
     }
     float wsum = 0.f;
     for (int k = 0; k < top_k; k++) {               // moe.go:89-92: fp32 sum in rank order
@@ -1142,7 +1142,8 @@ struct GroupRouteArgs { const float* logits; int64_t ld; const float* correction
                         int softmax, n_always; };                                                // n_always: gate columns E .. that are one
 template <typename ActT>
 __global__ __launch_bounds__(256) void moe_route_grouped_kernel(GroupRouteArgs p) {
-    __shared__ float choice_s[4][ROUTE_MAX_E], group_s[4][ROUTE_MAX_E];
+    __shared__ float choice_s[4][ROUTE_MAX_E];
+    __shared__ int group_s[4][ROUTE_MAX_E], key_s[4][ROUTE_MAX_E];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = blockIdx.x * 4 + wave;
     if (blockIdx.y > 0) {
         const int f = (blockIdx.y - 1) * 256 + lane * 4;
@@ -1155,7 +1156,8 @@ __global__ __launch_bounds__(256) void moe_route_grouped_kernel(GroupRouteArgs p
         return;
     }
     const int size = p.E / p.groups;
-    float *choice = choice_s[wave], *group = group_s[wave];
+    float* choice = choice_s[wave];
+    int *group = group_s[wave], *key = key_s[wave];
     float s[ROUTE_MAX_E / 64];
     if (r < p.rows)
 #pragma unroll
@@ -1176,12 +1178,12 @@ __global__ __launch_bounds__(256) void moe_route_grouped_kernel(GroupRouteArgs p
                 const float c = choice[g * size + j];
                 if (c > a) { b = a; a = c; } else b = fmaxf(b, c);
             }
-            group[g] = size > 1 ? a + b : a;
+            group[g] = score_key(size > 1 ? a + b : a);
         }
     __syncthreads();
     auto kept = [&](int g) {
         int rank = 0;
-        const float v = group[g];
+        const int v = group[g];
         for (int j = 0; j < p.groups; j++) rank += group[j] > v || (group[j] == v && j < g);
         return rank < p.keep;
     };
@@ -1192,7 +1194,7 @@ __global__ __launch_bounds__(256) void moe_route_grouped_kernel(GroupRouteArgs p
         const int e = lane + 64 * i;
         in[i] = r < p.rows && e < p.E && kept(e / size);
         c[i] = r < p.rows && e < p.E ? choice[e] : 0.f;
-        if (r < p.rows && e < p.E && !in[i]) choice[e] = -INFINITY;       // (read by nobody but this lane so far)
+        if (r < p.rows && e < p.E) key[e] = in[i] ? score_key(c[i]) : -0x7fffffff - 1;       // (below every score)
     }
     __syncthreads();
     int ranks[ROUTE_MAX_E / 64];
@@ -1201,7 +1203,7 @@ __global__ __launch_bounds__(256) void moe_route_grouped_kernel(GroupRouteArgs p
     for (int i = 0; i < ROUTE_MAX_E / 64; i++) {
         const int e = lane + 64 * i;
         ranks[i] = p.top;
-        if (in[i]) { ranks[i] = 0; for (int j = 0; j < p.E; j++) { const float v = choice[j]; ranks[i] += v > c[i] || (v == c[i] && j < e); } }
+        if (in[i]) { ranks[i] = 0; const int own = key[e]; for (int j = 0; j < p.E; j++) { const int v = key[j]; ranks[i] += v > own || (v == own && j < e); } }
         if (in[i]) top_z = fmaxf(top_z, c[i]);
     }
     if (p.softmax) {

@@ -1307,11 +1307,11 @@ static __global__ __launch_bounds__(1024) void moe_router_gate_kernel(GemmArgs p
     for (int o = 1; o < 64; o <<= 1) sum += __shfl_xor(sum, o, 64);
     const float prob = (lane < E) ? e / sum : -1.f;
     int rank = 0;                                   // larger first, ties to the lower index (moe.go:75-92)
-    const int pbits = __builtin_bit_cast(int, prob);
+    const int pbits = __builtin_bit_cast(int, prob), key = score_key(prob);
 #pragma unroll 8
     for (int j = 0; j < E; j++) {                   // (lanes >= E hold -1: they never outrank an expert)
-        const float pj = __builtin_bit_cast(float, __builtin_amdgcn_readlane(pbits, j));
-        rank += (pj > prob || (pj == prob && j < lane)) ? 1 : 0;
+        const int kj = __builtin_amdgcn_readlane(key, j);
+        rank += (kj > key || (kj == key && j < lane)) ? 1 : 0;
     }
     float wsum = 0.f;
     for (int k = 0; k < top_k; k++) {               // moe.go:89-92: fp32 sum in rank order
