@@ -144,6 +144,7 @@ struct GemmArgs {
     // projection's K reduction the weighted combine itself (moe.go:105-120) — no sort, no plan, no combine launch.
     const float* moe_gate;
     int moe_E, moe_I;
+    int64_t split_bytes;    // size of split_ws (for the launchers)
 };
 // does any row of the batch (M <= 64: one per lane) route to expert e?  Call with all 64 lanes active.
 __device__ __forceinline__ bool moe_expert_live(const GemmArgs& p, int e) {
@@ -541,8 +542,17 @@ void gemm_bf16_kernel(GemmArgs p) {
 // written through and read past the L2 (sc0 sc1) instead of fencing, which would write back everything that XCD has dirty
 // (4096 x 2048 x 6144 in two parts: 85 us so, 156 us with __threadfence, 94 us unsplit).
 // ------------------------------------------------------------------------------------------
-constexpr int64_t SPLIT_WS_BYTES = 64ll << 20;      // 256 parts of 256 x 256 fp32, or 512 of 128 x 128
+constexpr int64_t SPLIT_WS_BYTES = 64ll << 20;      // all a launch can use: 256 parts of 256 x 256 fp32 (gemm_bf16_pp_kernel)
+constexpr int64_t SPLIT_MID_BYTES = 8ll << 20;      // ... gemm_mid_bf16_kernel, unless its parts are forced: 256 of 128 x 64 or 64 x 128
 constexpr int SPLIT_MAX_TILES = 512;
+constexpr int PP_MIN_STAGES = 12;                   // K-steps of 32 that a part of a 256 x 256 tile has at least
+constexpr int MID_MAX_PARTS = 8, MID_MIN_STAGES = 2;      // parts of a tile of gemm_mid_bf16_kernel; K-steps of 128 that one has at least
+// what the launches of an N x K projection of up to M rows can use of it
+static inline int64_t split_need(int64_t M, int64_t N, int64_t K) {
+    if (M > 64 && (K >> 5) >= 2 * PP_MIN_STAGES && cdiv(M, 256) * cdiv(N, 256) >= 8) return SPLIT_WS_BYTES;
+    if (cdiv(K, 128) < 2 * MID_MIN_STAGES) return 0;
+    return std::min(SPLIT_MID_BYTES, (int64_t)MID_MAX_PARTS * 4 * round_up(std::min<int64_t>(M, 512), 128) * round_up(N, 128));
+}
 constexpr int SPLIT_COHERENT = 0x11;      // buffer cache policy: sc0 | sc1
 
 // acc: this wave's F fragments; a part takes `bytes` of split_ws (waves one after the other, 1 KiB a fragment).  True in the workgroup
@@ -1711,7 +1721,7 @@ static inline double pp_cost(int M, int N, int K, int out_bytes, bool can_split,
     parts = 1;
     double best = 0;
     for (int c = 1; c <= 8 && rest * c <= 32; c++) {
-        if (c > 1 && (!can_split || !rest || T < 8 || stages / c < 12 || (g_pp_split && c != g_pp_split))) continue;
+        if (c > 1 && (!can_split || !rest || T < 8 || stages / c < PP_MIN_STAGES || (g_pp_split && c != g_pp_split))) continue;
         const double fill = rest * c / 32.0, t = rest ? (stages / c) * (0.46 + (fill > 0.45 ? 0.42 * (fill - 0.45) : 0.0)) + (c > 1 ? 10.0 + 2.5 * c : 0.0) : 0.0;
         if (c == 1 || t < 0.92 * best || g_pp_split == c) { best = t; parts = c; }
     }
@@ -1728,7 +1738,7 @@ static inline bool pp_wins(GemmArgs& a) {
     a.splits = 1;
     if (a.seg || a.a_rows || a.tile_map || a.sk_part || a.K < 160) return false;
     const int bytes = EPI == EPI_RESID ? 8 : EPI == EPI_GROUPED_RAW ? 4 : epi_glu(EPI) ? (int)sizeof(OutT) / 2 : (int)sizeof(OutT);
-    const bool parts = a.split_ws && (a.M > MID_MAX_ROWS || a.M <= std::max(64, g_chunk_max_m));      // (key 11 = 64: sums in one order whatever the rows, up to 512)
+    const bool parts = a.split_bytes >= SPLIT_WS_BYTES && (a.M > MID_MAX_ROWS || a.M <= std::max(64, g_chunk_max_m));      // (key 11 = 64: sums in one order whatever the rows, up to 512)
     return pp_cost(a.M, a.N, a.K, bytes, parts, a.splits) < 0.93 * tile128_cost(a.M, a.N, a.K, bytes, 1);
 }
 template <int EPI, typename OutT, int WAVES_N>
@@ -1773,7 +1783,6 @@ static inline void launch_gemm_grouped(hipStream_t st, const GemmArgs& a, int ma
 // What a projection of up to MID_MAX_ROWS rows takes on gemm_mid_bf16_kernel, in microseconds, and into how many parts its K goes (fitted to 8 .. 512
 // rows of 2048 .. 4544-wide models, good to 15 %): a stage of a CU moves at some 56 GB/s, all weights together at 6.6 TB/s; a part
 // more costs the hand-over 0.45 us and every round of workgroups beyond the first its ramp.
-constexpr int MID_MAX_PARTS = 8;
 static inline int mid_row_tiles(int M) { return cdiv(cdiv(M, cdiv(M, 128)), 32) * 2; }      // 16-row tiles of a row group: 2, 4, 6 or 8
 static inline double mid_cost(int M, int N, int K, int mt, int ct, bool can_split, int& parts) {
     const int tiles = cdiv(N, 32 * ct) * cdiv(M, 16 * mt), stages = cdiv(K, 128);
@@ -1781,7 +1790,7 @@ static inline double mid_cost(int M, int N, int K, int mt, int ct, bool can_spli
     double best = 0;
     parts = 1;
     for (int c = 1; c <= MID_MAX_PARTS; c++) {
-        if (c > 1 && (!can_split || tiles * c > 256 || stages / c < 2)) break;
+        if (c > 1 && (!can_split || tiles * c > 256 || stages / c < MID_MIN_STAGES)) break;
         const double rounds = cdiv(tiles * c, 256), t = std::max(rounds * cdiv(stages, c) * stage_us, hbm_us) + (c > 1 ? 2.5 + 0.45 * c : 0.0) + 2.0 * (rounds - 1);
         if (c == 1 || t < best) { best = t; parts = c; }
     }
@@ -1800,9 +1809,9 @@ template <int MT, int CT, int EPI, typename OutT>
 static inline void launch_gemm_mid_rows(hipStream_t st, const GemmArgs& a0) {
     GemmArgs a = a0;
     const int nb = cdiv(a.N, 32 * CT), groups = cdiv(a.M, 16 * MT);
-    mid_cost(a.M, a.N, a.K, MT, CT, a.split_ws != nullptr, a.splits);
-    if (a.split_ws && g_mid_splits) a.splits = std::min(g_mid_splits, std::max(1, a.K >> 7));
-    while (a.splits > 1 && (nb * groups > SPLIT_MAX_TILES || (int64_t)nb * groups * a.splits * MT * CT * 2048 > SPLIT_WS_BYTES)) a.splits--;
+    mid_cost(a.M, a.N, a.K, MT, CT, a.split_bytes > 0, a.splits);
+    if (a.split_bytes > 0 && g_mid_splits) a.splits = std::min(g_mid_splits, std::max(1, a.K >> 7));
+    while (a.splits > 1 && (nb * groups > SPLIT_MAX_TILES || (int64_t)nb * groups * a.splits * MT * CT * 2048 > a.split_bytes)) a.splits--;
     NVL_LDS_ATTR((gemm_mid_bf16_kernel<MT, CT, EPI, OutT>), (mid_lds_bytes<MT, CT>()));
     hipLaunchKernelGGL((gemm_mid_bf16_kernel<MT, CT, EPI, OutT>), dim3(cdiv(nb, 8) * 8 * groups * a.splits), dim3(512), (mid_lds_bytes<MT, CT>()), st, a);
 }
@@ -1824,7 +1833,7 @@ static inline bool mid_wins(const GemmArgs& a) {
         if (!split) while (ks > 1 && blocks * ks > g_narrow_waves) ks >>= 1;
         // a step in favour of the form that is there: 8 % is half the error of the two costs.  At 24 / 32 / 64 rows, decode form -> here:
         // 4096 x 14336 43 -> 28.6, 55 -> 29.9, 85.7 -> 32.6 us; 4544 x 18176 at 16 rows 48.7 -> 34.9; 2048 x 8192 stays at 15.3 up to 32 rows, 23.1 -> 18.4 at 64
-        return mid_cost(a.M, a.N, a.K, mid_row_tiles(a.M), 2, a.split_ws != nullptr, mid_parts) < 0.92 * narrow_cost(a.M, a.N, a.K, blocks, blocks * ks * (split ? cdiv(a.M, 16) : 1), split);
+        return mid_cost(a.M, a.N, a.K, mid_row_tiles(a.M), 2, a.split_bytes > 0, mid_parts) < 0.92 * narrow_cost(a.M, a.N, a.K, blocks, blocks * ks * (split ? cdiv(a.M, 16) : 1), split);
     }
     // (GPT-2's projections at 96 .. 104 rows: 768 x 768 12.7 us here and 8.8 in groups of the decode form, 768 x 3072 14.7 and 13.6)
     if (EPI != EPI_QKV && (a.K < 2048 || (int64_t)a.N * a.K < (4 << 20))) return false;

@@ -368,6 +368,7 @@ void* lay_alloc(nvl_model* m, int64_t bytes) {      // zero-filled
 void* lay_matrix(nvl_model* m, int64_t N, int64_t Kd) {       // zero matrix of the weight dtype; rows padded to whole GEMM tiles
     const int64_t bytes = round_up(N, W_ROW_PAD) * Kd * (int64_t)m->wsize;
     m->stats.weight_bytes += (double)bytes;
+    m->split_bytes = std::max(m->split_bytes, split_need(1 << 20, N, Kd));      // (some multiply the keys of whole contexts)
     return lay_alloc(m, bytes);
 }
 float* lay_vector(nvl_model* m, const DevTensor& t, int64_t padded) {

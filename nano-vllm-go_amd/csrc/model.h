@@ -207,6 +207,7 @@ struct nvl_model {
     void* q = nullptr;           // ActT [Mmax][nH*hd]
     void* attn_out = nullptr;    // ActT [Mmax][nH*hd]
     float* attn_part = nullptr;  // bf16: partial results of a decode attention whose keys are split over workgroups (attn.h AttnArgs::part)
+    int attn_records = 0;        // ... how many it has room for
     int32_t* attn_part_cnt = nullptr;   // ... and their arrival tickets per (sequence, kv head)
     void* hbuf = nullptr;        // ActT [Mmax][F]   (MoE: [Mmax*k][I])
     float* h2 = nullptr;         // fp32 [Mmax][2F]  (f32 mode un-fused gate|up; MoE f32 too)
@@ -229,7 +230,7 @@ struct nvl_model {
     int ctx_hint = 0;    // longest context (keys) of the batch being enqueued; 0 = unknown (decode attention sizing)
     float* sk_part = nullptr; int sk_max_slices = 4; int pending_slices = 0, pending_rows = 0; float pending_alpha = 1.f; const float* pending_part = nullptr;
     int sk_rows = 64;             // rows the sk_part slices are allocated for
-    float* split_ws = nullptr; int32_t* split_cnt = nullptr;      // K splits inside a launch (gemm.h split_finish): partial tiles, counters (zero between launches)
+    float* split_ws = nullptr; int32_t* split_cnt = nullptr; int64_t split_bytes = 0;      // K splits inside a launch (gemm.h split_finish): partial tiles, counters (zero between launches)
     const int32_t* pending_slot_of = nullptr; const float* pending_gate_w = nullptr;   // MoE combine folded into the next norm
     // per-call metadata (one pinned host block mirrored on the device)
     int32_t* meta_host = nullptr; int32_t* meta_dev = nullptr; int64_t meta_ints = 0;

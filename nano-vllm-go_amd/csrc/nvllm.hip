@@ -17,7 +17,7 @@
 using namespace nvl;
 
 static thread_local std::string g_create_err;
-constexpr int ATTN_SPLIT_RECORDS = 4096;      // split decode attention: most partial results of a launch (17 / 34 MB)
+constexpr int ATTN_SPLIT_PAIRS = 128;         // split decode attention: most (sequence, kv head, query tile) triples of a launch, unless forced
 constexpr int SK_TILE_MAX_M = 2048, SK_TILE_MAX_SLICES = 8;      // split-K of the tile kernel for mid-size residual projections (resid_gemm)
 static int g_sk_tile = 1;            // nvl_set_tuning key 26: that split (0 = off)
 constexpr int MOE_DOWN_SLICES = 4;    // at most this many K slices (workgroups per column tile) in the dense-masked MoE down projection
@@ -178,7 +178,7 @@ void gemm(nvl_model* m, int epi, bool out_f32, GemmArgs a, double flops = -1.0) 
         : ((double)a.N * a.K + (double)a.M * a.K) * (double)m->wsize + (double)a.M * a.N * (out_f32 || epi == EPI_RESID ? 4.0 : (double)m->wsize);
     KScope ks(m, KC_GEMM, flops >= 0 ? flops : 2.0 * (double)a.M * (double)a.N * (double)a.K, -1, gbytes);
     hipStream_t st = m->stream;
-    a.split_ws = m->split_ws; a.split_cnt = m->split_cnt; a.splits = 1;
+    a.split_ws = m->split_ws; a.split_cnt = m->split_cnt; a.split_bytes = m->split_bytes; a.splits = 1;
     if (m->f32) {
         switch (epi) {
             case EPI_STORE: launch_gemm_f32<EPI_STORE, float>(st, a); break;
@@ -666,10 +666,10 @@ std::vector<int32_t> swiglu_interleave(int64_t F, int64_t src_base) {
     return idx;
 }
 
-// gemm.h split_finish: launches on m->stream only, one at a time, so one workspace serves all of them
+// gemm.h split_finish: launches on m->stream only, one at a time, so one workspace (m->split_bytes, set by the caller) serves all of them
 void init_split(nvl_model* m) {
-    if (m->f32) return;
-    m->split_ws = (float*)dmalloc_bytes(SPLIT_WS_BYTES);
+    if (m->f32) { m->split_bytes = 0; return; }
+    if (m->split_bytes) m->split_ws = (float*)dmalloc_bytes(m->split_bytes);
     m->split_cnt = dmalloc<int32_t>(SPLIT_MAX_TILES);
     NVL_HIP(hipMemsetAsync(m->split_cnt, 0, SPLIT_MAX_TILES * 4, m->stream));
 }
@@ -848,9 +848,10 @@ extern "C" int nvl_finalize(nvl_model* m) {
     m->q = dmalloc_bytes(Mmax * qw * (int64_t)m->wsize);
     m->attn_out = dmalloc_bytes(Mp * qw * (int64_t)m->wsize);
     if (!m->f32 && (m->hd == 64 || m->hd == 128)) {     // partial results of a split decode attention (attn.h)
-        m->attn_part = dmalloc<float>((int64_t)ATTN_SPLIT_RECORDS * (m->hd == 64 ? attn_part_floats<64>() : attn_part_floats<128>()));
-        m->attn_part_cnt = dmalloc<int32_t>(ATTN_SPLIT_RECORDS);
-        NVL_HIP(hipMemset(m->attn_part_cnt, 0, ATTN_SPLIT_RECORDS * sizeof(int32_t)));
+        m->attn_records = (int)std::min<int64_t>(ATTN_SPLIT_PAIRS, S * m->nKV * cdiv(m->group, 16)) * ATTN_SPLIT_MAX;
+        m->attn_part = dmalloc<float>((int64_t)m->attn_records * (m->hd == 64 ? attn_part_floats<64>() : attn_part_floats<128>()));
+        m->attn_part_cnt = dmalloc<int32_t>(m->attn_records);
+        NVL_HIP(hipMemsetAsync(m->attn_part_cnt, 0, (size_t)m->attn_records * sizeof(int32_t), m->stream));
     }
     const int64_t k = c.use_moe ? c.num_experts_per_tok : 1;
     m->hbuf = dmalloc_bytes(round_up(Mmax * k, 64) * m->F * (int64_t)m->wsize);
@@ -907,6 +908,8 @@ extern "C" int nvl_finalize(nvl_model* m) {
     // split-K partial slices of the residual projections: decode (<= 64 rows) and mid-size batches (<= SK_TILE_MAX_M rows)
     m->sk_rows = (int)std::min<int64_t>(std::max<int64_t>(Mmax, 64), SK_TILE_MAX_M);
     if (!m->f32) m->sk_part = dmalloc<float>((int64_t)std::max(m->sk_max_slices, SK_TILE_MAX_SLICES) * m->sk_rows * H);
+    for (auto [N, K] : {std::pair<int64_t, int64_t>{m->n_qkv, H}, {H, qw}, {c.activation_type == NVL_ACT_SWIGLU ? 2 * m->F : m->F, H}, {H, m->F}, {m->V, H}, {m->mP, H}, {H, m->mEH}})
+        m->split_bytes = std::max(m->split_bytes, split_need(Mmax, N, K));
     init_split(m);
     if (!m->f32) m->rs_part = dmalloc<float>((int64_t)cdiv(H, 8) * DEFER_MAX_M);      // x^2 partials per 16 (half tiles: 8) columns
     if (m->tp > 1 || m->tp_force) m->tp_part = dmalloc<float>(Mmax * H);
@@ -1254,7 +1257,7 @@ int decode_attn_cfg(const nvl_model* m, int n_seqs) {
     int nw = n_kt <= 2 * per_wave ? 2 : (n_kt <= 4 * per_wave ? 4 : 8);
     nw = g_attn_nw ? g_attn_nw : std::min(nw, cap);
     auto cfg = [&](int waves, int most, int tiles) { return waves | most << 8 | tiles << 12; };
-    const int most = m->attn_part && m->ctx_hint > 0 ? std::min(ATTN_SPLIT_MAX, ATTN_SPLIT_RECORDS / wgs) : 1;
+    const int most = m->attn_part && m->ctx_hint > 0 ? std::min(ATTN_SPLIT_MAX, m->attn_records / wgs) : 1;
     if (g_attn_split >= 2) { const int tiles = (g_attn_split - 1) * nw * per_wave; return cfg(nw, std::max(1, std::min(most, cdiv(n_kt, tiles))), tiles); }
     if (g_attn_split && !g_attn_nw && most > 1) {
         int waves = 0;
@@ -1382,7 +1385,7 @@ GemmArgs mk(const void* A, int lda, const void* W, void* C, int ldc, const float
     a.M = M; a.N = N; a.K = K; a.seg = nullptr; a.c_row0 = 0;
     a.qkv = QkvEpi{};
     a.tile_map = nullptr; a.n_mtiles = nullptr; a.w_expert_stride = 0;
-    a.sk_part = nullptr; a.sk_slices = 1; a.split_ws = nullptr; a.split_cnt = nullptr; a.splits = 1; a.m_split = 0; a.rs_half = 0; a.grid_y = 1; a.nrm_w = nullptr; a.nrm_xn = nullptr; a.rs_out = nullptr; a.rs_in = nullptr; a.rs_tiles = 0; a.rs_inv_h = 0.f; a.rs_eps = 0.f;
+    a.sk_part = nullptr; a.sk_slices = 1; a.split_ws = nullptr; a.split_cnt = nullptr; a.split_bytes = 0; a.splits = 1; a.m_split = 0; a.rs_half = 0; a.grid_y = 1; a.nrm_w = nullptr; a.nrm_xn = nullptr; a.rs_out = nullptr; a.rs_in = nullptr; a.rs_tiles = 0; a.rs_inv_h = 0.f; a.rs_eps = 0.f;
     return a;
 }
 
@@ -1543,7 +1546,7 @@ void resid_gemm(nvl_model* m, const void* A, int lda, const void* W, const float
         if (tiles * slices < 64) slices = 1;
         // ... unless large tiles whose K is cut inside the launch are faster (1024 x 4096 x 14336: 118 us, and no slices for the norm)
         int parts;
-        if (slices > 1 && M > 256 && pp_cost(M, N, K, 8, m->split_ws != nullptr, parts) < 0.72 * tile128_cost(M, N, K, 8, slices)) slices = 1;
+        if (slices > 1 && M > 256 && pp_cost(M, N, K, 8, m->split_bytes >= SPLIT_WS_BYTES, parts) < 0.72 * tile128_cost(M, N, K, 8, slices)) slices = 1;
     }
     if (slices > 1) {
         a.sk_part = m->sk_part; a.sk_slices = slices;

@@ -16,13 +16,13 @@ struct OpCtx {   // a model-less nvl_model carrying just a stream and the fields
         m.f32 = precision == NVL_PRECISION_F32;
         m.wsize = m.f32 ? 4 : 2;
         NVL_HIP(hipStreamCreateWithFlags(&m.stream, hipStreamNonBlocking));
-        init_split(&m);
     }
     ~OpCtx() {
         if (m.stream) { (void)hipStreamSynchronize(m.stream); (void)hipStreamDestroy(m.stream); }
         for (void* p : bufs) dfree(p);
         dfree(m.split_ws); dfree(m.split_cnt);
     }
+    void will_multiply(int M, int N, int K) { m.split_bytes = split_need(M, N, K); init_split(&m); }
     void* alloc(int64_t bytes) { void* p = dmalloc_bytes(bytes); bufs.push_back(p); return p; }
     float* up_f32(const float* h, int64_t n) {
         float* d = (float*)alloc(n * 4);
@@ -69,6 +69,7 @@ extern "C" int nvl_op_matmul(int device, int precision, const float* a, const fl
     if (K % 64 != 0) return op_fail("nvl_op_matmul: K must be a multiple of 64");
     OP_TRY
     OpCtx cx(device, precision);
+    cx.will_multiply(M, N, K);
     void* A = cx.up_mat(a, M, K, false);
     void* W = cx.up_mat(b, N, K, true, W_ROW_PAD);
     const int ldc = (int)round_up(N, 4);
@@ -237,6 +238,7 @@ extern "C" int nvl_op_ffn(int device, int precision, const float* x, const float
     m.xn = cx.up_mat(x, rows, hidden, false);
     LayerW l;
     const int n1 = swiglu ? 2 * ffn : ffn;
+    cx.will_multiply(rows, std::max(n1, hidden), std::max(hidden, ffn));
     void* w1c = cx.up_mat(w1, n1, hidden, true, W_ROW_PAD);   // canonical [n1][H] (gate rows | up rows)
     if (swiglu && !m.f32) {
         auto idx = swiglu_interleave(ffn, 0);
@@ -352,6 +354,7 @@ extern "C" int nvl_bench_gemm(int device, int M, int N, int K, int epi, int forc
     if (!avg_us || M <= 0 || N <= 0 || K % 64 || iters <= 0) return op_fail("nvl_bench_gemm: bad arguments");
     OP_TRY
     OpCtx cx(device, NVL_PRECISION_BF16);
+    cx.will_multiply(M, N, K);
     const int64_t Np = round_up(N, W_ROW_PAD);
     std::vector<uint16_t> ha((size_t)round_up(M, 64) * K), hw((size_t)Np * K);
     uint32_t s = 12345u;

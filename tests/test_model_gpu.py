@@ -536,3 +536,20 @@ def test_mqa_decode_with_more_than_16_query_heads(gpu, oracle, precision):
         _, cur = hm.forward_batch(ids, [[int(t)] for t in cur], [len(prompts[i]) + s for i in ids], want_logits=False)
         assert (fused[s] == cur).all()
     hm.close()
+
+
+@pytest.mark.parametrize("family", ["llama", "gpt2", "granite_moe", "granite_hybrid"])
+def test_small_models_take_little_memory(gpu, family):
+    """Workspaces are sized by what the model's shapes can use: a model of a few MiB of weights, cache and activations stays below 40 MiB."""
+    import torch
+    cfg = gpu.synth.tiny_config(family)
+    w = gpu.synth.make_weights(cfg, seed=1)
+    gpu.HipTransformerModel(cfg, w, precision="bf16", max_seqs=1, max_batch_tokens=64).close()      # (what the first model of a process sets up)
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    m = gpu.HipTransformerModel(cfg, w, precision="bf16", max_seqs=1, max_batch_tokens=64)
+    m.seq_reset(0)
+    m.forward_batch([0], [[1, 2, 3]], [0])
+    used = before - torch.cuda.mem_get_info()[0]
+    m.close()
+    assert used < 40 << 20
