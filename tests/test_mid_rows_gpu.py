@@ -13,31 +13,33 @@ TOL = 1.5e-2
 @pytest.mark.parametrize("m,k,n", [(65, 2048, 64), (66, 2112, 200), (96, 2048, 130), (97, 4160, 2048), (128, 2048, 1003), (129, 2048, 256),
                                    (255, 2176, 320), (257, 2048, 2049), (512, 2048, 192), (1, 4096, 64), (33, 1984, 2049), (64, 64, 33)])
 def test_matmul_is_exact_on_integers(gpu, parts, m, k, n):
-    """Ragged rows, columns and K (a last stage of 64, K parts of unequal length); the sums are exact in fp32 in any order, twice in a
-    row (the counters of a split are zero again)."""
+    """Ragged rows, columns and K (a last stage of 64, K parts of unequal length), the kernel forced (by cost it would take few of these); the
+    sums are exact in fp32 in any order."""
     a = (np.arange(m * k).reshape(m, k) % 7).astype(np.float32) - 1.0
     b = (np.arange(k * n).reshape(k, n) % 5).astype(np.float32) - 2.0        # |sums| < 2^24
-    old = [(key, gpu.lib().nvl_set_tuning(key, v)) for key, v in ((39, parts), (38, 2 if m <= 64 else 1))]
+    old = [(key, gpu.lib().nvl_set_tuning(key, v)) for key, v in ((39, parts), (38, 2))]
     try:
-        got = [gpu.ops.mat_mul(a, b, precision="bf16") for _ in range(2)]
+        got = gpu.ops.mat_mul(a, b, precision="bf16")
     finally:
         for key, v in old:
             gpu.lib().nvl_set_tuning(key, v)
     want = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32)
-    assert np.array_equal(got[0], want) and np.array_equal(got[1], want)
+    assert np.array_equal(got, want)
 
 
 @pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("parts", [0, 3])                             # K split over workgroups; 0: the launcher's choice
 @pytest.mark.parametrize("n,mid", [(5, 2), (33, 2), (64, 1), (64, 2), (65, 1), (97, 1), (128, 1), (130, 1)])      # 130: past the deferred norm
-def test_decode_and_prompt_batches(gpu, hd, n, mid):
+def test_decode_and_prompt_batches(gpu, hd, parts, n, mid):
     """Every epilogue of the kernel in a model: decode batches (deferred norms, gate | up pairs) and short prompts (rotated heads, cache rows)
-    against the fp32 mode, and the greedy loop (graph replays) against single steps."""
+    against the fp32 mode; the same prompts again, and the greedy loop (graph replays) against single steps, bit for bit: the counters
+    of a split are zero again after each launch, whichever shape comes next."""
     cfg = gpu.synth.tiny_config("llama", hidden=2048, num_heads=2048 // hd, num_kv_heads=512 // hd, head_dim=hd, ffn_dim=2048, max_seq_len=64)
     w = gpu.synth.make_weights(cfg, seed=4, scale=0.02)
     r = np.random.default_rng(n)
     prompts = [r.integers(0, cfg["vocab_size"], 1 + i % 3).tolist() for i in range(n)]
     ids, got = list(range(n)), {}
-    old = gpu.lib().nvl_set_tuning(38, mid)
+    old = [(key, gpu.lib().nvl_set_tuning(key, v)) for key, v in ((38, mid), (39, parts))]
     for precision in ("bf16", "f32"):
         m = gpu.HipTransformerModel(cfg, w, precision=precision, max_seqs=n, max_batch_tokens=512)
         for i in ids:
@@ -53,11 +55,13 @@ def test_decode_and_prompt_batches(gpu, hd, n, mid):
                 one.append(am)
             for i in ids:
                 m.seq_reset(i)
-            m.forward_batch(ids, prompts, [0] * n, want_logits=False)
+            again, _ = m.forward_batch(ids, prompts, [0] * n)
+            assert np.array_equal(again, first)
             _, am = m.forward_batch(ids, [[7]] * n, [len(p) for p in prompts], want_logits=False)
             assert np.array_equal(m.decode_greedy(ids, am, 3), np.stack(one))
         m.close()
-    gpu.lib().nvl_set_tuning(38, old)
+    for key, v in old:
+        gpu.lib().nvl_set_tuning(key, v)
     assert rel_err(got["bf16"][0], got["f32"][0]) <= TOL and rel_err(got["bf16"][1], got["f32"][1]) <= TOL
 
 
@@ -94,20 +98,46 @@ def test_mamba_decode_step(gpu, oracle, hidden, heads, hd, state, groups, n):
 
 
 @pytest.mark.parametrize("parts", [2, 3, 5])
-@pytest.mark.parametrize("m,k,n", [(520, 2048, 1300), (2100, 2112, 2056), (256, 1984, 256 * 9), (1025, 2048, 256 * 53)])     # tiles: 18, 81, 9, 265
+@pytest.mark.parametrize("m,k,n", [(520, 2048, 1300), (1100, 2112, 2056), (2100, 2112, 2056), (256, 1984, 256 * 9), (1025, 2048, 256 * 53)])
 def test_large_tiles_of_the_last_round_in_parts(gpu, parts, m, k, n):
-    """The ping-pong kernel with its last round cut along K, uneven parts, XCDs with one tile less than others or none: exact on integers,
-    twice in a row."""
+    """The ping-pong kernel with its last round cut along K, uneven parts, XCDs with one tile less than others or none: exact on integers.
+    18, 45, 81, 9 and 265 tiles, at most 3, 6, 11, 2 and 34 = 32 + 2 of them an XCD: 32 workgroups hold the parts, so that 81 are cut in two only
+    and stay whole at 3 and 5."""
     a = (np.arange(m * k).reshape(m, k) % 7).astype(np.float32) - 1.0
     b = (np.arange(k * n).reshape(k, n) % 5).astype(np.float32) - 2.0
     old = [(key, gpu.lib().nvl_set_tuning(key, v)) for key, v in ((0, 5), (41, parts))]
     try:
-        got = [gpu.ops.mat_mul(a, b, precision="bf16") for _ in range(2)]
+        got = gpu.ops.mat_mul(a, b, precision="bf16")
     finally:
         for key, v in old:
             gpu.lib().nvl_set_tuning(key, v)
     want = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32)
-    assert np.array_equal(got[0], want) and np.array_equal(got[1], want)
+    assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("family,hd,tile", [("llama", 64, 5), ("llama", 128, 5), ("llama", 128, 0), ("gpt2", 64, 5)])
+@pytest.mark.parametrize("hidden,parts", [(1024, 2), (2048, 3), (2048, 5)])
+def test_epilogues_behind_large_tiles_in_parts(gpu, family, hd, tile, hidden, parts):
+    """Every epilogue of the ping-pong kernel behind a split of K: residual, gate | up, GELU, rotated heads of 64, and (tile 0: the large tiles
+    are not forced, heads of 128 take them all the same) of 128.  600 rows: 12 .. 48 tiles, 2 .. 6 an XCD, parts of 12 .. 21 K-steps.  The same
+    call whole and in parts differs in the order of fp32 sums, each within the bf16 bound of the fp32 mode; again bit for bit (the counters)."""
+    over = dict(num_kv_heads=256 // hd) if family == "llama" else {}
+    cfg = gpu.synth.tiny_config(family, hidden=hidden, num_heads=hidden // hd, head_dim=hd, ffn_dim=hidden, max_seq_len=640, **over)
+    m = gpu.HipTransformerModel(cfg, gpu.synth.make_weights(cfg, seed=12, scale=0.03), precision="bf16", max_seqs=1, max_batch_tokens=640)
+    tokens = np.random.default_rng(hd).integers(0, cfg["vocab_size"], 600).tolist()
+    got = []
+    for cut in (1, parts):
+        old = [(key, gpu.lib().nvl_set_tuning(key, v)) for key, v in ((0, tile), (41, cut))]
+        try:
+            for _ in range(2):
+                m.seq_reset(0)
+                got.append(m.forward_batch([0], [tokens], [0], all_logits=True)[0])
+        finally:
+            for key, v in old:
+                gpu.lib().nvl_set_tuning(key, v)
+    m.close()
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[2], got[3]) and not np.array_equal(got[0], got[2])
+    assert rel_err(got[2], got[0]) <= TOL
 
 
 @pytest.mark.parametrize("n", [1, 16, 17, 40, 64])
