@@ -135,6 +135,7 @@ struct GemmArgs {
     const float* rs_in;     // consumer: the same buffer
     int rs_tiles;
     float rs_inv_h, rs_eps;
+    int split_units;        // size of split_ws in SPLIT_UNITs (for the launchers)
     // MoE decode, "dense-masked" form (decode kernels only, M <= 64).  All experts are ONE projection each way:
     //   up   W = [E * 2I][H] (the experts' interleaved gate|up rows back to back), output column f belongs to expert f / I;
     //   down W = [H][E * I] (the experts concatenated along K), a wave's K range lies inside ONE expert.
@@ -144,7 +145,6 @@ struct GemmArgs {
     // projection's K reduction the weighted combine itself (moe.go:105-120) — no sort, no plan, no combine launch.
     const float* moe_gate;
     int moe_E, moe_I;
-    int64_t split_bytes;    // size of split_ws (for the launchers)
 };
 // does any row of the batch (M <= 64: one per lane) route to expert e?  Call with all 64 lanes active.
 __device__ __forceinline__ bool moe_expert_live(const GemmArgs& p, int e) {
@@ -544,6 +544,7 @@ void gemm_bf16_kernel(GemmArgs p) {
 // ------------------------------------------------------------------------------------------
 constexpr int64_t SPLIT_WS_BYTES = 64ll << 20;      // all a launch can use: 256 parts of 256 x 256 fp32 (gemm_bf16_pp_kernel)
 constexpr int64_t SPLIT_MID_BYTES = 8ll << 20;      // ... gemm_mid_bf16_kernel, unless its parts are forced: 256 of 128 x 64 or 64 x 128
+constexpr int64_t SPLIT_UNIT = 32 << 10;            // a 128 x 64 fp32 part
 constexpr int SPLIT_MAX_TILES = 512;
 constexpr int PP_MIN_STAGES = 12;                   // K-steps of 32 that a part of a 256 x 256 tile has at least
 constexpr int MID_MAX_PARTS = 8, MID_MIN_STAGES = 2;      // parts of a tile of gemm_mid_bf16_kernel; K-steps of 128 that one has at least
@@ -1738,7 +1739,7 @@ static inline bool pp_wins(GemmArgs& a) {
     a.splits = 1;
     if (a.seg || a.a_rows || a.tile_map || a.sk_part || a.K < 160) return false;
     const int bytes = EPI == EPI_RESID ? 8 : EPI == EPI_GROUPED_RAW ? 4 : epi_glu(EPI) ? (int)sizeof(OutT) / 2 : (int)sizeof(OutT);
-    const bool parts = a.split_bytes >= SPLIT_WS_BYTES && (a.M > MID_MAX_ROWS || a.M <= std::max(64, g_chunk_max_m));      // (key 11 = 64: sums in one order whatever the rows, up to 512)
+    const bool parts = a.split_units * SPLIT_UNIT >= SPLIT_WS_BYTES && (a.M > MID_MAX_ROWS || a.M <= std::max(64, g_chunk_max_m));      // (key 11 = 64: sums in one order whatever the rows, up to 512)
     return pp_cost(a.M, a.N, a.K, bytes, parts, a.splits) < 0.93 * tile128_cost(a.M, a.N, a.K, bytes, 1);
 }
 template <int EPI, typename OutT, int WAVES_N>
@@ -1809,9 +1810,9 @@ template <int MT, int CT, int EPI, typename OutT>
 static inline void launch_gemm_mid_rows(hipStream_t st, const GemmArgs& a0) {
     GemmArgs a = a0;
     const int nb = cdiv(a.N, 32 * CT), groups = cdiv(a.M, 16 * MT);
-    mid_cost(a.M, a.N, a.K, MT, CT, a.split_bytes > 0, a.splits);
-    if (a.split_bytes > 0 && g_mid_splits) a.splits = std::min(g_mid_splits, std::max(1, a.K >> 7));
-    while (a.splits > 1 && (nb * groups > SPLIT_MAX_TILES || (int64_t)nb * groups * a.splits * MT * CT * 2048 > a.split_bytes)) a.splits--;
+    mid_cost(a.M, a.N, a.K, MT, CT, a.split_units > 0, a.splits);
+    if (a.split_units > 0 && g_mid_splits) a.splits = std::min(g_mid_splits, std::max(1, a.K >> 7));
+    while (a.splits > 1 && (nb * groups > SPLIT_MAX_TILES || (int64_t)nb * groups * a.splits * MT * CT * 2048 > a.split_units * SPLIT_UNIT)) a.splits--;
     NVL_LDS_ATTR((gemm_mid_bf16_kernel<MT, CT, EPI, OutT>), (mid_lds_bytes<MT, CT>()));
     hipLaunchKernelGGL((gemm_mid_bf16_kernel<MT, CT, EPI, OutT>), dim3(cdiv(nb, 8) * 8 * groups * a.splits), dim3(512), (mid_lds_bytes<MT, CT>()), st, a);
 }
@@ -1833,7 +1834,7 @@ static inline bool mid_wins(const GemmArgs& a) {
         if (!split) while (ks > 1 && blocks * ks > g_narrow_waves) ks >>= 1;
         // a step in favour of the form that is there: 8 % is half the error of the two costs.  At 24 / 32 / 64 rows, decode form -> here:
         // 4096 x 14336 43 -> 28.6, 55 -> 29.9, 85.7 -> 32.6 us; 4544 x 18176 at 16 rows 48.7 -> 34.9; 2048 x 8192 stays at 15.3 up to 32 rows, 23.1 -> 18.4 at 64
-        return mid_cost(a.M, a.N, a.K, mid_row_tiles(a.M), 2, a.split_bytes > 0, mid_parts) < 0.92 * narrow_cost(a.M, a.N, a.K, blocks, blocks * ks * (split ? cdiv(a.M, 16) : 1), split);
+        return mid_cost(a.M, a.N, a.K, mid_row_tiles(a.M), 2, a.split_units > 0, mid_parts) < 0.92 * narrow_cost(a.M, a.N, a.K, blocks, blocks * ks * (split ? cdiv(a.M, 16) : 1), split);
     }
     // (GPT-2's projections at 96 .. 104 rows: 768 x 768 12.7 us here and 8.8 in groups of the decode form, 768 x 3072 14.7 and 13.6)
     if (EPI != EPI_QKV && (a.K < 2048 || (int64_t)a.N * a.K < (4 << 20))) return false;

@@ -178,7 +178,7 @@ void gemm(nvl_model* m, int epi, bool out_f32, GemmArgs a, double flops = -1.0) 
         : ((double)a.N * a.K + (double)a.M * a.K) * (double)m->wsize + (double)a.M * a.N * (out_f32 || epi == EPI_RESID ? 4.0 : (double)m->wsize);
     KScope ks(m, KC_GEMM, flops >= 0 ? flops : 2.0 * (double)a.M * (double)a.N * (double)a.K, -1, gbytes);
     hipStream_t st = m->stream;
-    a.split_ws = m->split_ws; a.split_cnt = m->split_cnt; a.split_bytes = m->split_bytes; a.splits = 1;
+    a.split_ws = m->split_ws; a.split_cnt = m->split_cnt; a.split_units = (int)(m->split_bytes / SPLIT_UNIT); a.splits = 1;
     if (m->f32) {
         switch (epi) {
             case EPI_STORE: launch_gemm_f32<EPI_STORE, float>(st, a); break;
@@ -1385,7 +1385,7 @@ GemmArgs mk(const void* A, int lda, const void* W, void* C, int ldc, const float
     a.M = M; a.N = N; a.K = K; a.seg = nullptr; a.c_row0 = 0;
     a.qkv = QkvEpi{};
     a.tile_map = nullptr; a.n_mtiles = nullptr; a.w_expert_stride = 0;
-    a.sk_part = nullptr; a.sk_slices = 1; a.split_ws = nullptr; a.split_cnt = nullptr; a.split_bytes = 0; a.splits = 1; a.m_split = 0; a.rs_half = 0; a.grid_y = 1; a.nrm_w = nullptr; a.nrm_xn = nullptr; a.rs_out = nullptr; a.rs_in = nullptr; a.rs_tiles = 0; a.rs_inv_h = 0.f; a.rs_eps = 0.f;
+    a.sk_part = nullptr; a.sk_slices = 1; a.split_ws = nullptr; a.split_cnt = nullptr; a.split_units = 0; a.splits = 1; a.m_split = 0; a.rs_half = 0; a.grid_y = 1; a.nrm_w = nullptr; a.nrm_xn = nullptr; a.rs_out = nullptr; a.rs_in = nullptr; a.rs_tiles = 0; a.rs_inv_h = 0.f; a.rs_eps = 0.f;
     return a;
 }
 
