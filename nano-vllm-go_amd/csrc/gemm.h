@@ -1050,9 +1050,12 @@ __device__ __forceinline__ void skinny_pass_remap(GemmArgs& p, int& bx) {
 // others pulled 256 KB each through one CU).  The other 8 lanes of every 16-lane row group feed zeros (their loads are
 // predicated off: 4 x 128-byte lines per k-step instead of 8); only the owned rows are stored; the x^2 partials are per
 // 8 columns (rs_tiles = N / 8).
-// SCALED: a residual projection whose input rows carry a deferred scale of their own (rs_in; its own instance: the others lose 1 % beside it).
-template <int MT, int NTW, int U, int EPI, typename OutT, bool PASSES = false, bool MOE = false, bool HALF = false, bool SCALED = false>
+// EXTRA: a residual projection whose input rows carry a deferred scale of their own (rs_in; SCALED), or with MOE one that completes its K slices
+// (rs_out; COMPLETES).  Instances of their own: beside it the others lose 1 %, and the experts' slices 16 % at 40 rows (4096 x 32 x 448:
+// 43.9 -> 51 us, their registers spill).
+template <int MT, int NTW, int U, int EPI, typename OutT, bool PASSES = false, bool MOE = false, bool HALF = false, bool EXTRA = false>
 __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
+    constexpr bool SCALED = EXTRA && !MOE, COMPLETES = EXTRA && MOE;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     f32x4* red = (f32x4*)smem;                       // [NTW][ksplit][MT][64]
     const int swg = blockIdx.y * gridDim.x + blockIdx.x;
@@ -1092,7 +1095,7 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
     // expert.  Down: a wave's K range is exactly one expert (launch_gemm_skinny_ntw), of any width; without a token it has nothing to stream.
     if constexpr (MOE) {
         if (epi_moe(EPI)) { if (!moe_expert_live(p, (nt0 * 16) / (2 * p.moe_I))) return; }          // (whole workgroup: uniform)
-        else if (!moe_expert_live(p, part)) my_steps = 0;
+        else my_steps = __builtin_amdgcn_readfirstlane(moe_expert_live(p, part) ? my_steps : 0);      // (uniform: scalar loops)
     }
 
     // EPI_QKV: the workgroup's two tiles are half a head apart (they rotate together)
@@ -1142,11 +1145,20 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
     // the residual operand of this wave's first epilogue element (deferred-norm producer form): fetched under the weight
     // stream, not as a dependent round trip after the K reduction (this launch is the only writer of these elements)
     f32x4 x_pre = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (EPI == EPI_RESID && p.rs_out && wave < NTW * MT) {
+    if (EPI == EPI_RESID && (!MOE || COMPLETES) && p.rs_out && wave < NTW * MT) {
         const int t = wave / MT, i = wave - t * MT;
         const int m = 16 * (i + i_off) + fr, n = (nt0 + t) * 16 + 4 * fg;
         if (m < p.M && n < p.N && (!HALF || (fg >> 1) == half)) x_pre = *(const f32x4*)((const float*)p.C + (int64_t)m * p.ldc + n);
     }
+    if constexpr (MOE && EPI == EPI_RESID) {
+        for (int b = 0; b < nblk; b += 2) {
+            if (b + 1 < nblk) load_blk(wB, xB, b + 1);
+            comp_blk(wA, xA);
+            if (b + 1 >= nblk) break;
+            if (b + 2 < nblk) load_blk(wA, xA, b + 2);
+            comp_blk(wB, xB);
+        }
+    } else {
     int b = 0;
     for (; b + 2 <= nblk; b += 2) {
         load_blk(wB, xB, b + 1);
@@ -1156,6 +1168,7 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
         comp_blk(wB, xB);
     }
     if (b < nblk) comp_blk(wA, xA);
+    }
     for (int s = nblk * U; s < my_steps; s++) {      // ragged tail: fewer than U k-steps
         const bf16x8 w = w_live ? weight_load<PASSES>((const bf16x8*)(wp + (int64_t)s * 512)) : x_zero;
 #pragma unroll
@@ -1191,13 +1204,11 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
         for (int e = wave; e < NTW * MT; e += NTW * ksplit) {
             const int t = e / MT, i = e - t * MT;
             const int m = 16 * i + fr, n = (nt0 + t) * 16 + 4 * fg;
-            if constexpr (MOE) {
-                if (p.rs_out) {
-                    f32x4 v = ksum(t, i);
-                    const int n16 = p.N >> 4;
-                    if (nt0 + t < n16 && split_finish_wave(p, i * n16 + nt0 + t, n16 * MT, slice, nslices, v)) resid_norm_tile(p, m, n, v, e == wave ? &x_pre : nullptr);
-                    continue;
-                }
+            if constexpr (COMPLETES) {
+                f32x4 v = ksum(t, i);
+                const int n16 = p.N >> 4;
+                if (nt0 + t < n16 && split_finish_wave(p, i * n16 + nt0 + t, n16 * MT, slice, nslices, v)) resid_norm_tile(p, m, n, v, e == wave ? &x_pre : nullptr);
+                continue;
             }
             if (m >= p.M || n >= p.N) continue;
             f32x4 v = ksum(t, i);
@@ -1622,11 +1633,18 @@ static inline bool launch_gemm_skinny_ntw(hipStream_t st, const GemmArgs& a) {
     dim3 grid(nblocks * (a.m_passes > 1 ? a.m_passes : 1), KS), block(NTW * ksplit * 64);
     if (a.grid_y != KS) { GemmArgs c = a; c.grid_y = KS; return launch_gemm_skinny_ntw<NTW, EPI, OutT>(st, c); }
 #define NVL_SK(MTv, Uv) hipLaunchKernelGGL((gemm_skinny_bf16_kernel<MTv, NTW, Uv, EPI, OutT>), grid, block, lds, st, a)
-#define NVL_SKM(MTv, Uv) hipLaunchKernelGGL((gemm_skinny_bf16_kernel<MTv, NTW, Uv, EPI, OutT, false, true>), grid, block, lds, st, a)
+#define NVL_SKM(MTv, Uv, Xv) hipLaunchKernelGGL((gemm_skinny_bf16_kernel<MTv, NTW, Uv, EPI, OutT, false, true, false, Xv>), grid, block, lds, st, a)
     if constexpr (epi_moe(EPI) || EPI == EPI_RESID) {
         if (a.moe_gate) {                                 // MoE decode instantiation (expert skip + gate weight)
             if (a.m_passes > 1) return false;
-            if (MT == 1) NVL_SKM(1, 4); else if (MT == 2) NVL_SKM(2, 4); else NVL_SKM(4, 2);
+            if constexpr (EPI == EPI_RESID) {
+                if (a.rs_out) {
+                    if (KS < 2) return false;
+                    if (MT == 1) NVL_SKM(1, 4, true); else if (MT == 2) NVL_SKM(2, 4, true); else NVL_SKM(4, 2, true);
+                    return true;
+                }
+            }
+            if (MT == 1) NVL_SKM(1, 4, false); else if (MT == 2) NVL_SKM(2, 4, false); else NVL_SKM(4, 2, false);
             return true;
         }
     }
