@@ -1189,12 +1189,14 @@ __global__ __launch_bounds__(256) void moe_route_grouped_kernel(GroupRouteArgs p
     };
     bool in[ROUTE_MAX_E / 64];
     float c[ROUTE_MAX_E / 64];
+    int own[ROUTE_MAX_E / 64];
 #pragma unroll
     for (int i = 0; i < ROUTE_MAX_E / 64; i++) {
         const int e = lane + 64 * i;
         in[i] = r < p.rows && e < p.E && kept(e / size);
         c[i] = r < p.rows && e < p.E ? choice[e] : 0.f;
-        if (r < p.rows && e < p.E) key[e] = in[i] ? score_key(c[i]) : -0x7fffffff - 1;       // (below every score)
+        own[i] = in[i] ? score_key(c[i]) : -0x7fffffff - 1;       // (below every score)
+        if (r < p.rows && e < p.E) key[e] = own[i];
     }
     __syncthreads();
     int ranks[ROUTE_MAX_E / 64];
@@ -1203,7 +1205,7 @@ __global__ __launch_bounds__(256) void moe_route_grouped_kernel(GroupRouteArgs p
     for (int i = 0; i < ROUTE_MAX_E / 64; i++) {
         const int e = lane + 64 * i;
         ranks[i] = p.top;
-        if (in[i]) { ranks[i] = 0; const int own = key[e]; for (int j = 0; j < p.E; j++) { const int v = key[j]; ranks[i] += v > own || (v == own && j < e); } }
+        if (in[i]) { ranks[i] = 0; for (int j = 0; j < p.E; j++) { const int v = key[j]; ranks[i] += v > own[i] || (v == own[i] && j < e); } }
         if (in[i]) top_z = fmaxf(top_z, c[i]);
     }
     if (p.softmax) {
