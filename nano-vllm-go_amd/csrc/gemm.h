@@ -555,6 +555,7 @@ static inline int64_t split_need(int64_t M, int64_t N, int64_t K) {
     return std::min(SPLIT_MID_BYTES, (int64_t)MID_MAX_PARTS * 4 * round_up(std::min<int64_t>(M, 512), 128) * round_up(N, 128));
 }
 constexpr int SPLIT_COHERENT = 0x11;      // buffer cache policy: sc0 | sc1
+constexpr int LOAD_NT = 2;                // ... nt: a line read once
 
 // acc: this wave's F fragments; a part takes `bytes` of split_ws (waves one after the other, 1 KiB a fragment).  True in the workgroup
 // that holds the sum.  Whole workgroups call it; `flag`: one int of LDS that nothing else uses.
@@ -839,6 +840,10 @@ __global__ __launch_bounds__(512, 1) void gemm_mid_bf16_kernel(GemmArgs p) {
     const int k0 = (int)((int64_t)part * stages / p.splits), n = (int)((int64_t)(part + 1) * stages / p.splits) - k0;
     const bool ragged = (p.K & 64) && k0 + n == stages;          // K % 128 == 64: the last stage has its first half only
 
+    // Weights that a single row group reads once go past what the caches hold: states, keys and values of the next launches stay there (without nt a
+    // delta-rule scan behind an input projection at 20 rows 31.5 -> 36.0 us, a lightning scan at 32 29.9 -> 34.4), and the ring is
+    // faster itself (4544 x 18176 at 16 rows 32.5 -> 29.8 us, 4096 x 14336 at 32 26.4 -> 24.9)
+    const bool stream = groups == 1;
     // 1-KiB blocks (row tile, k-step) of a stage, PW for each wave: rows first, then columns
     const bf16_t* src[PW];
 #pragma unroll
@@ -857,8 +862,10 @@ __global__ __launch_bounds__(512, 1) void gemm_mid_bf16_kernel(GemmArgs p) {
 #pragma unroll
         for (int i = 0; i < PW; i++) {
             if (cut && ((wave8 * PW + i) & 2)) continue;        // (k-steps 2 and 3; waited for with vmcnt(0))
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] + (int64_t)s * 2048),
-                                             (__attribute__((address_space(3))) void*)(base + i * 1024), 16, 0, 0);
+            const auto from = (const __attribute__((address_space(1))) void*)(src[i] + (int64_t)s * 2048);
+            const auto to = (__attribute__((address_space(3))) void*)(base + i * 1024);
+            if (stream && wave8 * PW + i >= NA) __builtin_amdgcn_global_load_lds(from, to, 16, 0, LOAD_NT);
+            else __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
         }
     };
     // a wave's column tiles: neighbours for gate | up pairs, else two apart (a head's rotated halves then lie in one wave)
