@@ -1822,12 +1822,20 @@ static inline double mid_cost(int M, int N, int K, int mt, int ct, bool can_spli
     }
     return best + 4.0;
 }
-// ... and on the narrow decode form (M <= 64): every 16-row tile of the activations comes beside the weights, at 11.5 TB/s with all CUs at work.
+// ... and on the narrow decode form (M <= 64), where the activations come beside the weights once per 16 of their rows.  us a MB of weights with every
+// CU at work, from the activation rows that a launch fetches (whole row tiles, or the live rows: x_mask), over the share of its last round of
+// workgroups that is at work, and not faster than 6.56 TB/s.  Fitted to 1 .. 64 rows of 1024 .. 15360 x 2048 .. 18176, good to 20 %.
 // `blocks`: workgroups of one row tile; tile_split: each row tile has its own workgroups (GemmArgs::m_split)
 static inline double narrow_cost(int M, int N, int K, int blocks, int waves, bool tile_split) {
-    const double mb = 2e-6 * N * K, rows = M < 16 ? M / 16.0 : cdiv(M, 16), wgs = tile_split ? blocks * cdiv(M, 16) : blocks;
-    const double rate = 11.5 * std::min(1.0, wgs / 256.0) * (waves >= 2048 ? 1.0 : pow(waves / 2048.0, 0.6)) * (!tile_split && rows > 2 ? 1.25 : 1.0);
-    return std::max(mb / 5.9, mb * (tile_split ? 2.0 * cdiv(M, 16) : 1.0 + rows) / rate) + 2.5;
+    const double mb = 2e-6 * N * K;
+    if (tile_split) {
+        const double rate = 11.5 * std::min(1.0, blocks * cdiv(M, 16) / 256.0) * (waves >= 2048 ? 1.0 : pow(waves / 2048.0, 0.6));
+        return std::max(mb / 5.9, mb * 2.0 * cdiv(M, 16) / rate) + 2.5;
+    }
+    const double rows = M > 32 && blocks > 512 ? 4.0 : M % 16 ? M / 16.0 : M <= 32 ? M / 16 : 4.0;
+    double full = blocks / (256.0 * cdiv(blocks, 256));
+    if (blocks > 512 && M <= 32) full = std::max(full, 0.88);      // (of one or two waves each: they even out)
+    return std::max(mb / 6.56, mb * (M <= 16 ? 0.113 + 0.03 * rows : 0.14 + 0.032 * rows) / full) + 3.6;
 }
 inline int g_mid = 1;               // nvl_set_tuning key 38: 0 never, 2 wherever it applies
 inline int g_mid_splits = 0;        // nvl_set_tuning key 39: parts of K (0: from the cost)
@@ -1857,9 +1865,12 @@ static inline bool mid_wins(const GemmArgs& a) {
         const int blocks = cdiv(a.N, 16);
         int ks = split ? 8 : 16, mid_parts;                       // (waves of a workgroup: launch_gemm_skinny_ntw)
         if (!split) while (ks > 1 && blocks * ks > g_narrow_waves) ks >>= 1;
-        // a step in favour of the form that is there: 8 % is half the error of the two costs.  At 24 / 32 / 64 rows, decode form -> here:
-        // 4096 x 14336 43 -> 28.6, 55 -> 29.9, 85.7 -> 32.6 us; 4544 x 18176 at 16 rows 48.7 -> 34.9; 2048 x 8192 stays at 15.3 up to 32 rows, 23.1 -> 18.4 at 64
-        return mid_cost(a.M, a.N, a.K, mid_row_tiles(a.M), 2, a.split_units > 0, mid_parts) < 0.92 * narrow_cost(a.M, a.N, a.K, blocks, blocks * ks * (split ? cdiv(a.M, 16) : 1), split);
+        // a small step in favour of the form that is there.  Decode form -> here, us, weights from HBM: 4544 x 18176 at 5 / 16 / 32 rows 37.1 -> 29.4,
+        // 46.4 -> 29.8, 62.9 -> 31.5; 2560 x 8192 at 40 / 64 16.7 -> 13.6, 20.7 -> 14.2; not 4096 x 14336 at 5 / 16 19.8 / 22.8, 22.4 / 23.3 here,
+        // 8192 x 4096 at 17 / 32 16.7 / 16.8, 17.9 / 18.1 here.  Row tiles apart, at 24 / 32 / 64 rows: 4096 x 14336 43 -> 28.6, 55 -> 29.9,
+        // 85.7 -> 32.6; 2048 x 8192 stays at 15.3 up to 32 rows, 23.1 -> 18.4 at 64
+        return mid_cost(a.M, a.N, a.K, mid_row_tiles(a.M), 2, a.split_units > 0, mid_parts) <
+               (split ? 0.92 : 0.98) * narrow_cost(a.M, a.N, a.K, blocks, blocks * ks * (split ? cdiv(a.M, 16) : 1), split);
     }
     // (GPT-2's projections at 96 .. 104 rows: 768 x 768 12.7 us here and 8.8 in groups of the decode form, 768 x 3072 14.7 and 13.6)
     if (EPI != EPI_QKV && (a.K < 2048 || (int64_t)a.N * a.K < (4 << 20))) return false;
