@@ -1764,8 +1764,15 @@ static inline bool pp_wins(GemmArgs& a) {
     a.splits = 1;
     if (a.seg || a.a_rows || a.tile_map || a.sk_part || a.K < 160) return false;
     const int bytes = EPI == EPI_RESID ? 8 : EPI == EPI_GROUPED_RAW ? 4 : epi_glu(EPI) ? (int)sizeof(OutT) / 2 : (int)sizeof(OutT);
-    const bool parts = a.split_units * SPLIT_UNIT >= SPLIT_WS_BYTES && (a.M > MID_MAX_ROWS || a.M <= std::max(64, g_chunk_max_m));      // (key 11 = 64: sums in one order whatever the rows, up to 512)
-    return pp_cost(a.M, a.N, a.K, bytes, parts, a.splits) < 0.93 * tile128_cost(a.M, a.N, a.K, bytes, 1);
+    // (key 11 = 64: sums in one order whatever the rows, up to 512.  EPI_GROUPED, whose epilogue is long: not where one round of parts would leave
+    // it to a few workgroups, 17424 x 4096 at 140 / 200 rows 82 / 86 us in parts, 74 / 78 on 128x128 tiles)
+    const bool parts = a.split_units * SPLIT_UNIT >= SPLIT_WS_BYTES && (a.M > MID_MAX_ROWS || a.M <= std::max(64, g_chunk_max_m)) &&
+                       (EPI != EPI_GROUPED || cdiv(a.M, 256) * cdiv(a.N, 256) > 256);
+    const bool faster = pp_cost(a.M, a.N, a.K, bytes, parts, a.splits) < 0.93 * tile128_cost(a.M, a.N, a.K, bytes, 1);
+    // Whole tiles lose to 128x128 tiles that fit one round of two a CU, which the costs miss.  Large / 128x128, us, weights from HBM: 12288 x 4096 at 600
+    // rows 94 / 75, 6144 x 4096 at 1100 87 / 73, 28672 x 4096 (gate | up) at 200 82 / 77, 16384 x 2048 at 400 46 / 39; in a second round
+    // 12288 x 4096 at 700 92 / 129, 28672 x 4096 at 300 119 / 131
+    return faster && (a.splits > 1 || cdiv(a.M, 128) * cdiv(a.N, 128) > 512);
 }
 template <int EPI, typename OutT, int WAVES_N>
 static inline void launch_pp(hipStream_t st, const GemmArgs& a) {
