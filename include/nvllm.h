@@ -560,7 +560,7 @@ int nvl_bench_gemm(int device, int M, int N, int K, int epi, int force_bnt, int 
  * ping-pong kernel, 128 / 256 = the lock-step tile kernels with that many rows per m-tile.
  * key 19: decode-sized MoE batches run the grouped GEMMs on the four-stage 128x128 instance (1, default) or two stages (0).
  * key 18: largest prompt batch (tokens) whose QKV projection leaves fp32 rows to rope_kv_kernel instead of rotating and placing
- * them itself (default 0: none).
+ * them itself (default -1: by size; 0: none).
  * key 38: projections of up to 512 rows (beyond 64 as far as key 11 goes) on their own kernel, K split over workgroups (1, default,
  * by cost; 0 never; 2 wherever it applies);
  * key 39: the parts of K there (0, default: by cost); key 40: rows up to which it completes residual projections (default 256).

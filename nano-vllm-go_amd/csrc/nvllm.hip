@@ -1478,7 +1478,18 @@ void tp_p2p_allreduce_resid(nvl_model* m, const float* part, int M, int N, float
 // Prefill and the fp32 mode fuse the add into the GEMM epilogue.  Decode-sized batches split K over
 // `slices` workgroups per column block so that all 256 CUs stream weights (a 2048-column projection has
 // only 128 column blocks), and leave the add to the norm kernel that always follows (PendingResid).
-static int g_qkv_store_max_m = 0;    // nvl_set_tuning key 18: largest prompt batch whose QKV projection leaves fp32 rows to rope_kv_kernel
+static int g_qkv_store_max_m = -1;   // nvl_set_tuning key 18: largest prompt batch whose QKV projection leaves fp32 rows to rope_kv_kernel; -1: by size
+// Rows and a launch of their own, or heads rotated and placed by the projection, for a prompt of M tokens.  us a prompt, placed / rows:
+//   Llama-3.2-1B (3072 x 2048) 16 869 / 863, 24 926 / 904, 32 949 / 917, 33 1149 / 1064, 64 1235 / 1136, 65 1221 / 1244, 256 1820 / 1903
+//   GPT-2 (2304 x 768) 11 444 / 464, 32 483 / 498, 48 519 / 515, 128 644 / 657       Granite-3.0-1B (2048 x 1024) 11 1225 / 1281, 32 1375 / 1389,
+//   33 1558 / 1501, 64 1694 / 1620, 65 2143 / 2077, 128 2252 / 2236, 150 2284 / 2327       Llama-3-8B (6144 x 4096) 11 3448 / 3558, 48 4418 / 4107, 200 6469 / 6627
+//   Falcon-7B (4672 x 4544) 16 3607 / 3634, 24 3692 / 3597, 64 4997 / 4484, 65 4799 / 4875
+// A row tile is a launch less; two to four of them halve the workgroups of the projection beside its pairs of columns; beyond 64 rows
+// the ring kernel takes the heads.
+bool qkv_rows(int M, int64_t N, int64_t K) {
+    if (g_qkv_store_max_m >= 0) return M <= g_qkv_store_max_m;
+    return M <= 16 ? false : M <= 32 ? N * K >= (4 << 20) : M <= 64 ? true : M <= 128 && K < 2048;
+}
 static int g_moe_dense = 1;    // nvl_set_tuning key 22: decode MoE as two dense-masked projections (gemm.h moe_gate); 0 = sort + grouped GEMMs
 static int g_moe_deep = 1;     // nvl_set_tuning key 19: four-stage grouped GEMM for decode-sized MoE batches (0 = two stages)
 static int g_moe_bm = 0;       // nvl_set_tuning key 17: prefill MoE grouped GEMMs: 0 = 256-row tiles on the ping-pong kernel, 128 / 256 = the lock-step tile kernels
@@ -1994,9 +2005,8 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
         bool fused_dec = false;
         // a decode batch of 64 < M <= g_chunk_max_m rows keeps the decode form (64-row passes, gemm.h) and the fused
         // decode attention
-        // Prompts: RoPE + Q/K/V placement fused into the projection's epilogue (no fp32 qkv round trip; up to 64 tokens it is a launch
-        // less a layer: GPT-2 at 11 tokens 76 launches instead of 88, 9 %)
-        const bool store_rows = max_len > 1 && M <= g_qkv_store_max_m && M <= g_chunk_max_m && g_force_tile == 0;
+        // Prompts: RoPE + Q/K/V placement fused into the projection's epilogue (no fp32 qkv round trip, a launch less a layer), or not: qkv_rows
+        const bool store_rows = max_len > 1 && qkv_rows(M, m->n_qkv, H) && M <= g_chunk_max_m && g_force_tile == 0;
         if (!m->f32 && (M > 64 ? !big_decode : max_len > 1 && m->hd % 32 == 0) && !store_rows) {
             GemmArgs a = mk(m->xn, H, l.w_qkv, nullptr, 0, l.b_qkv, 1.f, M, m->n_qkv, H);
             if (qkv_deferred) set_deferred_in(m, a);
