@@ -567,8 +567,9 @@ int nvl_bench_gemm(int device, int M, int N, int K, int epi, int force_bnt, int 
  * key 21: hipGraph replay of decode passes (1, default; 0 = every launch eager).  key 22: decode MoE as two dense-masked
  * weight-streaming projections (1, default) or sort + grouped GEMMs (0).  key 23: largest payload (rows of the residual
  * stream) the tensor-parallel P2P all-reduce sends one-shot; above it reduce-scatter + all-gather (default 64).
- * key 25: a decode attention of up to 128 (sequence, kv head) pairs over more keys than a round of a workgroup holds deals its key
- * tiles over up to 8 workgroups per pair, the last of which combines the partial results (1, default; 0 never; 1 + n: n rounds each).
+ * key 25: a decode attention of up to 128 (sequence, kv head) pairs over long contexts (from 321 to 1281 keys on, the more the more
+ * pairs there are) deals its key tiles over up to 8 workgroups per pair, the last of which combines the partial results
+ * (1, default; 0 never; 1 + n: n rounds each).
  * key 26: residual projections of 65..2048 rows split K over up to 8 workgroups per 128x128 tile, the slices summed by the
  * norm that follows (1, default; 0 = the 64-row groups of the decode form / plain tiles).
  * key 24: the decode GEMM kernels do not fetch the activation rows >= M of a padded 16-row tile (1, default).

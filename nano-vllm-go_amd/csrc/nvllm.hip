@@ -1245,10 +1245,17 @@ static int g_attn_split = 1;   // nvl_set_tuning key 25: split a decode attentio
 // workgroup | most workgroups per (sequence, kv head) << 8 | key tiles a workgroup has at least << 12.
 // Split: a workgroup pulls all K/V of its (sequence, kv head) through ONE CU, one round of tiles after the other; with few of
 // them and a long context that, not HBM, is the time.  A sequence is then dealt over workgroups of one round each (attn.h), and the
-// last of them combines the parts: about 2 us, so that contexts of one round stay whole.  Beyond 128 pairs the launch fills the
-// chip and a split only adds traffic.  us per launch whole / split, Llama-3.2-1B (8 kv heads of 64): 1 x 700 keys 11.6 / 10.6,
-// 4 x 1800 16.9 / 12.8, 8 x 1800 20.1 / 15.6, 8 x 300..1800 17.9 / 13.1, 16 x 200..1000 13.5 / 12.8, but 12 x 600 10.7 / 12.0,
-// 32 x 1500 23.2 / 27.0; Llama-3-8B (8 of 128): 1 x 700 15.2 / 13.0, 8 x 1500 27.0 / 20.1, 16 x 300..1200 22.2 / 25.3.
+// last of them combines the parts.  That costs every launch about 2 us, in parts written, counted and read back, so that a
+// context has to be longer the fuller the chip already is; beyond 128 pairs a split only adds traffic.  The lines lie where whole
+// decode steps change sides (a launch by itself favours the split earlier: it does not wait for the kernel before it).  A step
+// split against whole, per cent, at keys of each sequence:
+//   Llama-3.2-1B (8 kv heads of 64)    600   700   800   900   1000/1100  1500     Llama-3-8B (8 of 128)     340   530   650   800   1100
+//     1 sequence                      +1.1  -0.3  -1.8  -2.9  -3.5                   1 to 4 sequences       -0.3 and on to -1.1
+//     4                               +0.9  +0.3  -0.2  -1.0  -1.3                   6 to 12                      +2.4  +1.1  -1.0  -2.6
+//     6                               +1.2  +0.9  +0.5  -0.2  -0.5
+//     8                                           +1.5  +0.4  -1.6       -5.0
+//    12                                           +1.0        +1.2       +0.6 (contexts of a quarter to all of that: -0.9, -2.5)
+//    16                                           +2.2  +2.0  +1.5       +0.2 (ragged: -1.4 at 1100, -1.0)
 int decode_attn_cfg(const nvl_model* m, int n_seqs) {
     const int n_kt = m->ctx_hint > 0 ? (m->ctx_hint - 1) / 64 + 1 : 1 << 20;
     const int per_wave = m->hd == 64 ? 2 : 1;
@@ -1261,8 +1268,8 @@ int decode_attn_cfg(const nvl_model* m, int n_seqs) {
     if (g_attn_split >= 2) { const int tiles = (g_attn_split - 1) * nw * per_wave; return cfg(nw, std::max(1, std::min(most, cdiv(n_kt, tiles))), tiles); }
     if (g_attn_split && !g_attn_nw && most > 1) {
         int waves = 0;
-        if (m->hd == 64) waves = wgs <= 48 ? (n_kt > 20 ? 4 : n_kt > 8 ? 2 : 0) : wgs <= 128 && n_kt > 12 ? 4 : 0;
-        else waves = wgs <= 32 ? (n_kt > 16 ? 4 : n_kt > 5 ? 2 : 0) : wgs <= 96 && n_kt > 8 ? 8 : 0;
+        if (m->hd == 64) waves = wgs > 128 || n_kt <= (wgs <= 32 ? 12 : wgs <= 64 ? 16 : 20) ? 0 : wgs <= 48 && n_kt <= 20 ? 2 : 4;
+        else waves = wgs <= 32 ? (n_kt > 16 ? 4 : n_kt > 5 ? 2 : 0) : wgs <= 96 && n_kt > 12 ? 8 : 0;
         if (waves) return cfg(waves, std::min(most, cdiv(n_kt, waves * per_wave)), waves * per_wave);
     }
     return cfg(nw, 1, 1 << 16);
