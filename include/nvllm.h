@@ -548,9 +548,10 @@ int nvl_bench_gemm(int device, int M, int N, int K, int epi, int force_bnt, int 
  * key 1: K slices of the decode residual projections (0 automatic, 1 never split, 2, 4).
  * key 2: decode (M <= 64) GEMM form: 0 automatic, 1/2/4 = narrow form with that many weight tiles per workgroup,
  * 8 = wide-N form (4 weight tiles per wave).
- * key 3: deferred RMSNorm in decode (0 off, 1 on, 2 on without the activation-tile split, 3 only the O-proj -> FFN-up seam).
+ * key 3: deferred RMSNorm in decode (0 off, 1 on, 2 on without the activation-tile split, 3 only the O-proj -> FFN-up seam; with 2 or 3,
+ * or key 2 = 2 or 4, a hybrid's Mamba layers and 8-row half tiles keep their forms without a carried norm).
  * keys 4-6 (sweeps): K split of the wide form, waves per narrow-form launch, K split of the deferred-norm residual
- * projections.  key 7: decode seam kernel, 8: MoE small-batch fusion, 9: 16-row norm kernel, 10: query rows per
+ * projections.  key 7: decode seam kernel, 8: MoE small-batch fusion, 9: prompt norms in tiles of eight rows, 10: query rows per
  * workgroup of the prefill attention (0: 256, 1 from their number, 2: 128, 3: 64).  keys 11-14: decode batches of 65..512 rows (key 11, default 512; 64 = off) run the
  * projections whose 128x128 tile grid has fewer than key 12 (160) workgroups as ceil(M/64) groups of 64 rows of the
  * decode GEMM form, in one launch interleaved over the weight blocks (key 13 = 1) or one launch per group (0); up to
@@ -563,15 +564,15 @@ int nvl_bench_gemm(int device, int M, int N, int K, int epi, int force_bnt, int 
  * them itself (default -1: by size; 0: none).
  * key 38: projections of up to 512 rows (beyond 64 as far as key 11 goes) on their own kernel, K split over workgroups (1, default,
  * by cost; 0 never; 2 wherever it applies);
- * key 39: the parts of K there (0, default: by cost); key 40: rows up to which it completes residual projections (default 256).
+ * key 39: the parts of K there (0, default: by cost; fewer where the workspace or K is too small for them); key 40: rows up to which it completes residual projections (default 256).
  * key 21: hipGraph replay of decode passes (1, default; 0 = every launch eager).  key 22: decode MoE as two dense-masked
  * weight-streaming projections (1, default) or sort + grouped GEMMs (0).  key 23: largest payload (rows of the residual
  * stream) the tensor-parallel P2P all-reduce sends one-shot; above it reduce-scatter + all-gather (default 64).
  * key 25: a decode attention of up to 128 (sequence, kv head) pairs over long contexts (from 321 to 1281 keys on, the more the more
  * pairs there are) deals its key tiles over up to 8 workgroups per pair, the last of which combines the partial results
  * (1, default; 0 never; 1 + n: n rounds each).
- * key 26: residual projections of 65..2048 rows split K over up to 8 workgroups per 128x128 tile, the slices summed by the
- * norm that follows (1, default; 0 = the 64-row groups of the decode form / plain tiles).
+ * key 26: residual projections of up to 2048 rows, from 65 (K < 2048) or one more than key 40 on, split K over up to 8 workgroups per
+ * 128x128 tile, the slices summed by the norm that follows (1, default; 0 = the 64-row groups of the decode form / plain tiles).
  * key 24: the decode GEMM kernels do not fetch the activation rows >= M of a padded 16-row tile (1, default).
  * key 27: deferred-norm residual projections of <= 16 rows run on 8-row half tiles, twice the workgroups (1, default).
  * key 29: milliseconds a tensor-parallel rank waits for its peers inside a P2P all-reduce before the call fails (default 30000).

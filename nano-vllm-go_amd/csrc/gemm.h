@@ -1259,11 +1259,10 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
 // ------------------------------------------------------------------------------------------
 // MoE decode routing in ONE launch (moe.go:57-103): router logits of a 16-row activation tile (E <= 64 experts, all of K),
 // softmax, top-k, renormalised weights as the dense gate matrix GemmArgs::moe_gate of the expert projections.  Before:
-// the router as a skinny GEMM launch (4.6 us) + moe_gate_kernel (4.5 us).  grid = 16-row tiles of the batch x ROUTE_ROWS of their rows (the
-// logits of a tile are cheap, 96 KiB from L2; the ranking is serial: at 16 rows all of them in one workgroup 8.4 us, eight 7.2, four 7.0; at 6 rows two
-// workgroups lose 0.3), 1024
-// threads: wave w takes expert tile w % ET over K slice w / ET (fragments straight from L2 / HBM, as the skinny kernel),
-// the K slices are summed through LDS in wave order, then wave r routes the workgroup's row r with a lane per expert.
+// the router as a skinny GEMM launch (4.6 us) + moe_gate_kernel (4.5 us).  grid = 16-row tiles of the batch x ROUTE_ROWS of their rows: the
+// logits of a tile are cheap, 96 KiB from L2, and the ranking is serial (at 16 rows all of them in one workgroup 8.4 us, eight 7.2, four 7.0;
+// at 6 rows two workgroups lose 0.3).  1024 threads: wave w takes expert tile w % ET over K slice w / ET (fragments straight from L2 / HBM, as
+// the skinny kernel), the K slices are summed through LDS in wave order, then wave r routes the workgroup's row r with a lane per expert.
 // p: A (fragment-major operand, possibly the deferred-norm raw form with rs_in), W (router, fragment-major), bias, M, N = E, K.
 // The gate's columns E .. E + n_always - 1 are one (experts every token takes), those up to gate_ld zero.
 // ------------------------------------------------------------------------------------------

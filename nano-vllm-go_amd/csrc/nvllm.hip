@@ -1550,10 +1550,10 @@ void resid_gemm(nvl_model* m, const void* A, int lda, const void* W, const float
         if (g_sk_slices > 0) slices = g_sk_slices;
         else while (slices < m->sk_max_slices && nblocks * slices < 256 && (K >> 5) / (slices * 2) >= 8) slices *= 2;
     }
-    // 65..512 rows (a short prompt, a few hundred decode rows that do not take the decode form): N / 128 x M / 128 tiles of the
+    // More rows than the ring kernel completes (256 for K >= 2048; 64 for shorter K) and up to 2048: N / 128 x M / 128 tiles of the
     // lock-step kernel are a handful of workgroups (FFN-down of Llama-1B at 512 rows: 64), and the 64-row groups of the decode
     // form pull every activation row through every CU (1.3 GB of ingest for that projection: 85 us).  K split over
-    // gridDim.y workgroups per tile instead, the slices summed by the norm that follows (which must be the row kernel).
+    // gridDim.y workgroups per tile instead, the slices summed by the norm that follows (a row or a tile of eight a workgroup).
     const bool norm_ok = (M <= 512 && m->H <= 1024 * NORM_ROW_MAXCH) || (m->H % 32 == 0 && m->H <= 2048 && g_norm_t16);   // launch_norm
     if (g_sk_tile && !m->f32 && M > (g_mid && K >= 2048 ? std::max(64, std::min(g_mid_resid_rows, g_chunk_max_m)) : 64) && M <= m->sk_rows && !m->keep_hidden && m->sk_part && m->pending_slices == 0 &&
         N % 128 == 0 && K % 64 == 0 && norm_ok && N == m->H && g_force_tile == 0 && m->n_mamba == 0) {
@@ -1657,7 +1657,7 @@ void moe_expert_gemms(nvl_model* m, const MoeW& w, int M, int BM, bool pp, bool 
     if (!small && m->moe_xg && g_moe_gather) {
         // prefill: every m-tile's rows would be re-gathered 16 bytes at a time by each of its 2I/128 column tiles
         // (64 cache lines per load instruction); copy them into expert order once, then the GEMM streams whole
-        // 1-KiB operand blocks (Granite-1B, 16384 tokens: expert-up 1119 -> ? us per layer)
+        // 1-KiB operand blocks (Granite-1B, 16384 tokens: expert-up 1080 -> 390 us per layer)
         KScope ks(m, KC_OTHER);
         if (xn_rows) hipLaunchKernelGGL((moe_gather_fm_kernel<true>), dim3(cdiv(pairs, 16)), dim3(256), 0, m->stream, xn_rows, m->perm_token, (bf16_t*)m->moe_xg, pairs, H);
         else hipLaunchKernelGGL((moe_gather_fm_kernel<false>), dim3(cdiv(pairs, 16)), dim3(256), 0, m->stream, (const bf16_t*)m->xn, m->perm_token, (bf16_t*)m->moe_xg, pairs, H);

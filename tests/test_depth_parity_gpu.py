@@ -276,10 +276,10 @@ def test_full_depth_big_configs(gpu, oracle, capsys, key):
 
 
 def test_moe_down_as_deferred_norm_producer(gpu):
-    """MoE decode, tuning key 33 = 1 (off by default: slower): the experts' down projection keeps all of K in
-    one workgroup — a wave's range covers two experts, streamed block by block through a liveness mask — and carries the next
-    layer's attention norm, so no norm launch sums K slices.  Granite-3.0-1B shapes (the tiny test configs do not meet the
-    form's divisibility conditions), 3 layers, batches of 5 and 24 rows: a decode step against the default form."""
+    """MoE decode, tuning key 33 = 1 (the default): the last of the workgroups that hold K slices of the experts' down projection adds
+    them, completes the residual and carries the next layer's attention norm, so no norm launch sums K slices (0: it does).
+    Granite-3.0-1B shapes (the tiny test configs do not meet the form's divisibility conditions), 3 layers, batches of 5 and 24
+    rows: a decode step in both forms."""
     import torch
     from bench import gen_weights_on_device
     cfg = dict(gpu.synth.FULL_CONFIGS["granite-3.0-1b-a400m"])
