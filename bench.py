@@ -1,6 +1,6 @@
 #!/usr/bin/env python3
 """bench.py — prefill + decode tokens/s of the HIP forward path on synthetic fixed-seqlen/batch
-prompts (BASELINE.json metric), with the kernel roofline and the CPU restatement beside it.
+prompts, with the kernel roofline and the CPU restatement beside it.
 
 A "step" = one pass of the hot path over one batch: B sequences x S prompt tokens prefilled
 (TransformerModel.ForwardWithCache at pos 0), then G greedy decode steps per sequence (the
@@ -161,7 +161,7 @@ def gen_weights_on_device(pkg, cfg, model, torch, device, keep_host: bool):
 
 
 def flops_per_token(cfg):
-    """SURVEY.md §8(d): GEMM FLOPs per token for the layer stack, and for one LM-head row."""
+    """GEMM FLOPs per token for the layer stack, and for one LM-head row."""
     H, L, V = cfg["hidden"], cfg["num_layers"], cfg["vocab_size"]
     nH, hd, F = cfg["num_heads"], cfg["head_dim"], cfg["ffn_dim"]
     at = cfg["attention_type"]
@@ -249,7 +249,7 @@ def main():
         model.tp_p2p_attach(handles)
     t_load = time.time() - t0
 
-    # SURVEY.md §8(d): seed 1234 + cfg_idx; data parallel: +rank (own sequences); tensor parallel: same batch on all ranks
+    # seed 1234 + cfg_idx; data parallel: +rank (own sequences); tensor parallel: same batch on all ranks
     rng = np.random.default_rng(1234 + 1 + (0 if tp else rank))
     prompts = rng.integers(0, cfg["vocab_size"], (B, S)).astype(np.int32)
     seq_ids = list(range(B))

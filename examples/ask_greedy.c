@@ -1,5 +1,5 @@
 /* ask_greedy.c — the greedy generation loop of cmd/ask (generateResponse, cmd/ask/main.go:287-360) written against the C
- * ABI alone (include/nvllm.h): what the cgo shim of INTEGRATION.md does, without Go and without Python.
+ * ABI alone (include/nvllm.h): what the cgo shim does, without Go and without Python.
  *
  *   ask_greedy <model-dir> <max-new-tokens> <token id> [<token id> ...]
  *

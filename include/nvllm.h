@@ -2,8 +2,8 @@
  * nvllm.h — C ABI of libnvllm_hip.so: the MI355X (gfx950) forward path that
  * replaces nano-vllm-go's purego/tensor prefill + decode hot path.
  *
- * Drop-in boundary.  A Go maintainer binds these with cgo (stub in
- * INTEGRATION.md) and implements nanovllm.ModelRunner on top of them; nothing
+ * Drop-in boundary.  A Go maintainer binds these with cgo and
+ * implements nanovllm.ModelRunner on top of them; nothing
  * else in nano-vllm-go changes.  Every entry point names the reference
  * interface it replaces (file:line under the reference repository).
  *
@@ -302,7 +302,7 @@ int nvl_finalize(nvl_model* m);
 /* Replaces TensorModelRunner.Close (tensor_model_runner.go:114-117). */
 void nvl_destroy(nvl_model* m);
 
-/* ---- tensor parallelism (SURVEY.md §8 e-2; the reference's Config.TensorParallelSize is inert: nanovllm/config.go:61) ----
+/* ---- tensor parallelism (the reference's Config.TensorParallelSize is inert: nanovllm/config.go:61) ----
  * A model created with tp_size = T > 1 is rank tp_rank's shard: column-parallel Q/K/V and gate/up, row-parallel O and
  * down, one all-reduce (sum, fp32) after the O projection and one after the down projection; embeddings, norms and the
  * LM head are replicated, so every rank produces the same logits and the same greedy token.  Upload the FULL tensors:

@@ -568,8 +568,8 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t
     };
     // Load order (vector loads return in issue order): the new token's fp32 q/k/v row + cos/sin FIRST (a dozen small loads),
     // the round's K/V stream right behind them with no wait in between, THEN the RoPE arithmetic — it waits for the row only
-    // (counted vmcnt) and runs, like the first QK^T MFMAs after it, while the K/V tiles are still arriving.  Round 2 waited
-    // for the row with vmcnt(0) before issuing the first K load; the first round-3 order (K/V first, row behind) made the
+    // (counted vmcnt) and runs, like the first QK^T MFMAs after it, while the K/V tiles are still arriving.  An earlier form waited
+    // for the row with vmcnt(0) before issuing the first K load; the next order (K/V first, row behind) made the
     // RoPE and every MFMA wait for the whole K/V transfer (in-kernel stamps, scripts/decode_timeline.py: 2.3 us of compute
     // after 6 us of transfer, nothing overlapped).  Only the 8-wave hd-64 instantiation (GQA models at decode batches that
     // fill the chip with one workgroup per CU) has the 26 registers to spare.
@@ -589,7 +589,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t
         const float* vrow = row + (p.nH + p.nKV + kvh) * HD + dch * 8;
         v0 = *(const f32x4*)vrow; v1 = *(const f32x4*)(vrow + 4);
     }
-    // every other instantiation: the new token's row and its rotation BEFORE the K/V stream, as in round 2 — behind it the
+    // every other instantiation: the new token's row and its rotation BEFORE the K/V stream — behind it the
     // row's temporaries are live together with the round's 32 K/V fragments (hd 64, 2 / 4 waves — MHA models: 237 -> 276
     // registers, one wave per SIMD instead of two, GPT-2 B = 128 attention 46 -> 51 us; hd 128, 8 waves: 22 spilled)
     if (!ROW_FIRST && FUSED) {

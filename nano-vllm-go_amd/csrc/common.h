@@ -143,9 +143,9 @@ __device__ __forceinline__ float wave_max(float v) {
 // top of a kernel would make every later uniform load a vector load (the compiler may no longer assume the loaded
 // memory unclobbered, so it cannot use the scalar cache) — the instrumentation would change what it measures.
 #ifndef NVL_STAMPS
-// the product library: no stamp site at all.  (Round 3 first shipped the sites compiled in and disabled by a NULL buffer:
+// the product library: no stamp site at all.  (The sites compiled in and disabled by a NULL buffer are not free:
 // each one still is a branch with two scheduling barriers inside, which splits the kernel's scheduling regions — every
-// decode projection ran 3-7 % slower than in round 2, 31.0 K against 32.1 K decode tok/s at B = 32 on the same box,
+// decode projection ran 3-7 % slower than without, 31.0 K against 32.1 K decode tok/s at B = 32 on the same box,
 // profiles/r03_ab_vs_r02.txt.)  `make diag` builds libnvllm_hip_diag.so with -DNVL_STAMPS for scripts/decode_timeline.py.
 struct NvlStamps {
     __device__ __forceinline__ NvlStamps(unsigned long long*, int) {}

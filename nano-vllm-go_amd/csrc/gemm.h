@@ -1,5 +1,5 @@
 // gemm.h — projection GEMMs of the forward path (replaces tensor.MatMul,
-// purego/tensor/tensor.go:62-88, at every call site listed in SURVEY.md §8 a3).
+// purego/tensor/tensor.go:62-88, at every call site of the layer stack).
 //
 //   C[M,N] = A[M,K] · W[N,K]^T   (+ fused epilogue)
 //

@@ -1,5 +1,5 @@
-// loader.h — safetensors -> device, without the reference's fp32 host expansion and host transposes
-// (SURVEY §8 f-2).  Host-only C++; included at the end of nvllm.hip.
+// loader.h — safetensors -> device, without the reference's fp32 host expansion and host transposes.
+// Host-only C++; included at the end of nvllm.hip.
 //
 // Replaces tensor.LoadModelFromDirectory / LoadModel / LoadShardedModel (purego/tensor/generic_loader.go:184-265,
 // 1016-1163) and LoadModelConfig (:808-972).  The checkpoint is mmap'ed; every 2-D weight goes to nvl_upload_tensor

@@ -263,7 +263,7 @@ __global__ __launch_bounds__(256) void mamba_step_kernel(MambaArgs p, bf16_t* __
 //     G = C B^T (Q x Q, k = state);  Y_intra = (G o L) U (k = token);  Y_inter = C S_in^T (k = state);  S += (U o w)^T B (k = token)
 // Every decay factor is exp of a NON-POSITIVE fp32 number (s decreases), the state lives in fp32 accumulators across the
 // chunks and is rounded to bf16 only as the Y_inter operand; u, B, C and the masked decay matrix G o L are rounded to bf16 as
-// MFMA operands — the same kind of rounding point the projections around this kernel already have (DESIGN.md §3); the
+// MFMA operands — the same kind of rounding point the projections around this kernel already have; the
 // fp32 parity mode keeps mamba_scan_kernel.  Operands sit in LDS K-contiguous ([row][k], rows padded by 16 bytes: the
 // fragment reads are conflict-free), B and U additionally transposed.  A ragged last chunk runs with dt = 0 for the missing
 // tokens: they neither decay nor feed the state, and their rows are not stored.

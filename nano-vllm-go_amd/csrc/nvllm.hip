@@ -314,7 +314,7 @@ extern "C" int nvl_create(const nvl_model_config* cfg, const nvl_runtime_opts* o
     m->L = c.num_layers;
     m->nKV = c.attention_type == NVL_ATTN_MHA ? c.num_heads : (c.attention_type == NVL_ATTN_MQA ? 1 : c.num_kv_heads);
     if (m->nKV <= 0 || m->nH % m->nKV != 0) throw std::runtime_error("num_heads must be a multiple of num_kv_heads");
-    // tensor parallel shard (SURVEY.md §8 e-2): this rank owns nH/tp query heads, nKV/tp kv heads and F/tp FFN
+    // tensor parallel shard: this rank owns nH/tp query heads, nKV/tp kv heads and F/tp FFN
     // columns; from here on nH / nKV / F are the LOCAL sizes (hidden H, vocab V stay full: residual stream,
     // norms, embeddings and the LM head are replicated)
     m->tp = tp; m->tp_rank = tp > 1 ? opts->tp_rank : 0;
@@ -2277,7 +2277,7 @@ extern "C" int nvl_forward_rows(nvl_model* m, int n_seqs, const int64_t* seq_ids
     return forward_impl(m, n_seqs, seq_ids, tokens, seq_lens, pos_offsets, 0, n_rows, rows, false, logits_out, argmax_out);
 }
 
-// nvl_forward for a model whose KV cache is the host block manager's pool (SURVEY §8 f-1; block_manager.go:128-263,
+// nvl_forward for a model whose KV cache is the host block manager's pool (block_manager.go:128-263,
 // sequence.go:22-23): no per-sequence state here, the block tables say where every position lives.
 extern "C" int nvl_forward_paged(nvl_model* m, int n_seqs, const int32_t* tokens, const int32_t* seq_lens,
                                  const int32_t* pos_offsets, const int32_t* block_tables, const int32_t* table_offsets,
@@ -2361,7 +2361,7 @@ extern "C" int nvl_forward_paged(nvl_model* m, int n_seqs, const int32_t* tokens
 }
 
 // ModelRunner.Run over block tables: what a runner that honours Sequence.BlockTable / NumCachedTokens does
-// (the reference's runners ignore both: SURVEY §2 row 17).
+// (the reference's runners ignore both).
 extern "C" int nvl_runner_run_paged(nvl_model* m, int n_seqs, const int32_t* const* token_ptrs, const int32_t* token_lens,
                                     const int32_t* num_cached_tokens, const int32_t* const* block_table_ptrs,
                                     const int32_t* block_table_lens, int is_prefill, int32_t* next_tokens,
@@ -2872,7 +2872,7 @@ extern "C" int nvl_get_kernel_stats(nvl_model* m, nvl_kernel_stat* out, int cap)
 // runner: ModelRunner.Run semantics (tensor_model_runner.go:55-97)
 // =================================================================================================
 // =================================================================================================
-// on-device sampling (SURVEY §8 f-3): tensor.SampleWithHistory, sampling.go:33-102
+// on-device sampling: tensor.SampleWithHistory, sampling.go:33-102
 // =================================================================================================
 namespace {
 // rows of device logits -> sampled ids on the host.  `err` receives the reason when the arguments are refused.

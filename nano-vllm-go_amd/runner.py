@@ -1,7 +1,7 @@
 """Host-side mirror of nanovllm.TensorModelRunner (nanovllm/tensor_model_runner.go:11-117) and of the
 fields of nanovllm.Sequence a runner reads (nanovllm/sequence.go:15-28), over nvl_runner_run.
 
-In a Go build this file is replaced by the cgo shim in INTEGRATION.md; here it lets the parity tests
+In a Go build this file is replaced by the cgo shim; here it lets the parity tests
 read like tests of the reference's own runner."""
 from __future__ import annotations
 
@@ -100,7 +100,7 @@ class HipModelRunner:
 
 class HipPagedModelRunner:
     """A ModelRunner that honours what the scheduler's BlockManager computed (block_manager.go:128-263) — the
-    reference's runners ignore Sequence.BlockTable / NumCachedTokens (SURVEY §8 f-1).  The model must be created with
+    reference's runners ignore Sequence.BlockTable / NumCachedTokens.  The model must be created with
     kv_num_blocks = the block manager's pool size; the KV cache then IS that pool: prefix-cache hits skip their
     prefill work, finished sequences free memory the moment the block manager reuses their blocks."""
 

@@ -18,7 +18,7 @@ def round_bf16(a: np.ndarray) -> np.ndarray:
 
 
 def make_weights(cfg: dict, seed: int = 42, scale: float = 0.02, peaked_head: float = 0.0) -> dict:
-    """{(slot, layer): fp32 ndarray} in reference post-load layout.  SURVEY.md §8(d): weights
+    """{(slot, layer): fp32 ndarray} in reference post-load layout.  Weights
     N(0, scale^2) seeded per layer (seed+layer), norm weights 1+0.02n, biases 0.02n.
     peaked_head > 0 scales an UNTIED LM head (larger logits; used by the greedy fixtures)."""
     H, L, V = cfg["hidden"], cfg["num_layers"], cfg["vocab_size"]

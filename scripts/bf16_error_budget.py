@@ -1,7 +1,7 @@
 """Where does the bf16 mode's per-layer error come from?  CPU only: tests/bf16_emulator.py (float64 with a bf16 rounding at
 each point where the HIP path rounds an MFMA operand) on the bench model's weights and prompt, one rounding point at a time
 and all together, then the whole stack.  The "all together" curve is what tests/test_depth_parity_gpu.py measures on the
-device: round 3 found them equal to two digits at every one of the 16 layers.
+device: they are equal to two digits at every one of the 16 layers.
 usage: python scripts/bf16_error_budget.py [tokens] [layers]"""
 import importlib
 import sys

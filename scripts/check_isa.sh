@@ -6,7 +6,7 @@
 #     moment ago and serialise the LDS-DMA ring): the only vmcnt(0) in the kernel are the Q-fragment wait before the loop
 #     and the hand-written one for the last tile;
 #   * no register spills.
-# And the register budgets of the decode kernels (from the code object metadata in the same assembly): round 3 lost 5-14 % of
+# And the register budgets of the decode kernels (from the code object metadata in the same assembly): once lost were 5-14 % of
 # decode throughput on three configs to changes that were only measured on the headline one — the MHA / small-batch
 # decode-attention instantiations went from two waves per SIMD to one, the 64-row-group projections spilled 34-54 registers.
 set -e

@@ -1,5 +1,5 @@
 """Per-kernel roofline table (markdown) of the bench step from a scripts/prof_decode.py breakdown (rocprofv3 durations)
-and the algorithmic work of Llama-3.2-1B at 32 x 512 + 128 (DESIGN.md §5).  usage: profiles_table.py <breakdown.txt>"""
+and the algorithmic work of Llama-3.2-1B at 32 x 512 + 128.  usage: profiles_table.py <breakdown.txt>"""
 import re, sys
 M, H, F, V, NQKV = 16384, 2048, 8192, 128256, 3072
 work = {  # (phase, site) -> (flops, bytes, bound)

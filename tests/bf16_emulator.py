@@ -1,11 +1,11 @@
 """A CPU emulation (numpy, float64) of the bf16 PRODUCT path's rounding points — test infrastructure, like the oracle.
 
 The HIP path keeps the residual stream, norms, softmax statistics, RoPE and every accumulation in fp32 and rounds to bf16
-exactly where a value becomes an MFMA operand (DESIGN.md §3):
+exactly where a value becomes an MFMA operand:
     xn   normed input of the QKV projection        q    RoPE'd query             k, v  RoPE'd key / value in the KV cache
     p    softmax probabilities                      ao   attention output          xn2   normed input of the FFN-up projection
     h    silu(gate) * up                            xl   final-norm output (LM head operand)
-This module runs a Llama-family stack (GQA + RoPE + RMSNorm + SwiGLU, sequential blocks: BASELINE configs[1]) in float64
+This module runs a Llama-family stack (GQA + RoPE + RMSNorm + SwiGLU, sequential blocks) in float64
 with a bf16 rounding at each of those points, on the same weights and prompt as a device run.  If the kernels round there
 and nowhere else, the device's error against the oracle equals this emulation's error against the oracle, layer by layer
 — which is what tests/test_depth_parity_gpu.py asserts (and scripts/bf16_error_budget.py breaks down per rounding point).

@@ -1,7 +1,7 @@
 """Test helper: turn a HuggingFace state_dict into the tensors nano-vllm-go would hold after
 LoadModel (purego/tensor/generic_loader.go:184-265, weight mappings :60-181), using the ORACLE's
 restatements of the loader's layout functions (Transpose, splitGPT2QKV, splitFalconQKV, combineMQAKV,
-ConcatenateLastDim) so the layout contract (SURVEY.md §8 a14) is exercised end to end."""
+ConcatenateLastDim) so the layout contract is exercised end to end."""
 import numpy as np
 
 

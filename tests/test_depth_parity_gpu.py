@@ -1,6 +1,6 @@
-"""Parity at FULL DEPTH, per layer (round-3 item: "earn the tolerance").
+"""Parity at FULL DEPTH, per layer.
 
-DESIGN.md §3 holds the error model.  Its first version was written down BEFORE any per-layer measurement, with the wrong
+The first version of the error model was written down BEFORE any per-layer measurement, with the wrong
 constant (2^-9 taken for bf16's unit roundoff; bf16 keeps 8 significant bits: it is 2^-8) and a sqrt growth law: the first
 device run sat at 2.1x that bound at layer 0 and 1.2x at layer 15.  scripts/bf16_error_budget.py then rebuilt the path's
 roundings on the CPU (tests/bf16_emulator.py: float64 with a bf16 rounding at the eight points per layer where a value
@@ -24,7 +24,7 @@ becomes an MFMA operand) — and reproduces the device's error against the oracl
   * fp32 parity mode: 1e-4 (max norm) at every layer and depth.
 
 What runs:
-  * Llama-3.2-1B (16 layers, the bench model) and GPT-2 (configs[0], 12 layers): the CPU oracle at full
+  * Llama-3.2-1B (16 layers, the bench model) and GPT-2 (12 layers): the CPU oracle at full
     depth and width on a 24-token prompt + one decode token, every layer's residual stream of the bf16 PRODUCT path (debug
     mode 2: taps beside the unmodified kernel sequence — deferred RMSNorm, split-K partials and all) and of the fp32 mode.
   * Falcon-7B (32 layers, MQA 71/1, parallel block), Granite-3.0-1B-A400M (24 layers, 32 experts top-8), Llama-3-8B
@@ -32,7 +32,7 @@ What runs:
     the batch sizes profiles/r02_other_configs.txt was measured at — every layer of a B x 64-token prefill (the tile kernels)
     and of a decode step (the decode kernels) bf16 vs the fp32 mode, and the last-row logits of a B x 256 prefill + 4
     teacher-forced decode steps.
-The growth curves are printed (pytest -s shows them; DESIGN.md §3 records what round 3 measured).
+The growth curves are printed (pytest -s shows them).
 """
 import math
 import os

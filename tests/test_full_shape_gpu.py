@@ -1,4 +1,4 @@
-"""Parity at the BASELINE configs' FULL layer shapes, where the tiny fixtures cannot reach:
+"""Parity at the benchmark models' FULL layer shapes, where the tiny fixtures cannot reach:
 Falcon's H = 4544 = 71 x 64 (not a multiple of 128), MQA with 71 query heads on one KV head, Llama's 128256-row
 tied LM head, GPT-2's odd vocabulary, Granite's 32-expert top-8 routing.  Layer COUNT is reduced (the layers are
 identical in shape) so the CPU oracle finishes in seconds; widths, head counts, vocabularies and expert counts
@@ -94,7 +94,7 @@ def test_device_path_properties_at_full_width(gpu, name):
 
 @pytest.mark.parametrize("key,layers,B", [("llama-3.2-1b", 2, 16), ("llama-3-8b", 1, 8)])   # hd 64 / hd 128 QKV epilogues
 def test_bench_sized_prefill_pingpong(gpu, key, layers, B):
-    """The prefill form only BASELINE-sized batches reach (>= 256 tiles of 256x256: the ping-pong GEMM with its fused
+    """The prefill form only benchmark-sized batches reach (>= 256 tiles of 256x256: the ping-pong GEMM with its fused
     QKV / SwiGLU / residual epilogues) at 16 x 512 tokens of Llama-3.2-1B-wide layers.  The oracle cannot run 8192
     full-width tokens in test time, so: (a) the same batch in fp32 parity mode (validated against the oracle on the
     small cases) within the bf16 tolerance, (b) a sequence's logits equal to its solo (small-M kernels) run."""

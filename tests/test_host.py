@@ -25,7 +25,7 @@ def test_load_model_config_llama32_1b_with_reference_quirks(pkg):
     c = pkg.config.load_model_config(hf)
     assert (c.hidden, c.num_layers, c.num_heads, c.num_kv_heads, c.head_dim, c.ffn_dim) == (2048, 16, 32, 8, 64, 8192)
     assert c.rope_base == 500000.0 and c.norm_eps == 1e-5 and c.tied_embedding
-    assert c.max_seq_len == 4096          # max_position_embeddings is never read (SURVEY.md §3.3)
+    assert c.max_seq_len == 4096          # max_position_embeddings is never read
     assert c.eos_token_id == 2            # a JSON list is not a float64: the template value survives (:881-883)
     assert c.bos_token_id == 128000
 

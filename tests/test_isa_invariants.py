@@ -3,7 +3,7 @@ GPU, so this runs in the CPU suite.  What it pins: M0 is written only by the LDS
 declared as a clobber), the compiler has put no `s_waitcnt vmcnt(0)` into the tile loop (that serialises the LDS-DMA
 ring: the kernel then still computes the right thing, only ~25 % slower, so no numerical test would notice), no spills.
 And the register budgets of the decode kernels (two waves per SIMD for the hd-64 decode attention, bounded spills in the
-decode projections): round 3 lost 5-14 % of decode throughput on GPT-2, Llama-3-8B and the 64-row-group projections to
+decode projections): once lost were 5-14 % of decode throughput on GPT-2, Llama-3-8B and the 64-row-group projections to
 changes measured only on the headline config — no numerical test notices those either."""
 import os
 import shutil

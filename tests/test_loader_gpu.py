@@ -1,4 +1,4 @@
-"""SURVEY §8 f-2: nvl_load_safetensors (mmap -> device, dtype conversion + transposes + tiling on the device) must
+"""nvl_load_safetensors (mmap -> device, dtype conversion + transposes + tiling on the device) must
 build the same model as the reference's load path (checkpoint -> fp32 -> Transpose -> per-tensor placement, here the
 Python upload path fed the reference's post-load layout): logits IDENTICAL bit for bit, all four families, three
 dtypes, single-file and sharded, with and without the "transformer." name prefix."""
@@ -132,7 +132,7 @@ def _get_weight(gpu, hm, slot, layer, n_in, n_out):
 @pytest.mark.parametrize("precision", ["f32", "bf16"])
 def test_reference_falcon_fixture_through_the_librarys_own_split(gpu, oracle, precision):
     """purego/tensor/falcon_split_test.go:7-158 — the ONLY vectors the reference's tests hold on this path — replayed on
-    nvl_upload_falcon_qkv itself (round 2 replayed them on the oracle only): the fused query_key_value matrix goes in as
+    nvl_upload_falcon_qkv itself: the fused query_key_value matrix goes in as
     the reference holds it after Transpose ([hidden, (nH + 2) hd]), the device's Q and K|V weights are read back in the
     reference's post-load layout (nvl_get_weight) and compared with the fixture's expectations and, element for element,
     with the oracle's splitFalconQKV + combineMQAKV (generic_loader.go:705-765)."""

@@ -1,4 +1,4 @@
-"""SURVEY.md §8 (f-4): Mamba2 / Granite-4 hybrid layers on the device (csrc/mamba.h) against the CPU oracle's
+"""Mamba2 / Granite-4 hybrid layers on the device (csrc/mamba.h) against the CPU oracle's
 restatement of purego/tensor/mamba2.go:74-351 and of the hybrid dispatch (generic_model.go:67-202, 285-292, 456-459).
 
 Tolerances as everywhere: fp32 parity mode 1e-4, bf16 product path 1.5e-2 of the largest value.

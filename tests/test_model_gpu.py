@@ -81,7 +81,7 @@ def test_greedy_token_ids_bit_exact(gpu, oracle, family, precision):
     """cmd/ask's generateResponse loop (main.go:287-360) with argmax: identical token ids.
     A random-weight model has tiny top-2 margins, so the fixture prompt is the first seeded prompt
     whose ORACLE margins (top1-top2 over max|logit|) all exceed 2x the stated logits tolerance (the
-    reference itself is not reproducible below that: arm64 fuses FMAs, amd64 does not — SURVEY.md §7)."""
+    reference itself is not reproducible below that: arm64 fuses FMAs, amd64 does not)."""
     cfg, om, hm = build(gpu, oracle, family, precision, peaked=4.0, tied_embedding=False)
     need = 2 * TOL[precision]
     for seed in range(600):
@@ -417,8 +417,8 @@ def test_moe_decode_routing_one_launch_matches_two(gpu, oracle):
 
 def test_fused_loop_graph_survives_a_longer_second_call(gpu, oracle):
     """nvl_decode_greedy keeps its step tokens in a device ring that grows with n_steps x n_seqs; the captured step graph
-    holds the ring's address as a kernel argument, so growing the ring must drop the captured graphs (round-2 advisor
-    finding: a 4-step call followed by a 40-step call replayed a graph that wrote into the freed ring).  A short call, then
+    holds the ring's address as a kernel argument, so growing the ring must drop the captured graphs (it did not
+    once: a 4-step call followed by a 40-step call replayed a graph that wrote into the freed ring).  A short call, then
     a longer one on the same model and batch, against stepwise nvl_forward on a second model."""
     cfg, om, hm = build(gpu, oracle, "llama", "bf16")
     hs = gpu.HipTransformerModel(cfg, gpu.synth.make_weights(cfg, seed=7, scale=0.05), precision="bf16", max_seqs=4,

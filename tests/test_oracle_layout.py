@@ -1,4 +1,4 @@
-"""Layout contract of the load path (SURVEY.md §8 a14), checked on the CPU oracle.
+"""Layout contract of the load path, checked on the CPU oracle.
 
 test_split_falcon_qkv* replay the ONLY vectors the reference's own tests pin on the hot path:
 purego/tensor/falcon_split_test.go:7-158 (data regenerated in tests/golden/make_golden.py)."""

@@ -1,4 +1,4 @@
-"""the KV cache addressed through the host block manager's tables (nanovllm/block_manager.go,
+"""The KV cache addressed through the host block manager's tables (nanovllm/block_manager.go,
 Sequence.BlockTable / NumCachedTokens).  The block tables come from a restatement of that block manager
 (tests/block_manager_mirror.py), used the way scheduler.go uses it.
 

@@ -1,4 +1,4 @@
-"""Real-weight anchors the reference's own docs and CLIs record (SURVEY.md §8 c) — the only numbers of the Go binary this
+"""Real-weight anchors the reference's own docs and CLIs record — the only numbers of the Go binary this
 path can be pinned to.  They need checkpoints that are not in this image (there is no network), so every test SKIPS
 unless its model directory is given:
 

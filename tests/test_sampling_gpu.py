@@ -1,4 +1,4 @@
-"""SURVEY §8 f-3: tensor.SampleWithHistory (purego/tensor/sampling.go:33-102) on the device (nvl_op_sample, nvl_sample,
+"""tensor.SampleWithHistory (purego/tensor/sampling.go:33-102) on the device (nvl_op_sample, nvl_sample,
 nvl_runner_run_sampled) against the CPU oracle's restatement, with the rand.Float32() draw passed to both.
 
 Stated tolerance.  The reference sums V probabilities sequentially in fp32 (softmax denominator, renormalisation,

@@ -1,4 +1,4 @@
-"""Tensor parallelism (SURVEY.md §8 e-2) on ONE GPU: the T shard models of a group live in one process, are driven
+"""Tensor parallelism on ONE GPU: the T shard models of a group live in one process, are driven
 from one host thread each, and all-reduce through the library's local group (nvl_tp_attach_local) — the same
 forward code as the RCCL path, with the collective emulated.  Checks the sharded arithmetic (column-parallel
 Q/K/V/gate/up, row-parallel O/down, one all-reduce after each) against the un-sharded CPU oracle, and that every
@@ -109,7 +109,7 @@ def test_rccl_single_rank_communicator(gpu):
 
 
 def test_tp8_llama3_8b_shapes_match_unsharded_oracle(gpu, oracle):
-    """BASELINE config 5, "Llama-3-8B bf16 TP=8": the T = 8 slice at the real widths — hd 128, exactly ONE KV head and
+    """Llama-3-8B in bf16, TP = 8: the T = 8 slice at the real widths — hd 128, exactly ONE KV head and
     4 query heads per rank, F/8 = 1792 = 28 x 64 SwiGLU columns (an odd count of 128-wide tiles), V = 128256 — as 8
     shard models of a 1-layer model in one process (nvl_tp_attach_local; one GPU per box).  Prefill of 320 tokens
     (fused hd-128 QKV epilogue, tile kernels on the sharded widths) + 3 decode steps; every rank's logits equal the
