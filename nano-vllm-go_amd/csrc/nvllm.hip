@@ -1244,18 +1244,23 @@ static int g_attn_split = 1;   // nvl_set_tuning key 25: split a decode attentio
 // Launch shape of the decode attention for the batch being enqueued (also part of a captured graph's key): waves per
 // workgroup | most workgroups per (sequence, kv head) << 8 | key tiles a workgroup has at least << 12.
 // Split: a workgroup pulls all K/V of its (sequence, kv head) through ONE CU, one round of tiles after the other; with few of
-// them and a long context that, not HBM, is the time.  A sequence is then dealt over workgroups of one round each (attn.h), and the
-// last of them combines the parts.  That costs every launch about 2 us, in parts written, counted and read back, so that a
-// context has to be longer the fuller the chip already is; beyond 128 pairs a split only adds traffic.  The lines lie where whole
-// decode steps change sides (a launch by itself favours the split earlier: it does not wait for the kernel before it).  A step
-// split against whole, per cent, at keys of each sequence:
-//   Llama-3.2-1B (8 kv heads of 64)    600   700   800   900   1000/1100  1500     Llama-3-8B (8 of 128)     340   530   650   800   1100
-//     1 sequence                      +1.1  -0.3  -1.8  -2.9  -3.5                   1 to 4 sequences       -0.3 and on to -1.1
-//     4                               +0.9  +0.3  -0.2  -1.0  -1.3                   6 to 12                      +2.4  +1.1  -1.0  -2.6
-//     6                               +1.2  +0.9  +0.5  -0.2  -0.5
-//     8                                           +1.5  +0.4  -1.6       -5.0
-//    12                                           +1.0        +1.2       +0.6 (contexts of a quarter to all of that: -0.9, -2.5)
-//    16                                           +2.2  +2.0  +1.5       +0.2 (ragged: -1.4 at 1100, -1.0)
+// them and a long context that, not HBM, is the time.  A sequence is then dealt over workgroups (attn.h), and the last of them
+// combines the parts, which costs a launch about 2 us: a context has to be longer the fuller the chip already is.  No more parts than
+// leave a CU to each workgroup (256 / pairs), and as many as give each the same number of rounds: beyond 128 pairs a split only
+// adds traffic.  The lines lie where whole decode steps change sides (a launch by itself favours the split earlier: it does not wait for the
+// kernel before it).  Steps against the whole form, per cent (waves x parts; forms in random order, runs differ by 0.5):
+//   heads of 64, Llama-3.2-1B, 8 kv heads     keys  520 +0.8 (2 x 3)   700 -1.6 (2 x 3)  1000 -4.6 (2 x 4)  1500 -8.7 (4 x 3)     1 sequence
+//                                                   600 +0.8 (2 x 3)   800 -0.6 (2 x 4)  1200 -1.6 (4 x 3)  1800 -7.4 (4 x 4)     4
+//                                                   700 +0.6 (2 x 3)  1000 -0.6 (4 x 2)  1500 -6.9 (4 x 3)                        6
+//                                                   700 +0.5 (2 x 3)  1000 -1.4 (4 x 2)  1400 -4.5 (4 x 3)  1900 -3.4 (4 x 4)     8
+//                                                   900 -1.3 (4 x 2)  1300 -3.8 (4 x 3)                                          10
+//                                                  1100 +0.9 (4 x 3)  1500 +1.0 (4 x 3), -1.1 (8 x 2)  1900 -3.9 (8 x 2)         12
+//                                                  1000  0.0 (4 x 2)  1500 -0.2 (4 x 3), -0.6 (8 x 2)  1900 -3.1 (8 x 2)         16
+//   heads of 128, Llama-3-8B, 8 kv heads            400 -0.5 (2 x 4)   700 -2.4 (4 x 3)  1500 -9.4 (4 x 6)                        1
+//                                                   400 -1.1 (2 x 4)   800 -4.7 (4 x 4)  1500 -8.9 (4 x 6)                        4
+//                                                   400 -0.3 (2 x 4)   600 -1.9 (4 x 3)   900 -4.3 (4 x 4)  1500 -6.6 (4 x 3)     8
+//                                                   600 +0.8 (4 x 2)  1000 -3.0 (4 x 2)  1500 -4.3 (4 x 2), +3.6 (4 x 3)         12
+//                                                  1000 -1.6 (4 x 2), +2.6 (4 x 4)  1500 -3.0 (4 x 2)                            16
 int decode_attn_cfg(const nvl_model* m, int n_seqs) {
     const int n_kt = m->ctx_hint > 0 ? (m->ctx_hint - 1) / 64 + 1 : 1 << 20;
     const int per_wave = m->hd == 64 ? 2 : 1;
@@ -1268,9 +1273,13 @@ int decode_attn_cfg(const nvl_model* m, int n_seqs) {
     if (g_attn_split >= 2) { const int tiles = (g_attn_split - 1) * nw * per_wave; return cfg(nw, std::max(1, std::min(most, cdiv(n_kt, tiles))), tiles); }
     if (g_attn_split && !g_attn_nw && most > 1) {
         int waves = 0;
-        if (m->hd == 64) waves = wgs > 128 || n_kt <= (wgs <= 32 ? 12 : wgs <= 64 ? 16 : 20) ? 0 : wgs <= 48 && n_kt <= 20 ? 2 : 4;
-        else waves = wgs <= 32 ? (n_kt > 16 ? 4 : n_kt > 5 ? 2 : 0) : wgs <= 96 && n_kt > 12 ? 8 : 0;
-        if (waves) return cfg(waves, std::min(most, cdiv(n_kt, waves * per_wave)), waves * per_wave);
+        if (m->hd == 64) waves = wgs <= 32 ? (n_kt > 20 ? 4 : n_kt > 12 ? 2 : 0) : wgs <= 85 ? (n_kt > 14 ? 4 : 0) : wgs <= 128 && n_kt > 20 ? 8 : 0;
+        else waves = wgs <= 64 ? (n_kt > 10 ? 4 : n_kt > (wgs <= 32 ? 5 : 6) ? 2 : 0) : wgs <= 128 && n_kt > 12 ? 4 : 0;
+        if (waves) {
+            const int round = waves * per_wave, rounds = cdiv(n_kt, round);
+            const int each = cdiv(rounds, std::max(1, std::min(most, 256 / wgs)));      // rounds of a part
+            if (each < rounds) return cfg(waves, cdiv(rounds, each), each * round);
+        }
     }
     return cfg(nw, 1, 1 << 16);
 }
