@@ -293,6 +293,27 @@ def test_decode_attention_in_parts(gpu, hd, kv, waves, rounds):
     assert rel_err(got[1], got[0]) <= TOL
 
 
+@pytest.mark.parametrize("hd,n,longest", [(64, 10, 1900), (64, 12, 1500), (64, 16, 1300), (128, 8, 1500), (128, 12, 1500), (128, 16, 800)])
+def test_decode_attention_parts_by_pairs(gpu, hd, n, longest):
+    """The launcher's own parts where pairs bound them (parts of one, two and three rounds): ragged contexts down to one key, against the whole form."""
+    cfg = gpu.synth.tiny_config("llama", hidden=8 * hd, num_heads=8, head_dim=hd, num_kv_heads=8, max_seq_len=2048)
+    m = gpu.HipTransformerModel(cfg, gpu.synth.make_weights(cfg, seed=5, scale=0.05), precision="bf16", max_seqs=n, max_batch_tokens=2048)
+    r = np.random.default_rng(n)
+    lens = [longest, 1] + r.integers(2, longest + 1, n - 2).tolist()
+    prompts = [r.integers(0, cfg["vocab_size"], x).tolist() for x in lens]
+    ids, got = list(range(n)), []
+    for form in (0, 1):
+        old = gpu.lib().nvl_set_tuning(25, form)
+        for i in ids:
+            m.seq_reset(i)
+            m.forward_batch([i], [prompts[i]], [0], want_logits=False)
+        got.append([m.forward_batch(ids, [[7 + j]] * n, [x + j for x in lens])[0] for j in range(3)])      # (the tickets are zero again)
+        gpu.lib().nvl_set_tuning(25, old)
+    m.close()
+    for whole, parts in zip(*got):
+        assert rel_err(parts, whole) <= TOL and not np.array_equal(parts, whole)
+
+
 @pytest.mark.parametrize("family,hidden,heads", [("llama", 192, 3), ("llama", 2048, 16), ("falcon", 2112, 33), ("llama", 4096, 32), ("falcon", 4544, 71),
                                                  ("llama", 4608, 36), ("llama", 4672, 73)])       # up to 2048 / 4096 / 4608 columns, and beyond
 @pytest.mark.parametrize("lens", [[513], [1025], [600, 440], [1033]])      # a row per workgroup up to 1024 rows; tiles: remainders of 8 and of 16
