@@ -1261,6 +1261,12 @@ static int g_attn_split = 1;   // nvl_set_tuning key 25: split a decode attentio
 //                                                   400 -0.3 (2 x 4)   600 -1.9 (4 x 3)   900 -4.3 (4 x 4)  1500 -6.6 (4 x 3)     8
 //                                                   600 +0.8 (4 x 2)  1000 -3.0 (4 x 2)  1500 -4.3 (4 x 2), +3.6 (4 x 3)         12
 //                                                  1000 -1.6 (4 x 2), +2.6 (4 x 4)  1500 -3.0 (4 x 2)                            16
+// Ragged contexts leave room for more parts, since a sequence takes them by its own length and the other workgroups of the grid leave at
+// once: more while those with work stay within 208, the whole grid within 640.  "/ 6": contexts down to a sixth of the longest; without -> with:
+//   heads of 64    Granite-3.0-1B 16 of 900 / 6  0.0 -> -1.2 (4 x 2), 12 of 1100 / 6 -0.3 -> -1.6 (4 x 3), Llama-3.2-1B 12 of 1100 / 6 -0.4 -> -1.1,
+//                  14 of 1200 and short ones 0.0 -> -1.3; of 900 / 2  at 227 with work +0.4, so not
+//   heads of 128   12 of 1500 / 6 -3.6 -> -5.7 (4 x 3), 16 of 1100 / 6 -1.0 -> -2.1 (4 x 3), 12 of 1500 and short ones -5 -> -7.6 (4 x 6); 16 of 1500 and
+//                  short ones -6.4 (4 x 3), -1.9 (4 x 6: a grid of 768); 12 of 900 / 6 in four parts (238 with work) +0.4, 16 of 1500 / 6 in three (251) +0.9
 int decode_attn_cfg(const nvl_model* m, int n_seqs) {
     const int n_kt = m->ctx_hint > 0 ? (m->ctx_hint - 1) / 64 + 1 : 1 << 20;
     const int per_wave = m->hd == 64 ? 2 : 1;
@@ -1272,12 +1278,16 @@ int decode_attn_cfg(const nvl_model* m, int n_seqs) {
     const int most = m->attn_part && m->ctx_hint > 0 ? std::min(ATTN_SPLIT_MAX, m->attn_records / wgs) : 1;
     if (g_attn_split >= 2) { const int tiles = (g_attn_split - 1) * nw * per_wave; return cfg(nw, std::max(1, std::min(most, cdiv(n_kt, tiles))), tiles); }
     if (g_attn_split && !g_attn_nw && most > 1) {
+        const double mean_kt = m->kv_tok / (64.0 * n_seqs);
+        // the workgroups with work: a sequence has its tiles / `tiles` parts, rounded up
+        auto room = [&](int tiles) { return (mean_kt / tiles + 0.5) * wgs <= 208; };
         int waves = 0;
-        if (m->hd == 64) waves = wgs <= 32 ? (n_kt > 20 ? 4 : n_kt > 12 ? 2 : 0) : wgs <= 85 ? (n_kt > 14 ? 4 : 0) : wgs <= 128 && n_kt > 20 ? 8 : 0;
+        if (m->hd == 64) waves = wgs <= 32 ? (n_kt > 20 ? 4 : n_kt > 12 ? 2 : 0) : wgs <= 85 ? (n_kt > 14 ? 4 : 0) : wgs > 128 ? 0 : n_kt > 20 ? 8 : n_kt > 14 && room(8) ? 4 : 0;
         else waves = wgs <= 64 ? (n_kt > 10 ? 4 : n_kt > (wgs <= 32 ? 5 : 6) ? 2 : 0) : wgs <= 128 && n_kt > 12 ? 4 : 0;
         if (waves) {
             const int round = waves * per_wave, rounds = cdiv(n_kt, round);
-            const int each = cdiv(rounds, std::max(1, std::min(most, 256 / wgs)));      // rounds of a part
+            int each = cdiv(rounds, std::max(1, std::min(most, 256 / wgs)));      // rounds of a part
+            while (each > 1 && cdiv(rounds, each - 1) <= std::min(most, 640 / wgs) && room((each - 1) * round)) each--;
             if (each < rounds) return cfg(waves, cdiv(rounds, each), each * round);
         }
     }

@@ -293,7 +293,8 @@ def test_decode_attention_in_parts(gpu, hd, kv, waves, rounds):
     assert rel_err(got[1], got[0]) <= TOL
 
 
-@pytest.mark.parametrize("hd,n,longest", [(64, 10, 1900), (64, 12, 1500), (64, 16, 1300), (128, 8, 1500), (128, 12, 1500), (128, 16, 800)])
+@pytest.mark.parametrize("hd,n,longest", [(64, 10, 1900), (64, 12, 1500), (64, 16, 1300), (64, 16, 1000), (128, 8, 1500), (128, 12, 1500), (128, 16, 800),
+                                             (128, 16, 1100)])
 def test_decode_attention_parts_by_pairs(gpu, hd, n, longest):
     """The launcher's own parts where pairs bound them (parts of one, two and three rounds): ragged contexts down to one key, against the whole form."""
     cfg = gpu.synth.tiny_config("llama", hidden=8 * hd, num_heads=8, head_dim=hd, num_kv_heads=8, max_seq_len=2048)
