@@ -1249,7 +1249,7 @@ static int g_attn_split = 1;   // nvl_set_tuning key 25: split a decode attentio
 // leave a CU to each workgroup (256 / pairs), and as many as give each the same number of rounds: beyond 128 pairs a split only
 // adds traffic.  The lines lie where whole decode steps change sides (a launch by itself favours the split earlier: it does not wait for the
 // kernel before it).  Steps against the whole form, per cent (waves x parts; forms in random order, runs differ by 0.5):
-//   heads of 64, Llama-3.2-1B, 8 kv heads     keys  520 +0.8 (2 x 3)   700 -1.6 (2 x 3)  1000 -4.6 (2 x 4)  1500 -8.7 (4 x 3)     1 sequence
+//   heads of 64, Llama-3.2-1B, 8 kv heads     keys  560 +1.2 (2 x 3)   640..760 -0.3 (2 x 3, Granite -0.7)  1000 -4.6 (2 x 4)  1500 -8.7 (4 x 3)     1 sequence
 //                                                   600 +0.8 (2 x 3)   800 -0.6 (2 x 4)  1200 -1.6 (4 x 3)  1800 -7.4 (4 x 4)     4
 //                                                   700 +0.6 (2 x 3)  1000 -0.6 (4 x 2)  1500 -6.9 (4 x 3)                        6
 //                                                   700 +0.5 (2 x 3)  1000 -1.4 (4 x 2)  1400 -4.5 (4 x 3)  1900 -3.4 (4 x 4)     8
@@ -1282,7 +1282,7 @@ int decode_attn_cfg(const nvl_model* m, int n_seqs) {
         // the workgroups with work: a sequence has its tiles / `tiles` parts, rounded up
         auto room = [&](int tiles) { return (mean_kt / tiles + 0.5) * wgs <= 208; };
         int waves = 0;
-        if (m->hd == 64) waves = wgs <= 32 ? (n_kt > 20 ? 4 : n_kt > 12 ? 2 : 0) : wgs <= 85 ? (n_kt > 14 ? 4 : 0) : wgs > 128 ? 0 : n_kt > 20 ? 8 : n_kt > 14 && room(8) ? 4 : 0;
+        if (m->hd == 64) waves = wgs <= 32 ? (n_kt > 20 ? 4 : n_kt > (wgs <= 8 ? 10 : 12) ? 2 : 0) : wgs <= 85 ? (n_kt > 14 ? 4 : 0) : wgs > 128 ? 0 : n_kt > 20 ? 8 : n_kt > 14 && room(8) ? 4 : 0;
         else waves = wgs <= 64 ? (n_kt > 10 ? 4 : n_kt > (wgs <= 32 ? 5 : 6) ? 2 : 0) : wgs <= 128 && n_kt > 12 ? 4 : 0;
         if (waves) {
             const int round = waves * per_wave, rounds = cdiv(n_kt, round);
