@@ -824,7 +824,11 @@ __device__ __forceinline__ void epilogue_qkv_pair(const GemmArgs& p, int m, int 
     *(bf16x4*)(dst + half) = o2;
 }
 
-template <int MT, int CT, int EPI, typename OutT>
+// STREAM: a launch of a single row group, which reads each weight once.  The weights then go past what the caches hold: states, keys and values of the
+// next launches stay there (without nt a delta-rule scan behind an input projection at 20 rows 31.5 -> 36.0 us, a lightning scan at 32 29.9 -> 34.4),
+// and the ring is faster itself (4544 x 18176 at 16 rows 32.5 -> 29.8 us, 4096 x 14336 at 32 26.4 -> 24.9).  Its own instance: as a run-time branch
+// around the loads it cost launches of several groups 3 to 11 % (Falcon-7B at 200 rows, its products together, 5.4 -> 5.8 ms)
+template <int MT, int CT, int EPI, typename OutT, bool STREAM>
 __global__ __launch_bounds__(512, 1) void gemm_mid_bf16_kernel(GemmArgs p) {
     constexpr int NST = mid_stages<MT, CT>(), SB = mid_stage_bytes<MT, CT>(), NA = 4 * MT, PW = (MT + 2 * CT) / 2, TM = MT / 2;
     static_assert(MT % 2 == 0 && NST >= 3 && PW * (NST - 2) < 64, "two waves share the rows; vmcnt counts to 63");
@@ -840,10 +844,6 @@ __global__ __launch_bounds__(512, 1) void gemm_mid_bf16_kernel(GemmArgs p) {
     const int k0 = (int)((int64_t)part * stages / p.splits), n = (int)((int64_t)(part + 1) * stages / p.splits) - k0;
     const bool ragged = (p.K & 64) && k0 + n == stages;          // K % 128 == 64: the last stage has its first half only
 
-    // Weights that a single row group reads once go past what the caches hold: states, keys and values of the next launches stay there (without nt a
-    // delta-rule scan behind an input projection at 20 rows 31.5 -> 36.0 us, a lightning scan at 32 29.9 -> 34.4), and the ring is
-    // faster itself (4544 x 18176 at 16 rows 32.5 -> 29.8 us, 4096 x 14336 at 32 26.4 -> 24.9)
-    const bool stream = groups == 1;
     // 1-KiB blocks (row tile, k-step) of a stage, PW for each wave: rows first, then columns
     const bf16_t* src[PW];
 #pragma unroll
@@ -864,7 +864,7 @@ __global__ __launch_bounds__(512, 1) void gemm_mid_bf16_kernel(GemmArgs p) {
             if (cut && ((wave8 * PW + i) & 2)) continue;        // (k-steps 2 and 3; waited for with vmcnt(0))
             const auto from = (const __attribute__((address_space(1))) void*)(src[i] + (int64_t)s * 2048);
             const auto to = (__attribute__((address_space(3))) void*)(base + i * 1024);
-            if (stream && wave8 * PW + i >= NA) __builtin_amdgcn_global_load_lds(from, to, 16, 0, LOAD_NT);
+            if (STREAM && wave8 * PW + i >= NA) __builtin_amdgcn_global_load_lds(from, to, 16, 0, LOAD_NT);
             else __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
         }
     };
@@ -1852,8 +1852,13 @@ static inline void launch_gemm_mid_rows(hipStream_t st, const GemmArgs& a0) {
     mid_cost(a.M, a.N, a.K, MT, CT, a.split_units > 0, a.splits);
     if (a.split_units > 0 && g_mid_splits) a.splits = std::min(g_mid_splits, std::max(1, a.K >> 7));
     while (a.splits > 1 && (nb * groups > SPLIT_MAX_TILES || (int64_t)nb * groups * a.splits * MT * CT * 2048 > a.split_units * SPLIT_UNIT)) a.splits--;
-    NVL_LDS_ATTR((gemm_mid_bf16_kernel<MT, CT, EPI, OutT>), (mid_lds_bytes<MT, CT>()));
-    hipLaunchKernelGGL((gemm_mid_bf16_kernel<MT, CT, EPI, OutT>), dim3(cdiv(nb, 8) * 8 * groups * a.splits), dim3(512), (mid_lds_bytes<MT, CT>()), st, a);
+    auto launch = [&](auto stream) {
+        NVL_LDS_ATTR((gemm_mid_bf16_kernel<MT, CT, EPI, OutT, decltype(stream)::value>), (mid_lds_bytes<MT, CT>()));
+        hipLaunchKernelGGL((gemm_mid_bf16_kernel<MT, CT, EPI, OutT, decltype(stream)::value>), dim3(cdiv(nb, 8) * 8 * groups * a.splits), dim3(512), (mid_lds_bytes<MT, CT>()), st, a);
+    };
+    if (groups == 1) launch(std::true_type{});
+    else if constexpr (MT > 4 || CT > 2) launch(std::false_type{});      // (narrower tiles hold all rows: mid_row_tiles)
+    else throw std::runtime_error("gemm_mid: several groups of few rows");
 }
 // does the kernel take this projection, and is it the one to take it?
 template <int EPI, typename OutT>
