@@ -824,10 +824,11 @@ __device__ __forceinline__ void epilogue_qkv_pair(const GemmArgs& p, int m, int 
     *(bf16x4*)(dst + half) = o2;
 }
 
-// STREAM: a launch of a single row group, which reads each weight once.  The weights then go past what the caches hold: states, keys and values of the
+// STREAM: a launch of a single row group of up to 96 rows, which reads each weight once.  The weights then go past what the caches hold: states, keys and values of the
 // next launches stay there (without nt a delta-rule scan behind an input projection at 20 rows 31.5 -> 36.0 us, a lightning scan at 32 29.9 -> 34.4),
 // and the ring is faster itself (4544 x 18176 at 16 rows 32.5 -> 29.8 us, 4096 x 14336 at 32 26.4 -> 24.9).  Its own instance: as a run-time branch
-// around the loads it cost launches of several groups 3 to 11 % (Falcon-7B at 200 rows, its products together, 5.4 -> 5.8 ms)
+// around the loads it cost launches of several groups 3 to 11 % (Falcon-7B at 200 rows, its products together, 5.4 -> 5.8 ms).
+// Groups of 128 rows gain nothing by it (Falcon-7B, a decode step of 104 sequences 5.61 -> 5.71 ms, a 2048-wide model with a delta rule at 97 1.73 -> 1.75)
 template <int MT, int CT, int EPI, typename OutT, bool STREAM>
 __global__ __launch_bounds__(512, 1) void gemm_mid_bf16_kernel(GemmArgs p) {
     constexpr int NST = mid_stages<MT, CT>(), SB = mid_stage_bytes<MT, CT>(), NA = 4 * MT, PW = (MT + 2 * CT) / 2, TM = MT / 2;
@@ -1856,9 +1857,9 @@ static inline void launch_gemm_mid_rows(hipStream_t st, const GemmArgs& a0) {
         NVL_LDS_ATTR((gemm_mid_bf16_kernel<MT, CT, EPI, OutT, decltype(stream)::value>), (mid_lds_bytes<MT, CT>()));
         hipLaunchKernelGGL((gemm_mid_bf16_kernel<MT, CT, EPI, OutT, decltype(stream)::value>), dim3(cdiv(nb, 8) * 8 * groups * a.splits), dim3(512), (mid_lds_bytes<MT, CT>()), st, a);
     };
-    if (groups == 1) launch(std::true_type{});
-    else if constexpr (MT > 4 || CT > 2) launch(std::false_type{});      // (narrower tiles hold all rows: mid_row_tiles)
-    else throw std::runtime_error("gemm_mid: several groups of few rows");
+    if constexpr (MT < 8) if (groups == 1) { launch(std::true_type{}); return; }
+    if constexpr (MT > 4 || CT > 2) launch(std::false_type{});
+    else throw std::runtime_error("gemm_mid: several groups of few rows");      // (narrower tiles hold all rows: mid_row_tiles)
 }
 // does the kernel take this projection, and is it the one to take it?
 template <int EPI, typename OutT>

@@ -265,7 +265,7 @@ struct nvl_model {
     nvl_stats stats{};
     nvl::SiteStat site_stats[2][nvl::KS_COUNT];     // [phase: 0 prefill, 1 decode][site], filled when profiling
     int site = 0, phase = 0;     // set by the forward pass just before a launch (consumed by KScope)
-    double kv_tok = 0;           // cached + new keys of the batch being enqueued (attention's algorithmic KV bytes)
+    double kv_tok = 0;           // cached + new keys of the batch being enqueued (attention's algorithmic KV bytes; with ctx_hint the parts of a decode attention)
     double site_bytes = 0;       // algorithmic bytes of the next launch (0 = let the helper compute them)
     bool profile = false;
     std::vector<nvl::ProfRec> prof;
