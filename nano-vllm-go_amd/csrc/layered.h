@@ -803,6 +803,7 @@ void layered_finalize(nvl_model* m) {
     }
     m->logit_rows = S;
     m->logits = dmalloc<float>(S * (int64_t)m->Vpad);
+    init_readback(m);
     m->argmax_dev = dmalloc<int32_t>(std::max<int64_t>(S, Mmax));
     m->argmax_pval = dmalloc<float>(std::max<int64_t>(S, Mmax) * cdiv(m->V, ARGMAX_CHUNK));
     m->argmax_pidx = dmalloc<int32_t>(std::max<int64_t>(S, Mmax) * cdiv(m->V, ARGMAX_CHUNK));

@@ -253,7 +253,8 @@ struct nvl_model {
     std::set<std::array<int, 5>> graph_seen;
     std::vector<hipGraphExec_t> graphs_retired;       // evicted execs, destroyed after the next stream sync (reap_graphs)
     bool graphs_ok = true;
-    int32_t* am_host = nullptr;                       // pinned: argmax ids of a replayed decode pass
+    int32_t* am_host = nullptr;                       // pinned: argmax ids of a pass
+    char* rb_host = nullptr; int64_t rb_bytes = 0; int rb_slots = 0; std::vector<hipEvent_t> rb_ev;      // pinned: pieces of the logits on their way to the caller (readback.h)
     // debug
     // nvl_set_debug mode 4: in-kernel time stamps of the decode kernels (common.h nvl_stamp), one record per launch
     bool stamping = false; unsigned long long* stamp_buf = nullptr; int stamp_launches = 0;

@@ -16,6 +16,8 @@
 
 using namespace nvl;
 
+#include "readback.h"
+
 static thread_local std::string g_create_err;
 constexpr int ATTN_SPLIT_PAIRS = 128;         // split decode attention: most (sequence, kv head, query tile) triples of a launch, unless forced
 constexpr int SK_TILE_MAX_M = 2048, SK_TILE_MAX_SLICES = 8;      // split-K of the tile kernel for mid-size residual projections (resid_gemm)
@@ -382,6 +384,7 @@ extern "C" void nvl_destroy(nvl_model* m) {
     dfree(m->moe_gate); dfree(m->moe_hall); dfree(m->moe_part);
     clear_graphs(m);
     if (m->am_host) (void)hipHostFree(m->am_host);
+    free_readback(m);
     dfree(m->ring_pos0);
     dfree(m->conv_tail); dfree(m->stamp_buf); dfree(m->ssd_z); dfree(m->ssd_decay);
     dfree(m->ssm_state); dfree(m->mproj); dfree(m->mxbc); dfree(m->mdelta); dfree(m->mrs); dfree(m->my); dfree(m->myn);
@@ -863,6 +866,7 @@ extern "C" int nvl_finalize(nvl_model* m) {
     NVL_HIP(hipMemsetAsync(m->xn_last, 0, (size_t)(round_up(S, 64) * H) * m->wsize, m->stream));
     m->logit_rows = S;
     m->logits = dmalloc<float>(S * (int64_t)m->Vpad);
+    init_readback(m);
     m->argmax_dev = dmalloc<int32_t>(std::max<int64_t>(S, Mmax));
     m->argmax_pval = dmalloc<float>(std::max<int64_t>(S, Mmax) * cdiv(m->V, ARGMAX_CHUNK));
     m->argmax_pidx = dmalloc<int32_t>(std::max<int64_t>(S, Mmax) * cdiv(m->V, ARGMAX_CHUNK));
@@ -2237,8 +2241,7 @@ int forward_impl(nvl_model* m, int n_seqs, const int64_t* seq_ids, const int32_t
     int rows = all ? M : (custom ? n_rows : n_seqs);
     struct Named { nvl_model* m; ~Named() { m->rows_named = -1; } } named{m};
     m->rows_named = custom ? n_rows : -1;
-    std::vector<int32_t> am;
-    const int32_t* am_p = nullptr;
+    const int32_t* am_p = m->am_host;
     bool replayed = false;
     if (!prefill && rows <= m->logit_rows && !custom && !m->meta_dynamic) {
         // a decode pass (what TensorModelRunner.Run issues every step): metadata upload + all launches + the argmax
@@ -2249,19 +2252,15 @@ int forward_impl(nvl_model* m, int n_seqs, const int64_t* seq_ids, const int32_t
             enqueue_forward(m, md, n_seqs, M, max_len, attn_flops, flags);
             NVL_HIP(hipMemcpyAsync(m->am_host, m->argmax_dev, (size_t)rows * 4, hipMemcpyDeviceToHost, m->stream));
         });
-        if (replayed) { am_p = m->am_host; m->ctx_hint = 0; }
+        if (replayed) m->ctx_hint = 0;
     }
     if (!replayed) {
         NVL_HIP(hipMemcpyAsync(m->meta_dev, m->meta_host, meta_bytes(m, M), hipMemcpyHostToDevice, m->stream));
         rows = enqueue_forward(m, md, n_seqs, M, max_len, attn_flops, flags);
-        am.resize((size_t)rows);
-        if (rows) NVL_HIP(hipMemcpyAsync(am.data(), m->argmax_dev, (size_t)rows * 4, hipMemcpyDeviceToHost, m->stream));
-        am_p = am.data();
+        if (rows) NVL_HIP(hipMemcpyAsync(m->am_host, m->argmax_dev, (size_t)rows * 4, hipMemcpyDeviceToHost, m->stream));
     }
     NVL_HIP(hipEventRecord(m->ev1, m->stream));
-    if (logits_out && rows)
-        NVL_HIP(hipMemcpy2DAsync(logits_out, (size_t)m->V * 4, m->logits, (size_t)m->Vpad * 4, (size_t)m->V * 4,
-                                 (size_t)rows, hipMemcpyDeviceToHost, m->stream));
+    if (logits_out && rows) read_logits(m, logits_out, rows);
     NVL_HIP(hipStreamSynchronize(m->stream));
     reap_graphs(m);
     p2p_check(m);
@@ -2359,11 +2358,9 @@ extern "C" int nvl_forward_paged(nvl_model* m, int n_seqs, const int32_t* tokens
     const bool all = (flags & NVL_FWD_ALL_LOGITS) != 0;
     const int rows = enqueue_forward(m, md, n_seqs, M, max_len, attn_flops, flags);
     NVL_HIP(hipEventRecord(m->ev1, m->stream));
-    std::vector<int32_t> am((size_t)rows);
-    NVL_HIP(hipMemcpyAsync(am.data(), m->argmax_dev, (size_t)rows * 4, hipMemcpyDeviceToHost, m->stream));
-    if (logits_out)
-        NVL_HIP(hipMemcpy2DAsync(logits_out, (size_t)m->V * 4, m->logits, (size_t)m->Vpad * 4, (size_t)m->V * 4,
-                                 (size_t)rows, hipMemcpyDeviceToHost, m->stream));
+    const int32_t* am = m->am_host;
+    NVL_HIP(hipMemcpyAsync(m->am_host, m->argmax_dev, (size_t)rows * 4, hipMemcpyDeviceToHost, m->stream));
+    if (logits_out) read_logits(m, logits_out, rows);
     NVL_HIP(hipStreamSynchronize(m->stream));
     if (argmax_out) {
         if (all) for (int i = 0; i < n_seqs; i++) argmax_out[i] = am[(size_t)hm.last_rows[i]];
