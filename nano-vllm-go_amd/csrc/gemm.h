@@ -205,6 +205,11 @@ __device__ __forceinline__ void epilogue_grouped_raw4(const GemmArgs& p, int64_t
 }
 
 __device__ __forceinline__ float silu_f(float g) { return g / (1.0f + __expf(-g)); }
+// ... rounded to bf16 right away: the hardware's reciprocal in place of the division, whose ten instructions for each of a lane's 64 values were 28 of 828 us
+// (16384 x 16384 x 2048, all CUs in their epilogues at once; 4176 x 28672 x 4096 743 -> 730).  Error of the bf16 product silu(g) u against 64 bits: the
+// same to seven digits for |g| <= 0.01 .. 80 (1.64e-3 .. 1.66e-3 in the 2-norm); 4 results of a million round the other way.
+// exp2 -> inf gives 0 and -inf NaN, as the division does
+__device__ __forceinline__ float silu_bf16_f(float g) { return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * g)); }
 __device__ __forceinline__ float deferred_rstd(const GemmArgs& p, int m);
 
 // ------------------------------------------------------------------------------------------
@@ -294,7 +299,7 @@ __device__ __forceinline__ void epilogue_glu4(const GemmArgs& p, int m, int f, f
     for (int r = 0; r < 4; r++) {
         if constexpr (EPI == EPI_CLAMP_GLU) v[r] = clamp_glu_f(g[r], u[r], MOE && f >= p.glu_from2 ? p.glu_limit2 : p.glu_limit, p.glu_slope);
         else if constexpr (EPI == EPI_REGLU) v[r] = fmaxf(g[r], 0.f) * u[r];
-        else v[r] = (EPI == EPI_GEGLU ? gelu_tanh_f(g[r]) : silu_f(g[r])) * u[r];
+        else v[r] = (EPI == EPI_GEGLU ? gelu_tanh_f(g[r]) : sizeof(OutT) == 2 ? silu_bf16_f(g[r]) : silu_f(g[r])) * u[r];
     }
     if constexpr (MOE) v *= p.moe_gate[m * p.moe_E + f / p.moe_I];      // routing weight of (token, expert); 0 = not routed
     act_store4<OutT>((OutT*)p.C, (int64_t)p.c_row0 + m, f, p.ldc, v);
