@@ -79,6 +79,15 @@ struct GroupedEpi {         // EPI_GROUPED: columns [q | k | v | gate | feed-for
     float* raw; int64_t raw_ld; int raw0, silu1;
 };
 
+// MoE decode, experts' up projection: routing by the launch's first `wgs` workgroups (set by the launcher), `rows` rows each
+struct RouteJob {
+    const bf16_t* W;        // router, fragment-major [E][K], or NULL: no routing in this launch
+    const float* bias;      // [E] or NULL
+    float *gate, *logits;   // [rows][gate_ld]; logits [rows][logits_ld] or NULL
+    int E, top_k, gate_ld, logits_ld, n_always;      // columns E .. E + n_always - 1 of the gate are one (experts every token takes), those up to gate_ld zero
+    int wgs, rows;
+};
+
 struct GemmArgs {
     const void* A;          // bf16: fragment-major [M_pad16][K]; f32: row-major [M][lda]
     int lda;
@@ -104,7 +113,10 @@ struct GemmArgs {
     int x_mask;             // decode kernels: rows >= M of a 16-row activation tile are not fetched (set when M % 16 != 0)
     int grp_bm;             // rows per m-tile of the grouped launch (128, or 256: the 256x128 three-stage instance)
     int grp_deep;           // grouped launch on the four-stage 128x128 instance (decode-sized MoE batches)
-    QkvEpi qkv;             // EPI_QKV
+    union {
+        QkvEpi qkv;         // EPI_QKV
+        RouteJob route;     // masked experts (epi_moe with moe_gate)
+    };
     GroupedEpi grp;         // EPI_GROUPED
     // decode kernel, EPI_RESID only: K split over gridDim.y = sk_slices workgroups per column block.  Each
     // writes its fp32 partial tile to sk_part[slice][m][n] (ld = N) with plain stores; the NEXT kernel in the
@@ -141,16 +153,17 @@ struct GemmArgs {
     //   down W = [H][E * I] (the experts concatenated along K), a wave's K range lies inside ONE expert.
     // moe_gate [M][E] holds the renormalised routing weight of (token, expert), 0 when the token did not pick the expert.
     // A workgroup (up) / wave (down) whose expert no token of the batch picked returns before it loads a weight byte, so
-    // only the touched experts are streamed; the up epilogue multiplies row m by moe_gate[m][e], which makes the down
-    // projection's K reduction the weighted combine itself (moe.go:105-120) — no sort, no plan, no combine launch.
+    // only the touched experts are streamed; the down projection's waves multiply their sums, one expert each, by moe_gate[m][e],
+    // which makes its K reduction the weighted combine itself (moe.go:105-120) — no sort, no plan, no combine launch.
+    // Where a batch is expected to pick nearly all experts the up projection streams them all and needs no routing: its first
+    // workgroups then do the routing (route) beside it.
     const float* moe_gate;
     int moe_E, moe_I;
 };
-// does any row of the batch (M <= 64: one per lane) route to expert e?  Call with all 64 lanes active.
-__device__ __forceinline__ bool moe_expert_live(const GemmArgs& p, int e) {
+// the routing weight that row `lane` of the batch (M <= 64) gives expert e
+__device__ __forceinline__ float moe_gate_of(const GemmArgs& p, int e) {
     const int lane = threadIdx.x & 63;
-    const float g = lane < p.M ? p.moe_gate[lane * p.moe_E + e] : 0.f;
-    return __any(g != 0.f);
+    return lane < p.M ? p.moe_gate[lane * p.moe_E + e] : 0.f;
 }
 
 // four columns n .. n + 3 of token `row`, inside one column range
@@ -301,7 +314,6 @@ __device__ __forceinline__ void epilogue_glu4(const GemmArgs& p, int m, int f, f
         else if constexpr (EPI == EPI_REGLU) v[r] = fmaxf(g[r], 0.f) * u[r];
         else v[r] = (EPI == EPI_GEGLU ? gelu_tanh_f(g[r]) : sizeof(OutT) == 2 ? silu_bf16_f(g[r]) : silu_f(g[r])) * u[r];
     }
-    if constexpr (MOE) v *= p.moe_gate[m * p.moe_E + f / p.moe_I];      // routing weight of (token, expert); 0 = not routed
     act_store4<OutT>((OutT*)p.C, (int64_t)p.c_row0 + m, f, p.ldc, v);
 }
 
@@ -1002,6 +1014,127 @@ __device__ __forceinline__ bf16x8 weight_load(const bf16x8* p) {
     else return __builtin_nontemporal_load(p);
 }
 
+// ------------------------------------------------------------------------------------------
+// MoE routing (moe.go:57-103) of rows first .. first + n - 1 of a 16-row activation tile by a workgroup of `waves` waves: router logits of the tile (E <= 64
+// experts, all of K), softmax, top-k, renormalised weights as the dense gate matrix GemmArgs::moe_gate of the expert projections, or the
+// chosen experts in rank order (RouteIds).  A wave takes an expert tile over a K slice (fragments straight from L2 / HBM, as
+// the skinny kernel; with fewer waves than tiles, several tiles over all of K), the K slices are summed through LDS in order, then a wave
+// routes a row with a lane per expert.  U k-steps of T expert tiles travel together: few waves need more of them (a lone wave, K = 1024, 32 experts: 4 round
+// trips instead of 16; decode steps of 20 rows of 1024 +6 % without).
+// p: A (fragment-major operand, possibly the deferred-norm raw form with rs_in), M, K.  smem: max(waves, 4) + 4 KiB
+// ------------------------------------------------------------------------------------------
+struct RouteIds { int32_t* ids; float* w; };      // [row][top_k], or NULL
+template <int U, int T>
+__device__ __forceinline__ void moe_route_rows(const GemmArgs& p, const RouteJob& r, RouteIds out, int tile16, int first, int n, int waves, char* smem) {
+    f32x4* red = (f32x4*)smem;                                   // [waves or expert tiles][64]
+    const int E = r.E, ET = (E + 15) >> 4, KW = waves >= ET ? waves / ET : 1;         // expert tiles (1 .. 4), K slices
+    float* lg = (float*)(smem + (waves > 4 ? waves : 4) * 1024);     // [16][64]
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int fr = lane & 15, fg = lane >> 4;
+    const int row0 = tile16 * 16;
+    const int nks = p.K >> 5, q = nks / KW, rr = nks - q * KW;
+    const bool x_live = row0 + fr < p.M;
+    const bf16x8 zero = {};
+    const int TS = (ET + T - 1) / T;          // groups of T tiles, which share a row fragment
+    for (int it = wave; it < TS * KW; it += waves) {
+        const int t0 = it % TS * T, kw = it / TS;
+        const int my_steps = q + (kw < rr ? 1 : 0), ks0 = kw * q + (kw < rr ? kw : rr);
+        const bf16_t* wp[T];
+#pragma unroll
+        for (int t = 0; t < T; t++) wp[t] = r.W + (((int64_t)min(t0 + t, ET - 1) * nks + ks0) * 64 + lane) * 8;
+        const bf16_t* xp = (const bf16_t*)p.A + (((int64_t)tile16 * nks + ks0) * 64 + lane) * 8;
+        f32x4 acc[T];
+#pragma unroll
+        for (int t = 0; t < T; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        int s = 0;
+        for (; s + U <= my_steps; s += U) {
+            bf16x8 w[T][U], x[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+#pragma unroll
+                for (int t = 0; t < T; t++) w[t][u] = *(const bf16x8*)(wp[t] + (int64_t)(s + u) * 512);
+                x[u] = x_live ? *(const bf16x8*)(xp + (int64_t)(s + u) * 512) : zero;
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int t = 0; t < T; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t][u], x[u], acc[t], 0, 0, 0);
+        }
+        for (; s < my_steps; s++) {
+            const bf16x8 x = x_live ? *(const bf16x8*)(xp + (int64_t)s * 512) : zero;
+#pragma unroll
+            for (int t = 0; t < T; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(wp[t] + (int64_t)s * 512), x, acc[t], 0, 0, 0);
+        }
+#pragma unroll
+        for (int t = 0; t < T; t++)
+            if (t0 + t < ET) red[(kw * ET + t0 + t) * 64 + lane] = acc[t];
+    }
+    // deferred RMSNorm: the x^2 partials of a row, a lane per 16-byte chunk
+    auto sum_squares = [&](int m) {
+        const f32x4* src = (const f32x4*)(p.rs_in + (int64_t)m * p.rs_tiles);
+        f32x4 a4 = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int c = lane; c < (p.rs_tiles >> 2); c += 64) a4 += src[c];
+        float t = (a4[0] + a4[1]) + (a4[2] + a4[3]);
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) t += __shfl_xor(t, o, 64);
+        return t;
+    };
+    const int end = min(n, min(16, p.M - row0) - first);          // rows of this workgroup
+    float ssq = p.rs_in && wave < end ? sum_squares(row0 + first + wave) : 0.f;
+    __syncthreads();
+    for (int t = wave; t < ET; t += waves) {        // acc of lane (fr, fg): row fr, experts 16 t + 4 fg .. + 3
+        f32x4 v = red[t * 64 + lane];
+        for (int k = 1; k < KW; k++) v += red[(k * ET + t) * 64 + lane];
+        *(f32x4*)(lg + fr * 64 + 16 * t + 4 * fg) = v;
+    }
+    __syncthreads();
+    for (int i = wave; i < end; i += waves) {
+        const int row = first + i, m = row0 + row;
+        if (p.rs_in && i != wave) ssq = sum_squares(m);
+        const float rstd = p.rs_in ? 1.0f / sqrtf(ssq * p.rs_inv_h + p.rs_eps) : 1.0f;
+        const float v = (lane < E) ? lg[row * 64 + lane] * rstd + (r.bias ? r.bias[lane] : 0.f) : -INFINITY;
+        if (r.logits && lane < E) r.logits[(int64_t)m * r.logits_ld + lane] = v;
+        float mx = v;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+        const float e = (lane < E) ? expf(v - mx) : 0.f;
+        float sum = e;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) sum += __shfl_xor(sum, o, 64);
+        const float prob = (lane < E) ? e / sum : -1.f;
+        int rank = 0;                                   // larger first, ties to the lower index (moe.go:75-92)
+        const int pbits = __builtin_bit_cast(int, prob), key = score_key(prob);
+#pragma unroll 8
+        for (int j = 0; j < E; j++) {                   // (lanes >= E hold -1: they never outrank an expert)
+            const int kj = __builtin_amdgcn_readlane(key, j);
+            rank += (kj > key || (kj == key && j < lane)) ? 1 : 0;
+        }
+        float wsum = 0.f;
+        for (int k = 0; k < r.top_k; k++) {             // moe.go:89-92: fp32 sum in rank order
+            const int src = __ffsll((unsigned long long)__ballot(rank == k)) - 1;
+            wsum += __builtin_bit_cast(float, __builtin_amdgcn_readlane(pbits, src));
+        }
+        if (out.ids) {
+            if (lane < E && rank < r.top_k) { out.ids[(int64_t)m * r.top_k + rank] = lane; out.w[(int64_t)m * r.top_k + rank] = prob / wsum; }
+            continue;
+        }
+        if (lane < E) r.gate[(int64_t)m * r.gate_ld + lane] = rank < r.top_k ? prob / wsum : 0.f;      // moe.go:103
+        for (int e2 = E + lane; e2 < r.gate_ld; e2 += 64) r.gate[(int64_t)m * r.gate_ld + e2] = e2 < E + r.n_always ? 1.0f : 0.f;
+    }
+}
+// workgroup `id` of the RouteJob of a launch
+template <int U, int T>
+__device__ __forceinline__ void moe_route_part(const GemmArgs& p, int id, int waves, char* smem) {
+    const int per_tile = cdiv_dev(p.M < 16 ? p.M : 16, p.route.rows), t = id / per_tile;
+    moe_route_rows<U, T>(p, p.route, RouteIds{nullptr, nullptr}, t, (id - t * per_tile) * p.route.rows, p.route.rows, waves, smem);
+}
+static inline size_t moe_route_lds(int waves) { return (size_t)((waves > 4 ? waves : 4) + 4) * 1024; }
+// ... set up for a launch with workgroups of `waves` waves
+static inline void moe_route_share(GemmArgs& a, int waves) {
+    a.route.rows = waves >= 8 ? 8 : waves >= 4 ? 4 : 2;
+    a.route.wgs = cdiv(a.M, 16) * cdiv(a.M < 16 ? a.M : 16, a.route.rows);
+}
+
 // split_finish for one 16 x 16 tile held by one wave (a lane: four columns of a row): its parts are 1 KiB each, [part][tiles] in sk_part.
 __device__ __forceinline__ bool split_finish_wave(const GemmArgs& p, int tile, int tiles, int part, int parts, f32x4& v) {
     const int lane = threadIdx.x & 63, voff = lane * 16;
@@ -1072,9 +1205,10 @@ __device__ __forceinline__ void skinny_pass_remap(GemmArgs& p, int& bx) {
 // EXTRA: a residual projection whose input rows carry a deferred scale of their own (rs_in; SCALED), or with MOE one that completes its K slices
 // (rs_out; COMPLETES).  Instances of their own: beside it the others lose 1 %, and the experts' slices 16 % at 40 rows (4096 x 32 x 448:
 // 43.9 -> 51 us, their registers spill).
-template <int MT, int NTW, int U, int EPI, typename OutT, bool PASSES = false, bool MOE = false, bool HALF = false, bool EXTRA = false>
+// MOE: 1 masked experts, 2 (up) all experts, the launch's first workgroups route.
+template <int MT, int NTW, int U, int EPI, typename OutT, bool PASSES = false, int MOE = 0, bool HALF = false, bool EXTRA = false>
 __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
-    constexpr bool SCALED = EXTRA && !MOE, COMPLETES = EXTRA && MOE;
+    constexpr bool SCALED = EXTRA && MOE == 0, COMPLETES = EXTRA && MOE != 0;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     f32x4* red = (f32x4*)smem;                       // [NTW][ksplit][MT][64]
     const int swg = blockIdx.y * gridDim.x + blockIdx.x;
@@ -1088,6 +1222,10 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
                                                         // single-group kernels a few scratch dwords otherwise)
     const int half = HALF ? (bx & 1) : 0;
     if constexpr (HALF) bx >>= 1;
+    if constexpr (MOE == 2) {
+        if (bx < p.route.wgs) { moe_route_part<4, 1>(p, bx, blockDim.x >> 6, smem); return; }
+        bx -= p.route.wgs;
+    }
     const bool w_live = !HALF || (fr >> 3) == half;  // HALF: this lane's weight row belongs to the workgroup
     const int nt0 = bx * NTW;                        // first 16-row weight tile of this workgroup
     // K/32 k-steps dealt over (gridDim.y slices) x (ksplit waves) as evenly as possible (K need not divide:
@@ -1112,9 +1250,14 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
     const int ks0 = part * q + (part < rr ? part : rr);   // first k-step of this wave
     // MoE decode (its own instantiation): stream only the experts some token of the batch picked.  Up: a workgroup's rows belong to one
     // expert.  Down: a wave's K range is exactly one expert (launch_gemm_skinny_ntw), of any width; without a token it has nothing to stream.
-    if constexpr (MOE) {
-        if (epi_moe(EPI)) { if (!moe_expert_live(p, (nt0 * 16) / (2 * p.moe_I))) return; }          // (whole workgroup: uniform)
-        else my_steps = __builtin_amdgcn_readfirstlane(moe_expert_live(p, part) ? my_steps : 0);      // (uniform: scalar loops)
+    // Its rows' routing weights wait in LDS for the sums (in a register they spill others of the instances of several row tiles).
+    float* gates = (float*)(smem + NTW * ksplit * MT * 1024) + wave * 64;
+    if constexpr (MOE != 0) {
+        if (EPI == EPI_RESID) {
+            const float g = moe_gate_of(p, part);
+            gates[lane] = g;
+            my_steps = __builtin_amdgcn_readfirstlane(__any(g != 0.f) ? my_steps : 0);      // (uniform: scalar loops)
+        } else if (MOE == 1 && !__any(moe_gate_of(p, (nt0 * 16) / (2 * p.moe_I)) != 0.f)) return;          // (whole workgroup: uniform)
     }
 
     // EPI_QKV: the workgroup's two tiles are half a head apart (they rotate together)
@@ -1169,7 +1312,7 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
         const int m = 16 * (i + i_off) + fr, n = (nt0 + t) * 16 + 4 * fg;
         if (m < p.M && n < p.N && (!HALF || (fg >> 1) == half)) x_pre = *(const f32x4*)((const float*)p.C + (int64_t)m * p.ldc + n);
     }
-    if constexpr (MOE && EPI == EPI_RESID) {
+    if constexpr (MOE != 0 && EPI == EPI_RESID) {
         for (int b = 0; b < nblk; b += 2) {
             if (b + 1 < nblk) load_blk(wB, xB, b + 1);
             comp_blk(wA, xA);
@@ -1195,6 +1338,12 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
             acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x_live[i] ? *(const bf16x8*)(xp[i] + (int64_t)s * 512) : x_zero, acc[i], 0, 0, 0);
     }
 
+    if constexpr (MOE != 0 && EPI == EPI_RESID)
+#pragma unroll
+        for (int i = 0; i < MT; i++) {
+            const float g = gates[16 * i + fr];
+            acc[i] = g != 0.f ? acc[i] * g : f32x4{0.f, 0.f, 0.f, 0.f};       // (0: not routed, whatever the expert made of the row)
+        }
     // ---- reduce the K slices in wave order ----
 #pragma unroll
     for (int i = 0; i < MT; i++) red[((tile * ksplit + kw) * MT + i) * 64 + lane] = acc[i];
@@ -1209,7 +1358,7 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
     if (epi_glu(EPI)) {
         for (int i = wave; i < MT; i += NTW * ksplit) {
             const int f = (nt0 >> 1) * 16 + 4 * fg;    // NTW == 2: tiles [gate 16 | up 16] of features 8*nt0..
-            epilogue_glu4<EPI, OutT, MOE>(p, 16 * i + fr, f, ksum(0, i), ksum(NTW - 1, i),
+            epilogue_glu4<EPI, OutT, MOE != 0>(p, 16 * i + fr, f, ksum(0, i), ksum(NTW - 1, i),
                                         RSTD_PRE && i == i_pre ? rstd_pre : deferred_rstd(p, 16 * i + fr));
         }
     } else if constexpr (EPI == EPI_QKV) {
@@ -1269,101 +1418,18 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
 
 #ifndef NVL_GEMM_INST
 // ------------------------------------------------------------------------------------------
-// MoE decode routing in ONE launch (moe.go:57-103): router logits of a 16-row activation tile (E <= 64 experts, all of K),
-// softmax, top-k, renormalised weights as the dense gate matrix GemmArgs::moe_gate of the expert projections.  Before:
-// the router as a skinny GEMM launch (4.6 us) + moe_gate_kernel (4.5 us).  grid = 16-row tiles of the batch x ROUTE_ROWS of their rows: the
+// MoE routing as a launch of its own (moe_route_rows): prompts, which need the chosen experts before their rows can be sorted, and decode batches that leave
+// some experts alone.  grid = 16-row tiles of the batch x ROUTE_ROWS of their rows: the
 // logits of a tile are cheap, 96 KiB from L2, and the ranking is serial (at 16 rows all of them in one workgroup 8.4 us, eight 7.2, four 7.0;
-// at 6 rows two workgroups lose 0.3).  1024 threads: wave w takes expert tile w % ET over K slice w / ET (fragments straight from L2 / HBM, as
-// the skinny kernel), the K slices are summed through LDS in wave order, then wave r routes the workgroup's row r with a lane per expert.
-// p: A (fragment-major operand, possibly the deferred-norm raw form with rs_in), W (router, fragment-major), bias, M, N = E, K.
-// The gate's columns E .. E + n_always - 1 are one (experts every token takes), those up to gate_ld zero.
+// at 6 rows two workgroups lose 0.3).
 // ------------------------------------------------------------------------------------------
 constexpr int ROUTE_ROWS = 8;
 static inline dim3 router_gate_grid(int M) { return dim3(cdiv(M, 16), cdiv(M < 16 ? M : 16, ROUTE_ROWS)); }
-// prefill: ids / weights [row][top_k] in rank order instead of the gate matrix, all 16 rows of a tile in a workgroup (enough workgroups without)
-struct RouteOut { float* gate; int32_t* ids; float* w; };
-static __global__ __launch_bounds__(1024) void moe_router_gate_kernel(GemmArgs p, int top_k, RouteOut out, float* __restrict__ logits_out, int ld_logits,
-                                                                      int gate_ld, int n_always) {
-    float* gate = out.gate;
-    __shared__ f32x4 red[16][64];
-    __shared__ float lg[16][64];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int fr = lane & 15, fg = lane >> 4;
-    const int E = p.N, ET = (E + 15) >> 4, KW = 16 / ET;         // expert tiles (1, 2 or 4), K slices
-    const int tile = wave % ET, kw = wave / ET;
-    const int row0 = blockIdx.x * 16;
-    const int nks = p.K >> 5, q = nks / KW, rr = nks - q * KW;
-    const int my_steps = kw < KW ? q + (kw < rr ? 1 : 0) : 0;      // (ET = 3 leaves a wave idle)
-    const int ks0 = kw * q + (kw < rr ? kw : rr);
-    const bf16_t* wp = (const bf16_t*)p.W + (((int64_t)tile * nks + ks0) * 64 + lane) * 8;
-    const bf16_t* xp = (const bf16_t*)p.A + (((int64_t)blockIdx.x * nks + ks0) * 64 + lane) * 8;
-    const bool x_live = row0 + fr < p.M;
-    const bf16x8 zero = {};
-    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-    int s = 0;
-    for (; s + 4 <= my_steps; s += 4) {
-        bf16x8 w[4], x[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            w[u] = *(const bf16x8*)(wp + (int64_t)(s + u) * 512);
-            x[u] = x_live ? *(const bf16x8*)(xp + (int64_t)(s + u) * 512) : zero;
-        }
-#pragma unroll
-        for (int u = 0; u < 4; u++) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u], x[u], acc, 0, 0, 0);
-    }
-    for (; s < my_steps; s++)
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(wp + (int64_t)s * 512), x_live ? *(const bf16x8*)(xp + (int64_t)s * 512) : zero, acc, 0, 0, 0);
-    // deferred RMSNorm: wave r owns the workgroup's row r — its x^2 partials, a lane per 16-byte chunk
-    const int rows = out.ids ? 16 : ROUTE_ROWS, row = blockIdx.y * rows + wave, m = row0 + row;
-    const bool routes = wave < rows && m < p.M;
-    float ssq = 0.f;
-    if (p.rs_in && routes) {
-        const f32x4* src = (const f32x4*)(p.rs_in + (int64_t)m * p.rs_tiles);
-        f32x4 a4 = f32x4{0.f, 0.f, 0.f, 0.f};
-        for (int c = lane; c < (p.rs_tiles >> 2); c += 64) a4 += src[c];
-        ssq = (a4[0] + a4[1]) + (a4[2] + a4[3]);
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) ssq += __shfl_xor(ssq, o, 64);
-    }
-    red[wave][lane] = acc;
-    __syncthreads();
-    if (wave < ET) {        // acc of lane (fr, fg): row fr, experts 16 tile + 4 fg .. + 3
-        f32x4 v = red[wave][lane];
-        for (int k = 1; k < KW; k++) v += red[k * ET + wave][lane];
-#pragma unroll
-        for (int r = 0; r < 4; r++) lg[fr][16 * wave + 4 * fg + r] = v[r];
-    }
-    __syncthreads();
-    if (!routes) return;
-    const float rstd = p.rs_in ? 1.0f / sqrtf(ssq * p.rs_inv_h + p.rs_eps) : 1.0f;
-    const float v = (lane < E) ? lg[row][lane] * rstd + (p.bias ? p.bias[lane] : 0.f) : -INFINITY;
-    if (logits_out && lane < E) logits_out[(int64_t)m * ld_logits + lane] = v;
-    float mx = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-    const float e = (lane < E) ? expf(v - mx) : 0.f;
-    float sum = e;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) sum += __shfl_xor(sum, o, 64);
-    const float prob = (lane < E) ? e / sum : -1.f;
-    int rank = 0;                                   // larger first, ties to the lower index (moe.go:75-92)
-    const int pbits = __builtin_bit_cast(int, prob), key = score_key(prob);
-#pragma unroll 8
-    for (int j = 0; j < E; j++) {                   // (lanes >= E hold -1: they never outrank an expert)
-        const int kj = __builtin_amdgcn_readlane(key, j);
-        rank += (kj > key || (kj == key && j < lane)) ? 1 : 0;
-    }
-    float wsum = 0.f;
-    for (int k = 0; k < top_k; k++) {               // moe.go:89-92: fp32 sum in rank order
-        const int src = __ffsll((unsigned long long)__ballot(rank == k)) - 1;
-        wsum += __builtin_bit_cast(float, __builtin_amdgcn_readlane(pbits, src));
-    }
-    if (out.ids) {
-        if (lane < E && rank < top_k) { out.ids[(int64_t)m * top_k + rank] = lane; out.w[(int64_t)m * top_k + rank] = prob / wsum; }
-        return;
-    }
-    if (lane < E) gate[(int64_t)m * gate_ld + lane] = rank < top_k ? prob / wsum : 0.f;      // moe.go:103
-    for (int e = E + lane; e < gate_ld; e += 64) gate[(int64_t)m * gate_ld + e] = e < E + n_always ? 1.0f : 0.f;
+// prefill: ids / weights, all 16 rows of a tile in a workgroup (enough workgroups without)
+static __global__ __launch_bounds__(1024) void moe_router_gate_kernel(GemmArgs p, RouteJob job, RouteIds out) {
+    __shared__ __attribute__((aligned(16))) char smem[20 * 1024];
+    const int rows = out.ids ? 16 : ROUTE_ROWS;
+    moe_route_rows<4, 1>(p, job, out, blockIdx.x, blockIdx.y * rows, rows, 16, smem);
 }
 #endif
 
@@ -1446,7 +1512,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(GemmArgs p) {
 // register sets of U k-steps x (NTB weight + MT activation) fragments — for K = 2048 a wave's whole slice is in
 // flight at once.  Same deterministic in-LDS K reduction and fused epilogues as the narrow form.
 // ------------------------------------------------------------------------------------------
-template <int MT, int NTB, int U, int EPI, typename OutT, bool PASSES = false, bool MOE = false>
+template <int MT, int NTB, int U, int EPI, typename OutT, bool PASSES = false, int MOE = 0>
 __global__ __launch_bounds__(512) void gemm_skinny_wide_bf16_kernel(GemmArgs p) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     f32x4* red = (f32x4*)smem;                       // [ksplit][NTB][MT][64]
@@ -1458,8 +1524,12 @@ __global__ __launch_bounds__(512) void gemm_skinny_wide_bf16_kernel(GemmArgs p) 
     int bx = blockIdx.x;
     if constexpr (PASSES) skinny_pass_remap(p, bx);     // (its own instantiation: rewriting the arguments costs the
                                                         // single-group kernels a few scratch dwords otherwise)
+    if constexpr (MOE == 2) {
+        if (bx < p.route.wgs) { moe_route_part<8, 2>(p, bx, ksplit, smem); return; }
+        bx -= p.route.wgs;
+    }
     const int nt0 = bx * NTB;
-    if constexpr (MOE) { if (!moe_expert_live(p, (nt0 * 16) / (2 * p.moe_I))) return; }      // MoE decode: untouched expert (uniform)
+    if constexpr (MOE == 1) { if (!__any(moe_gate_of(p, (nt0 * 16) / (2 * p.moe_I)) != 0.f)) return; }      // MoE decode: untouched expert (uniform)
     const int nks = p.K >> 5, q = nks / ksplit, rr = nks - q * ksplit;
     const int my_steps = q + (kw < rr ? 1 : 0);
     const int ks0 = kw * q + (kw < rr ? kw : rr);
@@ -1539,7 +1609,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_wide_bf16_kernel(GemmArgs p) 
         for (int e = kw; e < (NTB / 2) * MT; e += ksplit) {
             const int j = e / MT, i = e - j * MT;
             const int f = ((nt0 >> 1) + j) * 16 + 4 * fg;
-            epilogue_glu4<EPI, OutT, MOE>(p, 16 * i + fr, f, ksum(2 * j, i), ksum(2 * j + 1, i),
+            epilogue_glu4<EPI, OutT, MOE != 0>(p, 16 * i + fr, f, ksum(2 * j, i), ksum(2 * j + 1, i),
                                         i == i_pre ? rstd_pre : deferred_rstd(p, 16 * i + fr));
         }
     } else {
@@ -1646,12 +1716,17 @@ static inline bool launch_gemm_skinny_ntw(hipStream_t st, const GemmArgs& a) {
         if (ksplit < 1 || ksplit * KS != a.moe_E || ksplit > 16 || (a.moe_I >> 5) < 1) return false;
     }
     if (a.K % 32 != 0) return false;
-    const size_t lds = (size_t)NTW * ksplit * MT * 64 * 16;
+    size_t lds = (size_t)NTW * ksplit * MT * 64 * 16;
+    if (EPI == EPI_RESID && a.moe_gate) lds += (size_t)NTW * ksplit * 256;      // (routing weights, a row a lane of every wave)
     if (a.m_passes > 1 && (nblocks % 8 != 0 || KS != 1)) return launch_skinny_passes_serial<EPI, OutT>(st, a);
     dim3 grid(nblocks * (a.m_passes > 1 ? a.m_passes : 1), KS), block(NTW * ksplit * 64);
     if (a.grid_y != KS) { GemmArgs c = a; c.grid_y = KS; return launch_gemm_skinny_ntw<NTW, EPI, OutT>(st, c); }
 #define NVL_SK(MTv, Uv) hipLaunchKernelGGL((gemm_skinny_bf16_kernel<MTv, NTW, Uv, EPI, OutT>), grid, block, lds, st, a)
-#define NVL_SKM(MTv, Uv, Xv) hipLaunchKernelGGL((gemm_skinny_bf16_kernel<MTv, NTW, Uv, EPI, OutT, false, true, false, Xv>), grid, block, lds, st, a)
+#define NVL_SKM(MTv, Uv, Xv)                                                                                             \
+    do {                                                                                                               \
+        NVL_LDS_ATTR((gemm_skinny_bf16_kernel<MTv, NTW, Uv, EPI, OutT, false, 1, false, Xv>), 16 * (MTv * 1024 + 256));     \
+        hipLaunchKernelGGL((gemm_skinny_bf16_kernel<MTv, NTW, Uv, EPI, OutT, false, 1, false, Xv>), grid, block, lds, st, a); \
+    } while (0)
     if constexpr (epi_moe(EPI) || EPI == EPI_RESID) {
         if (a.moe_gate) {                                 // MoE decode instantiation (expert skip + gate weight)
             if (a.m_passes > 1) return false;
@@ -1659,6 +1734,18 @@ static inline bool launch_gemm_skinny_ntw(hipStream_t st, const GemmArgs& a) {
                 if (a.rs_out) {
                     if (KS < 2) return false;
                     if (MT == 1) NVL_SKM(1, 4, true); else if (MT == 2) NVL_SKM(2, 4, true); else NVL_SKM(4, 2, true);
+                    return true;
+                }
+            }
+            if constexpr (epi_moe(EPI)) {
+                if (a.route.W) {
+                    GemmArgs c = a;
+                    moe_route_share(c, NTW * ksplit);
+                    grid.x += c.route.wgs;
+                    const size_t room = std::max(lds, moe_route_lds(NTW * ksplit));
+                    if (MT == 1) hipLaunchKernelGGL((gemm_skinny_bf16_kernel<1, NTW, 4, EPI, OutT, false, 2>), grid, block, room, st, c);
+                    else if (MT == 2) hipLaunchKernelGGL((gemm_skinny_bf16_kernel<2, NTW, 4, EPI, OutT, false, 2>), grid, block, room, st, c);
+                    else hipLaunchKernelGGL((gemm_skinny_bf16_kernel<4, NTW, 2, EPI, OutT, false, 2>), grid, block, room, st, c);
                     return true;
                 }
             }
@@ -1703,16 +1790,23 @@ static inline bool launch_gemm_skinny_wide(hipStream_t st, const GemmArgs& a) {
         hipLaunchKernelGGL((gemm_skinny_wide_bf16_kernel<MTv, NTB, Uv, EPI, OutT, Pv>), dim3(wgs), dim3(ksplit * 64),      \
                            lds, st, a);                                                                                \
     } while (0)
-#define NVL_SKWM(MTv, Uv)                                                                                                \
+#define NVL_SKWM(MTv, Uv, Rv, grid, room, args)                                                                          \
     do {                                                                                                               \
-        NVL_LDS_ATTR((gemm_skinny_wide_bf16_kernel<MTv, NTB, Uv, EPI, OutT, false, true>), 8 * NTB * MTv * 64 * 16);         \
-        hipLaunchKernelGGL((gemm_skinny_wide_bf16_kernel<MTv, NTB, Uv, EPI, OutT, false, true>), dim3(wgs), dim3(ksplit * 64), \
-                           lds, st, a);                                                                                \
+        NVL_LDS_ATTR((gemm_skinny_wide_bf16_kernel<MTv, NTB, Uv, EPI, OutT, false, Rv>), 8 * NTB * MTv * 64 * 16);           \
+        hipLaunchKernelGGL((gemm_skinny_wide_bf16_kernel<MTv, NTB, Uv, EPI, OutT, false, Rv>), dim3(grid), dim3(ksplit * 64), \
+                           room, st, args);                                                                            \
     } while (0)
     if constexpr (epi_moe(EPI)) {
         if (a.moe_gate) {
             if (a.m_passes > 1) return false;
-            if (MT == 1) NVL_SKWM(1, 4); else if (MT == 2) NVL_SKWM(2, 4); else NVL_SKWM(4, 2);
+            if (a.route.W) {
+                GemmArgs c = a;
+                moe_route_share(c, ksplit);
+                const size_t room = std::max(lds, moe_route_lds(ksplit));
+                if (MT == 1) NVL_SKWM(1, 4, 2, wgs + c.route.wgs, room, c); else if (MT == 2) NVL_SKWM(2, 4, 2, wgs + c.route.wgs, room, c); else NVL_SKWM(4, 2, 2, wgs + c.route.wgs, room, c);
+                return true;
+            }
+            if (MT == 1) NVL_SKWM(1, 4, 1, wgs, lds, a); else if (MT == 2) NVL_SKWM(2, 4, 1, wgs, lds, a); else NVL_SKWM(4, 2, 1, wgs, lds, a);
             return true;
         }
     }

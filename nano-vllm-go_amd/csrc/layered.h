@@ -1474,10 +1474,13 @@ SubOut expert_ffn(nvl_model* m, const LayerRun& r, const MixerW& w, int M, Exper
         glu_up(m, W, M, r.Fp, r.act, c.ffn_limit);
         y = sub_out(m, KS_FFN_DOWN, m->hbuf, w.w2, M, r.Fp);
     };
-    if (dense && E <= 64 && c.route_softmax) {
+    const RouteJob job{(const bf16_t*)w.router, w.route_bias, m->moe_gate, nullptr, E, k, r.Ep, 0, parts};
+    const bool one_route = dense && E <= 64 && c.route_softmax, route_beside = one_route && moe_route_beside(M, E, k, 2.0 * r.Ip * m->H * m->wsize);
+    if (route_beside) {
+    } else if (one_route) {
         GemmArgs a = mk(m->xn, m->H, w.router, nullptr, E, w.route_bias, 1.f, M, E, m->H);
         KScope ks(m, KC_OTHER, 2.0 * M * E * m->Hn, KS_MOE_ROUTER, ((double)E * m->Hn + (double)M * m->Hn) * (double)m->wsize + (double)M * E * 4.0);
-        hipLaunchKernelGGL(moe_router_gate_kernel, router_gate_grid(M), dim3(1024), 0, m->stream, a, k, RouteOut{m->moe_gate, nullptr, nullptr}, (float*)nullptr, 0, r.Ep, parts);
+        hipLaunchKernelGGL(moe_router_gate_kernel, router_gate_grid(M), dim3(1024), 0, m->stream, a, job, RouteIds{nullptr, nullptr});
         NVL_HIP(hipGetLastError());
     } else {
         m->site = KS_MOE_ROUTER;
@@ -1493,6 +1496,7 @@ SubOut expert_ffn(nvl_model* m, const LayerRun& r, const MixerW& w, int M, Exper
         const double touch = (double)std::min(E, pairs) * c.expert_dim + (parts ? c.ffn_dim : 0), work = (double)pairs * c.expert_dim + (parts ? (double)M * c.ffn_dim : 0.0);
         GemmArgs u = mk(m->xn, m->H, w.moe_up, m->moe_hall, r.Ep * r.Ip, nullptr, 1.f, M, (E + parts) * 2 * r.Ip, m->H);
         u.moe_gate = m->moe_gate; u.moe_E = r.Ep; u.moe_I = r.Ip;
+        if (route_beside) u.route = job;
         u.glu_limit = c.expert_limit; u.glu_limit2 = c.ffn_limit; u.glu_from2 = E * r.Ip; u.glu_slope = CLAMPED_GLU_SLOPE;
         m->site = KS_MOE_UP; m->site_bytes = (2 * touch * m->Hn + (double)M * m->Hn + work) * (double)m->wsize;
         gemm(m, c.expert_limit > 0.f ? EPI_CLAMP_GLU : EPI_SWIGLU, false, u, 4.0 * work * m->Hn);

@@ -1526,7 +1526,7 @@ static int g_moe_bm = 0;       // nvl_set_tuning key 17: prefill MoE grouped GEM
 static int g_moe_gather = 1;   // nvl_set_tuning key 16: prefill MoE gathers the token rows into expert order before the grouped GEMM (0 = per-lane gather inside it)
 static int g_moe_defer_down = 1;    // nvl_set_tuning key 33: MoE decode: the last of the K slices' workgroups completes the residual and carries the next norm
                                     // (deferred RMSNorm producer, gemm.h split_finish_wave); 0: slices left to a norm launch
-static int g_moe_fused_route = 1;   // nvl_set_tuning key 31: MoE decode routing (router GEMM + softmax / top-k / gate matrix) as one launch (0 = two)
+static int g_moe_fused_route = 1;   // nvl_set_tuning key 31: MoE decode routing (router GEMM + softmax / top-k / gate matrix): 1 one launch, or none (moe_route_beside), 2 always one, 0 two
 static int g_moe_small = 1;    // nvl_set_tuning key 8: fused MoE planning launch + combine folded into the next norm (0 = off)
 static int g_mamba_ssd = 1;    // nvl_set_tuning key 30: chunked (SSD) Mamba2 scan on MFMA for prefill-sized bf16 calls (0 = the sequential scan,
                                // 2 = chunk after chunk only, never the chunk-parallel three-launch form)
@@ -1701,6 +1701,13 @@ bool moe_dense_ok(const nvl_model* m, const LayerW& l, int M) {
     return !m->f32 && M <= 64 && g_moe_dense && l.moe_out_cat && m->moe_part && !m->keep_hidden && m->H % 4 == 0 &&
            m->H <= 1024 * NORM_ROW_MAXCH && g_force_tile == 0;
 }
+// Does a decode batch route inside the experts' up launch?  The launch that this saves is some 8 us (16 rows of 1024 and 32 experts; 2048 and 6 rows: 7.4
+// and the gap); not knowing the chosen experts, the up projection streams them all, at 6 TB/s.  Either all that a token leaves out costs
+// little more than that, or a batch is expected to leave out next to nothing, were its choices even.
+bool moe_route_beside(int M, int E, int k, double expert_bytes) {
+    const double out_us = E > k ? (E - k) * expert_bytes / 6e6 : 0.0, expected_us = E > k ? pow(1.0 - (double)k / E, M) * E * expert_bytes / 6e6 : 0.0;
+    return g_moe_fused_route == 1 && (expected_us < 1.5 || (out_us < 9.0 && expected_us < 6.0));
+}
 // deferred_norm: m->xn holds xn_raw = bf16(x * w_norm) and m->rs_part the x^2 partials (the O projection carried the FFN
 // norm): the router and the expert-up projection scale their accumulators by rstd[m] instead of reading a normed operand
 // next_norm_w (decode, dense-masked form only): the down projection carries the NEXT norm (the following layer's attention
@@ -1721,16 +1728,21 @@ bool moe(nvl_model* m, const LayerW& l, int M, bool deferred_norm = false, const
     // prefill: the same launch, leaving the chosen experts (6867 rows of 1024, 32 experts: 20 us on 54 tiles of 128 x 128 and 9 us of
     // routing before, 12.7 now)
     const bool route_ids = !m->f32 && !dense && !small && !deferred_norm && g_moe_fused_route && E <= 64 && H % 32 == 0 && g_force_tile == 0;
+    const RouteJob job{(const bf16_t*)l.t[NVL_T_ROUTER].p, nullptr, m->moe_gate, m->router_logits, E, k, E, 128, 0};
+    const bool route_beside = fused_route && moe_route_beside(M, E, k, 2.0 * I * H * m->wsize);
     {
         GemmArgs ar = mk(m->xn, H, l.t[NVL_T_ROUTER].p, m->router_logits, 128, nullptr, 1.f, M, E, H);
         if (deferred_norm) set_deferred_in(m, ar);
-        if (fused_route) {
+        if (route_beside) {
+        } else if (fused_route) {
             KScope ks(m, KC_GEMM, 2.0 * (double)M * E * H, -1, ((double)E * H + (double)M * H) * (double)m->wsize + (double)M * E * 8.0);
-            hipLaunchKernelGGL(moe_router_gate_kernel, router_gate_grid(M), dim3(1024), 0, m->stream, ar, k, RouteOut{m->moe_gate, nullptr, nullptr}, m->router_logits, 128, E, 0);
+            hipLaunchKernelGGL(moe_router_gate_kernel, router_gate_grid(M), dim3(1024), 0, m->stream, ar, job, RouteIds{nullptr, nullptr});
             NVL_HIP(hipGetLastError());
         } else if (route_ids) {
             KScope ks(m, KC_GEMM, 2.0 * (double)M * E * H, -1, ((double)E * H + (double)M * H) * (double)m->wsize + (double)pairs * 8.0);
-            hipLaunchKernelGGL(moe_router_gate_kernel, dim3(cdiv(M, 16)), dim3(1024), 0, m->stream, ar, k, RouteOut{nullptr, m->expert_ids, m->expert_w}, (float*)nullptr, 0, 0, 0);
+            RouteJob chosen = job;
+            chosen.logits = nullptr;
+            hipLaunchKernelGGL(moe_router_gate_kernel, dim3(cdiv(M, 16)), dim3(1024), 0, m->stream, ar, chosen, RouteIds{m->expert_ids, m->expert_w});
             NVL_HIP(hipGetLastError());
         } else {
             gemm(m, EPI_STORE, true, ar);
@@ -1749,6 +1761,7 @@ bool moe(nvl_model* m, const LayerW& l, int M, bool deferred_norm = false, const
         }
         GemmArgs a = mk(m->xn, H, l.moe_in, m->moe_hall, E * I, nullptr, 1.f, M, E * 2 * I, H);
         a.moe_gate = m->moe_gate; a.moe_E = E; a.moe_I = I;
+        if (route_beside) a.route = job;
         if (deferred_norm) set_deferred_in(m, a);
         m->site = KS_MOE_UP; m->site_bytes = (e_touch * 2 * I * H + (double)M * H + e_touch * M * I) * (double)m->wsize;
         gemm(m, EPI_SWIGLU, false, a, 2.0 * pairs * 2 * I * H);

@@ -21,7 +21,7 @@ def both(run):
 
 @pytest.mark.parametrize("precision", ["f32", "bf16"])
 @pytest.mark.parametrize("n", [3, 40])                                   # 6 and 80 rows of a prompt
-@pytest.mark.parametrize("settings", [{}, {31: 0}, {22: 0}, {22: 0, 8: 0}])     # routing in the router's launch, apart, planned in one launch, sorted
+@pytest.mark.parametrize("settings", [{}, {31: 2}, {31: 0}, {22: 0}, {22: 0, 8: 0}])     # routing in the router's launch, apart, planned in one launch, sorted
 def test_plain_models(gpu, precision, n, settings):
     cfg = gpu.synth.tiny_config("granite_moe", tied_embedding=False)
     w = gpu.synth.make_weights(cfg, seed=9, scale=0.05)
