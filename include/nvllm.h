@@ -548,7 +548,7 @@ int nvl_bench_gemm(int device, int M, int N, int K, int epi, int force_bnt, int 
  * key 1: K slices of the decode residual projections (0 automatic, 1 never split, 2, 4).
  * key 2: decode (M <= 64) GEMM form: 0 automatic, 1/2/4 = narrow form with that many weight tiles per workgroup,
  * 8 = wide-N form (4 weight tiles per wave).
- * key 3: deferred RMSNorm in decode (0 off, 1 on, 2 on without the activation-tile split, 3 only the O-proj -> FFN-up seam; with 2 or 3,
+ * key 3: deferred RMSNorm in decode, and layer norms of up to 64 rows (0 off, 1 on, 2 on without the activation-tile split, 3 only the O-proj -> FFN-up seam; layer norms: 1 only; with 2 or 3,
  * or key 2 = 2 or 4, a hybrid's Mamba layers and 8-row half tiles keep their forms without a carried norm).
  * keys 4-6 (sweeps): K split of the wide form, waves per narrow-form launch, K split of the deferred-norm residual
  * projections.  key 7: decode seam kernel, 8: MoE small-batch fusion, 9: prompt norms in tiles of eight rows, 10: query rows per

@@ -101,6 +101,23 @@ __device__ __forceinline__ float block256_sum(float v, float* red) {
     __syncthreads();
     return t;
 }
+// what a deferred layer norm takes from the weights behind it (GemmArgs::ln_s): s[n] = sum_k W[n][k] w[k], b[n] = bias[n] + sum_k W[n][k] nb[k];
+// zero for the rows n >= N that pad W.  One wave per 16 rows, W fragment-major
+static __global__ __launch_bounds__(64) void ln_fold_kernel(const bf16_t* __restrict__ W, const float* __restrict__ w, const float* __restrict__ nb, const float* __restrict__ bias,
+                                                            float* __restrict__ s, float* __restrict__ b, int N, int K) {
+    const int lane = threadIdx.x, fg = lane >> 4, n = blockIdx.x * 16 + (lane & 15);
+    float a = 0.f, c = 0.f;
+    for (int ks = 0; ks < (K >> 5); ks++) {
+        const bf16x8 v = *(const bf16x8*)(W + (((int64_t)blockIdx.x * (K >> 5) + ks) * 64 + lane) * 8);
+        const float *wk = w + ks * 32 + fg * 8, *bk = nb + ks * 32 + fg * 8;
+#pragma unroll
+        for (int e = 0; e < 8; e++) { a += (float)v[e] * wk[e]; c += (float)v[e] * bk[e]; }
+    }
+    a += __shfl_xor(a, 16, 64); c += __shfl_xor(c, 16, 64);
+    a += __shfl_xor(a, 32, 64); c += __shfl_xor(c, 32, 64);
+    if (fg == 0) { s[n] = n < N ? a : 0.f; b[n] = n < N ? c + (bias ? bias[n] : 0.f) : 0.f; }
+}
+
 // Pending residual: the decode GEMMs that precede a norm (O projection, W2) may leave their output as
 // split-K partial slices instead of adding it into x; this kernel then completes the residual add
 // (generic_model.go:320-326,383-389) while it reads the row:  x[row] += alpha * sum_s part[s][row]  (slice order).
@@ -230,7 +247,7 @@ __global__ __launch_bounds__(64 * NORM_TILE_ROWS) void norm_tile_kernel(float* _
 template <typename ActT>
 __device__ __forceinline__ void norm_row_finish(f32x4 (&v)[NORM_ROW_MAXCH], f32x4 (&ww)[NORM_ROW_MAXCH],
                                                 f32x4 (&bb)[NORM_ROW_MAXCH], const float* b, float eps, ActT* y, int r,
-                                                int H, float* red, int width = 0) {     // width: columns of the mean when the row is padded (0: H)
+                                                int H, float* red, int width = 0, float* mean_out = nullptr) {     // width: columns of the mean when the row is padded (0: H)
     const int H4 = H >> 2;
     if (b == nullptr) {
         float ss = 0.f;
@@ -253,6 +270,7 @@ __device__ __forceinline__ void norm_row_finish(f32x4 (&v)[NORM_ROW_MAXCH], f32x
         for (int c = 0; c < NORM_ROW_MAXCH; c++) s += v[c][0] + v[c][1] + v[c][2] + v[c][3];   // zero-filled beyond H
         const int W = width ? width : H;
         const float mean = block256_sum(s, red) / (float)W;
+        if (mean_out && threadIdx.x == 0) mean_out[r] = mean;
         float vs = 0.f;
 #pragma unroll
         for (int c = 0; c < NORM_ROW_MAXCH; c++) {
@@ -281,7 +299,7 @@ __global__ __launch_bounds__(256) void norm_row_kernel(float* __restrict__ x,
                                                        const int32_t* __restrict__ rows_idx,
                                                        const float* __restrict__ w,
                                                        const float* __restrict__ b, float eps,
-                                                       ActT* __restrict__ y, int H, PendingResid pr) {
+                                                       ActT* __restrict__ y, int H, PendingResid pr, float* mean_out) {      // mean_out: [rows] or NULL (layer norm)
     __shared__ float red[4];
     const int r = blockIdx.x;
     const int src = rows_idx ? rows_idx[r] : r;
@@ -312,7 +330,7 @@ __global__ __launch_bounds__(256) void norm_row_kernel(float* __restrict__ x,
             if (b) bb[c] = *(const f32x4*)(b + j * 4);
         }
     }
-    norm_row_finish<ActT>(v, ww, bb, b, eps, y, r, H, red);
+    norm_row_finish<ActT>(v, ww, bb, b, eps, y, r, H, red, 0, mean_out);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -917,7 +935,7 @@ __global__ __launch_bounds__(256) void decode_seam_kernel(const float* __restric
                                                           const bf16_t* __restrict__ emb, const bf16_t* __restrict__ pos_emb,
                                                           int max_seq, float mult, float* __restrict__ x,
                                                           const float* __restrict__ w, const float* __restrict__ b,
-                                                          float eps, bf16_t* __restrict__ y, int H, int width, SeamShift sh) {
+                                                          float eps, bf16_t* __restrict__ y, int H, int width, SeamShift sh, float* mean_out) {
     __shared__ float red[4];
     __shared__ int tok_s, pos_s, old_s;
     const int r = blockIdx.x;
@@ -981,7 +999,7 @@ __global__ __launch_bounds__(256) void decode_seam_kernel(const float* __restric
         }
     }
     if (!w) return;
-    norm_row_finish<bf16_t>(v, ww, bb, b, eps, y, r, H, red, width);
+    norm_row_finish<bf16_t>(v, ww, bb, b, eps, y, r, H, red, width, mean_out);
 }
 
 // ---------------------------------------------------------------------------------------

@@ -49,7 +49,12 @@ enum GemmEpi {
     EPI_GROUPED_RAW = 11,    // ... of attention whose queries and keys are normed or rotated first: those go to fp32 rows, as does what lies behind the gate
     EPI_REGLU = 10,      // C[m, f] = max(gate, 0) * up   W rows interleaved as for EPI_SWIGLU
     EPI_GELU_TOK = 8,    // C[m, n] = gelu_tanh(acc) * tok_table[tok_ids[m]][n]   (an input of the token's own, GemmArgs::tok_*)
+    // ... with a deferred layer norm (GemmArgs::ln_s): decode kernels alone
+    EPI_LN_STORE = 12, EPI_LN_RESID = 13, EPI_LN_GELU = 14, EPI_LN_QKV = 15,
 };
+constexpr bool epi_ln(int epi) { return epi >= 12; }
+constexpr int skinny_waves(int epi) { return epi_ln(epi) ? 8 : 16; }      // most waves of a workgroup of the narrow decode form (the pairs of a layer norm take registers)
+constexpr int epi_base(int epi) { return epi == 15 ? 4 : epi == 14 ? 3 : epi >= 12 ? epi - 12 : epi; }
 
 constexpr bool epi_moe(int epi) { return epi == 2 || epi == 6; }      // ... with instances for masked experts
 constexpr bool epi_glu(int epi) { return epi == 2 || epi == 5 || epi == 6 || epi == 10; }      // gate | up pairs in, one column out
@@ -159,6 +164,16 @@ struct GemmArgs {
     // workgroups then do the routing (route) beside it.
     const float* moe_gate;
     int moe_E, moe_I;
+    // Deferred layer norm (epi_ln; M <= 64): ((x - mean) w / sd + b) W == rstd ((x - s) w W - (mean - s) S) + B for any s, S[n] = sum_k W[n][k] w[k] and
+    // B[n] = bias[n] + sum_k W[n][k] b[k] from the weights alone.  Producer: xn_raw = bf16((x - s) w) and per tile the pair of sums of x - s and
+    // (x - s)^2; s is the row's mean at the norm before, so that a row far from zero loses nothing to the operand's rounding (ln_prev: that
+    // norm's pairs, or NULL, where it was a launch of its own that left its means in ln_mean_in).  Consumer: bias is B.
+    // A norm launch is 3.3 us (1 row) to 4.2 (16) and a boundary; the sums cost the four projections of a layer 0.5 to 1.7 us each.  GPT-2, us a step of
+    // 1 / 16 / 24 / 40 / 64 sequences: 434 -> 402, 493 -> 458, 540 -> 490, 567 -> 532, 690 -> 663; prompts of 11 / 3 x 11 / 64 tokens 514 -> 451, 595 -> 536, 586 -> 542.
+    // Error of the logits against 64 bits over 240 calls: mean log ratio to the norm launches +0.002 +- 0.002.
+    const float* ln_s;
+    const float *ln_prev, *ln_mean_in;
+    float* ln_mean_out;
 };
 // the routing weight that row `lane` of the batch (M <= 64) gives expert e
 __device__ __forceinline__ float moe_gate_of(const GemmArgs& p, int e) {
@@ -300,6 +315,55 @@ __device__ __forceinline__ float deferred_rstd(const GemmArgs& p, int m) {
     s += __shfl_xor(s, 16, 64);
     s += __shfl_xor(s, 32, 64);
     return 1.0f / sqrtf(s * p.rs_inv_h + p.rs_eps);
+}
+
+// deferred layer norm: a row's pairs of partial sums, `tiles` of them (a multiple of 16), by the four lanes that share the row.  The loads
+// leave together and are added where they are needed: a loop of eight and its remainder waited for memory five times, 2 us of a 5 us launch (768 columns).
+struct RowPairs {
+    static constexpr int NB = 12;
+    f32x4 t[NB];
+    int n;
+    const f32x4* src;
+    __device__ __forceinline__ void fetch(const float* pairs, int tiles, int m, bool live) {
+        n = tiles >> 3;
+        src = (const f32x4*)(pairs + 2 * ((int64_t)m * tiles)) + ((threadIdx.x & 63) >> 4) * n;
+#pragma unroll
+        for (int j = 0; j < NB; j++) t[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (live) {
+#pragma unroll
+            for (int j = 0; j < NB; j++) t[j] = src[j < n ? j : n - 1];
+        } else n = 0;
+    }
+    // sums of x - s and of its square, in every lane of the row
+    __device__ __forceinline__ f32x2 sum() const {
+        f32x4 a4 = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < NB; j++) a4 += j < n ? t[j] : f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int j = NB; j < n; j++) a4 += src[j];
+        float s = a4[0] + a4[2], ss = a4[1] + a4[3];
+        s += __shfl_xor(s, 16, 64); ss += __shfl_xor(ss, 16, 64);
+        s += __shfl_xor(s, 32, 64); ss += __shfl_xor(ss, 32, 64);
+        return f32x2{s, ss};
+    }
+};
+// what scales row m's sums, and what then adds ln_s
+struct RowNorm { float scale, shift; };
+__device__ __forceinline__ RowNorm layer_norm_of(const GemmArgs& p, f32x2 s) {
+    const float d = s[0] * p.rs_inv_h, rstd = 1.0f / sqrtf(fmaxf(s[1] * p.rs_inv_h - d * d, 0.f) + p.rs_eps);
+    return {rstd, -rstd * d};
+}
+template <int EPI>
+__device__ __forceinline__ RowNorm row_norm(const GemmArgs& p, int m) {
+    if constexpr (!epi_ln(EPI)) return {deferred_rstd(p, m), 0.f};
+    RowPairs r;
+    r.fetch(p.rs_in, p.rs_tiles, m, m < p.M);
+    return layer_norm_of(p, r.sum());
+}
+// ... applied to four columns from n on
+template <int EPI>
+__device__ __forceinline__ f32x4 normed(const GemmArgs& p, int n, f32x4 v, RowNorm r) {
+    if constexpr (epi_ln(EPI)) return v * r.scale + r.shift * *(const f32x4*)(p.ln_s + n);
+    else return v * r.scale;
 }
 
 template <int EPI, typename OutT, bool MOE = false>
@@ -1206,8 +1270,10 @@ __device__ __forceinline__ void skinny_pass_remap(GemmArgs& p, int& bx) {
 // (rs_out; COMPLETES).  Instances of their own: beside it the others lose 1 %, and the experts' slices 16 % at 40 rows (4096 x 32 x 448:
 // 43.9 -> 51 us, their registers spill).
 // MOE: 1 masked experts, 2 (up) all experts, the launch's first workgroups route.
-template <int MT, int NTW, int U, int EPI, typename OutT, bool PASSES = false, int MOE = 0, bool HALF = false, bool EXTRA = false>
-__global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
+template <int MT, int NTW, int U, int EPIV, typename OutT, bool PASSES = false, int MOE = 0, bool HALF = false, bool EXTRA = false>
+__global__ __launch_bounds__(skinny_waves(EPIV) * 64) void gemm_skinny_bf16_kernel(GemmArgs p) {
+    constexpr int EPI = epi_base(EPIV);
+    constexpr bool LN = epi_ln(EPIV);
     constexpr bool SCALED = EXTRA && MOE == 0, COMPLETES = EXTRA && MOE != 0;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     f32x4* red = (f32x4*)smem;                       // [NTW][ksplit][MT][64]
@@ -1240,7 +1306,14 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
     // (MT = 4 — batches above 32 and the 64-row groups of larger ones — has no registers to hold it across the stream:
     // 34-54 spilled there, QKV at 128 rows 7.2 -> 10.8 us; those launches are long enough to fetch it in the epilogue)
     constexpr bool RSTD_PRE = MT <= 2;
-    const float rstd_pre = (RSTD_PRE && (EPI == EPI_STORE || EPI == EPI_QKV || SCALED || epi_glu(EPI)) && wave < NTW * MT) ? deferred_rstd(p, 16 * (i_pre + (SCALED ? i_off : 0)) + fr) : 1.0f;   // (only the waves that run an epilogue element)
+    constexpr bool NORMED = EPI == EPI_STORE || EPI == EPI_QKV || SCALED || epi_glu(EPI) || (LN && EPI == EPI_GELU);
+    // (layer norms have the registers to add the sums up behind the stream)
+    constexpr bool LN_LATE = LN && NORMED;
+    RowPairs pairs;
+    if constexpr (LN_LATE) pairs.fetch(p.rs_in, p.rs_tiles, 16 * i_pre + fr, 16 * i_pre + fr < p.M && wave < NTW * MT);
+    RowNorm rn_pre = (!LN_LATE && RSTD_PRE && NORMED && wave < NTW * MT) ? row_norm<EPIV>(p, 16 * (i_pre + (SCALED ? i_off : 0)) + fr) : RowNorm{1.0f, 0.f};   // (only the waves that run an epilogue element)
+    const float rstd_pre = LN ? 1.0f : rn_pre.scale;
+    auto row_norm_of = [&](int i) { return (RSTD_PRE || LN_LATE) && i == i_pre ? rn_pre : row_norm<EPIV>(p, 16 * i + fr); };
     // (grid_y: gridDim.y as an explicit argument — the built-in lives in the hidden part of the kernarg block and costs a
     // dependent scalar round trip of its own before the first weight load)
     const int nslices = p.m_split ? 1 : p.grid_y, slice = p.m_split ? 0 : blockIdx.y;
@@ -1312,6 +1385,14 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
         const int m = 16 * (i + i_off) + fr, n = (nt0 + t) * 16 + 4 * fg;
         if (m < p.M && n < p.N && (!HALF || (fg >> 1) == half)) x_pre = *(const f32x4*)((const float*)p.C + (int64_t)m * p.ldc + n);
     }
+    float ln_shift = 0.f;      // (MT = 1: one row tile)
+    if constexpr (LN && EPI == EPI_RESID) {
+        static_assert(MT == 1 && NTW == 1, "one epilogue element");
+        const int m = 16 * i_off + fr;
+        const bool live = wave == 0 && m < p.M;
+        if (live) ln_shift = p.ln_mean_in[m];
+        pairs.fetch(p.ln_prev, p.rs_tiles, m, live && p.ln_prev);
+    }
     if constexpr (MOE != 0 && EPI == EPI_RESID) {
         for (int b = 0; b < nblk; b += 2) {
             if (b + 1 < nblk) load_blk(wB, xB, b + 1);
@@ -1344,6 +1425,11 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
             const float g = gates[16 * i + fr];
             acc[i] = g != 0.f ? acc[i] * g : f32x4{0.f, 0.f, 0.f, 0.f};       // (0: not routed, whatever the expert made of the row)
         }
+    if constexpr (LN_LATE) rn_pre = layer_norm_of(p, pairs.sum());
+    if constexpr (LN && EPI == EPI_RESID) {
+        ln_shift += pairs.sum()[0] * p.rs_inv_h;
+        if (blockIdx.x == 0 && wave == 0 && fg == 0 && 16 * i_off + fr < p.M) p.ln_mean_out[16 * i_off + fr] = ln_shift;
+    }
     // ---- reduce the K slices in wave order ----
 #pragma unroll
     for (int i = 0; i < MT; i++) red[((tile * ksplit + kw) * MT + i) * 64 + lane] = acc[i];
@@ -1363,8 +1449,9 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
         }
     } else if constexpr (EPI == EPI_QKV) {
         for (int i = wave; i < MT; i += NTW * ksplit) {
-            const float rs = RSTD_PRE && i == i_pre ? rstd_pre : deferred_rstd(p, 16 * i + fr);
-            epilogue_qkv_pair(p, 16 * i + fr, q_head, q_tile * 16 + 4 * fg, ksum(0, i) * rs, ksum(NTW - 1, i) * rs);
+            const RowNorm rn = row_norm_of(i);
+            const int n = q_head * p.qkv.hd + q_tile * 16 + 4 * fg;
+            epilogue_qkv_pair(p, 16 * i + fr, q_head, q_tile * 16 + 4 * fg, normed<EPIV>(p, n, ksum(0, i), rn), normed<EPIV>(p, n + (p.qkv.hd >> 1), ksum(NTW - 1, i), rn));
         }
     } else if (EPI == EPI_RESID && nslices > 1) {
         // split-K across workgroups: publish the partial tile (slice 0 carries the bias); the following norm
@@ -1390,16 +1477,30 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
             const int m = 16 * (i + i_off) + fr, n = (nt0 + t) * 16 + 4 * fg;      // N % 16 == 0 (hidden width)
             f32x4 v = ksum(t, i);
             if constexpr (SCALED) v *= rstd_pre;      // (MT = 1: one row tile)
-            float ss = 0.f;
+            float ss = 0.f, sx = 0.f;
             if (m < p.M && n < p.N && (!HALF || (fg >> 1) == half)) {
                 if (p.bias) v += *(const f32x4*)(p.bias + n);
                 float* x = (float*)p.C + (int64_t)m * p.ldc + n;
                 const f32x4 o = (e == wave ? x_pre : *(f32x4*)x) + p.alpha * v;
                 *(f32x4*)x = o;
+                if constexpr (LN) {
+                    const f32x4 c = o - ln_shift;
+                    act_store4<bf16_t>(p.nrm_xn, m, n, p.N, c * *(const f32x4*)(p.nrm_w + n));
+                    ss = c[0] * c[0] + c[1] * c[1] + c[2] * c[2] + c[3] * c[3];
+                    sx = (c[0] + c[1]) + (c[2] + c[3]);
+                } else {
                 act_store4<bf16_t>(p.nrm_xn, m, n, p.N, o * *(const f32x4*)(p.nrm_w + n));
                 ss = o[0] * o[0] + o[1] * o[1] + o[2] * o[2] + o[3] * o[3];
+                }
             }
             ss += __shfl_xor(ss, 16, 64);
+            if constexpr (LN) {
+                sx += __shfl_xor(sx, 16, 64);
+                const int tiles = p.N >> (HALF ? 3 : 4), tile = HALF ? 2 * (nt0 + t) + half : nt0 + t;
+                if constexpr (!HALF) { ss += __shfl_xor(ss, 32, 64); sx += __shfl_xor(sx, 32, 64); }
+                if (fg == (HALF ? 2 * half : 0) && m < p.M && (nt0 + t) * 16 < p.N) *(f32x2*)(p.rs_out + 2 * ((int64_t)m * tiles + tile)) = f32x2{sx, ss};
+                continue;
+            }
             if constexpr (HALF) {     // the two lane rows (fg = 2 half, 2 half + 1) of this workgroup's 8 columns
                 if (fg == 2 * half && (nt0 + t) * 16 < p.N) p.rs_out[(int64_t)m * (p.N >> 3) + 2 * (nt0 + t) + half] = ss;
                 continue;
@@ -1410,7 +1511,8 @@ __global__ __launch_bounds__(1024) void gemm_skinny_bf16_kernel(GemmArgs p) {
     } else {
         for (int e = wave; e < NTW * MT; e += NTW * ksplit) {
             const int t = e / MT, i = e - t * MT;
-            epilogue4<EPI, OutT>(p, 16 * i + fr, (nt0 + t) * 16 + 4 * fg, ksum(t, i),
+            if constexpr (LN) epilogue4<EPI, OutT>(p, 16 * i + fr, (nt0 + t) * 16 + 4 * fg, normed<EPIV>(p, (nt0 + t) * 16 + 4 * fg, ksum(t, i), row_norm_of(i)));
+            else epilogue4<EPI, OutT>(p, 16 * i + fr, (nt0 + t) * 16 + 4 * fg, ksum(t, i),
                                  EPI != EPI_STORE ? 1.0f : (RSTD_PRE && i == i_pre ? rstd_pre : deferred_rstd(p, 16 * i + fr)));
         }
     }
@@ -1710,7 +1812,7 @@ static inline bool launch_gemm_skinny_ntw(hipStream_t st, const GemmArgs& a) {
         const int64_t budget = (int64_t)g_narrow_waves * ((a.moe_gate && epi_moe(EPI)) ? 2 : 1);
         while (ksplit > 1 && (int64_t)nblocks * KS * NTW * ksplit > budget) ksplit >>= 1;
     }
-    while (ksplit > 1 && ((a.K >> 5) / (ksplit * KS) < U || ksplit * NTW > 16)) ksplit >>= 1;   // >= one block of U k-steps per wave
+    while (ksplit > 1 && ((a.K >> 5) / (ksplit * KS) < U || ksplit * NTW > skinny_waves(EPI))) ksplit >>= 1;   // >= one block of U k-steps per wave
     if (a.moe_gate && EPI == EPI_RESID) {      // MoE down: every wave's K range is exactly one expert (the skip test needs it)
         ksplit = a.moe_E / KS;
         if (ksplit < 1 || ksplit * KS != a.moe_E || ksplit > 16 || (a.moe_I >> 5) < 1) return false;
@@ -1817,7 +1919,8 @@ static inline bool launch_gemm_skinny_wide(hipStream_t st, const GemmArgs& a) {
 }
 template <int EPI, typename OutT>
 static inline bool launch_gemm_skinny_bf16(hipStream_t st, const GemmArgs& a0) {
-    if (EPI == EPI_QKV && (a0.qkv.hd % 32 != 0 || a0.m_passes > 1)) return false;
+    constexpr int E = epi_base(EPI);
+    if (E == EPI_QKV && (a0.qkv.hd % 32 != 0 || a0.m_passes > 1)) return false;
     if (skinny_rows(a0) > 64 || a0.a_rows || a0.seg || a0.tile_map) return false;
     GemmArgs a = a0;
     a.x_mask = (g_x_mask && a0.M % 16 != 0) ? 1 : 0;     // padded rows of the last 16-row activation tile are not fetched
@@ -1826,10 +1929,27 @@ static inline bool launch_gemm_skinny_bf16(hipStream_t st, const GemmArgs& a0) {
         const bool wide_ok = skinny_rows(a) > 16 && cdiv(a.N, 64) >= 256 && !a.sk_part;   // M <= 16: the narrow form streams as fast
         if (g_force_ntw == 8 || (g_force_ntw == 0 && wide_ok)) { if (launch_gemm_skinny_wide<EPI, OutT>(st, a)) return true; }
     }
-    if constexpr (epi_glu(EPI) || EPI == EPI_QKV) return launch_gemm_skinny_ntw<2, EPI, OutT>(st, a);      // (pairs: gate | up, the halves of a head)
+    if constexpr (epi_glu(EPI) || E == EPI_QKV) return launch_gemm_skinny_ntw<2, EPI, OutT>(st, a);      // (pairs: gate | up, the halves of a head)
+    if constexpr (epi_ln(EPI)) return launch_gemm_skinny_ntw<1, EPI, OutT>(st, a);
     if (g_force_ntw == 2) return launch_gemm_skinny_ntw<2, EPI, OutT>(st, a);
     if (g_force_ntw == 4) return launch_gemm_skinny_ntw<4, EPI, OutT>(st, a);
     return launch_gemm_skinny_ntw<1, EPI, OutT>(st, a);
+}
+
+// a residual projection that carries a layer norm: as one that carries an RMSNorm, a workgroup per (weight tile, 16-row tile) or half of the former
+template <typename OutT>
+static inline bool launch_gemm_ln_resid(hipStream_t st, const GemmArgs& a0) {
+    if (a0.M > 64 || a0.K % 32 != 0 || !a0.rs_out || (a0.rs_half && a0.M > 16)) return false;
+    GemmArgs a = a0;
+    a.grid_y = 1;
+    a.m_split = 1;
+    a.x_mask = (g_x_mask && a.M % 16 != 0) ? 1 : 0;
+    int ks = skinny_waves(EPI_LN_RESID);
+    while (ks > 1 && (a.K >> 5) / ks < 4) ks >>= 1;
+    const int tiles = cdiv(a.N, 16);
+    if (a.rs_half) hipLaunchKernelGGL((gemm_skinny_bf16_kernel<1, 1, 4, EPI_LN_RESID, OutT, false, 0, true>), dim3(2 * tiles, 1), dim3(ks * 64), (size_t)ks * 1024, st, a);
+    else hipLaunchKernelGGL((gemm_skinny_bf16_kernel<1, 1, 4, EPI_LN_RESID, OutT>), dim3(tiles, cdiv(a.M, 16)), dim3(ks * 64), (size_t)ks * 1024, st, a);
+    return true;
 }
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int EPI, typename OutT>
@@ -2015,6 +2135,13 @@ static inline bool launch_gemm_mid(hipStream_t st, const GemmArgs& a) {
 
 template <int EPI, typename OutT>
 void launch_gemm_bf16(hipStream_t st, const GemmArgs& a) {
+    if constexpr (epi_ln(EPI)) {
+        bool ok = a.M <= 64;
+        if constexpr (EPI == EPI_LN_RESID) ok = ok && launch_gemm_ln_resid<OutT>(st, a);
+        else ok = ok && launch_gemm_skinny_bf16<EPI, OutT>(st, a);
+        if (!ok) throw std::runtime_error("gemm: a deferred layer norm did not fit the decode kernels");
+        return;
+    } else {
     if (a.tile_map) { launch_gemm_grouped<EPI, OutT>(st, a, a.M); return; }   // a.M carries the m-tile bound
     if (launch_gemm_mid<EPI, OutT>(st, a)) return;
     if (launch_gemm_skinny_bf16<EPI, OutT>(st, a)) return;
@@ -2058,6 +2185,7 @@ void launch_gemm_bf16(hipStream_t st, const GemmArgs& a) {
     if (tile == 3) launch_gemm_tile<256, 256, 2, 4, 2, EPI, OutT>(st, a);
     else if (tile == 2) launch_gemm_tile<256, 128, 4, 2, 3, EPI, OutT>(st, a);
     else launch_gemm_tile<128, 128, 2, 2, 2, EPI, OutT>(st, a);
+    }
 }
 
 template <int EPI, typename OutT>
@@ -2070,7 +2198,7 @@ void launch_gemm_f32(hipStream_t st, const GemmArgs& a) {
 #define NVL_GEMM_BF16_INSTANCES(X)                                                                                              \
     X(EPI_STORE, float) X(EPI_STORE, bf16_t) X(EPI_RESID, float) X(EPI_SWIGLU, bf16_t) X(EPI_GELU, bf16_t) X(EPI_GEGLU, bf16_t) \
     X(EPI_CLAMP_GLU, bf16_t) X(EPI_QKV, bf16_t) X(EPI_GROUPED, bf16_t) X(EPI_RELU2, bf16_t) X(EPI_GELU_TOK, bf16_t) \
-    X(EPI_REGLU, bf16_t) X(EPI_GROUPED_RAW, bf16_t)
+    X(EPI_REGLU, bf16_t) X(EPI_GROUPED_RAW, bf16_t) X(EPI_LN_STORE, float) X(EPI_LN_RESID, float) X(EPI_LN_GELU, bf16_t) X(EPI_LN_QKV, bf16_t)
 #define NVL_GEMM_F32_INSTANCES(X) X(EPI_STORE) X(EPI_RESID) X(EPI_GELU)
 #ifndef NVL_GEMM_INST
 #define NVL_X(E, T) extern template void launch_gemm_bf16<E, T>(hipStream_t, const GemmArgs&);

@@ -14,7 +14,7 @@ template void launch_gemm_bf16<EPI_STORE, float>(hipStream_t, const GemmArgs&);
 template void launch_gemm_bf16<EPI_STORE, bf16_t>(hipStream_t, const GemmArgs&);
 #else
 constexpr int INST = NVL_GEMM_INST - 1;
-using InstT = std::conditional_t<INST == EPI_RESID, float, bf16_t>;
+using InstT = std::conditional_t<INST == EPI_RESID || INST == EPI_LN_RESID || INST == EPI_LN_STORE, float, bf16_t>;
 template void launch_gemm_bf16<INST, InstT>(hipStream_t, const GemmArgs&);
 #endif
 }  // namespace nvl

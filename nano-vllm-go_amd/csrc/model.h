@@ -36,6 +36,7 @@ struct LayerW {
     // frozen by finalize()
     void* w_qkv = nullptr; int n_qkv = 0; float* b_qkv = nullptr;
     void* w1 = nullptr; int n1 = 0;      // fused rows (2F for SwiGLU, F for GELU)
+    float *ln_qkv = nullptr, *ln_up = nullptr;      // deferred layer norms (nvl_model::ln_ok): S, then B of the projection behind each norm
     void* moe_in = nullptr;              // [E][2I (interleaved in bf16 mode)][H]
     void* moe_out_cat = nullptr;         // bf16: W_down of all experts along K, [H_pad][E*I] (decode "dense-masked" form)
     bool mamba = false;                  // a Mamba2 block (attention tensors absent); index among the Mamba2 layers
@@ -226,6 +227,9 @@ struct nvl_model {
     void* moe_xg = nullptr;           // bf16: the normed rows in expert order, fragment-major [round_up(Mmax*k, 64)][H] (prefill)
     int32_t *moe_counts = nullptr, *moe_cursor = nullptr, *moe_tile_map = nullptr, *moe_n_mtiles = nullptr;
     // decode split-K: partial slices of the last residual GEMM, consumed by the next norm launch
+    // deferred layer norms (gemm.h GemmArgs::ln_s): the weights' sums are there; the second buffer of partial sums, the rows' means [2][64]
+    bool ln_ok = false;
+    float *ln_part = nullptr, *ln_mean = nullptr;
     float* rs_part = nullptr;    // deferred RMSNorm: [H/16][64] partial sums of x^2 (gemm.h)
     int ctx_hint = 0;    // longest context (keys) of the batch being enqueued; 0 = unknown (decode attention sizing)
     float* sk_part = nullptr; int sk_max_slices = 4; int pending_slices = 0, pending_rows = 0; float pending_alpha = 1.f; const float* pending_part = nullptr;

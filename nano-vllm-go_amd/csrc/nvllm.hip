@@ -177,7 +177,7 @@ void gemm(nvl_model* m, int epi, bool out_f32, GemmArgs a, double flops = -1.0) 
     a.stamps = (m->stamping && !m->f32 && a.M <= 64 && !a.tile_map) ? next_stamps(m, m->site, STAMP_MAX_WG) : nullptr;
     // algorithmic bytes of a projection: every weight byte once + the activation operand + the output rows
     const double gbytes = m->site_bytes > 0 ? m->site_bytes
-        : ((double)a.N * a.K + (double)a.M * a.K) * (double)m->wsize + (double)a.M * a.N * (out_f32 || epi == EPI_RESID ? 4.0 : (double)m->wsize);
+        : ((double)a.N * a.K + (double)a.M * a.K) * (double)m->wsize + (double)a.M * a.N * (out_f32 || epi_base(epi) == EPI_RESID ? 4.0 : (double)m->wsize);
     KScope ks(m, KC_GEMM, flops >= 0 ? flops : 2.0 * (double)a.M * (double)a.N * (double)a.K, -1, gbytes);
     hipStream_t st = m->stream;
     a.split_ws = m->split_ws; a.split_cnt = m->split_cnt; a.split_units = (int)(m->split_bytes / SPLIT_UNIT); a.splits = 1;
@@ -205,6 +205,10 @@ void gemm(nvl_model* m, int epi, bool out_f32, GemmArgs a, double flops = -1.0) 
             case EPI_GELU_TOK: launch_gemm_bf16<EPI_GELU_TOK, bf16_t>(st, a); break;
             case EPI_REGLU: launch_gemm_bf16<EPI_REGLU, bf16_t>(st, a); break;
             case EPI_GROUPED_RAW: launch_gemm_bf16<EPI_GROUPED_RAW, bf16_t>(st, a); break;
+            case EPI_LN_STORE: launch_gemm_bf16<EPI_LN_STORE, float>(st, a); break;
+            case EPI_LN_RESID: launch_gemm_bf16<EPI_LN_RESID, float>(st, a); break;
+            case EPI_LN_GELU: launch_gemm_bf16<EPI_LN_GELU, bf16_t>(st, a); break;
+            case EPI_LN_QKV: launch_gemm_bf16<EPI_LN_QKV, bf16_t>(st, a); break;
             default: throw std::runtime_error("gemm: bad epilogue");
         }
     }
@@ -371,14 +375,14 @@ extern "C" void nvl_destroy(nvl_model* m) {
     for (int k = 0; k < NVL_T_COUNT; k++) dfree(m->g[k].p);
     for (auto& l : m->layers) {
         for (int k = 0; k < NVL_T_COUNT; k++) dfree(l.t[k].p);
-        dfree(l.w_qkv); dfree(l.b_qkv); dfree(l.w1); dfree(l.moe_in); dfree(l.moe_out_cat);
+        dfree(l.w_qkv); dfree(l.b_qkv); dfree(l.w1); dfree(l.moe_in); dfree(l.moe_out_cat); dfree(l.ln_qkv); dfree(l.ln_up);
     }
     if (m->lm_head && m->lm_head != m->g[NVL_T_TOK_EMB].p && m->lm_head != m->g[NVL_T_LM_HEAD].p) dfree(m->lm_head);
     dfree(m->rope_cos); dfree(m->rope_sin); dfree(m->kcache); dfree(m->vcache);
     dfree(m->x); dfree(m->xn); dfree(m->qkv); dfree(m->q); dfree(m->attn_out); dfree(m->attn_part); dfree(m->attn_part_cnt); dfree(m->hbuf); dfree(m->h2);
     dfree(m->xn_last); dfree(m->logits); dfree(m->argmax_dev); dfree(m->argmax_pval); dfree(m->argmax_pidx); dfree(m->router_logits); dfree(m->expert_ids);
     dfree(m->expert_w); dfree(m->seg_start); dfree(m->moe_counts); dfree(m->moe_cursor); dfree(m->moe_tile_map); dfree(m->moe_n_mtiles); dfree(m->perm_token); dfree(m->slot_of); dfree(m->moe_eo); dfree(m->moe_xg);
-    dfree(m->meta_dev); dfree(m->hidden); dfree(m->sk_part); dfree(m->split_ws); dfree(m->split_cnt); dfree(m->tp_part); dfree(m->ring); dfree(m->rs_part);
+    dfree(m->meta_dev); dfree(m->hidden); dfree(m->sk_part); dfree(m->split_ws); dfree(m->split_cnt); dfree(m->tp_part); dfree(m->ring); dfree(m->rs_part); dfree(m->ln_part); dfree(m->ln_mean);
     for (int r = 0; r < 8; r++) if (m->p2p_peer[r] && m->p2p_peer[r] != m->p2p_buf) (void)hipIpcCloseMemHandle(m->p2p_peer[r]);
     p2p_give_back(m->p2p_buf, m->p2p_bytes);
     dfree(m->moe_gate); dfree(m->moe_hall); dfree(m->moe_part);
@@ -696,6 +700,31 @@ void init_meta(nvl_model* m) {
     m->ring_pos0 = dmalloc<int32_t>(S);
 }
 
+int64_t ln_rows(int64_t N) { return round_up(N, 16); }      // (whole weight tiles)
+// layer norms that the projection in front of them carries: what the projections behind them need of the weights, once
+void init_deferred_layer_norms(nvl_model* m) {
+    const nvl_model_config& c = m->cfg;
+    const int H = m->H;
+    m->ln_ok = !m->f32 && c.norm_type == NVL_NORM_LAYER && c.block_style == NVL_BLOCK_SEQUENTIAL && c.activation_type != NVL_ACT_SWIGLU && !c.use_moe && m->n_mamba == 0 && m->tp == 1 &&
+               !m->tp_force && H % 256 == 0 && H <= 1024 * NORM_ROW_MAXCH && m->F % 32 == 0;
+    for (auto& l : m->layers) m->ln_ok = m->ln_ok && l.t[NVL_T_ATTN_NORM_B].present() && l.t[NVL_T_FFN_NORM_B].present();
+    if (!m->ln_ok) return;
+    auto fold = [&](const void* W, int N, const DevTensor& w, const DevTensor& b, const float* bias) {
+        const int64_t np = ln_rows(N);
+        float* out = dmalloc<float>(2 * np);
+        hipLaunchKernelGGL(ln_fold_kernel, dim3((unsigned)(np / 16)), dim3(64), 0, m->stream, (const bf16_t*)W, (const float*)w.p, (const float*)b.p, bias, out, out + np, N, H);
+        NVL_HIP(hipGetLastError());
+        return out;
+    };
+    for (auto& l : m->layers) {
+        l.ln_qkv = fold(l.w_qkv, m->n_qkv, l.t[NVL_T_ATTN_NORM_W], l.t[NVL_T_ATTN_NORM_B], l.b_qkv);
+        l.ln_up = fold(l.w1, m->F, l.t[NVL_T_FFN_NORM_W], l.t[NVL_T_FFN_NORM_B], (const float*)l.t[NVL_T_B1].p);
+    }
+    m->ln_part = dmalloc<float>((int64_t)cdiv(H, 8) * 128);
+    m->ln_mean = dmalloc<float>(128);
+    NVL_HIP(hipMemsetAsync(m->ln_mean, 0, 128 * sizeof(float), m->stream));
+}
+
 }  // namespace
 
 extern "C" int nvl_finalize(nvl_model* m) {
@@ -917,6 +946,7 @@ extern "C" int nvl_finalize(nvl_model* m) {
     init_split(m);
     if (!m->f32) m->rs_part = dmalloc<float>((int64_t)cdiv(H, 8) * DEFER_MAX_M);      // x^2 partials per 16 (half tiles: 8) columns
     if (m->tp > 1 || m->tp_force) m->tp_part = dmalloc<float>(Mmax * H);
+    init_deferred_layer_norms(m);
     init_meta(m);
     NVL_HIP(hipStreamSynchronize(m->stream));   // every memset/copy above ran on the model's own (non-blocking) stream
     m->finalized = true;
@@ -1199,7 +1229,7 @@ static int g_norm_t16 = 1;     // nvl_set_tuning key 9: norm_tile_kernel for pre
 constexpr int NORM_ROW_KERNEL_ROWS = 1024;
 template <typename ActT>
 void launch_norm(nvl_model* m, float* x, const int32_t* rows_idx, const float* w, const float* b,
-                 void* y, int rows, bf16_t* y_rows = nullptr) {
+                 void* y, int rows, bf16_t* y_rows = nullptr, float* mean_out = nullptr) {
     KScope ks(m, KC_OTHER, 0, KS_NORM, (double)rows * m->H * (4.0 + (double)m->wsize));
     PendingResid pr{nullptr, 0, 0, 0.f, nullptr, nullptr};
     if (m->pending_slices > 0) {            // complete the residual add the previous decode GEMM left as split-K slices
@@ -1213,7 +1243,7 @@ void launch_norm(nvl_model* m, float* x, const int32_t* rows_idx, const float* w
     const bool tiles = sizeof(ActT) == 2 && m->H % 32 == 0 && m->H <= 4608 && g_norm_t16 && !pr.slot_of && (!pr.part || m->H <= 2048);
     if (rows <= (tiles && !y_rows ? NORM_ROW_KERNEL_ROWS : 512) && m->H <= 1024 * NORM_ROW_MAXCH)
         hipLaunchKernelGGL((norm_row_kernel<ActT>), dim3(rows), dim3(256), 0, m->stream, x, rows_idx, w, b,
-                           m->cfg.norm_eps, (ActT*)y, m->H, pr);
+                           m->cfg.norm_eps, (ActT*)y, m->H, pr, mean_out);
     else if (tiles) {   // (two workgroups' tiles of wider rows would not fit the LDS of a CU: norm_kernel)
         // 8 rows x H bf16 of LDS (up to 73 KiB); the row sits in registers: instance by chunks per lane
 #define NVL_NT(CH, PEND)                                                                                             \
@@ -1232,9 +1262,9 @@ void launch_norm(nvl_model* m, float* x, const int32_t* rows_idx, const float* w
 }
 // does the norm of so many rows leave a row-major copy of its result (y_rows) too?
 bool norm_copies_rows(const nvl_model* m, int rows) { return !m->f32 && rows > 512 && m->H % 32 == 0 && m->H <= 4608 && g_norm_t16; }
-void norm(nvl_model* m, float* x, const int32_t* rows_idx, const DevTensor& w, const DevTensor& b, void* y, int rows, bf16_t* y_rows = nullptr) {
+void norm(nvl_model* m, float* x, const int32_t* rows_idx, const DevTensor& w, const DevTensor& b, void* y, int rows, bf16_t* y_rows = nullptr, float* mean_out = nullptr) {
     if (m->f32) launch_norm<float>(m, x, rows_idx, (const float*)w.p, (const float*)b.p, y, rows);
-    else launch_norm<bf16_t>(m, x, rows_idx, (const float*)w.p, (const float*)b.p, y, rows, y_rows);
+    else launch_norm<bf16_t>(m, x, rows_idx, (const float*)w.p, (const float*)b.p, y, rows, y_rows, mean_out);
     NVL_HIP(hipGetLastError());
 }
 
@@ -1598,9 +1628,31 @@ void resid_gemm(nvl_model* m, const void* A, int lda, const void* W, const float
     }
 }
 
+// Deferred layer norms of a pass (gemm.h GemmArgs::ln_s).  Two buffers in turn: a projection reads the norm before its own and writes its own.
+struct LnChain { int cur = 0; bool have = false; };      // where the last norm's means are (ln_mean), and its sums, if a projection carried it
+float* ln_buf(const nvl_model* m, int i) { return i ? m->ln_part : m->rs_part; }
+void set_ln_stats(const nvl_model* m, GemmArgs& a) {
+    a.rs_half = defer_half(m, a.M) ? 1 : 0;
+    a.rs_tiles = a.rs_half ? m->H / 8 : m->H / 16; a.rs_inv_h = 1.0f / (float)m->H; a.rs_eps = m->cfg.norm_eps;
+}
+void ln_resid_gemm(nvl_model* m, LnChain& ln, const void* A, int lda, const void* W, const float* bias, int M, int K, const DevTensor& norm_w) {
+    GemmArgs a = mk(A, lda, W, m->x, m->H, bias, m->resid_alpha, M, m->H, K);
+    set_ln_stats(m, a);
+    a.nrm_w = (const float*)norm_w.p; a.nrm_xn = (bf16_t*)m->xn; a.rs_out = ln_buf(m, ln.cur ^ 1);
+    a.ln_prev = ln.have ? ln_buf(m, ln.cur) : nullptr; a.ln_mean_in = m->ln_mean + 64 * ln.cur; a.ln_mean_out = m->ln_mean + 64 * (ln.cur ^ 1);
+    gemm(m, EPI_LN_RESID, true, a);
+    ln.cur ^= 1; ln.have = true;
+}
+// `sums`: S, then B
+void set_ln_in(const nvl_model* m, const LnChain& ln, GemmArgs& a, const float* sums) {
+    set_ln_stats(m, a);
+    a.rs_half = 0;
+    a.rs_in = ln_buf(m, ln.cur); a.ln_s = sums; a.bias = sums + ln_rows(a.N);
+}
+
 // FeedForward.Forward (transformer.go:40-96) up to (not including) the W2 projection:
 // leaves act(x·W1) in m->hbuf [M][F]
-void ffn_up(nvl_model* m, const LayerW& l, int M, bool deferred_norm = false) {
+void ffn_up(nvl_model* m, const LayerW& l, int M, bool deferred_norm = false, const LnChain* ln = nullptr) {
     const bool swiglu = m->cfg.activation_type == NVL_ACT_SWIGLU;
     const float* b1 = (const float*)l.t[NVL_T_B1].p;
     if (swiglu) {
@@ -1619,8 +1671,10 @@ void ffn_up(nvl_model* m, const LayerW& l, int M, bool deferred_norm = false) {
             gemm(m, EPI_SWIGLU, false, a);
         }
     } else {
+        GemmArgs a = mk(m->xn, m->H, l.w1, m->hbuf, m->F, b1, 1.f, M, m->F, m->H);
+        if (ln) set_ln_in(m, *ln, a, l.ln_up);
         m->site = KS_FFN_UP;
-        gemm(m, EPI_GELU, false, mk(m->xn, m->H, l.w1, m->hbuf, m->F, b1, 1.f, M, m->F, m->H));
+        gemm(m, ln ? EPI_LN_GELU : EPI_GELU, false, a);
     }
 }
 
@@ -1920,6 +1974,9 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
     const bool defer_moe_ok = g_defer_norm && c.use_moe && M <= 64 && m->tp == 1 && !m->tp_force && c.block_style == NVL_BLOCK_SEQUENTIAL &&
                               c.norm_type == NVL_NORM_RMS && H % 256 == 0 && m->rs_part && m->n_mamba == 0;
     const bool all_rows = (flags & NVL_FWD_ALL_LOGITS) != 0;
+    // layer norms of up to 64 rows, the same
+    const bool ln_defer = m->ln_ok && g_defer_norm == 1 && defer_tiles() && g_force_tile == 0 && M <= 64 && !m->keep_hidden;
+    LnChain ln;
     bool xn_deferred = false;       // m->xn holds xn_raw of the upcoming norm, m->rs_part its x^2 partials
     for (int li = 0; li < m->L && !m->layered; li++) {
         const LayerW& l = m->layers[li];
@@ -2043,7 +2100,7 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
         }
         const bool qkv_deferred = xn_deferred;
         if (!xn_deferred && !(li == 0 && (seam & 1)))
-            norm(m, m->x, nullptr, l.t[NVL_T_ATTN_NORM_W], l.t[NVL_T_ATTN_NORM_B], m->xn, M);
+            norm(m, m->x, nullptr, l.t[NVL_T_ATTN_NORM_W], l.t[NVL_T_ATTN_NORM_B], m->xn, M, nullptr, ln_defer ? m->ln_mean : nullptr);
         xn_deferred = false;
         bool fused_dec = false;
         // a decode batch of 64 < M <= g_chunk_max_m rows keeps the decode form (64-row passes, gemm.h) and the fused
@@ -2052,19 +2109,19 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
         const bool store_rows = max_len > 1 && qkv_rows(M, m->n_qkv, H) && M <= g_chunk_max_m && g_force_tile == 0;
         if (!m->f32 && (M > 64 ? !big_decode : max_len > 1 && m->hd % 32 == 0) && !store_rows) {
             GemmArgs a = mk(m->xn, H, l.w_qkv, nullptr, 0, l.b_qkv, 1.f, M, m->n_qkv, H);
-            if (qkv_deferred) set_deferred_in(m, a);
+            if (qkv_deferred) { if (ln_defer) set_ln_in(m, ln, a, l.ln_qkv); else set_deferred_in(m, a); }
             a.qkv.tok_pos = md.tok_pos; a.qkv.tok_tbl = md.tok_tbl; a.qkv.blk_table = md.blk_table; a.qkv.cos_t = m->rope_cos; a.qkv.sin_t = m->rope_sin;
             a.qkv.q_out = (bf16_t*)m->q;
             a.qkv.kcache = (bf16_t*)m->kcache + (int64_t)li * m->layer_stride;
             a.qkv.vcache = (bf16_t*)m->vcache + (int64_t)li * m->layer_stride;
             a.qkv.slot_stride = m->slot_stride; a.qkv.Tmax = m->Tmax; a.qkv.nH = m->nH; a.qkv.nKV = m->nKV; a.qkv.hd = m->hd;
             m->site = KS_QKV;
-            gemm(m, EPI_QKV, false, a);
+            gemm(m, qkv_deferred && ln_defer ? EPI_LN_QKV : EPI_QKV, false, a);
         } else {
             GemmArgs aq = mk(m->xn, H, l.w_qkv, m->qkv, m->n_qkv, l.b_qkv, 1.f, M, m->n_qkv, H);
-            if (qkv_deferred) set_deferred_in(m, aq);
+            if (qkv_deferred) { if (ln_defer) set_ln_in(m, ln, aq, l.ln_qkv); else set_deferred_in(m, aq); }
             m->site = KS_QKV;
-            gemm(m, EPI_STORE, true, aq);
+            gemm(m, qkv_deferred && ln_defer ? EPI_LN_STORE : EPI_STORE, true, aq);
             fused_dec = !m->f32 && max_len == 1;     // decode: RoPE + KV append live in the attention kernel
             if (!fused_dec) rope_kv(m, li, md, M);
         }
@@ -2084,7 +2141,9 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
             const bool defer = (defer_ok || (defer_moe_ok && moe_dense_ok(m, l, M))) && m->pending_slices == 0 && !l.t[NVL_T_FFN_NORM_B].present();
             m->site = KS_OPROJ;
             bf16_t* xn_rows = c.use_moe && !defer && norm_copies_rows(m, M) ? (bf16_t*)m->moe_eo : nullptr;      // (for the copy into expert order)
-            if (defer) {
+            if (ln_defer) {
+                ln_resid_gemm(m, ln, m->attn_out, qw, l.t[NVL_T_WO].p, bo, M, qw, l.t[NVL_T_FFN_NORM_W]);
+            } else if (defer) {
                 resid_gemm(m, m->attn_out, qw, l.t[NVL_T_WO].p, bo, m->resid_alpha, M, H, qw, (const float*)l.t[NVL_T_FFN_NORM_W].p);
             } else {
                 resid_gemm(m, m->attn_out, qw, l.t[NVL_T_WO].p, bo, m->resid_alpha, M, H, qw);
@@ -2098,6 +2157,13 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
                 const bool defer2 = defer && defer_moe_ok && g_defer_norm != 3 && !nxt_b->present() &&
                                     (li + 1 < m->L || (!all_rows && M == n_seqs && M <= 64));
                 xn_deferred = moe(m, l, M, defer, defer2 ? (const float*)nxt_w->p : nullptr, xn_rows);
+            } else if (ln_defer) {
+                ffn_up(m, l, M, false, &ln);
+                // (not the final norm: every workgroup of the LM head would add up the rows' sums: GPT-2 at 1 / 16 rows 14.4 -> 18.1, 15.7 -> 22.0 us)
+                xn_deferred = li + 1 < m->L;
+                m->site = KS_FFN_DOWN;
+                if (xn_deferred) ln_resid_gemm(m, ln, m->hbuf, m->F, l.t[NVL_T_W2].p, (const float*)l.t[NVL_T_B2].p, M, m->F, *nxt_w);
+                else resid_gemm(m, m->hbuf, m->F, l.t[NVL_T_W2].p, (const float*)l.t[NVL_T_B2].p, m->resid_alpha, M, H, m->F);
             } else {
                 ffn_up(m, l, M, defer);
                 const bool defer2 = defer_ok && g_defer_norm != 3 && m->pending_slices == 0 && !nxt_b->present() &&
@@ -2517,7 +2583,7 @@ void decode_loop(nvl_model* m, const Meta& hm, int n_seqs, int n_steps, int32_t*
                                md.seq_pos, (const bf16_t*)m->g[NVL_T_TOK_EMB].p, (const bf16_t*)pe, pe_rows,
                                m->cfg.embedding_multiplier, m->x, norm0, bias0, m->cfg.norm_eps, (bf16_t*)m->xn, m->H, m->Hn,
                                m->cfg.token_shift ? SeamShift{m->mixers[(size_t)m->runs[0].owner].shift, m->rec_state + m->runs[0].shift_off, m->rec_slot_stride, md.seq_slot}
-                                                  : SeamShift{});
+                                                  : SeamShift{}, m->ln_ok && n_seqs <= 64 ? m->ln_mean : (float*)nullptr);
         } else {
             hipLaunchKernelGGL(advance_decode_kernel, dim3(cdiv(n_seqs, 256)), dim3(256), 0, m->stream, m->argmax_dev, md.tokens,
                                md.tok_pos, md.seq_pos, m->ring + (int64_t)s * n_seqs, n_seqs);
