@@ -1977,6 +1977,7 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
     // layer norms of up to 64 rows, the same
     const bool ln_defer = m->ln_ok && g_defer_norm == 1 && defer_tiles() && g_force_tile == 0 && M <= 64 && !m->keep_hidden;
     LnChain ln;
+    const bool last_rows_only = !all_rows && m->rows_named < 0 && M == n_seqs && M <= 64;      // the LM head takes every row of the batch, in order
     bool xn_deferred = false;       // m->xn holds xn_raw of the upcoming norm, m->rs_part its x^2 partials
     for (int li = 0; li < m->L && !m->layered; li++) {
         const LayerW& l = m->layers[li];
@@ -2092,7 +2093,7 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
             ffn_up(m, l, M, defer);
             const DevTensor& nxt_w = li + 1 < m->L ? m->layers[li + 1].t[NVL_T_ATTN_NORM_W] : m->g[NVL_T_FINAL_NORM_W];
             const DevTensor& nxt_b = li + 1 < m->L ? m->layers[li + 1].t[NVL_T_ATTN_NORM_B] : m->g[NVL_T_FINAL_NORM_B];
-            xn_deferred = defer && g_defer_norm != 3 && m->pending_slices == 0 && !nxt_b.present() && (li + 1 < m->L || (!all_rows && M == n_seqs && M <= 64));
+            xn_deferred = defer && g_defer_norm != 3 && m->pending_slices == 0 && !nxt_b.present() && (li + 1 < m->L || last_rows_only);
             m->site = KS_FFN_DOWN;
             resid_gemm(m, m->hbuf, m->F, l.t[NVL_T_W2].p, (const float*)l.t[NVL_T_B2].p, m->resid_alpha, M, H, m->F, xn_deferred ? (const float*)nxt_w.p : nullptr);
             tap_layer(m, li, M);
@@ -2155,7 +2156,7 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
             const DevTensor* nxt_b = li + 1 < m->L ? &m->layers[li + 1].t[NVL_T_ATTN_NORM_B] : &m->g[NVL_T_FINAL_NORM_B];
             if (c.use_moe) {
                 const bool defer2 = defer && defer_moe_ok && g_defer_norm != 3 && !nxt_b->present() &&
-                                    (li + 1 < m->L || (!all_rows && M == n_seqs && M <= 64));
+                                    (li + 1 < m->L || last_rows_only);
                 xn_deferred = moe(m, l, M, defer, defer2 ? (const float*)nxt_w->p : nullptr, xn_rows);
             } else if (ln_defer) {
                 ffn_up(m, l, M, false, &ln);
@@ -2167,7 +2168,7 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
             } else {
                 ffn_up(m, l, M, defer);
                 const bool defer2 = defer_ok && g_defer_norm != 3 && m->pending_slices == 0 && !nxt_b->present() &&
-                                    (li + 1 < m->L || (!all_rows && M == n_seqs && M <= 64));   // (the LM head of a larger batch runs on the tile kernels)
+                                    (li + 1 < m->L || last_rows_only);   // (the LM head of a larger batch runs on the tile kernels)
                 m->site = KS_FFN_DOWN;
                 resid_gemm(m, m->hbuf, m->F, l.t[NVL_T_W2].p, (const float*)l.t[NVL_T_B2].p, m->resid_alpha, M, H, m->F,
                            defer2 ? (const float*)nxt_w->p : nullptr);
