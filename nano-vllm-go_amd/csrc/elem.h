@@ -1391,13 +1391,14 @@ __device__ __forceinline__ float ld_as_f32(const void* p, int dtype, int64_t i) 
 // of the logical [SN][SK] source, stored IN_OUT ([SK][SN]) or OUT_IN ([SN][SK]).  The sub-block form is how a
 // tensor-parallel rank takes its shard while the tensor is converted; FM selects the fragment-major
 // destination layout (bf16 MFMA operands), else row-major.
-struct Slice2D { int64_t SN, SK, sn0, sk0, dn0; };
+struct Slice2D { int64_t SN, SK, sn0, sk0, dn0, Kd, col0; };      // Kd: columns of the destination (0: K), col0: its first
 template <typename DT, bool FM>
 __global__ void convert_2d_kernel(const void* __restrict__ src, int dtype, int transpose_in,
                                   DT* __restrict__ dst, int64_t N, int64_t K, Slice2D sl) {
     __shared__ float tile[32][33];
     const int64_t n0 = (int64_t)blockIdx.y * 32, k0 = (int64_t)blockIdx.x * 32;
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;   // 256 threads: 8 rows per pass
+    const int64_t Kd = sl.Kd ? sl.Kd : K;
     if (transpose_in) {
         for (int r = ty; r < 32; r += 8) {
             const int64_t k = k0 + r, n = n0 + tx;
@@ -1406,13 +1407,13 @@ __global__ void convert_2d_kernel(const void* __restrict__ src, int dtype, int t
         __syncthreads();
         for (int r = ty; r < 32; r += 8) {
             const int64_t n = n0 + r, k = k0 + tx;
-            if (n < N && k < K) dst[FM ? fm_index(sl.dn0 + n, k, K) : (sl.dn0 + n) * K + k] = (DT)tile[tx][r];
+            if (n < N && k < K) dst[FM ? fm_index(sl.dn0 + n, sl.col0 + k, Kd) : (sl.dn0 + n) * Kd + sl.col0 + k] = (DT)tile[tx][r];
         }
     } else {
         for (int r = ty; r < 32; r += 8) {
             const int64_t n = n0 + r, k = k0 + tx;
             if (n < N && k < K)
-                dst[FM ? fm_index(sl.dn0 + n, k, K) : (sl.dn0 + n) * K + k] =
+                dst[FM ? fm_index(sl.dn0 + n, sl.col0 + k, Kd) : (sl.dn0 + n) * Kd + sl.col0 + k] =
                     (DT)ld_as_f32(src, dtype, (sl.sn0 + n) * sl.SK + sl.sk0 + k);
         }
     }

@@ -51,10 +51,11 @@ enum GemmEpi {
     EPI_GELU_TOK = 8,    // C[m, n] = gelu_tanh(acc) * tok_table[tok_ids[m]][n]   (an input of the token's own, GemmArgs::tok_*)
     // ... with a deferred layer norm (GemmArgs::ln_s): decode kernels alone
     EPI_LN_STORE = 12, EPI_LN_RESID = 13, EPI_LN_GELU = 14, EPI_LN_QKV = 15,
+    EPI_JOINT = 16,      // two projections of one operand: the first joint.n columns are stored to fp32 rows, the others C = gelu_tanh(acc + bias)
 };
-constexpr bool epi_ln(int epi) { return epi >= 12; }
+constexpr bool epi_ln(int epi) { return epi >= 12 && epi <= 15; }
 constexpr int skinny_waves(int epi) { return epi_ln(epi) ? 8 : 16; }      // most waves of a workgroup of the narrow decode form (the pairs of a layer norm take registers)
-constexpr int epi_base(int epi) { return epi == 15 ? 4 : epi == 14 ? 3 : epi >= 12 ? epi - 12 : epi; }
+constexpr int epi_base(int epi) { return !epi_ln(epi) ? epi : epi == 15 ? 4 : epi == 14 ? 3 : epi - 12; }
 
 constexpr bool epi_moe(int epi) { return epi == 2 || epi == 6; }      // ... with instances for masked experts
 constexpr bool epi_glu(int epi) { return epi == 2 || epi == 5 || epi == 6 || epi == 10; }      // gate | up pairs in, one column out
@@ -93,6 +94,8 @@ struct RouteJob {
     int wgs, rows;
 };
 
+struct JointEpi { float* rows; int ld, n; };      // EPI_JOINT; n a multiple of 16
+
 struct GemmArgs {
     const void* A;          // bf16: fragment-major [M_pad16][K]; f32: row-major [M][lda]
     int lda;
@@ -121,6 +124,7 @@ struct GemmArgs {
     union {
         QkvEpi qkv;         // EPI_QKV
         RouteJob route;     // masked experts (epi_moe with moe_gate)
+        JointEpi joint;     // EPI_JOINT
     };
     GroupedEpi grp;         // EPI_GROUPED
     // decode kernel, EPI_RESID only: K split over gridDim.y = sk_slices workgroups per column block.  Each
@@ -253,7 +257,11 @@ __device__ __forceinline__ void epilogue4(const GemmArgs& p, int m, int n, f32x4
         for (int r = 0; r < 4; r++)
             if (n + r < p.N) v[r] += p.bias[n + r];
     }
-    if (EPI == EPI_GELU) {
+    if (EPI == EPI_JOINT) {
+        if (n < p.joint.n) { *(f32x4*)(p.joint.rows + ((int64_t)p.c_row0 + m) * p.joint.ld + n) = v; return; }
+        n -= p.joint.n;
+    }
+    if (EPI == EPI_GELU || EPI == EPI_JOINT) {
 #pragma unroll
         for (int r = 0; r < 4; r++) v[r] = gelu_tanh_f(v[r]);
     }
@@ -1924,7 +1932,7 @@ static inline bool launch_gemm_skinny_bf16(hipStream_t st, const GemmArgs& a0) {
     if (skinny_rows(a0) > 64 || a0.a_rows || a0.seg || a0.tile_map) return false;
     GemmArgs a = a0;
     a.x_mask = (g_x_mask && a0.M % 16 != 0) ? 1 : 0;     // padded rows of the last 16-row activation tile are not fetched
-    if constexpr (epi_glu(EPI) || EPI == EPI_STORE || EPI == EPI_GELU || EPI == EPI_RELU2 || EPI == EPI_GROUPED || EPI == EPI_GROUPED_RAW) {
+    if constexpr (epi_glu(EPI) || EPI == EPI_STORE || EPI == EPI_GELU || EPI == EPI_RELU2 || EPI == EPI_GROUPED || EPI == EPI_GROUPED_RAW || EPI == EPI_JOINT) {
         // wide-N form once its 64-row groups fill the chip (g_force_ntw: 8 forces it, 1/2/4 force the narrow form)
         const bool wide_ok = skinny_rows(a) > 16 && cdiv(a.N, 64) >= 256 && !a.sk_part;   // M <= 16: the narrow form streams as fast
         if (g_force_ntw == 8 || (g_force_ntw == 0 && wide_ok)) { if (launch_gemm_skinny_wide<EPI, OutT>(st, a)) return true; }
@@ -2198,7 +2206,8 @@ void launch_gemm_f32(hipStream_t st, const GemmArgs& a) {
 #define NVL_GEMM_BF16_INSTANCES(X)                                                                                              \
     X(EPI_STORE, float) X(EPI_STORE, bf16_t) X(EPI_RESID, float) X(EPI_SWIGLU, bf16_t) X(EPI_GELU, bf16_t) X(EPI_GEGLU, bf16_t) \
     X(EPI_CLAMP_GLU, bf16_t) X(EPI_QKV, bf16_t) X(EPI_GROUPED, bf16_t) X(EPI_RELU2, bf16_t) X(EPI_GELU_TOK, bf16_t) \
-    X(EPI_REGLU, bf16_t) X(EPI_GROUPED_RAW, bf16_t) X(EPI_LN_STORE, float) X(EPI_LN_RESID, float) X(EPI_LN_GELU, bf16_t) X(EPI_LN_QKV, bf16_t)
+    X(EPI_REGLU, bf16_t) X(EPI_GROUPED_RAW, bf16_t) X(EPI_LN_STORE, float) X(EPI_LN_RESID, float) X(EPI_LN_GELU, bf16_t) X(EPI_LN_QKV, bf16_t) \
+    X(EPI_JOINT, bf16_t)
 #define NVL_GEMM_F32_INSTANCES(X) X(EPI_STORE) X(EPI_RESID) X(EPI_GELU)
 #ifndef NVL_GEMM_INST
 #define NVL_X(E, T) extern template void launch_gemm_bf16<E, T>(hipStream_t, const GemmArgs&);

@@ -28,6 +28,7 @@ struct DevTensor {
     void* p = nullptr;      // canonical device copy: 2-D [rows_pad][cols] in weight dtype, 1-D fp32
     int64_t rows = 0, cols = 0, rows_pad = 0;
     int raw_dtype = -1;     // >= 0: a staged copy in the checkpoint's dtype, row-major (models described by a list of layers, before finalize)
+    int64_t ld = 0, row0 = 0, col0 = 0;      // ld > 0: rows from row0 and columns from col0 on of the matrix p of ld columns (LayerW::w_in, w_out, which own it)
     bool present() const { return p != nullptr; }
 };
 
@@ -36,6 +37,8 @@ struct LayerW {
     // frozen by finalize()
     void* w_qkv = nullptr; int n_qkv = 0; float* b_qkv = nullptr;
     void* w1 = nullptr; int n1 = 0;      // fused rows (2F for SwiGLU, F for GELU)
+    void *w_in = nullptr, *w_out = nullptr;         // parallel blocks (nvl_model::joint): QKV and W1 as one matrix (w_qkv and w1 point into it), WO and W2 side by side along K
+    float *b_in = nullptr, *b_out = nullptr;
     float *ln_qkv = nullptr, *ln_up = nullptr;      // deferred layer norms (nvl_model::ln_ok): S, then B of the projection behind each norm
     void* moe_in = nullptr;              // [E][2I (interleaved in bf16 mode)][H]
     void* moe_out_cat = nullptr;         // bf16: W_down of all experts along K, [H_pad][E*I] (decode "dense-masked" form)
@@ -227,6 +230,7 @@ struct nvl_model {
     void* moe_xg = nullptr;           // bf16: the normed rows in expert order, fragment-major [round_up(Mmax*k, 64)][H] (prefill)
     int32_t *moe_counts = nullptr, *moe_cursor = nullptr, *moe_tile_map = nullptr, *moe_n_mtiles = nullptr;
     // decode split-K: partial slices of the last residual GEMM, consumed by the next norm launch
+    bool joint = false;          // LayerW::w_in, w_out; hbuf holds attention and feed-forward side by side, [Mmax][nH hd + F]
     // deferred layer norms (gemm.h GemmArgs::ln_s): the weights' sums are there; the second buffer of partial sums, the rows' means [2][64]
     bool ln_ok = false;
     float *ln_part = nullptr, *ln_mean = nullptr;

@@ -205,6 +205,7 @@ void gemm(nvl_model* m, int epi, bool out_f32, GemmArgs a, double flops = -1.0) 
             case EPI_GELU_TOK: launch_gemm_bf16<EPI_GELU_TOK, bf16_t>(st, a); break;
             case EPI_REGLU: launch_gemm_bf16<EPI_REGLU, bf16_t>(st, a); break;
             case EPI_GROUPED_RAW: launch_gemm_bf16<EPI_GROUPED_RAW, bf16_t>(st, a); break;
+            case EPI_JOINT: launch_gemm_bf16<EPI_JOINT, bf16_t>(st, a); break;
             case EPI_LN_STORE: launch_gemm_bf16<EPI_LN_STORE, float>(st, a); break;
             case EPI_LN_RESID: launch_gemm_bf16<EPI_LN_RESID, float>(st, a); break;
             case EPI_LN_GELU: launch_gemm_bf16<EPI_LN_GELU, bf16_t>(st, a); break;
@@ -353,6 +354,16 @@ extern "C" int nvl_create(const nvl_model_config* cfg, const nvl_runtime_opts* o
         m->m_K = c.mamba_conv_kernel; m->m_hd = c.mamba_head_dim > 0 ? c.mamba_head_dim : m->mEH / m->m_nh;
         m->mConv = m->mEH + 2 * m->m_ng * m->m_ss; m->mP = m->mEH + m->mConv + m->m_nh;
     }
+    {
+        // Parallel blocks: both branches read one norm and end in one sum, so that a layer is two products, [QKV | W1] and [WO | W2], in place of four,
+        // where nothing stands between them: fp32 rows of queries and keys (decode steps, some prompts) on the way in, one multiplier on the way
+        // out.  Falcon-7B, us a layer at 5 rows: QKV 13.0 and W1 32.5 -> 35.4 (208 MB at 6 TB/s), WO 13.0 and W2 30.4 -> 36.7, and two boundaries less; ms of 12
+        // steps of 1 / 5 / 16 / 24 / 40 / 64 / 104 sequences: 39.6 -> 33.7, 39.7 -> 33.3, 41.9 -> 33.9, 43.6 -> 36.8, 51.4 -> 44.4, 56.5 -> 47.7, 70.2 -> 60.2; prompts
+        // of 11 / 40 / 200 / 800 / 4000 tokens 3.5 -> 3.2, 4.3 -> 3.7, 8.3 -> 8.0, 15.8 -> 14.2, 49.4 -> 47.2
+        const bool mults = c.attention_multiplier != 0.f && c.residual_multiplier != 0.f;
+        m->joint = !m->f32 && c.block_style == NVL_BLOCK_PARALLEL && c.activation_type != NVL_ACT_SWIGLU && !c.use_moe && m->n_mamba == 0 && m->tp == 1 && !m->tp_force &&
+                   !m->layered && (!mults || c.attention_multiplier == c.residual_multiplier) && m->H % 64 == 0 && m->n_qkv % 16 == 0 && m->nH * m->hd % 64 == 0 && m->F % 64 == 0;
+    }
     if (m->opts.max_batch_tokens <= 0) m->opts.max_batch_tokens = c.max_seq_len;
     *out = m;
     return NVL_OK;
@@ -367,6 +378,11 @@ extern "C" int nvl_create(const nvl_model_config* cfg, const nvl_runtime_opts* o
     }
 }
 
+namespace {
+// joint: the matrices of a layer that are parts of `whole`
+void forget_parts(LayerW& l, const void* whole) { for (auto& t : l.t) if (t.ld > 0 && t.p == whole) t.p = nullptr; }
+}  // namespace
+
 extern "C" void nvl_destroy(nvl_model* m) {
     if (!m) return;
     (void)hipSetDevice(m->device);
@@ -374,7 +390,11 @@ extern "C" void nvl_destroy(nvl_model* m) {
     layered_free(m);
     for (int k = 0; k < NVL_T_COUNT; k++) dfree(m->g[k].p);
     for (auto& l : m->layers) {
+        forget_parts(l, l.w_in);
+        forget_parts(l, l.w_out);
         for (int k = 0; k < NVL_T_COUNT; k++) dfree(l.t[k].p);
+        if (m->joint) l.w_qkv = l.w1 = nullptr;
+        dfree(l.w_in); dfree(l.w_out); dfree(l.b_in); dfree(l.b_out);
         dfree(l.w_qkv); dfree(l.b_qkv); dfree(l.w1); dfree(l.moe_in); dfree(l.moe_out_cat); dfree(l.ln_qkv); dfree(l.ln_up);
     }
     if (m->lm_head && m->lm_head != m->g[NVL_T_TOK_EMB].p && m->lm_head != m->g[NVL_T_LM_HEAD].p) dfree(m->lm_head);
@@ -417,13 +437,16 @@ namespace {
 // `sl` selects the sub-block of the uploaded tensor that lands in rows [dn0, dn0+N) (the whole tensor for
 // replicated kinds, this rank's shard for tensor-parallel kinds); total_rows sizes the destination.
 void upload_2d(nvl_model* m, DevTensor* t, const void* data, int dtype, int64_t N, int64_t K, bool src_is_in_out,
-               Slice2D sl, int64_t total_rows, bool first_piece) {
+               Slice2D sl, int64_t total_rows, bool first_piece, void* into = nullptr) {
     const size_t esz = dtype == NVL_DTYPE_F32 ? 4 : 2;
     const int64_t src_elems = sl.SN * sl.SK;
     void* raw = dmalloc_bytes(src_elems * (int64_t)esz);
     NVL_HIP(hipMemcpyAsync(raw, data, (size_t)src_elems * esz, hipMemcpyDefault, m->stream));
     const int64_t Npad = round_up(total_rows, W_ROW_PAD);
-    if (first_piece) {
+    if (into) {                  // a part of a matrix that is there
+        t->p = into; t->ld = sl.Kd; t->row0 = sl.dn0; t->col0 = sl.col0;
+        m->stats.weight_bytes += (double)N * K * m->wsize;
+    } else if (first_piece) {
         dfree(t->p);
         t->p = dmalloc_bytes(Npad * K * (int64_t)m->wsize);
         NVL_HIP(hipMemsetAsync(t->p, 0, (size_t)(Npad * K) * m->wsize, m->stream));
@@ -560,6 +583,21 @@ extern "C" int nvl_upload_tensor(nvl_model* m, int kind, int layer, const void* 
         return fail(m, NVL_ERR_INVALID, buf);
     }
     const bool io = layout == NVL_LAYOUT_IN_OUT;
+    const bool qkv_part = kind == NVL_T_WQ || (m->cfg.attention_type == NVL_ATTN_MQA ? kind == NVL_T_WKV : kind == NVL_T_WK || kind == NVL_T_WV);
+    if (m->joint && (qkv_part || kind == NVL_T_W1 || kind == NVL_T_WO || kind == NVL_T_W2)) {
+        LayerW& l = m->layers[(size_t)layer];
+        const int64_t H = m->H, qw = (int64_t)m->nH * m->hd, nkv = (int64_t)m->nKV * m->hd, ko = qw + m->F;
+        auto place = [&](void*& mat, int64_t mat_rows, int64_t mat_cols, int64_t row0, int64_t col0) {
+            if (!mat) {
+                mat = dmalloc_bytes(mat_rows * mat_cols * (int64_t)m->wsize);
+                NVL_HIP(hipMemsetAsync(mat, 0, (size_t)(mat_rows * mat_cols) * m->wsize, m->stream));
+            }
+            upload_2d(m, t, data, dtype, SN, SK, io, Slice2D{SN, SK, 0, 0, row0, mat_cols, col0}, SN, true, mat);
+        };
+        if (kind == NVL_T_WO || kind == NVL_T_W2) place(l.w_out, round_up(H, W_ROW_PAD), ko, 0, kind == NVL_T_WO ? 0 : qw);
+        else place(l.w_in, m->n_qkv + round_up((int64_t)m->F, W_ROW_PAD), H, kind == NVL_T_WQ ? 0 : kind == NVL_T_W1 ? m->n_qkv : kind == NVL_T_WV ? qw + nkv : qw, 0);
+        return NVL_OK;
+    }
     if (m->tp == 1) {
         upload_2d(m, t, data, dtype, SN, SK, io, Slice2D{SN, SK, 0, 0, 0}, SN, true);
         return NVL_OK;
@@ -700,6 +738,27 @@ void init_meta(nvl_model* m) {
     m->ring_pos0 = dmalloc<int32_t>(S);
 }
 
+// the biases of the joint matrices
+void join_biases(nvl_model* m, LayerW& l) {
+    const int64_t H = m->H, F = m->F, nq = m->n_qkv;
+    const DevTensor &b1 = l.t[NVL_T_B1], &bo = l.t[NVL_T_BO], &b2 = l.t[NVL_T_B2];
+    if (l.b_qkv || b1.present()) {
+        l.b_in = dmalloc<float>(nq + F);
+        NVL_HIP(hipMemsetAsync(l.b_in, 0, (size_t)(nq + F) * 4, m->stream));
+        if (l.b_qkv) NVL_HIP(hipMemcpyAsync(l.b_in, l.b_qkv, (size_t)nq * 4, hipMemcpyDeviceToDevice, m->stream));
+        if (b1.present()) NVL_HIP(hipMemcpyAsync(l.b_in + nq, b1.p, (size_t)F * 4, hipMemcpyDeviceToDevice, m->stream));
+    }
+    if (!bo.present() && !b2.present()) return;
+    std::vector<float> sum((size_t)H, 0.f), b((size_t)H);
+    for (const DevTensor* t : {&bo, &b2})
+        if (t->present()) {
+            NVL_HIP(hipMemcpy(b.data(), t->p, (size_t)H * 4, hipMemcpyDeviceToHost));
+            for (int64_t i = 0; i < H; i++) sum[(size_t)i] += b[(size_t)i];
+        }
+    l.b_out = dmalloc<float>(H);
+    NVL_HIP(hipMemcpy(l.b_out, sum.data(), (size_t)H * 4, hipMemcpyHostToDevice));
+}
+
 int64_t ln_rows(int64_t N) { return round_up(N, 16); }      // (whole weight tiles)
 // layer norms that the projection in front of them carries: what the projections behind them need of the weights, once
 void init_deferred_layer_norms(nvl_model* m) {
@@ -769,6 +828,9 @@ extern "C" int nvl_finalize(nvl_model* m) {
         // ---- fused QKV [n_qkv_pad][H]: rows Q | K | V (canonical rows are contiguous: plain copies)
         const int64_t nq = (int64_t)m->nH * hd, nkv = (int64_t)m->nKV * hd;
         const int64_t npad = round_up(m->n_qkv, W_ROW_PAD);
+        if (m->joint) {
+            l.w_qkv = l.w_in;
+        } else {
         l.w_qkv = dmalloc_bytes(npad * H * (int64_t)m->wsize);
         NVL_HIP(hipMemsetAsync(l.w_qkv, 0, (size_t)(npad * H) * m->wsize, m->stream));
         char* dst = (char*)l.w_qkv;
@@ -780,6 +842,7 @@ extern "C" int nvl_finalize(nvl_model* m) {
             NVL_HIP(hipMemcpyAsync(dst + nq * rowb, l.t[NVL_T_WK].p, nkv * rowb, hipMemcpyDeviceToDevice, m->stream));
             NVL_HIP(hipMemcpyAsync(dst + (nq + nkv) * rowb, l.t[NVL_T_WV].p, nkv * rowb, hipMemcpyDeviceToDevice, m->stream));
         }
+        }
         l.n_qkv = m->n_qkv;
         if (l.t[NVL_T_BQ].present() || l.t[NVL_T_BK].present() || l.t[NVL_T_BV].present()) {
             l.b_qkv = dmalloc<float>(m->n_qkv);
@@ -789,7 +852,7 @@ extern "C" int nvl_finalize(nvl_model* m) {
             if (l.t[NVL_T_BV].present()) NVL_HIP(hipMemcpyAsync(l.b_qkv + nq + nkv, l.t[NVL_T_BV].p, nkv * 4, hipMemcpyDeviceToDevice, m->stream));
         }
         NVL_HIP(hipStreamSynchronize(m->stream));
-        for (int k : {NVL_T_WQ, NVL_T_WK, NVL_T_WV, NVL_T_WKV}) { dfree(l.t[k].p); l.t[k].p = nullptr; }
+        if (!m->joint) for (int k : {NVL_T_WQ, NVL_T_WK, NVL_T_WV, NVL_T_WKV}) { dfree(l.t[k].p); l.t[k].p = nullptr; }
 
         // ---- FFN / MoE
         if (c.use_moe) {
@@ -830,6 +893,10 @@ extern "C" int nvl_finalize(nvl_model* m) {
                 l.w1 = dmalloc_bytes(np * H * (int64_t)m->wsize);
                 gather_rows(m, l.t[NVL_T_W1].p, idx, l.w1, H);
                 dfree(l.t[NVL_T_W1].p); l.t[NVL_T_W1].p = nullptr;
+            } else if (m->joint) {
+                l.w1 = (char*)l.w_in + (int64_t)m->n_qkv * H * m->wsize;
+                forget_parts(l, l.w_in);      // (WO and W2 can still be read back)
+                join_biases(m, l);
             } else {
                 l.w1 = l.t[NVL_T_W1].p; l.t[NVL_T_W1].p = nullptr;
             }
@@ -886,10 +953,11 @@ extern "C" int nvl_finalize(nvl_model* m) {
         NVL_HIP(hipMemsetAsync(m->attn_part_cnt, 0, (size_t)m->attn_records * sizeof(int32_t), m->stream));
     }
     const int64_t k = c.use_moe ? c.num_experts_per_tok : 1;
-    m->hbuf = dmalloc_bytes(round_up(Mmax * k, 64) * m->F * (int64_t)m->wsize);
+    const int64_t hw = m->F + (m->joint ? qw : 0);
+    m->hbuf = dmalloc_bytes(round_up(Mmax * k, 64) * hw * (int64_t)m->wsize);
     NVL_HIP(hipMemsetAsync(m->xn, 0, (size_t)(Mp * H) * m->wsize, m->stream));
     NVL_HIP(hipMemsetAsync(m->attn_out, 0, (size_t)(Mp * qw) * m->wsize, m->stream));
-    NVL_HIP(hipMemsetAsync(m->hbuf, 0, (size_t)(round_up(Mmax * k, 64) * m->F) * m->wsize, m->stream));
+    NVL_HIP(hipMemsetAsync(m->hbuf, 0, (size_t)(round_up(Mmax * k, 64) * hw) * m->wsize, m->stream));
     if (m->f32 && (c.activation_type == NVL_ACT_SWIGLU || c.use_moe)) m->h2 = dmalloc<float>(Mmax * k * 2 * m->F);
     m->xn_last = dmalloc_bytes(round_up(S, 64) * H * (int64_t)m->wsize);
     NVL_HIP(hipMemsetAsync(m->xn_last, 0, (size_t)(round_up(S, 64) * H) * m->wsize, m->stream));
@@ -941,7 +1009,7 @@ extern "C" int nvl_finalize(nvl_model* m) {
     // split-K partial slices of the residual projections: decode (<= 64 rows) and mid-size batches (<= SK_TILE_MAX_M rows)
     m->sk_rows = (int)std::min<int64_t>(std::max<int64_t>(Mmax, 64), SK_TILE_MAX_M);
     if (!m->f32) m->sk_part = dmalloc<float>((int64_t)std::max(m->sk_max_slices, SK_TILE_MAX_SLICES) * m->sk_rows * H);
-    for (auto [N, K] : {std::pair<int64_t, int64_t>{m->n_qkv, H}, {H, qw}, {c.activation_type == NVL_ACT_SWIGLU ? 2 * m->F : m->F, H}, {H, m->F}, {m->V, H}, {m->mP, H}, {H, m->mEH}})
+    for (auto [N, K] : {std::pair<int64_t, int64_t>{m->n_qkv, H}, {H, qw}, {c.activation_type == NVL_ACT_SWIGLU ? 2 * m->F : m->F, H}, {H, m->F}, {m->V, H}, {m->mP, H}, {H, m->mEH}, {H, m->joint ? qw + m->F : 0}})
         m->split_bytes = std::max(m->split_bytes, split_need(Mmax, N, K));
     init_split(m);
     if (!m->f32) m->rs_part = dmalloc<float>((int64_t)cdiv(H, 8) * DEFER_MAX_M);      // x^2 partials per 16 (half tiles: 8) columns
@@ -1343,7 +1411,7 @@ int attn_prefill_rows(const nvl_model* m, int n_seqs, int M) {
 void attention(nvl_model* m, int li, const Meta& md, int n_seqs, int M, int max_len, double flops, bool fused_qkv = false) {
     AttnArgs a{};
     a.q = m->q; a.q_stride = m->nH * m->hd;
-    a.out = m->attn_out; a.out_stride = m->nH * m->hd;
+    a.out = m->joint ? m->hbuf : m->attn_out; a.out_stride = m->nH * m->hd + (m->joint ? m->F : 0);
     a.kcache = (char*)m->kcache + (size_t)li * m->layer_stride * m->wsize;
     a.vcache = (char*)m->vcache + (size_t)li * m->layer_stride * m->wsize;
     a.slot_stride = m->slot_stride; a.Tmax = m->Tmax;
@@ -1650,6 +1718,9 @@ void set_ln_in(const nvl_model* m, const LnChain& ln, GemmArgs& a, const float* 
     a.rs_in = ln_buf(m, ln.cur); a.ln_s = sums; a.bias = sums + ln_rows(a.N);
 }
 
+// joint: where the feed-forward's part of hbuf begins (column blocks of 32)
+void* ffn_columns(const nvl_model* m) { return (bf16_t*)m->hbuf + (int64_t)(m->nH * m->hd >> 5) * 512; }
+
 // FeedForward.Forward (transformer.go:40-96) up to (not including) the W2 projection:
 // leaves act(x·W1) in m->hbuf [M][F]
 void ffn_up(nvl_model* m, const LayerW& l, int M, bool deferred_norm = false, const LnChain* ln = nullptr) {
@@ -1671,7 +1742,7 @@ void ffn_up(nvl_model* m, const LayerW& l, int M, bool deferred_norm = false, co
             gemm(m, EPI_SWIGLU, false, a);
         }
     } else {
-        GemmArgs a = mk(m->xn, m->H, l.w1, m->hbuf, m->F, b1, 1.f, M, m->F, m->H);
+        GemmArgs a = m->joint ? mk(m->xn, m->H, l.w1, ffn_columns(m), m->nH * m->hd + m->F, b1, 1.f, M, m->F, m->H) : mk(m->xn, m->H, l.w1, m->hbuf, m->F, b1, 1.f, M, m->F, m->H);
         if (ln) set_ln_in(m, *ln, a, l.ln_up);
         m->site = KS_FFN_UP;
         gemm(m, ln ? EPI_LN_GELU : EPI_GELU, false, a);
@@ -2103,7 +2174,7 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
         if (!xn_deferred && !(li == 0 && (seam & 1)))
             norm(m, m->x, nullptr, l.t[NVL_T_ATTN_NORM_W], l.t[NVL_T_ATTN_NORM_B], m->xn, M, nullptr, ln_defer ? m->ln_mean : nullptr);
         xn_deferred = false;
-        bool fused_dec = false;
+        bool fused_dec = false, up_done = false;
         // a decode batch of 64 < M <= g_chunk_max_m rows keeps the decode form (64-row passes, gemm.h) and the fused
         // decode attention
         // Prompts: RoPE + Q/K/V placement fused into the projection's epilogue (no fp32 qkv round trip, a launch less a layer), or not: qkv_rows
@@ -2121,8 +2192,13 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
         } else {
             GemmArgs aq = mk(m->xn, H, l.w_qkv, m->qkv, m->n_qkv, l.b_qkv, 1.f, M, m->n_qkv, H);
             if (qkv_deferred) { if (ln_defer) set_ln_in(m, ln, aq, l.ln_qkv); else set_deferred_in(m, aq); }
-            m->site = KS_QKV;
-            gemm(m, qkv_deferred && ln_defer ? EPI_LN_STORE : EPI_STORE, true, aq);
+            up_done = m->joint;
+            m->site = up_done ? KS_FFN_UP : KS_QKV;
+            if (up_done) {
+                GemmArgs a = mk(m->xn, H, l.w_in, ffn_columns(m), qw + m->F, l.b_in, 1.f, M, m->n_qkv + m->F, H);
+                a.joint = JointEpi{m->qkv, m->n_qkv, m->n_qkv};
+                gemm(m, EPI_JOINT, false, a);
+            } else gemm(m, qkv_deferred && ln_defer ? EPI_LN_STORE : EPI_STORE, true, aq);
             fused_dec = !m->f32 && max_len == 1;     // decode: RoPE + KV append live in the attention kernel
             if (!fused_dec) rope_kv(m, li, md, M);
         }
@@ -2131,7 +2207,13 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
         if (parallel) {
             // generic_model.go:395-418: r + [am*]attn + [rm*]ffn, both branches read the same normed x
             const bool mults = c.attention_multiplier != 0.f && c.residual_multiplier != 0.f;
-            ffn_up(m, l, M);
+            if (!up_done) ffn_up(m, l, M);
+            if (m->joint) {
+                m->site = KS_FFN_DOWN;
+                resid_gemm(m, m->hbuf, qw + m->F, l.w_out, l.b_out, mults ? c.attention_multiplier : 1.f, M, H, qw + m->F);
+                tap_layer(m, li, M);
+                continue;
+            }
             m->site = KS_OPROJ;
             resid_gemm(m, m->attn_out, qw, l.t[NVL_T_WO].p, bo, mults ? c.attention_multiplier : 1.f, M, H, qw);
             m->site = KS_FFN_DOWN;
@@ -2897,14 +2979,14 @@ extern "C" int nvl_get_weight(nvl_model* m, int kind, int layer, float* out, int
     NVL_TRY(m)
     NVL_HIP(hipSetDevice(m->device));
     NVL_HIP(hipStreamSynchronize(m->stream));
-    const int64_t N = t->rows, K = t->cols, n_el = t->rows_pad * K;
+    const int64_t N = t->rows, K = t->cols, ld = t->ld ? t->ld : K, n_el = (t->row0 + t->rows_pad) * ld;
     std::vector<char> raw((size_t)n_el * m->wsize);
     NVL_HIP(hipMemcpy(raw.data(), t->p, raw.size(), hipMemcpyDeviceToHost));
     for (int64_t n = 0; n < N; n++)
         for (int64_t k = 0; k < K; k++) {
             float v;
             if (m->f32) v = ((const float*)raw.data())[n * K + k];
-            else { const uint32_t u = ((uint32_t)((const uint16_t*)raw.data())[fm_index(n, k, K)]) << 16; memcpy(&v, &u, 4); }
+            else { const uint32_t u = ((uint32_t)((const uint16_t*)raw.data())[fm_index(t->row0 + n, t->col0 + k, ld)]) << 16; memcpy(&v, &u, 4); }
             out[k * N + n] = v;      // the reference's [in, out]
         }
     return NVL_OK;

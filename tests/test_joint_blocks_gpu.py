@@ -1,0 +1,44 @@
+"""Parallel blocks whose projections of one operand, and into one sum, are one matrix each, against the fp32 mode, which keeps them apart."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from conftest import rel_err
+
+pytestmark = pytest.mark.gpu
+TOL = 1.5e-2
+
+
+@pytest.mark.parametrize("at,mult,joint", [("mqa", 0.0, True), ("mha", 0.0, True), ("mha", 0.25, True), ("gqa", 0.5, False)])      # biases with mha; joint False: two multipliers
+@pytest.mark.parametrize("n", [1, 5, 17, 40, 70])               # narrow, wide, ring and grouped forms of a step; prompts of 1 .. 200 rows with and without fp32 rows
+def test_against_fp32(gpu, at, mult, joint, n):
+    kv = dict(mqa=1, mha=4, gqa=2)[at]
+    cfg = gpu.synth.tiny_config("falcon", hidden=256, num_heads=4, num_kv_heads=kv, ffn_dim=4096, attention_type=at, num_layers=2, max_seq_len=256, attention_multiplier=mult,
+                                residual_multiplier=mult if joint else 0.75)
+    w = gpu.synth.make_weights(cfg, seed=8, scale=0.05)
+    r = np.random.default_rng(n)
+    ids = list(range(n))
+    prompts = [r.integers(0, cfg["vocab_size"], 1 + 129 * (i == 0) * (n > 5)).tolist() for i in ids]
+    steps = r.integers(0, cfg["vocab_size"], (2, n)).tolist()
+
+    def logits(m):
+        for i in ids:
+            m.seq_reset(i)
+        out, at_ = [m.forward_batch(ids, prompts, [0] * n)[0]], [len(p) for p in prompts]
+        for s in steps:
+            out.append(m.forward_batch(ids, [[t] for t in s], at_)[0])
+            at_ = [a + 1 for a in at_]
+        return np.stack(out)
+
+    got = []
+    for precision in ("f32", "bf16"):
+        m = gpu.HipTransformerModel(cfg, w, precision=precision, max_seqs=n, max_batch_tokens=256)
+        got.append(logits(m))
+        if precision == "bf16":          # what stays readable behind finalize
+            for slot, n_in in (("wo", 256), ("w2", 4096)):
+                back = np.empty((n_in, 256), np.float32)
+                gpu._lib.check(m.lib.nvl_get_weight(m.h, gpu._lib.SLOT_ID[slot], 1, back.ctypes.data_as(C.c_void_p), n_in, 256), m.h)
+                assert np.array_equal(back, gpu.synth.round_bf16(w[slot, 1]))
+        m.close()
+    assert rel_err(got[1], got[0]) <= TOL
