@@ -428,12 +428,19 @@ __device__ __forceinline__ void epilogue_qkv_head(const GemmArgs& p, int m, int 
 }
 
 // ------------------------------------------------------------------------------------------
-// bf16 MFMA kernel (prefill), one template, three instances chosen per shape by the launcher:
-//   <128,128, 2,2, 2>  4 waves, wave tile  64x64, 2 LDS stages (64 KiB, 2 workgroups/CU): small M, MoE segments
+// bf16 MFMA kernel (prefill), one template, instances chosen per shape by the launcher:
+//   <128,128, 2,2, 4, BK 32>  4 waves, wave tile 64x64, a ring of 4 K tiles of 32 (64 KiB, 2 workgroups/CU): what does not fill
+//                             256x256 tiles (below)
+//   <128,128, 2,2, 4>  4 waves, four K tiles of 64 (128 KiB): decode-sized MoE batches
 //   <256,128, 4,2, 3>  8 waves, wave tile  64x64, 3 LDS stages (144 KiB): two K tiles in flight
 //   <256,256, 2,4, 2>  8 waves, wave tile 128x64, 2 LDS stages (128 KiB): least LDS traffic per MFMA
-//                      ((8+4) fragment reads per 32 MFMAs instead of (4+4) per 16) — the large-M default
-// BK = 64 (two MFMA k-steps).  Every operand tile is a run of 1-KiB fragment-major blocks, so one
+//                      ((8+4) fragment reads per 32 MFMAs instead of (4+4) per 16)
+// BK 32: the fragments of a K tile are read, and the loads of another issued, between the products of the tile before.  A lone workgroup's K tile is
+// 0.125 us of products; with reads and loads in a row in front of them it took 0.234, between them 0.188 (two workgroups a CU 0.34 and 0.33 for
+// both), and three K tiles in flight instead of one cover the weights' way from HBM.  The lock-step loop over two tiles of 64 that was here -> now, us:
+// 487 x 3072 x 2048 33.5 -> 22.7, 487 x 2048 x 8192 112 -> 73, 200 x 16384 x 2048 33 -> 24, 974 x 3072 x 2048 26.5 -> 21.0, 600 x 768 x 3072 37.5 -> 26.9,
+// 2000 x 2048 x 2048 31.7 -> 26.6, 487 x 16384 x 2048 (two a CU) 40.8 -> 39.5, 900 x 4672 x 4544 60.7 -> 58.2.  Deeper rings, and 256x128 tiles of this form, are slower.
+// Every operand tile is a run of 1-KiB fragment-major blocks, so one
 // global_load_lds_dwordx4 per block fills LDS lane-linearly and the fragment ds_read_b128s are
 // conflict-free.  Raw s_barrier + counted s_waitcnt vmcnt keep (STAGES-2) later tiles in flight
 // across the barrier (never vmcnt(0) in the steady state of the 3-stage instance).
@@ -463,17 +470,18 @@ __device__ __forceinline__ void tile_coords(int pid, int tiles_m, int tiles_n, i
     tn = r / gsz;
 }
 
-template <int BM, int BN, int STAGES>
-constexpr int gemm_lds_bytes() { return STAGES * (BM + BN) * G_BK * 2; }
+template <int BM, int BN, int STAGES, int BK = G_BK>
+constexpr int gemm_lds_bytes() { return STAGES * (BM + BN) * BK * 2; }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int EPI, typename OutT>
-__global__ __launch_bounds__(WAVES_M * WAVES_N * 64, (WAVES_M * WAVES_N == 4 && STAGES == 2) ? 2 : 1)
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int EPI, typename OutT, int BK = G_BK>
+__global__ __launch_bounds__(WAVES_M * WAVES_N * 64, (WAVES_M * WAVES_N == 4 && STAGES * BK <= 160) ? 2 : 1)
 void gemm_bf16_kernel(GemmArgs p) {
     constexpr int NW = WAVES_M * WAVES_N;
     constexpr int TM = BM / WAVES_M / 16, TN = BN / WAVES_N / 16;   // 16x16 accumulator tiles per wave
-    constexpr int NA = BM / 16 * 2, NB = BN / 16 * 2;               // 1-KiB blocks per stage (A, W)
+    constexpr int KS = BK / 32;                                      // MFMA k-steps of a K tile
+    constexpr int NA = BM / 16 * KS, NB = BN / 16 * KS;               // 1-KiB blocks per stage (A, W)
     constexpr int PW = (NA + NB) / NW;                               // blocks staged per wave per K tile
-    constexpr int STAGE_BYTES = (BM + BN) * G_BK * 2;
+    constexpr int STAGE_BYTES = (BM + BN) * BK * 2;
     static_assert((NA + NB) % NW == 0, "blocks must divide evenly over the waves");
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -510,37 +518,40 @@ void gemm_bf16_kernel(GemmArgs p) {
     for (int i = 0; i < PW; i++) {
         const int blk = wave * PW + i;
         if (blk < NA) {
-            const int rt = blk >> 1, ksb = blk & 1;
+            const int rt = blk / KS, ksb = blk % KS;
             int am = m0 + rt * 16 + fr;
             if (am > p.M - 1) am = p.M - 1;                 // clamp: rows >= M are never stored
             am += row_base;
             if (p.a_rows) am = p.a_rows[am];
             src[i] = (const bf16_t*)p.A + ((((int64_t)(am >> 4) * (p.K >> 5) + ksb) * 64) + (am & 15) + 16 * fg) * 8;
         } else {
-            const int wb = blk - NA, rt = wb >> 1, ksb = wb & 1;
+            const int wb = blk - NA, rt = wb / KS, ksb = wb % KS;
             src[i] = (const bf16_t*)p.W + (((int64_t)((n0 >> 4) + rt) * (p.K >> 5) + ksb) * 64 + lane) * 8;
         }
     }
     auto stage = [&](int buf, int kt) {
         char* base = smem + buf * STAGE_BYTES + wave * (PW * 1024);
-        const int64_t koff = (int64_t)kt * 1024;            // 2 k-steps x 512 elements per K tile
+        const int64_t koff = (int64_t)kt * (512 * KS);
 #pragma unroll
         for (int i = 0; i < PW; i++)
             __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] + koff),
                                              (__attribute__((address_space(3))) void*)(base + i * 1024), 16, 0, 0);
     };
+    auto stage_one = [&](int buf, int kt, int i) {
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] + (int64_t)kt * (512 * KS)),
+                                         (__attribute__((address_space(3))) void*)(smem + buf * STAGE_BYTES + wave * (PW * 1024) + i * 1024), 16, 0, 0);
+    };
     auto wait_tiles_in_flight = [&](int tiles) {   // s_waitcnt needs an immediate
         if (tiles <= 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        else if (PW == 6) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
-        else if (tiles == 1) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(16)" ::: "memory");       // four stages: two younger tiles of 8 loads each
+        else if (tiles == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PW) : "memory");
+        else if (tiles == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PW) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * PW) : "memory");
     };
-    static_assert(STAGES == 2 || PW == 6 || PW == 8, "add the immediate for this PW");
-    static_assert(STAGES <= 3 || PW == 8, "four stages: only the PW = 8 immediates exist");
+    static_assert(STAGES <= 8 && 3 * PW < 64, "at most three younger tiles");
 
     // ---- fragment reads: stage image [A row-tile][k-step][lane][16 B] then [W row-tile][k-step][lane][16 B]
-    const int a_blk_off = wm * TM * 2048 + lane * 16;                 // activation rows -> MFMA B operand (output col m)
-    const int w_blk_off = NA * 1024 + wn * TN * 2048 + lane * 16;     // weight rows     -> MFMA A operand (output row n)
+    const int a_blk_off = wm * TM * (1024 * KS) + lane * 16;                 // activation rows -> MFMA B operand (output col m)
+    const int w_blk_off = NA * 1024 + wn * TN * (1024 * KS) + lane * 16;     // weight rows     -> MFMA A operand (output row n)
 
     f32x4 acc[TM][TN];
 #pragma unroll
@@ -551,13 +562,67 @@ void gemm_bf16_kernel(GemmArgs p) {
     // K split over gridDim.y workgroups per tile (residual projections of 65..512 rows: N / 128 x M / 128 tiles alone are
     // far too few workgroups): slice y takes K tiles [kt0, kt0 + nt) and leaves an fp32 partial tile in sk_part[y]; the
     // norm that follows sums the slices into x (PendingResid: the kernel boundary is the synchronisation)
-    const int nt_all = p.K / G_BK;
+    const int nt_all = p.K / BK;
     int nt = nt_all, kt0 = 0;
     if (EPI == EPI_RESID && p.sk_part) {
         const int per = nt_all / (int)gridDim.y, extra = nt_all - per * (int)gridDim.y;
         kt0 = (int)blockIdx.y * per + ((int)blockIdx.y < extra ? (int)blockIdx.y : extra);
         nt = per + ((int)blockIdx.y < extra ? 1 : 0);
     }
+    if constexpr (BK == 32) {
+        static_assert(BM == 128 && BN == 128 && TM + TN == 8 && PW == 4, "eight reads and four loads between sixteen products");
+        // a K tile's fragments are read while the products of the one before run; its slot is filled again as soon as every wave holds them
+        bf16x8 fa[2][TM], fw[2][TN];
+        auto fragments = [&](int slot, bf16x8 (&af)[TM], bf16x8 (&wf)[TN]) {
+            const char* sbuf = smem + slot * STAGE_BYTES;
+#pragma unroll
+            for (int j = 0; j < TN; j++) wf[j] = *(const bf16x8*)(sbuf + w_blk_off + j * 1024);
+#pragma unroll
+            for (int i = 0; i < TM; i++) af[i] = *(const bf16x8*)(sbuf + a_blk_off + i * 1024);
+        };
+#pragma unroll
+        for (int s = 0; s < STAGES; s++)
+            if (s < nt) stage(s, kt0 + s);
+        wait_tiles_in_flight((nt < STAGES ? nt : STAGES) - 1);
+        __builtin_amdgcn_s_barrier();
+        fragments(0, fa[0], fw[0]);
+        wait_tiles_in_flight((nt < STAGES ? nt : STAGES) - 2);
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        __builtin_amdgcn_s_barrier();
+        int slot = 0, t = 0;
+        // FULL: all of the ring is in flight, so that the wait is an immediate and nothing is asked
+        auto step = [&](auto full, int t, bf16x8 (&af)[TM], bf16x8 (&wf)[TN], bf16x8 (&an)[TM], bf16x8 (&wn)[TN]) __attribute__((always_inline)) {
+            constexpr bool FULL = decltype(full)::value;
+            const int next = slot + 1 == STAGES ? 0 : slot + 1;
+            const char* sbuf = smem + next * STAGE_BYTES;
+            const bool load = FULL || t + STAGES < nt;
+            // reads and loads between the products: issued in a row they hold the products up (0.234 -> 0.188 us a tile of a lone workgroup)
+#pragma unroll
+            for (int e = 0; e < TM * TN; e++) {
+                const int i = e / TN, j = e % TN;
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], af[i], acc[i][j], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                if (e % 2 == 0 && e / 2 < TN) wn[e / 2] = *(const bf16x8*)(sbuf + w_blk_off + e / 2 * 1024);
+                if (e % 2 == 0 && e / 2 >= TN) an[e / 2 - TN] = *(const bf16x8*)(sbuf + a_blk_off + (e / 2 - TN) * 1024);
+                if (e % 2 == 1 && e / 2 < PW && load) stage_one(slot, kt0 + t + STAGES, e / 2);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            slot = next;
+            // tile t + 2 must have landed; the younger ones stay in flight
+            __builtin_amdgcn_s_waitcnt(0xC07F);      // lgkmcnt(0); the builtin, which the compiler counts: behind asm it waits for the reads a second time, in front of the products
+            if (FULL) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PW * (STAGES - 2)) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+        };
+        for (; t + 1 + STAGES < nt; t += 2) {
+            step(std::true_type{}, t, fa[0], fw[0], fa[1], fw[1]);
+            step(std::true_type{}, t + 1, fa[1], fw[1], fa[0], fw[0]);
+        }
+        for (; t < nt; t += 2) {
+            step(std::false_type{}, t, fa[0], fw[0], fa[1], fw[1]);
+            if (t + 1 < nt) step(std::false_type{}, t + 1, fa[1], fw[1], fa[0], fw[0]);
+        }
+    } else {
 #pragma unroll
     for (int s = 0; s < STAGES - 1; s++)
         if (s < nt) stage(s, kt0 + s);
@@ -572,12 +637,12 @@ void gemm_bf16_kernel(GemmArgs p) {
         }
         const char* sbuf = smem + cur * STAGE_BYTES;
 #pragma unroll
-        for (int ks = 0; ks < 2; ks++) {
+        for (int ks = 0; ks < KS; ks++) {
             bf16x8 af[TM], wf[TN];
 #pragma unroll
-            for (int j = 0; j < TN; j++) wf[j] = *(const bf16x8*)(sbuf + w_blk_off + j * 2048 + ks * 1024);
+            for (int j = 0; j < TN; j++) wf[j] = *(const bf16x8*)(sbuf + w_blk_off + j * (1024 * KS) + ks * 1024);
 #pragma unroll
-            for (int i = 0; i < TM; i++) af[i] = *(const bf16x8*)(sbuf + a_blk_off + i * 2048 + ks * 1024);
+            for (int i = 0; i < TM; i++) af[i] = *(const bf16x8*)(sbuf + a_blk_off + i * (1024 * KS) + ks * 1024);
             __builtin_amdgcn_s_setprio(1);
 #pragma unroll
             for (int i = 0; i < TM; i++)
@@ -592,6 +657,7 @@ void gemm_bf16_kernel(GemmArgs p) {
         wait_tiles_in_flight(younger);
         __builtin_amdgcn_s_barrier();
         cur = cur + 1 == STAGES ? 0 : cur + 1;
+    }
     }
 
     // ---- epilogue: lane holds rows n = 4*fg + r of column m = fr of each 16x16 tile ----
@@ -1960,18 +2026,19 @@ static inline bool launch_gemm_ln_resid(hipStream_t st, const GemmArgs& a0) {
     return true;
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int EPI, typename OutT>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int EPI, typename OutT, int BK = G_BK>
 static inline void launch_gemm_tile(hipStream_t st, const GemmArgs& a) {
-    constexpr int lds = gemm_lds_bytes<BM, BN, STAGES>();
-    NVL_LDS_ATTR((gemm_bf16_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, EPI, OutT>), lds);
+    constexpr int lds = gemm_lds_bytes<BM, BN, STAGES, BK>();
+    NVL_LDS_ATTR((gemm_bf16_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, EPI, OutT, BK>), lds);
     const int tiles = cdiv(a.M, BM) * cdiv(a.N, BN);
-    hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, EPI, OutT>),
+    hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, EPI, OutT, BK>),
                        dim3(tiles, (EPI == EPI_RESID && a.sk_part) ? a.sk_slices : 1), dim3(WAVES_M * WAVES_N * 64), lds, st, a);
 }
 
-// What a projection takes on the two prefill forms, in microseconds: fitted to launches of 10 .. 600 us between 480 and 8500 rows, good to
-// 15 %.  Ping-pong 256x256 tiles: a K-step is 0.46 us while power does not bind (up to half of the CUs busy) and 0.69 with all of
-// them; the last round's tiles (`rest` of 32 per XCD) may be cut into parts, which costs 10 + 2.5 us a part.
+// What a projection takes on the two prefill forms, in microseconds: fitted to 200 launches of 300 .. 16384 rows of 768 .. 28672 x 768 .. 22720, good to
+// 11 %; the form that they choose is 0.5 % above the faster one in the mean, 18 % at worst.  Ping-pong 256x256 tiles: a K-step is 0.53 us while
+// power does not bind (up to half of the CUs busy) and 0.79 with all of them; the last round's tiles (`rest` of 32 per XCD) may be cut into
+// parts, which costs 9.3 + 2.4 us a part.
 constexpr int PP_LDS = 4 * 32 * 1024 + 16;
 inline int g_pp_split = 0;          // nvl_set_tuning key 41: 0 from the grid, 1 never, n parts
 static inline double gemm_epilogue_us(int M, int N, int bytes) { return (double)M * N * bytes / 4.5e6; }
@@ -1981,16 +2048,34 @@ static inline double pp_cost(int M, int N, int K, int out_bytes, bool can_split,
     double best = 0;
     for (int c = 1; c <= 8 && rest * c <= 32; c++) {
         if (c > 1 && (!can_split || !rest || T < 8 || stages / c < PP_MIN_STAGES || (g_pp_split && c != g_pp_split))) continue;
-        const double fill = rest * c / 32.0, t = rest ? (stages / c) * (0.46 + (fill > 0.45 ? 0.42 * (fill - 0.45) : 0.0)) + (c > 1 ? 10.0 + 2.5 * c : 0.0) : 0.0;
+        const double fill = rest * c / 32.0, t = rest ? (stages / c) * (0.525 + (fill > 0.45 ? 0.41 * (fill - 0.45) : 0.0)) + (c > 1 ? 9.3 + 2.4 * c : 0.0) : 0.0;
         if (c == 1 || t < 0.92 * best || g_pp_split == c) { best = t; parts = c; }
     }
-    return (n >> 5) * (stages * 0.69 + 4.0) + best + gemm_epilogue_us(M, N, out_bytes) + 6.0;
+    return (n >> 5) * (stages * 0.79 + 3.0) + best + 0.36 * gemm_epilogue_us(M, N, out_bytes) + 13.7;
 }
-// 128x128 tiles, two workgroups a CU; K in `slices` whose sums somebody else adds up
+// 128x128 tiles, up to two workgroups a CU; K in `slices` whose sums somebody else adds up
 static inline double tile128_cost(int M, int N, int K, int out_bytes, int slices) {
-    const double wgs = (double)cdiv(M, 128) * cdiv(N, 128) * slices, per = 9.7 * wgs / 256.0 + 1.5;
-    return K / 1024.0 / slices * (per > 10.2 ? per : 10.2) + 4.0 + (slices > 1 ? gemm_epilogue_us(M, N, 8 * slices) : 0.5 * gemm_epilogue_us(M, N, out_bytes));
+    const double x = (double)cdiv(M, 128) * cdiv(N, 128) * slices / 256.0, per = x <= 1.0 ? 6.7 + x : x <= 2.0 ? 11.6 + 2.0 * (x - 1.0) : 1.1 + 8.3 * x;
+    return K / 1024.0 / slices * per + 7.1 + (slices > 1 ? gemm_epilogue_us(M, N, 8 * slices) : 0.44 * gemm_epilogue_us(M, N, out_bytes));
 }
+// ... and how many slices cost least, the norm that sums them counted.  Beyond a workgroup a CU more of them only add traffic (487 x 2048 x 8192:
+// eight 27.5 us, four 26.0, and half as much for the norm to read)
+static inline int tile128_slices(int M, int N, int K, int most, double& cost) {
+    int slices = 1;
+    cost = tile128_cost(M, N, K, 8, 1);
+    if (g_chunk_max_m <= 64) {           // (key 11 = 64: sums in one order whatever the rows)
+        while (slices < most && cdiv(M, 128) * cdiv(N, 128) * slices < 512 && K / (slices * 2) >= 512) slices *= 2;
+        cost = tile128_cost(M, N, K, 8, slices);
+        return slices;
+    }
+    for (int s = 2; s <= most && K / s >= 512; s *= 2) {
+        const double c = tile128_cost(M, N, K, 8, s);
+        if (c < 0.97 * cost) { cost = c; slices = s; }
+    }
+    return slices;
+}
+// the 64-row groups of the decode form (65 .. 512 rows): every group pulls the weights through the CUs again
+static inline double passes_cost(int M, int N, int K) { return 4.0 + 0.3 * cdiv(M, 64) * 2e-6 * N * K; }
 // is the ping-pong form the faster one?  (its parts in a.splits)
 template <int EPI, typename OutT>
 static inline bool pp_wins(GemmArgs& a) {
@@ -2001,10 +2086,8 @@ static inline bool pp_wins(GemmArgs& a) {
     // it to a few workgroups, 17424 x 4096 at 140 / 200 rows 82 / 86 us in parts, 74 / 78 on 128x128 tiles)
     const bool parts = a.split_units * SPLIT_UNIT >= SPLIT_WS_BYTES && (a.M > MID_MAX_ROWS || a.M <= std::max(64, g_chunk_max_m)) &&
                        (EPI != EPI_GROUPED || cdiv(a.M, 256) * cdiv(a.N, 256) > 256);
-    const bool faster = pp_cost(a.M, a.N, a.K, bytes, parts, a.splits) < 0.93 * tile128_cost(a.M, a.N, a.K, bytes, 1);
-    // Whole tiles lose to 128x128 tiles that fit one round of two a CU, which the costs miss.  Large / 128x128, us, weights from HBM: 12288 x 4096 at 600
-    // rows 94 / 75, 6144 x 4096 at 1100 87 / 73, 28672 x 4096 (gate | up) at 200 82 / 77, 16384 x 2048 at 400 46 / 39; in a second round
-    // 12288 x 4096 at 700 92 / 129, 28672 x 4096 at 300 119 / 131
+    const bool faster = pp_cost(a.M, a.N, a.K, bytes, parts, a.splits) < 1.05 * tile128_cost(a.M, a.N, a.K, bytes, 1);      // (ties: 4176 x 4096 x 4096 161 / 172, 200 x 18176 x 4544 67 / 79)
+    // (whole tiles lose to 128x128 tiles that fit one round of two a CU, which the costs miss at times: 12288 x 2048 at 520 rows 42.6 / 30.2, 16384 x 2048 at 400 42 / 38)
     return faster && (a.splits > 1 || cdiv(a.M, 128) * cdiv(a.N, 128) > 512);
 }
 template <int EPI, typename OutT, int WAVES_N>
@@ -2040,9 +2123,9 @@ static inline void launch_gemm_grouped(hipStream_t st, const GemmArgs& a, int ma
                            lds4, st, a);
         return;
     }
-    constexpr int lds = gemm_lds_bytes<128, 128, 2>();
-    NVL_LDS_ATTR((gemm_bf16_kernel<128, 128, 2, 2, 2, EPI, OutT>), lds);
-    hipLaunchKernelGGL((gemm_bf16_kernel<128, 128, 2, 2, 2, EPI, OutT>), dim3(cdiv(a.N, 128) * max_mtiles), dim3(256),
+    constexpr int lds = gemm_lds_bytes<128, 128, 4, 32>();
+    NVL_LDS_ATTR((gemm_bf16_kernel<128, 128, 2, 2, 4, EPI, OutT, 32>), lds);
+    hipLaunchKernelGGL((gemm_bf16_kernel<128, 128, 2, 2, 4, EPI, OutT, 32>), dim3(cdiv(a.N, 128) * max_mtiles), dim3(256),
                        lds, st, a);
 }
 
@@ -2122,6 +2205,11 @@ static inline bool mid_wins(const GemmArgs& a) {
     // One row group reads the weights once at any width up to a few rounds of workgroups (a workgroup per CU: each round has its own
     // ramp; LM head at 128 rows 168 us against 152 on the tiles, 28672 x 4096 72 against 74).  Several groups pay while one round holds
     // them (3072 x 2048: 192 rows 12.5 against 17.4 us, 512 rows 18.3 against 29; 16384 x 2048 at 512 rows 68 against 43).
+    // Long K: parts of large tiles (4544 x 22720 at 140 / 300 rows 117 / 154 us here, 94 / 128 there; not 4096 x 14336 at 300, 92 and 95).
+    if (a.M > 128 && a.split_units * SPLIT_UNIT >= SPLIT_WS_BYTES && EPI == EPI_RESID) {
+        int parts, mid_parts;
+        if (1.05 * pp_cost(a.M, a.N, a.K, 8, true, parts) < mid_cost(a.M, a.N, a.K, mid_row_tiles(a.M), 2, true, mid_parts)) return false;
+    }
     return cdiv(a.N, 64) * cdiv(a.M, 128) <= (a.M <= 128 ? 512 : 256);
 }
 template <int EPI, typename OutT>
@@ -2159,7 +2247,8 @@ void launch_gemm_bf16(hipStream_t st, const GemmArgs& a) {
         // in one launch instead (GemmArgs::m_passes): the groups of a weight block run side by side on one XCD, so the
         // weights cross HBM once.  Only the narrow projections (QKV, O, FFN-down) do; FFN-up and the LM head have enough
         // tiles (g_chunk_all_m: below it every projection would).
-        const bool few_tiles = cdiv(a.M, 128) * cdiv(a.N, 128) < g_chunk_min_tiles;
+        // (us, groups / tiles: 768 x 768 at 300 rows 5.5 / 12.3, 2304 x 768 10.3 / 11.0, 3072 x 768 12.2 / 17.5; 6144 x 4096 62.8 / 39.4, 8512 x 2048 at 140 41.2 / 22.9)
+        const bool few_tiles = cdiv(a.M, 128) * cdiv(a.N, 128) < g_chunk_min_tiles && passes_cost(a.M, a.N, a.K) < tile128_cost(a.M, a.N, a.K, EPI == EPI_RESID ? 8 : (int)sizeof(OutT), 1);
         if (a.M > 64 && a.M <= g_chunk_max_m && (a.M <= g_chunk_all_m || few_tiles || a.rs_in || a.rs_out) && !a.a_rows && !a.seg && !a.sk_part && a.K % 32 == 0 &&
             g_force_tile == 0) {
             GemmArgs c = a;
@@ -2192,7 +2281,7 @@ void launch_gemm_bf16(hipStream_t st, const GemmArgs& a) {
     if (tile == 5 && !a.seg && !a.a_rows) { launch_pp<EPI, OutT, 4>(st, as); return; }      // (4-slot ring: 5 slots -3 %, 3 slots -3 %, r01 sweep)
     if (tile == 3) launch_gemm_tile<256, 256, 2, 4, 2, EPI, OutT>(st, a);
     else if (tile == 2) launch_gemm_tile<256, 128, 4, 2, 3, EPI, OutT>(st, a);
-    else launch_gemm_tile<128, 128, 2, 2, 2, EPI, OutT>(st, a);
+    else launch_gemm_tile<128, 128, 2, 2, 4, EPI, OutT, 32>(st, a);
     }
 }
 

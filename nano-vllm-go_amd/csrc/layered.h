@@ -940,7 +940,8 @@ SubOut sub_out(nvl_model* m, int site, const void* A, const void* W, int M, int 
         while (slices < m->sk_max_slices && nblocks * slices < 256 && (K >> 5) / (slices * 2) >= 8) slices *= 2;
     } else if (!m->f32 && M <= 512 && M <= m->sk_rows && N % 128 == 0 && g_force_tile == 0) {
         const int tiles = cdiv(M, 128) * (N / 128);
-        while (slices < SK_TILE_MAX_SLICES && tiles * slices < 512 && K / (slices * 2) >= 512) slices *= 2;
+        double cost;
+        slices = tile128_slices(M, N, K, SK_TILE_MAX_SLICES, cost);
         if (tiles * slices < 64) slices = 1;
     }
     m->site = site;

@@ -1679,13 +1679,14 @@ void resid_gemm(nvl_model* m, const void* A, int lda, const void* W, const float
     if (g_sk_tile && !m->f32 && M > (g_mid && K >= 2048 ? std::max(64, std::min(g_mid_resid_rows, g_chunk_max_m)) : 64) && M <= m->sk_rows && !m->keep_hidden && m->sk_part && m->pending_slices == 0 &&
         N % 128 == 0 && K % 64 == 0 && norm_ok && N == m->H && g_force_tile == 0 && m->n_mamba == 0) {
         const int tiles = cdiv(M, 128) * (N / 128);
-        while (slices < SK_TILE_MAX_SLICES && tiles * slices < 512 && K / (slices * 2) >= 512) slices *= 2;
+        double best;
+        slices = tile128_slices(M, N, K, SK_TILE_MAX_SLICES, best);
         // (fewer than 64 workgroups even so — GPT-2's 768 columns below 512 rows —: the decode form's 64-row groups stream
         // better, profiles/r03_gpt2_large_decode_batches.txt: B = 128 147.5 K -> 159.0 K, B = 256 224.8 K -> 237.2 K tok/s)
         if (tiles * slices < 64) slices = 1;
-        // ... unless large tiles whose K is cut inside the launch are faster (1024 x 4096 x 14336: 118 us, and no slices for the norm)
+        // ... unless large tiles whose K is cut inside the launch are faster, and leave no slices for the norm
         int parts;
-        if (slices > 1 && M > 256 && pp_cost(M, N, K, 8, m->split_bytes >= SPLIT_WS_BYTES, parts) < 0.72 * tile128_cost(M, N, K, 8, slices)) slices = 1;
+        if (slices > 1 && M > 256 && pp_cost(M, N, K, 8, m->split_bytes >= SPLIT_WS_BYTES, parts) < 0.95 * best) slices = 1;
     }
     if (slices > 1) {
         a.sk_part = m->sk_part; a.sk_slices = slices;

@@ -1,0 +1,40 @@
+"""128x128 tiles with a ring of K tiles of 32: fewer of them than the ring holds, even and odd numbers, ragged rows and columns."""
+import numpy as np
+import pytest
+
+from conftest import rel_err
+
+pytestmark = pytest.mark.gpu
+TOL = 1.5e-2
+
+
+@pytest.mark.parametrize("k", [64, 128, 192, 256, 320, 2048])          # 2, 4, 6, 8, 10 and 64 K tiles; the ring holds 4
+@pytest.mark.parametrize("m,n", [(65, 130), (128, 128), (129, 384), (700, 96), (1000, 1000)])
+def test_products_are_exact(gpu, m, n, k):
+    """Small whole numbers: every sum is exact in fp32, whatever its order."""
+    r = np.random.default_rng(m + n + k)
+    a, b = (r.integers(-4, 5, s).astype(np.float32) for s in ((m, k), (k, n)))
+    old = gpu.lib().nvl_set_tuning(0, 1)
+    try:
+        got = gpu.ops.mat_mul(a, b, precision="bf16")
+    finally:
+        gpu.lib().nvl_set_tuning(0, old)
+    assert np.array_equal(got, (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32))
+
+
+@pytest.mark.parametrize("rows", [70, 200, 513, 900])
+def test_slices_of_odd_numbers_of_tiles(gpu, rows):
+    """A prompt whose residual projections run in slices that the norm behind them sums: 66 K tiles in 2 .. 4 slices of 16 and 17, against the fp32 mode."""
+    cfg = gpu.synth.tiny_config("llama", hidden=2048, num_heads=8, num_kv_heads=8, head_dim=64, ffn_dim=2112, num_layers=2, max_seq_len=1024)
+    w = gpu.synth.make_weights(cfg, seed=4, scale=0.03)
+    tokens = np.random.default_rng(rows).integers(0, cfg["vocab_size"], rows).tolist()
+    got = []
+    for precision in ("f32", "bf16"):
+        m = gpu.HipTransformerModel(cfg, w, precision=precision, max_seqs=1, max_batch_tokens=1024)
+        m.seq_reset(0)
+        got.append(m.forward_batch([0], [tokens], [0], all_logits=True)[0])
+        if precision == "bf16":
+            m.seq_reset(0)
+            assert np.array_equal(got[1], m.forward_batch([0], [tokens], [0], all_logits=True)[0])
+        m.close()
+    assert rel_err(got[1], got[0]) <= TOL
