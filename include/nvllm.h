@@ -558,7 +558,7 @@ int nvl_bench_gemm(int device, int M, int N, int K, int epi, int force_bnt, int 
  * key 14 rows (64) every projection does.  key 15: waves per decode-attention workgroup (0 = from context length and
  * grid size, 2, 4, 8).  key 16: prefill MoE copies the token rows into expert order before the grouped GEMM (1, default)
  * or gathers them per lane inside it (0).  key 17: prefill MoE grouped GEMMs: 0 (default) = 256-row segments on the
- * ping-pong kernel, 128 / 256 = the lock-step tile kernels with that many rows per m-tile.
+ * ping-pong kernel beyond 64 rows an expert in the mean, 128-row segments up to there; 128 / 256 = the tile kernels with that many rows per m-tile.
  * key 19: decode-sized MoE batches run the grouped GEMMs on the four-stage 128x128 instance (1, default) or two stages (0).
  * key 18: largest prompt batch (tokens) whose QKV projection leaves fp32 rows to rope_kv_kernel instead of rotating and placing
  * them itself (default -1: by size; 0: none).

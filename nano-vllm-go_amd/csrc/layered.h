@@ -1438,7 +1438,7 @@ ExpertOut parallel_ffn(nvl_model* m, const LayerRun& r, const MixerW& w, int M) 
         gemm(m, EPI_RESID, true, d, 2.0 * pairs * m->Hn * c.expert_dim);
         return {m->moe_part, r.moe_slices, (int64_t)M * m->H, nullptr, nullptr};
     }
-    const bool pp = moe_pp_ok(m, r.Ip, false);
+    const bool pp = moe_pp_ok(m, r.Ip, false, (int64_t)M * k, E);
     const int BM = pp ? 256 : ((!m->f32 && g_moe_bm == 256) ? 256 : 128);
     moe_sort(m, E, k, M, BM);
     moe_expert_gemms(m, MoeW{E, k, r.Ip, w.moe_up, w.moe_down}, M, BM, pp, false);
@@ -1510,7 +1510,7 @@ SubOut expert_ffn(nvl_model* m, const LayerRun& r, const MixerW& w, int M, Exper
         shared();
         return y;
     }
-    const bool pp = moe_pp_ok(m, r.Ip, false);
+    const bool pp = moe_pp_ok(m, r.Ip, false, (int64_t)M * k, E);
     const int BM = pp ? 256 : ((!m->f32 && g_moe_bm == 256) ? 256 : 128);
     moe_sort(m, E, k, M, BM);
     moe_expert_gemms(m, MoeW{E, k, r.Ip, w.moe_up, w.moe_down, c.expert_limit}, M, BM, pp, false, xn_rows);

@@ -38,3 +38,26 @@ def test_slices_of_odd_numbers_of_tiles(gpu, rows):
             assert np.array_equal(got[1], m.forward_batch([0], [tokens], [0], all_logits=True)[0])
         m.close()
     assert rel_err(got[1], got[0]) <= TOL
+
+
+@pytest.mark.parametrize("n", [1, 100, 256, 257])          # 256 tokens x 8 of 32 experts: 64 rows an expert, the last prompt that takes 128-row tiles
+def test_experts_of_few_rows(gpu, n):
+    """The experts' products of a short prompt against forced 256-row tiles (key 17), which add up in the same order."""
+    import torch
+    from bench import gen_weights_on_device
+    cfg = dict(gpu.synth.FULL_CONFIGS["granite-3.0-1b-a400m"], num_layers=2, vocab_size=1000)
+    m = gpu.HipTransformerModel(cfg, None, precision="bf16", max_seqs=2, max_batch_tokens=320)
+    gen_weights_on_device(gpu, cfg, m, torch, torch.device("cuda", 0), keep_host=False)
+    m.finalize()
+    prompts = [np.random.default_rng(n).integers(0, 1000, k).tolist() for k in (n, 66)][: 2 if n < 200 else 1]
+    ids, got = list(range(len(prompts))), []
+    for rows in (0, 256):
+        old = gpu.lib().nvl_set_tuning(17, rows)
+        try:
+            for i in ids:
+                m.seq_reset(i)
+            got.append(m.forward_batch(ids, prompts, [0] * len(ids))[0])
+        finally:
+            gpu.lib().nvl_set_tuning(17, old)
+    m.close()
+    assert rel_err(got[0], got[1]) <= TOL
