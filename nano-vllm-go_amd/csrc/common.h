@@ -20,6 +20,9 @@ typedef __attribute__((ext_vector_type(2))) float f32x2;
 // weight matrices are allocated with their row count padded to the largest GEMM N-tile (zero rows), so every
 // tile instance may read a whole tile; outputs beyond N are never stored
 constexpr int64_t W_ROW_PAD = 256;
+constexpr int64_t weight_rows(int64_t N) { return (N + W_ROW_PAD - 1) / W_ROW_PAD * W_ROW_PAD; }
+// rows of a matrix whose first `a` rows and the `b` behind them are read both by themselves and as one operand
+constexpr int64_t joint_weight_rows(int64_t a, int64_t b) { return weight_rows(a + b) > a + weight_rows(b) ? weight_rows(a + b) : a + weight_rows(b); }
 
 // ---- bf16 conversions -------------------------------------------------------
 __device__ __forceinline__ float bf2f(bf16_t v) { return (float)v; }

@@ -38,7 +38,7 @@ struct LayerW {
     void* w_qkv = nullptr; int n_qkv = 0; float* b_qkv = nullptr;
     void* w1 = nullptr; int n1 = 0;      // fused rows (2F for SwiGLU, F for GELU)
     void *w_in = nullptr, *w_out = nullptr;         // parallel blocks (nvl_model::joint): QKV and W1 as one matrix (w_qkv and w1 point into it), WO and W2 side by side along K
-    float *b_in = nullptr, *b_out = nullptr;
+    float *b_in = nullptr, *b_out = nullptr; int64_t in_rows = 0;      // (rows w_in is allocated with)
     float *ln_qkv = nullptr, *ln_up = nullptr;      // deferred layer norms (nvl_model::ln_ok): S, then B of the projection behind each norm
     void* moe_in = nullptr;              // [E][2I (interleaved in bf16 mode)][H]
     void* moe_out_cat = nullptr;         // bf16: W_down of all experts along K, [H_pad][E*I] (decode "dense-masked" form)

@@ -595,7 +595,7 @@ extern "C" int nvl_upload_tensor(nvl_model* m, int kind, int layer, const void* 
             upload_2d(m, t, data, dtype, SN, SK, io, Slice2D{SN, SK, 0, 0, row0, mat_cols, col0}, SN, true, mat);
         };
         if (kind == NVL_T_WO || kind == NVL_T_W2) place(l.w_out, round_up(H, W_ROW_PAD), ko, 0, kind == NVL_T_WO ? 0 : qw);
-        else place(l.w_in, m->n_qkv + round_up((int64_t)m->F, W_ROW_PAD), H, kind == NVL_T_WQ ? 0 : kind == NVL_T_W1 ? m->n_qkv : kind == NVL_T_WV ? qw + nkv : qw, 0);
+        else place(l.w_in, l.in_rows = joint_weight_rows(m->n_qkv, m->F), H, kind == NVL_T_WQ ? 0 : kind == NVL_T_W1 ? m->n_qkv : kind == NVL_T_WV ? qw + nkv : qw, 0);
         return NVL_OK;
     }
     if (m->tp == 1) {
@@ -2201,6 +2201,7 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
             if (up_done) {
                 GemmArgs a = mk(m->xn, H, l.w_in, ffn_columns(m), qw + m->F, l.b_in, 1.f, M, m->n_qkv + m->F, H);
                 a.joint = JointEpi{m->qkv, m->n_qkv, m->n_qkv};
+                if (l.in_rows < weight_rows(a.N)) throw std::runtime_error("gemm: whole tiles of a joint matrix read past it");
                 gemm(m, EPI_JOINT, false, a);
             } else gemm(m, qkv_deferred && ln_defer ? EPI_LN_STORE : EPI_STORE, true, aq);
             fused_dec = !m->f32 && max_len == 1;     // decode: RoPE + KV append live in the attention kernel

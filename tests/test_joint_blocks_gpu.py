@@ -42,3 +42,30 @@ def test_against_fp32(gpu, at, mult, joint, n):
                 assert np.array_equal(back, gpu.synth.round_bf16(w[slot, 1]))
         m.close()
     assert rel_err(got[1], got[0]) <= TOL
+
+
+@pytest.fixture(scope="module")
+def wide(gpu):
+    """Falcon-7B's widths, one layer: [QKV | W1] is 22848 = 178.5 x 128 rows of 4544."""
+    cfg = dict(gpu.synth.FULL_CONFIGS["falcon-7b"], num_layers=1, vocab_size=1000, max_seq_len=64)
+    w = gpu.synth.make_weights(cfg, seed=9, scale=0.02)
+    models = [gpu.HipTransformerModel(cfg, w, precision=p, max_seqs=450, max_batch_tokens=450) for p in ("f32", "bf16")]
+    yield cfg, models
+    for m in models:
+        m.close()
+
+
+@pytest.mark.parametrize("n", [5, 24, 100, 140, 450])          # steps: narrow and wide decode form, ring kernel, 128x128 and 256x256 tiles
+def test_last_tiles_of_the_joint_matrix(wide, n):
+    """Whole tiles reach past the matrix's last rows; the first sequence's prompt of 40 tokens leaves fp32 rows of queries and keys too."""
+    cfg, models = wide
+    r = np.random.default_rng(n)
+    ids, first = list(range(n)), r.integers(0, cfg["vocab_size"], 40).tolist()
+    tokens, steps = r.integers(0, cfg["vocab_size"], n).tolist(), r.integers(0, cfg["vocab_size"], n).tolist()
+    got = []
+    for m in models:
+        for i in ids:
+            m.seq_reset(i)
+        out = [m.forward_batch([0], [first], [0])[0], m.forward_batch(ids, [[t] for t in tokens], [40] + [0] * (n - 1))[0], m.forward_batch(ids, [[t] for t in steps], [41] + [1] * (n - 1))[0]]
+        got.append(np.concatenate(out))
+    assert rel_err(got[1], got[0]) <= TOL
