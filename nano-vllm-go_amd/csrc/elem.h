@@ -118,6 +118,26 @@ static __global__ __launch_bounds__(64) void ln_fold_kernel(const bf16_t* __rest
     if (fg == 0) { s[n] = n < N ? a : 0.f; b[n] = n < N ? c + (bias ? bias[n] : 0.f) : 0.f; }
 }
 
+// what a residual projection adds to the mean of a row of its result (gemm.h MeanShift): the mean of W's N rows (whole tiles), in two bf16 parts.  One wave per
+// 32 columns, W fragment-major
+static __global__ __launch_bounds__(64) void ln_mean_row_kernel(const bf16_t* __restrict__ W, bf16_t* __restrict__ out, int N, int K) {
+    const int lane = threadIdx.x, fr = lane & 15, fg = lane >> 4, ks = blockIdx.x;
+    float a[8] = {};
+    for (int t = 0; t < (N >> 4); t++) {
+        const bf16x8 v = *(const bf16x8*)(W + (((int64_t)t * (K >> 5) + ks) * 64 + lane) * 8);
+#pragma unroll
+        for (int e = 0; e < 8; e++) a[e] += (float)v[e];
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) a[e] += __shfl_xor(a[e], o, 64);
+        const float mean = a[e] / (float)N;
+        const bf16_t hi = (bf16_t)mean;
+        if (fr < 2) out[(int64_t)ks * 64 + fr * 32 + fg * 8 + e] = fr == 0 ? hi : (bf16_t)(mean - (float)hi);
+    }
+}
+
 // Pending residual: the decode GEMMs that precede a norm (O projection, W2) may leave their output as
 // split-K partial slices instead of adding it into x; this kernel then completes the residual add
 // (generic_model.go:320-326,383-389) while it reads the row:  x[row] += alpha * sum_s part[s][row]  (slice order).

@@ -96,6 +96,9 @@ struct RouteJob {
 
 struct JointEpi { float* rows; int ld, n; };      // EPI_JOINT; n a multiple of 16
 
+// EPI_LN_RESID: what the projection adds to a row's mean.  w: the mean of W's rows, in bf16 and the rest of it in bf16, [K/32][those two][32]; b: the mean of the bias
+struct MeanShift { const bf16_t* w; float b; };
+
 struct GemmArgs {
     const void* A;          // bf16: fragment-major [M_pad16][K]; f32: row-major [M][lda]
     int lda;
@@ -125,6 +128,7 @@ struct GemmArgs {
         QkvEpi qkv;         // EPI_QKV
         RouteJob route;     // masked experts (epi_moe with moe_gate)
         JointEpi joint;     // EPI_JOINT
+        MeanShift mean;     // EPI_LN_RESID
     };
     GroupedEpi grp;         // EPI_GROUPED
     // decode kernel, EPI_RESID only: K split over gridDim.y = sk_slices workgroups per column block.  Each
@@ -170,11 +174,13 @@ struct GemmArgs {
     int moe_E, moe_I;
     // Deferred layer norm (epi_ln; M <= 64): ((x - mean) w / sd + b) W == rstd ((x - s) w W - (mean - s) S) + B for any s, S[n] = sum_k W[n][k] w[k] and
     // B[n] = bias[n] + sum_k W[n][k] b[k] from the weights alone.  Producer: xn_raw = bf16((x - s) w) and per tile the pair of sums of x - s and
-    // (x - s)^2; s is the row's mean at the norm before, so that a row far from zero loses nothing to the operand's rounding (ln_prev: that
-    // norm's pairs, or NULL, where it was a launch of its own that left its means in ln_mean_in).  Consumer: bias is B.
-    // A norm launch is 3.3 us (1 row) to 4.2 (16) and a boundary; the sums cost the four projections of a layer 0.5 to 1.7 us each.  GPT-2, us a step of
-    // 1 / 16 / 24 / 40 / 64 sequences: 434 -> 402, 493 -> 458, 540 -> 490, 567 -> 532, 690 -> 663; prompts of 11 / 3 x 11 / 64 tokens 514 -> 451, 595 -> 536, 586 -> 542.
-    // Error of the logits against 64 bits over 240 calls: mean log ratio to the norm launches +0.002 +- 0.002.
+    // (x - s)^2.  The operand's rounding and the variance cost sqrt(1 + d^2) times a norm launch's where s misses the row's mean by d of its deviations, so s is
+    // that mean but for rounding: the mean before (ln_prev: the pairs of the norm before, or NULL, where it was a launch of its own, and ln_mean_in) and what
+    // the projection adds to it, its operand times `mean` (one more product a K step; a mean that is 100 deviations away: d < 0.01).  Consumer: bias is B.
+    // A norm launch is 3.3 us (1 row) to 4.2 (16) and a boundary; the sums cost the four projections of a layer 0.5 to 1.7 us each, finding s
+    // the two residual ones 0.6 (GPT-2, a step of 1 sequence: with the mean before in its place 357 us, 371 so).  GPT-2, norm launches -> carried, us a step of 1 / 16 / 24 / 40 / 64 sequences:
+    // 388 -> 371, 448 -> 430, 495 -> 468, 518 -> 498, 575 -> 565; prompts of 11 / 3 x 11 / 64 tokens 470 -> 445, 544 -> 520, 550 -> 536.
+    // Error of the logits against 64 bits over 240 calls: mean log ratio to the norm launches -0.001 +- 0.002.
     const float* ln_s;
     const float *ln_prev, *ln_mean_in;
     float* ln_mean_out;
@@ -1430,7 +1436,13 @@ __global__ __launch_bounds__(skinny_waves(EPIV) * 64) void gemm_skinny_bf16_kern
     // flight while the current block's MFMAs issue (the compiler emits counted vmcnt for these).
     const int nblk = my_steps / U;
     bf16x8 wA[U], xA[U][MT], wB[U], xB[U][MT];
-    auto load_blk = [&](bf16x8 (&w)[U], bf16x8 (&x)[U][MT], int b) {
+    // carried layer norm: the mean row as rows 0, 2, .. and its rest as rows 1, 3, .. of a weight tile, so that every lane gets its row's sum of both
+    constexpr bool LN_SHIFT = LN && EPI == EPI_RESID;
+    constexpr int UC = LN_SHIFT ? U : 1;
+    bf16x8 cA[UC], cB[UC];
+    f32x4 mean_acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    const bf16x8* cp = LN_SHIFT ? (const bf16x8*)p.mean.w + (int64_t)ks0 * 8 + (fr & 1) * 4 + fg : nullptr;
+    auto load_blk = [&](bf16x8 (&w)[U], bf16x8 (&x)[U][MT], bf16x8 (&c)[UC], int b) {
 #pragma unroll
         for (int u = 0; u < U; u++) {
             if constexpr (HALF) w[u] = w_live ? weight_load<PASSES>((const bf16x8*)(wp + (int64_t)(b * U + u) * 512)) : x_zero;
@@ -1440,16 +1452,19 @@ __global__ __launch_bounds__(skinny_waves(EPIV) * 64) void gemm_skinny_bf16_kern
                 const bf16x8* src = (const bf16x8*)(xp[i] + (int64_t)(b * U + u) * 512);
                 if (p.x_mask) x[u][i] = x_live[i] ? *src : x_zero; else x[u][i] = *src;      // (uniform branch)
             }
+            if constexpr (LN_SHIFT) c[u] = cp[(b * U + u) * 8];
         }
     };
-    auto comp_blk = [&](bf16x8 (&w)[U], bf16x8 (&x)[U][MT]) {
+    auto comp_blk = [&](bf16x8 (&w)[U], bf16x8 (&x)[U][MT], bf16x8 (&c)[UC]) {
 #pragma unroll
-        for (int u = 0; u < U; u++)
+        for (int u = 0; u < U; u++) {
 #pragma unroll
             for (int i = 0; i < MT; i++)
                 acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u], x[u][i], acc[i], 0, 0, 0);
+            if constexpr (LN_SHIFT) mean_acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c[u], x[u][0], mean_acc, 0, 0, 0);
+        }
     };
-    if (nblk > 0) load_blk(wA, xA, 0);
+    if (nblk > 0) load_blk(wA, xA, cA, 0);
     stamps.mark(1);                     // first block of loads issued
     // the residual operand of this wave's first epilogue element (deferred-norm producer form): fetched under the weight
     // stream, not as a dependent round trip after the K reduction (this launch is the only writer of these elements)
@@ -1460,7 +1475,7 @@ __global__ __launch_bounds__(skinny_waves(EPIV) * 64) void gemm_skinny_bf16_kern
         if (m < p.M && n < p.N && (!HALF || (fg >> 1) == half)) x_pre = *(const f32x4*)((const float*)p.C + (int64_t)m * p.ldc + n);
     }
     float ln_shift = 0.f;      // (MT = 1: one row tile)
-    if constexpr (LN && EPI == EPI_RESID) {
+    if constexpr (LN_SHIFT) {
         static_assert(MT == 1 && NTW == 1, "one epilogue element");
         const int m = 16 * i_off + fr;
         const bool live = wave == 0 && m < p.M;
@@ -1469,25 +1484,31 @@ __global__ __launch_bounds__(skinny_waves(EPIV) * 64) void gemm_skinny_bf16_kern
     }
     if constexpr (MOE != 0 && EPI == EPI_RESID) {
         for (int b = 0; b < nblk; b += 2) {
-            if (b + 1 < nblk) load_blk(wB, xB, b + 1);
-            comp_blk(wA, xA);
+            if (b + 1 < nblk) load_blk(wB, xB, cB, b + 1);
+            comp_blk(wA, xA, cA);
             if (b + 1 >= nblk) break;
-            if (b + 2 < nblk) load_blk(wA, xA, b + 2);
-            comp_blk(wB, xB);
+            if (b + 2 < nblk) load_blk(wA, xA, cA, b + 2);
+            comp_blk(wB, xB, cB);
         }
     } else {
     int b = 0;
     for (; b + 2 <= nblk; b += 2) {
-        load_blk(wB, xB, b + 1);
-        comp_blk(wA, xA);
+        load_blk(wB, xB, cB, b + 1);
+        comp_blk(wA, xA, cA);
         if (b == 0) stamps.mark_used(2, acc[0]);       // first block's data arrived and was used
-        if (b + 2 < nblk) load_blk(wA, xA, b + 2);
-        comp_blk(wB, xB);
+        if (b + 2 < nblk) load_blk(wA, xA, cA, b + 2);
+        comp_blk(wB, xB, cB);
     }
-    if (b < nblk) comp_blk(wA, xA);
+    if (b < nblk) comp_blk(wA, xA, cA);
     }
     for (int s = nblk * U; s < my_steps; s++) {      // ragged tail: fewer than U k-steps
         const bf16x8 w = w_live ? weight_load<PASSES>((const bf16x8*)(wp + (int64_t)s * 512)) : x_zero;
+        if constexpr (LN_SHIFT) {
+            const bf16x8 c = cp[s * 8], x = x_live[0] ? *(const bf16x8*)(xp[0] + (int64_t)s * 512) : x_zero;
+            acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x, acc[0], 0, 0, 0);
+            mean_acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c, x, mean_acc, 0, 0, 0);
+            continue;
+        }
 #pragma unroll
         for (int i = 0; i < MT; i++)
             acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x_live[i] ? *(const bf16x8*)(xp[i] + (int64_t)s * 512) : x_zero, acc[i], 0, 0, 0);
@@ -1500,9 +1521,10 @@ __global__ __launch_bounds__(skinny_waves(EPIV) * 64) void gemm_skinny_bf16_kern
             acc[i] = g != 0.f ? acc[i] * g : f32x4{0.f, 0.f, 0.f, 0.f};       // (0: not routed, whatever the expert made of the row)
         }
     if constexpr (LN_LATE) rn_pre = layer_norm_of(p, pairs.sum());
-    if constexpr (LN && EPI == EPI_RESID) {
+    float* mean_red = (float*)(smem + ksplit * 1024);      // [16][8]
+    if constexpr (LN_SHIFT) {
         ln_shift += pairs.sum()[0] * p.rs_inv_h;
-        if (blockIdx.x == 0 && wave == 0 && fg == 0 && 16 * i_off + fr < p.M) p.ln_mean_out[16 * i_off + fr] = ln_shift;
+        if (fg == 0) mean_red[fr * 8 + kw] = mean_acc[0] + mean_acc[1];
     }
     // ---- reduce the K slices in wave order ----
 #pragma unroll
@@ -1510,6 +1532,15 @@ __global__ __launch_bounds__(skinny_waves(EPIV) * 64) void gemm_skinny_bf16_kern
     stamps.mark(3);                     // wave 0's stream done
     __syncthreads();
     stamps.mark(4);                     // every wave's stream done
+    if constexpr (LN_SHIFT) {
+        static_assert(skinny_waves(EPIV) == 8, "two reads a row");
+        const f32x4 lo = *(const f32x4*)(mean_red + fr * 8), hi = *(const f32x4*)(mean_red + fr * 8 + 4);
+        float added = lo[0];
+#pragma unroll
+        for (int w = 1; w < 8; w++) added += w < ksplit ? (w < 4 ? lo[w] : hi[w - 4]) : 0.f;
+        ln_shift += p.alpha * (added + p.mean.b);
+        if (blockIdx.x == 0 && wave == 0 && fg == 0 && 16 * i_off + fr < p.M) p.ln_mean_out[16 * i_off + fr] = ln_shift;
+    }
     auto ksum = [&](int t, int i) {
         f32x4 s = red[((t * ksplit) * MT + i) * 64 + lane];
         for (int w = 1; w < ksplit; w++) s += red[((t * ksplit + w) * MT + i) * 64 + lane];
@@ -2021,8 +2052,9 @@ static inline bool launch_gemm_ln_resid(hipStream_t st, const GemmArgs& a0) {
     int ks = skinny_waves(EPI_LN_RESID);
     while (ks > 1 && (a.K >> 5) / ks < 4) ks >>= 1;
     const int tiles = cdiv(a.N, 16);
-    if (a.rs_half) hipLaunchKernelGGL((gemm_skinny_bf16_kernel<1, 1, 4, EPI_LN_RESID, OutT, false, 0, true>), dim3(2 * tiles, 1), dim3(ks * 64), (size_t)ks * 1024, st, a);
-    else hipLaunchKernelGGL((gemm_skinny_bf16_kernel<1, 1, 4, EPI_LN_RESID, OutT>), dim3(tiles, cdiv(a.M, 16)), dim3(ks * 64), (size_t)ks * 1024, st, a);
+    const size_t lds = (size_t)ks * 1024 + 512;      // (the waves' sums of a tile, and of 16 rows' means)
+    if (a.rs_half) hipLaunchKernelGGL((gemm_skinny_bf16_kernel<1, 1, 4, EPI_LN_RESID, OutT, false, 0, true>), dim3(2 * tiles, 1), dim3(ks * 64), lds, st, a);
+    else hipLaunchKernelGGL((gemm_skinny_bf16_kernel<1, 1, 4, EPI_LN_RESID, OutT>), dim3(tiles, cdiv(a.M, 16)), dim3(ks * 64), lds, st, a);
     return true;
 }
 

@@ -40,6 +40,7 @@ struct LayerW {
     void *w_in = nullptr, *w_out = nullptr;         // parallel blocks (nvl_model::joint): QKV and W1 as one matrix (w_qkv and w1 point into it), WO and W2 side by side along K
     float *b_in = nullptr, *b_out = nullptr; int64_t in_rows = 0;      // (rows w_in is allocated with)
     float *ln_qkv = nullptr, *ln_up = nullptr;      // deferred layer norms (nvl_model::ln_ok): S, then B of the projection behind each norm
+    void *ln_wo = nullptr, *ln_w2 = nullptr; float ln_bo = 0.f, ln_b2 = 0.f;      // ... and what the projections in front of them add to a row's mean (MeanShift)
     void* moe_in = nullptr;              // [E][2I (interleaved in bf16 mode)][H]
     void* moe_out_cat = nullptr;         // bf16: W_down of all experts along K, [H_pad][E*I] (decode "dense-masked" form)
     bool mamba = false;                  // a Mamba2 block (attention tensors absent); index among the Mamba2 layers

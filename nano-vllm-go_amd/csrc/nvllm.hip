@@ -395,7 +395,7 @@ extern "C" void nvl_destroy(nvl_model* m) {
         for (int k = 0; k < NVL_T_COUNT; k++) dfree(l.t[k].p);
         if (m->joint) l.w_qkv = l.w1 = nullptr;
         dfree(l.w_in); dfree(l.w_out); dfree(l.b_in); dfree(l.b_out);
-        dfree(l.w_qkv); dfree(l.b_qkv); dfree(l.w1); dfree(l.moe_in); dfree(l.moe_out_cat); dfree(l.ln_qkv); dfree(l.ln_up);
+        dfree(l.w_qkv); dfree(l.b_qkv); dfree(l.w1); dfree(l.moe_in); dfree(l.moe_out_cat); dfree(l.ln_qkv); dfree(l.ln_up); dfree(l.ln_wo); dfree(l.ln_w2);
     }
     if (m->lm_head && m->lm_head != m->g[NVL_T_TOK_EMB].p && m->lm_head != m->g[NVL_T_LM_HEAD].p) dfree(m->lm_head);
     dfree(m->rope_cos); dfree(m->rope_sin); dfree(m->kcache); dfree(m->vcache);
@@ -775,7 +775,23 @@ void init_deferred_layer_norms(nvl_model* m) {
         NVL_HIP(hipGetLastError());
         return out;
     };
+    auto mean_row = [&](const DevTensor& W, int K) {
+        void* out = dmalloc_bytes((int64_t)K * 4);
+        hipLaunchKernelGGL(ln_mean_row_kernel, dim3(K / 32), dim3(64), 0, m->stream, (const bf16_t*)W.p, (bf16_t*)out, H, K);
+        NVL_HIP(hipGetLastError());
+        return out;
+    };
+    auto mean_of = [&](const DevTensor& b) {
+        std::vector<float> v((size_t)H, 0.f);
+        if (b.present()) NVL_HIP(hipMemcpy(v.data(), b.p, (size_t)H * 4, hipMemcpyDeviceToHost));
+        double sum = 0.0;
+        for (float f : v) sum += f;
+        return (float)(sum / H);
+    };
+    NVL_HIP(hipStreamSynchronize(m->stream));      // (the biases are there)
     for (auto& l : m->layers) {
+        l.ln_wo = mean_row(l.t[NVL_T_WO], m->nH * m->hd); l.ln_bo = mean_of(l.t[NVL_T_BO]);
+        l.ln_w2 = mean_row(l.t[NVL_T_W2], m->F); l.ln_b2 = mean_of(l.t[NVL_T_B2]);
         l.ln_qkv = fold(l.w_qkv, m->n_qkv, l.t[NVL_T_ATTN_NORM_W], l.t[NVL_T_ATTN_NORM_B], l.b_qkv);
         l.ln_up = fold(l.w1, m->F, l.t[NVL_T_FFN_NORM_W], l.t[NVL_T_FFN_NORM_B], (const float*)l.t[NVL_T_B1].p);
     }
@@ -1704,11 +1720,12 @@ void set_ln_stats(const nvl_model* m, GemmArgs& a) {
     a.rs_half = defer_half(m, a.M) ? 1 : 0;
     a.rs_tiles = a.rs_half ? m->H / 8 : m->H / 16; a.rs_inv_h = 1.0f / (float)m->H; a.rs_eps = m->cfg.norm_eps;
 }
-void ln_resid_gemm(nvl_model* m, LnChain& ln, const void* A, int lda, const void* W, const float* bias, int M, int K, const DevTensor& norm_w) {
+void ln_resid_gemm(nvl_model* m, LnChain& ln, const void* A, int lda, const void* W, const float* bias, MeanShift mean, int M, int K, const DevTensor& norm_w) {
     GemmArgs a = mk(A, lda, W, m->x, m->H, bias, m->resid_alpha, M, m->H, K);
     set_ln_stats(m, a);
     a.nrm_w = (const float*)norm_w.p; a.nrm_xn = (bf16_t*)m->xn; a.rs_out = ln_buf(m, ln.cur ^ 1);
     a.ln_prev = ln.have ? ln_buf(m, ln.cur) : nullptr; a.ln_mean_in = m->ln_mean + 64 * ln.cur; a.ln_mean_out = m->ln_mean + 64 * (ln.cur ^ 1);
+    a.mean = mean;
     gemm(m, EPI_LN_RESID, true, a);
     ln.cur ^= 1; ln.have = true;
 }
@@ -2230,7 +2247,7 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
             m->site = KS_OPROJ;
             bf16_t* xn_rows = c.use_moe && !defer && norm_copies_rows(m, M) ? (bf16_t*)m->moe_eo : nullptr;      // (for the copy into expert order)
             if (ln_defer) {
-                ln_resid_gemm(m, ln, m->attn_out, qw, l.t[NVL_T_WO].p, bo, M, qw, l.t[NVL_T_FFN_NORM_W]);
+                ln_resid_gemm(m, ln, m->attn_out, qw, l.t[NVL_T_WO].p, bo, MeanShift{(const bf16_t*)l.ln_wo, l.ln_bo}, M, qw, l.t[NVL_T_FFN_NORM_W]);
             } else if (defer) {
                 resid_gemm(m, m->attn_out, qw, l.t[NVL_T_WO].p, bo, m->resid_alpha, M, H, qw, (const float*)l.t[NVL_T_FFN_NORM_W].p);
             } else {
@@ -2250,7 +2267,7 @@ int enqueue_forward(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len
                 // (not the final norm: every workgroup of the LM head would add up the rows' sums: GPT-2 at 1 / 16 rows 14.4 -> 18.1, 15.7 -> 22.0 us)
                 xn_deferred = li + 1 < m->L;
                 m->site = KS_FFN_DOWN;
-                if (xn_deferred) ln_resid_gemm(m, ln, m->hbuf, m->F, l.t[NVL_T_W2].p, (const float*)l.t[NVL_T_B2].p, M, m->F, *nxt_w);
+                if (xn_deferred) ln_resid_gemm(m, ln, m->hbuf, m->F, l.t[NVL_T_W2].p, (const float*)l.t[NVL_T_B2].p, MeanShift{(const bf16_t*)l.ln_w2, l.ln_b2}, M, m->F, *nxt_w);
                 else resid_gemm(m, m->hbuf, m->F, l.t[NVL_T_W2].p, (const float*)l.t[NVL_T_B2].p, m->resid_alpha, M, H, m->F);
             } else {
                 ffn_up(m, l, M, defer);
