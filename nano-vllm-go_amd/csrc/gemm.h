@@ -246,8 +246,10 @@ __device__ __forceinline__ float silu_f(float g) { return g / (1.0f + __expf(-g)
 // ... rounded to bf16 right away: the hardware's reciprocal in place of the division, whose ten instructions for each of a lane's 64 values were 28 of 828 us
 // (16384 x 16384 x 2048, all CUs in their epilogues at once; 4176 x 28672 x 4096 743 -> 730).  Error of the bf16 product silu(g) u against 64 bits: the
 // same to seven digits for |g| <= 0.01 .. 80 (1.64e-3 .. 1.66e-3 in the 2-norm); 4 results of a million round the other way.
-// exp2 -> inf gives 0 and -inf NaN, as the division does
-__device__ __forceinline__ float silu_bf16_f(float g) { return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * g)); }
+// The quarters keep the reciprocal of sums above 2^126 (g < -87.3) out of the denormals, which it returns as zero.  exp2 -> inf gives 0 and -inf NaN, as the division does
+__device__ __forceinline__ float silu_bf16_f(float g) {
+    return 0.25f * g * __builtin_amdgcn_rcpf(__builtin_fmaf(0.25f, __builtin_amdgcn_exp2f(-1.4426950408889634f * g), 0.25f));
+}
 __device__ __forceinline__ float deferred_rstd(const GemmArgs& p, int m);
 
 // ------------------------------------------------------------------------------------------
