@@ -1163,28 +1163,32 @@ __device__ __forceinline__ bf16x8 weight_load(const bf16x8* p) {
 // ------------------------------------------------------------------------------------------
 // MoE routing (moe.go:57-103) of rows first .. first + n - 1 of a 16-row activation tile by a workgroup of `waves` waves: router logits of the tile (E <= 64
 // experts, all of K), softmax, top-k, renormalised weights as the dense gate matrix GemmArgs::moe_gate of the expert projections, or the
-// chosen experts in rank order (RouteIds).  A wave takes an expert tile over a K slice (fragments straight from L2 / HBM, as
-// the skinny kernel; with fewer waves than tiles, several tiles over all of K), the K slices are summed through LDS in order, then a wave
-// routes a row with a lane per expert.  U k-steps of T expert tiles travel together: few waves need more of them (a lone wave, K = 1024, 32 experts: 4 round
-// trips instead of 16; decode steps of 20 rows of 1024 +6 % without).
-// p: A (fragment-major operand, possibly the deferred-norm raw form with rs_in), M, K.  smem: max(waves, 4) + 4 KiB
+// chosen experts in rank order (RouteIds).  A wave takes expert tiles over K slices that lie together (fragments straight from L2 / HBM, as the skinny
+// kernel), the K slices are summed through LDS in order, then a wave routes a row with a lane per expert.  The slices are those of sixteen waves whatever
+// the launch has, so that a row's logits, and with them near ties between experts, depend neither on the batch nor on prompt or step.
+// U k-steps of T expert tiles travel together: few waves need more of them (a lone wave, K = 1024, 32 experts: 4 round trips instead of 16; decode steps
+// of 20 rows of 1024 +6 % without).
+// p: A (fragment-major operand, possibly the deferred-norm raw form with rs_in), M, K.  smem: MOE_ROUTE_LDS
 // ------------------------------------------------------------------------------------------
 struct RouteIds { int32_t* ids; float* w; };      // [row][top_k], or NULL
 template <int U, int T>
 __device__ __forceinline__ void moe_route_rows(const GemmArgs& p, const RouteJob& r, RouteIds out, int tile16, int first, int n, int waves, char* smem) {
-    f32x4* red = (f32x4*)smem;                                   // [waves or expert tiles][64]
-    const int E = r.E, ET = (E + 15) >> 4, KW = waves >= ET ? waves / ET : 1;         // expert tiles (1 .. 4), K slices
-    float* lg = (float*)(smem + (waves > 4 ? waves : 4) * 1024);     // [16][64]
+    f32x4* red = (f32x4*)smem;                                   // [K slices][expert tiles][64]
+    const int E = r.E, ET = (E + 15) >> 4, KW = 16 / ET;         // expert tiles (1 .. 4), K slices
+    float* lg = (float*)(smem + 16 * 1024);                      // [16][64]
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int fr = lane & 15, fg = lane >> 4;
     const int row0 = tile16 * 16;
     const int nks = p.K >> 5, q = nks / KW, rr = nks - q * KW;
     const bool x_live = row0 + fr < p.M;
     const bf16x8 zero = {};
-    const int TS = (ET + T - 1) / T;          // groups of T tiles, which share a row fragment
-    for (int it = wave; it < TS * KW; it += waves) {
-        const int t0 = it % TS * T, kw = it / TS;
-        const int my_steps = q + (kw < rr ? 1 : 0), ks0 = kw * q + (kw < rr ? kw : rr);
+    const int TS = (ET + T - 1) / T, G = waves >= TS ? waves / TS : 1;          // groups of T tiles, which share a row fragment; waves a group
+    auto first_step = [&](int kw) { return kw * q + (kw < rr ? kw : rr); };
+    for (int it = wave; it < TS * G; it += waves) {
+        const int t0 = it % TS * T, part = it / TS, last = (part + 1) * KW / G;
+        int kw = part * KW / G;
+        const int ks0 = first_step(kw), n = first_step(last) - ks0;
+        int slice_end = first_step(kw + 1) - ks0;
         const bf16_t* wp[T];
 #pragma unroll
         for (int t = 0; t < T; t++) wp[t] = r.W + (((int64_t)min(t0 + t, ET - 1) * nks + ks0) * 64 + lane) * 8;
@@ -1192,28 +1196,35 @@ __device__ __forceinline__ void moe_route_rows(const GemmArgs& p, const RouteJob
         f32x4 acc[T];
 #pragma unroll
         for (int t = 0; t < T; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-        int s = 0;
-        for (; s + U <= my_steps; s += U) {
+        auto finish = [&](int done) {          // the slices that end here (several of them where K has fewer steps than slices)
+            while (kw < last && slice_end == done) {
+#pragma unroll
+                for (int t = 0; t < T; t++) {
+                    if (t0 + t < ET) red[(kw * ET + t0 + t) * 64 + lane] = acc[t];
+                    acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+                kw++;
+                slice_end = first_step(kw + 1) - ks0;
+            }
+        };
+        finish(0);
+        for (int s = 0; s < n; s += U) {
             bf16x8 w[T][U], x[U];
 #pragma unroll
             for (int u = 0; u < U; u++) {
+                const int64_t at = (int64_t)min(s + u, n - 1) * 512;
 #pragma unroll
-                for (int t = 0; t < T; t++) w[t][u] = *(const bf16x8*)(wp[t] + (int64_t)(s + u) * 512);
-                x[u] = x_live ? *(const bf16x8*)(xp + (int64_t)(s + u) * 512) : zero;
+                for (int t = 0; t < T; t++) w[t][u] = *(const bf16x8*)(wp[t] + at);
+                x[u] = x_live ? *(const bf16x8*)(xp + at) : zero;
             }
 #pragma unroll
             for (int u = 0; u < U; u++)
+                if (s + u < n) {
 #pragma unroll
-                for (int t = 0; t < T; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t][u], x[u], acc[t], 0, 0, 0);
+                    for (int t = 0; t < T; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t][u], x[u], acc[t], 0, 0, 0);
+                    finish(s + u + 1);
+                }
         }
-        for (; s < my_steps; s++) {
-            const bf16x8 x = x_live ? *(const bf16x8*)(xp + (int64_t)s * 512) : zero;
-#pragma unroll
-            for (int t = 0; t < T; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(wp[t] + (int64_t)s * 512), x, acc[t], 0, 0, 0);
-        }
-#pragma unroll
-        for (int t = 0; t < T; t++)
-            if (t0 + t < ET) red[(kw * ET + t0 + t) * 64 + lane] = acc[t];
     }
     // deferred RMSNorm: the x^2 partials of a row, a lane per 16-byte chunk
     auto sum_squares = [&](int m) {
@@ -1230,6 +1241,7 @@ __device__ __forceinline__ void moe_route_rows(const GemmArgs& p, const RouteJob
     __syncthreads();
     for (int t = wave; t < ET; t += waves) {        // acc of lane (fr, fg): row fr, experts 16 t + 4 fg .. + 3
         f32x4 v = red[t * 64 + lane];
+#pragma unroll 4
         for (int k = 1; k < KW; k++) v += red[(k * ET + t) * 64 + lane];
         *(f32x4*)(lg + fr * 64 + 16 * t + 4 * fg) = v;
     }
@@ -1274,7 +1286,7 @@ __device__ __forceinline__ void moe_route_part(const GemmArgs& p, int id, int wa
     const int per_tile = cdiv_dev(p.M < 16 ? p.M : 16, p.route.rows), t = id / per_tile;
     moe_route_rows<U, T>(p, p.route, RouteIds{nullptr, nullptr}, t, (id - t * per_tile) * p.route.rows, p.route.rows, waves, smem);
 }
-static inline size_t moe_route_lds(int waves) { return (size_t)((waves > 4 ? waves : 4) + 4) * 1024; }
+constexpr size_t MOE_ROUTE_LDS = 20 * 1024;
 // ... set up for a launch with workgroups of `waves` waves
 static inline void moe_route_share(GemmArgs& a, int waves) {
     a.route.rows = waves >= 8 ? 8 : waves >= 4 ? 4 : 2;
@@ -1636,7 +1648,7 @@ constexpr int ROUTE_ROWS = 8;
 static inline dim3 router_gate_grid(int M) { return dim3(cdiv(M, 16), cdiv(M < 16 ? M : 16, ROUTE_ROWS)); }
 // prefill: ids / weights, all 16 rows of a tile in a workgroup (enough workgroups without)
 static __global__ __launch_bounds__(1024) void moe_router_gate_kernel(GemmArgs p, RouteJob job, RouteIds out) {
-    __shared__ __attribute__((aligned(16))) char smem[20 * 1024];
+    __shared__ __attribute__((aligned(16))) char smem[MOE_ROUTE_LDS];
     const int rows = out.ids ? 16 : ROUTE_ROWS;
     moe_route_rows<4, 1>(p, job, out, blockIdx.x, blockIdx.y * rows, rows, 16, smem);
 }
@@ -1951,7 +1963,7 @@ static inline bool launch_gemm_skinny_ntw(hipStream_t st, const GemmArgs& a) {
                     GemmArgs c = a;
                     moe_route_share(c, NTW * ksplit);
                     grid.x += c.route.wgs;
-                    const size_t room = std::max(lds, moe_route_lds(NTW * ksplit));
+                    const size_t room = std::max(lds, MOE_ROUTE_LDS);
                     if (MT == 1) hipLaunchKernelGGL((gemm_skinny_bf16_kernel<1, NTW, 4, EPI, OutT, false, 2>), grid, block, room, st, c);
                     else if (MT == 2) hipLaunchKernelGGL((gemm_skinny_bf16_kernel<2, NTW, 4, EPI, OutT, false, 2>), grid, block, room, st, c);
                     else hipLaunchKernelGGL((gemm_skinny_bf16_kernel<4, NTW, 2, EPI, OutT, false, 2>), grid, block, room, st, c);
@@ -2001,7 +2013,7 @@ static inline bool launch_gemm_skinny_wide(hipStream_t st, const GemmArgs& a) {
     } while (0)
 #define NVL_SKWM(MTv, Uv, Rv, grid, room, args)                                                                          \
     do {                                                                                                               \
-        NVL_LDS_ATTR((gemm_skinny_wide_bf16_kernel<MTv, NTB, Uv, EPI, OutT, false, Rv>), 8 * NTB * MTv * 64 * 16);           \
+        NVL_LDS_ATTR((gemm_skinny_wide_bf16_kernel<MTv, NTB, Uv, EPI, OutT, false, Rv>), std::max<size_t>(8 * NTB * MTv * 1024, MOE_ROUTE_LDS)); \
         hipLaunchKernelGGL((gemm_skinny_wide_bf16_kernel<MTv, NTB, Uv, EPI, OutT, false, Rv>), dim3(grid), dim3(ksplit * 64), \
                            room, st, args);                                                                            \
     } while (0)
@@ -2011,7 +2023,7 @@ static inline bool launch_gemm_skinny_wide(hipStream_t st, const GemmArgs& a) {
             if (a.route.W) {
                 GemmArgs c = a;
                 moe_route_share(c, ksplit);
-                const size_t room = std::max(lds, moe_route_lds(ksplit));
+                const size_t room = std::max(lds, MOE_ROUTE_LDS);
                 if (MT == 1) NVL_SKWM(1, 4, 2, wgs + c.route.wgs, room, c); else if (MT == 2) NVL_SKWM(2, 4, 2, wgs + c.route.wgs, room, c); else NVL_SKWM(4, 2, 2, wgs + c.route.wgs, room, c);
                 return true;
             }

@@ -3,8 +3,6 @@ four expert tiles over one to sixteen waves, one and several row tiles, the narr
 import numpy as np
 import pytest
 
-from conftest import rel_err
-
 pytestmark = pytest.mark.gpu
 
 
@@ -26,4 +24,4 @@ def test_routing_beside_the_up_projection(gpu, experts, top, ffn, n):
         finally:
             gpu.lib().nvl_set_tuning(31, old)
     m.close()
-    assert rel_err(got[1], got[2]) <= 2e-3          # (the router's K slices are summed in another order; what follows rounds to bf16)
+    assert np.array_equal(got[1], got[2])          # (the router's K slices are summed in one order, whatever the launch)
