@@ -1171,7 +1171,9 @@ __device__ __forceinline__ bf16x8 weight_load(const bf16x8* p) {
 // p: A (fragment-major operand, possibly the deferred-norm raw form with rs_in), M, K.  smem: MOE_ROUTE_LDS
 // ------------------------------------------------------------------------------------------
 struct RouteIds { int32_t* ids; float* w; };      // [row][top_k], or NULL
-template <int U, int T>
+// ALONE: sixteen waves, a slice of a tile and a row each: without the loops a launch of its own takes 5.5 us instead of 6.4 (1 row of 1024, 32 experts; code
+// that is fetched cold)
+template <int U, int T, bool ALONE = false>
 __device__ __forceinline__ void moe_route_rows(const GemmArgs& p, const RouteJob& r, RouteIds out, int tile16, int first, int n, int waves, char* smem) {
     f32x4* red = (f32x4*)smem;                                   // [K slices][expert tiles][64]
     const int E = r.E, ET = (E + 15) >> 4, KW = 16 / ET;         // expert tiles (1 .. 4), K slices
@@ -1182,8 +1184,30 @@ __device__ __forceinline__ void moe_route_rows(const GemmArgs& p, const RouteJob
     const int nks = p.K >> 5, q = nks / KW, rr = nks - q * KW;
     const bool x_live = row0 + fr < p.M;
     const bf16x8 zero = {};
-    const int TS = (ET + T - 1) / T, G = waves >= TS ? waves / TS : 1;          // groups of T tiles, which share a row fragment; waves a group
     auto first_step = [&](int kw) { return kw * q + (kw < rr ? kw : rr); };
+    if constexpr (ALONE) {
+        static_assert(T == 1, "a tile a wave");
+        const int tile = wave % ET, kw = wave / ET;
+        const int n = kw < KW ? q + (kw < rr ? 1 : 0) : 0, ks0 = first_step(kw);      // (three tiles leave a wave idle)
+        const bf16_t* wp = r.W + (((int64_t)tile * nks + ks0) * 64 + lane) * 8;
+        const bf16_t* xp = (const bf16_t*)p.A + (((int64_t)tile16 * nks + ks0) * 64 + lane) * 8;
+        f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+        int s = 0;
+        for (; s + U <= n; s += U) {
+            bf16x8 w[U], x[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                w[u] = *(const bf16x8*)(wp + (int64_t)(s + u) * 512);
+                x[u] = x_live ? *(const bf16x8*)(xp + (int64_t)(s + u) * 512) : zero;
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u], x[u], acc, 0, 0, 0);
+        }
+        for (; s < n; s++)
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(wp + (int64_t)s * 512), x_live ? *(const bf16x8*)(xp + (int64_t)s * 512) : zero, acc, 0, 0, 0);
+        red[wave * 64 + lane] = acc;
+    } else {
+    const int TS = (ET + T - 1) / T, G = waves >= TS ? waves / TS : 1;          // groups of T tiles, which share a row fragment; waves a group
     for (int it = wave; it < TS * G; it += waves) {
         const int t0 = it % TS * T, part = it / TS, last = (part + 1) * KW / G;
         int kw = part * KW / G;
@@ -1226,6 +1250,7 @@ __device__ __forceinline__ void moe_route_rows(const GemmArgs& p, const RouteJob
                 }
         }
     }
+    }
     // deferred RMSNorm: the x^2 partials of a row, a lane per 16-byte chunk
     auto sum_squares = [&](int m) {
         const f32x4* src = (const f32x4*)(p.rs_in + (int64_t)m * p.rs_tiles);
@@ -1246,9 +1271,9 @@ __device__ __forceinline__ void moe_route_rows(const GemmArgs& p, const RouteJob
         *(f32x4*)(lg + fr * 64 + 16 * t + 4 * fg) = v;
     }
     __syncthreads();
-    for (int i = wave; i < end; i += waves) {
+    for (int i = wave; i < end; i += ALONE ? 16 : waves) {
         const int row = first + i, m = row0 + row;
-        if (p.rs_in && i != wave) ssq = sum_squares(m);
+        if (!ALONE && p.rs_in && i != wave) ssq = sum_squares(m);
         const float rstd = p.rs_in ? 1.0f / sqrtf(ssq * p.rs_inv_h + p.rs_eps) : 1.0f;
         const float v = (lane < E) ? lg[row * 64 + lane] * rstd + (r.bias ? r.bias[lane] : 0.f) : -INFINITY;
         if (r.logits && lane < E) r.logits[(int64_t)m * r.logits_ld + lane] = v;
@@ -1274,10 +1299,12 @@ __device__ __forceinline__ void moe_route_rows(const GemmArgs& p, const RouteJob
         }
         if (out.ids) {
             if (lane < E && rank < r.top_k) { out.ids[(int64_t)m * r.top_k + rank] = lane; out.w[(int64_t)m * r.top_k + rank] = prob / wsum; }
+            if (ALONE) return;
             continue;
         }
         if (lane < E) r.gate[(int64_t)m * r.gate_ld + lane] = rank < r.top_k ? prob / wsum : 0.f;      // moe.go:103
         for (int e2 = E + lane; e2 < r.gate_ld; e2 += 64) r.gate[(int64_t)m * r.gate_ld + e2] = e2 < E + r.n_always ? 1.0f : 0.f;
+        if (ALONE) return;
     }
 }
 // workgroup `id` of the RouteJob of a launch
@@ -1650,7 +1677,7 @@ static inline dim3 router_gate_grid(int M) { return dim3(cdiv(M, 16), cdiv(M < 1
 static __global__ __launch_bounds__(1024) void moe_router_gate_kernel(GemmArgs p, RouteJob job, RouteIds out) {
     __shared__ __attribute__((aligned(16))) char smem[MOE_ROUTE_LDS];
     const int rows = out.ids ? 16 : ROUTE_ROWS;
-    moe_route_rows<4, 1>(p, job, out, blockIdx.x, blockIdx.y * rows, rows, 16, smem);
+    moe_route_rows<4, 1, true>(p, job, out, blockIdx.x, blockIdx.y * rows, rows, 16, smem);
 }
 #endif
 
