@@ -1847,13 +1847,7 @@ bool moe_dense_ok(const nvl_model* m, const LayerW& l, int M) {
     return !m->f32 && M <= 64 && g_moe_dense && l.moe_out_cat && m->moe_part && !m->keep_hidden && m->H % 4 == 0 &&
            m->H <= 1024 * NORM_ROW_MAXCH && g_force_tile == 0;
 }
-// Does a decode batch route inside the experts' up launch?  The launch that this saves is some 8 us (16 rows of 1024 and 32 experts; 2048 and 6 rows: 7.4
-// and the gap); not knowing the chosen experts, the up projection streams them all, at 6 TB/s.  Either all that a token leaves out costs
-// little more than that, or a batch is expected to leave out next to nothing, were its choices even.
-bool moe_route_beside(int M, int E, int k, double expert_bytes) {
-    const double out_us = E > k ? (E - k) * expert_bytes / 6e6 : 0.0, expected_us = E > k ? pow(1.0 - (double)k / E, M) * E * expert_bytes / 6e6 : 0.0;
-    return g_moe_fused_route == 1 && (expected_us < 1.5 || (out_us < 9.0 && expected_us < 6.0));
-}
+bool moe_route_beside(int M, int E, int k, double expert_bytes) { return g_moe_fused_route == 1 && moe_streams_all(M, E, k, expert_bytes); }
 // deferred_norm: m->xn holds xn_raw = bf16(x * w_norm) and m->rs_part the x^2 partials (the O projection carried the FFN
 // norm): the router and the expert-up projection scale their accumulators by rstd[m] instead of reading a normed operand
 // next_norm_w (decode, dense-masked form only): the down projection carries the NEXT norm (the following layer's attention

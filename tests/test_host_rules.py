@@ -1,0 +1,53 @@
+"""Rules of the host code that no result shows, compiled from the headers and run without a device."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HIPCC = "/opt/rocm/bin/hipcc" if os.path.exists("/opt/rocm/bin/hipcc") else shutil.which("hipcc")
+
+
+def run(tmp_path, source):
+    src, exe = tmp_path / "rule.hip", tmp_path / "rule"
+    src.write_text(source)
+    subprocess.run([HIPCC, "-std=c++17", "--offload-arch=gfx950", "-w", "-DNVL_GEMM_INST=0", "-I", os.path.join(ROOT, "nano-vllm-go_amd", "csrc"), str(src), "-o", str(exe)], check=True, timeout=300)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
+
+
+# tiles: columns a workgroup covers, 16 .. 64 in the decode and ring kernels, 128 and 256 in the tile kernels
+@pytest.mark.skipif(HIPCC is None, reason="no hipcc")
+def test_tiles_of_joint_matrices_stay_inside(tmp_path):
+    run(tmp_path, r"""
+#include "common.h"
+int main() {
+    const int tiles[] = {16, 32, 64, 128, 256};
+    auto last = [](int64_t first, int64_t n, int bn) { return first + (n + bn - 1) / bn * bn; };
+    for (int64_t a = 16; a <= 5120; a += 16)
+        for (int64_t b = 64; b <= 20480; b += 64)
+            for (int bn : tiles) {
+                const int64_t rows = nvl::joint_weight_rows(a, b);
+                if (last(0, a + b, bn) > rows || last(a, b, bn) > rows || last(0, a, bn) > rows) { printf("%lld + %lld rows: tiles of %d read past %lld\n", (long long)a, (long long)b, bn, (long long)rows); return 1; }
+            }
+    return 0;
+}
+""")
+
+
+@pytest.mark.skipif(HIPCC is None, reason="no hipcc")
+def test_all_experts_are_streamed_only_at_little_cost(tmp_path):
+    """Rows that choose the same experts, answers to one prompt for instance, leave the others alone however many rows there are: what streaming them costs then
+    stays near the launch that it saves (8 us; 9 at 6 TB/s)."""
+    run(tmp_path, r"""
+#include "gemm.h"
+int main() {
+    for (int M = 1; M <= 64; M++)
+        for (int E = 2; E <= 64; E++)
+            for (int k = 1; k <= E; k++)
+                for (double bytes = 1 << 14; bytes < 1 << 29; bytes *= 1.5)
+                    if (nvl::moe_streams_all(M, E, k, bytes) && (E - k) * bytes / 6e6 > 9.0) { printf("%d rows, %d of %d experts of %.0f bytes\n", M, k, E, bytes); return 1; }
+    return 0;
+}
+""")
