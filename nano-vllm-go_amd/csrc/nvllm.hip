@@ -961,7 +961,7 @@ extern "C" int nvl_finalize(nvl_model* m) {
     m->xn = dmalloc_bytes(Mp * H * (int64_t)m->wsize);
     m->qkv = dmalloc<float>(Mmax * m->n_qkv);
     m->q = dmalloc_bytes(Mmax * qw * (int64_t)m->wsize);
-    m->attn_out = dmalloc_bytes(Mp * qw * (int64_t)m->wsize);
+    if (!m->joint) m->attn_out = dmalloc_bytes(Mp * qw * (int64_t)m->wsize);      // (joint: columns of hbuf)
     if (!m->f32 && (m->hd == 64 || m->hd == 128)) {     // partial results of a split decode attention (attn.h)
         m->attn_records = (int)std::min<int64_t>(ATTN_SPLIT_PAIRS, S * m->nKV * cdiv(m->group, 16)) * ATTN_SPLIT_MAX;
         m->attn_part = dmalloc<float>((int64_t)m->attn_records * (m->hd == 64 ? attn_part_floats<64>() : attn_part_floats<128>()));
@@ -972,7 +972,7 @@ extern "C" int nvl_finalize(nvl_model* m) {
     const int64_t hw = m->F + (m->joint ? qw : 0);
     m->hbuf = dmalloc_bytes(round_up(Mmax * k, 64) * hw * (int64_t)m->wsize);
     NVL_HIP(hipMemsetAsync(m->xn, 0, (size_t)(Mp * H) * m->wsize, m->stream));
-    NVL_HIP(hipMemsetAsync(m->attn_out, 0, (size_t)(Mp * qw) * m->wsize, m->stream));
+    if (m->attn_out) NVL_HIP(hipMemsetAsync(m->attn_out, 0, (size_t)(Mp * qw) * m->wsize, m->stream));
     NVL_HIP(hipMemsetAsync(m->hbuf, 0, (size_t)(round_up(Mmax * k, 64) * hw) * m->wsize, m->stream));
     if (m->f32 && (c.activation_type == NVL_ACT_SWIGLU || c.use_moe)) m->h2 = dmalloc<float>(Mmax * k * 2 * m->F);
     m->xn_last = dmalloc_bytes(round_up(S, 64) * H * (int64_t)m->wsize);

@@ -69,3 +69,17 @@ def test_last_tiles_of_the_joint_matrix(wide, n):
         out = [m.forward_batch([0], [first], [0])[0], m.forward_batch(ids, [[t] for t in tokens], [40] + [0] * (n - 1))[0], m.forward_batch(ids, [[t] for t in steps], [41] + [1] * (n - 1))[0]]
         got.append(np.concatenate(out))
     assert rel_err(got[1], got[0]) <= TOL
+
+
+def test_workspace_holds_attention_once(gpu):
+    """Attention writes beside the feed-forward's columns: as much memory as blocks whose projections are apart (two multipliers) take, not 64 MiB more."""
+    import torch
+    used = []
+    for residual in (0.25, 0.75, 0.25):          # (the first one is where the library's own first allocations go)
+        cfg = gpu.synth.tiny_config("falcon", hidden=256, num_heads=8, num_kv_heads=2, head_dim=64, ffn_dim=2048, attention_type="gqa", num_layers=1, attention_multiplier=0.25, residual_multiplier=residual)
+        w = gpu.synth.make_weights(cfg, seed=8, scale=0.05)
+        free = torch.cuda.mem_get_info()[0]
+        m = gpu.HipTransformerModel(cfg, w, precision="bf16", max_seqs=1, max_batch_tokens=65536)
+        used.append(free - torch.cuda.mem_get_info()[0])
+        m.close()
+    assert used[2] - used[1] < 32 << 20, used
