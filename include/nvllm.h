@@ -544,7 +544,7 @@ int nvl_op_sample(int device, const float* logits, int rows, int V, const nvl_sa
 int nvl_bench_gemm(int device, int M, int N, int K, int epi, int force_bnt, int force_ksplit, int iters,
                    float* avg_us);
 /* Process-wide tuning override used by tests and sweeps.  key 0: prefill GEMM kernel (0 automatic,
- * 1 = 128x128 two-stage, 2 = 256x128 three-stage, 3 = 256x256 two-stage, 5 = 256x256 ping-pong).
+ * 1 = 128x128, a ring of K tiles, 2 = 256x128 three-stage, 3 = 256x256 two-stage, 5 = 256x256 ping-pong).
  * key 1: K slices of the decode residual projections (0 automatic, 1 never split, 2, 4).
  * key 2: decode (M <= 64) GEMM form: 0 automatic, 1/2/4 = narrow form with that many weight tiles per workgroup,
  * 8 = wide-N form (4 weight tiles per wave).
@@ -559,7 +559,6 @@ int nvl_bench_gemm(int device, int M, int N, int K, int epi, int force_bnt, int 
  * grid size, 2, 4, 8).  key 16: prefill MoE copies the token rows into expert order before the grouped GEMM (1, default)
  * or gathers them per lane inside it (0).  key 17: prefill MoE grouped GEMMs: 0 (default) = 256-row segments on the
  * ping-pong kernel beyond 64 rows an expert in the mean, 128-row segments up to there; 128 / 256 = the tile kernels with that many rows per m-tile.
- * key 19: decode-sized MoE batches run the grouped GEMMs on the four-stage 128x128 instance (1, default) or two stages (0).
  * key 18: largest prompt batch (tokens) whose QKV projection leaves fp32 rows to rope_kv_kernel instead of rotating and placing
  * them itself (default -1: by size; 0: none).
  * key 38: projections of up to 512 rows (beyond 64 as far as key 11 goes) on their own kernel, K split over workgroups (1, default,

@@ -12,9 +12,9 @@
 //     apart, K in 32-wide stages through a 4-slot LDS ring filled by global_load_lds_dwordx4, so one group's fragment
 //     reads run beside the other's MFMAs.  MFMA-bound.  Also the grouped launch of the MoE prefill (GemmArgs::tile_map:
 //     an m-tile = an expert's 256-row segment of the expert-ordered row buffer).
-//   * gemm_bf16_kernel (prefill, fewer tiles; decode-sized MoE expert groups): lock-step tiles, by default 128x128x64 with 4 waves
+//   * gemm_bf16_kernel (prefill, fewer tiles; decode-sized MoE expert groups): by default 128x128 tiles with 4 waves
 //     (2x2), each wave a 64x64 sub-tile as 4x4 v_mfma_f32_16x16x32_bf16 accumulators; operand blocks go HBM->LDS with
-//     global_load_lds_dwordx4 (one contiguous KiB per wave-instruction, no VGPR round trip), double-buffered; the LDS
+//     global_load_lds_dwordx4 (one contiguous KiB per wave-instruction, no VGPR round trip), a ring of four K tiles of 32; the LDS
 //     image is lane-linear so the fragment ds_read_b128s are bank-conflict-free with no swizzle.
 //   * gemm_skinny_bf16_kernel / gemm_skinny_wide_bf16_kernel (decode, M <= 64): weight-streaming, HBM-bound (see below);
 //     the residual projections also carry the deferred RMSNorm (GemmArgs::rs_out / rs_in); their MOE instantiations run
@@ -123,7 +123,6 @@ struct GemmArgs {
     int64_t w_expert_stride;
     int x_mask;             // decode kernels: rows >= M of a 16-row activation tile are not fetched (set when M % 16 != 0)
     int grp_bm;             // rows per m-tile of the grouped launch (128, or 256: the 256x128 three-stage instance)
-    int grp_deep;           // grouped launch on the four-stage 128x128 instance (decode-sized MoE batches)
     union {
         QkvEpi qkv;         // EPI_QKV
         RouteJob route;     // masked experts (epi_moe with moe_gate)
@@ -439,7 +438,6 @@ __device__ __forceinline__ void epilogue_qkv_head(const GemmArgs& p, int m, int 
 // bf16 MFMA kernel (prefill), one template, instances chosen per shape by the launcher:
 //   <128,128, 2,2, 4, BK 32>  4 waves, wave tile 64x64, a ring of 4 K tiles of 32 (64 KiB, 2 workgroups/CU): what does not fill
 //                             256x256 tiles (below)
-//   <128,128, 2,2, 4>  4 waves, four K tiles of 64 (128 KiB): decode-sized MoE batches
 //   <256,128, 4,2, 3>  8 waves, wave tile  64x64, 3 LDS stages (144 KiB): two K tiles in flight
 //   <256,256, 2,4, 2>  8 waves, wave tile 128x64, 2 LDS stages (128 KiB): least LDS traffic per MFMA
 //                      ((8+4) fragment reads per 32 MFMAs instead of (4+4) per 16)
@@ -2198,13 +2196,8 @@ static inline void launch_gemm_grouped(hipStream_t st, const GemmArgs& a, int ma
                            lds3, st, a);
         return;
     }
-    if (a.grp_deep) {           // decode MoE: a handful of rows per expert, one workgroup per CU streaming 128 weight rows —
-        constexpr int lds4 = gemm_lds_bytes<128, 128, 4>();   // latency-bound with two stages (16 K tiles, one round trip each)
-        NVL_LDS_ATTR((gemm_bf16_kernel<128, 128, 2, 2, 4, EPI, OutT>), lds4);
-        hipLaunchKernelGGL((gemm_bf16_kernel<128, 128, 2, 2, 4, EPI, OutT>), dim3(cdiv(a.N, 128) * max_mtiles), dim3(256),
-                           lds4, st, a);
-        return;
-    }
+    // (decode-sized batches too, a handful of rows an expert: us a layer of 1 / 4 / 16 / 64 rows, 32 experts, 8 a token, with four K tiles of 64 in 128 KiB ->
+    // here: 512 x 2048 75 -> 69.6, 86.6 -> 79.7, 97.2 -> 92.8, 120.2 -> 117.2; 1024 x 4096 128 -> 124, 202 -> 184, 235 -> 229, 271 -> 267; 512 x 1024 3 %)
     constexpr int lds = gemm_lds_bytes<128, 128, 4, 32>();
     NVL_LDS_ATTR((gemm_bf16_kernel<128, 128, 2, 2, 4, EPI, OutT, 32>), lds);
     hipLaunchKernelGGL((gemm_bf16_kernel<128, 128, 2, 2, 4, EPI, OutT, 32>), dim3(cdiv(a.N, 128) * max_mtiles), dim3(256),

@@ -1635,8 +1635,7 @@ bool qkv_rows(int M, int64_t N, int64_t K) {
     return M <= 16 ? false : M <= 32 ? N * K >= (4 << 20) : M <= 64 ? true : M <= 128 && K < 2048;
 }
 static int g_moe_dense = 1;    // nvl_set_tuning key 22: decode MoE as two dense-masked projections (gemm.h moe_gate); 0 = sort + grouped GEMMs
-static int g_moe_deep = 1;     // nvl_set_tuning key 19: four-stage grouped GEMM for decode-sized MoE batches (0 = two stages)
-static int g_moe_bm = 0;       // nvl_set_tuning key 17: prefill MoE grouped GEMMs: 0 = by the rows an expert has (moe_pp_ok), 128 / 256 = the lock-step tile kernels
+static int g_moe_bm = 0;       // nvl_set_tuning key 17: prefill MoE grouped GEMMs: 0 = by the rows an expert has (moe_pp_ok), 128 / 256 = gemm_bf16_kernel with that many rows a tile
 static int g_moe_gather = 1;   // nvl_set_tuning key 16: prefill MoE gathers the token rows into expert order before the grouped GEMM (0 = per-lane gather inside it)
 static int g_moe_defer_down = 1;    // nvl_set_tuning key 33: MoE decode: the last of the K slices' workgroups completes the residual and carries the next norm
                                     // (deferred RMSNorm producer, gemm.h split_finish_wave); 0: slices left to a norm launch
@@ -1833,12 +1832,12 @@ void moe_expert_gemms(nvl_model* m, const MoeW& w, int M, int BM, bool pp, bool 
         NVL_HIP(hipGetLastError());
         a.A = m->moe_xg; a.a_rows = nullptr;
     }
-    a.w_expert_stride = (int64_t)2 * I * H; a.grp_bm = pp ? 512 : BM; a.grp_deep = small && g_moe_deep;
+    a.w_expert_stride = (int64_t)2 * I * H; a.grp_bm = pp ? 512 : BM;
     m->site = KS_MOE_UP; m->site_bytes = (e_touch * 2 * I * H + (double)pairs * H + (double)pairs * I) * (double)m->wsize;
     a.glu_limit = w.limit; a.glu_slope = CLAMPED_GLU_SLOPE;
     gemm(m, w.limit > 0.f ? EPI_CLAMP_GLU : EPI_SWIGLU, false, a, 2.0 * pairs * 2 * I * H);
     GemmArgs d = mk(m->hbuf, I, w.down, m->moe_eo, H, nullptr, 1.f, max_mtiles, H, I);
-    d.tile_map = m->moe_tile_map; d.n_mtiles = m->moe_n_mtiles; d.w_expert_stride = (int64_t)H * I; d.grp_bm = pp ? 512 : BM; d.grp_deep = small && g_moe_deep;
+    d.tile_map = m->moe_tile_map; d.n_mtiles = m->moe_n_mtiles; d.w_expert_stride = (int64_t)H * I; d.grp_bm = pp ? 512 : BM;
     m->site = KS_MOE_DOWN; m->site_bytes = (e_touch * H * I + (double)pairs * I) * (double)m->wsize + (double)pairs * H * 4.0;
     gemm(m, EPI_STORE, true, d, 2.0 * pairs * H * I);
 }
