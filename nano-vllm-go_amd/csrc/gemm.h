@@ -96,8 +96,9 @@ struct RouteJob {
 
 struct JointEpi { float* rows; int ld, n; };      // EPI_JOINT; n a multiple of 16
 
-// EPI_LN_RESID: what the projection adds to a row's mean.  w: the mean of W's rows, in bf16 and the rest of it in bf16, [K/32][those two][32]; b: the mean of the bias
+// what a residual projection adds to a row's mean.  w: the mean of W's rows, in bf16 and the rest of it in bf16, [K/32][those two][32]; b: the mean of the bias
 struct MeanShift { const bf16_t* w; float b; };
+struct LnResidEpi { MeanShift added; const float *prev, *mean_in; float* mean_out; };      // EPI_LN_RESID (GemmArgs::ln_s)
 
 struct GemmArgs {
     const void* A;          // bf16: fragment-major [M_pad16][K]; f32: row-major [M][lda]
@@ -110,7 +111,11 @@ struct GemmArgs {
     float alpha;            // EPI_RESID multiplier
     float glu_limit, glu_slope;     // EPI_CLAMP_GLU
     float glu_limit2; int glu_from2;      // ... masked experts: the limit of output columns from glu_from2 on
-    const int32_t* tok_ids; const bf16_t* tok_table; int64_t tok_ld;      // EPI_GELU_TOK: row-major, rows of 4 k entries
+    const int32_t* tok_ids; int64_t tok_ld;      // EPI_GELU_TOK: row-major, rows of 4 k entries
+    union {
+        const bf16_t* tok_table;
+        const float* ln_s;      // epi_ln: S of the deferred layer norm, which the last comment here explains
+    };
     int M, N, K;            // logical sizes
     const int32_t* seg;     // optional device {start,end}: rows [start,end) of A (via a_rows if set)
                             // and of C; M is then only the grid bound (MoE expert segments)
@@ -127,7 +132,7 @@ struct GemmArgs {
         QkvEpi qkv;         // EPI_QKV
         RouteJob route;     // masked experts (epi_moe with moe_gate)
         JointEpi joint;     // EPI_JOINT
-        MeanShift mean;     // EPI_LN_RESID
+        LnResidEpi ln;      // EPI_LN_RESID
     };
     GroupedEpi grp;         // EPI_GROUPED
     // decode kernel, EPI_RESID only: K split over gridDim.y = sk_slices workgroups per column block.  Each
@@ -174,16 +179,15 @@ struct GemmArgs {
     // Deferred layer norm (epi_ln; M <= 64): ((x - mean) w / sd + b) W == rstd ((x - s) w W - (mean - s) S) + B for any s, S[n] = sum_k W[n][k] w[k] and
     // B[n] = bias[n] + sum_k W[n][k] b[k] from the weights alone.  Producer: xn_raw = bf16((x - s) w) and per tile the pair of sums of x - s and
     // (x - s)^2.  The operand's rounding and the variance cost sqrt(1 + d^2) times a norm launch's where s misses the row's mean by d of its deviations, so s is
-    // that mean but for rounding: the mean before (ln_prev: the pairs of the norm before, or NULL, where it was a launch of its own, and ln_mean_in) and what
-    // the projection adds to it, its operand times `mean` (one more product a K step; a mean that is 100 deviations away: d < 0.01).  Consumer: bias is B.
+    // that mean but for rounding: the mean before (ln.prev: the pairs of the norm before, or NULL, where it was a launch of its own, and ln.mean_in) and what
+    // the projection adds to it, its operand times ln.added (one more product a K step; a mean that is 100 deviations away: d < 0.01).  Consumer: bias is B.
     // A norm launch is 3.3 us (1 row) to 4.2 (16) and a boundary; the sums cost the four projections of a layer 0.5 to 1.7 us each, finding s
     // the two residual ones 0.6 (GPT-2, a step of 1 sequence: with the mean before in its place 357 us, 371 so).  GPT-2, norm launches -> carried, us a step of 1 / 16 / 24 / 40 / 64 sequences:
     // 388 -> 371, 448 -> 430, 495 -> 468, 518 -> 498, 575 -> 565; prompts of 11 / 3 x 11 / 64 tokens 470 -> 445, 544 -> 520, 550 -> 536.
     // Error of the logits against 64 bits over 240 calls: mean log ratio to the norm launches -0.001 +- 0.002.
-    const float* ln_s;
-    const float *ln_prev, *ln_mean_in;
-    float* ln_mean_out;
 };
+// blockDim lies 12 bytes behind the arguments.  The decode kernels load it with rs_in: a cache line more is 0.2 us of a 3.4 us launch (8 rows of 2048 x 1024)
+static_assert(((sizeof(GemmArgs) + 12) >> 6) == (offsetof(GemmArgs, rs_in) >> 6), "arguments that are loaded together");
 // the routing weight that row `lane` of the batch (M <= 64) gives expert e
 __device__ __forceinline__ float moe_gate_of(const GemmArgs& p, int e) {
     const int lane = threadIdx.x & 63;
@@ -1489,7 +1493,7 @@ __global__ __launch_bounds__(skinny_waves(EPIV) * 64) void gemm_skinny_bf16_kern
     constexpr int UC = LN_SHIFT ? U : 1;
     bf16x8 cA[UC], cB[UC];
     f32x4 mean_acc = f32x4{0.f, 0.f, 0.f, 0.f};
-    const bf16x8* cp = LN_SHIFT ? (const bf16x8*)p.mean.w + (int64_t)ks0 * 8 + (fr & 1) * 4 + fg : nullptr;
+    const bf16x8* cp = LN_SHIFT ? (const bf16x8*)p.ln.added.w + (int64_t)ks0 * 8 + (fr & 1) * 4 + fg : nullptr;
     auto load_blk = [&](bf16x8 (&w)[U], bf16x8 (&x)[U][MT], bf16x8 (&c)[UC], int b) {
 #pragma unroll
         for (int u = 0; u < U; u++) {
@@ -1527,8 +1531,8 @@ __global__ __launch_bounds__(skinny_waves(EPIV) * 64) void gemm_skinny_bf16_kern
         static_assert(MT == 1 && NTW == 1, "one epilogue element");
         const int m = 16 * i_off + fr;
         const bool live = wave == 0 && m < p.M;
-        if (live) ln_shift = p.ln_mean_in[m];
-        pairs.fetch(p.ln_prev, p.rs_tiles, m, live && p.ln_prev);
+        if (live) ln_shift = p.ln.mean_in[m];
+        pairs.fetch(p.ln.prev, p.rs_tiles, m, live && p.ln.prev);
     }
     if constexpr (MOE != 0 && EPI == EPI_RESID) {
         for (int b = 0; b < nblk; b += 2) {
@@ -1586,8 +1590,8 @@ __global__ __launch_bounds__(skinny_waves(EPIV) * 64) void gemm_skinny_bf16_kern
         float added = lo[0];
 #pragma unroll
         for (int w = 1; w < 8; w++) added += w < ksplit ? (w < 4 ? lo[w] : hi[w - 4]) : 0.f;
-        ln_shift += p.alpha * (added + p.mean.b);
-        if (blockIdx.x == 0 && wave == 0 && fg == 0 && 16 * i_off + fr < p.M) p.ln_mean_out[16 * i_off + fr] = ln_shift;
+        ln_shift += p.alpha * (added + p.ln.added.b);
+        if (blockIdx.x == 0 && wave == 0 && fg == 0 && 16 * i_off + fr < p.M) p.ln.mean_out[16 * i_off + fr] = ln_shift;
     }
     auto ksum = [&](int t, int i) {
         f32x4 s = red[((t * ksplit) * MT + i) * 64 + lane];

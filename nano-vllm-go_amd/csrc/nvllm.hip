@@ -1719,12 +1719,11 @@ void set_ln_stats(const nvl_model* m, GemmArgs& a) {
     a.rs_half = defer_half(m, a.M) ? 1 : 0;
     a.rs_tiles = a.rs_half ? m->H / 8 : m->H / 16; a.rs_inv_h = 1.0f / (float)m->H; a.rs_eps = m->cfg.norm_eps;
 }
-void ln_resid_gemm(nvl_model* m, LnChain& ln, const void* A, int lda, const void* W, const float* bias, MeanShift mean, int M, int K, const DevTensor& norm_w) {
+void ln_resid_gemm(nvl_model* m, LnChain& ln, const void* A, int lda, const void* W, const float* bias, MeanShift added, int M, int K, const DevTensor& norm_w) {
     GemmArgs a = mk(A, lda, W, m->x, m->H, bias, m->resid_alpha, M, m->H, K);
     set_ln_stats(m, a);
     a.nrm_w = (const float*)norm_w.p; a.nrm_xn = (bf16_t*)m->xn; a.rs_out = ln_buf(m, ln.cur ^ 1);
-    a.ln_prev = ln.have ? ln_buf(m, ln.cur) : nullptr; a.ln_mean_in = m->ln_mean + 64 * ln.cur; a.ln_mean_out = m->ln_mean + 64 * (ln.cur ^ 1);
-    a.mean = mean;
+    a.ln = LnResidEpi{added, ln.have ? ln_buf(m, ln.cur) : nullptr, m->ln_mean + 64 * ln.cur, m->ln_mean + 64 * (ln.cur ^ 1)};
     gemm(m, EPI_LN_RESID, true, a);
     ln.cur ^= 1; ln.have = true;
 }
