@@ -54,7 +54,8 @@ enum GemmEpi {
     EPI_JOINT = 16,      // two projections of one operand: the first joint.n columns are stored to fp32 rows, the others C = gelu_tanh(acc + bias)
 };
 constexpr bool epi_ln(int epi) { return epi >= 12 && epi <= 15; }
-constexpr int skinny_waves(int epi) { return epi_ln(epi) ? 8 : 16; }      // most waves of a workgroup of the narrow decode form (the pairs of a layer norm take registers)
+// most waves of a workgroup of the narrow decode form (the pairs of a layer norm take registers, and the routing beside several row tiles)
+constexpr int skinny_waves(int epi, bool route_rows = false) { return epi_ln(epi) || route_rows ? 8 : 16; }
 constexpr int epi_base(int epi) { return !epi_ln(epi) ? epi : epi == 15 ? 4 : epi == 14 ? 3 : epi - 12; }
 
 constexpr bool epi_moe(int epi) { return epi == 2 || epi == 6; }      // ... with instances for masked experts
@@ -1403,7 +1404,7 @@ __device__ __forceinline__ void skinny_pass_remap(GemmArgs& p, int& bx) {
 // 43.9 -> 51 us, their registers spill).
 // MOE: 1 masked experts, 2 (up) all experts, the launch's first workgroups route.
 template <int MT, int NTW, int U, int EPIV, typename OutT, bool PASSES = false, int MOE = 0, bool HALF = false, bool EXTRA = false>
-__global__ __launch_bounds__(skinny_waves(EPIV) * 64) void gemm_skinny_bf16_kernel(GemmArgs p) {
+__global__ __launch_bounds__(skinny_waves(EPIV, MOE == 2 && MT > 1) * 64) void gemm_skinny_bf16_kernel(GemmArgs p) {
     constexpr int EPI = epi_base(EPIV);
     constexpr bool LN = epi_ln(EPIV);
     constexpr bool SCALED = EXTRA && MOE == 0, COMPLETES = EXTRA && MOE != 0;
@@ -1969,7 +1970,7 @@ static inline bool launch_gemm_skinny_ntw(hipStream_t st, const GemmArgs& a) {
         const int64_t budget = (int64_t)g_narrow_waves * ((a.moe_gate && epi_moe(EPI)) ? 2 : 1);
         while (ksplit > 1 && (int64_t)nblocks * KS * NTW * ksplit > budget) ksplit >>= 1;
     }
-    while (ksplit > 1 && ((a.K >> 5) / (ksplit * KS) < U || ksplit * NTW > skinny_waves(EPI))) ksplit >>= 1;   // >= one block of U k-steps per wave
+    while (ksplit > 1 && ((a.K >> 5) / (ksplit * KS) < U || ksplit * NTW > skinny_waves(EPI, a.moe_gate && epi_moe(EPI) && MT > 1))) ksplit >>= 1;   // >= one block of U k-steps per wave
     if (a.moe_gate && EPI == EPI_RESID) {      // MoE down: every wave's K range is exactly one expert (the skip test needs it)
         ksplit = a.moe_E / KS;
         if (ksplit < 1 || ksplit * KS != a.moe_E || ksplit > 16 || (a.moe_I >> 5) < 1) return false;

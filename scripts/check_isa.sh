@@ -14,7 +14,7 @@ S=${TMPDIR:-/tmp}/nvllm_check.s
 cd "$(dirname "$0")/.."
 asm() { /opt/rocm/bin/hipcc -O3 -std=c++17 --offload-arch=gfx950 -mllvm -amdgpu-kernarg-preload-count=6 -Xclang -target-feature -Xclang -packed-fp32-ops -Wno-unused-function -Wno-unused-variable --cuda-device-only -S "$@" 2>/dev/null; }
 (asm nano-vllm-go_amd/csrc/nvllm.hip -o $S) & pids=$!
-for i in 1 2 3 4 5 6 7 8 9 10; do (asm -DNVL_GEMM_INST=$i nano-vllm-go_amd/csrc/gemm_inst.hip -o $S.gemm$i) & pids="$pids $!"; done
+for i in $(seq 1 17); do (asm -DNVL_GEMM_INST=$i nano-vllm-go_amd/csrc/gemm_inst.hip -o $S.gemm$i) & pids="$pids $!"; done
 for p in $pids; do wait $p; done
 rc=0
 for hd in 64 128; do for form in 2ELi8 1ELi8 1ELi4; do      # sub-tiles per wave, waves
@@ -52,8 +52,11 @@ def check(pattern, what, ok):
 check(r"attn_decode_bf16_kernelILi64ELi[248]ELb[01]ELb[01]ELb0E", "decode attention hd 64, 2 waves/SIMD", lambda r: r["vgpr"] <= 256 and r["spill"] == 0)
 check(r"attn_decode_bf16_kernelILi128ELi8ELb[01]ELb[01]ELb0E", "decode attention hd 128, 8 waves", lambda r: r["vgpr"] <= 256 and r["spill"] <= 8)
 # decode projections: the 64-row-group instantiations (PASSES) and the wide form
-check(r"gemm_skinny_bf16_kernelILi4ELi[124]ELi2ELi[0-4]E\w+Lb1ELi0ELb0E", "narrow projection, 64-row groups", lambda r: r["spill"] <= 12)
-check(r"gemm_skinny_bf16_kernelILi[12]ELi[124]ELi4ELi[0-4]E\w+Lb0ELi0ELb[01]E", "narrow projection, <= 32 rows", lambda r: r["spill"] <= 12)
+check(r"gemm_skinny_bf16_kernelILi4ELi[124]ELi2ELi(?:[0-4]|16)E\w+Lb1ELi0ELb0E", "narrow projection, 64-row groups", lambda r: r["spill"] <= 12)
+check(r"gemm_skinny_bf16_kernelILi[12]ELi[124]ELi4ELi(?:[0-4]|16)E\w+Lb0ELi0ELb[01]E", "narrow projection, <= 32 rows", lambda r: r["spill"] <= 12)
+check(r"gemm_skinny_bf16_kernelILi[124]ELi[124]ELi[24]ELi1[2-5]E", "narrow projection, carried layer norm", lambda r: r["spill"] <= 12)
+check(r"gemm_skinny_bf16_kernelILi[124]ELi[124]ELi[24]ELi[26]E\w+Lb0ELi2E", "experts' up projection, routing beside", lambda r: r["spill"] <= 12)
+check(r"gemm_bf16_kernelILi128ELi128ELi2ELi2ELi4ELi\d+E\w+Li32E", "128x128 tiles, ring of K tiles", lambda r: r["vgpr"] <= 256 and r["spill"] == 0)
 check(r"gemm_skinny_wide_bf16_kernelILi[12]ELi[24]ELi4E", "wide projection, <= 32 rows", lambda r: r["spill"] <= 12)
 sys.exit(1 if bad else 0)
 PY
