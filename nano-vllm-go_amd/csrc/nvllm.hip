@@ -1687,7 +1687,7 @@ void resid_gemm(nvl_model* m, const void* A, int lda, const void* W, const float
         else while (slices < m->sk_max_slices && nblocks * slices < 256 && (K >> 5) / (slices * 2) >= 8) slices *= 2;
     }
     // More rows than the ring kernel completes (256 for K >= 2048; 64 for shorter K) and up to 2048: N / 128 x M / 128 tiles of the
-    // lock-step kernel are a handful of workgroups (FFN-down of Llama-1B at 512 rows: 64), and the 64-row groups of the decode
+    // 128 x 128 kernel are a handful of workgroups (FFN-down of Llama-1B at 512 rows: 64), and the 64-row groups of the decode
     // form pull every activation row through every CU (1.3 GB of ingest for that projection: 85 us).  K split over
     // gridDim.y workgroups per tile instead, the slices summed by the norm that follows (a row or a tile of eight a workgroup).
     const bool norm_ok = (M <= 512 && m->H <= 1024 * NORM_ROW_MAXCH) || (m->H % 32 == 0 && m->H <= 2048 && g_norm_t16);   // launch_norm
@@ -1887,8 +1887,9 @@ bool moe(nvl_model* m, const LayerW& l, int M, bool deferred_norm = false, const
         }
     }
     // Decode: the dense-masked form (gemm.h GemmArgs::moe_gate).  Routing weights as a dense [M][E] matrix, then all experts
-    // as ONE weight-streaming projection each way; untouched experts are skipped inside the kernels, the gate weight in the up
-    // epilogue turns the down projection's K reduction into the weighted combine, its K slices are summed by the next norm.
+    // as ONE weight-streaming projection each way; experts that no token chose are skipped inside the kernels (by the up projection unless it routes beside:
+    // moe_hall then holds what they would make of the rows).  moe_hall is not weighted: the down projection's waves, an expert each, multiply their sums by
+    // the gate, or drop them where it is zero, which turns its K reduction into the weighted combine; its K slices are summed by the next norm.
     if (deferred_norm && !dense)
         throw std::runtime_error("moe: a deferred FFN norm needs the dense-masked decode form");
     if (dense) {

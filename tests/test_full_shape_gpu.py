@@ -108,7 +108,7 @@ def test_bench_sized_prefill_pingpong(gpu, key, layers, B):
         hm.seq_reset(i)
     big, am_big = hm.forward_batch(list(range(B)), prompts, [0] * B)
     assert hm.stats()["prefill_tokens"] == B * S
-    # (b) solo run of one sequence: lock-step tile kernels
+    # (b) solo run of one sequence: 128 x 128 tiles
     hm.seq_reset(0)
     solo, _ = hm.forward_batch([0], [prompts[3]], [0])
     assert rel_err(big[3], solo[0]) <= 1e-2          # GEMM forms are bit-identical; the two norm kernels reduce in

@@ -268,7 +268,7 @@ def test_moe(gpu, oracle, precision, rows, E, k):
 def test_moe_prefill_pingpong_tiles(gpu, oracle):
     """Prefill MoE on shapes the grouped ping-pong GEMM takes (H % 256 == 0, 2I % 256 == 0, rows in expert order):
     256-row m-tiles that start on arbitrary rows of the expert-ordered buffer and end ragged.  Same k order as the
-    lock-step 128-row tiles, so the two are bit-identical; against the oracle on the rows with a clear top-k."""
+    128-row tiles, so the two are bit-identical; against the oracle on the rows with a clear top-k."""
     r = rng(77)
     rows, E, k, H, I = 900, 8, 2, 256, 256
     x = r.standard_normal((rows, H), dtype=np.float32)

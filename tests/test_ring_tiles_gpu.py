@@ -22,10 +22,11 @@ def test_products_are_exact(gpu, m, n, k):
     assert np.array_equal(got, (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32))
 
 
-@pytest.mark.parametrize("rows", [70, 200, 513, 900])
-def test_slices_of_odd_numbers_of_tiles(gpu, rows):
-    """A prompt whose residual projections run in slices that the norm behind them sums: 66 K tiles in 2 .. 4 slices of 16 and 17, against the fp32 mode."""
-    cfg = gpu.synth.tiny_config("llama", hidden=2048, num_heads=8, num_kv_heads=8, head_dim=64, ffn_dim=2112, num_layers=2, max_seq_len=1024)
+# 2048 columns: two slices of 33 K tiles of FFN-down's 66, up to 200 rows the LDS-ring kernel instead; 512: four of 17, 17, 16 and 16
+@pytest.mark.parametrize("hidden,rows", [(2048, 70), (2048, 200), (2048, 513), (2048, 900), (512, 513), (512, 900)])
+def test_slices_of_odd_numbers_of_tiles(gpu, hidden, rows):
+    """A prompt whose residual projections run in slices that the norm behind them sums, against the fp32 mode."""
+    cfg = gpu.synth.tiny_config("llama", hidden=hidden, num_heads=8, num_kv_heads=8, head_dim=64, ffn_dim=2112, num_layers=2, max_seq_len=1024)
     w = gpu.synth.make_weights(cfg, seed=4, scale=0.03)
     tokens = np.random.default_rng(rows).integers(0, cfg["vocab_size"], rows).tolist()
     got = []
