@@ -1174,7 +1174,7 @@ __device__ __forceinline__ bf16x8 weight_load(const bf16x8* p) {
 // p: A (fragment-major operand, possibly the deferred-norm raw form with rs_in), M, K.  smem: MOE_ROUTE_LDS
 // ------------------------------------------------------------------------------------------
 struct RouteIds { int32_t* ids; float* w; };      // [row][top_k], or NULL
-// ALONE: sixteen waves, a slice of a tile and a row each: without the loops a launch of its own takes 5.5 us instead of 6.4 (1 row of 1024, 32 experts; code
+// ALONE: sixteen waves, a slice of a tile and a row each: without the loops a launch of its own takes 5.7 us instead of 6.4 (1 row of 1024, 32 experts; code
 // that is fetched cold)
 template <int U, int T, bool ALONE = false>
 __device__ __forceinline__ void moe_route_rows(const GemmArgs& p, const RouteJob& r, RouteIds out, int tile16, int first, int n, int waves, char* smem) {
