@@ -97,7 +97,7 @@ struct RouteJob {
 
 struct JointEpi { float* rows; int ld, n; };      // EPI_JOINT; n a multiple of 16
 
-// what a residual projection adds to a row's mean.  w: the mean of W's rows, in bf16 and the rest of it in bf16, [K/32][those two][32]; b: the mean of the bias
+// what a residual projection adds to a row's mean.  w: the mean of W's rows, in bf16 and the rest of it in bf16, [K/32][those two][32] and three K steps that nothing uses; b: the mean of the bias
 struct MeanShift { const bf16_t* w; float b; };
 struct LnResidEpi { MeanShift added; const float *prev, *mean_in; float* mean_out; };      // EPI_LN_RESID (GemmArgs::ln_s)
 
@@ -183,9 +183,9 @@ struct GemmArgs {
     // that mean but for rounding: the mean before (ln.prev: the pairs of the norm before, or NULL, where it was a launch of its own, and ln.mean_in) and what
     // the projection adds to it, its operand times ln.added (one more product a K step; a mean that is 100 deviations away: d < 0.01).  Consumer: bias is B.
     // A norm launch is 3.3 us (1 row) to 4.2 (16) and a boundary; the sums cost the four projections of a layer 0.5 to 1.7 us each, finding s
-    // the two residual ones 0.6 (GPT-2, a step of 1 sequence: with the mean before in its place 357 us, 371 so).  GPT-2, norm launches -> carried, us a step of 1 / 16 / 24 / 40 / 64 sequences:
-    // 388 -> 371, 448 -> 430, 495 -> 468, 518 -> 498, 575 -> 565; prompts of 11 / 3 x 11 / 64 tokens 470 -> 445, 544 -> 520, 550 -> 536.
-    // Error of the logits against 64 bits over 240 calls: mean log ratio to the norm launches -0.001 +- 0.002.
+    // the two residual ones 0.2 (GPT-2, a step of 1 sequence: with the mean before in its place 357 us, 361 so).  GPT-2, norm launches -> carried, us a step of
+    // 1 / 16 / 24 / 40 / 64 sequences: 387 -> 361, 444 -> 427, 494 -> 463, 517 -> 490, 584 -> 562; prompts of 11 / 3 x 11 / 64 tokens 498 -> 461, 583 -> 537, 574 -> 550.
+    // Error of the logits against 64 bits over 240 calls: mean log ratio to the norm launches -0.002 +- 0.002.
 };
 // blockDim lies 12 bytes behind the arguments.  The decode kernels load it with rs_in: a cache line more is 0.2 us of a 3.4 us launch (8 rows of 2048 x 1024)
 static_assert(((sizeof(GemmArgs) + 12) >> 6) == (offsetof(GemmArgs, rs_in) >> 6), "arguments that are loaded together");
@@ -1489,13 +1489,17 @@ __global__ __launch_bounds__(skinny_waves(EPIV, MOE == 2 && MT > 1) * 64) void g
     // flight while the current block's MFMAs issue (the compiler emits counted vmcnt for these).
     const int nblk = my_steps / U;
     bf16x8 wA[U], xA[U][MT], wB[U], xB[U][MT];
-    // carried layer norm: the mean row as rows 0, 2, .. and its rest as rows 1, 3, .. of a weight tile, so that every lane gets its row's sum of both
+    // carried layer norm: the mean row of U steps, and the rest of it, as rows 0, 2, .. and 1, 3, .. of one weight tile.  Step u's product is right in its two
+    // rows of an accumulator of its own, and the others are not looked at (a load a step instead, GPT-2, us a step of 1 / 40 sequences: 361 -> 373, 492 -> 498)
     constexpr bool LN_SHIFT = LN && EPI == EPI_RESID;
-    constexpr int UC = LN_SHIFT ? U : 1;
-    bf16x8 cA[UC], cB[UC];
-    f32x4 mean_acc = f32x4{0.f, 0.f, 0.f, 0.f};
-    const bf16x8* cp = LN_SHIFT ? (const bf16x8*)p.ln.added.w + (int64_t)ks0 * 8 + (fr & 1) * 4 + fg : nullptr;
-    auto load_blk = [&](bf16x8 (&w)[U], bf16x8 (&x)[U][MT], bf16x8 (&c)[UC], int b) {
+    static_assert(!LN_SHIFT || (U == 4 && MT == 1), "rows of four steps");
+    f32x4 mean_acc[U];
+    if constexpr (LN_SHIFT)
+#pragma unroll
+        for (int u = 0; u < U; u++) mean_acc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const bf16x8* cp = LN_SHIFT ? (const bf16x8*)p.ln.added.w + (int64_t)ks0 * 8 + (fr & 7) * 4 + fg : nullptr;
+    bf16x8 cA, cB;
+    auto load_blk = [&](bf16x8 (&w)[U], bf16x8 (&x)[U][MT], bf16x8& c, int b) {
 #pragma unroll
         for (int u = 0; u < U; u++) {
             if constexpr (HALF) w[u] = w_live ? weight_load<PASSES>((const bf16x8*)(wp + (int64_t)(b * U + u) * 512)) : x_zero;
@@ -1505,16 +1509,16 @@ __global__ __launch_bounds__(skinny_waves(EPIV, MOE == 2 && MT > 1) * 64) void g
                 const bf16x8* src = (const bf16x8*)(xp[i] + (int64_t)(b * U + u) * 512);
                 if (p.x_mask) x[u][i] = x_live[i] ? *src : x_zero; else x[u][i] = *src;      // (uniform branch)
             }
-            if constexpr (LN_SHIFT) c[u] = cp[(b * U + u) * 8];
         }
+        if constexpr (LN_SHIFT) c = cp[b * U * 8];
     };
-    auto comp_blk = [&](bf16x8 (&w)[U], bf16x8 (&x)[U][MT], bf16x8 (&c)[UC]) {
+    auto comp_blk = [&](bf16x8 (&w)[U], bf16x8 (&x)[U][MT], bf16x8& c) {
 #pragma unroll
         for (int u = 0; u < U; u++) {
 #pragma unroll
             for (int i = 0; i < MT; i++)
                 acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u], x[u][i], acc[i], 0, 0, 0);
-            if constexpr (LN_SHIFT) mean_acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c[u], x[u][0], mean_acc, 0, 0, 0);
+            if constexpr (LN_SHIFT) mean_acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c, x[u][0], mean_acc[u], 0, 0, 0);
         }
     };
     if (nblk > 0) load_blk(wA, xA, cA, 0);
@@ -1554,14 +1558,26 @@ __global__ __launch_bounds__(skinny_waves(EPIV, MOE == 2 && MT > 1) * 64) void g
     }
     if (b < nblk) comp_blk(wA, xA, cA);
     }
-    for (int s = nblk * U; s < my_steps; s++) {      // ragged tail: fewer than U k-steps
-        const bf16x8 w = w_live ? weight_load<PASSES>((const bf16x8*)(wp + (int64_t)s * 512)) : x_zero;
-        if constexpr (LN_SHIFT) {
-            const bf16x8 c = cp[s * 8], x = x_live[0] ? *(const bf16x8*)(xp[0] + (int64_t)s * 512) : x_zero;
-            acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x, acc[0], 0, 0, 0);
-            mean_acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c, x, mean_acc, 0, 0, 0);
-            continue;
+    if constexpr (LN_SHIFT) {          // ragged tail: fewer than U k-steps
+        const int s0 = nblk * U, rest = __builtin_amdgcn_readfirstlane(my_steps - s0);      // (uniform: matrix products heed no lane mask)
+        if (rest > 0) {
+            cA = cp[s0 * 8];
+#pragma unroll
+            for (int u = 0; u < U - 1; u++)
+                if (u < rest) {
+                    wA[u] = w_live ? weight_load<PASSES>((const bf16x8*)(wp + (int64_t)(s0 + u) * 512)) : x_zero;
+                    xA[u][0] = x_live[0] ? *(const bf16x8*)(xp[0] + (int64_t)(s0 + u) * 512) : x_zero;
+                }
+#pragma unroll
+            for (int u = 0; u < U - 1; u++)
+                if (u < rest) {
+                    acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wA[u], xA[u][0], acc[0], 0, 0, 0);
+                    mean_acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cA, xA[u][0], mean_acc[u], 0, 0, 0);
+                }
         }
+    } else
+    for (int s = nblk * U; s < my_steps; s++) {
+        const bf16x8 w = w_live ? weight_load<PASSES>((const bf16x8*)(wp + (int64_t)s * 512)) : x_zero;
 #pragma unroll
         for (int i = 0; i < MT; i++)
             acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x_live[i] ? *(const bf16x8*)(xp[i] + (int64_t)s * 512) : x_zero, acc[i], 0, 0, 0);
@@ -1574,10 +1590,11 @@ __global__ __launch_bounds__(skinny_waves(EPIV, MOE == 2 && MT > 1) * 64) void g
             acc[i] = g != 0.f ? acc[i] * g : f32x4{0.f, 0.f, 0.f, 0.f};       // (0: not routed, whatever the expert made of the row)
         }
     if constexpr (LN_LATE) rn_pre = layer_norm_of(p, pairs.sum());
-    float* mean_red = (float*)(smem + ksplit * 1024);      // [16][8]
+    float* mean_red = (float*)(smem + ksplit * 1024);      // [16][8][2]
     if constexpr (LN_SHIFT) {
         ln_shift += pairs.sum()[0] * p.rs_inv_h;
-        if (fg == 0) mean_red[fr * 8 + kw] = mean_acc[0] + mean_acc[1];
+        const f32x4 even = fg ? mean_acc[2] : mean_acc[0], odd = fg ? mean_acc[3] : mean_acc[1];
+        if (fg < 2) mean_red[(fr * 8 + kw) * 2 + fg] = (even[0] + even[1]) + (odd[2] + odd[3]);
     }
     // ---- reduce the K slices in wave order ----
 #pragma unroll
@@ -1586,11 +1603,15 @@ __global__ __launch_bounds__(skinny_waves(EPIV, MOE == 2 && MT > 1) * 64) void g
     __syncthreads();
     stamps.mark(4);                     // every wave's stream done
     if constexpr (LN_SHIFT) {
-        static_assert(skinny_waves(EPIV) == 8, "two reads a row");
-        const f32x4 lo = *(const f32x4*)(mean_red + fr * 8), hi = *(const f32x4*)(mean_red + fr * 8 + 4);
-        float added = lo[0];
+        static_assert(skinny_waves(EPIV) == 8, "four reads a row");
+        const f32x4* sums = (const f32x4*)(mean_red + fr * 16);
+        float added = 0.f;
 #pragma unroll
-        for (int w = 1; w < 8; w++) added += w < ksplit ? (w < 4 ? lo[w] : hi[w - 4]) : 0.f;
+        for (int w = 0; w < 8; w += 2) {
+            const f32x4 v = sums[w >> 1];
+            added += w < ksplit ? v[0] + v[1] : 0.f;
+            added += w + 1 < ksplit ? v[2] + v[3] : 0.f;
+        }
         ln_shift += p.alpha * (added + p.ln.added.b);
         if (blockIdx.x == 0 && wave == 0 && fg == 0 && 16 * i_off + fr < p.M) p.ln.mean_out[16 * i_off + fr] = ln_shift;
     }
@@ -2105,7 +2126,7 @@ static inline bool launch_gemm_ln_resid(hipStream_t st, const GemmArgs& a0) {
     int ks = skinny_waves(EPI_LN_RESID);
     while (ks > 1 && (a.K >> 5) / ks < 4) ks >>= 1;
     const int tiles = cdiv(a.N, 16);
-    const size_t lds = (size_t)ks * 1024 + 512;      // (the waves' sums of a tile, and of 16 rows' means)
+    const size_t lds = (size_t)ks * 1024 + 1024;      // (the waves' sums of a tile, and of 16 rows' means)
     if (a.rs_half) hipLaunchKernelGGL((gemm_skinny_bf16_kernel<1, 1, 4, EPI_LN_RESID, OutT, false, 0, true>), dim3(2 * tiles, 1), dim3(ks * 64), lds, st, a);
     else hipLaunchKernelGGL((gemm_skinny_bf16_kernel<1, 1, 4, EPI_LN_RESID, OutT>), dim3(tiles, cdiv(a.M, 16)), dim3(ks * 64), lds, st, a);
     return true;

@@ -776,7 +776,7 @@ void init_deferred_layer_norms(nvl_model* m) {
         return out;
     };
     auto mean_row = [&](const DevTensor& W, int K) {
-        void* out = dmalloc_bytes((int64_t)K * 4);
+        void* out = dmalloc_bytes((int64_t)K * 4 + 3 * 128);
         hipLaunchKernelGGL(ln_mean_row_kernel, dim3(K / 32), dim3(64), 0, m->stream, (const bf16_t*)W.p, (bf16_t*)out, H, K);
         NVL_HIP(hipGetLastError());
         return out;
