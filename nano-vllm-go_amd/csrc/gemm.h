@@ -1181,7 +1181,8 @@ __device__ __forceinline__ void moe_route_rows(const GemmArgs& p, const RouteJob
     f32x4* red = (f32x4*)smem;                                   // [K slices][expert tiles][64]
     const int E = r.E, ET = (E + 15) >> 4, KW = 16 / ET;         // expert tiles (1 .. 4), K slices
     float* lg = (float*)(smem + 16 * 1024);                      // [16][64]
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // (uniform, and known to be: matrix products heed no lane mask, and a step that a wave does not have is to be jumped over)
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int fr = lane & 15, fg = lane >> 4;
     const int row0 = tile16 * 16;
     const int nks = p.K >> 5, q = nks / KW, rr = nks - q * KW;
