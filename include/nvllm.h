@@ -578,7 +578,7 @@ int nvl_bench_gemm(int device, int M, int N, int K, int epi, int force_bnt, int 
  * key 30: Mamba2 prefill scan: 1 (default) the chunked SSD form on MFMA, chunks of a sequence in parallel when few (sequence, head)
  * pairs; 2 the chunked form, chunk after chunk only; 0 the sequential recurrence.
  * key 31: MoE decode routing (router logits, softmax, top-k, gate matrix): 1 (default) as one launch, or by the first workgroups of the
- * experts' up projection where streaming every expert costs less than that launch; 2 always as one launch; 0 router GEMM + gate kernel.
+ * experts' up projection where streaming every expert costs little beside that launch; 2 always as one launch; 0 router GEMM + gate kernel.
  * key 35: non-temporal K/V loads in the decode attention: 1 (default) when one workgroup serves a kv head's group and the launch
  * fills the chip (>= 160 workgroups) or the batch is one sequence; 0 never; 2 always.
  * key 36: weight tiles per wave of the wide decode projections (FFN-up, LM head): 0 (default) 2 for 17..32 rows and N < 65536, else 4;

@@ -1318,13 +1318,13 @@ __device__ __forceinline__ void moe_route_part(const GemmArgs& p, int id, int wa
     moe_route_rows<U, T>(p, p.route, RouteIds{nullptr, nullptr}, t, (id - t * per_tile) * p.route.rows, p.route.rows, waves, smem);
 }
 // Does a decode batch route inside the experts' up launch?  The launch that this saves is some 8 us (16 rows of 1024 and 32 experts; 2048 and 6 rows: 7.4
-// and the gap); not knowing the chosen experts, the up projection streams them all, at 6 TB/s.  So what a token leaves out may cost no more than the launch,
-// and a batch is expected to leave out less, were its choices even.  Larger experts would pay where the rows choose apart and lose where they choose alike
-// (answers to one prompt): us a layer of 32 rows, launch -> beside, 32 experts, 8 a token: 512 x 1024 apart 55.1 -> 53.5, alike 44.2 -> 47.8; not 512 x 2048 80.9 -> 77.7,
-// 59.8 -> 67.5; 1024 x 4096 223.9 -> 217.2, 132 -> 181
+// and the gap); not knowing the chosen experts, the up projection streams them all, at 6 TB/s.  Either all that a token leaves out costs little more than
+// that, or a batch is expected to leave out next to nothing, were its choices even; but rows that choose alike (answers to one prompt) leave out what
+// one does, and may not lose more than others gain.  Us a layer of 32 rows, launch -> beside, 32 experts, 8 a token: 512 x 1024 apart 55.1 -> 53.5, alike
+// 44.2 -> 47.8; 512 x 2048 80.9 -> 77.7, 59.8 -> 67.5; not 1024 x 4096 223.9 -> 217.2, 132 -> 181
 static inline bool moe_streams_all(int M, int E, int k, double expert_bytes) {
     const double out_us = E > k ? (E - k) * expert_bytes / 6e6 : 0.0, expected_us = E > k ? pow(1.0 - (double)k / E, M) * E * expert_bytes / 6e6 : 0.0;
-    return out_us < 9.0 && expected_us < 6.0;
+    return (out_us < 17.0 && expected_us < 1.5) || (out_us < 9.0 && expected_us < 6.0);
 }
 constexpr size_t MOE_ROUTE_LDS = 20 * 1024;
 // ... set up for a launch with workgroups of `waves` waves
