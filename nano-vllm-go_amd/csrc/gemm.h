@@ -1109,6 +1109,20 @@ __global__ __launch_bounds__(512, 1) void gemm_mid_bf16_kernel(GemmArgs p) {
 #pragma unroll
         for (int e = 0; e < H; e++) mine[e] = acc[e] + red[(wave * H + e) * 64];
     }
+    // residual: the rows' old values and the next norm's weights come under the hand-over (every part fetches them, one uses them)
+    f32x4 old[EPI == EPI_RESID ? H : 1], nrm[EPI == EPI_RESID ? H : 1];
+    const bool whole = EPI == EPI_RESID && (p.N & 3) == 0;
+    if constexpr (EPI == EPI_RESID) {
+        if (whole) {
+#pragma unroll
+            for (int e = 0; e < H; e++) {
+                const int idx = (BOTH ? kh * H : 0) + e, i = idx / CT, j = idx - i * CT;
+                const int m = min(m0 + (wm * TM + i) * 16 + fr, p.M - 1), nn = min(n0 + (wn + 2 * j) * 16 + 4 * fg, p.N - 4);
+                old[e] = *(const f32x4*)((const float*)p.C + (int64_t)m * p.ldc + nn);
+                if (p.rs_out) nrm[e] = *(const f32x4*)(p.nrm_w + nn);
+            }
+        }
+    }
     if (p.splits > 1 && !split_finish<H>(p, cb * groups + item / p.splits, part, p.splits, (BOTH ? 8 : 4) * H * 1024, BOTH ? wave8 : wave, mine, (int*)(smem + NST * SB), BOTH || kh == 0)) return;
     if (!BOTH && kh == 1) return;
 
@@ -1129,14 +1143,20 @@ __global__ __launch_bounds__(512, 1) void gemm_mid_bf16_kernel(GemmArgs p) {
             if (m < p.M && nn < p.N) {
                 if (p.bias) v += *(const f32x4*)(p.bias + nn);
                 float* x = (float*)p.C + (int64_t)m * p.ldc + nn;
-                const f32x4 o = *(f32x4*)x + p.alpha * v;
+                const f32x4 o = old[EPI == EPI_RESID ? e : 0] + p.alpha * v;
                 *(f32x4*)x = o;
-                act_store4<bf16_t>(p.nrm_xn, m, nn, p.N, o * *(const f32x4*)(p.nrm_w + nn));
+                act_store4<bf16_t>(p.nrm_xn, m, nn, p.N, o * nrm[EPI == EPI_RESID ? e : 0]);
                 ss = o[0] * o[0] + o[1] * o[1] + o[2] * o[2] + o[3] * o[3];
             }
             ss += __shfl_xor(ss, 16, 64);
             ss += __shfl_xor(ss, 32, 64);
             if (fg == 0 && m < p.M && nn < p.N) p.rs_out[(int64_t)m * (p.N >> 4) + (nn >> 4)] = ss;
+        } else if (EPI == EPI_RESID && whole) {
+            if (m < p.M && nn < p.N) {
+                f32x4 v = mine[e];
+                if (p.bias) v += *(const f32x4*)(p.bias + nn);
+                *(f32x4*)((float*)p.C + (int64_t)m * p.ldc + nn) = old[EPI == EPI_RESID ? e : 0] + p.alpha * v;
+            }
         } else epilogue4<EPI, OutT>(p, m, nn, mine[e], rs);
     }
 }
