@@ -473,11 +473,14 @@ __device__ __forceinline__ void attn_decode_merge(const AttnArgs& p, int pair, i
 // at B = 1, against 0.4 us in the projection kernels).
 // SPLIT: its own instance — the arguments and the branch that deal a sequence over workgroups cost an unsplit launch 0.6 us (GPT-2, 104 rows)
 template <int HD, int NW, bool FUSED, bool SPLIT, bool STAMP = false>
-__global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t* __restrict__ a_seq_pos, const int32_t* __restrict__ a_blk_table,
+__global__ __launch_bounds__(NW * 64, HD == 128 ? 2 : 1) void attn_decode_bf16_kernel(const int32_t* __restrict__ a_seq_pos, const int32_t* __restrict__ a_blk_table,
                                                                    int a_tbl_stride, int a_bs_shift, int a_Tmax, int a_group, AttnArgs p) {
     constexpr int KS = HD / 32, DT = HD / 16, HALF = HD / 2, CPR = HD / 8, KPI = 64 / CPR, NVL = 64 / KPI;
     constexpr int NT2 = HD <= 64 ? 2 : 1;                    // key tiles whose loads are in flight together, per wave
     constexpr int TILE_BYTES = 64 * HD * 2;
+    // The next round's loads leave as registers come free (do_round).  Heads of 128, steps: Llama-3-8B 96 of 500 keys -2.7 %, 8 of 1500 -1.7, 32 of 900 -0.6 (also for
+    // the registers, which then fit two waves a SIMD); heads of 64 96 of 1500 keys +4.2, 40 of 1900 +0.2, 32 of 512 0.0, GPT-2 32 of 900 -1.6: not there
+    constexpr bool PIPED = HD == 128;
     extern __shared__ __attribute__((aligned(16))) char smem[];     // [NW] wave-private V images (later: the partial O^T)
     __shared__ float red_m[NW][16];
     __shared__ float red_l[NW][16];
@@ -485,8 +488,9 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t
     // 71 heads = 5 tiles that stream the same K/V — it is tiny next to the weights — from L2)
     const int swg = ((SPLIT ? blockIdx.z * gridDim.y : 0) + blockIdx.y) * gridDim.x + blockIdx.x;
     NvlStampsT<STAMP> stamps(p.stamps, swg);          // (diagnostic instantiation only: see common.h)
-    const int QT = (a_group + 15) >> 4;
-    const int seq = blockIdx.y, kvh = blockIdx.x / QT, qt = blockIdx.x - kvh * QT;
+    // (ordered: the sequences from the longest context down, in the places before a_seq_pos[0])
+    const int ordered = a_group >> 16, QT = ((a_group & 0xffff) + 15) >> 4;
+    const int seq = ordered ? a_seq_pos[(int)blockIdx.y - ordered] : blockIdx.y, kvh = blockIdx.x / QT, qt = blockIdx.x - kvh * QT;
     const int32_t* tbl = a_blk_table + (int64_t)seq * a_tbl_stride;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -532,40 +536,44 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t
 
     bf16x8 kf[NT2][4][KS];
     bf16x8 vch[NT2][NVL];
-    // the K / V loads of one round (NT2 tiles of this wave): addresses depend on scalars only
+    // the K / V loads of a tile: addresses depend on scalars only
     // NT: non-temporal loads (AttnArgs::kv_nt, chosen by the host) — a (sequence, kv head)'s K/V are read ONCE per step when
     // one workgroup serves the whole group (GQA / MHA), and lines that stay out of L2 leave it to the projections'
     // activations: decode +5 % at B = 32 (32.0 K -> 33.7 K tok/s), GPT-2 B = 128 +3.2 %; it loses 2 % at 32-64 workgroups
     // (profiles/r03_kv_nontemporal.txt).  Falcon's MQA (5 workgroups share one K/V stream through L2) keeps the default policy.
-    auto issue_round_t = [&](int kt0, auto nt_tag) {
-        constexpr bool NT = decltype(nt_tag)::value;
+    auto tile_offset = [&](int kt, int blk) {
+        const int bi = kv_block_index(p, kt * 64), krow0 = kt * 64 - bi * p.Tmax;     // the KV block holding this tile
+        return (int64_t)blk * p.slot_stride + ((int64_t)kvh * p.Tmax + krow0) * HD;
+    };
+    auto issue_k_t = [&](int h, int64_t off, auto nt_tag) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int ks = 0; ks < KS; ks++) {
+                const bf16x8* src = (const bf16x8*)((const bf16_t*)p.kcache + off + (int64_t)(t * 16 + fq) * HD + ks * 32 + fg * 8);
+                if constexpr (decltype(nt_tag)::value) kf[h][t][ks] = __builtin_nontemporal_load(src); else kf[h][t][ks] = *src;
+            }
+    };
+    auto issue_v_t = [&](int h, int64_t off, auto nt_tag) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NVL; i++) {                                                                 // 1 KiB, contiguous
+            const bf16x8* src = (const bf16x8*)((const bf16_t*)p.vcache + off + (int64_t)lane * 8 + i * 512);
+            if constexpr (decltype(nt_tag)::value) vch[h][i] = __builtin_nontemporal_load(src); else vch[h][i] = *src;
+        }
+    };
+    auto issue_k = [&](int h, int64_t off) __attribute__((always_inline)) { if (p.kv_nt) issue_k_t(h, off, std::true_type{}); else issue_k_t(h, off, std::false_type{}); };
+    auto issue_v = [&](int h, int64_t off) __attribute__((always_inline)) { if (p.kv_nt) issue_v_t(h, off, std::true_type{}); else issue_v_t(h, off, std::false_type{}); };
+    auto issue_round_t = [&](int kt0, auto nt_tag) __attribute__((always_inline)) {
 #pragma unroll
         for (int h = 0; h < NT2; h++) {
             const int kt = kt0 + h * NW;
             if (kt >= n_kt) continue;
-            const int bi = kv_block_index(p, kt * 64), krow0 = kt * 64 - bi * p.Tmax;     // the KV block holding this tile
-            const int blk = kt0 == vw ? first_blk[h] : tbl[bi];
-            const int64_t blk_off = (int64_t)blk * p.slot_stride + ((int64_t)kvh * p.Tmax + krow0) * HD;
-            const bf16_t* kbase = (const bf16_t*)p.kcache + blk_off;
-            const bf16_t* vbase = (const bf16_t*)p.vcache + blk_off;
-#pragma unroll
-            for (int t = 0; t < 4; t++)
-#pragma unroll
-                for (int ks = 0; ks < KS; ks++)
-                {
-                    const bf16x8* src = (const bf16x8*)(kbase + (int64_t)(t * 16 + fq) * HD + ks * 32 + fg * 8);
-                    if constexpr (NT) kf[h][t][ks] = __builtin_nontemporal_load(src); else kf[h][t][ks] = *src;
-                }
-#pragma unroll
-            for (int i = 0; i < NVL; i++) {                                                                 // 1 KiB, contiguous
-                const bf16x8* src = (const bf16x8*)(vbase + (int64_t)lane * 8 + i * 512);
-                if constexpr (NT) vch[h][i] = __builtin_nontemporal_load(src); else vch[h][i] = *src;
-            }
+            const int64_t off = tile_offset(kt, kt0 == vw ? first_blk[h] : tbl[kv_block_index(p, kt * 64)]);
+            issue_k_t(h, off, nt_tag);
+            issue_v_t(h, off, nt_tag);
         }
     };
-    auto issue_round = [&](int kt0) {
-        if (p.kv_nt) issue_round_t(kt0, std::true_type{}); else issue_round_t(kt0, std::false_type{});
-    };
+    auto issue_round = [&](int kt0) __attribute__((always_inline)) { if (p.kv_nt) issue_round_t(kt0, std::true_type{}); else issue_round_t(kt0, std::false_type{}); };
     // Load order (vector loads return in issue order): the new token's fp32 q/k/v row + cos/sin FIRST (a dozen small loads),
     // the round's K/V stream right behind them with no wait in between, THEN the RoPE arithmetic — it waits for the row only
     // (counted vmcnt) and runs, like the first QK^T MFMAs after it, while the K/V tiles are still arriving.  An earlier form waited
@@ -623,24 +631,35 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t
         for (int e = 0; e < 4; e++) { vnew8[e] = (bf16_t)v0[e]; vnew8[4 + e] = (bf16_t)v1[e]; }
     }
     stamps.mark(2);                     // q/k/v of the new token rotated
-    // one round: scores, online softmax, O^T += V^T P^T of the tiles whose K/V fragments issue_round left in kf / vch.
+    // one round: scores, online softmax, O^T += V^T P^T of the tiles whose K/V fragments the loads left in kf / vch.
     // (The first round is peeled — its loads went out above, ahead of the RoPE arithmetic — instead of making the issue
     // conditional inside ONE loop: there every fragment register became a loop-carried value with a select per iteration,
-    // 213 -> 252 registers on the 2- and 4-wave hd-64 kernels (MHA models: one wave per SIMD instead of two) and 25
-    // spilled on the 8-wave hd-128 kernel.)
-    auto do_round = [&](int kt0) __attribute__((always_inline)) {
+    // 213 -> 252 registers on the 2- and 4-wave hd-64 kernels (MHA models: one wave per SIMD instead of two).)
+    // MORE: a round follows, and its K loads leave when the scores are there, a tile's V loads when its rows are in LDS: into the registers
+    // that have just been read, so that the stream goes on under the softmax and P·V.  Its own copy of the round, for the same reason.
+    auto do_round = [&](int kt0, auto more_tag) __attribute__((always_inline)) {
+        constexpr bool MORE = decltype(more_tag)::value;
+        const int kt1 = kt0 + stride;
+        int64_t off1[NT2];
+        if constexpr (MORE) {
+#pragma unroll
+            for (int h = 0; h < NT2; h++) {
+                const int kt = min(kt1 + h * NW, n_kt - 1);
+                off1[h] = tile_offset(kt, tbl[kv_block_index(p, kt * 64)]);
+            }
+        }
         // ---- scores of the round's tiles ----
         f32x4 s[NT2][4];
         float tmax = -INFINITY;
 #pragma unroll
         for (int h = 0; h < NT2; h++) {
             const int kt = kt0 + h * NW;
-            if (kt >= n_kt) {
+            if (!MORE && kt >= n_kt) {
 #pragma unroll
                 for (int t = 0; t < 4; t++) s[h][t] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
                 continue;
             }
-            if (FUSED && kt == n_kt - 1) {
+            if (FUSED && !MORE && kt == n_kt - 1) {
                 // the tile that holds key pos0: its slab row is not written yet (or not visible): patch the operands
                 const int kl = pos0 & 63;
 #pragma unroll
@@ -662,12 +681,13 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     float v = acc[r] * sl2;
-                    v = (t * 16 + r <= lim) ? v : -INFINITY;
+                    if (!MORE) v = (t * 16 + r <= lim) ? v : -INFINITY;
                     acc[r] = v;
                     tmax = fmaxf(tmax, v);
                 }
                 s[h][t] = acc;
             }
+            if constexpr (MORE) if (kt1 + h * NW < n_kt) issue_k(h, off1[h]);
         }
         tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
         tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
@@ -692,9 +712,10 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t
         // MFMA operand (ds_read_b64_tr_b16); a wave's LDS accesses execute in order, so no barrier ----
 #pragma unroll
         for (int h = 0; h < NT2; h++) {
-            if (kt0 + h * NW >= n_kt) continue;
+            if (!MORE && kt0 + h * NW >= n_kt) continue;
 #pragma unroll
             for (int i = 0; i < NVL; i++) *(bf16x8*)(vimg + w_base[i & 1] + i * (16 * KPI * CPR)) = vch[h][i];
+            if constexpr (MORE) if (kt1 + h * NW < n_kt) issue_v(h, off1[h]);
 #pragma unroll
             for (int u = 0; u < 2; u++) {
                 bf16x8 pf;
@@ -712,10 +733,18 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_bf16_kernel(const int32_t
             }
         }
     };
-    if (vw < n_kt) do_round(vw);
-    for (int kt0 = vw + stride; kt0 < n_kt; kt0 += stride) {
-        issue_round(kt0);
-        do_round(kt0);
+    if constexpr (PIPED) {
+        if (vw < n_kt) {
+            int kt0 = vw;
+            for (; kt0 + stride < n_kt; kt0 += stride) do_round(kt0, std::true_type{});
+            do_round(kt0, std::false_type{});
+        }
+    } else {
+        if (vw < n_kt) do_round(vw, std::false_type{});
+        for (int kt0 = vw + stride; kt0 < n_kt; kt0 += stride) {
+            issue_round(kt0);
+            do_round(kt0, std::false_type{});
+        }
     }
     if (FUSED && z == 0 && qt == 0) {
         // append the new key/value to the slabs for the following steps — after every load of this step (which used

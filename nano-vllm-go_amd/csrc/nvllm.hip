@@ -731,7 +731,7 @@ void init_slots(nvl_model* m) {
 // per-call metadata: see bind_meta
 void init_meta(nvl_model* m) {
     const int64_t Mmax = m->opts.max_batch_tokens, S = m->opts.max_seqs;
-    m->meta_ints = 5 * Mmax + (5 + (int64_t)m->masks.size()) * S + m->table_cap + 2 * (m->layered ? Mmax : 0) + 16;
+    m->meta_ints = 5 * Mmax + (6 + (int64_t)m->masks.size()) * S + m->table_cap + 2 * (m->layered ? Mmax : 0) + 16;
     NVL_HIP(hipHostMalloc((void**)&m->meta_host, (size_t)m->meta_ints * 4, hipHostMallocDefault));
     m->meta_dev = dmalloc<int32_t>(m->meta_ints);
     NVL_HIP(hipHostMalloc((void**)&m->am_host, (size_t)std::max<int64_t>(S, Mmax) * 4, hipHostMallocDefault));
@@ -1277,20 +1277,21 @@ struct Meta {   // device pointers into meta_dev
     int32_t *tokens, *tok_pos, *tok_tbl, *tok_seq, *seq_tok_start, *seq_len, *seq_pos, *seq_tbl, *seq_slot, *last_rows, *blk_table, *kbase, *abs_tok, *abs_seq;
 };
 // layout of meta_host / meta_dev for a call carrying M tokens:
-//   [seq_tok_start S | seq_len S | seq_pos S | seq_tbl S | seq_slot S | kbase masks x S | blk_table table_cap |
+//   [seq_tok_start S | seq_len S | order S | seq_pos S | seq_tbl S | seq_slot S | kbase masks x S | blk_table table_cap |
 //    tokens M | tok_pos M | tok_tbl M | tok_seq M | last_rows M (the rows whose logits are wanted) | (layered) abs_tok M | abs_seq M]
+// (order: where a decode pass of ragged contexts takes its sequences from the longest down, in the last n_seqs places, before seq_pos; decode_order)
 // (blk_table: sequence i's blocks start at i * blocks_per_seq; slab mode: one entry, its slot)
 Meta bind_meta(const nvl_model* m, int32_t* base, int M) {
     const int64_t S = m->opts.max_seqs;
     Meta md;
-    md.seq_tok_start = base; md.seq_len = base + S; md.seq_pos = base + 2 * S; md.seq_tbl = base + 3 * S; md.seq_slot = base + 4 * S;
-    md.kbase = base + 5 * S; md.blk_table = md.kbase + (int64_t)m->masks.size() * S;
+    md.seq_tok_start = base; md.seq_len = base + S; md.seq_pos = base + 3 * S; md.seq_tbl = base + 4 * S; md.seq_slot = base + 5 * S;
+    md.kbase = base + 6 * S; md.blk_table = md.kbase + (int64_t)m->masks.size() * S;
     md.tokens = md.blk_table + m->table_cap; md.tok_pos = md.tokens + M; md.tok_tbl = md.tok_pos + M; md.tok_seq = md.tok_tbl + M;
     md.last_rows = md.tok_seq + M; md.abs_tok = md.last_rows + M; md.abs_seq = md.abs_tok + M;
     return md;
 }
 size_t meta_bytes(const nvl_model* m, int M) {
-    return (size_t)((5 + (int64_t)m->masks.size()) * (int64_t)m->opts.max_seqs + m->table_cap + (m->layered ? 7 : 5) * (int64_t)M) * 4;
+    return (size_t)((6 + (int64_t)m->masks.size()) * (int64_t)m->opts.max_seqs + m->table_cap + (m->layered ? 7 : 5) * (int64_t)M) * 4;
 }
 // sequence i of the batch being assembled lives in `slot`: its table row, table start and slot
 void bind_slot(const nvl_model* m, const Meta& hm, int i, int slot) {
@@ -1357,6 +1358,7 @@ static int g_use_graphs = 1;   // nvl_set_tuning key 21: hipGraph replay of deco
 static int g_tune_epoch = 0;   // bumped by every nvl_set_tuning: captured graphs bake the tuning in (part of their key)
 static int g_attn_nw = 0;      // nvl_set_tuning key 15: waves per decode-attention workgroup (0 = from the context length, 2, 4, 8)
 static int g_attn_rows = 1;    // nvl_set_tuning key 10: query rows per workgroup of the prefill attention (0: 256, 1: from their number, 2: 128, 3: 64)
+static int g_attn_order = 1;   // nvl_set_tuning key 43: decode attention takes ragged contexts from the longest down (0 never, 1 automatic, 2 always)
 static int g_attn_kv_nt = 1;   // nvl_set_tuning key 35: non-temporal K/V loads in the decode attention (0 never, 1 automatic, 2 always)
 static int g_attn_split = 1;   // nvl_set_tuning key 25: split a decode attention's keys over up to 8 workgroups per (sequence, kv head) (0 never, 1 automatic, 1 + n: n rounds each)
 // Launch shape of the decode attention for the batch being enqueued (also part of a captured graph's key): waves per
@@ -1385,8 +1387,26 @@ static int g_attn_split = 1;   // nvl_set_tuning key 25: split a decode attentio
 //                  14 of 1200 and short ones 0.0 -> -1.3; of 900 / 2  at 227 with work +0.4, so not
 //   heads of 128   12 of 1500 / 6 -3.6 -> -5.7 (4 x 3), 16 of 1100 / 6 -1.0 -> -2.1 (4 x 3), 12 of 1500 and short ones -5 -> -7.6 (4 x 6); 16 of 1500 and
 //                  short ones -6.4 (4 x 3), -1.9 (4 x 6: a grid of 768); 12 of 900 / 6 in four parts (238 with work) +0.4, 16 of 1500 / 6 in three (251) +0.9
+// Whole sequences of ragged contexts: workgroups start in the grid's order, and a long one that starts in the second round of them runs on alone.
+// The longest start first (the kernel looks its sequence up: 0.3 % of a step where contexts are alike), and with them in front four waves a
+// workgroup pay where two did before, as the short ones fill up behind.  Steps against the batch's order, per cent (2 waves, 4 waves):
+//   heads of 64   Llama-3.2-1B 48 of 1500 / 25 -3.3 (8 waves)  64 of 1500 / 25 -0.1, -4.4  64 of 700 / 8 +0.5, -2.9  96 of 1500 / 25 -2.9, -4.6
+//                 96 of 1500 / 2 -2.0, +0.9  96 of 400 / 7 -1.0, +1.1  128 of 1900 / 12 -0.8, -3.5  128 of 700 / 12 -2.3, -1.4  128 of 300 / 8 -1.0, +0.7
+//                 GPT-2 24 of 900 / 15 -6.2 (8)  32 -9.8 (8)  64 -7.5, -10.7  96 -6.8, -6.0  128 of 500 / 10 -6.0, -0.5; 64 of 500 alike -0.1, +1.5
+//                 Granite-3.0-1B 64 of 1500 / 15 -0.5, -4.8  128 of 600 / 10 -0.2, +1.0; Falcon-7B 64 of 1500 / 15 -2.1 (4); Llama-3.2-1B 32 of 1500 / 25 (8) +0.3
+//   heads of 128  Llama-3-8B 48 of 1500 / 25 -4.3 (4)  96 of 1000 / 16 -2.9, -4.2  128 of 400 / 7 -2.3, -1.3; 32 of 1500 / 15 -0.1 (8)
+constexpr int ATTN_ORDERED = 1 << 30;
+bool decode_may_order(const nvl_model* m, int n_seqs) { return !m->f32 && !m->layered && n_seqs < 1 << 15 && m->nKV * cdiv(m->group, 16) * n_seqs > 256; }
+// (meta_host of a decode pass)
+void decode_order(const nvl_model* m, const Meta& hm, int n_seqs) {
+    if (!decode_may_order(m, n_seqs)) return;
+    int32_t* order = hm.seq_pos - n_seqs;
+    for (int i = 0; i < n_seqs; i++) order[i] = i;
+    std::sort(order, order + n_seqs, [&](int a, int b) { return hm.seq_pos[a] != hm.seq_pos[b] ? hm.seq_pos[a] > hm.seq_pos[b] : a < b; });
+}
 int decode_attn_cfg(const nvl_model* m, int n_seqs) {
     const int n_kt = m->ctx_hint > 0 ? (m->ctx_hint - 1) / 64 + 1 : 1 << 20;
+    const double mean_kt = m->kv_tok / (64.0 * n_seqs);
     const int per_wave = m->hd == 64 ? 2 : 1;
     const int wgs = m->nKV * cdiv(m->group, 16) * n_seqs;
     const int cap = wgs >= 512 ? 2 : (wgs >= 320 ? 4 : 8);
@@ -1396,7 +1416,6 @@ int decode_attn_cfg(const nvl_model* m, int n_seqs) {
     const int most = m->attn_part && m->ctx_hint > 0 ? std::min(ATTN_SPLIT_MAX, m->attn_records / wgs) : 1;
     if (g_attn_split >= 2) { const int tiles = (g_attn_split - 1) * nw * per_wave; return cfg(nw, std::max(1, std::min(most, cdiv(n_kt, tiles))), tiles); }
     if (g_attn_split && !g_attn_nw && most > 1) {
-        const double mean_kt = m->kv_tok / (64.0 * n_seqs);
         // the workgroups with work: a sequence has its tiles / `tiles` parts, rounded up
         auto room = [&](int tiles) { return (mean_kt / tiles + 0.5) * wgs <= 208; };
         int waves = 0;
@@ -1409,7 +1428,9 @@ int decode_attn_cfg(const nvl_model* m, int n_seqs) {
             if (each < rounds) return cfg(waves, cdiv(rounds, each), each * round);
         }
     }
-    return cfg(nw, 1, 1 << 16);
+    const bool ordered = g_attn_order && m->ctx_hint > 0 && decode_may_order(m, n_seqs) && (g_attn_order == 2 || n_kt >= 1.3 * mean_kt + 1);
+    if (ordered && !g_attn_nw && wgs >= 512 && wgs <= 1024 && n_kt >= 11 && n_kt >= 1.8 * mean_kt) nw = 4;
+    return cfg(nw, 1, 1 << 16) | (ordered ? ATTN_ORDERED : 0);
 }
 int layered_decode_key(const nvl_model* m);
 int decode_attn_waves(const nvl_model* m, int n_seqs) { return m->layered ? layered_decode_key(m) : decode_attn_cfg(m, n_seqs); }   // (graph keys: the whole shape)
@@ -1442,7 +1463,8 @@ void attention(nvl_model* m, int li, const Meta& md, int n_seqs, int M, int max_
         hipLaunchKernelGGL(attn_f32_kernel, dim3(max_len, m->nH, n_seqs), dim3(256), lds, m->stream, a, m->hd);
     } else if (max_len == 1) {
         const int cfg = decode_attn_cfg(m, n_seqs), nsplit = cfg >> 8 & 15;
-        a.split_max = nsplit; a.split_tiles = cfg >> 12;
+        a.split_max = nsplit; a.split_tiles = (cfg & ~ATTN_ORDERED) >> 12;
+        const int lead_group = a.group | (cfg & ATTN_ORDERED ? n_seqs << 16 : 0);
         dim3 grid(m->nKV * cdiv(m->group, 16), n_seqs, nsplit);      // (kv head x 16-head query tile, sequence, key split)
         a.part = m->attn_part; a.part_cnt = m->attn_part_cnt;
         // waves per workgroup: each wave takes NT2 key tiles per round trip (2 for hd 64, 1 for hd 128).  Short contexts
@@ -1458,7 +1480,7 @@ void attention(nvl_model* m, int li, const Meta& md, int n_seqs, int M, int max_
         if (fused_qkv) {   // RoPE + KV append + attention in one launch, straight from the QKV projection's fp32 output
             a.qkv = m->qkv; a.qkv_stride = m->n_qkv; a.cos_t = m->rope_cos; a.sin_t = m->rope_sin;
         }
-#define NVL_DEC_LEAD a.seq_pos, a.blk_table, a.tbl_stride, a.bs_shift, a.Tmax, a.group      /* the preloaded leading arguments (attn.h) */
+#define NVL_DEC_LEAD a.seq_pos, a.blk_table, a.tbl_stride, a.bs_shift, a.Tmax, lead_group      /* the preloaded leading arguments (attn.h) */
 #define NVL_DECN(HDv, NWv, FUSEDv, SPLITv, STv)                                                                         \
         do {                                                                                                           \
             NVL_LDS_ATTR((attn_decode_bf16_kernel<HDv, NWv, FUSEDv, SPLITv, STv>), NWv * 64 * HDv * 2);                \
@@ -2393,6 +2415,7 @@ int forward_impl(nvl_model* m, int n_seqs, const int64_t* seq_ids, const int32_t
         for (int i = 0; i < n_seqs; i++) bind_slot(m, hm, i, h_slot[(size_t)i]);
     }
     if (m->layered) layered_meta(m, hm, n_seqs, 1);
+    if (!prefill) decode_order(m, hm, n_seqs);
     bool custom = false;
     if (n_rows >= 0) {
         if ((flags & NVL_FWD_ALL_LOGITS) || n_rows > M || (n_rows > 0 && !row_list)) return fail(m, NVL_ERR_INVALID, "nvl_forward_rows: bad row list");
@@ -2521,6 +2544,7 @@ extern "C" int nvl_forward_paged(nvl_model* m, int n_seqs, const int32_t* tokens
         }
         hm.last_rows[i] = t - 1;
     }
+    if (!prefill) decode_order(m, hm, n_seqs);
     const Meta md = bind_meta(m, m->meta_dev, M);
     NVL_HIP(hipEventRecord(m->ev0, m->stream));
     NVL_HIP(hipMemcpyAsync(m->meta_dev, m->meta_host, meta_bytes(m, M), hipMemcpyHostToDevice, m->stream));
@@ -2641,6 +2665,7 @@ void decode_loop(nvl_model* m, const Meta& hm, int n_seqs, int n_steps, int32_t*
         m->ring_ints = (int64_t)n_steps * n_seqs;
         m->ring = dmalloc<int32_t>(m->ring_ints);
     }
+    decode_order(m, hm, n_seqs);
     NVL_HIP(hipEventRecord(m->ev0, m->stream));
     NVL_HIP(hipMemcpyAsync(m->meta_dev, m->meta_host, meta_bytes(m, M), hipMemcpyHostToDevice, m->stream));
     NVL_HIP(hipMemcpyAsync(m->ring_pos0, h_pos, (size_t)n_seqs * 4, hipMemcpyHostToDevice, m->stream));   // (pinned meta_host)
