@@ -314,7 +314,9 @@ __device__ __forceinline__ void norm_row_finish(f32x4 (&v)[NORM_ROW_MAXCH], f32x
     }
 }
 
-template <typename ActT>
+// EXPERTS: the residual add to complete are experts' rows.  us in moe_combine_kernel and here -> in one launch, 900 rows of 1024, 8 experts a row: 7.0 + 5.3 -> 9.2
+// (tiles of eight rows, a row a wave, keep too few loads on their way: 1800 rows 12.2 + 5.6 -> 32, so that above NORM_ROW_KERNEL_ROWS the two stay apart)
+template <typename ActT, bool EXPERTS = false>
 __global__ __launch_bounds__(256) void norm_row_kernel(float* __restrict__ x,
                                                        const int32_t* __restrict__ rows_idx,
                                                        const float* __restrict__ w,
@@ -332,11 +334,17 @@ __global__ __launch_bounds__(256) void norm_row_kernel(float* __restrict__ x,
         v[c] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (j < H4) {
             v[c] = *(const f32x4*)(xr + j * 4);
-            if (pr.part && pr.slot_of) {
+            if constexpr (EXPERTS) {
                 f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
-                for (int k = 0; k < pr.slices; k++)          // same order and arithmetic as moe_combine_kernel
-                    s += pr.gate_w[(int64_t)src * pr.slices + k] *
-                         *(const f32x4*)(pr.part + (int64_t)pr.slot_of[(int64_t)src * pr.slices + k] * H + j * 4);
+                const int32_t* slots = pr.slot_of + (int64_t)src * pr.slices;
+                const float* gw = pr.gate_w + (int64_t)src * pr.slices;
+                for (int k0 = 0; k0 < pr.slices; k0 += 8) {          // same order and arithmetic as moe_combine_kernel
+                    f32x4 e[8];
+#pragma unroll
+                    for (int k = 0; k < 8; k++) if (k0 + k < pr.slices) e[k] = *(const f32x4*)(pr.part + (int64_t)slots[k0 + k] * H + j * 4);
+#pragma unroll
+                    for (int k = 0; k < 8; k++) if (k0 + k < pr.slices) s += gw[k0 + k] * e[k];
+                }
                 v[c] = v[c] + (pr.alpha != 0.f ? pr.alpha * s : s);
                 *(f32x4*)(xr + j * 4) = v[c];
             } else if (pr.part) {
@@ -1295,16 +1303,18 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const float* __restric
     }
 }
 
-// Counting sort of the (token, rank) pairs by expert, three small launches:
-//   moe_hist_kernel    per-expert pair counts (atomics on E counters; zeroed by the host per call)
-//   moe_scan_kernel    one wave: segment starts, the per-expert placement cursors, and the m-tile table of
-//                      the grouped GEMM launch: tile_map[i] = {expert, row0, nrows, 0}, *n_mtiles
-//   moe_scatter_kernel each pair takes the next row of its expert's segment (atomic cursor).  The row a pair
+// Counting sort of the (token, rank) pairs by expert:
+//   moe_hist_kernel    per-expert pair counts (atomics on E counters, zero between layers); not where moe_place_kernel counts alone
+//   moe_place_kernel   segment starts and the m-tile table of the grouped GEMM launch, tile_map[i] = {expert, row0, nrows, 0} and *n_mtiles, from the counts
+//                      (every workgroup adds them up for itself); each pair takes the next row of its expert's segment.  The row a pair
 //                      lands on can differ from run to run, the VALUES cannot: every pair is computed
-//                      independently and moe_combine_kernel reads them back through slot_of in rank order.
+//                      independently and the combine reads them back through slot_of in rank order.
+// (Clearing the counts and the scan were launches of their own, four of 4.9 us instead of two; Granite-3.0-1B, prompts of 100 .. 900 tokens with the combine
+// under the next norm: -2.8 .. -4.1 %, decode steps of 96 sequences -5 %.  Counting alone: 100 tokens
+// -2.8 %, 400 -0.5, 96 sequences -1.6)
 // prefill-sized batches: per-workgroup counts in LDS first (E <= MOE_MAX_E), so the global counters see one atomic per
 // (workgroup, expert) instead of one per pair (32768 pairs on 32 addresses: 57 -> ~10 us)
-constexpr int MOE_PAIRS_PER_WG = 1024, MOE_MAX_E = 256;
+constexpr int MOE_PAIRS_PER_WG = 1024, MOE_MAX_E = 256, MOE_ALONE_PAIRS = 4096;
 __global__ __launch_bounds__(256) void moe_hist_kernel(const int32_t* __restrict__ expert_ids, int n_pairs, int32_t* __restrict__ counts) {
     __shared__ int lc[MOE_MAX_E];
     lc[threadIdx.x] = 0;
@@ -1340,63 +1350,75 @@ __global__ __launch_bounds__(256) void moe_gather_fm_kernel(const bf16_t* __rest
         *(bf16x8*)(d + (int64_t)(ks + 1) * 512) = y;
     }
 }
-__global__ __launch_bounds__(64) void moe_scan_kernel(const int32_t* __restrict__ counts, int E, int BM,
-                                                      int32_t* __restrict__ seg_start, int32_t* __restrict__ cursor,
-                                                      int32_t* __restrict__ tile_map, int32_t* __restrict__ n_mtiles) {
-    // exclusive scans over the experts, 64 at a time (one lane each): first row and first m-tile of every segment
-    const int lane = threadIdx.x;
-    int rows = 0, tiles = 0;                         // of the experts before this batch of 64
-    for (int e0 = 0; e0 < E; e0 += 64) {
-        const int e = e0 + lane, c = e < E ? counts[e] : 0;
-        const int nt_e = (c + BM - 1) / BM;
-        int row = c, tile = nt_e;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int yr = __shfl_up(row, o, 64), yt = __shfl_up(tile, o, 64);
-            if (lane >= o) { row += yr; tile += yt; }
-        }
-        const int row0 = rows + row - c, tile0 = tiles + tile - nt_e;
-        if (e < E) {
-            seg_start[e] = row0;
-            cursor[e] = row0;
-            for (int t = 0; t < nt_e; t++) {
-                const int r = t * BM;
-                tile_map[4 * (tile0 + t)] = e; tile_map[4 * (tile0 + t) + 1] = row0 + r;
-                tile_map[4 * (tile0 + t) + 2] = (c - r < BM) ? (c - r) : BM; tile_map[4 * (tile0 + t) + 3] = 0;
-            }
-        }
-        rows += __shfl(row, 63, 64); tiles += __shfl(tile, 63, 64);
-    }
-    if (lane == 0) { seg_start[E] = rows; *n_mtiles = tiles; }
-}
-__global__ __launch_bounds__(256) void moe_scatter_kernel(const int32_t* __restrict__ expert_ids, int n_pairs, int top_k,
-                                   int32_t* __restrict__ cursor, int32_t* __restrict__ perm_token,
-                                   int32_t* __restrict__ slot_of) {
+// ALONE: every workgroup counts all pairs for itself, and those before its own: no counters, no launch in front (up to MOE_ALONE_PAIRS)
+template <bool ALONE>
+__global__ __launch_bounds__(256) void moe_place_kernel(const int32_t* __restrict__ expert_ids, int n_pairs, int top_k, int E, int BM, int32_t* __restrict__ counts, int32_t* __restrict__ cursor,
+                                   int32_t* __restrict__ seg_start, int32_t* __restrict__ tile_map, int32_t* __restrict__ n_mtiles, int32_t* __restrict__ perm_token, int32_t* __restrict__ slot_of) {
     // rank inside the workgroup from LDS atomics, one global reservation per (workgroup, expert).  The row order inside
     // an expert's segment varies from run to run; no output depends on it (rows are independent, the combine sums a
     // token's slots in rank order through slot_of).
-    __shared__ int lc[MOE_MAX_E], base[MOE_MAX_E];
-    lc[threadIdx.x] = 0;
+    __shared__ int lc[MOE_MAX_E], base[MOE_MAX_E], all[ALONE ? MOE_MAX_E : 1], rows_of[4], tiles_of[4], last;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    lc[tid] = 0;
+    if constexpr (ALONE) {
+        all[tid] = 0; base[tid] = 0;
+        __syncthreads();
+        for (int i = tid; i < n_pairs; i += 256) {
+            const int x = expert_ids[i];
+            atomicAdd(&all[x], 1);
+            if (i < (int)blockIdx.x * MOE_PAIRS_PER_WG) atomicAdd(&base[x], 1);
+        }
+        __syncthreads();
+    }
+    const int c = ALONE ? all[tid] : tid < E ? counts[tid] : 0, nt = (c + BM - 1) / BM;      // a thread per expert
+    int row = c, tile = nt;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int yr = __shfl_up(row, o, 64), yt = __shfl_up(tile, o, 64);
+        if (lane >= o) { row += yr; tile += yt; }
+    }
+    if (lane == 63) { rows_of[wave] = row; tiles_of[wave] = tile; }
     __syncthreads();
     int e[MOE_PAIRS_PER_WG / 256], r[MOE_PAIRS_PER_WG / 256];
 #pragma unroll
     for (int j = 0; j < MOE_PAIRS_PER_WG / 256; j++) {
-        const int i = blockIdx.x * MOE_PAIRS_PER_WG + j * 256 + threadIdx.x;
+        const int i = blockIdx.x * MOE_PAIRS_PER_WG + j * 256 + tid;
         e[j] = 0; r[j] = 0;
         if (i < n_pairs) { e[j] = expert_ids[i]; r[j] = atomicAdd(&lc[e[j]], 1); }
     }
+    row -= c; tile -= nt;                                                   // the expert's first row and first m-tile
+    for (int w = 0; w < wave; w++) { row += rows_of[w]; tile += tiles_of[w]; }
+    if (tid < E) {
+        for (int t = blockIdx.x; t < nt; t += gridDim.x) {
+            const int r0 = t * BM, at = 4 * (tile + t);
+            tile_map[at] = tid; tile_map[at + 1] = row + r0; tile_map[at + 2] = c - r0 < BM ? c - r0 : BM; tile_map[at + 3] = 0;
+        }
+        if (blockIdx.x == 0) seg_start[tid] = row;
+        if (blockIdx.x == 0 && tid == E - 1) { seg_start[E] = row + c; *n_mtiles = tile + nt; }
+    }
     __syncthreads();
-    if (lc[threadIdx.x]) base[threadIdx.x] = atomicAdd(&cursor[threadIdx.x], lc[threadIdx.x]);
+    if constexpr (ALONE) base[tid] += row;
+    else base[tid] = row + (lc[tid] ? atomicAdd(&cursor[tid], lc[tid]) : 0);
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < MOE_PAIRS_PER_WG / 256; j++) {
-        const int i = blockIdx.x * MOE_PAIRS_PER_WG + j * 256 + threadIdx.x;
+        const int i = blockIdx.x * MOE_PAIRS_PER_WG + j * 256 + tid;
         if (i < n_pairs) {
             const int pos = base[e[j]] + r[j];
             perm_token[pos] = i / top_k;
             slot_of[i] = pos;
         }
     }
+    if constexpr (ALONE) return;
+    // counts, cursors and the tickets (counts[E]) are zero again for the next layer: by the workgroup that ends last, when all have read them
+    if (tid == 0) last = atomicAdd(&counts[E], 1) == (int)gridDim.x - 1;
+    __syncthreads();
+    if (!last) return;
+    if (tid < E) {
+        __hip_atomic_store(counts + tid, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(cursor + tid, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (tid == 0) __hip_atomic_store(counts + E, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ---------------------------------------------------------------------------------------

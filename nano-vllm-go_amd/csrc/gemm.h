@@ -788,7 +788,10 @@ __device__ __forceinline__ bool split_finish(const GemmArgs& p, int tile, int pa
 // stage s+1 is waited for at the end of L(s) by every wave, one barrier before the early group reads it (RAW).
 // ------------------------------------------------------------------------------------------
 // SPLIT: its own instance, the unsplit loop loses 3 % beside the code of the sum
-template <int EPI, typename OutT, int STAGES = 4, int PRIO = 0, int WAVES_N = 4, int BN = 256, bool SPLIT = false>
+// ROWS: a grouped launch whose A is row-major, a segment's rows wherever a_rows says.  Against a copy in expert order, us of copy and product ->
+// product, 32 experts of 1024 x 512, 8 a row: 900 rows 7 + 30.5 -> 35.5, 3600 18 + 77 -> 85, 6867 32.6 + 118 -> 122, 14400 67 + 215 -> 229 (a line is fetched in two
+// k-steps, and the first stage waits for the rows' places).  From a fragment-major operand every 16 bytes would be a line of their own: those are copied.
+template <int EPI, typename OutT, int STAGES = 4, int PRIO = 0, int WAVES_N = 4, int BN = 256, bool SPLIT = false, bool ROWS = false>
 __global__ __launch_bounds__(512, 1) void gemm_bf16_pp_kernel(GemmArgs p) {
     // BN 256: WAVES_N = 4 -> wave tile 128x64 (a head of 64 per wave), WAVES_N = 2 -> 64x128 (a head of 128 per wave);
     // BN 128 (mid-size M: twice the tiles): WAVES_N = 2 -> wave tile 64x64
@@ -850,17 +853,20 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_pp_kernel(GemmArgs p) {
             int am = m0 + blk * 16 + fr;
             if (am > p.M - 1) am = p.M - 1;
             am += row_base;                               // (a segment may start on any row: per-lane 16-byte sources)
-            src[i] = (const bf16_t*)p.A + (((int64_t)(am >> 4) * (p.K >> 5) * 64) + (am & 15) + 16 * fg) * 8;
+            if constexpr (ROWS) src[i] = (const bf16_t*)p.A + (int64_t)p.a_rows[am] * p.K + 8 * fg;
+            else src[i] = (const bf16_t*)p.A + (((int64_t)(am >> 4) * (p.K >> 5) * 64) + (am & 15) + 16 * fg) * 8;
         } else {
             src[i] = (const bf16_t*)p.W + ((int64_t)((n0 >> 4) + blk - NA) * (p.K >> 5) * 64 + lane) * 8;
         }
         src[i] += (int64_t)k0 * 512;
     }
+    static_assert(!ROWS || (!SPLIT && NA % PW == 0), "a wave's blocks are all rows or all columns");
+    const int step = ROWS && wave * PW < NA ? 32 : 512;      // a k-step further
     auto stage = [&](int buf, int ks) {
         char* base = smem + buf * STAGE_BYTES + wave * (PW * 1024);
 #pragma unroll
         for (int i = 0; i < PW; i++)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] + (int64_t)ks * 512),
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] + (ROWS ? (int64_t)(ks * step) : (int64_t)ks * 512)),
                                              (__attribute__((address_space(3))) void*)(base + i * 1024), 16, 0, 0);
     };
     const int a_off = wm * TM * 1024 + lane * 16;
@@ -2232,6 +2238,12 @@ static inline void launch_pp(hipStream_t st, const GemmArgs& a) {
 template <int EPI, typename OutT>
 static inline void launch_gemm_grouped(hipStream_t st, const GemmArgs& a, int max_mtiles) {
     if (a.grp_bm == 512) {      // prefill MoE, the default: 256-row m-tiles on the ping-pong kernel
+        if constexpr (epi_glu(EPI))
+            if (a.a_rows) {
+                NVL_LDS_ATTR((gemm_bf16_pp_kernel<EPI, OutT, 4, 0, 4, 256, false, true>), PP_LDS);
+                hipLaunchKernelGGL((gemm_bf16_pp_kernel<EPI, OutT, 4, 0, 4, 256, false, true>), dim3(cdiv(a.N, 256) * max_mtiles), dim3(512), PP_LDS, st, a);
+                return;
+            }
         NVL_LDS_ATTR((gemm_bf16_pp_kernel<EPI, OutT, 4, 0>), PP_LDS);
         hipLaunchKernelGGL((gemm_bf16_pp_kernel<EPI, OutT, 4, 0>), dim3(cdiv(a.N, 256) * max_mtiles), dim3(512), PP_LDS, st, a);
         return;

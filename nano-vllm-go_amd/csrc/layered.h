@@ -754,7 +754,7 @@ void layered_finalize(nvl_model* m) {
     if (m->f32) m->h2 = dmalloc<float>(Mmax * std::max<int64_t>(2 * std::max<int64_t>(m->F, moe_kI), sd4));
     if (moe_k) {
         m->expert_ids = dmalloc<int32_t>(Mmax * moe_k); m->expert_w = dmalloc<float>(Mmax * moe_k);
-        m->seg_start = dmalloc<int32_t>(moe_e + 1); m->moe_counts = dmalloc<int32_t>(moe_e); m->moe_cursor = dmalloc<int32_t>(moe_e);
+        m->seg_start = dmalloc<int32_t>(moe_e + 1); moe_counters(m, moe_e);
         m->moe_tile_map = dmalloc<int32_t>(4 * (cdiv(Mmax * moe_k, 128) + moe_e)); m->moe_n_mtiles = dmalloc<int32_t>(4);
         m->perm_token = dmalloc<int32_t>(Mmax * moe_k); m->slot_of = dmalloc<int32_t>(Mmax * moe_k);
         m->moe_eo = dmalloc<float>(Mmax * moe_k * H);

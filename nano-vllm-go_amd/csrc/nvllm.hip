@@ -728,6 +728,12 @@ void init_slots(nvl_model* m) {
     m->free_blocks.clear();
     if (m->pool) for (int b = m->num_blocks - 1; b >= 0; b--) m->free_blocks.push_back(b);
 }
+// counts of moe_sort, and its cursors: zero between layers
+void moe_counters(nvl_model* m, int64_t E) {
+    m->moe_counts = dmalloc<int32_t>(E + 1); m->moe_cursor = dmalloc<int32_t>(E);
+    NVL_HIP(hipMemsetAsync(m->moe_counts, 0, (size_t)(E + 1) * 4, m->stream));
+    NVL_HIP(hipMemsetAsync(m->moe_cursor, 0, (size_t)E * 4, m->stream));
+}
 // per-call metadata: see bind_meta
 void init_meta(nvl_model* m) {
     const int64_t Mmax = m->opts.max_batch_tokens, S = m->opts.max_seqs;
@@ -988,8 +994,7 @@ extern "C" int nvl_finalize(nvl_model* m) {
         m->expert_ids = dmalloc<int32_t>(Mmax * k);
         m->expert_w = dmalloc<float>(Mmax * k);
         m->seg_start = dmalloc<int32_t>(c.num_experts + 1);
-        m->moe_counts = dmalloc<int32_t>(c.num_experts);
-        m->moe_cursor = dmalloc<int32_t>(c.num_experts);
+        moe_counters(m, c.num_experts);
         m->moe_tile_map = dmalloc<int32_t>(4 * (cdiv(Mmax * k, 128) + c.num_experts));
         m->moe_n_mtiles = dmalloc<int32_t>(4);
         m->perm_token = dmalloc<int32_t>(Mmax * k);
@@ -1321,14 +1326,15 @@ void launch_norm(nvl_model* m, float* x, const int32_t* rows_idx, const float* w
         pr.part = m->pending_part; pr.slices = m->pending_slices; pr.rows_total = m->pending_rows; pr.alpha = m->pending_alpha;
         pr.slot_of = m->pending_slot_of; pr.gate_w = m->pending_gate_w;
         m->pending_slices = 0; m->pending_slot_of = nullptr; m->pending_gate_w = nullptr;
-        const bool row_kernel = rows <= 512 && m->H <= 1024 * NORM_ROW_MAXCH;
+        const bool row_kernel = rows <= (pr.slot_of ? NORM_ROW_KERNEL_ROWS : 512) && m->H <= 1024 * NORM_ROW_MAXCH;
         const bool tile_kernel = sizeof(ActT) == 2 && m->H % 32 == 0 && m->H <= 2048 && g_norm_t16 && !pr.slot_of;   // (the 16-chunk instance would spill)
         if (!row_kernel && !tile_kernel) throw std::runtime_error("norm: no kernel for this pending residual");
     }
-    const bool tiles = sizeof(ActT) == 2 && m->H % 32 == 0 && m->H <= 4608 && g_norm_t16 && !pr.slot_of && (!pr.part || m->H <= 2048);
-    if (rows <= (tiles && !y_rows ? NORM_ROW_KERNEL_ROWS : 512) && m->H <= 1024 * NORM_ROW_MAXCH)
-        hipLaunchKernelGGL((norm_row_kernel<ActT>), dim3(rows), dim3(256), 0, m->stream, x, rows_idx, w, b,
-                           m->cfg.norm_eps, (ActT*)y, m->H, pr, mean_out);
+    const bool tiles = sizeof(ActT) == 2 && m->H % 32 == 0 && m->H <= 4608 && g_norm_t16 && (!pr.part || m->H <= 2048);
+    if (pr.slot_of || (rows <= (tiles && !y_rows ? NORM_ROW_KERNEL_ROWS : 512) && m->H <= 1024 * NORM_ROW_MAXCH)) {
+        if (pr.slot_of) hipLaunchKernelGGL((norm_row_kernel<ActT, true>), dim3(rows), dim3(256), 0, m->stream, x, rows_idx, w, b, m->cfg.norm_eps, (ActT*)y, m->H, pr, mean_out);
+        else hipLaunchKernelGGL((norm_row_kernel<ActT>), dim3(rows), dim3(256), 0, m->stream, x, rows_idx, w, b, m->cfg.norm_eps, (ActT*)y, m->H, pr, mean_out);
+    }
     else if (tiles) {   // (two workgroups' tiles of wider rows would not fit the LDS of a CU: norm_kernel)
         // 8 rows x H bf16 of LDS (up to 73 KiB); the row sits in registers: instance by chunks per lane
 #define NVL_NT(CH, PEND)                                                                                             \
@@ -1804,12 +1810,11 @@ bool moe_pp_ok(const nvl_model* m, int I, bool small, int64_t pairs, int E) {
 void moe_sort(nvl_model* m, int E, int k, int M, int BM) {
     const int pairs = M * k;
     KScope ks(m, KC_OTHER, 0, KS_MOE_PLAN);
-    hipLaunchKernelGGL(fill_i32_kernel, dim3(cdiv(E, 256)), dim3(256), 0, m->stream, m->moe_counts, 0, E);     // (a captured pass must hold no memset node)
-    hipLaunchKernelGGL(moe_hist_kernel, dim3(cdiv(pairs, MOE_PAIRS_PER_WG)), dim3(256), 0, m->stream, m->expert_ids, pairs, m->moe_counts);
-    hipLaunchKernelGGL(moe_scan_kernel, dim3(1), dim3(64), 0, m->stream, m->moe_counts, E, BM, m->seg_start, m->moe_cursor,
-                       m->moe_tile_map, m->moe_n_mtiles);
-    hipLaunchKernelGGL(moe_scatter_kernel, dim3(cdiv(pairs, MOE_PAIRS_PER_WG)), dim3(256), 0, m->stream, m->expert_ids, pairs, k,
-                       m->moe_cursor, m->perm_token, m->slot_of);
+    const dim3 grid(cdiv(pairs, MOE_PAIRS_PER_WG));
+    const bool alone = pairs <= MOE_ALONE_PAIRS;
+    if (!alone) hipLaunchKernelGGL(moe_hist_kernel, grid, dim3(256), 0, m->stream, m->expert_ids, pairs, m->moe_counts);
+    hipLaunchKernelGGL((alone ? moe_place_kernel<true> : moe_place_kernel<false>), grid, dim3(256), 0, m->stream, m->expert_ids, pairs, k, E, BM,
+                       m->moe_counts, m->moe_cursor, m->seg_start, m->moe_tile_map, m->moe_n_mtiles, m->perm_token, m->slot_of);
     NVL_HIP(hipGetLastError());
 }
 // the experts' feed-forwards over the sorted pairs: rows of m->xn -> m->moe_eo (pair order of m->slot_of)
@@ -1843,7 +1848,8 @@ void moe_expert_gemms(nvl_model* m, const MoeW& w, int M, int BM, bool pp, bool 
     }
     GemmArgs a = mk(m->xn, H, w.up, m->hbuf, I, nullptr, 1.f, max_mtiles, 2 * I, H);
     a.a_rows = m->perm_token; a.tile_map = m->moe_tile_map; a.n_mtiles = m->moe_n_mtiles;
-    if (!small && m->moe_xg && g_moe_gather) {
+    if (pp && xn_rows) a.A = xn_rows;      // (each row of a 256-row tile from its place: gemm.h)
+    else if (!small && m->moe_xg && g_moe_gather) {
         // prefill: every m-tile's rows would be re-gathered 16 bytes at a time by each of its 2I/128 column tiles
         // (64 cache lines per load instruction); copy them into expert order once, then the GEMM streams whole
         // 1-KiB operand blocks (Granite-1B, 16384 tokens: expert-up 1080 -> 390 us per layer)
@@ -1957,7 +1963,7 @@ bool moe(nvl_model* m, const LayerW& l, int M, bool deferred_norm = false, const
         moe_sort(m, E, k, M, BM);
     }
     moe_expert_gemms(m, MoeW{E, k, I, l.moe_in, l.t[NVL_T_MOE_OUT].p}, M, BM, pp, small, xn_rows);
-    if (small && !m->keep_hidden && m->pending_slices == 0 && H % 4 == 0 && H <= 1024 * NORM_ROW_MAXCH) {
+    if ((small || (!m->f32 && M <= NORM_ROW_KERNEL_ROWS && g_moe_small)) && !m->keep_hidden && m->pending_slices == 0 && H % 4 == 0 && H <= 1024 * NORM_ROW_MAXCH) {
         // x += rm * sum_k w[t][k] * eo[slot[t][k]] is completed by the next norm's read of x (PendingResid)
         m->pending_part = m->moe_eo; m->pending_slices = k; m->pending_rows = M; m->pending_alpha = c.residual_multiplier;
         m->pending_slot_of = m->slot_of; m->pending_gate_w = m->expert_w;

@@ -292,7 +292,9 @@ extern "C" int nvl_op_moe(int device, int precision, const float* x, const float
     m.router_logits = (float*)cx.alloc((int64_t)rows * 128 * 4);
     m.expert_ids = (int32_t*)cx.alloc(pairs * 4); m.expert_w = (float*)cx.alloc(pairs * 4);
     m.seg_start = (int32_t*)cx.alloc((n_experts + 1) * 4);
-    m.moe_counts = (int32_t*)cx.alloc(n_experts * 4); m.moe_cursor = (int32_t*)cx.alloc(n_experts * 4);
+    m.moe_counts = (int32_t*)cx.alloc((n_experts + 1) * 4); m.moe_cursor = (int32_t*)cx.alloc(n_experts * 4);
+    NVL_HIP(hipMemsetAsync(m.moe_counts, 0, (size_t)(n_experts + 1) * 4, m.stream));
+    NVL_HIP(hipMemsetAsync(m.moe_cursor, 0, (size_t)n_experts * 4, m.stream));
     m.moe_tile_map = (int32_t*)cx.alloc(16 * (cdiv(pairs, 128) + n_experts)); m.moe_n_mtiles = (int32_t*)cx.alloc(16);
     m.perm_token = (int32_t*)cx.alloc(pairs * 4); m.slot_of = (int32_t*)cx.alloc(pairs * 4);
     m.moe_eo = (float*)cx.alloc(pairs * hidden * 4);
