@@ -31,9 +31,9 @@ struct GroupedArgs {
     float scale, softcap;                         // softcap 0: none
     const float *r1, *r2;                         // [H] or NULL: no distance bias
     const float* sink;                            // [H] scores of the denominator's own entry, or NULL
-    float out_scale;
     const void* q; int64_t q_ld;                  // queries of head h at column h dp, its gate at column gate_col + h vp: bf16 (fragment-major) or the fp32 rows of proj
     int gate_col;                                 // < 0: no gate
+    float out_scale;                              // (beside gate_col: with padding behind it the compiler kept a copy of it and what follows in scratch memory)
     const float* proj; int64_t proj_ld;           // fp32 mode: [token][q : H dp | k : G dp | v : G vp | gate : H vp | ...] of the fused input projection
     int k_off, v_off;                             // k_off < 0: the keys are in the cache already
     // normed and / or rotated queries and keys (grouped_qk_*_kernel): fp32 columns [0, H dp) and [qk_koff, + G dp) of proj
@@ -54,6 +54,9 @@ struct GroupedArgs {
     float* part; int32_t* part_cnt;               // keys split over workgroups: partial results, arrival tickets (zero between launches)
     int row_wgs;                                  // grouped_short_kernel: workgroups of the rows of a sequence and key split
     GatedNormArgs gn; void* gn_out;               // ... QK: what one more workgroup per sequence does, the gated norm of its token's row (gn_out NULL: none)
+    // ... or one more per head of a second mixer (lin_heads > 0): its recurrence, and by the last of a sequence's to end the gated norm
+    int lin_heads; int32_t* lin_cnt;              // tickets, zero between launches
+    LinRecArgs lin;
 };
 
 // ---- fp32 mode: keys and values of the batch's tokens into the cache (bf16: gemm.h EPI_GROUPED): grid (32-token units of a sequence's new positions, sequences, G) ----
@@ -652,6 +655,7 @@ struct GroupedTurnRow {
 // QK (one token per sequence): queries and the new key come from the fp32 rows of proj, normed and rotated here, a head a wave, under the
 // first key tile's loads; the wave with the last key tile puts the new key in its operand and appends it to the cache.  Besides, the
 // launch may carry the gated norm of a second mixer's rows.  (As launches of their own those two took 6.4 and 6.3 us.)
+constexpr int GROUPED_LIN_ROWS = 8;      // state rows a thread of a carried recurrence keeps
 template <int KS, int DT, int NW, bool QK>
 __global__ __launch_bounds__(NW * 64) void grouped_short_kernel(GroupedArgs p) {
     extern __shared__ __attribute__((aligned(16))) char grp_sm[];       // [NW][DT][64] f32x4
@@ -660,8 +664,21 @@ __global__ __launch_bounds__(NW * 64) void grouped_short_kernel(GroupedArgs p) {
     constexpr int QLD = KS * 32 + 8;
     __shared__ __attribute__((aligned(16))) bf16_t qsm[QK ? 17 : 1][QLD];      // QK: the row tile's queries, the new key
     if constexpr (QK) {
-        if ((int)blockIdx.x == p.row_wgs) {
-            if (blockIdx.z == 0) gated_norm_row<NW * 64>(p.gn, p.seq_tok_start[blockIdx.y], (bf16_t*)p.gn_out, &red_m[0][0]);
+        if ((int)blockIdx.x >= p.row_wgs) {
+            if (blockIdx.z) return;
+            if constexpr (NW * 64 == LR_STEP_THREADS)
+                if (p.lin_heads) {
+                    linrec_step_head<0, GROUPED_LIN_ROWS, float, true>(p.lin, blockIdx.x - p.row_wgs, blockIdx.y, (float*)grp_sm, &red_m[0][0], &red_l[0][0]);
+                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // (as for the parts of split keys, below)
+                    __syncthreads();
+                    if (threadIdx.x == 0) ticket = __hip_atomic_fetch_add(p.lin_cnt + blockIdx.y, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __syncthreads();
+                    if (ticket != p.lin_heads - 1) return;
+                    if (threadIdx.x == 0) __hip_atomic_store(p.lin_cnt + blockIdx.y, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    gated_norm_row<NW * 64, true>(p.gn, p.seq_tok_start[blockIdx.y], (bf16_t*)p.gn_out, &red_m[0][0]);
+                    return;
+                }
+            gated_norm_row<NW * 64>(p.gn, p.seq_tok_start[blockIdx.y], (bf16_t*)p.gn_out, &red_m[0][0]);
             return;
         }
     }

@@ -38,7 +38,7 @@ static void run_short(hipStream_t st, const GroupedArgs& p, dim3 grid) {
     if constexpr (KS == 2 || KS == 4) {
         if (p.qk_koff >= 0) {
             NVL_LDS_ATTR((grouped_short_kernel<KS, DT, nw, true>), nw * DT * 1024);
-            hipLaunchKernelGGL((grouped_short_kernel<KS, DT, nw, true>), dim3(grid.x + (p.gn_out ? 1 : 0), grid.y, grid.z), dim3(nw * 64), nw * DT * 1024, st, p);
+            hipLaunchKernelGGL((grouped_short_kernel<KS, DT, nw, true>), dim3(grid.x + (p.gn_out ? std::max(1, p.lin_heads) : 0), grid.y, grid.z), dim3(nw * 64), nw * DT * 1024, st, p);
             return;
         }
     }

@@ -773,6 +773,7 @@ void layered_finalize(nvl_model* m) {
         m->grp_cap = GROUPED_SPLIT_WGS;
         m->grp_part = (float*)lay_alloc(m, m->grp_cap * (grp_vp * 16 + 32) * 4);
         m->grp_cnt = (int32_t*)lay_alloc(m, m->grp_cap * 4);
+        m->lin_cnt = (int32_t*)lay_alloc(m, (int64_t)m->opts.max_seqs * 4);
     }
     m->lproj = f32buf(Mmax * ld_in);
     m->ly = f32buf(Mmax * H);
@@ -1280,15 +1281,26 @@ void tap_layer(nvl_model* m, int li, int M);
 
 // ---- lightning attention beside another mixer: columns of the joint input projection -> m->lmix columns [ko, ko + ko2) ----
 // carry: not NULL: the gated norm of its rows is left to another launch (gn, gn_out) where that can do it
+static int g_lin_rides = 1;          // nvl_set_tuning key 44: decode: a second mixer's recurrence in the attention launch (0 never, 1 automatic, 2 wherever it fits)
+// Does the attention launch of a decode pass (workgroups of 512 threads) take the recurrence too?  It runs beside the attention and its launch (6.9 us of
+// a step of 6 sequences, 16 heads of 128 x 128) is gone: a 2048-wide model, requests of 24 steps of 1 / 6 / 16 / 32 / 64 / 128 sequences -3.6, -2.8, -0.6, -0.5, -1.7, +0.1 %.
+bool lightning_rides(const LayerRun& r, const LinRecArgs& a, int n_seqs) {
+    int tv = 1;
+    while (tv < a.DVp / 4) tv <<= 1;
+    if (!g_lin_rides || (g_lin_rides == 1 && n_seqs > 64) || r.vp > 128 || r.dp > 128 || cdiv(a.DK, LR_STEP_THREADS / tv) > GROUPED_LIN_ROWS || linrec_step_lds_bytes(a.DK, a.DVp) > 8 * (r.vp >> 4) * 1024) return false;
+    return true;
+}
 void mix_lightning(nvl_model* m, const LayerRun& r, const MixerW& w, const Meta& md, int n_seqs, int M, int max_len, GroupedArgs* carry) {
     const nvl_layer_config& c = r.c;
     LinRecArgs a = linrec_args(m, r, md);
     a.H = c.heads2; a.DK = c.dim2; a.DV = c.vdim2; a.DVp = (int)round_up(c.vdim2, 4); a.kdiv = 1; a.q_scale = 1.f;
     a.q = m->lproj + r.lq_off; a.k = m->lproj + r.lk_off; a.v = m->lproj + r.lv_off; a.ld = m->lproj_ld;
     a.decay = w.decay; a.log2_decay = w.log2_decay;
-    linrec<false>(m, a, n_seqs, M, max_len, false, KS_LIN_SCAN);
     GatedNormArgs g{m->lo, m->lo_ld, m->lproj + r.lg_off, m->lproj_ld, w.lin_norm, M, 1, c.heads2 * c.vdim2, m->cfg.norm_eps, r.kd, 0, 1};
-    if (carry && gated_norm_v4(g) && ((uintptr_t)g.w & 15) == 0) { carry->gn = g; carry->gn_out = (bf16_t*)m->lmix + (int64_t)(r.ko >> 5) * 512; }
+    const bool rides = carry && gated_norm_v4(g) && ((uintptr_t)g.w & 15) == 0;
+    if (rides && lightning_rides(r, a, n_seqs)) { a.len_lo = 1; a.len_hi = 1 << 30; carry->lin = a; carry->lin_heads = a.H; carry->lin_cnt = m->lin_cnt; }
+    else linrec<false>(m, a, n_seqs, M, max_len, false, KS_LIN_SCAN);
+    if (rides) { carry->gn = g; carry->gn_out = (bf16_t*)m->lmix + (int64_t)(r.ko >> 5) * 512; }
     else gated_norm<false>(m, g, KS_LIN_GATE, r.ko);
 }
 

@@ -68,21 +68,20 @@ static inline int linrec_step_lds_bytes(int DK, int DVp) {
     while (tv < DVp / 4) tv <<= 1;
     return 4 * (3 * ((DK + 3) & ~3) + DVp + LR_STEP_THREADS / tv * DVp);
 }
-template <int KIND, int LR_STEP_ROWS, typename ActT>      // LR_STEP_ROWS: state rows a thread keeps in registers
-__global__ __launch_bounds__(LR_STEP_THREADS, LR_STEP_ROWS <= 8 ? 4 : 2) void linrec_step_kernel(LinRecArgs p) {
+// PAST: o goes past the L2 of this XCD, for another workgroup of the launch
+template <int KIND, int LR_STEP_ROWS, typename ActT, bool PAST = false>      // LR_STEP_ROWS: state rows a thread keeps in registers
+__device__ __forceinline__ void linrec_step_head(const LinRecArgs& p, const int h, const int seq, float* lr_sm, float* s_red, float* s_sc) {
     constexpr bool CH = KIND & 1, FUSED = KIND & 2;
     constexpr int NT = LR_STEP_THREADS;
-    const int h = blockIdx.x, seq = blockIdx.y, tid = threadIdx.x;
+    const int tid = threadIdx.x;
     const int n = p.seq_len[seq];
     if (n < p.len_lo || n > p.len_hi) return;
-    extern __shared__ __attribute__((aligned(16))) float lr_sm[];
     const int DK4 = (p.DK + 3) & ~3;
     float* sq = lr_sm;                   // [DK]
     float* sk = sq + DK4;                // [DK]
     float* sa = sk + DK4;                // [DK]   decay (CH)
     float* sv = sa + DK4;                // [DVp]
     float* red = sv + p.DVp;             // [waves or groups of rows][DVp]
-    __shared__ float s_red[NT / 64], s_sc[2];
     const int nv4 = p.DVp >> 2;
     int tv = 1;
     while (tv < nv4) tv <<= 1;           // host: nv4 <= NT
@@ -193,7 +192,10 @@ __global__ __launch_bounds__(LR_STEP_THREADS, LR_STEP_ROWS <= 8 ? 4 : 2) void li
                 if (!CH && p.Dskip) a = fmaf(p.Dskip[h], sv[i], a);
                 ov[c] = a;
                 ss = fmaf(a, a, ss);
-                if (!(CH && FUSED)) p.o[t * p.o_ld + (int64_t)h * p.DV + i] = a;
+                if (!(CH && FUSED)) {
+                    float* o = p.o + t * p.o_ld + (int64_t)h * p.DV + i;
+                    if constexpr (PAST) __hip_atomic_store(o, a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); else *o = a;
+                }
             }
         }
         if constexpr (CH && FUSED) {
@@ -215,6 +217,12 @@ __global__ __launch_bounds__(LR_STEP_THREADS, LR_STEP_ROWS <= 8 ? 4 : 2) void li
         }
         __syncthreads();
     }
+}
+template <int KIND, int LR_STEP_ROWS, typename ActT>
+__global__ __launch_bounds__(LR_STEP_THREADS, LR_STEP_ROWS <= 8 ? 4 : 2) void linrec_step_kernel(LinRecArgs p) {
+    extern __shared__ __attribute__((aligned(16))) float lr_sm[];
+    __shared__ float s_red[LR_STEP_THREADS / 64], s_sc[2];
+    linrec_step_head<KIND, LR_STEP_ROWS, ActT>(p, blockIdx.x, blockIdx.y, lr_sm, s_red, s_sc);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -742,11 +750,19 @@ __global__ __launch_bounds__(256) void gated_norm_kernel(GatedNormArgs p, ActT* 
 }
 
 // the same for one bf16 row by one workgroup of NT threads (a single part; 16-byte rows): part of another launch.  red: NT / 64 floats of LDS
-template <int NT>
+// PAST: y comes from other workgroups of the launch, past the L2 of this XCD
+template <int NT, bool PAST = false>
 __device__ __forceinline__ void gated_norm_row(const GatedNormArgs& p, int64_t t, bf16_t* __restrict__ out, float* red) {
     const float *y = p.y + t * p.y_ld, *g = p.gate + t * p.gate_ld;
     float ss = 0.f;
-    for (int c = threadIdx.x * 4; c < p.part; c += NT * 4) { const f32x4 v = *(const f32x4*)(y + c); ss += (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]); }
+    auto load = [&](int c) {
+        if constexpr (!PAST) return *(const f32x4*)(y + c);
+        union { f32x4 f; unsigned long long u[2]; } v;
+#pragma unroll
+        for (int i = 0; i < 2; i++) v.u[i] = __hip_atomic_load((const unsigned long long*)(y + c) + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return v.f;
+    };
+    for (int c = threadIdx.x * 4; c < p.part; c += NT * 4) { const f32x4 v = load(c); ss += (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]); }
     ss = wave_sum(ss);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
     __syncthreads();
@@ -754,7 +770,7 @@ __device__ __forceinline__ void gated_norm_row(const GatedNormArgs& p, int64_t t
     for (int w = 0; w < NT / 64; w++) ss += red[w];
     const float inv = 1.0f / sqrtf(ss / (float)p.part + p.eps);
     for (int c = threadIdx.x * 4; c < p.part; c += NT * 4) {
-        f32x4 v = *(const f32x4*)(y + c);
+        f32x4 v = load(c);
         const f32x4 s = *(const f32x4*)(g + c), w = *(const f32x4*)(p.w + c);
 #pragma unroll
         for (int r = 0; r < 4; r++) v[r] *= inv * w[r] * (p.sig ? lr_sigmoid(s[r]) : lr_silu(s[r]));

@@ -186,7 +186,7 @@ struct nvl_model {
     float* lshift = nullptr; int64_t* shift_offs = nullptr;         // token shift: the kept rows a pass began with, where each layer's lies in a slot
     float* lvf = nullptr; int64_t lvf_ld = 0;                       // grouped attention: the first mixing layer's values of the running batch
     void *side_emb = nullptr, *lside = nullptr; int64_t side_ld = 0; int side_kp = 0;     // per-layer token inputs: table (rows of L * side4 entries), operand of the projection
-    float* grp_part = nullptr; int32_t* grp_cnt = nullptr; int64_t grp_cap = 0;           // grouped attention: key splits
+    float* grp_part = nullptr; int32_t *grp_cnt = nullptr, *lin_cnt = nullptr; int64_t grp_cap = 0;           // grouped attention: key splits; tickets of a second mixer's heads
     std::vector<nvl::KeyMask> masks;    // distinct key masks of the attention layers
     void* lat_cache = nullptr; int64_t lat_block_stride = 0;
     float* rec_state = nullptr; int64_t rec_slot_stride = 0;

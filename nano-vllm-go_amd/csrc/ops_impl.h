@@ -432,6 +432,7 @@ extern "C" int nvl_set_tuning(int key, int value) {
     if (key == 31) { const int old = g_moe_fused_route; g_moe_fused_route = value; return old; }
     if (key == 33) { const int old = g_moe_defer_down; g_moe_defer_down = value; return old; }
     if (key == 41) { const int old = g_pp_split; g_pp_split = value; return old; }
+    if (key == 44) { const int old = g_lin_rides; g_lin_rides = value; return old; }
     if (key == 43) { const int old = g_attn_order; g_attn_order = value; return old; }
     if (key == 35) { const int old = g_attn_kv_nt; g_attn_kv_nt = value; return old; }
     if (key == 37) { const int old = g_grouped_split; g_grouped_split = value < 0 || value > GROUPED_SPLITS ? 0 : value; return old; }

@@ -1,0 +1,43 @@
+"""Decode steps whose attention launch also takes a second mixer's recurrence and, by the last of a sequence's workgroups, its gated norm (grouped.h
+grouped_short_kernel): the bits of the launches of their own."""
+import numpy as np
+import pytest
+
+import medulorn_models as MM
+from layered_helpers import build
+
+pytestmark = pytest.mark.gpu
+rot = MM.rot
+LAYERS = {      # key and value widths of the recurrence: what a thread's eight rows hold at most, ragged rows and columns, one head, more heads than attention
+    "128x128": dict(heads=4, kv_heads=2, dim=128, vdim=128, window=65, keep=3, turn=rot(128), heads2=5, dim2=128, vdim2=128),
+    "20x32": dict(heads=4, kv_heads=2, dim=64, vdim=64, window=None, turn=rot(64), heads2=3, dim2=20, vdim2=32),
+    "one-head": dict(heads=4, kv_heads=4, dim=64, vdim=32, window=70, turn=rot(64), heads2=1, dim2=64, vdim2=52),
+    "many-heads": dict(heads=2, kv_heads=1, dim=64, vdim=128, window=None, turn=rot(64), heads2=24, dim2=16, vdim2=16),
+    "256x64": dict(heads=4, kv_heads=2, dim=128, vdim=64, window=None, turn=rot(128), heads2=2, dim2=256, vdim2=64),
+    "256x128": dict(heads=4, kv_heads=2, dim=128, vdim=128, window=None, turn=rot(128), heads2=2, dim2=256, vdim2=128),      # sixteen rows a thread: a launch of its own
+}
+
+
+@pytest.mark.parametrize("split", [0, 3])
+@pytest.mark.parametrize("n", [1, 5, 40])
+@pytest.mark.parametrize("name", list(LAYERS))
+def test_same_bits(gpu, tmp_path, name, n, split):
+    cfg = MM.config([MM.parallel(**LAYERS[name]), MM.parallel(**LAYERS[name])], width=128, vocab=90)
+    m = build(gpu, tmp_path, cfg, MM.weights(cfg, 4), "bf16", max_seqs=40, kv_num_blocks=160)
+    r = np.random.default_rng(n)
+    ids, lens = list(range(n)), [1 + (37 * i) % 90 for i in range(n)]
+    prompts = [r.integers(0, 90, k).tolist() for k in lens]
+    lib, got = gpu.lib(), []
+    for rides in (0, 2):
+        old = [(key, lib.nvl_set_tuning(key, v)) for key, v in ((44, rides), (37, split))]
+        for i in ids:
+            m.seq_open(i)
+        for a in range(0, n, 8):
+            m.forward_batch(ids[a:a + 8], prompts[a:a + 8], [0] * len(ids[a:a + 8]), want_logits=False)
+        got.append(np.stack([m.forward_batch(ids, [[(5 * i + j) % 90] for i in ids], [k + j for k in lens])[0] for j in range(6)]))      # (replays from the third)
+        for i in ids:
+            m.seq_close(i)
+        for key, v in old:
+            lib.nvl_set_tuning(key, v)
+    m.close()
+    assert np.isfinite(got[0]).all() and np.array_equal(got[0], got[1])
