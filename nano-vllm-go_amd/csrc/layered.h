@@ -1390,7 +1390,8 @@ void mix_grouped(nvl_model* m, const LayerRun& r, const MixerW& w, const Meta& m
         const int64_t wgs = (int64_t)a.G * cdiv(std::min<int64_t>((int64_t)max_len * a.group, a.short_rows), 16);
         // Key tiles are split over workgroups once a wave would walk more than two: a split costs a round trip to memory and back (one
         // sequence of 2048 tokens with a window of 1024: 13.1 us unsplit, 13.7 in four; without a window, 3900 tokens: 27.8 -> 16.6 us)
-        const int key_tiles = 1 << layered_kt_log2(m), nw = dt <= 8 ? 8 : 4;
+        // (a window or chunk holds no more: requests of 6 x 1100 keys with windows and chunks of 512, in two 13.9 and 12.1 us, whole 13.4 and 11.6)
+        const int key_tiles = std::min(1 << layered_kt_log2(m), span > 0 ? span / 64 + 2 + cdiv(a.mask.keep, 64) : 1 << 30), nw = dt <= 8 ? 8 : 4;
         int z = 1;
         while (z < GROUPED_SPLITS && wgs * n_seqs * z * 2 <= 256 && z * 2 * 2 * nw <= key_tiles) z *= 2;
         if (g_grouped_split) z = (int)std::min<int64_t>(g_grouped_split, std::max<int64_t>(1, m->grp_cap / (wgs * n_seqs)));

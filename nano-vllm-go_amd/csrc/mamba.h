@@ -331,23 +331,18 @@ __global__ __launch_bounds__(256) void mamba_ssd_kernel(MambaArgs p) {
         rdt = lane < nv ? p.delta[(int64_t)(t0 + c0 + lane) * p.nh + h] : 0.f;
 #pragma unroll
         for (int k = 0; k < NBI; k++) {
-            const int i = tid + 256 * k, t = 4 * (i & 15), q4 = (i >> 4) * 4;
+            const int i = tid + 256 * k, t = 4 * (i & 15), q4 = (min(i, BI - 1) >> 4) * 4;
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                rb[k][e] = rc[k][e] = f32x4{0.f, 0.f, 0.f, 0.f};
-                if (i < BI && t + e < nv) {
-                    const float* xr = x0 + (int64_t)(t + e) * p.conv_dim + p.EH + g * SS + q4;
-                    rb[k][e] = *(const f32x4*)xr;
-                    if (MODE != 1) rc[k][e] = *(const f32x4*)(xr + p.ng * SS);
-                }
+                // (tokens past the end: the last one's values, replaced below.  With the loads under a condition instead some of these registers lay in scratch memory)
+                const float* xr = x0 + (int64_t)min(t + e, nv - 1) * p.conv_dim + p.EH + g * SS + q4;
+                rb[k][e] = *(const f32x4*)xr;
+                if (MODE != 1) rc[k][e] = *(const f32x4*)(xr + p.ng * SS);
             }
         }
-        const int t = 4 * (tid & 15), d4 = (tid >> 4) * 4;
+        const int t = 4 * (tid & 15), d4 = (min(tid, UI - 1) >> 4) * 4;
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            ru[e] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (tid < UI && t + e < nv) ru[e] = *(const f32x4*)(x0 + (int64_t)(t + e) * p.conv_dim + h * HD + d4);
-        }
+        for (int e = 0; e < 4; e++) ru[e] = *(const f32x4*)(x0 + (int64_t)min(t + e, nv - 1) * p.conv_dim + h * HD + d4);
     };
     const int c_first = MODE == 0 ? 0 : (int)blockIdx.z * Q, c_end = MODE == 0 ? n : c_first + 1;
     fetch(c_first);
@@ -368,6 +363,16 @@ __global__ __launch_bounds__(256) void mamba_ssd_kernel(MambaArgs p) {
                 for (int r = 0; r < 4; r++) Sb[(16 * sd + 4 * fg + r) * LC + 16 * (sn0 + j) + fr] = (bf16_t)sacc[j][r];
         }
         // ---- u, B, C of the chunk as bf16, K-contiguous; B and u also transposed ----
+        {
+            const int t = 4 * (tid & 15);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (t + e >= nv) {
+                    ru[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int k = 0; k < NBI; k++) { rb[k][e] = f32x4{0.f, 0.f, 0.f, 0.f}; if (MODE != 1) rc[k][e] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+                }
+        }
 #pragma unroll
         for (int k = 0; k < NBI; k++) {
             const int i = tid + 256 * k, t = 4 * (i & 15), q4 = (i >> 4) * 4;
