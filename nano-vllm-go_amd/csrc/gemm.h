@@ -442,15 +442,16 @@ __device__ __forceinline__ void epilogue_qkv_head(const GemmArgs& p, int m, int 
 // ------------------------------------------------------------------------------------------
 // bf16 MFMA kernel (prefill), one template, instances chosen per shape by the launcher:
 //   <128,128, 2,2, 4, BK 32>  4 waves, wave tile 64x64, a ring of 4 K tiles of 32 (64 KiB, 2 workgroups/CU): what does not fill
-//                             256x256 tiles (below)
-//   <256,128, 4,2, 3>  8 waves, wave tile  64x64, 3 LDS stages (144 KiB): two K tiles in flight
+//                             256x256 tiles (below); <128,128, 4,2, 4, BK 32> on 8 waves of 32x64 (ring_eight)
+//   <256,128, 4,2, 6, BK 32>  8 waves, wave tile 64x64, a ring of 6 (144 KiB): wide projections of few rows (ring256_wins)
+//   <256,128, 4,2, 3>  8 waves, wave tile  64x64, 3 LDS stages (144 KiB): two K tiles in flight (experts, a tuning option)
 //   <256,256, 2,4, 2>  8 waves, wave tile 128x64, 2 LDS stages (128 KiB): least LDS traffic per MFMA
 //                      ((8+4) fragment reads per 32 MFMAs instead of (4+4) per 16)
 // BK 32: the fragments of a K tile are read, and the loads of another issued, between the products of the tile before.  A lone workgroup's K tile is
 // 0.125 us of products; with reads and loads in a row in front of them it took 0.234, between them 0.188 (two workgroups a CU 0.34 and 0.33 for
 // both), and three K tiles in flight instead of one cover the weights' way from HBM.  The lock-step loop over two tiles of 64 that was here -> now, us:
 // 487 x 3072 x 2048 33.5 -> 22.7, 487 x 2048 x 8192 112 -> 73, 200 x 16384 x 2048 33 -> 24, 974 x 3072 x 2048 26.5 -> 21.0, 600 x 768 x 3072 37.5 -> 26.9,
-// 2000 x 2048 x 2048 31.7 -> 26.6, 487 x 16384 x 2048 (two a CU) 40.8 -> 39.5, 900 x 4672 x 4544 60.7 -> 58.2.  Deeper rings, and 256x128 tiles of this form, are slower.
+// 2000 x 2048 x 2048 31.7 -> 26.6, 487 x 16384 x 2048 (two a CU) 40.8 -> 39.5, 900 x 4672 x 4544 60.7 -> 58.2.  Deeper rings of 128x128 tiles are slower.
 // Every operand tile is a run of 1-KiB fragment-major blocks, so one
 // global_load_lds_dwordx4 per block fills LDS lane-linearly and the fragment ds_read_b128s are
 // conflict-free.  Raw s_barrier + counted s_waitcnt vmcnt keep (STAGES-2) later tiles in flight
@@ -485,7 +486,7 @@ template <int BM, int BN, int STAGES, int BK = G_BK>
 constexpr int gemm_lds_bytes() { return STAGES * (BM + BN) * BK * 2; }
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int EPI, typename OutT, int BK = G_BK>
-__global__ __launch_bounds__(WAVES_M * WAVES_N * 64, (WAVES_M * WAVES_N == 4 && STAGES * BK <= 160) ? 2 : 1)
+__global__ __launch_bounds__(WAVES_M * WAVES_N * 64, (WAVES_M * WAVES_N == 4 && STAGES * BK <= 160) ? 2 : (BK == 32 && BM == 128) ? 4 : 1)
 void gemm_bf16_kernel(GemmArgs p) {
     constexpr int NW = WAVES_M * WAVES_N;
     constexpr int TM = BM / WAVES_M / 16, TN = BN / WAVES_N / 16;   // 16x16 accumulator tiles per wave
@@ -511,7 +512,7 @@ void gemm_bf16_kernel(GemmArgs p) {
         p.W = (const bf16_t*)p.W + (int64_t)e * p.w_expert_stride;
         tm = 0;
     } else {
-        tile_coords(xcd_remap(blockIdx.x, gridDim.x), gridDim.x / tiles_n, tiles_n, NW == 4 ? 8 : 4, tm, tn);
+        tile_coords(xcd_remap(blockIdx.x, gridDim.x), gridDim.x / tiles_n, tiles_n, NW == 4 || BK == 32 ? 8 : 4, tm, tn);
         if (p.seg) {
             row_base = p.seg[0];
             p.M = p.seg[1] - row_base;
@@ -581,7 +582,8 @@ void gemm_bf16_kernel(GemmArgs p) {
         nt = per + ((int)blockIdx.y < extra ? 1 : 0);
     }
     if constexpr (BK == 32) {
-        static_assert(BM == 128 && BN == 128 && TM + TN == 8 && PW == 4, "eight reads and four loads between sixteen products");
+        constexpr bool ONE = TM * TN < 16;      // eight products: a read at each, the loads beside the first; sixteen: reads and loads in turn
+        static_assert(TM + TN <= TM * TN / (ONE ? 1 : 2) && PW <= TM * TN / (ONE ? 1 : 2), "reads and loads between the products");
         // a K tile's fragments are read while the products of the one before run; its slot is filled again as soon as every wave holds them
         bf16x8 fa[2][TM], fw[2][TN];
         auto fragments = [&](int slot, bf16x8 (&af)[TM], bf16x8 (&wf)[TN]) {
@@ -613,16 +615,17 @@ void gemm_bf16_kernel(GemmArgs p) {
                 const int i = e / TN, j = e % TN;
                 acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], af[i], acc[i][j], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
-                if (e % 2 == 0 && e / 2 < TN) wn[e / 2] = *(const bf16x8*)(sbuf + w_blk_off + e / 2 * 1024);
-                if (e % 2 == 0 && e / 2 >= TN) an[e / 2 - TN] = *(const bf16x8*)(sbuf + a_blk_off + (e / 2 - TN) * 1024);
-                if (e % 2 == 1 && e / 2 < PW && load) stage_one(slot, kt0 + t + STAGES, e / 2);
+                const int rd = ONE ? e : e % 2 == 0 ? e / 2 : TM + TN, ld = ONE ? e : e % 2 == 1 ? e / 2 : PW;
+                if (rd < TN) wn[rd < TN ? rd : 0] = *(const bf16x8*)(sbuf + w_blk_off + rd * 1024);
+                else if (rd < TM + TN) an[rd < TM + TN ? rd - TN : 0] = *(const bf16x8*)(sbuf + a_blk_off + (rd - TN) * 1024);
+                if (ld < PW && load) stage_one(slot, kt0 + t + STAGES, ld);
                 __builtin_amdgcn_sched_barrier(0);
             }
             slot = next;
             // tile t + 2 must have landed; the younger ones stay in flight
             __builtin_amdgcn_s_waitcnt(0xC07F);      // lgkmcnt(0); the builtin, which the compiler counts: behind asm it waits for the reads a second time, in front of the products
             if (FULL) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PW * (STAGES - 2)) : "memory");
-            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            else wait_tiles_in_flight(nt - 3 - t);
             __builtin_amdgcn_s_barrier();
         };
         for (; t + 1 + STAGES < nt; t += 2) {
@@ -1942,7 +1945,7 @@ inline int g_narrow_waves = 2048;   // waves per narrow-form launch (nvl_set_tun
 inline int g_wide_ksplit = 0;   // experiment (nvl_set_tuning key 4): K split of the wide form when groups <= 512
 inline int g_x_mask = 1;            // nvl_set_tuning key 24: decode kernels skip the activation fetch of padded rows (M % 16 != 0)
 inline int g_force_ntw = 0, g_force_ksplit = 0;   // tuning overrides (nvl_bench_gemm only)
-inline int g_force_tile = 0;                      // 0 automatic, 1: 128x128x2st, 2: 256x128x3st, 3: 256x256x2st, 5: ping-pong 256x256
+inline int g_force_tile = 0;                      // 0 automatic, 1: 128x128 (ring), 2: 256x128 (ring), 3: 256x256x2st, 5: ping-pong 256x256
 
 template <int EPI, typename OutT>
 static inline bool launch_gemm_skinny_bf16(hipStream_t st, const GemmArgs& a);
@@ -2223,6 +2226,28 @@ static inline bool pp_wins(GemmArgs& a) {
     // (whole tiles lose to 128x128 tiles that fit one round of two a CU, which the costs miss at times: 12288 x 2048 at 520 rows 42.6 / 30.2, 16384 x 2048 at 400 42 / 38)
     return faster && (a.splits > 1 || cdiv(a.M, 128) * cdiv(a.N, 128) > 512);
 }
+// 128x128 tiles on eight waves of 32x64 instead of four of 64x64: twice the waves to cover the way to the operands, half as long an epilogue each, half as many
+// products more to read for.  Better while each CU has one tile at most, whatever the K (487 x 2048 x 2048 24.4 -> 22.8 us, 600 x 768 x 3072 27.1 -> 25.4, 700 x 6144 x 4096
+// 37.1 -> 36.5), with GELUs always (700 x 3072 x 768 16.8 -> 12.6, 3200 of them 35.9 -> 29.0, 520 x 18176 x 4544 123 -> 103), with fp32 results of a short K (4100 x 2048 x 2048
+// 55.7 -> 52.3, 3200 x 3072 36.7 -> 35.8); not two a CU of a long one (1800 x 4096 x 4096 64.1 / 66.0, 900 x 28672 x 4096 221 / 236)
+template <int EPI, typename OutT>
+static inline bool ring_eight(const GemmArgs& a) {
+    const int tiles = cdiv(a.M, 128) * cdiv(a.N, 128) * (a.sk_part ? a.sk_slices : 1);
+    return tiles <= 256 || EPI == EPI_GELU || EPI == EPI_GELU_TOK || EPI == EPI_JOINT || (sizeof(OutT) == 4 && a.K <= 2048);
+}
+// Up to 512 rows of a wide projection: 256x128 tiles of the ring, six K tiles deep, one a CU, where 128x128 tiles would be two on some.  What bounds both is the way
+// from L2 to the CUs (487 x 16384 x 2048 without its products 37.8 of 39.4 us; some 100 lines a CU on their way, 460 cycles each), and a tile of twice the size asks for
+// a quarter less.  us, 128x128 -> here: 16384 x 2048 at 260 / 350 / 400 / 487 rows 36.7 -> 32.2, 40.2 -> 32.8, 36.4 -> 33.2, 41.1 -> 35.0; 12288 x 2048 at 300 / 450 33.3 -> 29.9, 35.4 -> 32.4;
+// 28672 x 4096 at 130 / 256 61.5 -> 55.0, 73.8 -> 63.4; 22848 x 4544 at 140 74.9 -> 65.1; 16384 x 1024 at 300 23.6 -> 19.7.  Not for fp32 results (1300 x 4096 x 4096 57.1 / 59.4: nothing beside
+// the epilogue) nor more rows (700 x 8192 x 2048 27.7 / 28.8, 1000 x 6144 x 2048 27.6 / 28.9).  The cost is good to 5 %; large tiles in parts: 18176 x 4544 at 140 / 256 65.4 / 69.9, here 62.9 / 73.0
+template <int EPI, typename OutT>
+static inline bool ring256_wins(const GemmArgs& a, bool pp) {
+    if (EPI == EPI_RESID || EPI == EPI_QKV || sizeof(OutT) == 4 || a.seg || a.a_rows || a.sk_part || a.M > 512 || a.M <= 128) return false;
+    if (cdiv(a.M, 256) * cdiv(a.N, 128) > 256 || cdiv(a.M, 128) * cdiv(a.N, 128) <= 256) return false;
+    int parts;
+    const double cost = 7.5 + (a.K >> 5) * (0.34 + 0.10 * a.M / (256.0 * cdiv(a.M, 256)));
+    return !pp || cost < pp_cost(a.M, a.N, a.K, epi_glu(EPI) ? (int)sizeof(OutT) / 2 : (int)sizeof(OutT), a.splits > 1, parts);
+}
 template <int EPI, typename OutT, int WAVES_N>
 static inline void launch_pp(hipStream_t st, const GemmArgs& a) {
     const int T = cdiv(a.M, 256) * cdiv(a.N, 256), n = cdiv(T, 8);
@@ -2258,8 +2283,8 @@ static inline void launch_gemm_grouped(hipStream_t st, const GemmArgs& a, int ma
     // (decode-sized batches too, a handful of rows an expert: us a layer of 1 / 4 / 16 / 64 rows, 32 experts, 8 a token, with four K tiles of 64 in 128 KiB ->
     // here: 512 x 2048 75 -> 69.6, 86.6 -> 79.7, 97.2 -> 92.8, 120.2 -> 117.2; 1024 x 4096 128 -> 124, 202 -> 184, 235 -> 229, 271 -> 267; 512 x 1024 3 %)
     constexpr int lds = gemm_lds_bytes<128, 128, 4, 32>();
-    NVL_LDS_ATTR((gemm_bf16_kernel<128, 128, 2, 2, 4, EPI, OutT, 32>), lds);
-    hipLaunchKernelGGL((gemm_bf16_kernel<128, 128, 2, 2, 4, EPI, OutT, 32>), dim3(cdiv(a.N, 128) * max_mtiles), dim3(256),
+    NVL_LDS_ATTR((gemm_bf16_kernel<128, 128, 4, 2, 4, EPI, OutT, 32>), lds);
+    hipLaunchKernelGGL((gemm_bf16_kernel<128, 128, 4, 2, 4, EPI, OutT, 32>), dim3(cdiv(a.N, 128) * max_mtiles), dim3(512),
                        lds, st, a);
 }
 
@@ -2411,13 +2436,14 @@ void launch_gemm_bf16(hipStream_t st, const GemmArgs& a) {
     int tile = g_force_tile;
     GemmArgs as = a;
     as.splits = 1;
-    // 5: the ping-pong form; else 128x128 tiles (the lock-step 256-wide forms and a ping-pong 256x128 variant with wave tiles of 64x64
-    // never win, profiles/r01e_gemm_sweep_mid.txt)
-    if (tile == 0) tile = pp_wins<EPI, OutT>(as) ? 5 : 1;
+    // 5: the ping-pong form; 2: 256x128 tiles on the ring; else 128x128 tiles (the lock-step 256-wide forms and a ping-pong 256x128 variant with wave
+    // tiles of 64x64 never win, profiles/r01e_gemm_sweep_mid.txt)
+    if (tile == 0) { tile = pp_wins<EPI, OutT>(as) ? 5 : 1; if (ring256_wins<EPI, OutT>(as, tile == 5)) tile = 2; }
     else if (tile == 5) pp_wins<EPI, OutT>(as);
     if (tile == 5 && !a.seg && !a.a_rows) { launch_pp<EPI, OutT, 4>(st, as); return; }      // (4-slot ring: 5 slots -3 %, 3 slots -3 %, r01 sweep)
     if (tile == 3) launch_gemm_tile<256, 256, 2, 4, 2, EPI, OutT>(st, a);
-    else if (tile == 2) launch_gemm_tile<256, 128, 4, 2, 3, EPI, OutT>(st, a);
+    else if (tile == 2) launch_gemm_tile<256, 128, 4, 2, 6, EPI, OutT, 32>(st, a);
+    else if (ring_eight<EPI, OutT>(a)) launch_gemm_tile<128, 128, 4, 2, 4, EPI, OutT, 32>(st, a);
     else launch_gemm_tile<128, 128, 2, 2, 4, EPI, OutT, 32>(st, a);
     }
 }
