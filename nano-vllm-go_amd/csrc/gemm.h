@@ -2406,11 +2406,10 @@ void launch_gemm_bf16(hipStream_t st, const GemmArgs& a) {
         // in one launch instead (GemmArgs::m_passes): the groups of a weight block run side by side on one XCD, so the
         // weights cross HBM once.  Only the narrow projections (QKV, O, FFN-down) do; FFN-up and the LM head have enough
         // tiles (g_chunk_all_m: below it every projection would).
-        // (us, groups / tiles: 768 x 768 at 300 rows 5.5 / 12.3, 2304 x 768 10.3 / 11.0, 6144 x 4096 62.8 / 39.4, 8512 x 2048 at 140 41.2 / 22.9.  A lane of the
-        // tiles has 64 GELUs, 5 us beside a K as short: 3072 x 768 at 400 / 450 / 512 rows 16.4 / 17.4, 15.8 / 17.7, 17.6 / 18.2; 4096 x 1024 at
-        // 300 / 350 / 400 17.2 / 19.3, 19.0 / 19.8, 23.0 / 19.4)
+        // (us, groups / tiles: 768 x 768 at 300 rows 5.5 / 12.3, 2304 x 768 10.3 / 11.0, 6144 x 4096 62.8 / 39.4, 8512 x 2048 at 140 41.2 / 22.9.  With GELUs: 3072 x 768 at
+        // 300 / 350 / 400 / 512 rows 11.9 / 13.2, 14.7 / 13.6, 16.2 / 13.3, 17.4 / 13.9; 4096 x 1024 at 200 / 260 / 350 12.2 / 15.4, 16.1 / 15.1, 19.2 / 15.7; 6144 x 1024 at 200 14.5 / 16.1)
         const bool few_tiles = cdiv(a.M, 128) * cdiv(a.N, 128) < g_chunk_min_tiles &&
-                               passes_cost(a.M, a.N, a.K) < tile128_cost(a.M, a.N, a.K, EPI == EPI_RESID ? 8 : (int)sizeof(OutT), 1) + (EPI == EPI_GELU || EPI == EPI_JOINT ? 5.0 : 0.0);
+                               passes_cost(a.M, a.N, a.K) < tile128_cost(a.M, a.N, a.K, EPI == EPI_RESID ? 8 : (int)sizeof(OutT), 1) + (EPI == EPI_GELU || EPI == EPI_JOINT ? 1.0 : 0.0);
         if (a.M > 64 && a.M <= g_chunk_max_m && (a.M <= g_chunk_all_m || few_tiles || a.rs_in || a.rs_out) && !a.a_rows && !a.seg && !a.sk_part && a.K % 32 == 0 &&
             g_force_tile == 0) {
             GemmArgs c = a;
