@@ -443,6 +443,7 @@ __device__ __forceinline__ void epilogue_qkv_head(const GemmArgs& p, int m, int 
 // bf16 MFMA kernel (prefill), one template, instances chosen per shape by the launcher:
 //   <128,128, 2,2, 4, BK 32>  4 waves, wave tile 64x64, a ring of 4 K tiles of 32 (64 KiB, 2 workgroups/CU): what does not fill
 //                             256x256 tiles (below); <128,128, 4,2, 4, BK 32> on 8 waves of 32x64 (ring_eight)
+//   < 64,128, 2,2, 4 or 6, BK 32>  4 waves, wave tile 32x64: few tiles (ring64_fits)
 //   <256,128, 4,2, 6, BK 32>  8 waves, wave tile 64x64, a ring of 6 (144 KiB): wide projections of few rows (ring256_wins)
 //   <256,128, 4,2, 3>  8 waves, wave tile  64x64, 3 LDS stages (144 KiB): two K tiles in flight (experts, a tuning option)
 //   <256,256, 2,4, 2>  8 waves, wave tile 128x64, 2 LDS stages (128 KiB): least LDS traffic per MFMA
@@ -2194,18 +2195,32 @@ static inline double tile128_cost(int M, int N, int K, int out_bytes, int slices
     const double x = (double)cdiv(M, 128) * cdiv(N, 128) * slices / 256.0, per = x <= 1.0 ? 6.7 + x : x <= 2.0 ? 11.6 + 2.0 * (x - 1.0) : 1.1 + 8.3 * x;
     return K / 1024.0 / slices * per + 7.1 + (slices > 1 ? gemm_epilogue_us(M, N, 8 * slices) : 0.44 * gemm_epilogue_us(M, N, out_bytes));
 }
+// 64x128 tiles of the ring on four waves of 32x64, where each CU has one at most: twice the CUs at work of a launch of few 128x128 tiles.  us, 128x128 -> here (weights from
+// HBM): 600 x 3072 x 2048 22.9 -> 20.1, 900 x 2048 x 2048 23.3 -> 21.2, 520 / 2000 x 768 x 768 11.7 -> 9.1, 12.8 -> 10.1, 900 x 768 x 3072 29.2 -> 25.7, 520 x 2304 x 768 10.9 -> 9.2,
+// 900 x 1536 x 1024 12.7 -> 10.5, 260 x 6144 x 4096 39.7 -> 33.8; not two a CU (1100 x 2048 x 2048 24.1 / 24.4, 700 x 3072 x 2048 22.7 / 23.5).  Six K tiles deep for a long K
+// (6144 x 4096 36.2 -> 33.8, 4096 x 4096 at 260 38.3 -> 36.0; 2048 x 2048 20.6 -> 21.3, 768 x 768 9.1 -> 10.9).  Another wave that touches the weights 12 or 24 K tiles ahead
+// makes all forms slower (487 x 16384 x 2048 36 -> 37.6, 39.6)
+static inline bool ring64_fits(int M, int N, int slices) { return cdiv(M, 64) * cdiv(N, 128) * slices <= 256; }
+static inline double ring64_cost(int M, int N, int K, int out_bytes, int slices) {
+    const double fill = cdiv(M, 64) * cdiv(N, 128) * slices / 256.0;
+    return 3.7 + (0.235 + 0.05 * fill) * (K >> 5) / slices + (slices > 1 ? gemm_epilogue_us(M, N, 8 * slices) : 0.44 * gemm_epilogue_us(M, N, out_bytes));
+}
+static inline double tile_cost(int M, int N, int K, int out_bytes, int slices) {
+    const double c = tile128_cost(M, N, K, out_bytes, slices);
+    return ring64_fits(M, N, slices) ? std::min(c, ring64_cost(M, N, K, out_bytes, slices)) : c;
+}
 // ... and how many slices cost least, the norm that sums them counted.  Beyond a workgroup a CU more of them only add traffic (487 x 2048 x 8192:
 // eight 27.5 us, four 26.0, and half as much for the norm to read)
 static inline int tile128_slices(int M, int N, int K, int most, double& cost) {
     int slices = 1;
-    cost = tile128_cost(M, N, K, 8, 1);
+    cost = tile_cost(M, N, K, 8, 1);
     if (g_chunk_max_m <= 64) {           // (key 11 = 64: sums in one order whatever the rows)
         while (slices < most && cdiv(M, 128) * cdiv(N, 128) * slices < 512 && K / (slices * 2) >= 512) slices *= 2;
-        cost = tile128_cost(M, N, K, 8, slices);
+        cost = tile_cost(M, N, K, 8, slices);
         return slices;
     }
     for (int s = 2; s <= most && K / s >= 512; s *= 2) {
-        const double c = tile128_cost(M, N, K, 8, s);
+        const double c = tile_cost(M, N, K, 8, s);
         if (c < 0.97 * cost) { cost = c; slices = s; }
     }
     return slices;
@@ -2222,7 +2237,7 @@ static inline bool pp_wins(GemmArgs& a) {
     // it to a few workgroups, 17424 x 4096 at 140 / 200 rows 82 / 86 us in parts, 74 / 78 on 128x128 tiles)
     const bool parts = a.split_units * SPLIT_UNIT >= SPLIT_WS_BYTES && (a.M > MID_MAX_ROWS || a.M <= std::max(64, g_chunk_max_m)) &&
                        (EPI != EPI_GROUPED || cdiv(a.M, 256) * cdiv(a.N, 256) > 256);
-    const bool faster = pp_cost(a.M, a.N, a.K, bytes, parts, a.splits) < 1.05 * tile128_cost(a.M, a.N, a.K, bytes, 1);      // (ties: 4176 x 4096 x 4096 161 / 172, 200 x 18176 x 4544 67 / 79)
+    const bool faster = pp_cost(a.M, a.N, a.K, bytes, parts, a.splits) < 1.05 * tile_cost(a.M, a.N, a.K, bytes, 1);      // (ties: 4176 x 4096 x 4096 161 / 172, 200 x 18176 x 4544 67 / 79)
     // (whole tiles lose to 128x128 tiles that fit one round of two a CU, which the costs miss at times: 12288 x 2048 at 520 rows 42.6 / 30.2, 16384 x 2048 at 400 42 / 38)
     return faster && (a.splits > 1 || cdiv(a.M, 128) * cdiv(a.N, 128) > 512);
 }
@@ -2409,7 +2424,7 @@ void launch_gemm_bf16(hipStream_t st, const GemmArgs& a) {
         // (us, groups / tiles: 768 x 768 at 300 rows 5.5 / 12.3, 2304 x 768 10.3 / 11.0, 6144 x 4096 62.8 / 39.4, 8512 x 2048 at 140 41.2 / 22.9.  With GELUs: 3072 x 768 at
         // 300 / 350 / 400 / 512 rows 11.9 / 13.2, 14.7 / 13.6, 16.2 / 13.3, 17.4 / 13.9; 4096 x 1024 at 200 / 260 / 350 12.2 / 15.4, 16.1 / 15.1, 19.2 / 15.7; 6144 x 1024 at 200 14.5 / 16.1)
         const bool few_tiles = cdiv(a.M, 128) * cdiv(a.N, 128) < g_chunk_min_tiles &&
-                               passes_cost(a.M, a.N, a.K) < tile128_cost(a.M, a.N, a.K, EPI == EPI_RESID ? 8 : (int)sizeof(OutT), 1) + (EPI == EPI_GELU || EPI == EPI_JOINT ? 1.0 : 0.0);
+                               passes_cost(a.M, a.N, a.K) < tile_cost(a.M, a.N, a.K, EPI == EPI_RESID ? 8 : (int)sizeof(OutT), 1) + (EPI == EPI_GELU || EPI == EPI_JOINT ? 1.0 : 0.0);
         if (a.M > 64 && a.M <= g_chunk_max_m && (a.M <= g_chunk_all_m || few_tiles || a.rs_in || a.rs_out) && !a.a_rows && !a.seg && !a.sk_part && a.K % 32 == 0 &&
             g_force_tile == 0) {
             GemmArgs c = a;
@@ -2442,7 +2457,10 @@ void launch_gemm_bf16(hipStream_t st, const GemmArgs& a) {
     if (tile == 5 && !a.seg && !a.a_rows) { launch_pp<EPI, OutT, 4>(st, as); return; }      // (4-slot ring: 5 slots -3 %, 3 slots -3 %, r01 sweep)
     if (tile == 3) launch_gemm_tile<256, 256, 2, 4, 2, EPI, OutT>(st, a);
     else if (tile == 2) launch_gemm_tile<256, 128, 4, 2, 6, EPI, OutT, 32>(st, a);
-    else if (ring_eight<EPI, OutT>(a)) launch_gemm_tile<128, 128, 4, 2, 4, EPI, OutT, 32>(st, a);
+    else if (ring64_fits(a.M, a.N, a.sk_part ? a.sk_slices : 1) && !a.seg && !a.a_rows) {
+        if (a.K >= 4096) launch_gemm_tile<64, 128, 2, 2, 6, EPI, OutT, 32>(st, a);
+        else launch_gemm_tile<64, 128, 2, 2, 4, EPI, OutT, 32>(st, a);
+    } else if (ring_eight<EPI, OutT>(a)) launch_gemm_tile<128, 128, 4, 2, 4, EPI, OutT, 32>(st, a);
     else launch_gemm_tile<128, 128, 2, 2, 4, EPI, OutT, 32>(st, a);
     }
 }
