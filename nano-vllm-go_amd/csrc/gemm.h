@@ -444,7 +444,7 @@ __device__ __forceinline__ void epilogue_qkv_head(const GemmArgs& p, int m, int 
 //   <128,128, 2,2, 4, BK 32>  4 waves, wave tile 64x64, a ring of 4 K tiles of 32 (64 KiB, 2 workgroups/CU): what does not fill
 //                             256x256 tiles (below); <128,128, 4,2, 4, BK 32> on 8 waves of 32x64 (ring_eight)
 //   < 64,128, 2,2, 4 or 6, BK 32>  4 waves, wave tile 32x64: few tiles (ring64_fits)
-//   <256,128, 4,2, 6, BK 32>  8 waves, wave tile 64x64, a ring of 6 (144 KiB): wide projections of few rows (ring256_wins)
+//   <256,128, 4,2, 6, BK 32>  8 waves, wave tile 64x64, a ring of 6 (144 KiB): where 128x128 tiles would be two on some CUs (ring256_wins)
 //   <256,128, 4,2, 3>  8 waves, wave tile  64x64, 3 LDS stages (144 KiB): two K tiles in flight (experts, a tuning option)
 //   <256,256, 2,4, 2>  8 waves, wave tile 128x64, 2 LDS stages (128 KiB): least LDS traffic per MFMA
 //                      ((8+4) fragment reads per 32 MFMAs instead of (4+4) per 16)
@@ -2237,7 +2237,9 @@ static inline bool pp_wins(GemmArgs& a) {
     // it to a few workgroups, 17424 x 4096 at 140 / 200 rows 82 / 86 us in parts, 74 / 78 on 128x128 tiles)
     const bool parts = a.split_units * SPLIT_UNIT >= SPLIT_WS_BYTES && (a.M > MID_MAX_ROWS || a.M <= std::max(64, g_chunk_max_m)) &&
                        (EPI != EPI_GROUPED || cdiv(a.M, 256) * cdiv(a.N, 256) > 256);
-    const bool faster = pp_cost(a.M, a.N, a.K, bytes, parts, a.splits) < 1.05 * tile_cost(a.M, a.N, a.K, bytes, 1);      // (ties: 4176 x 4096 x 4096 161 / 172, 200 x 18176 x 4544 67 / 79)
+    // (one round of whole tiles with a GLU starts and ends sooner than the fit has it: 520 / 700 x 16384 x 2048 53.4 / 46.2, 57.2 / 47.5 us on 128x128 / large tiles, 700 x 12288 50.5 / 45.2)
+    const double cost = pp_cost(a.M, a.N, a.K, bytes, parts, a.splits) - (epi_glu(EPI) && a.splits == 1 && cdiv(a.M, 256) * cdiv(a.N, 256) <= 256 ? 6.0 : 0.0);
+    const bool faster = cost < 1.05 * tile_cost(a.M, a.N, a.K, bytes, 1);      // (ties: 4176 x 4096 x 4096 161 / 172, 200 x 18176 x 4544 67 / 79)
     // (whole tiles lose to 128x128 tiles that fit one round of two a CU, which the costs miss at times: 12288 x 2048 at 520 rows 42.6 / 30.2, 16384 x 2048 at 400 42 / 38)
     return faster && (a.splits > 1 || cdiv(a.M, 128) * cdiv(a.N, 128) > 512);
 }
@@ -2250,18 +2252,32 @@ static inline bool ring_eight(const GemmArgs& a) {
     const int tiles = cdiv(a.M, 128) * cdiv(a.N, 128) * (a.sk_part ? a.sk_slices : 1);
     return tiles <= 256 || EPI == EPI_GELU || EPI == EPI_GELU_TOK || EPI == EPI_JOINT || (sizeof(OutT) == 4 && a.K <= 2048);
 }
-// Up to 512 rows of a wide projection: 256x128 tiles of the ring, six K tiles deep, one a CU, where 128x128 tiles would be two on some.  What bounds both is the way
-// from L2 to the CUs (487 x 16384 x 2048 without its products 37.8 of 39.4 us; some 100 lines a CU on their way, 460 cycles each), and a tile of twice the size asks for
-// a quarter less.  us, 128x128 -> here: 16384 x 2048 at 260 / 350 / 400 / 487 rows 36.7 -> 32.2, 40.2 -> 32.8, 36.4 -> 33.2, 41.1 -> 35.0; 12288 x 2048 at 300 / 450 33.3 -> 29.9, 35.4 -> 32.4;
-// 28672 x 4096 at 130 / 256 61.5 -> 55.0, 73.8 -> 63.4; 22848 x 4544 at 140 74.9 -> 65.1; 16384 x 1024 at 300 23.6 -> 19.7.  Not for fp32 results (1300 x 4096 x 4096 57.1 / 59.4: nothing beside
-// the epilogue) nor more rows (700 x 8192 x 2048 27.7 / 28.8, 1000 x 6144 x 2048 27.6 / 28.9).  The cost is good to 5 %; large tiles in parts: 18176 x 4544 at 140 / 256 65.4 / 69.9, here 62.9 / 73.0
+// 256x128 tiles of the ring, six K tiles deep, one a CU, where 128x128 tiles would be two on some.  What bounds both is the way from L2 to the CUs (487 x 16384 x 2048
+// without its products 37.8 of 39.4 us; some 100 lines a CU on their way, 460 cycles each), and a tile of twice the size asks for a quarter less.  us, 128x128 -> here (weights
+// from HBM): 16384 x 2048 at 260 / 350 / 400 / 487 rows 36.7 -> 32.2, 40.2 -> 32.8, 36.4 -> 33.2, 41.1 -> 35.0; 12288 x 2048 at 300 / 450 33.3 -> 29.9, 35.4 -> 32.4; 28672 x 4096 at 130 / 256
+// 61.5 -> 55.0, 73.8 -> 63.4; 22848 x 4544 at 140 74.9 -> 65.1; 16384 x 1024 at 300 23.6 -> 19.7.  The cost of up to 512 rows is good to 5 %; large tiles in parts: 18176 x 4544 at 140 / 256
+// 65.4 / 69.9, here 62.9 / 73.0.
+// More rows, where the 128x128 tiles are 1.2 a CU at least: 8512 x 2048 at 520 / 640 / 768 rows 38.0 -> 34.2, 42.3 -> 35.1, 44.3 -> 38.8; 4096 x 4096 at 1400 / 2048 75.2 -> 60.2, 86.4 -> 69.8
+// (large tiles 70.7, 79.3); 4544 x 4544 at 1100 / 1700 80.4 -> 64.7, 84.8 -> 71.9; 3072 x 2048 at 1700 / 2048 / 2560 36.2 -> 33.2, 40.0 -> 34.8, 40.8 -> 36.0; 2048 x 4096 at 2560 / 4096 69.4 -> 60.0,
+// 80.8 -> 70.5; 4096 x 1024 at 1100 .. 2048 4 %.  Not 288 tiles (768 x 6144 x 4096 57.7 / 60.8, 2300 x 2048 x 2048 34.2 / 36.4), a K below 1024 (2048 x 3072 x 768 20.5 / 23.5), nor 2048 x 2048 (3000
+// rows 35.8 / 38.0, 3500 40.0 / 40.1), nor the long epilogue of raw queries and keys (1600 x 3072 x 2048 42.5 / 46.1); a long K may be better in parts of large tiles (1280 x 4096 x 14336
+// 136 / 181, 1900 207 / 210)
 template <int EPI, typename OutT>
 static inline bool ring256_wins(const GemmArgs& a, bool pp) {
-    if (EPI == EPI_RESID || EPI == EPI_QKV || sizeof(OutT) == 4 || a.seg || a.a_rows || a.sk_part || a.M > 512 || a.M <= 128) return false;
-    if (cdiv(a.M, 256) * cdiv(a.N, 128) > 256 || cdiv(a.M, 128) * cdiv(a.N, 128) <= 256) return false;
+    if (a.seg || a.a_rows || a.sk_part || a.M <= 128) return false;
+    const int tiles = cdiv(a.M, 128) * cdiv(a.N, 128), bytes = EPI == EPI_RESID ? 8 : epi_glu(EPI) ? (int)sizeof(OutT) / 2 : (int)sizeof(OutT);
+    if (cdiv(a.M, 256) * cdiv(a.N, 128) > 256 || tiles <= 256) return false;
+    const double rows = a.M / (256.0 * cdiv(a.M, 256));
+    double cost;
+    if (a.M <= 512) {
+        if (EPI == EPI_RESID || EPI == EPI_QKV || sizeof(OutT) == 4) return false;
+        cost = 7.5 + (a.K >> 5) * (0.34 + 0.10 * rows);
+    } else {
+        if (EPI == EPI_GROUPED_RAW || tiles <= 288 || a.K < 1024 || (a.K < 4096 && a.N < 3072)) return false;
+        cost = 7.1 + 0.44 * gemm_epilogue_us(a.M, a.N, bytes) + (a.K >> 5) * (0.30 + 0.12 * rows);
+    }
     int parts;
-    const double cost = 7.5 + (a.K >> 5) * (0.34 + 0.10 * a.M / (256.0 * cdiv(a.M, 256)));
-    return !pp || cost < pp_cost(a.M, a.N, a.K, epi_glu(EPI) ? (int)sizeof(OutT) / 2 : (int)sizeof(OutT), a.splits > 1, parts);
+    return !pp || cost < (a.M <= 512 ? 1.0 : 0.93) * pp_cost(a.M, a.N, a.K, bytes, a.splits > 1, parts);
 }
 template <int EPI, typename OutT, int WAVES_N>
 static inline void launch_pp(hipStream_t st, const GemmArgs& a) {

@@ -48,3 +48,24 @@ def test_prompts(gpu, family, ffn, rows):
         m.close()
     assert np.array_equal(got[1], got[2])
     assert rel_err(got[1], got[0]) <= TOL
+
+
+@pytest.mark.parametrize("rows,tile,hidden,heads,kv", [(513, 2, 256, 4, 2), (769, 2, 320, 5, 5),       # every projection on 256x128 tiles: rotated heads and residuals too
+                                                       (1537, 0, 1024, 32, 8), (2560, 0, 1024, 32, 8)])      # 312 and 480 tiles of 3072 columns: they are chosen for queries, keys and values
+def test_wide_tiles_of_heads_and_residuals(gpu, rows, tile, hidden, heads, kv):
+    cfg = gpu.synth.tiny_config("llama", hidden=hidden, num_heads=heads, num_kv_heads=kv, head_dim=64, ffn_dim=512, num_layers=2, max_seq_len=2560)
+    w = gpu.synth.make_weights(cfg, seed=5, scale=0.03)
+    tokens = np.random.default_rng(rows).integers(0, cfg["vocab_size"], rows).tolist()
+    got = []
+    old = gpu.lib().nvl_set_tuning(0, tile)
+    try:
+        for precision in ("f32", "bf16"):
+            m = gpu.HipTransformerModel(cfg, w, precision=precision, max_seqs=1, max_batch_tokens=2560)
+            for _ in range(2 if precision == "bf16" else 1):
+                m.seq_reset(0)
+                got.append(m.forward_batch([0], [tokens], [0], all_logits=True)[0])
+            m.close()
+    finally:
+        gpu.lib().nvl_set_tuning(0, old)
+    assert np.array_equal(got[1], got[2])
+    assert rel_err(got[1], got[0]) <= TOL
