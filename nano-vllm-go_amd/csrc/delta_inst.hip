@@ -36,25 +36,25 @@ template <int NK, int NW, int KSP>
 static void scan(hipStream_t st, const DeltaArgs& p, int n_seqs) {
     constexpr int lds = delta_scan_lds_bytes<NK, NW, KSP>();
     NVL_LDS_ATTR((delta_scan_kernel<NK, NW, KSP>), lds);
-    hipLaunchKernelGGL((delta_scan_kernel<NK, NW, KSP>), dim3(p.H, n_seqs, cdiv(p.DV, 16 * NW / KSP)), dim3(NW * 64), lds, st, p);
+    hipLaunchKernelGGL((delta_scan_kernel<NK, NW, KSP>), dim3(p.H, cdiv(p.DV, 16 * NW / KSP), n_seqs), dim3(NW * 64), lds, st, p);
 }
-// Columns per workgroup (64 or 128) and parts of the key channels (KSP): more parts shorten the chain of a sequence's chunks, whose fp32
-// products bound a wave, and cost each of them an exchange.  us, fitted to 1 .. 64 sequences of 100 .. 1900 tokens x 16 heads of 128,
-// good to 20 %: the longest sequence's chain, all chunks at the chip's rate, the larger of them and a third of the other.
-// 5 x 300..1900 x 16 heads: 297 with whole channels, 237 in two parts; 1 x 1900 271 / 194 / 155 in one / two / four; 16 x 900 237 / 314 / 553.
-static double scan_cost(const DeltaArgs& p, int n_seqs, int nk, int nw, int ksp, int max_len, int tokens) {
+// Parts of the key channels (KSP): more parts shorten the chain of a sequence's chunks, whose fp32 products bound a wave, and cost each of them an exchange.
+// us, fitted to 1 .. 64 sequences of 100 .. 1900 tokens x 16 heads of 128, good to 20 %: the longest sequence's chain, all chunks at the chip's rate, the larger of them
+// and a quarter of the other.  Sequences of several lengths, longest first, fill the chip's gaps with the short ones; of one length they end together.
+// One / two / four parts, ms a prompt: 1 x 1900 6.5 / 5.9 / 5.6; 5 x 300..1900 12.5 / 11.9 / 11.7; 12 x 300..1900 22.9 / 22.3 / 23.0; 10 x 100..900 10.0 / 9.7 / 9.9; 16 x 900 25.6 / 26.2 / 27.4.
+static double scan_cost(const DeltaArgs& p, int n_seqs, int nk, int ksp, int max_len, int tokens) {
     const double size = nk / 8.0, heads = p.H * cdiv(p.DV, 64) / 2.0;
-    const double chain = cdiv(max_len, DELTA_C) * (1.95 + size * 2.55 * (nw / 4) / ksp);
-    const double all = heads * ((double)tokens / DELTA_C + 0.5 * n_seqs) * (size * 0.0225 + 0.0105 * ksp + (nw == 8 ? 0.0025 : 0.0));
-    return std::max(chain, all) + 0.35 * std::min(chain, all);
+    const double chain = cdiv(max_len, DELTA_C) * (1.95 + size * 2.55 / ksp);
+    const double ragged = n_seqs <= DELTA_ORDERED ? 0.4 + 0.6 * tokens / ((double)n_seqs * max_len) : 1.0;
+    const double all = heads * ((double)tokens / DELTA_C + 0.5 * n_seqs) * (size * 0.0225 + 0.0105 * ksp) * ragged;
+    return std::max(chain, all) + 0.25 * std::min(chain, all);
 }
 template <int NK, int... PARTS>
 static void scan_shape(hipStream_t st, const DeltaArgs& p, int n_seqs, int max_len, int tokens) {
     int best = 1;
-    double t = scan_cost(p, n_seqs, NK, 4, 1, max_len, tokens);
-    auto consider = [&](int ksp) { const double c = scan_cost(p, n_seqs, NK, 4, ksp, max_len, tokens); if (c < 0.95 * t) { t = c; best = ksp; } };
+    double t = scan_cost(p, n_seqs, NK, 1, max_len, tokens);
+    auto consider = [&](int ksp) { const double c = scan_cost(p, n_seqs, NK, ksp, max_len, tokens); if (c < 0.95 * t) { t = c; best = ksp; } };
     (consider(PARTS), ...);
-    if (p.DV > 64 && scan_cost(p, n_seqs, NK, 8, 1, max_len, tokens) < t) { scan<NK, 8, 1>(st, p, n_seqs); return; }
     if (best == 1) { scan<NK, 4, 1>(st, p, n_seqs); return; }
     ((best == PARTS ? scan<NK, 4, PARTS>(st, p, n_seqs) : void()), ...);
 }

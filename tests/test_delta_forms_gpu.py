@@ -30,6 +30,25 @@ def test_scan_parts(gpu, tmp_path, heads, dim, vdim):
     m.close()
 
 
+@pytest.mark.parametrize("lens", [[40, 97], [97, 40, 40], [17, 130, 3, 97, 64], [33, 1, 160, 160, 9, 34], list(range(20, 83)) + [200], [20] * 3 + list(range(80, 19, -1)) + [100]])
+def test_scan_order(gpu, tmp_path, lens):
+    """The scan takes up to 64 sequences by their lengths (64 and 65 at the end): ties, sequences that another kernel serves, every sequence against the restatement."""
+    cfg = LM.config([LM.delta(heads=2, kv_heads=2, dim=40, vdim=72, ff=None)], width=64, vocab=60)
+    w = LM.weights(cfg, 17)
+    g = np.random.default_rng(len(lens))
+    tok = [g.integers(0, 60, n).tolist() for n in lens]
+    m = build(gpu, tmp_path, cfg, w, "f32", max_seqs=len(lens), max_batch_tokens=4096, kv_num_blocks=192)
+    ids = list(range(len(lens)))
+    for i in ids:
+        m.seq_reset(i)
+    got = np.asarray(m.forward_batch(ids, tok, [0] * len(ids), all_logits=True)[0])
+    m.close()
+    at = 0
+    for t in tok:
+        assert err(got[at:at + len(t)], O.forward(cfg, w, t), "f32") < F32_LAYER, len(t)
+        at += len(t)
+
+
 @pytest.mark.parametrize("width", [64, 1056, 2080, 4096])             # 4 / 8 / 16 chunks of a row per lane
 @pytest.mark.parametrize("lens", [[513], [519, 9]])                    # 513 and 528 rows: remainders of 8 and of 16, whole halves
 def test_sandwich_tiles(gpu, tmp_path, width, lens):
