@@ -1717,10 +1717,11 @@ void resid_gemm(nvl_model* m, const void* A, int lda, const void* W, const float
     // More rows than the ring kernel completes (256 for K >= 2048; 64 for shorter K) and up to 2048: N / 128 x M / 128 tiles of the
     // 128 x 128 kernel are a handful of workgroups (FFN-down of Llama-1B at 512 rows: 64), and the 64-row groups of the decode
     // form pull every activation row through every CU (1.3 GB of ingest for that projection: 85 us).  K split over
-    // gridDim.y workgroups per tile instead, the slices summed by the norm that follows (a row or a tile of eight a workgroup).
+    // gridDim.y workgroups per tile instead, the slices summed by the norm that follows (a row or a tile of eight a workgroup).  In models with Mamba layers
+    // too (2048 columns of 24 layers, a prompt of 300 / 600 / 750 / 1000 tokens 1726 -> 1668, 2553 -> 2289, 2731 -> 2498, 3063 -> 2875 us; from 1400 on no slices pay).
     const bool norm_ok = (M <= 512 && m->H <= 1024 * NORM_ROW_MAXCH) || (m->H % 32 == 0 && m->H <= 2048 && g_norm_t16);   // launch_norm
     if (g_sk_tile && !m->f32 && M > (g_mid && K >= 2048 ? std::max(64, std::min(g_mid_resid_rows, g_chunk_max_m)) : 64) && M <= m->sk_rows && !m->keep_hidden && m->sk_part && m->pending_slices == 0 &&
-        N % 128 == 0 && K % 64 == 0 && norm_ok && N == m->H && g_force_tile == 0 && m->n_mamba == 0) {
+        N % 128 == 0 && K % 64 == 0 && norm_ok && N == m->H && g_force_tile == 0) {
         const int tiles = cdiv(M, 128) * (N / 128);
         double best;
         slices = tile128_slices(M, N, K, SK_TILE_MAX_SLICES, best);

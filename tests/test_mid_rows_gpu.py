@@ -199,6 +199,25 @@ def test_mamba_prompts(gpu, heads, hd, groups, lens):
     assert rel_err(got["bf16"], got["f32"]) <= TOL
 
 
+@pytest.mark.parametrize("lens,all_logits", [([600], True), ([641], False), ([700, 330], False), ([1100], True)])
+def test_mamba_prompts_in_slices(gpu, lens, all_logits):
+    """Residual projections of 600 .. 1100 rows whose K is cut and summed by the norm behind them, in Mamba and attention layers, up to the final norm: against the fp32
+    mode, and a step from the state they leave."""
+    cfg = gpu.synth.tiny_config("granite_hybrid", hidden=512, num_heads=4, num_kv_heads=2, ffn_dim=2048, mamba_num_heads=16, mamba_head_dim=64, mamba_state_size=32, max_seq_len=1200)
+    w = gpu.synth.make_weights(cfg, seed=31, scale=0.03)
+    r = np.random.default_rng(sum(lens))
+    prompts, ids, got = [r.integers(0, cfg["vocab_size"], n).tolist() for n in lens], list(range(len(lens))), {}
+    for precision in ("bf16", "f32"):
+        m = gpu.HipTransformerModel(cfg, w, precision=precision, max_seqs=len(lens), max_batch_tokens=1200)
+        for i in ids:
+            m.seq_reset(i)
+        z = m.forward_batch(ids, prompts, [0] * len(ids), all_logits=all_logits)[0]
+        got[precision] = [z, m.forward_batch(ids, [[7]] * len(ids), lens)[0]]
+        m.close()
+    for a, b in zip(got["bf16"], got["f32"]):
+        assert rel_err(a, b) <= TOL
+
+
 @pytest.mark.parametrize("n", [65, 513, 530, 1040])
 def test_moe_prompt_forms(gpu, n):
     """Routing in the router's launch, expert-ordered rows copied from the norm's row-major result (beyond 512 tokens): against the separate
