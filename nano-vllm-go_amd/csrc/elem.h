@@ -388,7 +388,7 @@ struct SandwichArgs {
     const float* y2;          // a second source, added as it is: [slices2][.][H], or with slot_of the rows slot_of[r * slices2 + k], weighted by gate_w
     int slices2; int64_t stride2;
     const int32_t* slot_of; const float* gate_w;
-    bf16_t* xn_rows;          // tile kernel: not NULL: xn a second time, row-major
+    bf16_t* xn_rows;          // bf16: not NULL: xn a second time, row-major
 };
 // four columns of everything that joins row r (EXT)
 __device__ __forceinline__ f32x4 sandwich_more(const SandwichArgs& p, int r, int col) {
@@ -426,6 +426,15 @@ __global__ __launch_bounds__(256) void sandwich_row_kernel(SandwichArgs p, ActT*
     const int src = p.rows_idx ? p.rows_idx[r] : r;
     float* xr = p.x + (int64_t)src * p.H;
     f32x4 x[MAXCH], y[MAXCH];
+    auto put = [&](int j, f32x4 v) {
+        act_store4<ActT>(xn, r, j * 4, p.H, v);
+        if constexpr (sizeof(ActT) == 2) if (p.xn_rows) {
+            bf16x4 o;
+#pragma unroll
+            for (int i = 0; i < 4; i++) o[i] = (bf16_t)v[i];
+            *(bf16x4*)(p.xn_rows + (int64_t)r * p.H + j * 4) = o;
+        }
+    };
     float ss = 0.f;
 #pragma unroll
     for (int c = 0; c < MAXCH; c++) {
@@ -498,7 +507,7 @@ __global__ __launch_bounds__(256) void sandwich_row_kernel(SandwichArgs p, ActT*
             }
         } else if (p.raw_next)
 #pragma unroll
-            for (int c = 0; c < MAXCH; c++) { const int j = threadIdx.x + c * 256; if (j < H4) act_store4<ActT>(xn, r, j * 4, p.H, x[c]); }
+            for (int c = 0; c < MAXCH; c++) { const int j = threadIdx.x + c * 256; if (j < H4) put(j, x[c]); }
         return;
     }
     if constexpr (EXT) if (p.b_next) {
@@ -515,7 +524,7 @@ __global__ __launch_bounds__(256) void sandwich_row_kernel(SandwichArgs p, ActT*
                 f32x4 o;
 #pragma unroll
                 for (int k = 0; k < 4; k++) o[k] = ((x[c][k] - mean) / sd) * w[k] + b[k];
-                act_store4<ActT>(xn, r, j * 4, p.H, o);
+                put(j, o);
             }
         }
         return;
@@ -532,7 +541,7 @@ __global__ __launch_bounds__(256) void sandwich_row_kernel(SandwichArgs p, ActT*
             f32x4 o;
 #pragma unroll
             for (int k = 0; k < 4; k++) o[k] = (x[c][k] / rms) * w[k];
-            act_store4<ActT>(xn, r, j * 4, p.H, o);
+            put(j, o);
         }
     }
 }

@@ -895,7 +895,11 @@ struct ExpertOut { const float* y = nullptr; int slices = 0; int64_t stride = 0;
 struct ShiftOut { const float* mu = nullptr; float* state = nullptr; const Meta* md = nullptr; };
 
 // does it leave a row-major copy of xn (xn_rows) too?
-bool sandwich_copies_rows(const nvl_model* m, SubOut y, int rows) { return !m->f32 && rows > 512 && m->H <= 4096 && y.slices <= 1; }
+bool sandwich_copies_rows(const nvl_model* m, int rows) { return !m->f32 && rows > 512 && m->H <= 4096; }
+// a workgroup per row up to here, tiles of eight rows above: fewer tiles than CUs wait for one another's loads.  Up to here K slices of the projection in front too.
+// us a prompt of 2048 columns, tiles and whole K from 513 rows on -> here: 18 layers with experts 513 / 750 / 1000 rows 3505 -> 3174, 3813 -> 3517, 4060 -> 3847; delta rule
+// and latent attention 513 / 750 / 1000 2786 -> 2596, 3217 -> 3070, 3512 -> 3479
+constexpr int SANDWICH_ROW_KERNEL_ROWS = 1024;
 // x += rms(y) * w_post (w_post NULL: x += y + experts; NVL_BLOCK_SUM_NORM: x = rms(stream_scale x + y + experts) * w_post) and / or
 // xn = next(x) (elem.h SandwichArgs)
 void sandwich(nvl_model* m, SubOut y, const float* w_post, NextNorm next, void* xn, int rows, const int32_t* rows_idx = nullptr, ExpertOut ex = {}, ShiftOut sh = {}, bf16_t* xn_rows = nullptr) {
@@ -908,7 +912,7 @@ void sandwich(nvl_model* m, SubOut y, const float* w_post, NextNorm next, void* 
     if (sh.mu) { a.shift = sh.mu; a.before = sh.state; a.before_stride = m->rec_slot_stride; a.seq_slot = sh.md->seq_slot; a.seq_pos = sh.md->seq_pos; }
     const bool ext = (y.y && !w_post) || next.b || a.sum_scale != 0.f || sh.mu;
     a.xn_rows = xn_rows;
-    if (sandwich_copies_rows(m, y, rows) && !sh.mu) {
+    if (!m->f32 && rows > SANDWICH_ROW_KERNEL_ROWS && m->H <= 4096 && y.slices <= 1 && !sh.mu) {
         const size_t lds = (size_t)NORM_TILE_ROWS * tile16_pitch(m->H) * 2;
 #define NVL_SWTE(CH, EXT)                                                                                                  \
         do {                                                                                                                \
@@ -939,7 +943,7 @@ SubOut sub_out(nvl_model* m, int site, const void* A, const void* W, int M, int 
     if (!m->f32 && M <= 64) {
         const int nblocks = N / 16;
         while (slices < m->sk_max_slices && nblocks * slices < 256 && (K >> 5) / (slices * 2) >= 8) slices *= 2;
-    } else if (!m->f32 && M <= 512 && M <= m->sk_rows && N % 128 == 0 && g_force_tile == 0) {
+    } else if (!m->f32 && M <= SANDWICH_ROW_KERNEL_ROWS && M <= m->sk_rows && N % 128 == 0 && g_force_tile == 0) {
         const int tiles = cdiv(M, 128) * (N / 128);
         double cost;
         slices = tile128_slices(M, N, K, SK_TILE_MAX_SLICES, cost);
@@ -1619,7 +1623,7 @@ bool layered_stack(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len,
         if (sum || shift) {
             const bool apart = shift && !ones && li + 1 < m->L, ff = r.c.ffn_dim || r.c.experts;      // apart: the next mixer's input comes from shift_rows
             const NextNorm own{nullptr, nullptr, true}, close = apart ? NextNorm{nullptr, nullptr, false} : after;
-            bf16_t* xn_rows = r.c.experts && sandwich_copies_rows(m, y, M) ? (bf16_t*)m->moe_eo : nullptr;      // (for the copy into expert order)
+            bf16_t* xn_rows = r.c.experts && sandwich_copies_rows(m, M) ? (bf16_t*)m->moe_eo : nullptr;      // (for the copy into expert order)
             sandwich(m, y, w.norm1b, ff ? own : close, m->xn, M, nullptr, {}, ff ? ShiftOut{} : shift_out(li + 1), xn_rows);
             if (ff) {
                 ExpertOut ex;

@@ -1,0 +1,32 @@
+"""Sandwich norms of 513 .. 1024 rows, a workgroup per row with a row-major copy for experts and K slices to add up, and of more rows, tiles of eight."""
+import numpy as np
+import pytest
+
+import medulorn_models as MM
+from layered_helpers import build, err
+
+pytestmark = pytest.mark.gpu
+BF16_LAYER = 0.03       # a single bf16 layer, as in the other tests of these models
+
+
+def against_fp32(gpu, tmp_path, cfg, w, tok):
+    got = {}
+    for precision in ("bf16", "f32"):
+        m = build(gpu, tmp_path, cfg, w, precision, max_seqs=2, max_seq_len=1088, max_batch_tokens=1088)
+        m.seq_reset(0)
+        got[precision] = np.asarray(m.forward_batch([0], [tok], [0], all_logits=True)[0])
+        m.close()
+    assert err(got["bf16"], got["f32"], "bf16") < BF16_LAYER
+
+
+@pytest.mark.parametrize("n", [513, 1024, 1025, 1031])
+@pytest.mark.parametrize("layer,width", [(MM.attention(mlp=MM.moe()), 96), (MM.attention(mlp=MM.moe()), 1056), (MM.parallel(mlp=MM.dense(48)), 96),
+                                         (MM.attention(heads=16, kv_heads=4, dim=64, vdim=64, turn=MM.rot(64), mlp=MM.dense(2048)), 1024)],      # 64 and more slices of both residual projections
+                         ids=["experts-96", "experts-1056", "parallel", "slices"])
+def test_rows_and_tiles(gpu, tmp_path, layer, width, n):
+    cfg = MM.config([layer], width=width, vocab=130)
+    w = MM.weights(cfg, 11)
+    tok = np.random.default_rng(n).integers(0, 130, n).tolist()
+    if "experts" in str(layer):
+        tok = MM.clear_tokens(cfg, w, n, 1)[0]          # (no near tie between experts)
+    against_fp32(gpu, tmp_path, cfg, w, list(tok))
