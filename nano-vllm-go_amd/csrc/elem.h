@@ -263,12 +263,22 @@ __global__ __launch_bounds__(64 * NORM_TILE_ROWS) void norm_tile_kernel(float* _
     store_norm_tile(tile, y, rows, H, lane, wave);
 }
 
+__device__ __forceinline__ void store_row4(bf16_t* p, f32x4 v) {
+    bf16x4 o;
+#pragma unroll
+    for (int i = 0; i < 4; i++) o[i] = (bf16_t)v[i];
+    *(bf16x4*)p = o;
+}
 // the arithmetic of one row once it sits in registers (shared by norm_row_kernel and decode_seam_kernel)
 template <typename ActT>
 __device__ __forceinline__ void norm_row_finish(f32x4 (&v)[NORM_ROW_MAXCH], f32x4 (&ww)[NORM_ROW_MAXCH],
                                                 f32x4 (&bb)[NORM_ROW_MAXCH], const float* b, float eps, ActT* y, int r,
-                                                int H, float* red, int width = 0, float* mean_out = nullptr) {     // width: columns of the mean when the row is padded (0: H)
+                                                int H, float* red, int width = 0, float* mean_out = nullptr, bf16_t* y_rows = nullptr) {     // width: columns of the mean when the row is padded (0: H)
     const int H4 = H >> 2;
+    auto put = [&](int j, f32x4 o) {
+        act_store4<ActT>(y, r, j * 4, H, o);
+        if constexpr (sizeof(ActT) == 2) if (y_rows) store_row4(y_rows + (int64_t)r * H + j * 4, o);
+    };
     if (b == nullptr) {
         float ss = 0.f;
 #pragma unroll
@@ -281,7 +291,7 @@ __device__ __forceinline__ void norm_row_finish(f32x4 (&v)[NORM_ROW_MAXCH], f32x
                 f32x4 o;
 #pragma unroll
                 for (int k = 0; k < 4; k++) o[k] = (v[c][k] / rms) * ww[c][k];
-                act_store4<ActT>(y, r, j * 4, H, o);
+                put(j, o);
             }
         }
     } else {
@@ -308,7 +318,7 @@ __device__ __forceinline__ void norm_row_finish(f32x4 (&v)[NORM_ROW_MAXCH], f32x
                 f32x4 o;
 #pragma unroll
                 for (int k = 0; k < 4; k++) o[k] = ((v[c][k] - mean) / sd) * ww[c][k] + bb[c][k];
-                act_store4<ActT>(y, r, j * 4, H, o);
+                put(j, o);
             }
         }
     }
@@ -321,7 +331,7 @@ __global__ __launch_bounds__(256) void norm_row_kernel(float* __restrict__ x,
                                                        const int32_t* __restrict__ rows_idx,
                                                        const float* __restrict__ w,
                                                        const float* __restrict__ b, float eps,
-                                                       ActT* __restrict__ y, int H, PendingResid pr, float* mean_out) {      // mean_out: [rows] or NULL (layer norm)
+                                                       ActT* __restrict__ y, int H, PendingResid pr, float* mean_out, bf16_t* y_rows) {      // mean_out: [rows] or NULL (layer norm); y_rows: not NULL: y a second time, row-major
     __shared__ float red[4];
     const int r = blockIdx.x;
     const int src = rows_idx ? rows_idx[r] : r;
@@ -358,7 +368,7 @@ __global__ __launch_bounds__(256) void norm_row_kernel(float* __restrict__ x,
             if (b) bb[c] = *(const f32x4*)(b + j * 4);
         }
     }
-    norm_row_finish<ActT>(v, ww, bb, b, eps, y, r, H, red, 0, mean_out);
+    norm_row_finish<ActT>(v, ww, bb, b, eps, y, r, H, red, 0, mean_out, y_rows);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -428,12 +438,7 @@ __global__ __launch_bounds__(256) void sandwich_row_kernel(SandwichArgs p, ActT*
     f32x4 x[MAXCH], y[MAXCH];
     auto put = [&](int j, f32x4 v) {
         act_store4<ActT>(xn, r, j * 4, p.H, v);
-        if constexpr (sizeof(ActT) == 2) if (p.xn_rows) {
-            bf16x4 o;
-#pragma unroll
-            for (int i = 0; i < 4; i++) o[i] = (bf16_t)v[i];
-            *(bf16x4*)(p.xn_rows + (int64_t)r * p.H + j * 4) = o;
-        }
+        if constexpr (sizeof(ActT) == 2) if (p.xn_rows) store_row4(p.xn_rows + (int64_t)r * p.H + j * 4, v);
     };
     float ss = 0.f;
 #pragma unroll

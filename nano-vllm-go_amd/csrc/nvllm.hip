@@ -1315,7 +1315,8 @@ static int g_norm_t16 = 1;     // nvl_set_tuning key 9: norm_tile_kernel for pre
 //   2048 columns with slices to add: 520 11.0 / 23.7, 700 12.4 / 23.5, 1000 13.4 / 20.0, 1500 19.8 / 21.4, 2000 18.5 / 19.0
 //   768: 520 6.8 / 8.9, 1000 7.9 / 9.3, 1500 9.9 / 9.5, 2000 10.9 / 9.6        4096: 1000 15.3 / 17.0, 2000 20.1 / 17.3
 //   4544: 520 11.3 / 15.7, 1000 14.9 / 17.0, 1500 20.0 / 18.5
-// (a row-major copy is the tiles' alone: with one, and where there are no tiles, the line is 512 rows)
+//   with a row-major copy for experts, a prompt of 24 layers of 1024 columns: 513 / 600 / 800 / 1024 tokens 2739 -> 2651, 2834 -> 2760, 3055 -> 2982, 3195 -> 3138
+// (where there are no tiles, the line is 512 rows)
 constexpr int NORM_ROW_KERNEL_ROWS = 1024;
 template <typename ActT>
 void launch_norm(nvl_model* m, float* x, const int32_t* rows_idx, const float* w, const float* b,
@@ -1331,9 +1332,9 @@ void launch_norm(nvl_model* m, float* x, const int32_t* rows_idx, const float* w
         if (!row_kernel && !tile_kernel) throw std::runtime_error("norm: no kernel for this pending residual");
     }
     const bool tiles = sizeof(ActT) == 2 && m->H % 32 == 0 && m->H <= 4608 && g_norm_t16 && (!pr.part || m->H <= 2048);
-    if (pr.slot_of || (rows <= (tiles && !y_rows ? NORM_ROW_KERNEL_ROWS : 512) && m->H <= 1024 * NORM_ROW_MAXCH)) {
-        if (pr.slot_of) hipLaunchKernelGGL((norm_row_kernel<ActT, true>), dim3(rows), dim3(256), 0, m->stream, x, rows_idx, w, b, m->cfg.norm_eps, (ActT*)y, m->H, pr, mean_out);
-        else hipLaunchKernelGGL((norm_row_kernel<ActT>), dim3(rows), dim3(256), 0, m->stream, x, rows_idx, w, b, m->cfg.norm_eps, (ActT*)y, m->H, pr, mean_out);
+    if (pr.slot_of || (rows <= (tiles ? NORM_ROW_KERNEL_ROWS : 512) && m->H <= 1024 * NORM_ROW_MAXCH)) {
+        if (pr.slot_of) hipLaunchKernelGGL((norm_row_kernel<ActT, true>), dim3(rows), dim3(256), 0, m->stream, x, rows_idx, w, b, m->cfg.norm_eps, (ActT*)y, m->H, pr, mean_out, y_rows);
+        else hipLaunchKernelGGL((norm_row_kernel<ActT>), dim3(rows), dim3(256), 0, m->stream, x, rows_idx, w, b, m->cfg.norm_eps, (ActT*)y, m->H, pr, mean_out, y_rows);
     }
     else if (tiles) {   // (two workgroups' tiles of wider rows would not fit the LDS of a CU: norm_kernel)
         // 8 rows x H bf16 of LDS (up to 73 KiB); the row sits in registers: instance by chunks per lane
