@@ -544,7 +544,7 @@ int nvl_op_sample(int device, const float* logits, int rows, int V, const nvl_sa
 int nvl_bench_gemm(int device, int M, int N, int K, int epi, int force_bnt, int force_ksplit, int iters,
                    float* avg_us);
 /* Process-wide tuning override used by tests and sweeps.  key 0: prefill GEMM kernel (0 automatic,
- * 1 = 128x128, a ring of K tiles, 2 = 256x128 three-stage, 3 = 256x256 two-stage, 5 = 256x256 ping-pong).
+ * 1 = 128x128, a ring of K tiles, 2 = 256x128 on the ring, 3 = 256x256 two-stage, 5 = 256x256 ping-pong).
  * key 1: K slices of the decode residual projections (0 automatic, 1 never split, 2, 4).
  * key 2: decode (M <= 64) GEMM form: 0 automatic, 1/2/4 = narrow form with that many weight tiles per workgroup,
  * 8 = wide-N form (4 weight tiles per wave).
@@ -587,6 +587,8 @@ int nvl_bench_gemm(int device, int M, int N, int K, int epi, int force_bnt, int 
  * key 41: parts of K for the 256x256 tiles of the last, partly filled round (0, default: from the grid; 1 never; up to 512 rows only with key 11 above them).
  * key 42: lists of layers, decode: the grouped attention launch norms and rotates queries and keys and carries a second mixer's gated
  * norm (1, default; 0 = launches of their own).
+ * key 43: decode attention takes ragged contexts from the longest down (0 never, 1 (default) where the contexts differ enough, 2 always).
+ * key 44: lists of layers, decode: a second mixer's recurrence in the attention launch (0 never, 1 (default) up to 64 sequences, 2 wherever it fits).
  * key 33: MoE decode: the experts' down projection completes the residual and carries the next RMSNorm (1, default; 0: K slices that a
  * norm launch before the next QKV sums).
  * The settings are PROCESS-GLOBAL and unsynchronised (every model in the process sees them): set them from one thread
