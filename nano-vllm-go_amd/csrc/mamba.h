@@ -560,8 +560,9 @@ __global__ __launch_bounds__(256) void mamba_gate_norm_kernel(MambaArgs p, ActT*
 
 // Prefill-sized bf16 batches, EH <= 4096: a wave holds a row in registers (y is read once and not written back), eight rows a workgroup, so
 // that the operand leaves in whole 128-byte lines (row by row each lane's 8 bytes were a line of their own: 2326 x 4096 48 us, 34
-// here).  Below some 128 rows too few workgroups.
-constexpr int MAMBA_GATE_TILE_ROWS = 128;
+// here).  Below 512 rows too few workgroups: a prompt of 24 layers of 4096 columns, here -> row by row, 130 / 200 / 300 / 400 tokens 1343 -> 1310, 1433 -> 1401, 1681 -> 1658, 1885 -> 1872 us;
+// 600 as long either way, 1000 / 1900 2952 -> 2982, 4754 -> 4863.
+constexpr int MAMBA_GATE_TILE_ROWS = 512;
 static inline constexpr int mamba_gate_tile_lds_bytes(int EH) { return 8 * (EH + 8) * 2; }
 static __global__ __launch_bounds__(512) void mamba_gate_norm_tile_kernel(MambaArgs p, bf16_t* __restrict__ out, int tokens) {
     constexpr int CH = 16;

@@ -199,6 +199,24 @@ def test_mamba_prompts(gpu, heads, hd, groups, lens):
     assert rel_err(got["bf16"], got["f32"]) <= TOL
 
 
+@pytest.mark.parametrize("heads,hd,groups", [(16, 64, 2), (8, 32, 1), (10, 64, 1)])
+@pytest.mark.parametrize("lens", [[511], [512], [300, 217]])
+def test_mamba_gate_rows_and_tiles(gpu, heads, hd, groups, lens):
+    """The gated norm row by row up to 511 rows and in tiles of eight from 512 on: every row of the bf16 mode against the fp32 mode."""
+    cfg = gpu.synth.tiny_config("granite_hybrid", hidden=heads * hd // 2, num_heads=heads * hd // 128, num_kv_heads=1, mamba_num_heads=heads, mamba_head_dim=hd, mamba_state_size=32,
+                                mamba_n_groups=groups, max_seq_len=520)
+    w = gpu.synth.make_weights(cfg, seed=37, scale=0.05)
+    r = np.random.default_rng(sum(lens))
+    prompts, ids, got = [r.integers(0, cfg["vocab_size"], n).tolist() for n in lens], list(range(len(lens))), {}
+    for precision in ("bf16", "f32"):
+        m = gpu.HipTransformerModel(cfg, w, precision=precision, max_seqs=len(lens), max_batch_tokens=520)
+        for i in ids:
+            m.seq_reset(i)
+        got[precision] = m.forward_batch(ids, prompts, [0] * len(ids), all_logits=True)[0]
+        m.close()
+    assert rel_err(got["bf16"], got["f32"]) <= TOL
+
+
 @pytest.mark.parametrize("lens,all_logits", [([600], True), ([641], False), ([700, 330], False), ([1100], True)])
 def test_mamba_prompts_in_slices(gpu, lens, all_logits):
     """Residual projections of 600 .. 1100 rows whose K is cut and summed by the norm behind them, in Mamba and attention layers, up to the final norm: against the fp32
