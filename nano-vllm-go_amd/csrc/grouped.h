@@ -934,6 +934,8 @@ __global__ __launch_bounds__(256) void grouped_plain_kernel(GroupedArgs p) {
 void grouped_prefill_launch(hipStream_t st, const GroupedArgs& p, dim3 grid, size_t lds, bool fast);
 void grouped_short_launch(hipStream_t st, const GroupedArgs& p, dim3 grid);
 void grouped_qk_launch(hipStream_t st, const GroupedArgs& p, bool f32);
-constexpr int GROUPED_QK_ROW_MAX = 512;           // bf16: larger batches are worked in tiles of 16 tokens
+// bf16: larger batches are worked in tiles of 16 tokens, too few workgroups below (18 layers of 32 heads, a prompt of 513 / 600 / 750 tokens in tiles -> head by head 3197 -> 3163,
+// 3302 -> 3266, 3546 -> 3526 us; 1000 / 1600 3881 -> 3891, 5314 -> 5392)
+constexpr int GROUPED_QK_ROW_MAX = 768;
 
 }  // namespace nvl
