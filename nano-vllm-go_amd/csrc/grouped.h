@@ -930,6 +930,34 @@ __global__ __launch_bounds__(256) void grouped_plain_kernel(GroupedArgs p) {
     }
 }
 
+// ---- host rules: a layer's form (padded widths of its keys and values) and what its launches need ----
+static inline bool grouped_fits(int dp, int vp) { return dp <= 256 && vp <= 256; }      // (wider heads: grouped_plain_kernel)
+// May a decode launch of the short kernel take a second mixer's recurrence (state DK x DVp)?  Workgroups of 512 threads, the state rows of a thread, its LDS.
+static inline bool grouped_takes_recurrence(int dp, int vp, int DK, int DVp) {
+    int tv = 1;
+    while (tv < DVp / 4) tv <<= 1;
+    return dp <= 128 && vp <= 128 && cdiv(DK, LR_STEP_THREADS / tv) <= GROUPED_LIN_ROWS && linrec_step_lds_bytes(DK, DVp) <= 8 * (vp >> 4) * 1024;
+}
+constexpr int GROUPED_SPLIT_WGS = 512;      // workgroups of a launch whose keys are split, at most
+// What the bf16 layers of a model share.  Each layer counts by itself: one that the short kernel does not serve neither needs a buffer nor keeps the others from theirs.
+struct GroupedBuffers {
+    int vp = 0;                  // widest padded values of the layers whose keys may be split: records of vp * 16 + 32 floats; 0: none
+    bool tickets = false;        // a second mixer's recurrence may ride
+    void layer(int dp, int vpad, bool second) {
+        if (!grouped_fits(dp, vpad)) return;
+        vp = std::max(vp, vpad);
+        tickets = tickets || second;
+    }
+    int cap() const { return vp ? GROUPED_SPLIT_WGS : 0; }
+};
+// Key splits of a launch of `wgs` workgroups of NW waves: once a wave would walk more than two tiles, while the parts find room on the chip and in the buffers.  force: that many, where there is room.
+static inline int grouped_key_splits(int64_t wgs, int64_t cap, int key_tiles, int nw, int force) {
+    if (force) return (int)std::min<int64_t>(force, std::max<int64_t>(1, cap / wgs));
+    int z = 1;
+    while (z < GROUPED_SPLITS && wgs * z * 2 <= std::min<int64_t>(256, cap) && z * 2 * 2 * nw <= key_tiles) z *= 2;
+    return z;
+}
+
 // launches (grouped_inst.hip): the instance follows from p.dp and p.vp
 void grouped_prefill_launch(hipStream_t st, const GroupedArgs& p, dim3 grid, size_t lds, bool fast);
 void grouped_short_launch(hipStream_t st, const GroupedArgs& p, dim3 grid);

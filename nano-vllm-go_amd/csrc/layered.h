@@ -31,7 +31,7 @@ namespace {
 constexpr int LAT_ABSORB_MAX = 16, LAT_ABSORB_MAX_RP = 512, REC_STEP_MAX = 4;
 constexpr int GLU_IN_MAX = 1024;       // widest shared expert whose gate and up columns pass through fp32 rows instead of a launch of their own
 constexpr int SHARED_PARTS_MAX = 16;   // widest shared expert, in experts, that joins the masked experts of a decode step
-constexpr int GROUPED_SHORT_ROWS = 64, GROUPED_SPLIT_WGS = 512;      // GROUPED_SPLIT_WGS: workgroups of a launch whose keys are split
+constexpr int GROUPED_SHORT_ROWS = 64;
 
 bool same_rotation(const nvl_layer_config& a, const nvl_layer_config& b) {
     return a.rot_dim == b.rot_dim && a.rot_base == b.rot_base && a.rot_factor == b.rot_factor && a.rot_original == b.rot_original &&
@@ -497,7 +497,8 @@ void layered_finalize(nvl_model* m) {
     m->g[NVL_T_POS_EMB].p = pos;
 
     int64_t ld_in = 0, q_cols = 0, cq_cols = 0, ko = 0, conv = 0, ocols = 0, Fmax = 0, abs_cols = 0, z_cols = 0, g_cols = 0, pa_cols = 0, pg_cols = 0;
-    int64_t moe_k = 0, moe_e = 0, moe_kI = 0, moe_ep = 0, moe_all = 0, moe_sl = 0, grp_vp = 0, qg_cols = 0;
+    int64_t moe_k = 0, moe_e = 0, moe_kI = 0, moe_ep = 0, moe_all = 0, moe_sl = 0, qg_cols = 0;
+    GroupedBuffers grp;
     for (int i = 0; i < m->L; i++) {
         LayerRun& r = m->runs[(size_t)i];
         const nvl_layer_config& c = r.c;
@@ -731,7 +732,7 @@ void layered_finalize(nvl_model* m) {
             cq_cols = std::max<int64_t>(cq_cols, r.qrp);
             if (lat_absorb_ok(m, r)) abs_cols = std::max(abs_cols, round_up(c.heads, 16) * (r.rp + r.rotp));
         } else if (c.mixer == NVL_MIXER_ATTENTION) {
-            grp_vp = std::max<int64_t>(grp_vp, r.vp);
+            if (!m->f32) grp.layer(r.dp, r.vp, c.mixer2 != 0);
             if (c.mixer2) ocols = std::max<int64_t>(ocols, (int64_t)c.heads2 * c.vdim2);
         } else {
             ocols = std::max<int64_t>(ocols, (int64_t)c.heads * c.vdim);
@@ -769,12 +770,12 @@ void layered_finalize(nvl_model* m) {
     if (sd) m->lside = lay_alloc(m, Mp * m->side_kp * ws);
     if (qg_cols) m->lqg = lay_alloc(m, Mp * qg_cols * ws);
     if (m->lvf_ld) m->lvf = (float*)lay_alloc(m, Mmax * m->lvf_ld * 4);
-    if (grp_vp && !m->f32 && grp_vp <= 256) {
-        m->grp_cap = GROUPED_SPLIT_WGS;
-        m->grp_part = (float*)lay_alloc(m, m->grp_cap * (grp_vp * 16 + 32) * 4);
+    if (grp.vp) {
+        m->grp_cap = grp.cap();
+        m->grp_part = (float*)lay_alloc(m, m->grp_cap * (grp.vp * 16 + 32) * 4);
         m->grp_cnt = (int32_t*)lay_alloc(m, m->grp_cap * 4);
-        m->lin_cnt = (int32_t*)lay_alloc(m, (int64_t)m->opts.max_seqs * 4);
     }
+    if (grp.tickets) m->lin_cnt = (int32_t*)lay_alloc(m, (int64_t)m->opts.max_seqs * 4);
     m->lproj = f32buf(Mmax * ld_in);
     m->ly = f32buf(Mmax * H);
     if (q_cols) { m->lq = f32buf(Mmax * q_cols); m->lcq = lay_alloc(m, Mp * cq_cols * ws); }
@@ -1289,10 +1290,7 @@ static int g_lin_rides = 1;          // nvl_set_tuning key 44: decode: a second 
 // Does the attention launch of a decode pass (workgroups of 512 threads) take the recurrence too?  It runs beside the attention and its launch (6.9 us of
 // a step of 6 sequences, 16 heads of 128 x 128) is gone: a 2048-wide model, requests of 24 steps of 1 / 6 / 16 / 32 / 64 / 128 sequences -3.6, -2.8, -0.6, -0.5, -1.7, +0.1 %.
 bool lightning_rides(const LayerRun& r, const LinRecArgs& a, int n_seqs) {
-    int tv = 1;
-    while (tv < a.DVp / 4) tv <<= 1;
-    if (!g_lin_rides || (g_lin_rides == 1 && n_seqs > 64) || r.vp > 128 || r.dp > 128 || cdiv(a.DK, LR_STEP_THREADS / tv) > GROUPED_LIN_ROWS || linrec_step_lds_bytes(a.DK, a.DVp) > 8 * (r.vp >> 4) * 1024) return false;
-    return true;
+    return g_lin_rides && (g_lin_rides != 1 || n_seqs <= 64) && grouped_takes_recurrence(r.dp, r.vp, a.DK, a.DVp);
 }
 void mix_lightning(nvl_model* m, const LayerRun& r, const MixerW& w, const Meta& md, int n_seqs, int M, int max_len, GroupedArgs* carry) {
     const nvl_layer_config& c = r.c;
@@ -1340,7 +1338,7 @@ void mix_grouped(nvl_model* m, const LayerRun& r, const MixerW& w, const Meta& m
         m->site = KS_MIX_IN;
         gemm(m, r.raw ? EPI_GROUPED_RAW : EPI_GROUPED, false, g);
     }
-    const bool plain = m->f32 || r.dp > 256 || r.vp > 256;
+    const bool plain = m->f32 || !grouped_fits(r.dp, r.vp);
     a.short_rows = GROUPED_SHORT_ROWS;
     // one token per sequence: the attention launch norms and rotates them itself, and carries the second mixer's gated norm
     const bool in_attn = g_grouped_qk && r.raw && !plain && max_len == 1 && M == n_seqs && a.group <= a.short_rows && c.ungated && c.dim == r.dp && (r.dp == 64 || r.dp == 128) &&
@@ -1396,9 +1394,7 @@ void mix_grouped(nvl_model* m, const LayerRun& r, const MixerW& w, const Meta& m
         // sequence of 2048 tokens with a window of 1024: 13.1 us unsplit, 13.7 in four; without a window, 3900 tokens: 27.8 -> 16.6 us)
         // (a window or chunk holds no more: requests of 6 x 1100 keys with windows and chunks of 512, in two 13.9 and 12.1 us, whole 13.4 and 11.6)
         const int key_tiles = std::min(1 << layered_kt_log2(m), span > 0 ? span / 64 + 2 + cdiv(a.mask.keep, 64) : 1 << 30), nw = dt <= 8 ? 8 : 4;
-        int z = 1;
-        while (z < GROUPED_SPLITS && wgs * n_seqs * z * 2 <= 256 && z * 2 * 2 * nw <= key_tiles) z *= 2;
-        if (g_grouped_split) z = (int)std::min<int64_t>(g_grouped_split, std::max<int64_t>(1, m->grp_cap / (wgs * n_seqs)));
+        const int z = grouped_key_splits(wgs * n_seqs, m->grp_cap, key_tiles, nw, g_grouped_split);
         a.part = m->grp_part; a.part_cnt = m->grp_cnt;
         a.row_wgs = (int)wgs;
         const dim3 grid((unsigned)wgs, n_seqs, z);

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 import medulorn_models as MM
-from layered_helpers import build
+from layered_helpers import build, err
 
 pytestmark = pytest.mark.gpu
 rot = MM.rot
@@ -41,3 +41,27 @@ def test_same_bits(gpu, tmp_path, name, n, split):
             lib.nvl_set_tuning(key, v)
     m.close()
     assert np.isfinite(got[0]).all() and np.array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("wide", [dict(dim=64, vdim=272, turn=rot(64)), dict(dim=320, vdim=64, turn=rot(64))], ids=["values-272", "keys-320"])
+@pytest.mark.parametrize("at", [0, 1])                      # the wide layer in front and behind
+def test_beside_a_wider_layer(gpu, tmp_path, wide, at):
+    """Another layer's heads fit no instance: this one's recurrence rides all the same (tickets of its own), and the keys of a long context are split (2100 keys: two
+    parts).  Steps against the fp32 mode, and the same bits as the launches of their own."""
+    layers = [MM.parallel(**LAYERS["128x128"] | dict(window=None))]
+    layers.insert(at, MM.attention(heads=2, kv_heads=1, chunk=None, **wide))
+    cfg = MM.config(layers, width=128, vocab=90)
+    w = MM.weights(cfg, 4)
+    r, got = np.random.default_rng(at), {}
+    prompts = [r.integers(0, 90, k).tolist() for k in (2100, 40)]
+    for mode, rides in (("f32", 1), ("bf16", 1), ("bf16", 0)):
+        old = gpu.lib().nvl_set_tuning(44, rides)
+        m = build(gpu, tmp_path, cfg, w, mode, max_seqs=2, max_seq_len=2112, max_batch_tokens=2144, kv_num_blocks=72)
+        for i in (0, 1):
+            m.seq_open(i)
+        m.forward_batch([0, 1], prompts, [0, 0], want_logits=False)
+        got[mode, rides] = np.stack([m.forward_batch([0, 1], [[7 + j], [3 + j]], [2100 + j, 40 + j])[0] for j in range(4)])
+        m.close()
+        gpu.lib().nvl_set_tuning(44, old)
+    assert np.array_equal(got["bf16", 1], got["bf16", 0])
+    assert err(got["bf16", 1], got["f32", 1]) < 0.06            # two bf16 layers, the worst row (0.03 a layer in the other tests of these models)

@@ -51,3 +51,40 @@ int main() {
     return 0;
 }
 """)
+
+
+@pytest.mark.skipif(HIPCC is None, reason="no hipcc")
+def test_every_attention_layer_finds_its_buffers(tmp_path):
+    """Layers of different widths in one model: those whose heads fit the short kernel have partial records, and tickets for a second mixer's recurrence that rides,
+    whatever the others take; a launch whose keys are split stays inside the records."""
+    run(tmp_path, r"""
+#include "grouped.h"
+using namespace nvl;
+struct Layer { int dp, vp; bool second; };
+int main() {
+    const int widths[] = {32, 64, 128, 256, 320, 2048};
+    std::vector<Layer> all;
+    for (int dp : widths) for (int vp : widths) for (bool second : {false, true}) all.push_back({dp, vp, second});
+    for (const Layer& a : all)
+        for (const Layer& b : all) {
+            GroupedBuffers g;
+            for (const Layer& l : {a, b}) g.layer(l.dp, l.vp, l.second);
+            for (const Layer& l : {a, b}) {
+                const bool served = l.dp <= 256 && l.vp <= 256;
+                if (served != grouped_fits(l.dp, l.vp)) { printf("form of %d x %d\n", l.dp, l.vp); return 1; }
+                if (!served) continue;
+                const char* bad = g.vp < l.vp || g.cap() <= 0 ? "no room for its records" : nullptr;
+                for (int dk : {16, 128, 256}) for (int dv : {16, 128}) if (l.second && grouped_takes_recurrence(l.dp, l.vp, dk, dv) && !g.tickets) bad = "no tickets";
+                for (int wgs = 1; wgs <= 1024; wgs++)
+                    for (int tiles = 1; tiles <= 1024; tiles *= 2)
+                        for (int force : {0, 3, 16}) {
+                            const int z = grouped_key_splits(wgs, g.cap(), tiles, 8, force);
+                            if (z < 1 || z > GROUPED_SPLITS || (z > 1 && (int64_t)wgs * z > g.cap())) bad = "parts past the records";
+                            if (z > 1 && grouped_key_splits(wgs, 0, tiles, 8, force) != 1) bad = "parts without records";
+                        }
+                if (bad) { printf("%d x %d%s beside %d x %d: %s\n", l.dp, l.vp, l.second ? " and another mixer" : "", a.dp == l.dp ? b.dp : a.dp, a.vp == l.vp ? b.vp : a.vp, bad); return 1; }
+            }
+        }
+    return 0;
+}
+""")
