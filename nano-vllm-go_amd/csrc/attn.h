@@ -472,8 +472,10 @@ __device__ __forceinline__ void attn_decode_merge(const AttnArgs& p, int pair, i
 // fetched the argument block in two dependent pieces first (in-kernel stamps: 2.4 us from entry to the first vector load
 // at B = 1, against 0.4 us in the projection kernels).
 // SPLIT: its own instance — the arguments and the branch that deal a sequence over workgroups cost an unsplit launch 0.6 us (GPT-2, 104 rows)
-template <int HD, int NW, bool FUSED, bool SPLIT, bool STAMP = false>
-__global__ __launch_bounds__(NW * 64, HD == 128 ? 2 : 1) void attn_decode_bf16_kernel(const int32_t* __restrict__ a_seq_pos, const int32_t* __restrict__ a_blk_table,
+// ORDERED: likewise, launches that take their sequences from the longest context down (a_group: the number of sequences in the upper 16 bits).  As a test in front of
+// every launch it was 11 instructions of 139 and a third scalar round trip before the first load: steps of 1 and 32 sequences 0 .. 0.7 % in eight comparisons that scatter as much
+template <int HD, int NW, bool FUSED, bool SPLIT, bool ORDERED = false, bool STAMP = false>
+__global__ __launch_bounds__(NW * 64, HD == 128 ? 2 : 0) void attn_decode_bf16_kernel(const int32_t* __restrict__ a_seq_pos, const int32_t* __restrict__ a_blk_table,
                                                                    int a_tbl_stride, int a_bs_shift, int a_Tmax, int a_group, AttnArgs p) {
     constexpr int KS = HD / 32, DT = HD / 16, HALF = HD / 2, CPR = HD / 8, KPI = 64 / CPR, NVL = 64 / KPI;
     constexpr int NT2 = HD <= 64 ? 2 : 1;                    // key tiles whose loads are in flight together, per wave
@@ -488,9 +490,10 @@ __global__ __launch_bounds__(NW * 64, HD == 128 ? 2 : 1) void attn_decode_bf16_k
     // 71 heads = 5 tiles that stream the same K/V — it is tiny next to the weights — from L2)
     const int swg = ((SPLIT ? blockIdx.z * gridDim.y : 0) + blockIdx.y) * gridDim.x + blockIdx.x;
     NvlStampsT<STAMP> stamps(p.stamps, swg);          // (diagnostic instantiation only: see common.h)
-    // (ordered: the sequences from the longest context down, in the places before a_seq_pos[0])
-    const int ordered = a_group >> 16, QT = ((a_group & 0xffff) + 15) >> 4;
-    const int seq = ordered ? a_seq_pos[(int)blockIdx.y - ordered] : blockIdx.y, kvh = blockIdx.x / QT, qt = blockIdx.x - kvh * QT;
+    static_assert(!ORDERED || !SPLIT, "a split launch takes the batch's order");
+    const int QT = ((ORDERED ? a_group & 0xffff : a_group) + 15) >> 4;
+    // (ordered: in the places before a_seq_pos[0])
+    const int seq = ORDERED ? a_seq_pos[(int)blockIdx.y - (a_group >> 16)] : blockIdx.y, kvh = blockIdx.x / QT, qt = blockIdx.x - kvh * QT;
     const int32_t* tbl = a_blk_table + (int64_t)seq * a_tbl_stride;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -541,8 +544,9 @@ __global__ __launch_bounds__(NW * 64, HD == 128 ? 2 : 1) void attn_decode_bf16_k
     // one workgroup serves the whole group (GQA / MHA), and lines that stay out of L2 leave it to the projections'
     // activations: decode +5 % at B = 32 (32.0 K -> 33.7 K tok/s), GPT-2 B = 128 +3.2 %; it loses 2 % at 32-64 workgroups
     // (profiles/r03_kv_nontemporal.txt).  Falcon's MQA (5 workgroups share one K/V stream through L2) keeps the default policy.
-    auto tile_offset = [&](int kt, int blk) {
+    auto tile_offset = [&](int kt, bool known, int known_blk) __attribute__((always_inline)) {
         const int bi = kv_block_index(p, kt * 64), krow0 = kt * 64 - bi * p.Tmax;     // the KV block holding this tile
+        const int blk = known ? known_blk : tbl[bi];
         return (int64_t)blk * p.slot_stride + ((int64_t)kvh * p.Tmax + krow0) * HD;
     };
     auto issue_k_t = [&](int h, int64_t off, auto nt_tag) __attribute__((always_inline)) {
@@ -568,7 +572,7 @@ __global__ __launch_bounds__(NW * 64, HD == 128 ? 2 : 1) void attn_decode_bf16_k
         for (int h = 0; h < NT2; h++) {
             const int kt = kt0 + h * NW;
             if (kt >= n_kt) continue;
-            const int64_t off = tile_offset(kt, kt0 == vw ? first_blk[h] : tbl[kv_block_index(p, kt * 64)]);
+            const int64_t off = tile_offset(kt, kt0 == vw, first_blk[h]);
             issue_k_t(h, off, nt_tag);
             issue_v_t(h, off, nt_tag);
         }
@@ -645,7 +649,7 @@ __global__ __launch_bounds__(NW * 64, HD == 128 ? 2 : 1) void attn_decode_bf16_k
 #pragma unroll
             for (int h = 0; h < NT2; h++) {
                 const int kt = min(kt1 + h * NW, n_kt - 1);
-                off1[h] = tile_offset(kt, tbl[kv_block_index(p, kt * 64)]);
+                off1[h] = tile_offset(kt, false, 0);
             }
         }
         // ---- scores of the round's tiles ----

@@ -1471,7 +1471,6 @@ void attention(nvl_model* m, int li, const Meta& md, int n_seqs, int M, int max_
     } else if (max_len == 1) {
         const int cfg = decode_attn_cfg(m, n_seqs), nsplit = cfg >> 8 & 15;
         a.split_max = nsplit; a.split_tiles = (cfg & ~ATTN_ORDERED) >> 12;
-        const int lead_group = a.group | (cfg & ATTN_ORDERED ? n_seqs << 16 : 0);
         dim3 grid(m->nKV * cdiv(m->group, 16), n_seqs, nsplit);      // (kv head x 16-head query tile, sequence, key split)
         a.part = m->attn_part; a.part_cnt = m->attn_part_cnt;
         // waves per workgroup: each wave takes NT2 key tiles per round trip (2 for hd 64, 1 for hd 128).  Short contexts
@@ -1484,27 +1483,33 @@ void attention(nvl_model* m, int li, const Meta& md, int n_seqs, int M, int max_
         // B = 1 +1.7 %, 2 +-0, 4 -2.3 %, 8 -2.4 %, 16 +-0, 24 +2.7 %, 32 +5 %, 48 +1 %; GPT-2 B = 128 (1536 workgroups) +3.2 %
         a.kv_nt = g_attn_kv_nt == 2 || (g_attn_kv_nt == 1 && cdiv(m->group, 16) == 1 && (m->nKV * n_seqs >= 160 || n_seqs == 1));
         a.stamps = (fused_qkv && m->hd == 64) ? next_stamps(m, KS_ATTN, (int)(grid.x * grid.y * grid.z)) : nullptr;
+        const bool ordered = (cfg & ATTN_ORDERED) && !a.stamps;
+        const int lead_group = a.group | (ordered ? n_seqs << 16 : 0);
         if (fused_qkv) {   // RoPE + KV append + attention in one launch, straight from the QKV projection's fp32 output
             a.qkv = m->qkv; a.qkv_stride = m->n_qkv; a.cos_t = m->rope_cos; a.sin_t = m->rope_sin;
         }
 #define NVL_DEC_LEAD a.seq_pos, a.blk_table, a.tbl_stride, a.bs_shift, a.Tmax, lead_group      /* the preloaded leading arguments (attn.h) */
-#define NVL_DECN(HDv, NWv, FUSEDv, SPLITv, STv)                                                                         \
+#define NVL_DECN(HDv, NWv, ...)                                                                                         \
         do {                                                                                                           \
-            NVL_LDS_ATTR((attn_decode_bf16_kernel<HDv, NWv, FUSEDv, SPLITv, STv>), NWv * 64 * HDv * 2);                \
-            hipLaunchKernelGGL((attn_decode_bf16_kernel<HDv, NWv, FUSEDv, SPLITv, STv>), grid, dim3(NWv * 64), NWv * 64 * HDv * 2, m->stream, NVL_DEC_LEAD, a); \
+            NVL_LDS_ATTR((attn_decode_bf16_kernel<HDv, NWv, __VA_ARGS__>), NWv * 64 * HDv * 2);                        \
+            hipLaunchKernelGGL((attn_decode_bf16_kernel<HDv, NWv, __VA_ARGS__>), grid, dim3(NWv * 64), NWv * 64 * HDv * 2, m->stream, NVL_DEC_LEAD, a); \
         } while (0)
-#define NVL_DEC(HDv, FUSEDv, SPLITv, STv)                                                                               \
+#define NVL_DEC(HDv, ...)                                                                                               \
         do {                                                                                                           \
-            if (nw == 2) NVL_DECN(HDv, 2, FUSEDv, SPLITv, STv); else if (nw == 4) NVL_DECN(HDv, 4, FUSEDv, SPLITv, STv); \
-            else NVL_DECN(HDv, 8, FUSEDv, SPLITv, STv);                                                                \
+            if (nw == 2) NVL_DECN(HDv, 2, __VA_ARGS__); else if (nw == 4) NVL_DECN(HDv, 4, __VA_ARGS__); else NVL_DECN(HDv, 8, __VA_ARGS__); \
         } while (0)
-        if (a.stamps && fused_qkv && m->hd == 64 && nsplit == 1) NVL_DEC(64, true, false, true);      // diagnostic instantiation with the in-kernel stamps compiled in
-        else if (fused_qkv && nsplit > 1) { if (m->hd == 64) NVL_DEC(64, true, true, false); else NVL_DEC(128, true, true, false); }
-        else if (fused_qkv) { if (m->hd == 64) NVL_DEC(64, true, false, false); else NVL_DEC(128, true, false, false); }
-        else if (nsplit > 1) { if (m->hd == 64) NVL_DEC(64, false, true, false); else NVL_DEC(128, false, true, false); }
-        else { if (m->hd == 64) NVL_DEC(64, false, false, false); else NVL_DEC(128, false, false, false); }
+#define NVL_DEC_FORM(FUSEDv)                                                                                            \
+        do {                                                                                                           \
+            if (nsplit > 1) { if (m->hd == 64) NVL_DEC(64, FUSEDv, true); else NVL_DEC(128, FUSEDv, true); }            \
+            else if (ordered) { if (m->hd == 64) NVL_DEC(64, FUSEDv, false, true); else NVL_DEC(128, FUSEDv, false, true); } \
+            else { if (m->hd == 64) NVL_DEC(64, FUSEDv, false); else NVL_DEC(128, FUSEDv, false); }                     \
+        } while (0)
+        if (a.stamps && nsplit == 1) NVL_DEC(64, true, false, false, true);      // diagnostic instantiation with the in-kernel stamps compiled in (a.stamps: heads of 64, fused)
+        else if (fused_qkv) NVL_DEC_FORM(true);
+        else NVL_DEC_FORM(false);
 #undef NVL_DECN
 #undef NVL_DEC
+#undef NVL_DEC_FORM
 #undef NVL_DEC_LEAD
     } else {
         // query rows (position x head-in-group, position-major) in workgroups of 4 or 8 waves; K/V tiles by LDS-DMA

@@ -28,6 +28,23 @@ for hd in 64 128; do for form in 2ELi8 1ELi8 1ELi4; do      # sub-tiles per wave
   [ "$m0" = 0 ] && [ "$spills" = 0 ] && [ "$all0" = "$loop0" ] || rc=1
 done; done
 cat $S $S.gemm* > $S.all
+# The entry of the fused decode attention: scalar round trips in front of the first vector load, two in launches that take the batch's order and are not
+# split, three in split ones (the order of ragged contexts, an instance of its own, takes one more)
+python3 - $S <<'PY' || rc=1
+import re, sys
+cur, seen, bad = None, 0, 0
+for line in open(sys.argv[1]):
+    m = re.match(r"_ZN3nvl23attn_decode_bf16_kernelILi(\d+)ELi(\d)ELb1ELb(\d)ELb0ELb0EE\w*:", line)
+    if m: cur, waits = m.groups(), 0; continue
+    op = line.split(";")[0].split()
+    if cur is None or not op: continue
+    waits += op[0] == "s_waitcnt"
+    if op[0].startswith("global_load"):
+        ok = waits <= (3 if cur[2] == "1" else 2)
+        print(("ok  " if ok else "BAD ") + "decode attention hd %s, %s waves%s: %d waits before the first load" % (cur[0], cur[1], ", split" if cur[2] == "1" else "", waits))
+        seen += 1; bad += not ok; cur = None
+sys.exit(1 if bad or seen != 12 else 0)
+PY
 python3 - $S.all <<'PY' || rc=1
 import re, sys
 meta = open(sys.argv[1]).read()
@@ -49,8 +66,8 @@ def check(pattern, what, ok):
         print(("ok  " if good else "BAD ") + what + ": " + k[:96] + "  vgpr(+agpr) %d spills %d" % (r["vgpr"], r["spill"]))
         bad += 0 if good else 1
 # decode attention, hd 64 (fused and plain): two waves per SIMD (<= 256 unified registers), nothing spilled
-check(r"attn_decode_bf16_kernelILi64ELi[248]ELb[01]ELb[01]ELb0E", "decode attention hd 64, 2 waves/SIMD", lambda r: r["vgpr"] <= 256 and r["spill"] == 0)
-check(r"attn_decode_bf16_kernelILi128ELi8ELb[01]ELb[01]ELb0E", "decode attention hd 128, 8 waves", lambda r: r["vgpr"] <= 256 and r["spill"] <= 8)
+check(r"attn_decode_bf16_kernelILi64ELi[248]ELb[01]ELb[01]ELb[01]ELb0E", "decode attention hd 64, 2 waves/SIMD", lambda r: r["vgpr"] <= 256 and r["spill"] == 0)
+check(r"attn_decode_bf16_kernelILi128ELi8ELb[01]ELb[01]ELb[01]ELb0E", "decode attention hd 128, 8 waves", lambda r: r["vgpr"] <= 256 and r["spill"] <= 8)
 # decode projections: the 64-row-group instantiations (PASSES) and the wide form
 check(r"gemm_skinny_bf16_kernelILi4ELi[124]ELi2ELi(?:[0-4]|16)E\w+Lb1ELi0ELb0E", "narrow projection, 64-row groups", lambda r: r["spill"] <= 12)
 check(r"gemm_skinny_bf16_kernelILi[12]ELi[124]ELi4ELi(?:[0-4]|16)E\w+Lb0ELi0ELb[01]E", "narrow projection, <= 32 rows", lambda r: r["spill"] <= 12)
