@@ -466,6 +466,12 @@ __device__ __forceinline__ void attn_decode_merge(const AttnArgs& p, int pair, i
         act_store4<bf16_t>((bf16_t*)p.out, tok, head * HD + d * 16 + fg * 4, p.out_stride, O[d] * inv);
 }
 
+// Host rules of the order of ragged contexts (the figures: decode_attn_cfg).  n_kt: 64-key tiles of the longest, mean_kt: of the mean
+static inline bool attn_order_pays(int n_kt, double mean_kt) { return n_kt >= 1.3 * mean_kt + 1; }
+// ... before the first of some steps, from the sequences' positions: can any of them take it?  (the tiles of pos + 1 keys are pos / 64 + 1 at most, and a step adds
+// as many keys to the mean as to the longest: if not the first, then none)
+static inline bool attn_order_possible(int longest_pos, double mean_pos) { return longest_pos >= 1.3 * (mean_pos + 1); }
+
 // The six leading arguments repeat fields of AttnArgs: the library is built with -amdgpu-kernarg-preload-count=6, so they
 // sit in SGPRs when a wave starts and the two scalar loads every wave needs before it can issue its first K/V load (the
 // sequence's position, the block id of its first tile) leave at once — with everything inside the struct the compiler

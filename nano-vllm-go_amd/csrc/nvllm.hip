@@ -1395,7 +1395,7 @@ static int g_attn_split = 1;   // nvl_set_tuning key 25: split a decode attentio
 //   heads of 128   12 of 1500 / 6 -3.6 -> -5.7 (4 x 3), 16 of 1100 / 6 -1.0 -> -2.1 (4 x 3), 12 of 1500 and short ones -5 -> -7.6 (4 x 6); 16 of 1500 and
 //                  short ones -6.4 (4 x 3), -1.9 (4 x 6: a grid of 768); 12 of 900 / 6 in four parts (238 with work) +0.4, 16 of 1500 / 6 in three (251) +0.9
 // Whole sequences of ragged contexts: workgroups start in the grid's order, and a long one that starts in the second round of them runs on alone.
-// The longest start first (the kernel looks its sequence up: 0.3 % of a step where contexts are alike), and with them in front four waves a
+// The longest start first (in instances of their own, where the kernel looks its sequence up), and with them in front four waves a
 // workgroup pay where two did before, as the short ones fill up behind.  Steps against the batch's order, per cent (2 waves, 4 waves):
 //   heads of 64   Llama-3.2-1B 48 of 1500 / 25 -3.3 (8 waves)  64 of 1500 / 25 -0.1, -4.4  64 of 700 / 8 +0.5, -2.9  96 of 1500 / 25 -2.9, -4.6
 //                 96 of 1500 / 2 -2.0, +0.9  96 of 400 / 7 -1.0, +1.1  128 of 1900 / 12 -0.8, -3.5  128 of 700 / 12 -2.3, -1.4  128 of 300 / 8 -1.0, +0.7
@@ -1404,9 +1404,13 @@ static int g_attn_split = 1;   // nvl_set_tuning key 25: split a decode attentio
 //   heads of 128  Llama-3-8B 48 of 1500 / 25 -4.3 (4)  96 of 1000 / 16 -2.9, -4.2  128 of 400 / 7 -2.3, -1.3; 32 of 1500 / 15 -0.1 (8)
 constexpr int ATTN_ORDERED = 1 << 30;
 bool decode_may_order(const nvl_model* m, int n_seqs) { return !m->f32 && !m->layered && n_seqs < 1 << 15 && m->nKV * cdiv(m->group, 16) * n_seqs > 256; }
-// (meta_host of a decode pass)
+// (meta_host of a decode pass, or of the first of some; contexts that are alike are not sorted)
 void decode_order(const nvl_model* m, const Meta& hm, int n_seqs) {
-    if (!decode_may_order(m, n_seqs)) return;
+    if (!g_attn_order || !decode_may_order(m, n_seqs)) return;
+    int longest = 0;
+    double sum = 0;
+    for (int i = 0; i < n_seqs; i++) { longest = std::max(longest, hm.seq_pos[i]); sum += hm.seq_pos[i]; }
+    if (g_attn_order != 2 && !attn_order_possible(longest, sum / n_seqs)) return;
     int32_t* order = hm.seq_pos - n_seqs;
     for (int i = 0; i < n_seqs; i++) order[i] = i;
     std::sort(order, order + n_seqs, [&](int a, int b) { return hm.seq_pos[a] != hm.seq_pos[b] ? hm.seq_pos[a] > hm.seq_pos[b] : a < b; });
@@ -1435,7 +1439,7 @@ int decode_attn_cfg(const nvl_model* m, int n_seqs) {
             if (each < rounds) return cfg(waves, cdiv(rounds, each), each * round);
         }
     }
-    const bool ordered = g_attn_order && m->ctx_hint > 0 && decode_may_order(m, n_seqs) && (g_attn_order == 2 || n_kt >= 1.3 * mean_kt + 1);
+    const bool ordered = g_attn_order && m->ctx_hint > 0 && decode_may_order(m, n_seqs) && (g_attn_order == 2 || attn_order_pays(n_kt, mean_kt));
     if (ordered && !g_attn_nw && wgs >= 512 && wgs <= 1024 && n_kt >= 11 && n_kt >= 1.8 * mean_kt) nw = 4;
     return cfg(nw, 1, 1 << 16) | (ordered ? ATTN_ORDERED : 0);
 }

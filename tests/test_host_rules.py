@@ -88,3 +88,29 @@ int main() {
     return 0;
 }
 """)
+
+
+@pytest.mark.skipif(HIPCC is None, reason="no hipcc")
+def test_contexts_are_sorted_wherever_a_step_takes_them_by_length(tmp_path):
+    """The sort of a call's first step serves all its steps, and is left out where none of them can ask for it."""
+    run(tmp_path, r"""
+#include "attn.h"
+int main() {
+    unsigned seed = 1;
+    auto rnd = [&](int n) { seed = seed * 1664525u + 1013904223u; return (int)((seed >> 8) % n); };
+    int sorted = 0, left = 0;
+    for (int t = 0; t < 20000; t++) {
+        const int n = 33 + rnd(200), spread = 1 + rnd(t % 2 ? 60 : 1500), least = rnd(1500);
+        int longest = 0; double sum = 0;
+        for (int i = 0; i < n; i++) { const int pos = least + rnd(spread); longest = longest > pos ? longest : pos; sum += pos; }
+        const bool possible = nvl::attn_order_possible(longest, sum / n);
+        (possible ? sorted : left)++;
+        for (int s = 0; s < 200; s++) {
+            const int keys = longest + s + 1;
+            if (nvl::attn_order_pays((keys - 1) / 64 + 1, (sum / n + s + 1) / 64) && !possible) { printf("%d sequences, longest %d, mean %f, step %d\n", n, longest, sum / n, s); return 1; }
+        }
+    }
+    printf("%d sorted, %d not\n", sorted, left);
+    return sorted < 1000 || left < 1000;
+}
+""")
