@@ -962,8 +962,11 @@ static inline int grouped_key_splits(int64_t wgs, int64_t cap, int key_tiles, in
 void grouped_prefill_launch(hipStream_t st, const GroupedArgs& p, dim3 grid, size_t lds, bool fast);
 void grouped_short_launch(hipStream_t st, const GroupedArgs& p, dim3 grid);
 void grouped_qk_launch(hipStream_t st, const GroupedArgs& p, bool f32);
-// bf16: larger batches are worked in tiles of 16 tokens, too few workgroups below (18 layers of 32 heads, a prompt of 513 / 600 / 750 tokens in tiles -> head by head 3197 -> 3163,
-// 3302 -> 3266, 3546 -> 3526 us; 1000 / 1600 3881 -> 3891, 5314 -> 5392)
-constexpr int GROUPED_QK_ROW_MAX = 768;
+// bf16: larger batches are worked in tiles of 16 tokens, too few workgroups below.  us a launch, head by head / in tiles, at 513, 768, 1000 and 1600 rows:
+//   heads of 128   4 + 1 6.5 / 7.8, 6.9 / 8.0, 7.4 / 8.1, 8.9 / 8.2     8 + 2 7.6 / 10.3, 9.0 / 10.3, 10.8 / 10.4, 12.8 / 10.5     16 + 4 10.7 / 15.6, 12.8 / 15.6, 14.5 / 15.7, 19.2 / 16.1
+//                  32 + 8 17.0 / 28.3, 22.1 / 28.9, 26.2 / 28.8, 37.5 / 29.0     64 + 8 (no registers for them: grouped_qk_tile_kernel) 32.8 / 103.6, 44.3 / 104.8, 54.9 / 105.4, 83.5 / 106.4
+//   heads of 64    64 + 8 (likewise) 24.3 / 54.5, 32.1 / 54.9, 39.6 / 55.7, 58.1 / 56.0     16 + 4 10.1 / 10.3, 12.2 / 10.4, 14.3 / 10.5     40 + 8 16.7 / 17.8, 22.0 / 17.8, 26.3 / 18.0
+static inline bool grouped_qk_in_regs(const GroupedArgs& p) { return p.dim == p.dp && p.rot == p.dp && (p.dp == 64 || p.dp == 128) && p.H + p.G <= 48; }
+static inline int grouped_qk_row_max(const GroupedArgs& p) { return p.dp == 64 && grouped_qk_in_regs(p) ? 512 : 768; }
 
 }  // namespace nvl

@@ -19,7 +19,7 @@ def against_fp32(gpu, tmp_path, cfg, w, tok):
     assert err(got["bf16"], got["f32"], "bf16") < BF16_LAYER
 
 
-@pytest.mark.parametrize("n", [513, 768, 769, 1024, 1025, 1031])      # 768: queries and keys normed and turned head by head up to here, in tiles of 16 tokens above
+@pytest.mark.parametrize("n", [513, 768, 769, 1024, 1025, 1031])      # queries and keys normed and turned head by head up to 768 rows (heads of 64 in registers: 512), in tiles of 16 tokens above
 @pytest.mark.parametrize("layer,width", [(MM.attention(mlp=MM.moe()), 96), (MM.attention(mlp=MM.moe()), 1056), (MM.parallel(mlp=MM.dense(48)), 96),
                                          (MM.attention(heads=16, kv_heads=4, dim=64, vdim=64, turn=MM.rot(64), mlp=MM.dense(2048)), 1024),      # 64 and more slices of both residual projections
                                          (MM.attention(heads=4, kv_heads=2, dim=128, vdim=128, turn=MM.rot(128), mlp=MM.dense(48)), 128)],
