@@ -1082,12 +1082,14 @@ void mix_latent(nvl_model* m, const LayerRun& r, const MixerW& w, const Meta& md
     }
 }
 
+double linrec_flops(const LinRecArgs& a, int M) { return 4.0 * (double)M * a.H * a.DK * a.DV; }
+double linrec_bytes(const LinRecArgs& a, int n_seqs, int M) {       // rows in and out, the states once each way
+    return (double)M * a.H * (2.0 * a.DK / a.kdiv + 2.0 * a.DV) * 4.0 + 2.0 * n_seqs * (double)a.H * a.DK * a.DVp * 4.0;
+}
 // the recurrence of a layer over the batch; fused: one token (or a few) per sequence, everything between the projections in one launch
 template <bool CH>
 void linrec(nvl_model* m, LinRecArgs a, int n_seqs, int M, int max_len, bool fused, int site) {
-    const double elems = (double)a.H * a.DK * a.DVp;
-    const double bytes = (double)M * a.H * (2.0 * a.DK / a.kdiv + 2.0 * a.DV) * 4.0 + 2.0 * n_seqs * elems * 4.0;
-    KScope ks(m, KC_OTHER, 4.0 * (double)M * a.H * a.DK * a.DV, site, bytes);
+    KScope ks(m, KC_OTHER, linrec_flops(a, M), site, linrec_bytes(a, n_seqs, M));
     a.len_lo = 1; a.len_hi = 1 << 30;
     if (fused) {
         linrec_step_launch(m->stream, a, n_seqs, CH, true, m->f32);
@@ -1369,7 +1371,8 @@ void mix_grouped(nvl_model* m, const LayerRun& r, const MixerW& w, const Meta& m
     const bool any_short = m->min_len * a.group <= a.short_rows, any_long = max_len * a.group > a.short_rows;
     auto scope = [&](int several) {
         const double pairs = m->win_pairs[(size_t)r.win][(size_t)several], keys = m->win_keys[(size_t)r.win][(size_t)several];
-        return KScope(m, KC_ATTN, 2.0 * pairs * a.H * (c.dim + c.vdim), KS_ATTN, (keys * a.G * (c.dim + c.vdim) + (double)M * a.H * (c.dim + 2.0 * c.vdim)) * ws);
+        return KScope(m, KC_ATTN, 2.0 * pairs * a.H * (c.dim + c.vdim) + (a.lin_heads ? linrec_flops(a.lin, M) : 0.0), KS_ATTN,
+                      (keys * a.G * (c.dim + c.vdim) + (double)M * a.H * (c.dim + 2.0 * c.vdim)) * ws + (a.lin_heads ? linrec_bytes(a.lin, n_seqs, M) : 0.0));
     };
     if (plain) {
         KScope ks = scope(max_len > 1);

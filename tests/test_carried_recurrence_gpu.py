@@ -65,3 +65,26 @@ def test_beside_a_wider_layer(gpu, tmp_path, wide, at):
         gpu.lib().nvl_set_tuning(44, old)
     assert np.array_equal(got["bf16", 1], got["bf16", 0])
     assert err(got["bf16", 1], got["f32", 1]) < 0.06            # two bf16 layers, the worst row (0.03 a layer in the other tests of these models)
+
+
+def test_profile_counts_the_recurrence(gpu, tmp_path):
+    """Work and traffic of a step's launches are the same whether the recurrence rides or not."""
+    cfg = MM.config([MM.parallel(**LAYERS["128x128"])], width=128, vocab=90)
+    m = build(gpu, tmp_path, cfg, MM.weights(cfg, 4), "bf16", max_seqs=3)
+    for i in range(3):
+        m.seq_open(i)
+    m.forward_batch([0, 1, 2], [[3, 4, 5]] * 3, [0, 0, 0], want_logits=False)
+    total = []
+    for rides in (0, 2):
+        old = gpu.lib().nvl_set_tuning(44, rides)
+        m.reset_stats()
+        m.set_profile(True)
+        m.forward_batch([0, 1, 2], [[7]] * 3, [3 + len(total)] * 3, want_logits=False)
+        m.set_profile(False)
+        gpu.lib().nvl_set_tuning(44, old)
+        ks = [k for k in m.kernel_stats() if k["site"] in ("attention", "lightning_scan") and k["launches"]]
+        assert len(ks) == (1 if rides else 2)
+        total.append((sum(k["flops"] for k in ks), sum(k["bytes"] for k in ks)))
+    m.close()
+    state = 2 * 3 * 5 * 128 * 128 * 4                           # every sequence's five states, in and out
+    assert total[0][1] > state and abs(total[1][0] / total[0][0] - 1) < 0.05 and abs(total[1][1] / total[0][1] - 1) < 0.05      # (a key more in the second step)
