@@ -50,6 +50,7 @@ struct DeltaArgs {
 
 constexpr int DELTA_C = 32;            // tokens per chunk
 constexpr int DELTA_ORDERED = 64;       // sequences that the scan takes in the order of their lengths, at most
+constexpr int DELTA_SCAN_WAVES = 4;    // of a workgroup of the scan
 static inline __host__ __device__ int64_t delta_ws_floats(int dkp) { return (int64_t)dkp * (3 * DELTA_C + 1); }     // -W | Q' | K^T | e^{b_end}
 __device__ __forceinline__ int64_t delta_chunk(const DeltaArgs& p, int seq, int c) { return p.seq_tok_start[seq] / DELTA_C + seq + c; }
 
@@ -321,7 +322,7 @@ __global__ __launch_bounds__(512, NK > 8 ? 2 : 4) void delta_prep_kernel(DeltaAr
 }
 
 // ------------------------------------------------------------------------------------------
-// scan: grid (heads, slices of 16 NW / KSP value columns, sequences).  A wave keeps DK / KSP x 16 of the state in accumulators: 16 columns,
+// scan: grid (heads, slices of 64 / KSP value columns, sequences).  A wave keeps DK / KSP x 16 of the state in accumulators: 16 columns,
 // and with KSP > 1 (few heads and sequences) a part of the key channels — the parts' sums of U and O meet in LDS.
 // The next chunk's operands are on their way to registers while the state is updated.
 // ------------------------------------------------------------------------------------------
@@ -339,11 +340,11 @@ __device__ __forceinline__ int delta_scan_seq(const int* seq_len, int i, int n_s
     }
     return __builtin_amdgcn_readfirstlane(__builtin_ctzll(__ballot(rank == (i == 0 ? n_seqs - 1 : i - 1) && lane < n_seqs)));
 }
-template <int NK, int NW, int KSP> constexpr int delta_scan_lds_bytes() { return 4 * (2 * DELTA_C * (NK * 16 + 4) + NK * 16 * 36 + NK * 16 + (KSP > 1 ? NW * 1024 : 0)); }
+template <int NK, int KSP> constexpr int delta_scan_lds_bytes() { return 4 * (2 * DELTA_C * (NK * 16 + 4) + NK * 16 * 36 + NK * 16 + (KSP > 1 ? DELTA_SCAN_WAVES * 1024 : 0)); }
 
-template <int NK, int NW, int KSP>
-__global__ __launch_bounds__(NW * 64, NK > 8 ? 1 : 3) void delta_scan_kernel(DeltaArgs p) {
-    constexpr int C = DELTA_C, DKP = NK * 16, LQ = DKP + 4, LK = 36, NT = NW * 64, NKW = NK / KSP, NCG = NW / KSP;
+template <int NK, int KSP>
+__global__ __launch_bounds__(DELTA_SCAN_WAVES * 64, NK > 8 ? 1 : 3) void delta_scan_kernel(DeltaArgs p) {
+    constexpr int NW = DELTA_SCAN_WAVES, C = DELTA_C, DKP = NK * 16, LQ = DKP + 4, LK = 36, NT = NW * 64, NKW = NK / KSP, NCG = NW / KSP;
     const int h = blockIdx.x, seq = delta_scan_seq(p.seq_len, (int)blockIdx.z, (int)gridDim.z);
     const int n = p.seq_len[seq];
     if (n < p.len_lo || n > p.len_hi) return;

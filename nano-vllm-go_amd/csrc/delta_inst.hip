@@ -32,11 +32,11 @@ static void prep(hipStream_t st, const DeltaArgs& p, dim3 grid) {
 void delta_prep_launch(hipStream_t st, const DeltaArgs& p, dim3 grid, int nk) {
     if (nk == 2) prep<2>(st, p, grid); else if (nk == 4) prep<4>(st, p, grid); else if (nk == 8) prep<8>(st, p, grid); else prep<16>(st, p, grid);
 }
-template <int NK, int NW, int KSP>
+template <int NK, int KSP>
 static void scan(hipStream_t st, const DeltaArgs& p, int n_seqs) {
-    constexpr int lds = delta_scan_lds_bytes<NK, NW, KSP>();
-    NVL_LDS_ATTR((delta_scan_kernel<NK, NW, KSP>), lds);
-    hipLaunchKernelGGL((delta_scan_kernel<NK, NW, KSP>), dim3(p.H, cdiv(p.DV, 16 * NW / KSP), n_seqs), dim3(NW * 64), lds, st, p);
+    constexpr int lds = delta_scan_lds_bytes<NK, KSP>();
+    NVL_LDS_ATTR((delta_scan_kernel<NK, KSP>), lds);
+    hipLaunchKernelGGL((delta_scan_kernel<NK, KSP>), dim3(p.H, cdiv(p.DV, 16 * DELTA_SCAN_WAVES / KSP), n_seqs), dim3(DELTA_SCAN_WAVES * 64), lds, st, p);
 }
 // Parts of the key channels (KSP): more parts shorten the chain of a sequence's chunks, whose fp32 products bound a wave, and cost each of them an exchange.
 // us, fitted to 1 .. 64 sequences of 100 .. 1900 tokens x 16 heads of 128, good to 20 %: the longest sequence's chain, all chunks at the chip's rate, the larger of them
@@ -55,11 +55,11 @@ static void scan_shape(hipStream_t st, const DeltaArgs& p, int n_seqs, int max_l
     double t = scan_cost(p, n_seqs, NK, 1, max_len, tokens);
     auto consider = [&](int ksp) { const double c = scan_cost(p, n_seqs, NK, ksp, max_len, tokens); if (c < 0.95 * t) { t = c; best = ksp; } };
     (consider(PARTS), ...);
-    if (best == 1) { scan<NK, 4, 1>(st, p, n_seqs); return; }
-    ((best == PARTS ? scan<NK, 4, PARTS>(st, p, n_seqs) : void()), ...);
+    if (best == 1) { scan<NK, 1>(st, p, n_seqs); return; }
+    ((best == PARTS ? scan<NK, PARTS>(st, p, n_seqs) : void()), ...);
 }
 void delta_scan_launch(hipStream_t st, const DeltaArgs& p, int n_seqs, int nk, int max_len, int tokens) {
-    if (nk == 2) scan<2, 4, 1>(st, p, n_seqs);
+    if (nk == 2) scan<2, 1>(st, p, n_seqs);
     else if (nk == 4) scan_shape<4, 2>(st, p, n_seqs, max_len, tokens);
     else if (nk == 8) scan_shape<8, 2, 4>(st, p, n_seqs, max_len, tokens);
     else scan_shape<16, 2, 4>(st, p, n_seqs, max_len, tokens);
