@@ -301,6 +301,19 @@ def test_prompt_of_many_hundred_tokens(gpu, tmp_path):
     m.close()
 
 
+@pytest.mark.parametrize("mlp,width,side", [(BM.dense(40), 96, None), (moe(6, 2, None, 24), 96, 20), (moe(6, 2, None, 24), 1056, None), (BM.dense(40), 2080, 20), (moe(6, 2, None, 24), 4096, None)])
+def test_prompt_of_more_than_a_thousand_tokens(gpu, tmp_path, mlp, width, side):
+    """Sums, their second sources and layer norms in tiles of eight rows (4, 8 and 16 chunks of a row per lane): 1031 rows, a remainder of seven, in one piece, and
+    as many in portions that go row by row."""
+    cfg = BM.config([att(heads=2, kv_heads=1, window=40, mlp=mlp)], width=width, vocab=90, side=side, positions=1088)
+    w = BM.weights(cfg, 18)
+    tok, want, _ = BM.clear_tokens(cfg, w, 1031, 6)
+    m = build(gpu, tmp_path, cfg, w, "bf16", max_seq_len=1088, max_batch_tokens=1088, kv_num_blocks=80)
+    for i, cuts in enumerate(([1031], [700, 331])):
+        assert err(feed(m, i, tok, cuts), want, "bf16") < ONE["bf16"], cuts
+    m.close()
+
+
 # ---- the framework's own entry points ----
 def test_greedy_generation(gpu, tmp_path, stack):
     """Stepwise, fused on the device, and through the runner give the restatement's tokens (fp32)."""

@@ -50,15 +50,15 @@ def test_scan_order(gpu, tmp_path, lens):
 
 
 @pytest.mark.parametrize("width", [64, 1056, 2080, 4096])             # 4 / 8 / 16 chunks of a row per lane
-@pytest.mark.parametrize("lens", [[513], [519, 9]])                    # 513 and 528 rows: remainders of 8 and of 16, whole halves
+@pytest.mark.parametrize("lens", [[513], [519, 9], [1025], [1031, 9]])  # a row per workgroup; 1025 and 1040 rows: tiles of eight, one row over and whole tiles
 def test_sandwich_tiles(gpu, tmp_path, width, lens):
-    """The prompt's sandwich norms in tiles of eight rows against portions of up to 300 rows, a row per workgroup: two bf16 runs whose
-    operands may round apart, each within the bf16 bound of a layer."""
+    """The prompt's sandwich norms, above 1024 rows in tiles of eight, against portions of up to 300 rows, a row per workgroup: two bf16 runs
+    whose operands may round apart, each within the bf16 bound of a layer."""
     cfg = LM.config([LM.delta(heads=2, kv_heads=2, dim=32, vdim=32)], width=width, vocab=60)
     w = LM.weights(cfg, 17)
     g = np.random.default_rng(width)
     tok = [g.integers(0, 60, n).tolist() for n in lens]
-    m = build(gpu, tmp_path, cfg, w, "bf16", max_seqs=4, max_batch_tokens=1024)
+    m = build(gpu, tmp_path, cfg, w, "bf16", max_seqs=4, max_seq_len=1088, max_batch_tokens=1088, kv_num_blocks=80)
     ids = list(range(len(lens)))
     for i in range(4):
         m.seq_reset(i)

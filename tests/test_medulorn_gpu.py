@@ -394,12 +394,13 @@ def test_key_splits(gpu, tmp_path, layer):
 
 
 def test_prompt_of_many_hundred_tokens(gpu, tmp_path):
-    """Long enough for the kernels of whole row tiles: norms of sums, shift, query/key norms and rotation, experts gathered."""
+    """Long enough for the kernels of whole row tiles (norms of sums above 1024 rows, query/key norms and rotation above 768), for those of up to as many rows that
+    are larger than a decode step's, and for gathered experts."""
     cfg = MM.config([att(chunk=40), par(window=40, mlp=moe(6, 2, 24))], width=520, vocab=90)
     w = MM.weights(cfg, 18)
-    tok, want, _ = MM.clear_tokens(cfg, w, 690, 6)
-    m = build(gpu, tmp_path, cfg, w, "bf16")
-    for i, cuts in enumerate(([690], [530, 160], [64, 600, 26])):
+    tok, want, _ = MM.clear_tokens(cfg, w, 1060, 6)
+    m = build(gpu, tmp_path, cfg, w, "bf16", max_seq_len=1088, max_batch_tokens=1088, kv_num_blocks=80)
+    for i, cuts in enumerate(([1060], [690, 370], [530, 160, 370], [64, 600, 26, 370])):
         assert err(feed(m, i, tok, cuts), want, "bf16") < 1.5 * ONE["bf16"], cuts
     m.close()
 

@@ -177,7 +177,7 @@ def test_moe_down_completes_its_slices(gpu, n):
 @pytest.mark.parametrize("heads,hd,groups", [(16, 64, 2), (8, 32, 1), (10, 64, 1)])      # 10 heads: rows that are no multiple of 16 bytes
 @pytest.mark.parametrize("lens", [[1, 2, 3, 4, 117], [128], [5, 7, 9, 130, 1, 8, 23]])
 def test_mamba_prompts(gpu, heads, hd, groups, lens):
-    """The convolution over runs of tokens (sequences that begin anywhere in a run) and the gated norm of eight rows: a batch against each
+    """The convolution over runs of tokens (sequences that begin anywhere in a run) and the gated norm row by row: a batch against each
     prompt alone in the fp32 mode (the same sums), and the bf16 mode against it."""
     cfg = gpu.synth.tiny_config("granite_hybrid", hidden=heads * hd // 2, num_heads=heads * hd // 128, num_kv_heads=1, mamba_num_heads=heads, mamba_head_dim=hd, mamba_state_size=32,
                                 mamba_n_groups=groups, max_seq_len=256)
