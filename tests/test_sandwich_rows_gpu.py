@@ -1,4 +1,5 @@
-"""Sandwich norms of 513 .. 1024 rows, a workgroup per row with a row-major copy for experts and K slices to add up, and of more rows, tiles of eight."""
+"""Sandwich norms of 513 .. 1024 rows, a workgroup per row with a row-major copy for experts and K slices to add up, and of more rows, tiles of eight.
+Experts of whole 256-wide tiles (experts-in-place) read their rows from that copy, in 256-row segments that end anywhere."""
 import numpy as np
 import pytest
 
@@ -20,10 +21,11 @@ def against_fp32(gpu, tmp_path, cfg, w, tok):
 
 
 @pytest.mark.parametrize("n", [513, 768, 769, 1024, 1025, 1031])      # queries and keys normed and turned head by head up to 768 rows (heads of 64 in registers: 512), in tiles of 16 tokens above
-@pytest.mark.parametrize("layer,width", [(MM.attention(mlp=MM.moe()), 96), (MM.attention(mlp=MM.moe()), 1056), (MM.parallel(mlp=MM.dense(48)), 96),
+@pytest.mark.parametrize("layer,width", [(MM.attention(mlp=MM.moe()), 96), (MM.attention(mlp=MM.moe()), 1056), (MM.attention(mlp=MM.moe()), 2080), (MM.parallel(mlp=MM.dense(48)), 96),
+                                         (MM.attention(mlp=MM.moe(experts=6, top=2, ff=256)), 256), (MM.attention(mlp=MM.moe(experts=6, top=2, ff=256)), 512),
                                          (MM.attention(heads=16, kv_heads=4, dim=64, vdim=64, turn=MM.rot(64), mlp=MM.dense(2048)), 1024),      # 64 and more slices of both residual projections
                                          (MM.attention(heads=4, kv_heads=2, dim=128, vdim=128, turn=MM.rot(128), mlp=MM.dense(48)), 128)],
-                         ids=["experts-96", "experts-1056", "parallel", "slices", "heads-128"])
+                         ids=["experts-96", "experts-1056", "experts-2080", "parallel", "experts-in-place-256", "experts-in-place-512", "slices", "heads-128"])
 def test_rows_and_tiles(gpu, tmp_path, layer, width, n):
     cfg = MM.config([layer], width=width, vocab=130)
     w = MM.weights(cfg, 11)
