@@ -2312,7 +2312,10 @@ static inline void launch_gemm_grouped(hipStream_t st, const GemmArgs& a, int ma
         return;
     }
     // (decode-sized batches too, a handful of rows an expert: us a layer of 1 / 4 / 16 / 64 rows, 32 experts, 8 a token, with four K tiles of 64 in 128 KiB ->
-    // here: 512 x 2048 75 -> 69.6, 86.6 -> 79.7, 97.2 -> 92.8, 120.2 -> 117.2; 1024 x 4096 128 -> 124, 202 -> 184, 235 -> 229, 271 -> 267; 512 x 1024 3 %)
+    // four of 32 on four waves: 512 x 2048 75 -> 69.6, 86.6 -> 79.7, 97.2 -> 92.8, 120.2 -> 117.2; 1024 x 4096 128 -> 124, 202 -> 184, 235 -> 229, 271 -> 267; 512 x 1024 3 %.
+    // Eight waves of 32x64, us a launch on four -> here, 32 experts, 8 a token: up 1024 x 1024 at 100 / 200 / 255 rows 21.3 -> 20.3, 23.2 -> 21.8, 24.2 -> 22.4, a decode step of
+    // 96 21.2 -> 20.4, down 1024 x 512 14.0 -> 13.6, 15.6 -> 15.3, 16.2 -> 16.0, 13.5 -> 13.4; up 1024 x 2048 at 40 / 100 / 200 37.5 / 37.7, 35.8 -> 35.6, 38.9 -> 38.6, down 2048 x 512
+    // 27.1 / 27.1, 19.9 -> 19.2, 23.3 -> 23.0, a step of 96 22.5 -> 21.9)
     constexpr int lds = gemm_lds_bytes<128, 128, 4, 32>();
     NVL_LDS_ATTR((gemm_bf16_kernel<128, 128, 4, 2, 4, EPI, OutT, 32>), lds);
     hipLaunchKernelGGL((gemm_bf16_kernel<128, 128, 4, 2, 4, EPI, OutT, 32>), dim3(cdiv(a.N, 128) * max_mtiles), dim3(512),

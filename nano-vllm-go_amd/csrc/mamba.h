@@ -561,7 +561,10 @@ __global__ __launch_bounds__(256) void mamba_gate_norm_kernel(MambaArgs p, ActT*
 // Prefill-sized bf16 batches, EH <= 4096: a wave holds a row in registers (y is read once and not written back), eight rows a workgroup, so
 // that the operand leaves in whole 128-byte lines (row by row each lane's 8 bytes were a line of their own: 2326 x 4096 48 us, 34
 // here).  Below 512 rows too few workgroups: a prompt of 24 layers of 4096 columns, here -> row by row, 130 / 200 / 300 / 400 tokens 1343 -> 1310, 1433 -> 1401, 1681 -> 1658, 1885 -> 1872 us;
-// 600 as long either way, 1000 / 1900 2952 -> 2982, 4754 -> 4863.
+// 600 as long either way, 1000 / 1900 2952 -> 2982, 4754 -> 4863.  us a launch, row by row / in tiles, at 130, 300, 512, 600, 1000 and 1900 rows: 4096 columns 11.6 / 15.0, 13.3 / 15.4,
+// 15.8 / 15.9, 16.8 / 16.1, 20.5 / 17.6, 33.5 / 21.2; 3072 9.7 / 12.3, 11.0 / 12.7, 11.5 / 12.8, 12.4 / 13.0, 15.3 / 14.9, 26.0 / 17.8; 2048 8.2 / 11.3, 8.7 / 11.2, 9.6 / 11.3, 9.8 / 11.3,
+// 11.5 / 12.0, 16.4 / 14.1; 1024 6.5 / 10.0, 7.1 / 10.3, 7.3 / 10.2, 7.5 / 10.3, 8.1 / 10.3, 10.4 / 11.5; 512 6.6 / 9.5, 6.9 / 10.0, 7.0 / 10.4, 6.7 / 9.8, 6.8 / 10.1, 7.8 / 10.6.  So up to 512 rows
+// no width is better off in tiles; narrower ones would be row by row for some more.
 constexpr int MAMBA_GATE_TILE_ROWS = 512;
 static inline constexpr int mamba_gate_tile_lds_bytes(int EH) { return 8 * (EH + 8) * 2; }
 static __global__ __launch_bounds__(512) void mamba_gate_norm_tile_kernel(MambaArgs p, bf16_t* __restrict__ out, int tokens) {
