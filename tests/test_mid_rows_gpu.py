@@ -238,8 +238,8 @@ def test_mamba_prompts_in_slices(gpu, lens, all_logits):
 
 @pytest.mark.parametrize("n", [65, 513, 530, 1040])
 def test_moe_prompt_forms(gpu, n):
-    """Routing in the router's launch, expert-ordered rows copied from the norm's row-major result (beyond 512 tokens): against the separate
-    launches and the fragment-major source."""
+    """Routing in the router's launch, experts that read their rows from the norm's row-major result (beyond 512 tokens): against the separate
+    launches and rows copied into expert order from the fragment-major operand."""
     import torch
     from bench import gen_weights_on_device
     cfg = dict(gpu.synth.FULL_CONFIGS["granite-3.0-1b-a400m"], num_layers=1, vocab_size=1000)

@@ -35,7 +35,7 @@ def test_matmul(gpu, oracle, m, k, n, precision):
 @pytest.mark.parametrize("tile", [1, 2, 3, 5])
 @pytest.mark.parametrize("m,k,n", [(300, 128, 200), (517, 256, 384), (256, 64, 128)])
 def test_matmul_prefill_tile_kernels(gpu, oracle, tile, m, k, n):
-    """All prefill tile instances (128x128x2st, 256x128x3st, 256x256x2st, 256x256 ping-pong) on ragged M/N edges."""
+    """Prefill tiles (64x128 on the K ring, where key 0 = 1 takes so few of them; 256x128 on the ring; 256x256x2st; 256x256 ping-pong) on ragged M/N edges."""
     r = rng(m + n)
     a = r.standard_normal((m, k), dtype=np.float32)
     b = r.standard_normal((k, n), dtype=np.float32) * 0.05

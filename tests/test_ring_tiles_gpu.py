@@ -9,7 +9,8 @@ TOL = 1.5e-2
 
 
 @pytest.mark.parametrize("k", [64, 128, 192, 256, 320, 2048])          # 2, 4, 6, 8, 10 and 64 K tiles; the ring holds 4
-@pytest.mark.parametrize("m,n", [(65, 130), (128, 128), (129, 384), (700, 96), (1000, 1000)])
+@pytest.mark.parametrize("m,n", [(65, 130), (128, 128), (129, 384), (700, 96), (1000, 1000),      # 64x128 tiles
+                                 (1500, 1601), (2049, 1030)])                                       # 312 and 297 of those: 128x128, on eight waves
 def test_products_are_exact(gpu, m, n, k):
     """Small whole numbers: every sum is exact in fp32, whatever its order."""
     r = np.random.default_rng(m + n + k)
@@ -20,6 +21,25 @@ def test_products_are_exact(gpu, m, n, k):
     finally:
         gpu.lib().nvl_set_tuning(0, old)
     assert np.array_equal(got, (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32))
+
+
+@pytest.mark.parametrize("hidden", [64, 128, 192, 256, 320])           # 2 .. 10 K tiles
+def test_few_tiles_of_k_on_four_waves(gpu, hidden):
+    """Gate | up columns of a prompt on 660 tiles of 128x128, whose gated results are bf16: four waves, against the fp32 mode."""
+    cfg = gpu.synth.tiny_config("llama", hidden=hidden, num_heads=hidden // 64, num_kv_heads=hidden // 64, head_dim=64, ffn_dim=8448, num_layers=2, max_seq_len=640)
+    w = gpu.synth.make_weights(cfg, seed=4, scale=0.03)
+    tokens = np.random.default_rng(hidden).integers(0, cfg["vocab_size"], 601).tolist()
+    got = []
+    old = gpu.lib().nvl_set_tuning(0, 1)
+    try:
+        for precision in ("f32", "bf16"):
+            m = gpu.HipTransformerModel(cfg, w, precision=precision, max_seqs=1, max_batch_tokens=640)
+            m.seq_reset(0)
+            got.append(m.forward_batch([0], [tokens], [0], all_logits=True)[0])
+            m.close()
+    finally:
+        gpu.lib().nvl_set_tuning(0, old)
+    assert rel_err(got[1], got[0]) <= TOL
 
 
 # 2048 columns: two slices of 33 K tiles of FFN-down's 66, up to 200 rows the LDS-ring kernel instead; 512: four of 17, 17, 16 and 16
