@@ -6,7 +6,7 @@
 //   delta_step_kernel   token by token, the state streamed once per token (decode).  FUSED (one token per sequence): the short
 //                       convolutions, the low-rank decay and gate projections, the head norm and the output gate in the same launch.
 //   delta_prep_kernel   32 tokens of one head, independent of the state that enters them (prefill, all chunks at once).
-//   delta_scan_kernel   carries the state through the chunks of a sequence: three products per chunk.
+//   delta_scan_kernel, delta_scan_parts_kernel   carry the state through the chunks of a sequence: three products per chunk.
 //
 // Chunk form.  With b_t = the inclusive sum of log a inside the chunk and S_in the state that enters it:
 //     u_t = beta_t (v_t - (k_t e^{b_t})^T S_in - sum_{s<t} M[t][s] u_s),      M[t][s] = sum_c k_t[c] k_s[c] e^{b_t[c] - b_s[c]}
@@ -51,7 +51,10 @@ struct DeltaArgs {
 constexpr int DELTA_C = 32;            // tokens per chunk
 constexpr int DELTA_ORDERED = 64;       // sequences that the scan takes in the order of their lengths, at most
 constexpr int DELTA_SCAN_WAVES = 4;    // of a workgroup of the scan
-static inline __host__ __device__ int64_t delta_ws_floats(int dkp) { return (int64_t)dkp * (3 * DELTA_C + 1); }     // -W | Q' | K^T | e^{b_end}
+// A chunk of a head in scratch: -W, Q' and (K e^{b_end - b})^T as operands of the scan's products, a KiB each of its 64 lanes' 16 bytes: per 16 key channels
+// tokens 0 .. 15 and 16 .. 31 of -W, of Q' and of K.  Then e^{b_end}.
+static inline __host__ __device__ int64_t delta_ws_floats(int dkp) { return (int64_t)dkp * (3 * DELTA_C + 1); }
+static inline __host__ __device__ constexpr int delta_piece(int i, int x) { return (6 * i + x) * 64; }
 __device__ __forceinline__ int64_t delta_chunk(const DeltaArgs& p, int seq, int c) { return p.seq_tok_start[seq] / DELTA_C + seq + c; }
 
 // log(1 + e^x) from the hardware's base-2 exponential and logarithm; what 1 + y rounds away is added back
@@ -222,12 +225,15 @@ __global__ __launch_bounds__(512, NK > 8 ? 2 : 4) void delta_prep_kernel(DeltaAr
 #pragma unroll
         for (int r = 0; r < 4; r++) Ms[(o + 4 * fg + r) * LA + o + fr] = xd[r];
     } else {
-        // (K e^{b_end - b})^T and e^{b_end}; 32 tokens of a channel side by side
-        float* kt = ws + 2 * C * DKP;
+        // (K e^{b_end - b})^T and e^{b_end}
 #pragma unroll 2
-        for (int i = tid - 128; i < C * DKP; i += NT - 128) {
-            const int t = i & 31, d = i >> 5;
-            kt[d * C + t] = ks[t * LQ + d] * ex2(bs[31 * LQ + d] - bs[t * LQ + d]);
+        for (int i = tid - 128; i < 2 * NK * 64; i += NT - 128) {
+            const int l = i & 63, sb = (i >> 6) & 1, d = 16 * (i >> 7) + (l & 15), t = 16 * sb + 4 * (l >> 4);
+            const float b_end = bs[31 * LQ + d];
+            f32x4 x;
+#pragma unroll
+            for (int r = 0; r < 4; r++) x[r] = ks[(t + r) * LQ + d] * ex2(b_end - bs[(t + r) * LQ + d]);
+            ((f32x4*)ws)[delta_piece(i >> 7, 4 + sb) + l] = x;
         }
         for (int d = tid - 128; d < DKP; d += NT - 128) ws[3 * C * DKP + d] = ex2(bs[31 * LQ + d]);
     }
@@ -296,8 +302,8 @@ __global__ __launch_bounds__(512, NK > 8 ? 2 : 4) void delta_prep_kernel(DeltaAr
         times(k, ba, q);
 #pragma unroll
         for (int tt = 0; tt < 2; tt++) {
-            *(f32x4*)(ws + (16 * tt + fr) * DKP + 16 * i + 4 * fg) = w[tt];
-            *(f32x4*)(ws + (C + 16 * tt + fr) * DKP + 16 * i + 4 * fg) = q[tt];
+            ((f32x4*)ws)[delta_piece(i, tt) + lane] = w[tt];
+            ((f32x4*)ws)[delta_piece(i, 2 + tt) + lane] = q[tt];
         }
     }
     for (int i = wave; i < nvb; i += NW) {                       // 16 value channels: U0 and O0
@@ -322,13 +328,12 @@ __global__ __launch_bounds__(512, NK > 8 ? 2 : 4) void delta_prep_kernel(DeltaAr
 }
 
 // ------------------------------------------------------------------------------------------
-// scan: grid (heads, slices of 64 / KSP value columns, sequences).  A wave keeps DK / KSP x 16 of the state in accumulators: 16 columns,
-// and with KSP > 1 (few heads and sequences) a part of the key channels — the parts' sums of U and O meet in LDS.
-// The next chunk's operands are on their way to registers while the state is updated.
+// scan: grid (heads, slices of value columns, sequences).  A wave keeps 16 columns of the state in accumulators: of all key channels (delta_scan_kernel), or of a part
+// of them (delta_scan_parts_kernel).
 // ------------------------------------------------------------------------------------------
 // Which sequence a workgroup takes: the shortest first, then the longest to the second shortest.  The chain of the longest one is what a launch lasts; started early it has
-// its CU to itself until workgroups have to share, and shares with the start of the shortest.  us a layer, order of the call -> here: 5 sequences of 300 .. 1900 tokens 249 -> 233,
-// 10 of 100 .. 900 and 24 of them a prompt 10080 -> 9750, 18680 -> 18010; longest first and shortest last 1 % behind at the first, equal at the others; equal lengths keep their order.
+// its CU to itself until workgroups have to share, and shares with the start of the shortest.  us a layer, order of the call -> here: 5 sequences of 300 .. 1900 tokens 125 -> 114,
+// 12 of them 274 -> 234, 24 of 100 .. 900 220 -> 194; equal lengths keep their order.
 // (Beyond 64 sequences, more than the lanes that rank them, the order of the call: there are chains enough to even out)
 __device__ __forceinline__ int delta_scan_seq(const int* seq_len, int i, int n_seqs) {
     if (n_seqs == 1 || n_seqs > DELTA_ORDERED) return i;
@@ -340,91 +345,107 @@ __device__ __forceinline__ int delta_scan_seq(const int* seq_len, int i, int n_s
     }
     return __builtin_amdgcn_readfirstlane(__builtin_ctzll(__ballot(rank == (i == 0 ? n_seqs - 1 : i - 1) && lane < n_seqs)));
 }
-template <int NK, int KSP> constexpr int delta_scan_lds_bytes() { return 4 * (2 * DELTA_C * (NK * 16 + 4) + NK * 16 * 36 + NK * 16 + (KSP > 1 ? DELTA_SCAN_WAVES * 1024 : 0)); }
+// Value column `col` of a chunk's U0, O0 and O, tokens 16 tt + 4 fg + r.  The descriptor ends with the sequence and columns beyond DV lie outside it: what is read
+// there is zero (U: the state's padding columns stay zero), and what is written there is dropped.
+struct DeltaRows { char* base; uint32_t pitch; };
+template <typename Rsrc> __device__ __forceinline__ f32x4 delta_rows_get(Rsrc rs, uint32_t at, uint32_t pitch) {
+    f32x4 x;
+#pragma unroll
+    for (int r = 0; r < 4; r++) x[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, at + r * pitch, 0, 0));
+    return x;
+}
+// (chunk's rows: a pitch is below 2^26 bytes.  readfirstlane: the compiler doesn't see that these are uniform, and loops over the lanes' descriptors)
+__device__ __forceinline__ auto delta_rows(const DeltaRows& w, int c0, int left) {
+    const uint64_t at = (uint64_t)(w.base + (int64_t)c0 * w.pitch);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)at), hi = __builtin_amdgcn_readfirstlane((uint32_t)(at >> 32));
+    return __builtin_amdgcn_make_buffer_rsrc((void*)((uint64_t)hi << 32 | lo), 0, __builtin_amdgcn_readfirstlane(max(min(left, DELTA_C), 0) * (int)w.pitch), 0x00020000);
+}
+template <typename Rsrc> __device__ __forceinline__ f32x4 buffer_f32x4(Rsrc rs, int lane_off, int off) {
+    union { f32x4 f; u32x4 u; } t;
+    t.u = __builtin_amdgcn_raw_buffer_load_b128(rs, lane_off, off, 0);
+    return t.f;
+}
+template <int N>      // key channels ch0 .. ch0 + 16 N - 1 of a lane's column
+__device__ __forceinline__ void delta_state_in(const DeltaArgs& p, const float* st, int ch0, int fg, int col, bool fresh, f32x4 (&S)[N]) {
+    const int sc = min(col, p.DVp - 1);              // (clamped addresses instead of branches)
+#pragma unroll
+    for (int i = 0; i < N; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int row = ch0 + 16 * i + 4 * fg + r;
+            const float x = st[min(row, p.DK - 1) * p.DVp + sc];
+            S[i][r] = !fresh && col < p.DVp && row < p.DK ? x : 0.f;
+        }
+}
+template <int N>
+__device__ __forceinline__ void delta_state_out(const DeltaArgs& p, float* st, int ch0, int fg, int col, const f32x4 (&S)[N]) {
+    int so = 4 * fg * p.DVp + col;
+    asm volatile("" : "+v"(so));                     // (or addresses are kept in registers all along)
+    st += ch0 * p.DVp;
+#pragma unroll
+    for (int i = 0; i < N; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            if (col < p.DVp && ch0 + 16 * i + 4 * fg + r < p.DK) (st + (16 * i + r) * p.DVp)[so] = S[i][r];
+}
 
-template <int NK, int KSP>
+// All key channels of 16 columns a wave: a chunk's operands are in LDS for the workgroup's 64 columns, as they lie in scratch (three workgroups a CU; with padded rows
+// two: 16 x 900 tokens 250 -> 242 us a layer, 32 x 512 322 -> 272).  192 products of 32 cycles a chunk bound a wave.
+template <int NK> constexpr int delta_scan_lds_bytes() { return 4 * NK * 16 * (3 * DELTA_C + 1); }
+
+template <int NK>
 __global__ __launch_bounds__(DELTA_SCAN_WAVES * 64, NK > 8 ? 1 : 3) void delta_scan_kernel(DeltaArgs p) {
-    constexpr int NW = DELTA_SCAN_WAVES, C = DELTA_C, DKP = NK * 16, LQ = DKP + 4, LK = 36, NT = NW * 64, NKW = NK / KSP, NCG = NW / KSP;
+    constexpr int NW = DELTA_SCAN_WAVES, C = DELTA_C, DKP = NK * 16, NT = NW * 64;
     const int h = blockIdx.x, seq = delta_scan_seq(p.seq_len, (int)blockIdx.z, (int)gridDim.z);
     const int n = p.seq_len[seq];
     if (n < p.len_lo || n > p.len_hi) return;
     extern __shared__ __attribute__((aligned(16))) float dl_sm[];
-    float* wl = dl_sm;                   // [C][LQ]   -W
-    float* ql = wl + C * LQ;             // [C][LQ]   Q'
-    float* kl = ql + C * LQ;             // [DKP][LK] (K e^{b_end - b})^T
-    float* dl = kl + DKP * LK;           // [DKP]     e^{b_end}
-    f32x4* xb = (f32x4*)(dl + DKP);      // KSP > 1: [part][column group][U, U, O, O][lane]
+    f32x4* ol = (f32x4*)dl_sm;           // the chunk as it lies in scratch
+    float* dl = dl_sm + 3 * C * DKP;     // [DKP]     e^{b_end}
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int fr = lane & 15, fg = lane >> 4;
-    const int cg = wave % NCG, kq = wave / NCG, ch0 = kq * NKW * 16;       // this wave's column group, part and first key channel
-    const int col = (blockIdx.y * NCG + cg) * 16 + fr;
-    const bool live = col < p.DV, slive = col < p.DVp;
-    const int64_t tok0 = p.seq_tok_start[seq];
-    const bool fresh = p.seq_pos[seq] == 0;
+    const int col = (blockIdx.y * NW + wave) * 16 + fr;
     float* st = p.state + (int64_t)p.seq_slot[seq] * p.slot_stride + (int64_t)h * p.DK * p.DVp;
-    f32x4 S[NKW];
-    {   // (clamped addresses instead of branches)
-        const int sc = min(col, p.DVp - 1);
-#pragma unroll
-        for (int i = 0; i < NKW; i++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int row = ch0 + 16 * i + 4 * fg + r;
-                const float x = st[min(row, p.DK - 1) * p.DVp + sc];
-                S[i][r] = !fresh && slive && row < p.DK ? x : 0.f;
-            }
-    }
+    f32x4 S[NK];
+    delta_state_in(p, st, 0, fg, col, p.seq_pos[seq] == 0, S);
     constexpr int E = 3 * C * DKP / 4, NL = E / NT;              // 16-byte pieces of a chunk's operands, per thread
-    static_assert(NKW % 2 == 0 && NW % KSP == 0, "pairs of 16 channels");
-    static_assert(E % (3 * NT) == 0 && NT >= DKP, "whole pieces, one decay per thread");
+    static_assert(E % NT == 0 && NT >= DKP, "whole pieces, one decay per thread");
     const int64_t stride = p.H * delta_ws_floats(DKP);
     const float* src = p.ws + (delta_chunk(p, seq, 0) * p.H + h) * delta_ws_floats(DKP);
     f32x4 rg[NL], u[2], o[2];
     float rd = 0.f;
-    const int ld = (int)p.ld, old = (int)p.o_ld;
-    const char* vb = (const char*)(p.v + tok0 * p.ld + (int64_t)h * p.DV);
-    char* ob = (char*)(p.o + tok0 * p.o_ld + (int64_t)h * p.DV);
-    const uint32_t cb = 4 * min(col, p.DV - 1);
-    auto fetch = [&]() {
+    const int64_t tok0 = p.seq_tok_start[seq];
+    const DeltaRows vr{(char*)(p.v + tok0 * p.ld + (int64_t)h * p.DV), 4 * (uint32_t)p.ld}, orow{(char*)(p.o + tok0 * p.o_ld + (int64_t)h * p.DV), 4 * (uint32_t)p.o_ld};
+    const uint32_t cb = col < p.DV ? 4 * col : 1u << 31;
+    constexpr int Q = NK / 2;                                    // a chunk's loads go out in as many portions, between the products of two state tiles each
+    auto fetch = [&](int c0, int part) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < NL; i++) rg[i] = ((const f32x4*)src + i * NT)[tid];
-        rd = src[3 * C * DKP + min(tid, DKP - 1)];
-    };
-    // U0 and O0 of 32 tokens.  Beyond the sequence's end the last token is read again: finite, against zero columns of K, never stored.
-    auto fetch_uo = [&](const char* v, const char* oc, int left) {
-        if (KSP > 1 && kq > 0) {         // (wave-uniform: the first part starts from U0 and O0)
-            u[0] = u[1] = o[0] = o[1] = f32x4{0.f, 0.f, 0.f, 0.f};
-            return;
+        for (int i = 0; i < NL; i++) if (i * Q / NL == part) rg[i] = ((const f32x4*)src + i * NT)[tid];
+        if (part == 0) {
+            const auto rv = delta_rows(vr, c0, n - c0);
+            rd = src[3 * C * DKP + min(tid, DKP - 1)];
+#pragma unroll
+            for (int tt = 0; tt < 2; tt++) u[tt] = delta_rows_get(rv, (16 * tt + 4 * fg) * vr.pitch + cb, vr.pitch);
         }
+        if (part == Q - 1) {
+            const auto ro = delta_rows(orow, c0, n - c0);
 #pragma unroll
-        for (int tt = 0; tt < 2; tt++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const uint32_t t = min(16 * tt + 4 * fg + r, left - 1);
-                const float x = *(const float*)(v + (t * (uint32_t)ld * 4 + cb));
-                u[tt][r] = live ? x : 0.f;                       // (the state's padding columns stay zero)
-                o[tt][r] = *(const float*)(oc + (t * (uint32_t)old * 4 + cb));
-            }
+            for (int tt = 0; tt < 2; tt++) o[tt] = delta_rows_get(ro, (16 * tt + 4 * fg) * orow.pitch + cb, orow.pitch);
+        }
     };
-    fetch();
-    fetch_uo(vb, ob, n);
+#pragma unroll
+    for (int i = 0; i < Q; i++) fetch(0, i);
     for (int c0 = 0; c0 < n; c0 += C) {
         __syncthreads();                                         // the previous chunk's readers are done
-        float *w0 = wl + tid / (DKP / 4) * LQ + tid % (DKP / 4) * 4, *k0 = kl + (tid >> 3) * LK + (tid & 7) * 4;
 #pragma unroll
-        for (int i = 0; i < NL; i++)
-            if (i < NL / 3 * 2) *(f32x4*)(w0 + i * (NT / (DKP / 4)) * LQ) = rg[i];
-            else *(f32x4*)(k0 + (i - NL / 3 * 2) * (NT / 8) * LK) = rg[i];
+        for (int i = 0; i < NL; i++) ol[i * NT + tid] = rg[i];
         if (tid < DKP) dl[tid] = rd;
         __syncthreads();
 #pragma unroll
-        for (int i = 0; i < NKW; i++) {
+        for (int i = 0; i < NK; i++) {
             f32x4 a[4];
 #pragma unroll
-            for (int tt = 0; tt < 2; tt++) {
-                a[tt] = *(const f32x4*)(wl + (16 * tt + fr) * LQ + ch0 + 16 * i + 4 * fg);
-                a[2 + tt] = *(const f32x4*)(ql + (16 * tt + fr) * LQ + ch0 + 16 * i + 4 * fg);
-            }
+            for (int x = 0; x < 4; x++) a[x] = ol[delta_piece(i, x) + lane];
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 u[0] = mfma_f32(a[0][r], S[i][r], u[0]); u[1] = mfma_f32(a[1][r], S[i][r], u[1]);
@@ -432,42 +453,28 @@ __global__ __launch_bounds__(DELTA_SCAN_WAVES * 64, NK > 8 ? 1 : 3) void delta_s
             }
             if (i & 1) __builtin_amdgcn_sched_barrier(0);        // (or all reads are hoisted to the front, and registers spill)
         }
-        if constexpr (KSP > 1) {
-            f32x4* x = xb + (kq * NCG + cg) * 256 + lane;
-            x[0] = u[0]; x[64] = u[1]; x[128] = o[0]; x[192] = o[1];
-            __syncthreads();
-            u[0] = u[1] = o[0] = o[1] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int q = 0; q < KSP; q++) {
-                const f32x4* y = xb + (q * NCG + cg) * 256 + lane;
-                u[0] += y[0]; u[1] += y[64];
-                if (kq == 0) o[0] += y[128];                     // (the first two parts store 16 tokens each)
-                if (kq == 1) o[1] += y[192];
-            }
-        }
+        const auto ro = delta_rows(orow, c0, n - c0);
 #pragma unroll
         for (int tt = 0; tt < 2; tt++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int t = 16 * tt + 4 * fg + r;
-                if (live && c0 + t < n && (KSP == 1 || kq == tt)) *(float*)(ob + ((uint32_t)t * (uint32_t)old * 4 + cb)) = o[tt][r];
+                const float x = o[tt][r];        // (a bit_cast of the vector's element itself takes the first)
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, x), ro, (16 * tt + 4 * fg + r) * orow.pitch + cb, 0, 0);
             }
         f32x4 ub[2] = {u[0], u[1]};
         __builtin_amdgcn_sched_barrier(0);
         const bool more = c0 + C < n;                            // (the last chunk is fetched once more instead of a branch)
-        src += more ? stride : 0; vb += more ? (int64_t)C * ld * 4 : 0; ob += more ? (int64_t)C * old * 4 : 0;
-        fetch();
-        fetch_uo(vb, ob, more ? n - c0 - C : n - c0);
-        __builtin_amdgcn_sched_barrier(0);
+        src += more ? stride : 0;
 #pragma unroll
-        for (int i = 0; i < NKW; i += 2) {
+        for (int i = 0; i < NK; i += 2) {
             f32x4 a[2][2];
 #pragma unroll
             for (int x = 0; x < 2; x++)
 #pragma unroll
-                for (int sb = 0; sb < 2; sb++) a[x][sb] = *(const f32x4*)(kl + (ch0 + 16 * (i + x) + fr) * LK + 16 * sb + 4 * fg);
-            S[i] *= *(const f32x4*)(dl + ch0 + 16 * i + 4 * fg);
-            S[i + 1] *= *(const f32x4*)(dl + ch0 + 16 * (i + 1) + 4 * fg);
+                for (int sb = 0; sb < 2; sb++) a[x][sb] = ol[delta_piece(i + x, 4 + sb) + lane];
+            S[i] *= *(const f32x4*)(dl + 16 * i + 4 * fg);
+            S[i + 1] *= *(const f32x4*)(dl + 16 * (i + 1) + 4 * fg);
+            fetch(more ? c0 + C : c0, i / 2);
 #pragma unroll
             for (int sb = 0; sb < 2; sb++)
 #pragma unroll
@@ -475,14 +482,139 @@ __global__ __launch_bounds__(DELTA_SCAN_WAVES * 64, NK > 8 ? 1 : 3) void delta_s
             __builtin_amdgcn_sched_barrier(0);
         }
     }
-    int so = 4 * fg * p.DVp + col;
-    asm volatile("" : "+v"(so));                                 // (or addresses are kept in registers all along)
-    st += ch0 * p.DVp;
+    delta_state_out(p, st, 0, fg, col, S);
+}
+
+// Key channels over the KSP waves of a workgroup that has 16 columns: a chunk's operands belong to one wave each and go from scratch to its registers, a chunk ahead and
+// between the products (in front of them the workgroup's 52 KB kept its waves from their first product for 360 .. 1070 cycles).  The waves' sums of U and O meet in LDS:
+// U's on their way while O is multiplied, O's a chunk later.  Bound by the chain of a sequence: a chunk of a head of 128 is 48 products of 32 cycles in 2600 .. 2800 (1.1 us),
+// the rest the exchange (150 to write and meet, 140 to add) and what is issued beside the products.  With operands through LDS and their loads behind the products of U
+// and O it was 2.6 us: 1 x 1900 tokens 157 -> 72 us a layer, 5 x 300 .. 1900 195 -> 115.
+template <int NK, int KSP>
+__global__ __launch_bounds__(KSP * 64, 2) void delta_scan_parts_kernel(DeltaArgs p) {
+    constexpr int C = DELTA_C, DKP = NK * 16, N = NK / KSP;
+    const int h = blockIdx.x, seq = delta_scan_seq(p.seq_len, (int)blockIdx.z, (int)gridDim.z);
+    const int n = p.seq_len[seq];
+    if (n < p.len_lo || n > p.len_hi) return;
+    __shared__ f32x4 xb[2][KSP][4][64];      // [chunk & 1][part][U, U, O, O]
+    const int lane = threadIdx.x & 63, kq = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int fr = lane & 15, fg = lane >> 4, col = blockIdx.y * 16 + fr, ch0 = kq * N * 16;
+    float* st = p.state + (int64_t)p.seq_slot[seq] * p.slot_stride + (int64_t)h * p.DK * p.DVp;
+    f32x4 S[N];
+    delta_state_in(p, st, ch0, fg, col, p.seq_pos[seq] == 0, S);
+    const int64_t stride = p.H * delta_ws_floats(DKP), tok0 = p.seq_tok_start[seq];
+    const float* src = p.ws + (delta_chunk(p, seq, 0) * p.H + h) * delta_ws_floats(DKP);
+    const DeltaRows vr{(char*)(p.v + tok0 * p.ld + (int64_t)h * p.DV), 4 * (uint32_t)p.ld}, orow{(char*)(p.o + tok0 * p.o_ld + (int64_t)h * p.DV), 4 * (uint32_t)p.o_ld};
+    const uint32_t cb = col < p.DV ? 4 * col : 1u << 31;
+    // what U and O start from is dealt over the parts: U's two pieces to the first two, O's to the next two or the same
+    constexpr int NI = KSP >= 4 ? 1 : 2;
+    const int stt = kq & 1;
+    const DeltaRows first = NI == 2 || kq < 2 ? vr : orow;
+    const uint32_t at_v = (16 * stt + 4 * fg) * first.pitch + cb, at_o = (16 * stt + 4 * fg) * orow.pitch + cb;
+    // ... and what becomes of O: two parts store 16 tokens each, or four 8
+    constexpr int NS = KSP == 2 ? 4 : 2;
+    const int ott = KSP == 2 ? kq : (kq >> 1) & 1, or0 = KSP == 2 ? 0 : 2 * (kq & 1);
+    const uint32_t at_s = KSP <= 4 || kq < 4 ? (16 * ott + 4 * fg + or0) * orow.pitch + cb : 1u << 31;
+    struct Chunk { f32x4 op[N][6], d[N], start[NI]; };
+    auto fetch_start = [&](Chunk& k, int c0) __attribute__((always_inline)) {
+        k.start[0] = delta_rows_get(delta_rows(first, c0, n - c0), at_v, first.pitch);
+        if constexpr (NI == 2) k.start[1] = delta_rows_get(delta_rows(orow, c0, n - c0), at_o, orow.pitch);
+    };
+    auto fetch_op = [&](Chunk& k, int j) __attribute__((always_inline)) {      // load j of 7 N
+        const auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)src, 0, 4 * (int)delta_ws_floats(DKP), 0x00020000);
+        const int x = j / N, i = j % N;
+        if (x < 6) k.op[i][x] = buffer_f32x4(rs, lane * 16, 16 * delta_piece(kq * N + i, x));
+        else if (x == 6) k.d[i] = buffer_f32x4(rs, fg * 16, 4 * (3 * C * DKP + ch0 + 16 * i));
+    };
+    const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto barrier = [&]() __attribute__((always_inline)) {      // (without the wait for loads on their way)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    float oq[KSP][NS];
+    auto read_o = [&](int turn) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < NKW; i++)
+        for (int q = 0; q < KSP; q++)
 #pragma unroll
-        for (int r = 0; r < 4; r++)
-            if (slive && ch0 + 16 * i + 4 * fg + r < p.DK) (st + (16 * i + r) * p.DVp)[so] = S[i][r];
+            for (int r = 0; r < NS; r++) oq[q][r] = ((const float*)&xb[turn][q][2 + ott][lane])[or0 + r];
+    };
+    auto store_o = [&](int c0) __attribute__((always_inline)) {      // (c0 < 0: none)
+        const auto ro = delta_rows(orow, c0, c0 < 0 ? 0 : n - c0);
+#pragma unroll
+        for (int r = 0; r < NS; r++) {
+            float y = oq[0][r];
+#pragma unroll
+            for (int q = 1; q < KSP; q++) y += oq[q][r];
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, y), ro, at_s + r * orow.pitch, 0, 0);
+        }
+    };
+    auto step = [&](Chunk& k, Chunk& next, int c0, int turn) __attribute__((always_inline)) {
+        const bool more = c0 + C < n;
+        src += more ? stride : 0;                                // (the last chunk is fetched once more instead of a branch)
+        f32x4 u[2], o[2], uq[KSP][2];
+#pragma unroll
+        for (int tt = 0; tt < 2; tt++) {
+            u[tt] = (NI == 2 || kq < 2) && stt == tt ? k.start[0] : zero;
+            o[tt] = NI == 2 ? (stt == tt ? k.start[NI - 1] : zero) : (kq == 2 + tt ? k.start[0] : zero);
+        }
+#pragma unroll
+        for (int i = 0; i < N; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                u[0] = mfma_f32(k.op[i][0][r], S[i][r], u[0]); u[1] = mfma_f32(k.op[i][1][r], S[i][r], u[1]);
+                if (i == 0 && r == 1) fetch_start(next, more ? c0 + C : c0);
+                if (r % 2 == 0) fetch_op(next, 2 * i + r / 2);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        xb[turn][kq][0][lane] = u[0]; xb[turn][kq][1][lane] = u[1];
+        barrier();                                               // (one a chunk: who writes this half of xb again has passed the next)
+#pragma unroll
+        for (int q = 0; q < KSP; q++) { uq[q][0] = xb[turn][q][0][lane]; uq[q][1] = xb[turn][q][1][lane]; }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < N; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                o[0] = mfma_f32(k.op[i][2][r], S[i][r], o[0]); o[1] = mfma_f32(k.op[i][3][r], S[i][r], o[1]);
+                if (r % 2 == 0) fetch_op(next, 2 * N + 2 * i + r / 2);
+                if (i == N - 1 && r == 1) read_o(turn ^ 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        u[0] = uq[0][0]; u[1] = uq[0][1];
+#pragma unroll
+        for (int q = 1; q < KSP; q++) { u[0] += uq[q][0]; u[1] += uq[q][1]; }
+#pragma unroll
+        for (int i = 0; i < N; i++) S[i] *= k.d[i];
+#pragma unroll
+        for (int sb = 0; sb < 2; sb++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+#pragma unroll
+                for (int i = 0; i < N; i++) S[i] = mfma_f32(k.op[i][4 + sb][r], u[sb][r], S[i]);
+#pragma unroll
+                for (int j = 0; j < 3 * N; j++) if (j * 8 / (3 * N) == 4 * sb + r) fetch_op(next, 4 * N + j);
+                if (sb == 0 && r == 1) { xb[turn][kq][2][lane] = o[0]; xb[turn][kq][3][lane] = o[1]; }
+                if (sb == 0 && r == 3) store_o(c0 - C);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+    };
+    Chunk a, b;
+    fetch_start(a, 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < 7 * N; j++) fetch_op(a, j);
+    int c0 = 0;
+    for (;;) {
+        step(a, b, c0, 0);
+        if (c0 + C >= n) { barrier(); read_o(0); break; }
+        c0 += C;
+        step(b, a, c0, 1);
+        if (c0 + C >= n) { barrier(); read_o(1); break; }
+        c0 += C;
+    }
+    store_o(c0);
+    delta_state_out(p, st, ch0, fg, col, S);
 }
 
 // ------------------------------------------------------------------------------------------

@@ -32,36 +32,39 @@ static void prep(hipStream_t st, const DeltaArgs& p, dim3 grid) {
 void delta_prep_launch(hipStream_t st, const DeltaArgs& p, dim3 grid, int nk) {
     if (nk == 2) prep<2>(st, p, grid); else if (nk == 4) prep<4>(st, p, grid); else if (nk == 8) prep<8>(st, p, grid); else prep<16>(st, p, grid);
 }
-template <int NK, int KSP>
+template <int NK>
 static void scan(hipStream_t st, const DeltaArgs& p, int n_seqs) {
-    constexpr int lds = delta_scan_lds_bytes<NK, KSP>();
-    NVL_LDS_ATTR((delta_scan_kernel<NK, KSP>), lds);
-    hipLaunchKernelGGL((delta_scan_kernel<NK, KSP>), dim3(p.H, cdiv(p.DV, 16 * DELTA_SCAN_WAVES / KSP), n_seqs), dim3(DELTA_SCAN_WAVES * 64), lds, st, p);
+    constexpr int lds = delta_scan_lds_bytes<NK>();
+    NVL_LDS_ATTR((delta_scan_kernel<NK>), lds);
+    hipLaunchKernelGGL((delta_scan_kernel<NK>), dim3(p.H, cdiv(p.DV, 16 * DELTA_SCAN_WAVES), n_seqs), dim3(DELTA_SCAN_WAVES * 64), lds, st, p);
 }
-// Parts of the key channels (KSP): more parts shorten the chain of a sequence's chunks, whose fp32 products bound a wave, and cost each of them an exchange.
-// us, fitted to 1 .. 64 sequences of 100 .. 1900 tokens x 16 heads of 128, good to 20 %: the longest sequence's chain, all chunks at the chip's rate, the larger of them
-// and a quarter of the other.  Sequences of several lengths, longest first, fill the chip's gaps with the short ones; of one length they end together.
-// One / two / four parts, ms a prompt: 1 x 1900 6.5 / 5.9 / 5.6; 5 x 300..1900 12.5 / 11.9 / 11.7; 12 x 300..1900 22.9 / 22.3 / 23.0; 10 x 100..900 10.0 / 9.7 / 9.9; 16 x 900 25.6 / 26.2 / 27.4.
-static double scan_cost(const DeltaArgs& p, int n_seqs, int nk, int ksp, int max_len, int tokens) {
-    const double size = nk / 8.0, heads = p.H * cdiv(p.DV, 64) / 2.0;
-    const double chain = cdiv(max_len, DELTA_C) * (1.95 + size * 2.55 / ksp);
-    const double ragged = n_seqs <= DELTA_ORDERED ? 0.4 + 0.6 * tokens / ((double)n_seqs * max_len) : 1.0;
-    const double all = heads * ((double)tokens / DELTA_C + 0.5 * n_seqs) * (size * 0.0225 + 0.0105 * ksp) * ragged;
-    return std::max(chain, all) + 0.25 * std::min(chain, all);
+template <int NK, int KSP>
+static void scan_parts(hipStream_t st, const DeltaArgs& p, int n_seqs) {
+    hipLaunchKernelGGL((delta_scan_parts_kernel<NK, KSP>), dim3(p.H, cdiv(p.DV, 16), n_seqs), dim3(KSP * 64), 0, st, p);
 }
-template <int NK, int... PARTS>
+// All key channels a wave (64 columns a workgroup, operands shared through LDS), or the channels over the KSP waves of a workgroup of 16 columns: a chunk's step is three
+// times as short, and each costs an exchange and its operands four reads from L2.  us: the longest sequence's chain, all chunks at the chip's rate, the larger of them and
+// 0.4 of the other; fitted to 1 .. 64 sequences of 100 .. 1900 tokens x 2048 columns of heads of 64, 128 and 256, good to 20 %.
+// Heads of 128, whole / parts, us a layer: 1 x 1900 220 / 72; 4 x 900 119 / 71; 8 x 900 145 / 153; 12 x 900 222 / 214; 16 x 900 242 / 280; 32 x 512 272 / 310; 64 x 200 246 / 315;
+// 5 x 300..1900 244 / 115; 10 x 100..900 135 / 92; 12 x 300..1900 312 / 235.  Heads of 64: 1 x 1900 135 / 64, 4 x 900 79 / 56, 16 x 900 180 / 227; of 256: 432 / 119, 225 / 137, 495 / 579.
+struct ScanCost { double start, step, chunk; };          // of the chain: before the first chunk, a chunk; of all: a chunk of 32 columns' worth of a head
+static double scan_cost(const DeltaArgs& p, int n_seqs, const ScanCost& k, int max_len, int tokens) {
+    const double chain = k.start + k.step * cdiv(max_len, DELTA_C);
+    const double all = k.chunk * p.H * cdiv(p.DV, 64) / 2.0 * ((double)tokens / DELTA_C + n_seqs);
+    return std::max(chain, all) + 0.4 * std::min(chain, all);
+}
+template <int NK, int KSP>
 static void scan_shape(hipStream_t st, const DeltaArgs& p, int n_seqs, int max_len, int tokens) {
-    int best = 1;
-    double t = scan_cost(p, n_seqs, NK, 1, max_len, tokens);
-    auto consider = [&](int ksp) { const double c = scan_cost(p, n_seqs, NK, ksp, max_len, tokens); if (c < 0.95 * t) { t = c; best = ksp; } };
-    (consider(PARTS), ...);
-    if (best == 1) { scan<NK, 1>(st, p, n_seqs); return; }
-    ((best == PARTS ? scan<NK, PARTS>(st, p, n_seqs) : void()), ...);
+    constexpr double size = NK / 8.0;
+    const ScanCost whole{8.0, 0.4 + 3.3 * size, 0.008 + 0.023 * size};
+    const ScanCost parts = KSP == 2 ? ScanCost{5.0, 1.0, 0.029} : KSP == 4 ? ScanCost{5.0, 1.1, 0.036} : ScanCost{8.0, 1.85, 0.075};
+    if (scan_cost(p, n_seqs, parts, max_len, tokens) < scan_cost(p, n_seqs, whole, max_len, tokens)) scan_parts<NK, KSP>(st, p, n_seqs);
+    else scan<NK>(st, p, n_seqs);
 }
 void delta_scan_launch(hipStream_t st, const DeltaArgs& p, int n_seqs, int nk, int max_len, int tokens) {
-    if (nk == 2) scan<2, 1>(st, p, n_seqs);
+    if (nk == 2) scan<2>(st, p, n_seqs);
     else if (nk == 4) scan_shape<4, 2>(st, p, n_seqs, max_len, tokens);
-    else if (nk == 8) scan_shape<8, 2, 4>(st, p, n_seqs, max_len, tokens);
-    else scan_shape<16, 2, 4>(st, p, n_seqs, max_len, tokens);
+    else if (nk == 8) scan_shape<8, 4>(st, p, n_seqs, max_len, tokens);
+    else scan_shape<16, 8>(st, p, n_seqs, max_len, tokens);
 }
 }  // namespace nvl
