@@ -5,7 +5,7 @@
 //
 //   delta_step_kernel   token by token, the state streamed once per token (decode).  FUSED (one token per sequence): the short
 //                       convolutions, the low-rank decay and gate projections, the head norm and the output gate in the same launch.
-//   delta_prep_kernel   32 tokens of one head, independent of the state that enters them (prefill, all chunks at once).
+//   delta_prep_kernel   32 tokens of one head, independent of the state that enters them (prefill; a workgroup goes from chunk to chunk).
 //   delta_scan_kernel, delta_scan_parts_kernel   carry the state through the chunks of a sequence: three products per chunk.
 //
 // Chunk form.  With b_t = the inclusive sum of log a inside the chunk and S_in the state that enters it:
@@ -14,8 +14,8 @@
 //     S_out = diag(e^{b_end}) S_in + sum_s (k_s e^{b_end - b_s}) u_s^T
 // With T = (I + diag(beta) M)^-1 diag(beta):  U = U0 - W S_in,  U0 = T V,  W = T (K e^b);  O = O0 + Q' S_in,  O0 = (A T) V,
 // Q' = Q e^b - (A T) (K e^b).  prep leaves -W, Q', (K e^{b_end - b})^T and e^{b_end} in scratch, U0 in the place of v and O0 in the place of o.
-// Every exponent that is evaluated is <= 0: a decay per channel cannot be split into e^{b_t} e^{-b_s}, so the two 16 x 16 diagonal
-// blocks of A and M are summed pair by pair, and the block below the diagonal takes token 15's sums as its reference.  T is built
+// Every exponent that is evaluated is <= 0: a decay per channel cannot be split into e^{b_t} e^{-b_s}, so the four 8 x 8 diagonal
+// blocks of A and M are summed pair by pair, and the blocks below take the sums of the token before their rows (7, 15, 23) as their reference.  T is built
 // block by block from exact inverses: the powers of M that a series would need can be far larger than T itself.
 // Products are v_mfma_f32_16x16x4_f32: operand element i of lane group g stands for k = 16 n + 4 g + i on both sides, so that an
 // accumulator (lane = column, rows 4 g + r) is the B operand of the next product as it stands.
@@ -48,6 +48,10 @@ struct DeltaArgs {
     const float* norm_w; float eps; void* out; int64_t out_ld;
 };
 
+// Products whose results are stored next.  The compiler spaces the store from the product by counting instructions of any kind; where an earlier store and a lane read
+// were among them, the 11 it counted were too few with two workgroups a CU, and the last four columns of the tile were stored as they had been.
+__device__ __forceinline__ void products_done(f32x4& a, f32x4& b, f32x4& c, f32x4& d) { asm volatile("s_nop 15" : "+v"(a), "+v"(b), "+v"(c), "+v"(d)); }
+
 constexpr int DELTA_C = 32;            // tokens per chunk
 constexpr int DELTA_ORDERED = 64;       // sequences that the scan takes in the order of their lengths, at most
 constexpr int DELTA_SCAN_WAVES = 4;    // of a workgroup of the scan
@@ -63,18 +67,84 @@ __device__ __forceinline__ float delta_softplus(float x) {
     return fmaxf(x, 0.f) + fmaf(0.6931471805599453f, __builtin_amdgcn_logf(u), (y - (u - 1.0f)) * __builtin_amdgcn_rcpf(u));
 }
 
+// Rows of a chunk, from its first.  The descriptor ends with the sequence and columns beyond a head lie outside it (OUTSIDE): what is read there is zero, and what is
+// written there is dropped.
+struct DeltaRows { char* base; uint32_t pitch; };
+constexpr uint32_t DELTA_OUTSIDE = 1u << 31;
+// (a chunk's rows are below 2^31 bytes.  readfirstlane: the compiler doesn't see that these are uniform, and loops over the lanes' descriptors)
+__device__ __forceinline__ auto delta_rows(const DeltaRows& w, int64_t row, int rows) {
+    const uint64_t at = (uint64_t)(w.base + row * w.pitch);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)at), hi = __builtin_amdgcn_readfirstlane((uint32_t)(at >> 32));
+    return __builtin_amdgcn_make_buffer_rsrc((void*)((uint64_t)hi << 32 | lo), 0, __builtin_amdgcn_readfirstlane(max(min(rows, DELTA_C), 0) * (int)w.pitch), 0x00020000);
+}
+template <typename Rsrc> __device__ __forceinline__ float buffer_f32(Rsrc rs, uint32_t at) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, at, 0, 0)); }
+template <typename Rsrc> __device__ __forceinline__ f32x4 buffer_f32x4(Rsrc rs, int lane_off, int off) {
+    union { f32x4 f; u32x4 u; } t;
+    t.u = __builtin_amdgcn_raw_buffer_load_b128(rs, lane_off, off, 0);
+    return t.f;
+}
+template <typename Rsrc> __device__ __forceinline__ void buffer_put(Rsrc rs, uint32_t at, float x) { __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, x), rs, at, 0, 0); }
+template <typename Rsrc> __device__ __forceinline__ void buffer_put4(Rsrc rs, int lane_off, int off, f32x4 x) {
+    union { f32x4 f; u32x4 u; } t; t.f = x;
+    __builtin_amdgcn_raw_buffer_store_b128(t.u, rs, lane_off, off, 0);
+}
+template <typename Rsrc> __device__ __forceinline__ f32x4 delta_rows_get(Rsrc rs, uint32_t at, uint32_t pitch) {       // a column of four rows
+    f32x4 x;
+#pragma unroll
+    for (int r = 0; r < 4; r++) x[r] = buffer_f32(rs, at + r * pitch);
+    return x;
+}
+
 // ------------------------------------------------------------------------------------------
-// prep: grid (heads, sequences, chunks), 8 waves
+// prep: grid (heads, workgroups that share its chunks), 8 waves.  Bound by what it moves, 145 KB a chunk of a head of 128 (q, k, v, z in, five operands out): 5.3 TB/s while
+// two workgroups a CU go from chunk to chunk.  They wait for little but stores because a chunk's loads leave when the one before has read its registers, and because
+// pairs are summed one by one inside blocks of 8 tokens only (of 16: 8500 of 46000 cycles a chunk, and two of eight waves had the products as well).
+// us a layer, a workgroup per chunk and blocks of 16 -> here: 5 x 300 .. 1900 tokens x 16 heads 143 -> 109, 10 x 100 .. 900 134 -> 90, 16 x 900 370 -> 290.
 // ------------------------------------------------------------------------------------------
 template <int NK> constexpr int delta_prep_lds_bytes() { return 4 * (3 * DELTA_C * (NK * 16 + 4) + 2 * DELTA_C * 36 + DELTA_C + 512); }
+// The chunks of all sequences that a launch serves, from the last to the first: the scan begins with those that were written last
+struct DeltaChunk { int seq, tok0, rows; int64_t at; };       // sequence, first token, tokens; place in scratch
+struct DeltaChunks {
+    const int *seq_len, *seq_tok_start;
+    int n_seqs, len_lo, len_hi;
+    int first, len, tok0, count, end;    // 64 sequences from `first` on: this lane's, its chunks, and all from there on
+    __device__ __forceinline__ DeltaChunks(const DeltaArgs& p, int n) : seq_len(p.seq_len), seq_tok_start(p.seq_tok_start), n_seqs(n), len_lo(p.len_lo), len_hi(p.len_hi) { load((n - 1) & ~63, 0); }
+    __device__ __forceinline__ void load(int f, int behind) {
+        const int lane = threadIdx.x & 63;
+        len = f + lane < n_seqs ? seq_len[f + lane] : 0;
+        tok0 = f + lane < n_seqs ? seq_tok_start[f + lane] : 0;
+        first = f;
+        count = len >= len_lo && len <= len_hi ? (len + DELTA_C - 1) / DELTA_C : 0;
+        end = count;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) { const int v = __shfl_down(end, o, 64); if (lane + o < 64) end += v; }
+        end += behind;
+    }
+    __device__ __forceinline__ bool find(int j, DeltaChunk& k) {         // chunk j, or false: there are no more (j grows from call to call)
+        for (;;) {
+            const unsigned long long m = __ballot(end > j);
+            if (m) {
+                const int l = 63 - __builtin_clzll(m), c = __builtin_amdgcn_readlane(end, l) - 1 - j, t = __builtin_amdgcn_readlane(tok0, l);
+                k.seq = first + l;
+                k.tok0 = t + c * DELTA_C;
+                k.rows = min(DELTA_C, __builtin_amdgcn_readlane(len, l) - c * DELTA_C);
+                k.at = t / DELTA_C + k.seq + c;
+                return true;
+            }
+            if (first == 0) return false;
+            load(first - 64, __builtin_amdgcn_readlane(end, 0));
+        }
+    }
+};
 
-template <int NK>
-__global__ __launch_bounds__(512, NK > 8 ? 2 : 4) void delta_prep_kernel(DeltaArgs p) {
+template <int NK, bool VEC>           // VEC: DeltaArgs::vec4 and vec4v
+__global__ __launch_bounds__(512, NK > 8 ? 2 : 4) void delta_prep_kernel(DeltaArgs p, int n_seqs) {
     constexpr int C = DELTA_C, DKP = NK * 16, LQ = DKP + 4, LA = 36, NT = 512, NW = NT / 64;
     constexpr float LOG2E = 1.4426950408889634f;
-    const int h = blockIdx.x, seq = blockIdx.y, c0 = blockIdx.z * C;
-    const int n = p.seq_len[seq];
-    if (n < p.len_lo || n > p.len_hi || c0 >= n) return;         // (uniform: before any barrier)
+    const int h = blockIdx.x;
+    DeltaChunks chunks(p, n_seqs);
+    DeltaChunk now, next;
+    if (!chunks.find(blockIdx.y, now)) return;                   // (uniform: before any barrier)
     extern __shared__ __attribute__((aligned(16))) float dl_sm[];
     float* qs = dl_sm;                   // [C][LQ]  q, later q e^b
     float* ks = qs + C * LQ;             // [C][LQ]  k, later k e^b
@@ -83,47 +153,64 @@ __global__ __launch_bounds__(512, NK > 8 ? 2 : 4) void delta_prep_kernel(DeltaAr
     float* Ms = As + C * LA;             // [C][LA]  M, later X = (I + diag(beta) M)^-1
     float* be = Ms + C * LA;             // [C]
     float* aux = be + C;                 // [512]
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int fr = lane & 15, fg = lane >> 4;
-    const int nv = min(C, n - c0);
-    const int64_t tb = (int64_t)p.seq_tok_start[seq] + c0;
-    const int g = h / (p.H / p.G);
-    // every load of the chunk first: q and k (DKP / 4 lanes hold a row), z (a channel per thread, NG groups share the tokens) and the
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = h / (p.H / p.G);
+    // the loads of a chunk: q and k (DKP / 4 lanes hold a row), z (a channel per thread, NG groups share the tokens), beta and the
     // first value channels of this wave
     constexpr int LR = DKP / 4, R = NT / LR, NQ = (C + R - 1) / R, NG = NT / DKP, TPG = C / NG;
-    const int qt = tid / LR, qd = tid % LR * 4, zd = tid % DKP, grp = tid / DKP, nvb = (p.DV + 15) >> 4;
+    const int nvb = (p.DV + 15) >> 4;
+    // (a thread's number anew for each part of a chunk, or everything that follows from it is kept in registers all along)
+    auto thread = [&]() __attribute__((always_inline)) { int t = threadIdx.x; asm volatile("" : "+v"(t)); return t; };
     f32x4 q4[NQ], k4[NQ], v4[2];
-    float pre[TPG];
-    auto ld4 = [&](const float* src) {
-        f32x4 x = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (p.vec4) { if (qd < p.DK) x = *(const f32x4*)(src + qd); }
-        else {
+    float pre[TPG], be_raw = 0.f;
+    const DeltaRows qr{(char*)(p.q + (int64_t)g * p.DK), 4 * (uint32_t)p.ld}, kr{(char*)(p.k + (int64_t)g * p.DK), qr.pitch}, vr{(char*)(p.v + (int64_t)h * p.DV), qr.pitch};
+    const DeltaRows zr{(char*)(p.z + (int64_t)h * p.DK), 4 * (uint32_t)p.z_ld}, br{(char*)(p.beta + h), 4 * (uint32_t)p.beta_ld}, orow{(char*)(p.o + (int64_t)h * p.DV), 4 * (uint32_t)p.o_ld};
+    auto ld4 = [&](auto rs, int qd, uint32_t at) __attribute__((always_inline)) {
+        if (VEC) return buffer_f32x4(rs, qd < p.DK ? at : DELTA_OUTSIDE, 0);
+        f32x4 x;
 #pragma unroll
-            for (int r = 0; r < 4; r++) if (qd + r < p.DK) x[r] = src[qd + r];
-        }
+        for (int r = 0; r < 4; r++) x[r] = buffer_f32(rs, qd + r < p.DK ? at + 4 * r : DELTA_OUTSIDE);
         return x;
     };
-    auto ldv = [&](int i, f32x4 (&v)[2]) {       // 16 value channels as the A operand of a transposed product
-        const int c = 16 * i + fr;
-        const float* vb = p.v + tb * p.ld + (int64_t)h * p.DV + min(c, p.DV - 1);
-#pragma unroll
-        for (int sb = 0; sb < 2; sb++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int t = 16 * sb + 4 * fg + r;
-                const float x = vb[min(t, nv - 1) * p.ld];
-                v[sb][r] = c < p.DV && t < nv ? x : 0.f;
-            }
+    auto ldv = [&](int64_t tb, int nv, int i, f32x4 (&v)[2]) __attribute__((always_inline)) {       // 16 value channels as the A operand of a transposed product
+        const auto rs = delta_rows(vr, tb, nv);
+        const int lane = thread() & 63, fr = lane & 15, fg = lane >> 4, c = 16 * i + fr;
+        const uint32_t at = 4 * fg * vr.pitch + (c < p.DV ? 4 * c : DELTA_OUTSIDE);
+        v[0] = delta_rows_get(rs, at, vr.pitch); v[1] = delta_rows_get(rs, at + 16 * vr.pitch, vr.pitch);
     };
+    auto load_qk = [&](int64_t tb, int nv) __attribute__((always_inline)) {
+        const int tid = thread(), qt = tid / LR, qd = tid % LR * 4;
+        const auto rq = delta_rows(qr, tb, nv), rk = delta_rows(kr, tb, nv);
+        const uint32_t at_q = qt * qr.pitch + 4 * qd;
 #pragma unroll
-    for (int i = 0; i < NQ; i++) {
-        const int t = qt + i * R;
-        q4[i] = k4[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (t < nv) { q4[i] = ld4(p.q + (tb + t) * p.ld + (int64_t)g * p.DK); k4[i] = ld4(p.k + (tb + t) * p.ld + (int64_t)g * p.DK); }
-    }
+        for (int i = 0; i < NQ; i++) { q4[i] = ld4(rq, qd, at_q + i * R * qr.pitch); k4[i] = ld4(rk, qd, at_q + i * R * qr.pitch); }
+    };
+    auto load_z = [&](int64_t tb, int nv) __attribute__((always_inline)) {
+        const int tid = thread(), zd = tid % DKP, grp = tid / DKP;
+        const auto rz = delta_rows(zr, tb, nv);
+        const uint32_t at_z = grp * TPG * zr.pitch + (zd < p.DK ? 4 * zd : DELTA_OUTSIDE);
 #pragma unroll
-    for (int j = 0; j < TPG; j++) pre[j] = p.z[(tb + min(grp * TPG + j, nv - 1)) * p.z_ld + (int64_t)h * p.DK + min(zd, p.DK - 1)];
-    if (wave < nvb) ldv(wave, v4);
+        for (int j = 0; j < TPG; j++) pre[j] = buffer_f32(rz, at_z + j * zr.pitch);
+        be_raw = buffer_f32(delta_rows(br, tb, nv), (tid & (C - 1)) * br.pitch);
+    };
+    auto barrier = [&]() __attribute__((always_inline)) {            // (without the wait for the next chunk's loads)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    const float A = -expf(p.a_log[h]) * LOG2E, bias = (int)threadIdx.x % DKP < p.DK ? p.dt_bias[h * p.DK + threadIdx.x % DKP] : 0.f;
+    load_qk(now.tok0, now.rows);
+    load_z(now.tok0, now.rows);
+    __builtin_amdgcn_sched_barrier(0);
+    ldv(now.tok0, now.rows, wave, v4);                           // (beyond DV: zeros)
+    for (int job = blockIdx.y;;) {
+    const auto ws = __builtin_amdgcn_make_buffer_rsrc(p.ws + (now.at * p.H + h) * delta_ws_floats(DKP), 0, 4 * (int)delta_ws_floats(DKP), 0x00020000);
+    // the chunk behind this one, whose loads go out as soon as this one's registers are read
+    job += gridDim.y;
+    const bool more = chunks.find(job, next);
+    if (!more) next = now;                                       // (the last one's are fetched again instead of a branch)
+    const int nv = now.rows, tb = now.tok0;
+    int tid = thread();
+    const int qt = tid / LR, qd = tid % LR * 4, zd = tid % DKP, grp = tid / DKP;
 #pragma unroll
     for (int i = 0; i < NQ; i++) {               // unit vectors
         const f32x4 q = q4[i], k = k4[i];
@@ -134,67 +221,86 @@ __global__ __launch_bounds__(512, NK > 8 ? 2 : 4) void delta_prep_kernel(DeltaAr
         *(f32x4*)(qs + (qt + i * R) * LQ + qd) = q * (p.q_scale / sqrtf(sq + DELTA_UNIT_EPS));
         *(f32x4*)(ks + (qt + i * R) * LQ + qd) = k * (1.0f / sqrtf(sk + DELTA_UNIT_EPS));
     }
+    __builtin_amdgcn_sched_barrier(0);
+    load_qk(next.tok0, next.rows);
+    __builtin_amdgcn_sched_barrier(0);
     {   // decays
-        const float A = -expf(p.a_log[h]) * LOG2E, bias = zd < p.DK ? p.dt_bias[h * p.DK + zd] : 0.f;
+        float s[TPG];
 #pragma unroll
-        for (int j = 0; j < TPG; j++) pre[j] = zd < p.DK && grp * TPG + j < nv ? A * delta_softplus(pre[j] + bias) : 0.f;
+        for (int j = 0; j < TPG; j++) s[j] = zd < p.DK && grp * TPG + j < nv ? A * delta_softplus(pre[j] + bias) : 0.f;
+        if (tid < C) be[tid] = tid < nv ? lr_sigmoid(be_raw) : 0.f;
+        __builtin_amdgcn_sched_barrier(0);
+        load_z(next.tok0, next.rows);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 1; j < TPG; j++) pre[j] += pre[j - 1];
-        aux[grp * DKP + zd] = pre[TPG - 1];
-        if (tid < C) be[tid] = tid < nv ? lr_sigmoid(p.beta[(tb + tid) * p.beta_ld + h]) : 0.f;
-        __syncthreads();
+        for (int j = 1; j < TPG; j++) s[j] += s[j - 1];
+        aux[grp * DKP + zd] = s[TPG - 1];
+        barrier();
         float off = 0.f;
         for (int j = 0; j < grp; j++) off += aux[j * DKP + zd];
 #pragma unroll
-        for (int j = 0; j < TPG; j++) bs[(grp * TPG + j) * LQ + zd] = off + pre[j];
+        for (int j = 0; j < TPG; j++) bs[(grp * TPG + j) * LQ + zd] = off + s[j];
     }
     for (int i = tid; i < 2 * C * LA; i += NT) As[i] = 0.f;      // (what lies above the diagonals stays zero)
-    __syncthreads();
-    // ---- A (s <= t) and M (s < t): 240 pairs of the two diagonal blocks, two threads each; the other 32 threads take A's diagonal ----
-    if (tid < 480) {
-        const int pr = tid >> 1, half = pr >= 120, x = pr - 120 * half;
+    barrier();
+    tid = thread();
+    // ---- A (s <= t) and M (s < t): 112 pairs of the four 8 x 8 diagonal blocks, four threads each; the last wave takes A's diagonal ----
+    if (tid < 448) {
+        const int pr = tid >> 2, blk = pr / 28, x = pr - 28 * blk;
         int t = (int)((sqrtf(8.f * (float)x + 1.f) - 1.f) * 0.5f);
         if ((t + 1) * (t + 2) / 2 <= x) t++;
         if (t * (t + 1) / 2 > x) t--;
-        const int s = x - t * (t + 1) / 2, tr = (16 * half + t + 1) * LQ, sr = (16 * half + s) * LQ;
+        const int s = x - t * (t + 1) / 2, tr = (8 * blk + t + 1) * LQ, sr = (8 * blk + s) * LQ;
         f32x4 aq = f32x4{0.f, 0.f, 0.f, 0.f}, ak = aq;
 #pragma unroll 2
-        for (int d = 4 * (tid & 1); d < DKP; d += 8) {
+        for (int d = 4 * (tid & 3); d < DKP; d += 16) {
             const f32x4 q4 = *(const f32x4*)(qs + tr + d), k4 = *(const f32x4*)(ks + tr + d), k2 = *(const f32x4*)(ks + sr + d);
             const f32x4 bt = *(const f32x4*)(bs + tr + d), b2 = *(const f32x4*)(bs + sr + d);
 #pragma unroll
             for (int r = 0; r < 4; r++) { const float e = ex2(bt[r] - b2[r]) * k2[r]; aq[r] = fmaf(q4[r], e, aq[r]); ak[r] = fmaf(k4[r], e, ak[r]); }
         }
-        const int at = (16 * half + t + 1) * LA + 16 * half + s;
+        const int at = (8 * blk + t + 1) * LA + 8 * blk + s;
         float sa = (aq[0] + aq[1]) + (aq[2] + aq[3]), sm = (ak[0] + ak[1]) + (ak[2] + ak[3]);
-        sa += __shfl_xor(sa, 1, 64);
-        sm += __shfl_xor(sm, 1, 64);
-        if (tid & 1) Ms[at] = sm; else As[at] = sa;
+        sa += __shfl_xor(sa, 1, 64); sm += __shfl_xor(sm, 1, 64);
+        sa += __shfl_xor(sa, 2, 64); sm += __shfl_xor(sm, 2, 64);
+        if ((tid & 3) == 0) As[at] = sa; else if ((tid & 3) == 1) Ms[at] = sm;
     } else {
-        const int t = tid - 480;
+        const int t = (tid - 448) >> 1;
         f32x4 a = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 2
-        for (int d = 0; d < DKP; d += 4) a += *(const f32x4*)(qs + t * LQ + d) * *(const f32x4*)(ks + t * LQ + d);
-        As[t * LA + t] = (a[0] + a[1]) + (a[2] + a[3]);
+        for (int d = 4 * (tid & 1); d < DKP; d += 8) a += *(const f32x4*)(qs + t * LQ + d) * *(const f32x4*)(ks + t * LQ + d);
+        float s = (a[0] + a[1]) + (a[2] + a[3]);
+        s += __shfl_xor(s, 1, 64);
+        if ((tid & 1) == 0) As[t * LA + t] = s;
     }
-    if (wave < 2) {                                              // tokens 16..31 against 0..15: wave 0 A, wave 1 M
-        const float* x = wave == 0 ? qs : ks;
-        f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    int lane = tid & 63, fr = lane & 15, fg = lane >> 4;
+    if (wave < 4) {                                              // wave 0: A, 1: M of tokens 16..31 against 0..15; 2, 3: of 8..15 against 0..7 and of 24..31 against 16..23
+        const float* x = wave & 1 ? ks : qs;
+        const int half = 16 * (fr >> 3), ta = wave < 2 ? 16 + fr : half + 8 + (fr & 7), ts = wave < 2 ? fr : half + (fr & 7), tref = wave < 2 ? 15 : half + 7;
+        f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f}, odd = acc;
 #pragma unroll 2
         for (int i = 0; i < NK; i++) {
             const int c = 16 * i + 4 * fg;
-            const f32x4 ref = *(const f32x4*)(bs + 15 * LQ + c);
-            const f32x4 a = *(const f32x4*)(x + (16 + fr) * LQ + c), b = *(const f32x4*)(ks + fr * LQ + c);
-            const f32x4 ba = *(const f32x4*)(bs + (16 + fr) * LQ + c), bb = *(const f32x4*)(bs + fr * LQ + c);
+            const f32x4 ref = *(const f32x4*)(bs + tref * LQ + c);
+            const f32x4 a = *(const f32x4*)(x + ta * LQ + c), b = *(const f32x4*)(ks + ts * LQ + c);
+            const f32x4 ba = *(const f32x4*)(bs + ta * LQ + c), bb = *(const f32x4*)(bs + ts * LQ + c);
 #pragma unroll
-            for (int r = 0; r < 4; r++) acc = mfma_f32(a[r] * ex2(ba[r] - ref[r]), b[r] * ex2(ref[r] - bb[r]), acc);
+            for (int r = 0; r < 4; r++) {
+                f32x4& d = r & 1 ? odd : acc;
+                d = mfma_f32(a[r] * ex2(ba[r] - ref[r]), b[r] * ex2(ref[r] - bb[r]), d);
+            }
         }
-        float* dst = wave == 0 ? As : Ms;
+        acc += odd;
+        float* dst = wave & 1 ? Ms : As;
+        // (waves 2 and 3: rows of one half against columns of the other are of no use)
+        if (wave < 2 || fg >> 1 == fr >> 3) {
+            const int row = wave < 2 ? 16 + 4 * fg : half + 8 + 4 * (fg & 1);
 #pragma unroll
-        for (int r = 0; r < 4; r++) dst[(16 + 4 * fg + r) * LA + fr] = acc[r];
+            for (int r = 0; r < 4; r++) dst[(row + r) * LA + ts] = acc[r];
+        }
     }
-    __syncthreads();
-    float* ws = p.ws + (delta_chunk(p, seq, blockIdx.z) * p.H + h) * delta_ws_floats(DKP);
+    barrier();
+    tid = thread(); lane = tid & 63; fr = lane & 15; fg = lane >> 4;
     if (wave < 2) {
         // inverses of the two diagonal blocks of I + N, N = diag(beta) M, from 1 x 1 blocks upwards: with X the inverse of the part inside
         // b x b blocks and N_b the part that a 2b x 2b block adds, X - X N_b X is the inverse inside 2b x 2b blocks
@@ -226,18 +332,21 @@ __global__ __launch_bounds__(512, NK > 8 ? 2 : 4) void delta_prep_kernel(DeltaAr
         for (int r = 0; r < 4; r++) Ms[(o + 4 * fg + r) * LA + o + fr] = xd[r];
     } else {
         // (K e^{b_end - b})^T and e^{b_end}
-#pragma unroll 2
-        for (int i = tid - 128; i < 2 * NK * 64; i += NT - 128) {
+#pragma unroll
+        for (int j = 0; j < (2 * NK * 64 + NT - 129) / (NT - 128); j++) {      // (as often for each thread: the compiler counts the stores behind the next chunk's loads)
+            const int i = min(tid - 128 + j * (NT - 128), 2 * NK * 64 - 1);
             const int l = i & 63, sb = (i >> 6) & 1, d = 16 * (i >> 7) + (l & 15), t = 16 * sb + 4 * (l >> 4);
             const float b_end = bs[31 * LQ + d];
             f32x4 x;
 #pragma unroll
             for (int r = 0; r < 4; r++) x[r] = ks[(t + r) * LQ + d] * ex2(b_end - bs[(t + r) * LQ + d]);
-            ((f32x4*)ws)[delta_piece(i >> 7, 4 + sb) + l] = x;
+            buffer_put4(ws, 16 * (delta_piece(i >> 7, 4 + sb) + l), 0, x);
         }
-        for (int d = tid - 128; d < DKP; d += NT - 128) ws[3 * C * DKP + d] = ex2(bs[31 * LQ + d]);
+        const int d = min(tid - 128, DKP - 1);
+        buffer_put(ws, 4 * (3 * C * DKP + d), ex2(bs[31 * LQ + d]));
     }
-    __syncthreads();
+    barrier();
+    tid = thread(); lane = tid & 63; fr = lane & 15; fg = lane >> 4;
     if (wave == 0) {
         // the block below the diagonal: -X22 N21 X11; then A T, T = X diag(beta), in A's place
         const f32x4 n21 = *(const f32x4*)(Ms + (16 + fr) * LA + 4 * fg) * be[16 + fr], x22 = *(const f32x4*)(Ms + (16 + fr) * LA + 16 + 4 * fg);
@@ -274,7 +383,8 @@ __global__ __launch_bounds__(512, NK > 8 ? 2 : 4) void delta_prep_kernel(DeltaAr
             *(f32x4*)(ks + t * LQ + d) = k;
         }
     }
-    __syncthreads();
+    barrier();
+    tid = thread(); lane = tid & 63; fr = lane & 15; fg = lane >> 4;
     // rows of T and of A T, blocks (0,0), (1,0), (1,1): B operands of the transposed products, whose accumulators hold four channels of a token
     f32x4 ta[3], ba[3];
 #pragma unroll
@@ -289,7 +399,10 @@ __global__ __launch_bounds__(512, NK > 8 ? 2 : 4) void delta_prep_kernel(DeltaAr
 #pragma unroll
         for (int r = 0; r < 4; r++) d[1] = mfma_f32(x[1][r], m[2][r], d[1]);
     };
-    for (int i = wave; i < NK; i += NW) {                         // 16 key channels: -W and Q'
+#pragma unroll
+    for (int i0 = 0; i0 < NK; i0 += NW) {                        // 16 key channels: -W and Q'
+        const int i = i0 + wave;
+        if (NK % NW && i >= NK) break;
         f32x4 k[2], w[2], q[2];
 #pragma unroll
         for (int sb = 0; sb < 2; sb++) {
@@ -300,30 +413,40 @@ __global__ __launch_bounds__(512, NK > 8 ? 2 : 4) void delta_prep_kernel(DeltaAr
         }
         times(k, ta, w);
         times(k, ba, q);
+        products_done(w[0], w[1], q[0], q[1]);
 #pragma unroll
         for (int tt = 0; tt < 2; tt++) {
-            ((f32x4*)ws)[delta_piece(i, tt) + lane] = w[tt];
-            ((f32x4*)ws)[delta_piece(i, 2 + tt) + lane] = q[tt];
+            buffer_put4(ws, 16 * lane, 16 * delta_piece(i, tt), w[tt]);
+            buffer_put4(ws, 16 * lane, 16 * delta_piece(i, 2 + tt), q[tt]);
         }
     }
-    for (int i = wave; i < nvb; i += NW) {                       // 16 value channels: U0 and O0
-        f32x4 v[2] = {v4[0], v4[1]}, u[2], o[2];
-        if (i != wave) ldv(i, v);
+    auto values = [&](int i, const f32x4 (&v)[2]) __attribute__((always_inline)) {       // 16 value channels: U0 and O0
+        f32x4 u[2], o[2];
         u[0] = u[1] = o[0] = o[1] = f32x4{0.f, 0.f, 0.f, 0.f};
         times(v, ta, u);
         times(v, ba, o);
+        products_done(u[0], u[1], o[0], o[1]);
+        const auto ru = delta_rows(vr, tb, nv), ro = delta_rows(orow, tb, nv);
         const int c = 16 * i + 4 * fg;
 #pragma unroll
         for (int tt = 0; tt < 2; tt++) {
-            const int t = 16 * tt + fr;
-            float* ub = p.v + (tb + t) * p.ld + (int64_t)h * p.DV + c;
-            float* ob = p.o + (tb + t) * p.o_ld + (int64_t)h * p.DV + c;
-            if (t >= nv) continue;
-            if (p.vec4v) { if (c < p.DV) { *(f32x4*)ub = u[tt]; *(f32x4*)ob = o[tt]; } }
+            const uint32_t at_u = (16 * tt + fr) * vr.pitch + 4 * c, at_o = (16 * tt + fr) * orow.pitch + 4 * c;
+            if (VEC) { buffer_put4(ru, c < p.DV ? at_u : DELTA_OUTSIDE, 0, u[tt]); buffer_put4(ro, c < p.DV ? at_o : DELTA_OUTSIDE, 0, o[tt]); }
             else
 #pragma unroll
-                for (int r = 0; r < 4; r++) if (c + r < p.DV) { ub[r] = u[tt][r]; ob[r] = o[tt][r]; }
+                for (int r = 0; r < 4; r++) { buffer_put(ru, c + r < p.DV ? at_u + 4 * r : DELTA_OUTSIDE, u[tt][r]); buffer_put(ro, c + r < p.DV ? at_o + 4 * r : DELTA_OUTSIDE, o[tt][r]); }
         }
+    };
+    values(wave, v4);                                            // (beyond DV: nothing is stored)
+    for (int i = wave + NW; i < nvb; i += NW) {
+        f32x4 v[2];
+        ldv(tb, nv, i, v);
+        values(i, v);
+    }
+    if (!more) return;
+    ldv(next.tok0, next.rows, wave, v4);
+    barrier();                                                   // the last readers of this chunk are done
+    now = next;
     }
 }
 
@@ -344,26 +467,6 @@ __device__ __forceinline__ int delta_scan_seq(const int* seq_len, int i, int n_s
         rank += other > mine || (other == mine && j < lane) ? 1 : 0;
     }
     return __builtin_amdgcn_readfirstlane(__builtin_ctzll(__ballot(rank == (i == 0 ? n_seqs - 1 : i - 1) && lane < n_seqs)));
-}
-// Value column `col` of a chunk's U0, O0 and O, tokens 16 tt + 4 fg + r.  The descriptor ends with the sequence and columns beyond DV lie outside it: what is read
-// there is zero (U: the state's padding columns stay zero), and what is written there is dropped.
-struct DeltaRows { char* base; uint32_t pitch; };
-template <typename Rsrc> __device__ __forceinline__ f32x4 delta_rows_get(Rsrc rs, uint32_t at, uint32_t pitch) {
-    f32x4 x;
-#pragma unroll
-    for (int r = 0; r < 4; r++) x[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, at + r * pitch, 0, 0));
-    return x;
-}
-// (chunk's rows: a pitch is below 2^26 bytes.  readfirstlane: the compiler doesn't see that these are uniform, and loops over the lanes' descriptors)
-__device__ __forceinline__ auto delta_rows(const DeltaRows& w, int c0, int left) {
-    const uint64_t at = (uint64_t)(w.base + (int64_t)c0 * w.pitch);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)at), hi = __builtin_amdgcn_readfirstlane((uint32_t)(at >> 32));
-    return __builtin_amdgcn_make_buffer_rsrc((void*)((uint64_t)hi << 32 | lo), 0, __builtin_amdgcn_readfirstlane(max(min(left, DELTA_C), 0) * (int)w.pitch), 0x00020000);
-}
-template <typename Rsrc> __device__ __forceinline__ f32x4 buffer_f32x4(Rsrc rs, int lane_off, int off) {
-    union { f32x4 f; u32x4 u; } t;
-    t.u = __builtin_amdgcn_raw_buffer_load_b128(rs, lane_off, off, 0);
-    return t.f;
 }
 template <int N>      // key channels ch0 .. ch0 + 16 N - 1 of a lane's column
 __device__ __forceinline__ void delta_state_in(const DeltaArgs& p, const float* st, int ch0, int fg, int col, bool fresh, f32x4 (&S)[N]) {
@@ -416,7 +519,7 @@ __global__ __launch_bounds__(DELTA_SCAN_WAVES * 64, NK > 8 ? 1 : 3) void delta_s
     float rd = 0.f;
     const int64_t tok0 = p.seq_tok_start[seq];
     const DeltaRows vr{(char*)(p.v + tok0 * p.ld + (int64_t)h * p.DV), 4 * (uint32_t)p.ld}, orow{(char*)(p.o + tok0 * p.o_ld + (int64_t)h * p.DV), 4 * (uint32_t)p.o_ld};
-    const uint32_t cb = col < p.DV ? 4 * col : 1u << 31;
+    const uint32_t cb = col < p.DV ? 4 * col : DELTA_OUTSIDE;
     constexpr int Q = NK / 2;                                    // a chunk's loads go out in as many portions, between the products of two state tiles each
     auto fetch = [&](int c0, int part) __attribute__((always_inline)) {
 #pragma unroll
@@ -453,13 +556,13 @@ __global__ __launch_bounds__(DELTA_SCAN_WAVES * 64, NK > 8 ? 1 : 3) void delta_s
             }
             if (i & 1) __builtin_amdgcn_sched_barrier(0);        // (or all reads are hoisted to the front, and registers spill)
         }
+        products_done(u[0], u[1], o[0], o[1]);
         const auto ro = delta_rows(orow, c0, n - c0);
 #pragma unroll
         for (int tt = 0; tt < 2; tt++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const float x = o[tt][r];        // (a bit_cast of the vector's element itself takes the first)
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, x), ro, (16 * tt + 4 * fg + r) * orow.pitch + cb, 0, 0);
+                buffer_put(ro, (16 * tt + 4 * fg + r) * orow.pitch + cb, o[tt][r]);
             }
         f32x4 ub[2] = {u[0], u[1]};
         __builtin_amdgcn_sched_barrier(0);
@@ -505,7 +608,7 @@ __global__ __launch_bounds__(KSP * 64, 2) void delta_scan_parts_kernel(DeltaArgs
     const int64_t stride = p.H * delta_ws_floats(DKP), tok0 = p.seq_tok_start[seq];
     const float* src = p.ws + (delta_chunk(p, seq, 0) * p.H + h) * delta_ws_floats(DKP);
     const DeltaRows vr{(char*)(p.v + tok0 * p.ld + (int64_t)h * p.DV), 4 * (uint32_t)p.ld}, orow{(char*)(p.o + tok0 * p.o_ld + (int64_t)h * p.DV), 4 * (uint32_t)p.o_ld};
-    const uint32_t cb = col < p.DV ? 4 * col : 1u << 31;
+    const uint32_t cb = col < p.DV ? 4 * col : DELTA_OUTSIDE;
     // what U and O start from is dealt over the parts: U's two pieces to the first two, O's to the next two or the same
     constexpr int NI = KSP >= 4 ? 1 : 2;
     const int stt = kq & 1;
@@ -514,7 +617,7 @@ __global__ __launch_bounds__(KSP * 64, 2) void delta_scan_parts_kernel(DeltaArgs
     // ... and what becomes of O: two parts store 16 tokens each, or four 8
     constexpr int NS = KSP == 2 ? 4 : 2;
     const int ott = KSP == 2 ? kq : (kq >> 1) & 1, or0 = KSP == 2 ? 0 : 2 * (kq & 1);
-    const uint32_t at_s = KSP <= 4 || kq < 4 ? (16 * ott + 4 * fg + or0) * orow.pitch + cb : 1u << 31;
+    const uint32_t at_s = KSP <= 4 || kq < 4 ? (16 * ott + 4 * fg + or0) * orow.pitch + cb : DELTA_OUTSIDE;
     struct Chunk { f32x4 op[N][6], d[N], start[NI]; };
     auto fetch_start = [&](Chunk& k, int c0) __attribute__((always_inline)) {
         k.start[0] = delta_rows_get(delta_rows(first, c0, n - c0), at_v, first.pitch);
@@ -546,7 +649,7 @@ __global__ __launch_bounds__(KSP * 64, 2) void delta_scan_parts_kernel(DeltaArgs
             float y = oq[0][r];
 #pragma unroll
             for (int q = 1; q < KSP; q++) y += oq[q][r];
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, y), ro, at_s + r * orow.pitch, 0, 0);
+            buffer_put(ro, at_s + r * orow.pitch, y);
         }
     };
     auto step = [&](Chunk& k, Chunk& next, int c0, int turn) __attribute__((always_inline)) {
@@ -831,7 +934,7 @@ __global__ __launch_bounds__(64) void pack_rows_kernel(PackArgs p) {
 
 // launches (delta_inst.hip); nk: template argument of the chunk kernels
 void delta_step_launch(hipStream_t st, const DeltaArgs& p, int n_seqs, bool fused, bool f32);
-void delta_prep_launch(hipStream_t st, const DeltaArgs& p, dim3 grid, int nk);
+void delta_prep_launch(hipStream_t st, const DeltaArgs& p, int n_seqs, int nk, int tokens);
 void delta_scan_launch(hipStream_t st, const DeltaArgs& p, int n_seqs, int nk, int max_len, int tokens);
 
 }  // namespace nvl

@@ -1267,11 +1267,10 @@ void mix_delta(nvl_model* m, const LayerRun& r, const MixerW& w, const Meta& md,
         const int nk = c.dim <= 32 ? 2 : (c.dim <= 64 ? 4 : (c.dim <= 128 ? 8 : 16));
         grow(m, m->delta_ws, m->delta_ws_cap, (int64_t)(m->opts.max_batch_tokens / DELTA_C + m->opts.max_seqs + 1) * c.heads * delta_ws_floats(nk * 16));
         a.ws = m->delta_ws;
-        const dim3 pgrid(c.heads, n_seqs, cdiv(max_len, DELTA_C));
         const double scratch = (double)M * c.heads * (3.0 * nk * 16 + 2.0 * c.vdim) * 4.0;
         {
             KScope ks(m, KC_OTHER, 0, KS_DELTA_PREP, io + scratch);
-            delta_prep_launch(m->stream, a, pgrid, nk);
+            delta_prep_launch(m->stream, a, n_seqs, nk, M);
             NVL_HIP(hipGetLastError());
         }
         {
