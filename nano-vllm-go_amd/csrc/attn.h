@@ -430,40 +430,48 @@ __device__ __forceinline__ f32x4 part_load(const float* base, int64_t floats) {
     t.u = __builtin_amdgcn_raw_buffer_load_b128(__builtin_amdgcn_make_buffer_rsrc((void*)base, 0, 1 << 30, 0x00020000), (int)(floats * 4), 0, 0x11);
     return t.f;
 }
-// combine of a split decode launch: the nsplit partial results of one (sequence, kv head, query tile), in workgroup order
-// whichever workgroup runs it.  One wave, the lanes of real heads; lane (fq, fg) as in the kernel's own combine.
-template <int HD>
-__device__ __forceinline__ void attn_decode_merge(const AttnArgs& p, int pair, int tok, int head, int nsplit, int lane) {
-    constexpr int DT = HD / 16;
+__device__ __forceinline__ float part_load1(const float* base, int floats) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(__builtin_amdgcn_make_buffer_rsrc((void*)base, 0, 1 << 30, 0x00020000), floats * 4, 0, 0x11));
+}
+// combine of a split decode launch: the nsplit <= MOST partial results of one (sequence, kv head, query tile), in workgroup order whichever workgroup runs it.  The
+// lanes of real heads; wave w takes output blocks w, w + NW, ..; lane (fq, fg) as in the kernel's own combine.  All loads leave together (results beyond the last:
+// the last one again): one wave with a branch per result went to memory 2 nsplit times, one after the other.
+template <int HD, int NW, int MOST>
+__device__ __forceinline__ void attn_decode_merge(const AttnArgs& p, int pair, int tok, int head, int nsplit, int wave, int lane) {
+    constexpr int DT = HD / 16, REC = attn_part_floats<HD>(), PER = DT > NW ? DT / NW : 1;
+    if (wave >= DT) return;
     const int fq = lane & 15, fg = lane >> 4;
-    // (a record ends in m | l of its 16 rows, four rows a lane group: (m, l) of row fq by two loads of four)
-    const float* rec0 = p.part + (int64_t)pair * p.split_max * attn_part_floats<HD>();
-    float mz[ATTN_SPLIT_MAX], lz[ATTN_SPLIT_MAX], mstar = -INFINITY, L = 0.f;
+    const float* rec0 = p.part + (int64_t)pair * p.split_max * REC;
+    float mz[MOST], lz[MOST], mstar = -INFINITY, L = 0.f;
+    f32x4 t[MOST][PER];
 #pragma unroll
-    for (int z = 0; z < ATTN_SPLIT_MAX; z++) {
-        if (z >= nsplit) break;
-        const int at = z * attn_part_floats<HD>() + DT * 256 + (fq & ~3);
-        const f32x4 m4 = part_load(rec0, at), l4 = part_load(rec0, at + 16);
-        mz[z] = fq & 2 ? (fq & 1 ? m4[3] : m4[2]) : (fq & 1 ? m4[1] : m4[0]);
-        lz[z] = fq & 2 ? (fq & 1 ? l4[3] : l4[2]) : (fq & 1 ? l4[1] : l4[0]);
+    for (int z = 0; z < MOST; z++) {
+        const int at = min(z, nsplit - 1) * REC;
+        mz[z] = part_load1(rec0, at + DT * 256 + fq);
+        lz[z] = part_load1(rec0, at + DT * 256 + 16 + fq);
     }
-    f32x4 O[DT];
 #pragma unroll
-    for (int d = 0; d < DT; d++) O[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int z = 0; z < MOST; z++)
 #pragma unroll
-    for (int z = 0; z < ATTN_SPLIT_MAX; z++) if (z < nsplit) mstar = fmaxf(mstar, mz[z]);
+        for (int i = 0; i < PER; i++) t[z][i] = part_load(rec0, min(z, nsplit - 1) * REC + ((wave + i * NW) * 64 + lane) * 4);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int z = 0; z < ATTN_SPLIT_MAX; z++) {
+    for (int z = 0; z < MOST; z++) mstar = fmaxf(mstar, mz[z]);
+    f32x4 O[PER];
+#pragma unroll
+    for (int i = 0; i < PER; i++) O[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int z = 0; z < MOST; z++) {
         if (z >= nsplit) break;
         const float sc = __builtin_amdgcn_exp2f(mz[z] - mstar);      // (no tile: m = -inf, O = l = 0)
         L += lz[z] * sc;
 #pragma unroll
-        for (int d = 0; d < DT; d++) O[d] += part_load(rec0, z * attn_part_floats<HD>() + (d * 64 + lane) * 4) * sc;
+        for (int i = 0; i < PER; i++) O[i] += t[z][i] * sc;
     }
     const float inv = 1.0f / L;
 #pragma unroll
-    for (int d = 0; d < DT; d++)
-        act_store4<bf16_t>((bf16_t*)p.out, tok, head * HD + d * 16 + fg * 4, p.out_stride, O[d] * inv);
+    for (int i = 0; i < PER; i++)
+        act_store4<bf16_t>((bf16_t*)p.out, tok, head * HD + (wave + i * NW) * 16 + fg * 4, p.out_stride, O[i] * inv);
 }
 
 // Host rules of the order of ragged contexts (the figures: decode_attn_cfg).  n_kt: 64-key tiles of the longest, mean_kt: of the mean
@@ -797,6 +805,42 @@ __global__ __launch_bounds__(NW * 64, HD == 128 ? 2 : 0) void attn_decode_bf16_k
         act_store4<bf16_t>((bf16_t*)p.out, tok, head * HD + wave * 16 + fg * 4, p.out_stride, Od * (1.0f / Ls));
         return;
     }
+    if (SPLIT && nz > 1) {
+        __shared__ int ticket;
+        const int pair = seq * gridDim.x + blockIdx.x;               // (sequence, kv head, query tile)
+        float* rec = p.part + ((int64_t)pair * p.split_max + z) * attn_part_floats<HD>();
+        float ms = red_m[0][fq], Ls = 0.f, sc[NW];
+#pragma unroll
+        for (int w = 1; w < NW; w++) ms = fmaxf(ms, red_m[w][fq]);
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+            sc[w] = ms > -INFINITY ? __builtin_amdgcn_exp2f(red_m[w][fq] - ms) : 0.f;      // (a workgroup of a split launch may have had no tile at all; idle waves: exp2(-inf) = 0)
+            Ls += red_l[w][fq] * sc[w];
+        }
+        if (row_ok) {
+#pragma unroll
+            for (int d = wave; d < DT; d += NW) {
+                f32x4 Od = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int w = 0; w < NW; w++) Od += ((const f32x4*)(smem + w * TILE_BYTES))[d * 64 + lane] * sc[w];
+                part_store(rec, (d * 64 + lane) * 4, Od);
+            }
+            if (wave == 0 && fg < 2)
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, fg ? Ls : ms), __builtin_amdgcn_make_buffer_rsrc(rec, 0, 1 << 30, 0x00020000), (DT * 256 + 16 * fg + fq) * 4, 0, 0x11);
+        }
+        // Last arriver combines (no second launch: a merge kernel cost 5-7 us of the 8-11 the split saves); the order of the sum is z
+        // order regardless.
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // this wave's part of the record has reached memory
+        __syncthreads();
+        if (tid == 0) ticket = __hip_atomic_fetch_add(p.part_cnt + pair, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (ticket != nz - 1) return;
+        if (tid == 0) __hip_atomic_store(p.part_cnt + pair, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);    // for the next launch
+        if (!row_ok) return;
+        if (nz <= 3) attn_decode_merge<HD, NW, 3>(p, pair, tok, head, nz, wave, lane);
+        else attn_decode_merge<HD, NW, ATTN_SPLIT_MAX>(p, pair, tok, head, nz, wave, lane);
+        return;
+    }
     if (wave != 0 || !row_ok) return;
     float mstar = red_m[0][fq];
 #pragma unroll
@@ -805,38 +849,13 @@ __global__ __launch_bounds__(NW * 64, HD == 128 ? 2 : 0) void attn_decode_bf16_k
     f32x4 O[DT];
 #pragma unroll
     for (int d = 0; d < DT; d++) O[d] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (!SPLIT || mstar > -INFINITY) {       // (a workgroup of a split launch may have had no tile at all)
 #pragma unroll
-        for (int w = 0; w < NW; w++) {
-            const float sc = __builtin_amdgcn_exp2f(red_m[w][fq] - mstar);   // idle waves: exp2(-inf) = 0
-            L += red_l[w][fq] * sc;
-            const f32x4* wo = (const f32x4*)(smem + w * TILE_BYTES);
+    for (int w = 0; w < NW; w++) {
+        const float sc = __builtin_amdgcn_exp2f(red_m[w][fq] - mstar);   // idle waves: exp2(-inf) = 0
+        L += red_l[w][fq] * sc;
+        const f32x4* wo = (const f32x4*)(smem + w * TILE_BYTES);
 #pragma unroll
-            for (int d = 0; d < DT; d++) O[d] += wo[d * 64 + lane] * sc;
-        }
-    }
-    if (SPLIT && nz > 1) {
-        const int pair = seq * gridDim.x + blockIdx.x;               // (sequence, kv head, query tile)
-        float* rec = p.part + ((int64_t)pair * p.split_max + z) * attn_part_floats<HD>();
-#pragma unroll
-        for (int d = 0; d < DT; d++) part_store(rec, (d * 64 + lane) * 4, O[d]);
-        // (m and l of four rows by the lane of the first: 16-byte stores)
-        f32x4 m4, l4;
-#pragma unroll
-        for (int r = 0; r < 4; r++) { m4[r] = __shfl(mstar, (lane & ~3) + r, 64); l4[r] = __shfl(L, (lane & ~3) + r, 64); }
-        if (fg == 0 && (fq & 3) == 0) { part_store(rec, DT * 256 + fq, m4); part_store(rec, DT * 256 + 16 + fq, l4); }
-        // Last arriver combines (no second launch: a merge kernel cost 5-7 us of the 8-11 the split saves); the order of the sum is z
-        // order regardless.
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // the record has reached memory
-        int ticket = 0;
-        int32_t* cnt = p.part_cnt + pair;
-        if (lane == 0) ticket = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        ticket = __builtin_amdgcn_readfirstlane(ticket);
-        if (ticket != nz - 1) return;
-        asm volatile("" ::: "memory");
-        attn_decode_merge<HD>(p, pair, tok, head, nz, lane);
-        if (lane == 0) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);    // for the next launch
-        return;
+        for (int d = 0; d < DT; d++) O[d] += wo[d * 64 + lane] * sc;
     }
     const float inv = 1.0f / L;
 #pragma unroll

@@ -1372,24 +1372,19 @@ static int g_attn_split = 1;   // nvl_set_tuning key 25: split a decode attentio
 // workgroup | most workgroups per (sequence, kv head) << 8 | key tiles a workgroup has at least << 12.
 // Split: a workgroup pulls all K/V of its (sequence, kv head) through ONE CU, one round of tiles after the other; with few of
 // them and a long context that, not HBM, is the time.  A sequence is then dealt over workgroups (attn.h), and the last of them
-// combines the parts, which costs a launch about 2 us: a context has to be longer the fuller the chip already is.  No more parts than
+// combines the parts, which costs a launch about 1.3 us: a context has to be longer the fuller the chip already is.  No more parts than
 // leave a CU to each workgroup (256 / pairs), and as many as give each the same number of rounds: beyond 128 pairs a split only
-// adds traffic.  The lines lie where whole decode steps change sides (a launch by itself favours the split earlier: it does not wait for the
-// kernel before it).  Steps against the whole form, per cent (waves x parts; forms in random order, runs differ by 0.5):
-//   heads of 64, Llama-3.2-1B, 8 kv heads     keys  560 +1.2 (2 x 3)   640..760 -0.3 (2 x 3, Granite -0.7)  1000 -4.6 (2 x 4)  1500 -8.7 (4 x 3)     1 sequence
-//                                                   600 +0.8 (2 x 3)   800 -0.6 (2 x 4)  1200 -1.6 (4 x 3)  1800 -7.4 (4 x 4)     4
-//                                                   700 +0.6 (2 x 3)  1000 -0.6 (4 x 2)  1500 -6.9 (4 x 3)                        6
-//                                                   700 +0.5 (2 x 3)  1000 -1.4 (4 x 2)  1400 -4.5 (4 x 3)  1900 -3.4 (4 x 4)     8
-//                                                   900 -1.3 (4 x 2)  1300 -3.8 (4 x 3)                                          10
-//                                                  1100 +0.9 (4 x 3)  1500 +1.0 (4 x 3), -1.1 (8 x 2)  1900 -3.9 (8 x 2)         12
-//                                                  1000  0.0 (4 x 2)  1500 -0.2 (4 x 3), -0.6 (8 x 2)  1900 -3.1 (8 x 2)         16
-//   heads of 128, Llama-3-8B, 8 kv heads            400 -0.5 (2 x 4)   700 -2.4 (4 x 3)  1500 -9.4 (4 x 6)                        1
-//                                                   400 -1.1 (2 x 4)   800 -4.7 (4 x 4)  1500 -8.9 (4 x 6)                        4
-//                                                   400 -0.3 (2 x 4)   600 -1.9 (4 x 3)   900 -4.3 (4 x 4)  1500 -6.6 (4 x 3)     8
-//                                                   600 +0.8 (4 x 2)  1000 -3.0 (4 x 2)  1500 -4.3 (4 x 2), +3.6 (4 x 3)         12
-//                                                  1000 -1.6 (4 x 2), +2.6 (4 x 4)  1500 -3.0 (4 x 2)                            16
+// adds traffic.  Up to 64 pairs two waves a workgroup, so that most sequences are one round of many parts.  The lines lie where whole decode steps change sides (a
+// launch by itself favours the split earlier: it does not wait for the kernel before it).  us a step, whole / split (waves x most parts):
+//   heads of 64, Llama-3.2-1B, 8 kv heads     keys  400  729 / 741 (2 x 2)   500  742 / 738 (2 x 2)   700  764 / 741 (2 x 3)  1000  806 / 758 (2 x 4), 783 (4 x 2)  1900  914 / 763 (2 x 8), 800 (4 x 4)     1 sequence
+//                                                   700  772 / 765 (2 x 3)  1000  820 / 774 (2 x 4), 791 (4 x 2)  1900  892 / 804 (2 x 8), 806 (4 x 4)    4
+//                                                  1200  836 / 800 (2 x 5), 799 (4 x 3)                                                                        6
+//                                                   700  779 / 788 (2 x 3)  1000  825 / 813 (2 x 4), 820 (4 x 2)  1500  913 / 855 (2 x 6), 847 (4 x 3)         8
+//                                                  1200  958 / 945 (4 x 3), 976 (8 x 2)                                                                       12
+//                                                   900  947 / 956 (4 x 2)  1000  966 / 968 (4 x 2)  1900 1068 / 1048 (8 x 2)                                 16
+//   heads of 128, hybrid-2k, 4 kv heads (requests)  500  713 / 701 (2 x 4)   700  949 / 929 (2 x 6), 932 (4 x 3)  1000 1003 / 971 (2 x 8), 973 (4 x 4)         1
 // Ragged contexts leave room for more parts, since a sequence takes them by its own length and the other workgroups of the grid leave at
-// once: more while those with work stay within 208, the whole grid within 640.  "/ 6": contexts down to a sixth of the longest; without -> with:
+// once: more while those with work stay within 208 (heads of 64, whose parts are smaller: 300, and 280 beyond 85 pairs: 16 of 900 keys, 292 with work, +1.0), the whole grid within 640.  "/ 6": contexts down to a sixth of the longest; without -> with:
 //   heads of 64    Granite-3.0-1B 16 of 900 / 6  0.0 -> -1.2 (4 x 2), 12 of 1100 / 6 -0.3 -> -1.6 (4 x 3), Llama-3.2-1B 12 of 1100 / 6 -0.4 -> -1.1,
 //                  14 of 1200 and short ones 0.0 -> -1.3; of 900 / 2  at 227 with work +0.4, so not
 //   heads of 128   12 of 1500 / 6 -3.6 -> -5.7 (4 x 3), 16 of 1100 / 6 -1.0 -> -2.1 (4 x 3), 12 of 1500 and short ones -5 -> -7.6 (4 x 6); 16 of 1500 and
@@ -1428,10 +1423,10 @@ int decode_attn_cfg(const nvl_model* m, int n_seqs) {
     if (g_attn_split >= 2) { const int tiles = (g_attn_split - 1) * nw * per_wave; return cfg(nw, std::max(1, std::min(most, cdiv(n_kt, tiles))), tiles); }
     if (g_attn_split && !g_attn_nw && most > 1) {
         // the workgroups with work: a sequence has its tiles / `tiles` parts, rounded up
-        auto room = [&](int tiles) { return (mean_kt / tiles + 0.5) * wgs <= 208; };
+        auto room = [&](int tiles) { return (mean_kt / tiles + 0.5) * wgs <= (m->hd == 64 ? wgs > 85 ? 280 : 300 : 208); };
         int waves = 0;
-        if (m->hd == 64) waves = wgs <= 32 ? (n_kt > 20 ? 4 : n_kt > (wgs <= 8 ? 10 : 12) ? 2 : 0) : wgs <= 85 ? (n_kt > 14 ? 4 : 0) : wgs > 128 ? 0 : n_kt > 20 ? 8 : n_kt > 14 && room(8) ? 4 : 0;
-        else waves = wgs <= 64 ? (n_kt > 10 ? 4 : n_kt > (wgs <= 32 ? 5 : 6) ? 2 : 0) : wgs <= 128 && n_kt > 12 ? 4 : 0;
+        if (m->hd == 64) waves = wgs <= 32 ? (n_kt > 32 ? 4 : n_kt > (wgs <= 8 ? 7 : 9) ? 2 : 0) : wgs <= 85 ? (n_kt <= 14 ? 0 : n_kt <= 20 && wgs <= 64 && room(4) ? 2 : 4) : wgs > 128 ? 0 : n_kt > 20 ? 8 : n_kt > 14 && room(8) ? 4 : 0;
+        else waves = wgs <= 64 ? (n_kt > 16 ? 4 : n_kt > (wgs <= 32 ? 5 : 6) ? 2 : 0) : wgs <= 128 && n_kt > 12 ? 4 : 0;
         if (waves) {
             const int round = waves * per_wave, rounds = cdiv(n_kt, round);
             int each = cdiv(rounds, std::max(1, std::min(most, 256 / wgs)));      // rounds of a part
