@@ -429,18 +429,35 @@ __device__ __forceinline__ float sandwich_sq_dev(const f32x4 (&x)[MAXCH], float 
     return vs;
 }
 // EXT: layer norms, plain adds and a second source (layers whose sublayers join the stream together)
+// One trip to memory bounds it: everything that a row needs, up to four partial sums, the weights of both norms, the row before, is on its way before the first
+// sum.  One after the other (each partial sum, then each norm's weights behind its mean) a launch took 0.55 us longer: a step of 6 rows of 2048 through 24 of
+// them 892 -> 879 us
 template <typename ActT, int MAXCH, bool EXT = false>
 __global__ __launch_bounds__(256) void sandwich_row_kernel(SandwichArgs p, ActT* __restrict__ xn) {
     __shared__ float red[4];
+    constexpr bool AHEAD = MAXCH <= 4;      // (wider rows have no registers for it)
+    constexpr int PARTS = AHEAD ? 4 : 1;
     const int r = blockIdx.x, H4 = p.H >> 2;
     const int src = p.rows_idx ? p.rows_idx[r] : r;
     float* xr = p.x + (int64_t)src * p.H;
-    f32x4 x[MAXCH], y[MAXCH];
+    const bool shifted = EXT && !p.w_next && p.shift, any = shifted && p.seq_pos[r] > 0;
+    float* before = shifted ? p.before + (int64_t)p.seq_slot[r] * p.before_stride : nullptr;
+    f32x4 x[MAXCH], y[MAXCH], e[MAXCH][PARTS], w1[MAXCH], w2[MAXCH], w3[MAXCH];
     auto put = [&](int j, f32x4 v) {
         act_store4<ActT>(xn, r, j * 4, p.H, v);
         if constexpr (sizeof(ActT) == 2) if (p.xn_rows) store_row4(p.xn_rows + (int64_t)r * p.H + j * 4, v);
     };
-    float ss = 0.f;
+    auto post_weight = [&](int c, int j) { w1[c] = *(const f32x4*)(p.w_post + j * 4); };
+    auto next_weight = [&](int c, int j) {      // .. of the norm that follows, its bias; of the shift, the row before
+        if (p.w_next) {
+            w2[c] = *(const f32x4*)(p.w_next + j * 4);
+            if constexpr (EXT) if (p.b_next) w3[c] = *(const f32x4*)(p.b_next + j * 4);
+        } else if (shifted) {
+            w2[c] = *(const f32x4*)(p.shift + j * 4);
+            w3[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (any) w3[c] = *(const f32x4*)(before + j * 4);
+        }
+    };
 #pragma unroll
     for (int c = 0; c < MAXCH; c++) {
         const int j = threadIdx.x + c * 256;
@@ -449,9 +466,23 @@ __global__ __launch_bounds__(256) void sandwich_row_kernel(SandwichArgs p, ActT*
         if (j < H4) {
             x[c] = *(const f32x4*)(xr + j * 4);
             if (p.y) {
-                const float* yr = p.y + (int64_t)r * p.H + j * 4;
-                y[c] = *(const f32x4*)yr;
-                for (int k = 1; k < p.slices; k++) y[c] += *(const f32x4*)(yr + k * p.slice_stride);
+#pragma unroll
+                for (int k = 0; k < PARTS; k++) if (k == 0 || k < p.slices) e[c][k] = *(const f32x4*)(p.y + k * p.slice_stride + (int64_t)r * p.H + j * 4);
+                if (AHEAD && p.w_post) post_weight(c, j);
+            }
+            if (AHEAD) next_weight(c, j);
+        }
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < MAXCH; c++) {
+        const int j = threadIdx.x + c * 256;
+        if (j < H4) {
+            if (p.y) {
+                y[c] = e[c][0];
+#pragma unroll
+                for (int k = 1; k < PARTS; k++) if (k < p.slices) y[c] += e[c][k];
+                for (int k = PARTS; k < p.slices; k++) y[c] += *(const f32x4*)(p.y + k * p.slice_stride + (int64_t)r * p.H + j * 4);
             }
             if constexpr (EXT) if (p.y2) y[c] += sandwich_more(p, r, j * 4);
         }
@@ -469,9 +500,9 @@ __global__ __launch_bounds__(256) void sandwich_row_kernel(SandwichArgs p, ActT*
         for (int c = 0; c < MAXCH; c++) {
             const int j = threadIdx.x + c * 256;
             if (j < H4) {
-                const f32x4 w = *(const f32x4*)(p.w_post + j * 4);
+                if (!AHEAD) post_weight(c, j);
 #pragma unroll
-                for (int k = 0; k < 4; k++) x[c][k] = (x[c][k] / rms) * w[k];
+                for (int k = 0; k < 4; k++) x[c][k] = (x[c][k] / rms) * w1[c][k];
                 *(f32x4*)(xr + j * 4) = x[c];
             }
         }
@@ -488,26 +519,22 @@ __global__ __launch_bounds__(256) void sandwich_row_kernel(SandwichArgs p, ActT*
         for (int c = 0; c < MAXCH; c++) {
             const int j = threadIdx.x + c * 256;
             if (j < H4) {
-                const f32x4 w = *(const f32x4*)(p.w_post + j * 4);
+                if (!AHEAD) post_weight(c, j);
 #pragma unroll
-                for (int k = 0; k < 4; k++) x[c][k] += (y[c][k] / rms) * w[k];
+                for (int k = 0; k < 4; k++) x[c][k] += (y[c][k] / rms) * w1[c][k];
                 *(f32x4*)(xr + j * 4) = x[c];
             }
         }
     }
     if (!p.w_next) {
-        if (EXT && p.shift) {
-            float* before = p.before + (int64_t)p.seq_slot[r] * p.before_stride;
-            const bool any = p.seq_pos[r] > 0;
+        if (shifted) {
 #pragma unroll
             for (int c = 0; c < MAXCH; c++) {
                 const int j = threadIdx.x + c * 256;
                 if (j < H4) {
-                    const f32x4 mu = *(const f32x4*)(p.shift + j * 4);
-                    f32x4 h = f32x4{0.f, 0.f, 0.f, 0.f};
-                    if (any) h = *(const f32x4*)(before + j * 4);
+                    if (!AHEAD) next_weight(c, j);
                     *(f32x4*)(before + j * 4) = x[c];
-                    act_store4<ActT>(xn, r, j * 4, p.H, x[c] + (h - x[c]) * mu);
+                    act_store4<ActT>(xn, r, j * 4, p.H, x[c] + (w3[c] - x[c]) * w2[c]);
                 }
             }
         } else if (p.raw_next)
@@ -525,10 +552,10 @@ __global__ __launch_bounds__(256) void sandwich_row_kernel(SandwichArgs p, ActT*
         for (int c = 0; c < MAXCH; c++) {
             const int j = threadIdx.x + c * 256;
             if (j < H4) {
-                const f32x4 w = *(const f32x4*)(p.w_next + j * 4), b = *(const f32x4*)(p.b_next + j * 4);
+                if (!AHEAD) next_weight(c, j);
                 f32x4 o;
 #pragma unroll
-                for (int k = 0; k < 4; k++) o[k] = ((x[c][k] - mean) / sd) * w[k] + b[k];
+                for (int k = 0; k < 4; k++) o[k] = ((x[c][k] - mean) / sd) * w2[c][k] + w3[c][k];
                 put(j, o);
             }
         }
@@ -542,10 +569,10 @@ __global__ __launch_bounds__(256) void sandwich_row_kernel(SandwichArgs p, ActT*
     for (int c = 0; c < MAXCH; c++) {
         const int j = threadIdx.x + c * 256;
         if (j < H4) {
-            const f32x4 w = *(const f32x4*)(p.w_next + j * 4);
+            if (!AHEAD) next_weight(c, j);
             f32x4 o;
 #pragma unroll
-            for (int k = 0; k < 4; k++) o[k] = (x[c][k] / rms) * w[k];
+            for (int k = 0; k < 4; k++) o[k] = (x[c][k] / rms) * w2[c][k];
             put(j, o);
         }
     }

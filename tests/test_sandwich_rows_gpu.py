@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 import medulorn_models as MM
-from layered_helpers import build, err
+from layered_helpers import build, err, feed
 
 pytestmark = pytest.mark.gpu
 BF16_LAYER = 0.03       # a single bf16 layer, as in the other tests of these models
@@ -33,3 +33,18 @@ def test_rows_and_tiles(gpu, tmp_path, layer, width, n):
     if "experts" in str(layer):
         tok = MM.clear_tokens(cfg, w, n, 1)[0]          # (no near tie between experts)
     against_fp32(gpu, tmp_path, cfg, w, list(tok))
+
+
+@pytest.mark.parametrize("layer,width", [(MM.attention(mlp=MM.moe(experts=96)), 96), (MM.attention(mlp=MM.moe(experts=80)), 2080), (MM.attention(mlp=MM.dense(48)), 4128)],
+                         ids=["six-parts", "five-parts", "wide"])
+def test_one_row_a_workgroup(gpu, tmp_path, layer, width):
+    """Single rows: more than four partial sums of the experts, and rows too wide for the weights of both norms to be fetched ahead."""
+    cfg = MM.config([layer, layer], width=width, vocab=130)
+    w = MM.weights(cfg, 11)
+    tok = MM.clear_tokens(cfg, w, 7, 1, margin=0.01)[0]          # (no near tie between experts)
+    got = {}
+    for precision in ("bf16", "f32"):
+        m = build(gpu, tmp_path, cfg, w, precision, max_seqs=2, max_seq_len=64, max_batch_tokens=64)
+        got[precision] = feed(m, 0, tok, [1] * len(tok))
+        m.close()
+    assert err(got["bf16"], got["f32"], "bf16") < 2 * BF16_LAYER          # (two layers)
