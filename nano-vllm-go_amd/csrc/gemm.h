@@ -1204,6 +1204,37 @@ __device__ __forceinline__ bf16x8 weight_load(const bf16x8* p) {
 // p: A (fragment-major operand, possibly the deferred-norm raw form with rs_in), M, K.  smem: MOE_ROUTE_LDS
 // ------------------------------------------------------------------------------------------
 struct RouteIds { int32_t* ids; float* w; };      // [row][top_k], or NULL
+// one row's logits, an expert a lane (-inf beyond them) -> its column of the gate matrix, or the chosen experts in rank order
+__device__ __forceinline__ void moe_route_row(const RouteJob& r, const RouteIds& out, int m, float v, int lane) {
+    const int E = r.E;
+    if (r.logits && lane < E) r.logits[(int64_t)m * r.logits_ld + lane] = v;
+    float mx = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    const float e = (lane < E) ? expf(v - mx) : 0.f;
+    float sum = e;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) sum += __shfl_xor(sum, o, 64);
+    const float prob = (lane < E) ? e / sum : -1.f;
+    int rank = 0;                                   // larger first, ties to the lower index (moe.go:75-92)
+    const int pbits = __builtin_bit_cast(int, prob), key = score_key(prob);
+#pragma unroll 8
+    for (int j = 0; j < E; j++) {                   // (lanes >= E hold -1: they never outrank an expert)
+        const int kj = __builtin_amdgcn_readlane(key, j);
+        rank += (kj > key || (kj == key && j < lane)) ? 1 : 0;
+    }
+    float wsum = 0.f;
+    for (int k = 0; k < r.top_k; k++) {             // moe.go:89-92: fp32 sum in rank order
+        const int src = __ffsll((unsigned long long)__ballot(rank == k)) - 1;
+        wsum += __builtin_bit_cast(float, __builtin_amdgcn_readlane(pbits, src));
+    }
+    if (out.ids) {
+        if (lane < E && rank < r.top_k) { out.ids[(int64_t)m * r.top_k + rank] = lane; out.w[(int64_t)m * r.top_k + rank] = prob / wsum; }
+        return;
+    }
+    if (lane < E) r.gate[(int64_t)m * r.gate_ld + lane] = rank < r.top_k ? prob / wsum : 0.f;      // moe.go:103
+    for (int e2 = E + lane; e2 < r.gate_ld; e2 += 64) r.gate[(int64_t)m * r.gate_ld + e2] = e2 < E + r.n_always ? 1.0f : 0.f;
+}
 // ALONE: sixteen waves, a slice of a tile and a row each: without the loops a launch of its own takes 5.7 us instead of 6.4 (1 row of 1024, 32 experts; code
 // that is fetched cold)
 template <int U, int T, bool ALONE = false>
@@ -1309,35 +1340,7 @@ __device__ __forceinline__ void moe_route_rows(const GemmArgs& p, const RouteJob
         const int row = first + i, m = row0 + row;
         if (!ALONE && p.rs_in && i != wave) ssq = sum_squares(m);
         const float rstd = p.rs_in ? 1.0f / sqrtf(ssq * p.rs_inv_h + p.rs_eps) : 1.0f;
-        const float v = (lane < E) ? lg[row * 64 + lane] * rstd + (r.bias ? r.bias[lane] : 0.f) : -INFINITY;
-        if (r.logits && lane < E) r.logits[(int64_t)m * r.logits_ld + lane] = v;
-        float mx = v;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-        const float e = (lane < E) ? expf(v - mx) : 0.f;
-        float sum = e;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) sum += __shfl_xor(sum, o, 64);
-        const float prob = (lane < E) ? e / sum : -1.f;
-        int rank = 0;                                   // larger first, ties to the lower index (moe.go:75-92)
-        const int pbits = __builtin_bit_cast(int, prob), key = score_key(prob);
-#pragma unroll 8
-        for (int j = 0; j < E; j++) {                   // (lanes >= E hold -1: they never outrank an expert)
-            const int kj = __builtin_amdgcn_readlane(key, j);
-            rank += (kj > key || (kj == key && j < lane)) ? 1 : 0;
-        }
-        float wsum = 0.f;
-        for (int k = 0; k < r.top_k; k++) {             // moe.go:89-92: fp32 sum in rank order
-            const int src = __ffsll((unsigned long long)__ballot(rank == k)) - 1;
-            wsum += __builtin_bit_cast(float, __builtin_amdgcn_readlane(pbits, src));
-        }
-        if (out.ids) {
-            if (lane < E && rank < r.top_k) { out.ids[(int64_t)m * r.top_k + rank] = lane; out.w[(int64_t)m * r.top_k + rank] = prob / wsum; }
-            if (ALONE) return;
-            continue;
-        }
-        if (lane < E) r.gate[(int64_t)m * r.gate_ld + lane] = rank < r.top_k ? prob / wsum : 0.f;      // moe.go:103
-        for (int e2 = E + lane; e2 < r.gate_ld; e2 += 64) r.gate[(int64_t)m * r.gate_ld + e2] = e2 < E + r.n_always ? 1.0f : 0.f;
+        moe_route_row(r, out, m, lane < E ? lg[row * 64 + lane] * rstd + (r.bias ? r.bias[lane] : 0.f) : -INFINITY, lane);
         if (ALONE) return;
     }
 }

@@ -901,9 +901,101 @@ bool sandwich_copies_rows(const nvl_model* m, int rows) { return !m->f32 && rows
 // us a prompt of 2048 columns, tiles and whole K from 513 rows on -> here: 18 layers with experts 513 / 750 / 1000 rows 3505 -> 3174, 3813 -> 3517, 4060 -> 3847; delta rule
 // and latent attention 513 / 750 / 1000 2786 -> 2596, 3217 -> 3070, 3512 -> 3479
 constexpr int SANDWICH_ROW_KERNEL_ROWS = 1024;
+// sandwich_row_kernel of a row that experts' routing follows (bf16, a norm behind the sublayer and none in front of the next, up to 64 experts), and the routing: the
+// row's four waves have it in LDS when the sixteen that the router's K slices take (gemm.h moe_route_rows: the same slices and sums, so the same choice as in
+// a launch of its own) have their weights.  What a launch of its own waits for, it and the first of its weights, is then over.  Sums and stores of the row
+// as there.  us, norm + routing -> one launch, 6 rows of 2048, 32
+// experts: 4.4 + 7.3 -> 7.5, a step with six of them 879 -> 861; steps of 16 rows 0.4 % faster, of 40 the same
+template <int MAXCH>
+__global__ __launch_bounds__(1024) void sandwich_route_kernel(SandwichArgs p, bf16_t* __restrict__ xn, RouteJob job) {
+    constexpr int PARTS = MAXCH <= 2 ? 4 : 2, STEPS = MAXCH <= 2 ? 8 : 4;      // (128 registers a wave)
+    __shared__ float red[4];
+    __shared__ __attribute__((aligned(16))) bf16_t row[MAXCH * 1024];
+    __shared__ f32x4 sums[16 * 4];                  // [K slices][expert tiles][16 experts]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), fg = lane >> 4;
+    const int r = blockIdx.x, H4 = p.H >> 2;
+    const bool has_row = wave < 4;
+    float* xr = p.x + (int64_t)r * p.H;
+    f32x4 x[MAXCH], y[MAXCH], e[MAXCH][PARTS], w[MAXCH];
+#pragma unroll
+    for (int c = 0; c < MAXCH; c++) {
+        const int j = threadIdx.x + c * 256;
+        x[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+        y[c] = x[c];
+        if (has_row && j < H4) {
+            x[c] = *(const f32x4*)(xr + j * 4);
+#pragma unroll
+            for (int k = 0; k < PARTS; k++) if (k == 0 || k < p.slices) e[c][k] = *(const f32x4*)(p.y + k * p.slice_stride + (int64_t)r * p.H + j * 4);
+            w[c] = *(const f32x4*)(p.w_post + j * 4);
+        }
+    }
+    const int ET = (job.E + 15) >> 4, KW = 16 / ET, tile = wave % ET, kw = wave / ET;
+    const int nks = p.H >> 5, q = nks / KW, rr = nks - q * KW;
+    const int n = kw < KW ? q + (kw < rr ? 1 : 0) : 0, ks0 = kw * q + (kw < rr ? kw : rr);      // (three tiles leave a wave idle)
+    const bf16_t* wp = job.W + (((int64_t)tile * nks + ks0) * 64 + lane) * 8;
+    bf16x8 wr[STEPS];
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) if (s < n) wr[s] = *(const bf16x8*)(wp + (int64_t)s * 512);
+    const float bias = wave == 0 && job.bias && lane < job.E ? job.bias[lane] : 0.f;
+    if (has_row) {
+        float ss = 0.f;
+#pragma unroll
+        for (int c = 0; c < MAXCH; c++) {
+            const int j = threadIdx.x + c * 256;
+            if (j < H4) {
+                y[c] = e[c][0];
+#pragma unroll
+                for (int k = 1; k < PARTS; k++) if (k < p.slices) y[c] += e[c][k];
+                for (int k = PARTS; k < p.slices; k++) y[c] += *(const f32x4*)(p.y + k * p.slice_stride + (int64_t)r * p.H + j * 4);
+            }
+            if (p.sum_scale != 0.f) { x[c] = p.sum_scale * x[c] + y[c]; y[c] = x[c]; }
+            ss += y[c][0] * y[c][0] + y[c][1] * y[c][1] + y[c][2] * y[c][2] + y[c][3] * y[c][3];
+        }
+        ss = wave_sum(ss);
+        if (lane == 0) red[wave] = ss;
+    }
+    __syncthreads();
+    if (has_row) {
+        const float rms = sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)p.width + p.eps);
+#pragma unroll
+        for (int c = 0; c < MAXCH; c++) {
+            const int j = threadIdx.x + c * 256;
+            if (j < H4) {
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const float v = (y[c][k] / rms) * w[c][k];
+                    x[c][k] = p.sum_scale != 0.f ? v : x[c][k] + v;
+                }
+                *(f32x4*)(xr + j * 4) = x[c];
+                act_store4<bf16_t>(xn, r, j * 4, p.H, x[c]);
+                store_row4(row + j * 4, x[c]);
+            }
+        }
+    }
+    __syncthreads();
+    // (the row stands in all sixteen columns of the operand)
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < n; s0 += STEPS) {
+#pragma unroll
+        for (int s = 0; s < STEPS; s++) if (s0 + s < n) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[s], *(const bf16x8*)(row + (ks0 + s0 + s) * 32 + fg * 8), acc, 0, 0, 0);
+#pragma unroll
+        for (int s = 0; s < STEPS; s++) if (s0 + STEPS + s < n) wr[s] = *(const bf16x8*)(wp + (int64_t)(s0 + STEPS + s) * 512);
+    }
+    if ((lane & 15) == 0 && kw < KW) sums[wave * 4 + fg] = acc;
+    __syncthreads();
+    if (wave) return;
+    float v = -INFINITY;
+    if (lane < job.E) {
+        v = ((const float*)sums)[lane];
+#pragma unroll 4
+        for (int k = 1; k < KW; k++) v += ((const float*)sums)[k * ET * 16 + lane];
+        v += bias;
+    }
+    moe_route_row(job, RouteIds{nullptr, nullptr}, r, v, lane);
+}
 // x += rms(y) * w_post (w_post NULL: x += y + experts; NVL_BLOCK_SUM_NORM: x = rms(stream_scale x + y + experts) * w_post) and / or
 // xn = next(x) (elem.h SandwichArgs)
-void sandwich(nvl_model* m, SubOut y, const float* w_post, NextNorm next, void* xn, int rows, const int32_t* rows_idx = nullptr, ExpertOut ex = {}, ShiftOut sh = {}, bf16_t* xn_rows = nullptr) {
+void sandwich(nvl_model* m, SubOut y, const float* w_post, NextNorm next, void* xn, int rows, const int32_t* rows_idx = nullptr, ExpertOut ex = {}, ShiftOut sh = {}, bf16_t* xn_rows = nullptr, const RouteJob* route = nullptr) {
     KScope ks(m, KC_OTHER, 0, KS_SANDWICH, (double)rows * m->Hn * ((y.y ? 8.0 + 4.0 * (std::max(y.slices, 1) + ex.slices) : 4.0) + (next.w || next.raw ? (double)m->wsize : 0.0)));
     SandwichArgs a{};
     a.x = m->x; a.y = y.y; a.slices = y.slices; a.slice_stride = y.stride; a.w_post = w_post; a.w_next = next.w; a.b_next = next.b; a.rows_idx = rows_idx;
@@ -913,7 +1005,11 @@ void sandwich(nvl_model* m, SubOut y, const float* w_post, NextNorm next, void* 
     if (sh.mu) { a.shift = sh.mu; a.before = sh.state; a.before_stride = m->rec_slot_stride; a.seq_slot = sh.md->seq_slot; a.seq_pos = sh.md->seq_pos; }
     const bool ext = (y.y && !w_post) || next.b || a.sum_scale != 0.f || sh.mu;
     a.xn_rows = xn_rows;
-    if (!m->f32 && rows > SANDWICH_ROW_KERNEL_ROWS && m->H <= 4096 && y.slices <= 1 && !sh.mu) {
+    if (route) {         // (routes_ahead)
+        if (m->H <= 1024) hipLaunchKernelGGL((sandwich_route_kernel<1>), dim3(rows), dim3(1024), 0, m->stream, a, (bf16_t*)xn, *route);
+        else if (m->H <= 2048) hipLaunchKernelGGL((sandwich_route_kernel<2>), dim3(rows), dim3(1024), 0, m->stream, a, (bf16_t*)xn, *route);
+        else hipLaunchKernelGGL((sandwich_route_kernel<4>), dim3(rows), dim3(1024), 0, m->stream, a, (bf16_t*)xn, *route);
+    } else if (!m->f32 && rows > SANDWICH_ROW_KERNEL_ROWS && m->H <= 4096 && y.slices <= 1 && !sh.mu) {
         const size_t lds = (size_t)NORM_TILE_ROWS * tile16_pitch(m->H) * 2;
 #define NVL_SWTE(CH, EXT)                                                                                                  \
         do {                                                                                                                \
@@ -1479,21 +1575,32 @@ void glu_up(nvl_model* m, const void* W, int M, int Fp, int act, float limit) {
 }
 // ---- experts that read m->xn by themselves, and their shared expert: returns what is added, the rest of it in `ex` ----
 // xn_rows: a row-major copy of m->xn, or NULL (it may lie in m->moe_eo)
-SubOut expert_ffn(nvl_model* m, const LayerRun& r, const MixerW& w, int M, ExpertOut& ex, const bf16_t* xn_rows) {
+// decode: masked projections over all experts (gemm.h GemmArgs::moe_gate)
+bool experts_masked(const nvl_model* m, const LayerRun& r, int M) { return !m->f32 && M <= 64 && r.Ip <= 2048; }
+RouteJob route_job(nvl_model* m, const LayerRun& r, const MixerW& w, int M) {
+    return {(const bf16_t*)w.router, w.route_bias, m->moe_gate, nullptr, r.c.experts, r.c.top_k, r.Ep, 0, experts_masked(m, r, M) ? r.shared_parts : 0};
+}
+bool one_route(const nvl_model* m, const LayerRun& r, int M) { return experts_masked(m, r, M) && r.c.experts <= 64 && r.c.route_softmax; }
+bool route_beside(const nvl_model* m, const LayerRun& r, int M) { return one_route(m, r, M) && moe_route_beside(M, r.c.experts, r.c.top_k, 2.0 * r.Ip * m->H * m->wsize); }
+// does the norm that makes the experts' input route too?
+bool routes_ahead(const nvl_model* m, const LayerRun& r, const MixerW& w, int M) {
+    return g_moe_fused_route == 1 && r.c.experts && one_route(m, r, M) && !route_beside(m, r, M) && w.norm1b && m->H <= 4096;
+}
+// routed: m->moe_gate is there (routes_ahead)
+SubOut expert_ffn(nvl_model* m, const LayerRun& r, const MixerW& w, int M, ExpertOut& ex, const bf16_t* xn_rows, bool routed) {
     const nvl_layer_config& c = r.c;
     const int E = c.experts, k = c.top_k, pairs = M * k;
-    const bool dense = !m->f32 && M <= 64 && r.Ip <= 2048;          // decode: masked projections over all experts (gemm.h GemmArgs::moe_gate)
-    const int parts = dense ? r.shared_parts : 0;
+    const bool dense = experts_masked(m, r, M), beside = route_beside(m, r, M);
+    const RouteJob job = route_job(m, r, w, M);
+    const int parts = job.n_always;
     SubOut y{nullptr, 1, 0};
     auto shared = [&] {
         const void* W = r.shared_parts && !m->f32 ? (const void*)((const char*)w.moe_up + (int64_t)E * 2 * r.Ip * m->H * (int64_t)m->wsize) : w.w1;
         glu_up(m, W, M, r.Fp, r.act, c.ffn_limit);
         y = sub_out(m, KS_FFN_DOWN, m->hbuf, w.w2, M, r.Fp);
     };
-    const RouteJob job{(const bf16_t*)w.router, w.route_bias, m->moe_gate, nullptr, E, k, r.Ep, 0, parts};
-    const bool one_route = dense && E <= 64 && c.route_softmax, route_beside = one_route && moe_route_beside(M, E, k, 2.0 * r.Ip * m->H * m->wsize);
-    if (route_beside) {
-    } else if (one_route) {
+    if (routed || beside) {
+    } else if (one_route(m, r, M)) {
         GemmArgs a = mk(m->xn, m->H, w.router, nullptr, E, w.route_bias, 1.f, M, E, m->H);
         KScope ks(m, KC_OTHER, 2.0 * M * E * m->Hn, KS_MOE_ROUTER, ((double)E * m->Hn + (double)M * m->Hn) * (double)m->wsize + (double)M * E * 4.0);
         hipLaunchKernelGGL(moe_router_gate_kernel, router_gate_grid(M), dim3(1024), 0, m->stream, a, job, RouteIds{nullptr, nullptr});
@@ -1512,7 +1619,7 @@ SubOut expert_ffn(nvl_model* m, const LayerRun& r, const MixerW& w, int M, Exper
         const double touch = (double)std::min(E, pairs) * c.expert_dim + (parts ? c.ffn_dim : 0), work = (double)pairs * c.expert_dim + (parts ? (double)M * c.ffn_dim : 0.0);
         GemmArgs u = mk(m->xn, m->H, w.moe_up, m->moe_hall, r.Ep * r.Ip, nullptr, 1.f, M, (E + parts) * 2 * r.Ip, m->H);
         u.moe_gate = m->moe_gate; u.moe_E = r.Ep; u.moe_I = r.Ip;
-        if (route_beside) u.route = job;
+        if (beside) u.route = job;
         u.glu_limit = c.expert_limit; u.glu_limit2 = c.ffn_limit; u.glu_from2 = E * r.Ip; u.glu_slope = CLAMPED_GLU_SLOPE;
         m->site = KS_MOE_UP; m->site_bytes = (2 * touch * m->Hn + (double)M * m->Hn + work) * (double)m->wsize;
         gemm(m, c.expert_limit > 0.f ? EPI_CLAMP_GLU : EPI_SWIGLU, false, u, 4.0 * work * m->Hn);
@@ -1622,10 +1729,12 @@ bool layered_stack(nvl_model* m, const Meta& md, int n_seqs, int M, int max_len,
             const bool apart = shift && !ones && li + 1 < m->L, ff = r.c.ffn_dim || r.c.experts;      // apart: the next mixer's input comes from shift_rows
             const NextNorm own{nullptr, nullptr, true}, close = apart ? NextNorm{nullptr, nullptr, false} : after;
             bf16_t* xn_rows = r.c.experts && sandwich_copies_rows(m, M) ? (bf16_t*)m->moe_eo : nullptr;      // (for the copy into expert order)
-            sandwich(m, y, w.norm1b, ff ? own : close, m->xn, M, nullptr, {}, ff ? ShiftOut{} : shift_out(li + 1), xn_rows);
+            const bool routed = routes_ahead(m, r, w, M);
+            const RouteJob job = routed ? route_job(m, r, w, M) : RouteJob{};
+            sandwich(m, y, w.norm1b, ff ? own : close, m->xn, M, nullptr, {}, ff ? ShiftOut{} : shift_out(li + 1), xn_rows, routed ? &job : nullptr);
             if (ff) {
                 ExpertOut ex;
-                if (r.c.experts) y = expert_ffn(m, r, w, M, ex, xn_rows);
+                if (r.c.experts) y = expert_ffn(m, r, w, M, ex, xn_rows, routed);
                 else { glu_up(m, w.w1, M, r.Fp, r.act, r.c.ffn_limit); y = sub_out(m, KS_FFN_DOWN, m->hbuf, w.w2, M, r.Fp); }
                 sandwich(m, y, w.norm2b, close, m->xn, M, nullptr, ex, shift_out(li + 1));
             }

@@ -48,3 +48,27 @@ def test_one_row_a_workgroup(gpu, tmp_path, layer, width):
         got[precision] = feed(m, 0, tok, [1] * len(tok))
         m.close()
     assert err(got["bf16"], got["f32"], "bf16") < 2 * BF16_LAYER          # (two layers)
+
+
+@pytest.mark.parametrize("experts,top,ff,width", [(8, 2, 1100, 2080), (33, 3, 448, 1056), (48, 3, 330, 992), (64, 2, 256, 1024)])      # one to four expert tiles, one to four chunks of a row a thread
+def test_routing_with_the_norm(gpu, tmp_path, experts, top, ff, width):
+    """Single rows whose experts' routing is in the launch of the norm that makes their input, against one of its own (nvl_set_tuning key 31 = 2)."""
+    cfg = MM.config([MM.attention(mlp=MM.moe(experts=experts, top=top, ff=ff)), MM.attention(mlp=MM.moe(experts=experts, top=top, ff=ff, shared=None))], width=width, vocab=130)
+    m = build(gpu, tmp_path, cfg, MM.weights(cfg, 11), "bf16", max_seqs=20, max_seq_len=64, max_batch_tokens=64)
+    m.set_profile(True)
+    g = np.random.default_rng(1)
+    for n in (1, 5, 17):
+        tok, got, launches, ids = g.integers(0, 130, (3, n)).tolist(), {}, {}, list(range(n))
+        for key in (1, 2):
+            old = gpu.lib().nvl_set_tuning(31, key)
+            try:
+                for i in ids:
+                    m.seq_reset(i)
+                m.reset_stats()
+                got[key] = [np.asarray(m.forward_batch(ids, [[t] for t in row], [p] * n)[0]) for p, row in enumerate(tok)]
+                launches[key] = sum(k["launches"] for k in m.kernel_stats() if k["site"] == "moe_router")
+            finally:
+                gpu.lib().nvl_set_tuning(31, old)
+        assert all(np.array_equal(a, b) for a, b in zip(got[1], got[2]))          # (the router's K slices and their sums are the same)
+        assert launches[1] == 0 and launches[2] > 0
+    m.close()
