@@ -1413,17 +1413,18 @@ __device__ __forceinline__ void resid_norm_tile(const GemmArgs& p, int m, int n,
 
 // m_passes > 1: block id -> (weight block, 64-row activation group).  Ids that differ by 8 share an XCD and are
 // dispatched back to back: the groups of one weight block stream the same weights at the same time.
+template <int ROWS = 64>
 __device__ __forceinline__ void skinny_pass_remap(GemmArgs& p, int& bx) {
     const int slot = bx >> 3, z = slot % p.m_passes;
     bx = (slot / p.m_passes) * 8 + (bx & 7);
-    p.A = (const bf16_t*)p.A + (int64_t)z * 64 * p.K;      // fragment-major: 16-row tiles are contiguous
-    p.c_row0 += z * 64;
-    p.M = min(64, p.M - z * 64);                           // the last group may be ragged (operands are padded to 64 rows)
-    if (p.rs_in) p.rs_in += (int64_t)z * 64 * p.rs_tiles;  // deferred RMSNorm: this group's rows of the x^2 partials
+    p.A = (const bf16_t*)p.A + (int64_t)z * ROWS * p.K;    // fragment-major: 16-row tiles are contiguous
+    p.c_row0 += z * ROWS;
+    p.M = min(ROWS, p.M - z * ROWS);                       // the last group may be ragged (operands are padded to 64 rows)
+    if (p.rs_in) p.rs_in += (int64_t)z * ROWS * p.rs_tiles;    // deferred RMSNorm: this group's rows of the x^2 partials
     if (p.rs_out) {                                        // ... and on the producer side (its epilogue indexes rows locally)
-        p.C = (float*)p.C + (int64_t)z * 64 * p.ldc;
-        p.nrm_xn += (int64_t)z * 64 * p.N;
-        p.rs_out += (int64_t)z * 64 * (p.N >> 4);
+        p.C = (float*)p.C + (int64_t)z * ROWS * p.ldc;
+        p.nrm_xn += (int64_t)z * ROWS * p.N;
+        p.rs_out += (int64_t)z * ROWS * (p.N >> 4);
     }
 }
 
@@ -1825,7 +1826,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(GemmArgs p) {
 // NTB MFMAs instead of one: L2->CU traffic per weight byte drops from 1 + MT to 1 + MT/NTB (the activation
 // fetches were costing ~15 % of the streaming rate, r01 probe).  8 waves per workgroup (256-VGPR budget): two
 // register sets of U k-steps x (NTB weight + MT activation) fragments — for K = 2048 a wave's whole slice is in
-// flight at once.  Same deterministic in-LDS K reduction and fused epilogues as the narrow form.
+// flight at once.  Same deterministic in-LDS K reduction and fused epilogues as the narrow form.  launch_gemm_rows runs it over row groups of 32 .. 64.
 // ------------------------------------------------------------------------------------------
 template <int MT, int NTB, int U, int EPI, typename OutT, bool PASSES = false, int MOE = 0>
 __global__ __launch_bounds__(512) void gemm_skinny_wide_bf16_kernel(GemmArgs p) {
@@ -1837,7 +1838,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_wide_bf16_kernel(GemmArgs p) 
     const int ksplit = blockDim.x >> 6;
     const int fr = lane & 15, fg = lane >> 4;
     int bx = blockIdx.x;
-    if constexpr (PASSES) skinny_pass_remap(p, bx);     // (its own instantiation: rewriting the arguments costs the
+    if constexpr (PASSES) skinny_pass_remap<16 * MT>(p, bx);     // (its own instantiation: rewriting the arguments costs the
                                                         // single-group kernels a few scratch dwords otherwise)
     if constexpr (MOE == 2) {
         if (bx < p.route.wgs) { moe_route_part<8, 2>(p, bx, ksplit, smem); return; }
@@ -1886,6 +1887,12 @@ __global__ __launch_bounds__(512) void gemm_skinny_wide_bf16_kernel(GemmArgs p) 
     };
     if (nblk > 0) load_blk(wA, xA, 0);
     stamps.mark(1);
+    // (residual: the old values of this wave's epilogue element come under the stream)
+    f32x4 x_pre = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (EPI == EPI_RESID) {
+        const int t = kw / MT, m = 16 * (kw - t * MT) + fr, n = (nt0 + t) * 16 + 4 * fg;
+        if (t < NTB && m < p.M && n < p.N) x_pre = *(const f32x4*)((const float*)p.C + (int64_t)(p.rs_out ? m : p.c_row0 + m) * p.ldc + n);
+    }
     int b = 0;
     for (; b + 2 <= nblk; b += 2) {
         load_blk(wB, xB, b + 1);
@@ -1930,6 +1937,17 @@ __global__ __launch_bounds__(512) void gemm_skinny_wide_bf16_kernel(GemmArgs p) 
     } else {
         for (int e = kw; e < NTB * MT; e += ksplit) {
             const int t = e / MT, i = e - t * MT;
+            if constexpr (EPI == EPI_RESID) {
+                f32x4 v = ksum(t, i);
+                const int m = 16 * i + fr, n = (nt0 + t) * 16 + 4 * fg;
+                if (p.bias) v += *(const f32x4*)(p.bias + n);
+                if (p.rs_out) resid_norm_tile(p, m, n, v, e == kw ? &x_pre : nullptr);
+                else if (m < p.M) {
+                    float* x = (float*)p.C + (int64_t)(p.c_row0 + m) * p.ldc + n;
+                    *(f32x4*)x = (e == kw ? x_pre : *(f32x4*)x) + p.alpha * v;
+                }
+                continue;
+            }
             epilogue4<EPI, OutT>(p, 16 * i + fr, (nt0 + t) * 16 + 4 * fg, ksum(t, i),
                                  EPI != EPI_STORE ? 1.0f : (i == i_pre ? rstd_pre : deferred_rstd(p, 16 * i + fr)));
         }
@@ -2425,6 +2443,54 @@ static inline bool launch_gemm_mid(hipStream_t st, const GemmArgs& a) {
     return true;
 }
 
+// Projections of 33 .. 256 rows whose K is short (launch_gemm_rows): groups of 32, 48 or 64 rows by 16 or 32 columns on the wide decode form, all of K in each workgroup
+// and one round of them.  Up to eight k-steps of 32 a wave (K = 2048) are all in flight at once, four at a time above: nothing is handed over between workgroups, which is
+// what gemm_mid_bf16_kernel's parts of K spend 4 us on, and the groups of 64 rows on the narrow form, two k-steps at a time, wait for memory four times.
+// us by events, weights from HBM, before -> here: 3072 x 2048 at 70 / 96 / 128 rows 14.2 -> 11.1, 14.6 -> 11.8, 16.7 -> 13.6; 2048 x 2048 at 70 / 96 / 128 / 190 / 250
+// 12.8 -> 10.4, 13.1 -> 10.4, 14.4 -> 11.1, 13.3 -> 11.3, 14.9 -> 12.8; 1536 x 1024 at 96 / 190 8.4 -> 7.4, 12.2 -> 8.0; 2304 x 768 at 70 / 96 / 190 8.6 -> 7.8, 9.4 -> 7.5, 10.0 -> 8.9;
+// 768 x 768 8.5 -> 6.8, 768 x 3072 at 70 / 96 / 250 12.8 -> 9.8, 14.7 -> 10.0, 15.5 -> 12.1.  Not a longer K, where the hand-over is the smaller part: 2048 x 8192 at 96 / 150 / 250
+// 20.2 / 21.4, 20.8 / 24.1, 24.6 / 29.7, 2048 x 6144 at 96 17.1 / 18.4.
+inline int g_rows = 1;              // nvl_set_tuning key 46: 0 never, 2 wherever it applies
+static inline double rows_cost(int N, int K, int tiles) { return 1.3 + K / 256.0 * 0.14 * tiles + 0.14e-6 * N * K; }      // (in mid_cost's terms; tiles: of rows and columns)
+// row and column tiles of a workgroup: the fewest bytes that one round of workgroups allows (rows are padded to whole groups of 64)
+static inline bool rows_shape(int M, int N, int& mt, int& nt) {
+    mt = nt = 0;
+    for (int g = 1; g <= 8; g++)
+        for (int t = 1; t <= 2; t++) {
+            const int r = std::max(2, cdiv(cdiv(M, g), 16));
+            if (r > 4 || 16 * r * (g - 1) >= M || 16 * r * g > round_up(M, 64) || N % (128 * t) != 0 || N / (16 * t) * g > 256) continue;
+            if (!mt || r + t < mt + nt) { mt = r; nt = t; }
+        }
+    return mt > 0;
+}
+template <int MT, int NTB, int EPI, typename OutT>
+static inline void launch_gemm_rows_of(hipStream_t st, const GemmArgs& a) {
+    GemmArgs c = a;
+    c.m_passes = cdiv(a.M, 16 * MT);
+    const int nks = a.K >> 5;
+    int waves = std::min(8, std::max(1, nks / 4));
+    for (int w = waves; w >= 5; w--) if (nks % (4 * w) == 0) { waves = w; break; }      // (whole blocks of four steps)
+    NVL_LDS_ATTR((gemm_skinny_wide_bf16_kernel<MT, NTB, 4, EPI, OutT, true>), 8 * NTB * MT * 1024);
+    hipLaunchKernelGGL((gemm_skinny_wide_bf16_kernel<MT, NTB, 4, EPI, OutT, true>), dim3(a.N / (16 * NTB) * c.m_passes), dim3(waves * 64), waves * NTB * MT * 1024, st, c);
+}
+template <int EPI, typename OutT>
+static inline bool launch_gemm_rows(hipStream_t st, const GemmArgs& a) {
+    int mt, nt, parts;
+    if (!g_rows || a.M <= 32 || a.M > 256 || a.M > std::max(64, g_chunk_max_m) || a.K % 32 != 0 || a.a_rows || a.seg || a.sk_part || a.moe_gate || a.c_row0 || a.m_passes > 1 || g_force_tile || g_force_ntw ||
+        a.rs_half || (EPI == EPI_RESID && a.rs_in) || !rows_shape(a.M, a.N, mt, nt)) return false;
+    if (g_rows == 1) {
+        // (up to 64 rows: 2048 x 2048 at 40 / 64 10.2 -> 9.5, 10.6 -> 9.6; not 1024 x 1024 6.7 / 7.1, nor without a residual 3072 x 2048 at 40 10.6 / 10.6)
+        // (a short K leaves nothing to gain: measured from 768 on)
+        if (a.K < 768) return false;
+        if (a.M <= 64) { if (EPI != EPI_RESID || a.K <= 1024 || a.K > 2048) return false; }
+        else if (mid_wins<EPI, OutT>(a) && rows_cost(a.N, a.K, mt + nt) > mid_cost(a.M, a.N, a.K, mid_row_tiles(a.M), 2, a.split_units > 0, parts)) return false;
+    }
+#define NVL_RW(MT, NT) if (mt == MT && nt == NT) launch_gemm_rows_of<MT, NT, EPI, OutT>(st, a)
+    NVL_RW(2, 1); NVL_RW(2, 2); NVL_RW(3, 1); NVL_RW(3, 2); NVL_RW(4, 1); NVL_RW(4, 2);
+#undef NVL_RW
+    return true;
+}
+
 template <int EPI, typename OutT>
 void launch_gemm_bf16(hipStream_t st, const GemmArgs& a) {
     if constexpr (epi_ln(EPI)) {
@@ -2435,6 +2501,7 @@ void launch_gemm_bf16(hipStream_t st, const GemmArgs& a) {
         return;
     } else {
     if (a.tile_map) { launch_gemm_grouped<EPI, OutT>(st, a, a.M); return; }   // a.M carries the m-tile bound
+    if constexpr (EPI == EPI_RESID || (EPI == EPI_STORE && std::is_same_v<OutT, float>)) if (launch_gemm_rows<EPI, OutT>(st, a)) return;
     if (launch_gemm_mid<EPI, OutT>(st, a)) return;
     if (launch_gemm_skinny_bf16<EPI, OutT>(st, a)) return;
     if constexpr (EPI != EPI_QKV) {

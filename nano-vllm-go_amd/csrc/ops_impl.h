@@ -438,6 +438,7 @@ extern "C" int nvl_set_tuning(int key, int value) {
     if (key == 37) { const int old = g_grouped_split; g_grouped_split = value < 0 || value > GROUPED_SPLITS ? 0 : value; return old; }
     if (key == 42) { const int old = g_grouped_qk; g_grouped_qk = value; return old; }
     if (key == 38) { const int old = g_mid; g_mid = value; return old; }
+    if (key == 46) { const int old = g_rows; g_rows = value; return old; }
     if (key == 40) { const int old = g_mid_resid_rows; g_mid_resid_rows = value; return old; }
     if (key == 39) { const int old = g_mid_splits; g_mid_splits = value; return old; }
     if (key == 36) { const int old = g_wide_ntb; g_wide_ntb = value; return old; }

@@ -377,3 +377,41 @@ def test_norm_tiles(gpu, family, hidden, heads, lens):
             gpu.lib().nvl_set_tuning(9, old)
             m.close()
     assert np.isfinite(got[0]).all() and rel_err(got[0], got[1]) < 3 * 2.0 ** -8
+
+
+@pytest.mark.parametrize("m,k,n", [(33, 64, 128), (64, 2048, 128), (65, 768, 2304), (70, 2112, 256), (96, 3072, 768), (97, 1536, 1024), (128, 4544, 128), (129, 2048, 2048),
+                                   (145, 960, 1280), (200, 2048, 1024), (250, 1088, 2048), (256, 2048, 2048), (80, 2048, 3072), (100, 1024, 4096)])
+def test_rows_form_is_exact_on_integers(gpu, m, k, n):
+    """Groups of 32, 48 and 64 rows by one and two column tiles with all of K in a workgroup (forced), five to eight waves, K steps that leave a rest of a block of
+    four, waves without any; ragged last groups."""
+    a = (np.arange(m * k).reshape(m, k) % 7).astype(np.float32) - 1.0
+    b = (np.arange(k * n).reshape(k, n) % 5).astype(np.float32) - 2.0        # |sums| < 2^24
+    old = gpu.lib().nvl_set_tuning(46, 2)
+    try:
+        got = gpu.ops.mat_mul(a, b, precision="bf16")
+    finally:
+        gpu.lib().nvl_set_tuning(46, old)
+    assert np.array_equal(got, (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32))
+
+
+@pytest.mark.parametrize("hidden,norm", [(768, "rmsnorm"), (2048, "rmsnorm"), (768, "layernorm")])
+@pytest.mark.parametrize("n", [33, 49, 64, 65, 96, 97, 128, 129, 200, 256])      # 128: the most rows of a deferred norm
+def test_rows_form_in_a_model(gpu, hidden, norm, n):
+    """Its epilogues: rows of a deferred norm's consumer, residuals that carry the next norm and plain ones, in steps and short prompts, against the fp32 mode."""
+    family = "llama" if norm == "rmsnorm" else "gpt2"
+    cfg = gpu.synth.tiny_config(family, hidden=hidden, num_heads=hidden // 64, num_kv_heads=hidden // (256 if family == "llama" else 64), head_dim=64, ffn_dim=hidden, max_seq_len=64)
+    w = gpu.synth.make_weights(cfg, seed=4, scale=0.02)
+    tok, ids, got = np.random.default_rng(n).integers(0, cfg["vocab_size"], (3, n)).tolist(), list(range(n)), {}
+    old = gpu.lib().nvl_set_tuning(46, 2)
+    try:
+        for precision in ("bf16", "f32"):
+            m = gpu.HipTransformerModel(cfg, w, precision=precision, max_seqs=n, max_batch_tokens=512)
+            for i in ids:
+                m.seq_reset(i)
+            got[precision] = [np.asarray(m.forward_batch(ids, [[t] for t in row], [p] * n)[0]) for p, row in enumerate(tok)]
+            m.seq_reset(0)
+            got[precision].append(np.asarray(m.forward_batch([0], [(tok[0] + tok[1])[:min(n, 64)]], [0])[0]))
+            m.close()
+    finally:
+        gpu.lib().nvl_set_tuning(46, old)
+    assert all(rel_err(a, b) <= TOL for a, b in zip(got["bf16"], got["f32"]))
