@@ -1556,7 +1556,34 @@ __global__ __launch_bounds__(skinny_waves(EPIV, MOE == 2 && MT > 1) * 64) void g
             if constexpr (LN_SHIFT) mean_acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c, x[u][0], mean_acc[u], 0, 0, 0);
         }
     };
+    // carried layer norms: the steps behind the last whole block are on their way beside it.  One after the other behind it, GPT-2's six steps a wave waited for memory
+    // three times: us by events, 8 rows, 3072 x 768 8.1 -> 7.2; a prompt of 11 tokens 484 -> 453 us, a step of 1 / 8 / 24 / 48 sequences 372 -> 352, 409 -> 380,
+    // 461 -> 437, 557 -> 546.  The others have no such widths and lose by the code alone (Falcon-7B, 142 steps a wave, 37.8 -> 40.3 us a launch; Llama-3.2-1B steps
+    // 1 %), and spill where they have several row tiles and 128 registers
+    constexpr bool TAIL = LN;
+    const int tail = TAIL ? __builtin_amdgcn_readfirstlane(my_steps - nblk * U) : 0;      // (uniform: matrix products heed no lane mask)
+    auto load_tail = [&](bf16x8 (&w)[U], bf16x8 (&x)[U][MT], bf16x8& c) {
+#pragma unroll
+        for (int u = 0; u < U - 1; u++)
+            if (u < tail) {
+                const int64_t at = (int64_t)(nblk * U + u) * 512;
+                w[u] = w_live ? weight_load<PASSES>((const bf16x8*)(wp + at)) : x_zero;
+#pragma unroll
+                for (int i = 0; i < MT; i++) x[u][i] = x_live[i] ? *(const bf16x8*)(xp[i] + at) : x_zero;
+            }
+        if constexpr (LN_SHIFT) c = cp[nblk * U * 8];
+    };
+    auto comp_tail = [&](bf16x8 (&w)[U], bf16x8 (&x)[U][MT], bf16x8& c) {
+#pragma unroll
+        for (int u = 0; u < U - 1; u++)
+            if (u < tail) {
+#pragma unroll
+                for (int i = 0; i < MT; i++) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u], x[u][i], acc[i], 0, 0, 0);
+                if constexpr (LN_SHIFT) mean_acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c, x[u][0], mean_acc[u], 0, 0, 0);
+            }
+    };
     if (nblk > 0) load_blk(wA, xA, cA, 0);
+    else if (tail) load_tail(wA, xA, cA);
     stamps.mark(1);                     // first block of loads issued
     // the residual operand of this wave's first epilogue element (deferred-norm producer form): fetched under the weight
     // stream, not as a dependent round trip after the K reduction (this launch is the only writer of these elements)
@@ -1582,6 +1609,10 @@ __global__ __launch_bounds__(skinny_waves(EPIV, MOE == 2 && MT > 1) * 64) void g
             if (b + 2 < nblk) load_blk(wA, xA, cA, b + 2);
             comp_blk(wB, xB, cB);
         }
+        if (tail) {
+            if (nblk > 0) load_tail(wA, xA, cA);
+            comp_tail(wA, xA, cA);
+        }
     } else {
     int b = 0;
     for (; b + 2 <= nblk; b += 2) {
@@ -1589,28 +1620,16 @@ __global__ __launch_bounds__(skinny_waves(EPIV, MOE == 2 && MT > 1) * 64) void g
         comp_blk(wA, xA, cA);
         if (b == 0) stamps.mark_used(2, acc[0]);       // first block's data arrived and was used
         if (b + 2 < nblk) load_blk(wA, xA, cA, b + 2);
+        else if (tail) load_tail(wA, xA, cA);
         comp_blk(wB, xB, cB);
     }
-    if (b < nblk) comp_blk(wA, xA, cA);
+    if (b < nblk) {
+        if (tail) load_tail(wB, xB, cB);
+        comp_blk(wA, xA, cA);
+        if (tail) comp_tail(wB, xB, cB);
+    } else if (tail) comp_tail(wA, xA, cA);
     }
-    if constexpr (LN_SHIFT) {          // ragged tail: fewer than U k-steps
-        const int s0 = nblk * U, rest = __builtin_amdgcn_readfirstlane(my_steps - s0);      // (uniform: matrix products heed no lane mask)
-        if (rest > 0) {
-            cA = cp[s0 * 8];
-#pragma unroll
-            for (int u = 0; u < U - 1; u++)
-                if (u < rest) {
-                    wA[u] = w_live ? weight_load<PASSES>((const bf16x8*)(wp + (int64_t)(s0 + u) * 512)) : x_zero;
-                    xA[u][0] = x_live[0] ? *(const bf16x8*)(xp[0] + (int64_t)(s0 + u) * 512) : x_zero;
-                }
-#pragma unroll
-            for (int u = 0; u < U - 1; u++)
-                if (u < rest) {
-                    acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wA[u], xA[u][0], acc[0], 0, 0, 0);
-                    mean_acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cA, xA[u][0], mean_acc[u], 0, 0, 0);
-                }
-        }
-    } else
+    if constexpr (!TAIL)
     for (int s = nblk * U; s < my_steps; s++) {
         const bf16x8 w = w_live ? weight_load<PASSES>((const bf16x8*)(wp + (int64_t)s * 512)) : x_zero;
 #pragma unroll
