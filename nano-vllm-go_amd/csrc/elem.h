@@ -435,7 +435,7 @@ __device__ __forceinline__ float sandwich_sq_dev(const f32x4 (&x)[MAXCH], float 
 template <typename ActT, int MAXCH, bool EXT = false>
 __global__ __launch_bounds__(256) void sandwich_row_kernel(SandwichArgs p, ActT* __restrict__ xn) {
     __shared__ float red[4];
-    constexpr bool AHEAD = MAXCH <= 4;      // (wider rows have no registers for it)
+    constexpr bool AHEAD = MAXCH <= (EXT ? 2 : 4);      // (wider rows have no registers for it: 4096 columns with EXT 192 of them, two waves a SIMD)
     constexpr int PARTS = AHEAD ? 4 : 1;
     const int r = blockIdx.x, H4 = p.H >> 2;
     const int src = p.rows_idx ? p.rows_idx[r] : r;
