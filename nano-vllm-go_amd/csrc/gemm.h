@@ -401,6 +401,48 @@ __device__ __forceinline__ void epilogue_glu4(const GemmArgs& p, int m, int f, f
     act_store4<OutT>((OutT*)p.C, (int64_t)p.c_row0 + m, f, p.ldc, v);
 }
 
+// EPI_RESID of a wave's TM x TN tiles of 16 rows x 16 columns that all lie within N (N % 4 == 0): the old values of eight tiles are fetched ahead of the stores of the eight
+// before.  One at a time, a tile waits for its values and, since the counter runs in order, for the store of the tile before: 32 times for a wave of a 256 x 256 tile.
+// us, a prompt before -> here:
+// Llama-3-8B 6 of 200 .. 1400 tokens 49280 -> 48701 (O 158 -> 152, FFN-down 399 -> 387 by events), Llama-3.2-1B 8 x 512 7574 -> 7528 (32 x 512, whose CUs are all at it at once,
+// 137 both), hybrid 8 of 90 .. 600 5190 -> 5143, GPT-2 900 / 8 x 512 1019 -> 978, 1852 -> 1822
+template <int TM, int TN>
+__device__ __forceinline__ void epilogue_resid_tiles(const GemmArgs& p, int m0, int n0, f32x4 (&acc)[TM][TN]) {      // m0, n0: this lane's first row and column
+    constexpr int R = TN >= 8 ? 1 : 8 / TN < TM ? 8 / TN : TM;
+    static_assert(TM % R == 0, "whole groups of rows");
+    float* x = (float*)p.C + (int64_t)p.c_row0 * p.ldc + n0;
+    f32x4 old[2][R][TN], bias[TN];
+    if (p.bias)
+#pragma unroll
+        for (int j = 0; j < TN; j++) bias[j] = *(const f32x4*)(p.bias + n0 + 16 * j);
+    auto fetch = [&](int i0, f32x4 (&o)[R][TN]) {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const float* from = x + (int64_t)min(m0 + 16 * (i0 + r), p.M - 1) * p.ldc;
+#pragma unroll
+            for (int j = 0; j < TN; j++) o[r][j] = *(const f32x4*)(from + 16 * j);
+        }
+    };
+    fetch(0, old[0]);
+#pragma unroll
+    for (int i0 = 0; i0 < TM; i0 += R) {
+        if (i0 + R < TM) fetch(i0 + R, old[(i0 / R + 1) & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int m = m0 + 16 * (i0 + r);
+            if (m < p.M)
+#pragma unroll
+                for (int j = 0; j < TN; j++) {
+                    f32x4 v = acc[i0 + r][j];
+                    if (p.bias) v += bias[j];
+                    *(f32x4*)(x + (int64_t)m * p.ldc + 16 * j) = old[(i0 / R) & 1][r][j] + p.alpha * v;
+                }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
 // EPI_QKV: one wave sub-tile of TH*16 columns = one head (TH = 4: hd 64, TH = 8: hd 128).  The lane holds, for
 // token m, d = 16j + 4fg + r (j = 0..TH-1): the RoPE partner d + hd/2 is tile j + TH/2 of the SAME lane.
 template <int TH>
@@ -486,7 +528,8 @@ __device__ __forceinline__ void tile_coords(int pid, int tiles_m, int tiles_n, i
 template <int BM, int BN, int STAGES, int BK = G_BK>
 constexpr int gemm_lds_bytes() { return STAGES * (BM + BN) * BK * 2; }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int EPI, typename OutT, int BK = G_BK>
+// SLICES (EPI_RESID): K tiles dealt over gridDim.y, partial sums to sk_part (beside the residual's epilogue in one instance their launches lose 1 %)
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int EPI, typename OutT, int BK = G_BK, bool SLICES = false>
 __global__ __launch_bounds__(WAVES_M * WAVES_N * 64, (WAVES_M * WAVES_N == 4 && STAGES * BK <= 160) ? 2 : (BK == 32 && BM == 128) ? 4 : 1)
 void gemm_bf16_kernel(GemmArgs p) {
     constexpr int NW = WAVES_M * WAVES_N;
@@ -577,7 +620,7 @@ void gemm_bf16_kernel(GemmArgs p) {
     // norm that follows sums the slices into x (PendingResid: the kernel boundary is the synchronisation)
     const int nt_all = p.K / BK;
     int nt = nt_all, kt0 = 0;
-    if (EPI == EPI_RESID && p.sk_part) {
+    if (SLICES) {
         const int per = nt_all / (int)gridDim.y, extra = nt_all - per * (int)gridDim.y;
         kt0 = (int)blockIdx.y * per + ((int)blockIdx.y < extra ? (int)blockIdx.y : extra);
         nt = per + ((int)blockIdx.y < extra ? 1 : 0);
@@ -676,6 +719,8 @@ void gemm_bf16_kernel(GemmArgs p) {
     }
 
     // ---- epilogue: lane holds rows n = 4*fg + r of column m = fr of each 16x16 tile ----
+    if constexpr (EPI == EPI_RESID)
+        if (!SLICES && (p.N & 3) == 0 && n0 + (wn + 1) * (TN * 16) <= p.N) { epilogue_resid_tiles<TM, TN>(p, m0 + wm * (TM * 16) + fr, n0 + wn * (TN * 16) + 4 * fg, acc); return; }
 #pragma unroll
     for (int i = 0; i < TM; i++) {
         const int m = m0 + wm * (TM * 16) + i * 16 + fr;
@@ -690,7 +735,7 @@ void gemm_bf16_kernel(GemmArgs p) {
                 const int f = (ntile >> 1) * 16 + 4 * fg;
                 epilogue_glu4<EPI, OutT>(p, m, f, acc[i][j], acc[i][j + 1]);
             }
-        } else if (EPI == EPI_RESID && p.sk_part) {
+        } else if (SLICES) {
             GemmArgs q = p;                                   // this slice's partial tile: plain fp32 store, bias with slice 0
             q.C = p.sk_part + (int64_t)blockIdx.y * p.M * p.N; q.ldc = p.N; q.c_row0 = 0;
             if (blockIdx.y != 0) q.bias = nullptr;
@@ -946,6 +991,8 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_pp_kernel(GemmArgs p) {
     if (grp == 0) __builtin_amdgcn_s_barrier();         // pairs with the late group's last barrier
     if (SPLIT && split_tile >= 0 && !split_finish<TM * TN>(p, split_tile, part, p.splits, BM * BN * 4, wave, &acc[0][0], (int*)(smem + STAGES * STAGE_BYTES))) return;
 
+    if constexpr (EPI == EPI_RESID)
+        if ((p.N & 3) == 0 && n0 + (wn + 1) * (TN * 16) <= p.N) { epilogue_resid_tiles<TM, TN>(p, m0 + wm * (TM * 16) + fr, n0 + wn * (TN * 16) + 4 * fg, acc); return; }
 #pragma unroll
     for (int i = 0; i < TM; i++) {
         const int m = m0 + wm * (TM * 16) + i * 16 + fr;
@@ -2206,10 +2253,14 @@ static inline bool launch_gemm_ln_resid(hipStream_t st, const GemmArgs& a0) {
 template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int EPI, typename OutT, int BK = G_BK>
 static inline void launch_gemm_tile(hipStream_t st, const GemmArgs& a) {
     constexpr int lds = gemm_lds_bytes<BM, BN, STAGES, BK>();
-    NVL_LDS_ATTR((gemm_bf16_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, EPI, OutT, BK>), lds);
-    const int tiles = cdiv(a.M, BM) * cdiv(a.N, BN);
-    hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, EPI, OutT, BK>),
-                       dim3(tiles, (EPI == EPI_RESID && a.sk_part) ? a.sk_slices : 1), dim3(WAVES_M * WAVES_N * 64), lds, st, a);
+    auto launch = [&](auto slices, int n) {
+        constexpr bool SLICES = decltype(slices)::value;
+        NVL_LDS_ATTR((gemm_bf16_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, EPI, OutT, BK, SLICES>), lds);
+        hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, EPI, OutT, BK, SLICES>),
+                           dim3(cdiv(a.M, BM) * cdiv(a.N, BN), n), dim3(WAVES_M * WAVES_N * 64), lds, st, a);
+    };
+    if constexpr (EPI == EPI_RESID) if (a.sk_part) { launch(std::true_type{}, a.sk_slices); return; }
+    launch(std::false_type{}, 1);
 }
 
 // What a projection takes on the two prefill forms, in microseconds: fitted to 200 launches of 300 .. 16384 rows of 768 .. 28672 x 768 .. 22720, good to

@@ -82,3 +82,29 @@ def test_experts_of_few_rows(gpu, n):
             gpu.lib().nvl_set_tuning(17, old)
     m.close()
     assert rel_err(got[0], got[1]) <= TOL
+
+
+@pytest.mark.parametrize("tile", [1, 2, 3, 5])          # the ring, 256x128, lock-step 256x256, ping-pong
+@pytest.mark.parametrize("family,hd", [("llama", 64), ("llama", 128), ("gpt2", 64)])      # angles; biases
+@pytest.mark.parametrize("rows", [129, 300, 515])
+def test_epilogues_of_ragged_rows(gpu, tile, family, hd, rows):
+    """Residuals whose old values and query / key tiles whose angles are fetched ahead of the stores before them: last tiles of 1, 44 and 3 rows, against the fp32 mode; a second
+    sequence's keys in the blocks of a pool."""
+    cfg = gpu.synth.tiny_config(family, hidden=576, num_heads=8, num_kv_heads=8 if family == "gpt2" else 4, head_dim=hd, ffn_dim=1152, num_layers=2, max_seq_len=640)
+    w = gpu.synth.make_weights(cfg, seed=4, scale=0.03)
+    g = np.random.default_rng(rows)
+    tokens = [g.integers(0, cfg["vocab_size"], n).tolist() for n in (rows - 70, 70)]
+    got = []
+    old = gpu.lib().nvl_set_tuning(0, tile)
+    try:
+        for precision in ("f32", "bf16"):
+            m = gpu.HipTransformerModel(cfg, w, precision=precision, max_seqs=2, max_batch_tokens=640)
+            for i in (0, 1):
+                m.seq_reset(i)
+            out = list(m.forward_batch([0, 1], tokens, [0, 0], all_logits=True)[0])
+            out.append(np.asarray(m.forward_batch([0, 1], [[3], [5]], [len(t) for t in tokens])[0]))
+            got.append(np.concatenate([np.asarray(o).reshape(-1, cfg["vocab_size"]) for o in out]))
+            m.close()
+    finally:
+        gpu.lib().nvl_set_tuning(0, old)
+    assert rel_err(got[1], got[0]) <= TOL
