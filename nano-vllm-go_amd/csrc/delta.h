@@ -48,10 +48,6 @@ struct DeltaArgs {
     const float* norm_w; float eps; void* out; int64_t out_ld;
 };
 
-// Products whose results are stored next.  The compiler spaces the store from the product by counting instructions of any kind; where an earlier store and a lane read
-// were among them, the 11 it counted were too few with two workgroups a CU, and the last four columns of the tile were stored as they had been.
-__device__ __forceinline__ void products_done(f32x4& a, f32x4& b, f32x4& c, f32x4& d) { asm volatile("s_nop 15" : "+v"(a), "+v"(b), "+v"(c), "+v"(d)); }
-
 constexpr int DELTA_C = 32;            // tokens per chunk
 constexpr int DELTA_ORDERED = 64;       // sequences that the scan takes in the order of their lengths, at most
 constexpr int DELTA_SCAN_WAVES = 4;    // of a workgroup of the scan
@@ -413,7 +409,6 @@ __global__ __launch_bounds__(512, NK > 8 ? 2 : 4) void delta_prep_kernel(DeltaAr
         }
         times(k, ta, w);
         times(k, ba, q);
-        products_done(w[0], w[1], q[0], q[1]);
 #pragma unroll
         for (int tt = 0; tt < 2; tt++) {
             buffer_put4(ws, 16 * lane, 16 * delta_piece(i, tt), w[tt]);
@@ -425,7 +420,6 @@ __global__ __launch_bounds__(512, NK > 8 ? 2 : 4) void delta_prep_kernel(DeltaAr
         u[0] = u[1] = o[0] = o[1] = f32x4{0.f, 0.f, 0.f, 0.f};
         times(v, ta, u);
         times(v, ba, o);
-        products_done(u[0], u[1], o[0], o[1]);
         const auto ru = delta_rows(vr, tb, nv), ro = delta_rows(orow, tb, nv);
         const int c = 16 * i + 4 * fg;
 #pragma unroll
@@ -556,7 +550,6 @@ __global__ __launch_bounds__(DELTA_SCAN_WAVES * 64, NK > 8 ? 1 : 3) void delta_s
             }
             if (i & 1) __builtin_amdgcn_sched_barrier(0);        // (or all reads are hoisted to the front, and registers spill)
         }
-        products_done(u[0], u[1], o[0], o[1]);
         const auto ro = delta_rows(orow, c0, n - c0);
 #pragma unroll
         for (int tt = 0; tt < 2; tt++)
