@@ -563,7 +563,9 @@ int nvl_bench_gemm(int device, int M, int N, int K, int epi, int force_bnt, int 
  * them itself (default -1: by size; 0: none).
  * key 38: projections of up to 512 rows (beyond 64 as far as key 11 goes) on their own kernel, K split over workgroups (1, default,
  * by cost; 0 never; 2 wherever it applies);
- * key 39: the parts of K there (0, default: by cost; fewer where the workspace or K is too small for them); key 40: rows up to which it completes residual projections (default 256).
+ * key 39: the parts of K there (0, default: by cost; fewer where the workspace or K is too small for them);
+ * key 46: projections of 33 to 256 rows and a short K in one piece, in front of that kernel (1, default, by cost, and not where key 38 is 2 or key 39 is not 0; 0 never;
+ * 2 wherever it applies); key 40: rows up to which it completes residual projections (default 256).
  * key 21: hipGraph replay of decode passes (1, default; 0 = every launch eager).  key 22: decode MoE as two dense-masked
  * weight-streaming projections (1, default) or sort + grouped GEMMs (0).  key 23: largest payload (rows of the residual
  * stream) the tensor-parallel P2P all-reduce sends one-shot; above it reduce-scatter + all-gather (default 64).

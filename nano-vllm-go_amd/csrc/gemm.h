@@ -2557,7 +2557,7 @@ static inline bool launch_gemm_mid(hipStream_t st, const GemmArgs& a) {
 // 12.8 -> 10.4, 13.1 -> 10.4, 14.4 -> 11.1, 13.3 -> 11.3, 14.9 -> 12.8; 1536 x 1024 at 96 / 190 8.4 -> 7.4, 12.2 -> 8.0; 2304 x 768 at 70 / 96 / 190 8.6 -> 7.8, 9.4 -> 7.5, 10.0 -> 8.9;
 // 768 x 768 8.5 -> 6.8, 768 x 3072 at 70 / 96 / 250 12.8 -> 9.8, 14.7 -> 10.0, 15.5 -> 12.1.  Not a longer K, where the hand-over is the smaller part: 2048 x 8192 at 96 / 150 / 250
 // 20.2 / 21.4, 20.8 / 24.1, 24.6 / 29.7, 2048 x 6144 at 96 17.1 / 18.4.
-inline int g_rows = 1;              // nvl_set_tuning key 46: 0 never, 2 wherever it applies
+inline int g_rows = 1;              // nvl_set_tuning key 46: 0 never, 1 by cost unless keys 38 or 39 ask for the kernel of parts, 2 wherever it applies
 static inline double rows_cost(int N, int K, int tiles) { return 1.3 + K / 256.0 * 0.14 * tiles + 0.14e-6 * N * K; }      // (in mid_cost's terms; tiles: of rows and columns)
 // row and column tiles of a workgroup: the fewest bytes that one round of workgroups allows (rows are padded to whole groups of 64)
 static inline bool rows_shape(int M, int N, int& mt, int& nt) {
@@ -2586,6 +2586,7 @@ static inline bool launch_gemm_rows(hipStream_t st, const GemmArgs& a) {
     if (!g_rows || a.M <= 32 || a.M > 256 || a.M > std::max(64, g_chunk_max_m) || a.K % 32 != 0 || a.a_rows || a.seg || a.sk_part || a.moe_gate || a.c_row0 || a.m_passes > 1 || g_force_tile || g_force_ntw ||
         a.rs_half || (EPI == EPI_RESID && a.rs_in) || !rows_shape(a.M, a.N, mt, nt)) return false;
     if (g_rows == 1) {
+        if (g_mid == 2 || g_mid_splits) return false;
         // (up to 64 rows: 2048 x 2048 at 40 / 64 10.2 -> 9.5, 10.6 -> 9.6; not 1024 x 1024 6.7 / 7.1, nor without a residual 3072 x 2048 at 40 10.6 / 10.6)
         // (a short K leaves nothing to gain: measured from 768 on)
         if (a.K < 768) return false;

@@ -27,6 +27,58 @@ def test_matmul_is_exact_on_integers(gpu, parts, m, k, n):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("m,k,n", [(97, 4160, 2048), (129, 2048, 256), (70, 2048, 1024)])
+def test_a_forced_kernel_is_taken(gpu, m, k, n):
+    """Keys 38 and 39 go before the form that has all of K in a workgroup, which would take these sizes: K in one part, in three and in five are sums in three orders."""
+    r = np.random.default_rng(m)
+    a, b, got = r.standard_normal((m, k)).astype(np.float32), r.standard_normal((k, n)).astype(np.float32), {}
+    for mid, parts in ((2, 1), (2, 3), (2, 5), (1, 3)):
+        old = [(key, gpu.lib().nvl_set_tuning(key, v)) for key, v in ((38, mid), (39, parts))]
+        try:
+            got[mid, parts] = gpu.ops.mat_mul(a, b, precision="bf16")
+        finally:
+            for key, v in old:
+                gpu.lib().nvl_set_tuning(key, v)
+    assert not np.array_equal(got[2, 1], got[2, 3]) and not np.array_equal(got[2, 3], got[2, 5]) and not np.array_equal(got[2, 1], got[2, 5])
+    if k * n >= 4 << 20:                                                  # (below, one part by cost is not this kernel)
+        assert np.array_equal(got[1, 3], got[2, 3])
+    for y in got.values():
+        assert rel_err(y, got[2, 1]) <= 1e-5                                # (fp32 sums of the same products)
+
+
+@pytest.mark.parametrize("n", [65, 97, 128])
+def test_long_residual_projections_in_parts(gpu, n):
+    """FFN-down of 2048 x 8192 behind 65 .. 128 rows, with a deferred norm: K in one part and in several, one to three 16-row tiles a wave, against the fp32 mode."""
+    cfg = gpu.synth.tiny_config("llama", hidden=2048, num_heads=32, num_kv_heads=8, head_dim=64, ffn_dim=8192, num_layers=2, max_seq_len=64)
+    w = gpu.synth.make_weights(cfg, seed=8, scale=0.02)
+    r = np.random.default_rng(n)
+    prompts = [r.integers(0, cfg["vocab_size"], 1 + i % 3).tolist() for i in range(n)]
+    ids, got = list(range(n)), {}
+    m = gpu.HipTransformerModel(cfg, w, precision="bf16", max_seqs=n, max_batch_tokens=512)
+
+    def step(m):
+        for i in ids:
+            m.seq_reset(i)
+        m.forward_batch(ids, prompts, [0] * n, want_logits=False)
+        return m.forward_batch(ids, [[7]] * n, [len(p) for p in prompts])[0].copy()
+
+    for parts in (1, 3, 4):
+        old = [(key, gpu.lib().nvl_set_tuning(key, v)) for key, v in ((38, 2), (39, parts))]
+        try:
+            got[parts] = step(m)
+            assert np.array_equal(step(m), got[parts]), parts            # (the counters of the parts are zero again)
+        finally:
+            for key, v in old:
+                gpu.lib().nvl_set_tuning(key, v)
+    m.close()
+    m = gpu.HipTransformerModel(cfg, w, precision="f32", max_seqs=n, max_batch_tokens=512)
+    want = step(m)
+    m.close()
+    assert not np.array_equal(got[1], got[3]) and not np.array_equal(got[3], got[4])
+    for parts, y in got.items():
+        assert rel_err(y, want) <= TOL, parts
+
+
 @pytest.mark.parametrize("hd", [64, 128])
 @pytest.mark.parametrize("parts", [0, 3])                             # K split over workgroups; 0: the launcher's choice
 @pytest.mark.parametrize("n,mid", [(5, 2), (33, 2), (64, 1), (64, 2), (65, 1), (97, 1), (128, 1), (130, 1)])      # 130: past the deferred norm
