@@ -23,16 +23,17 @@ void delta_step_launch(hipStream_t st, const DeltaArgs& p, int n_seqs, bool fuse
     else if (f32) step_rows<true, float>(st, p, n_seqs);
     else step_rows<true, bf16_t>(st, p, n_seqs);
 }
-template <int NK, bool VEC>
+template <int NK, bool VEC, bool VECV>
 static void prep_as(hipStream_t st, const DeltaArgs& p, int n_seqs, int tokens) {
     constexpr int lds = delta_prep_lds_bytes<NK>();
-    NVL_LDS_ATTR((delta_prep_kernel<NK, VEC>), lds);
+    NVL_LDS_ATTR((delta_prep_kernel<NK, VEC, VECV>), lds);
     const int chunks = tokens / DELTA_C + n_seqs, per = 512;          // at most; workgroups that the chip holds
-    hipLaunchKernelGGL((delta_prep_kernel<NK, VEC>), dim3(p.H, std::min(chunks, std::max(1, per / p.H))), dim3(512), lds, st, p, n_seqs);
+    hipLaunchKernelGGL((delta_prep_kernel<NK, VEC, VECV>), dim3(p.H, std::min(chunks, std::max(1, per / p.H))), dim3(512), lds, st, p, n_seqs);
 }
 template <int NK>
 static void prep(hipStream_t st, const DeltaArgs& p, int n_seqs, int tokens) {
-    if (p.vec4 && p.vec4v) prep_as<NK, true>(st, p, n_seqs, tokens); else prep_as<NK, false>(st, p, n_seqs, tokens);
+    if (p.vec4) { if (p.vec4v) prep_as<NK, true, true>(st, p, n_seqs, tokens); else prep_as<NK, true, false>(st, p, n_seqs, tokens); }
+    else if (p.vec4v) prep_as<NK, false, true>(st, p, n_seqs, tokens); else prep_as<NK, false, false>(st, p, n_seqs, tokens);
 }
 void delta_prep_launch(hipStream_t st, const DeltaArgs& p, int n_seqs, int nk, int tokens) {
     if (nk == 2) prep<2>(st, p, n_seqs, tokens); else if (nk == 4) prep<4>(st, p, n_seqs, tokens); else if (nk == 8) prep<8>(st, p, n_seqs, tokens); else prep<16>(st, p, n_seqs, tokens);

@@ -30,7 +30,7 @@ def test_scan_parts(gpu, tmp_path, heads, dim, vdim):
     m.close()
 
 
-@pytest.mark.parametrize("dim,vdim", [(32, 32), (64, 64), (100, 72), (128, 136), (256, 256)])
+@pytest.mark.parametrize("dim,vdim", [(32, 32), (64, 64), (66, 64), (66, 66), (100, 72), (128, 130), (128, 136), (256, 256)])
 @pytest.mark.parametrize("lens", [[32], [33], [1, 31, 65, 96], [300] * 24])
 def test_scan_forms(gpu, tmp_path, dim, vdim, lens):
     """Chunks that end with the sequence or a token behind or before it, an odd and an even number of them; 24 equal sequences are more than the chip takes at once (all channels a wave).

@@ -70,7 +70,7 @@ def test_results_of_fp32_products_are_read_in_time(tmp_path):
     """A result of eight passes may be read ten wait states behind its product (the two passes beyond its own that the architecture asks for).  The compiler
     counts them; the kernels whose products are fp32 have no spacing of their own, so that what it leaves has to hold on every path to a store, to LDS and to a lane."""
     csrc = os.path.join(ROOT, "nano-vllm-go_amd", "csrc")
-    jobs = []
+    jobs, prep = [], {}
     for unit, macro in [("delta", None), ("linrec", 1), ("linrec", 2)]:
         out = tmp_path / f"{unit}{macro}.s"
         cmd = ["/opt/rocm/bin/hipcc", "-O3", "-std=c++17", "--offload-arch=gfx950", "-mllvm", "-amdgpu-kernarg-preload-count=6", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -79,11 +79,19 @@ def test_results_of_fp32_products_are_read_in_time(tmp_path):
     seen = set()
     for out, job in jobs:
         assert job.wait(timeout=600) == 0
-        found = product_readers(out.read_text())
+        asm = out.read_text()
+        found = product_readers(asm)
         assert found
+        for m in re.finditer(r"^_ZN3nvl17delta_prep_kernelILi(\d+)ELb(\d)ELb(\d)EEE\w*:.*?s_endpgm\n\t\.section", asm, re.M | re.S):
+            prep[m.groups()] = len(re.findall(r"buffer_load_dwordx4", m[0])), len(re.findall(r"buffer_load_dword ", m[0]))
         seen |= {k for k, _, _ in found}
         early = [f for f in found if f[1] < 10]
         assert not early, early[:5]
+    # the preparation reads keys 16 bytes at a time by their own width, whatever the values' is
+    assert len(prep) == 16
+    for (nk, keys, values), (wide, narrow) in prep.items():
+        assert wide == (prep[nk, "1", "1"][0] if keys == "1" else 0) and (narrow == prep[nk, "1", "1"][1] if keys == "1" else narrow > prep[nk, "1", "1"][1]), (nk, keys, values, wide, narrow)
+    assert prep["8", "1", "1"][0] > 0
     assert {n for n in ("delta_prep_kernel", "delta_scan_kernel", "delta_scan_parts_kernel") if any(n in k for k in seen)} == {"delta_prep_kernel", "delta_scan_kernel", "delta_scan_parts_kernel"}
 
 
