@@ -23,11 +23,15 @@ void delta_step_launch(hipStream_t st, const DeltaArgs& p, int n_seqs, bool fuse
     else if (f32) step_rows<true, float>(st, p, n_seqs);
     else step_rows<true, bf16_t>(st, p, n_seqs);
 }
+// Workgroups that the chip holds at once, by their LDS (160 KB a CU, 256 CUs) and by what a CU's registers hold of them; each goes from chunk to chunk.  Heads of 256 have one a CU:
+// launched for two, they made two rounds, us a layer 1 x 1900 tokens 98 -> 94, 5 x 300 .. 1900 215 -> 204, 200 x 128 channels, 10 x 400 175 -> 169
+template <int NK> constexpr int delta_prep_workgroups() { return 256 * std::min(160 * 1024 / delta_prep_lds_bytes<NK>(), 2); }
+static_assert(delta_prep_workgroups<8>() == 512 && delta_prep_workgroups<16>() == 256, "two workgroups a CU, heads of 256 one");
 template <int NK, bool VEC, bool VECV>
 static void prep_as(hipStream_t st, const DeltaArgs& p, int n_seqs, int tokens) {
     constexpr int lds = delta_prep_lds_bytes<NK>();
     NVL_LDS_ATTR((delta_prep_kernel<NK, VEC, VECV>), lds);
-    const int chunks = tokens / DELTA_C + n_seqs, per = 512;          // at most; workgroups that the chip holds
+    const int chunks = tokens / DELTA_C + n_seqs, per = delta_prep_workgroups<NK>();          // chunks: at most
     hipLaunchKernelGGL((delta_prep_kernel<NK, VEC, VECV>), dim3(p.H, std::min(chunks, std::max(1, per / p.H))), dim3(512), lds, st, p, n_seqs);
 }
 template <int NK>
