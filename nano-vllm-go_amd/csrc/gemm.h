@@ -2570,6 +2570,12 @@ static inline bool rows_shape(int M, int N, int& mt, int& nt) {
         }
     return mt > 0;
 }
+// ... of 33 to 64 rows, residual (others gain nothing: 3072 x 2048 at 40 rows 10.6 / 10.6).  Below 48 rows the narrow decode form leaves out what lies beyond them, and is as fast or
+// faster wherever it has workgroups for the whole chip.  us by events, that form / here, at 33, 47, 48 and 60 rows:
+//   1024 x 2048 7.2 / 5.9 at 34, 7.9 / 6.0 at 64   1024 x 1280 -7, -9, -15, -15 %   1024 x 1088 -2, -4, -9, -9 %
+//   2048 x 2048 -15, -17, -23, -23 %   x 1792 -9, -13, -21, -20 %   x 1536 +1, -2, -9, -8 %   x 1280 +5, +2, -5, -5 %   x 1088 +11, +8, +1, +2 %
+//   3072 x 2048 +7, +4, -5, -7 %   x 1536 +8, +5, -2, -4 %   4096 x 2048 +5, +1, -8, -9 %   x 1536 +4, +2, -5, -7 %   x 1088 +2, 0, -6, -2 %   1536 x 1088 +9, +7, 0, +1 %
+static inline bool rows_pay_few(int M, int N, int K) { return K > 1024 && K <= 2048 && (N <= 1024 || (M >= 48 ? K >= 1280 : N <= 2048 && K >= 1792)); }
 template <int MT, int NTB, int EPI, typename OutT>
 static inline void launch_gemm_rows_of(hipStream_t st, const GemmArgs& a) {
     GemmArgs c = a;
@@ -2587,10 +2593,10 @@ static inline bool launch_gemm_rows(hipStream_t st, const GemmArgs& a) {
         a.rs_half || (EPI == EPI_RESID && a.rs_in) || !rows_shape(a.M, a.N, mt, nt)) return false;
     if (g_rows == 1) {
         if (g_mid == 2 || g_mid_splits) return false;
-        // (up to 64 rows: 2048 x 2048 at 40 / 64 10.2 -> 9.5, 10.6 -> 9.6; not 1024 x 1024 6.7 / 7.1, nor without a residual 3072 x 2048 at 40 10.6 / 10.6)
         // (a short K leaves nothing to gain: measured from 768 on)
+        // (where the 64-row groups would be taken there is nothing to weigh: 18 sizes of 128 .. 4096 x 768 .. 16384 at 66 .. 250 rows, as they are and residual, +2 .. -46 %, most -10 .. -40)
         if (a.K < 768) return false;
-        if (a.M <= 64) { if (EPI != EPI_RESID || a.K <= 1024 || a.K > 2048) return false; }
+        if (a.M <= 64) { if (EPI != EPI_RESID || !rows_pay_few(a.M, a.N, a.K)) return false; }
         else if (mid_wins<EPI, OutT>(a) && rows_cost(a.N, a.K, mt + nt) > mid_cost(a.M, a.N, a.K, mid_row_tiles(a.M), 2, a.split_units > 0, parts)) return false;
     }
 #define NVL_RW(MT, NT) if (mt == MT && nt == NT) launch_gemm_rows_of<MT, NT, EPI, OutT>(st, a)

@@ -114,3 +114,18 @@ int main() {
     return sorted < 1000 || left < 1000;
 }
 """)
+
+
+@pytest.mark.skipif(HIPCC is None, reason="no hipcc")
+def test_few_rows_in_one_piece(tmp_path):
+    """Residual projections of 33 .. 64 rows: where the narrow form measured faster it is kept, where it measured slower it is not."""
+    run(tmp_path, r"""
+#include "gemm.h"
+int main() {
+    struct { int M, N, K; bool pays; } m[] = {{33, 4096, 2048, false}, {47, 4096, 1536, false}, {40, 3072, 1536, false}, {33, 2048, 1088, false}, {47, 2048, 1280, false}, {60, 2048, 1088, false},
+        {40, 1536, 1088, false}, {64, 1024, 1024, false}, {33, 2048, 2304, false}, {33, 2048, 2048, true}, {47, 2048, 1792, true}, {33, 1024, 1088, true}, {40, 512, 2048, true}, {48, 4096, 2048, true},
+        {60, 3072, 1536, true}, {48, 2048, 1280, true}};
+    for (auto& c : m) if (nvl::rows_pay_few(c.M, c.N, c.K) != c.pays) { printf("%d rows of %d x %d\n", c.M, c.N, c.K); return 1; }
+    return 0;
+}
+""")
