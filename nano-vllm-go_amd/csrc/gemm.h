@@ -447,7 +447,7 @@ __device__ __forceinline__ void epilogue_resid_tiles(const GemmArgs& p, int m0, 
 // token m, d = 16j + 4fg + r (j = 0..TH-1): the RoPE partner d + hd/2 is tile j + TH/2 of the SAME lane.
 // Positions and blocks of all rows are fetched together, a row's angles ahead of the stores of the row before (as epilogue_resid_tiles).  us by events, a row
 // after the other -> here: Llama-3.2-1B 32 x 512 / 8 x 512 / 1900 177 -> 169, 57.2 -> 54.4, 37.3 -> 34.9, Granite 16 of 150 .. 900 42.8 -> 38.9, GPT-2 8 x 512 32.9 -> 30.6,
-// heads of 128 87.7 -> 85.6 (Llama-3-8B 1500), Falcon-7B 900 60.9 -> 61.2
+// heads of 128 87.7 -> 85.6 (Llama-3-8B 1500); Falcon-7B 900, 71 of whose 73 heads are query heads, 60.9 -> 61.2 with lookups for all of them, 58.4 -> 58.1 without
 template <int TM, int TH>
 __device__ __forceinline__ void epilogue_qkv_tiles(const GemmArgs& p, int m0, int head, int fg, f32x4 (&acc)[TM][TH]) {      // m0: this lane's first row
     constexpr int HD = TH * 16;
@@ -476,7 +476,10 @@ __device__ __forceinline__ void epilogue_qkv_tiles(const GemmArgs& p, int m0, in
     };
     if (AHEAD) angles(0);
 #pragma unroll
-    for (int i = 0; i < TM; i++) kv_locate(q.blk_table, tbl[i], pos[i], q.Tmax, blk[i], row[i]);      // (query heads too: behind a branch each load is waited for)
+    for (int i = 0; i < TM; i++) blk[i] = row[i] = 0;
+    if (!AHEAD || cached)      // (one branch of the whole wave around all rows' lookups, which query heads don't need; for heads of 128 it costs more than they: Llama-3-8B 1500 84.0 -> 84.6)
+#pragma unroll
+        for (int i = 0; i < TM; i++) kv_locate(q.blk_table, tbl[i], pos[i], q.Tmax, blk[i], row[i]);
 #pragma unroll
     for (int i = 0; i < TM; i++) {
         if (!AHEAD) angles(i);
