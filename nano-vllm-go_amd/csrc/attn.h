@@ -254,6 +254,17 @@ __global__ __launch_bounds__(NW * 64, HD == 64 ? 4 : 2) void attn_prefill_bf16_k
             static_assert(PW == 2 || PW == 4 || PW == 8, "pieces of a tile per wave");
         } else {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            const int end = pos0 + S - 1;
+            if (end >> 6 == kt && (end & 63) != 63) {            // values behind the sequence's last key (common.h keys_up_to): by the wave that fetched them
+                int l = lane; unsigned z = 0;
+                asm volatile("" : "+v"(l), "+v"(z));             // (or rows, addresses and the zeros are kept in registers all along: 85 of them in place of 80, two workgroups a CU in place of three)
+#pragma unroll
+                for (int i = 0; i < PW; i++) {
+                    const int pc = wave * PW + i;
+                    if (pc >= PIECES && ((pc - PIECES) * 64 + l) / CPR > (end & 63)) *(u32x4*)(smem + buf * (2 * TILE_BYTES) + pc * 1024 + l * 16) = u32x4{z, z, z, z};
+                }
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            }
         }
         __builtin_amdgcn_s_barrier();
         if (kt + 2 < n_kt) { int nb = buf + 2; if (nb >= NBUF) nb -= NBUF; issue(kt + 2, nb); }
@@ -677,18 +688,19 @@ __global__ __launch_bounds__(NW * 64, HD == 128 ? 2 : 0) void attn_decode_bf16_k
                 for (int t = 0; t < 4; t++) s[h][t] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
                 continue;
             }
-            if (FUSED && !MORE && kt == n_kt - 1) {
-                // the tile that holds key pos0: its slab row is not written yet (or not visible): patch the operands
+            if (!MORE && kt == n_kt - 1) {
+                // the tile that holds key pos0: its slab row is not written yet (or not visible): patch the operands, and what lies behind (common.h keys_up_to)
                 const int kl = pos0 & 63;
+                if (FUSED)
 #pragma unroll
-                for (int t = 0; t < 4; t++)
-                    if (t == (kl >> 4) && fq == (kl & 15)) {
+                    for (int t = 0; t < 4; t++)
+                        if (t == (kl >> 4) && fq == (kl & 15)) {
 #pragma unroll
-                        for (int ks = 0; ks < KS; ks++) kf[h][t][ks] = knew[ks];
-                    }
+                            for (int ks = 0; ks < KS; ks++) kf[h][t][ks] = knew[ks];
+                        }
 #pragma unroll
                 for (int i = 0; i < NVL; i++)
-                    if (i == kl / KPI && ksub == kl % KPI) vch[h][i] = vnew8;
+                    if (i * KPI + ksub >= kl + (FUSED ? 0 : 1)) vch[h][i] = FUSED ? vnew8 : bf16x8{};
             }
 #pragma unroll
             for (int t = 0; t < 4; t++) {

@@ -73,6 +73,17 @@ __device__ __forceinline__ void kv_locate(const int32_t* __restrict__ blk_table,
     row = pos - bi * bs;
 }
 
+// The last tile of a sequence's keys ends in places that it has not written.  Their weights are zero, but they hold what another sequence left there, and zero times an
+// infinity or a NaN is a NaN: the attention kernels take zeros (or a row of the sequence's own) in their stead.  Mask of eight values of consecutive keys, of which
+// those behind key `last` (of 0 .. 7, any below: none) are to go:
+__device__ __forceinline__ u32x4 keys_up_to(int last) {
+    u32x4 m;
+#pragma unroll
+    for (int j = 0; j < 4; j++) m[j] = last > 2 * j ? ~0u : last == 2 * j ? 0xffffu : 0u;
+    return m;
+}
+__device__ __forceinline__ bf16x8 keep_keys(bf16x8 v, u32x4 m) { return __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, v) & m); }
+
 // Grouped-query attention of models described by a list of layers (grouped.h) keeps keys as MFMA operand blocks whose rows are in the
 // order that makes the score accumulators the next product's operand: tile row 16 t + 4 a + r holds token 8 a + 4 t + r of its
 // 32-token unit.  Where token row `row` sits:

@@ -423,7 +423,7 @@ __global__ __launch_bounds__(512, (KS <= 2 && DT <= 4) ? 4 : 2) void grouped_pre
     const int fq = lane & 15, fg = lane >> 4;
     // key tiles of the workgroup, and of this wave (rows w_row0 .. + 31)
     const int wg_first = pos0 + qt * 256 / p.group, wg_last = pos0 + (min(qt * 256 + 255, R - 1)) / p.group;
-    const int t0 = p.mask.lo(wg_first) >> 6, n_kt = (wg_last >> 6) + 1;
+    const int t0 = p.mask.lo(wg_first) >> 6, n_kt = (wg_last >> 6) + 1, end = pos0 + p.seq_len[seq] - 1;
     const int keep_kt = (p.mask.keep + 63) >> 6, n_pre = min(t0, keep_kt), n_tiles = n_pre + n_kt - t0;      // (tiles of kept tokens before the window's)
     auto tile_at = [&](int i) { return i < n_pre ? i : t0 + i - n_pre; };
     const int w_row0 = qt * 256 + wave * 32;
@@ -520,6 +520,7 @@ __global__ __launch_bounds__(512, (KS <= 2 && DT <= 4) ? 4 : 2) void grouped_pre
     int buf = 0;
     for (int it = 0; it < n_tiles; it++) {
         if (it + 1 < n_tiles) wait_vm<PW>(); else wait_vm<0>();      // my pieces of this tile have landed
+        if (it + 1 == n_tiles && (end >> 6) == n_kt - 1 && (end & 63) != 63) tile_values_up_to<4 * KS, PIECES, PW>(grp_sm + buf * TILE, wave, lane, end & 63);
         __builtin_amdgcn_s_barrier();
         if (it + 2 < n_tiles) { int nb = buf + 2; if (nb >= NBUF) nb -= NBUF; issue(it + 2, nb); }
         const int kt = tile_at(it);
@@ -780,6 +781,13 @@ __global__ __launch_bounds__(NW * 64) void grouped_short_kernel(GroupedArgs p) {
 #pragma unroll
             for (int r = 0; r < 4; r++) { s[t][r] = __builtin_amdgcn_exp2f(s[t][r] - mn); l += s[t][r]; }
         const bf16x8 p0 = latent_pack_p(s[0], s[1]), p1 = latent_pack_p(s[2], s[3]);
+        if (kt * 64 + 63 > last)      // (common.h keys_up_to)
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const u32x4 keep = keys_up_to(last - kt * 64 - 32 * u - 8 * fg);
+#pragma unroll
+                for (int d = 0; d < DT; d++) vf[d][u] = keep_keys(vf[d][u], keep);
+            }
 #pragma unroll
         for (int d = 0; d < DT; d++) {
             o[d] *= alpha;

@@ -229,6 +229,25 @@ __device__ __forceinline__ void latent_store_o(const LatentArgs& p, int64_t tok,
 
 template <int KS, int DT> constexpr int latent_prefill_pieces() { return 4 * KS + 2 * DT; }       // 1-KiB blocks of a tile
 template <int KS, int DT> constexpr int latent_prefill_lds_bytes() { return 3 * ((latent_prefill_pieces<KS, DT>() + 7) / 8 * 8) * 1024; }
+// Values of a tile in LDS, blocks of [16 value rows][32 keys] behind KB blocks of keys, that lie behind its key `last`: zeros.  By the wave that fetched them, which has waited for them.
+template <int KB, int PIECES, int PW>
+__device__ __forceinline__ void tile_values_up_to(char* tile, int wave, int lane, int last) {
+    asm volatile("" : "+v"(lane));      // (or masks and addresses are kept in registers all along)
+    bf16x8* v = (bf16x8*)(tile + wave * PW * 1024 + lane * 16);
+#pragma unroll
+    for (int i0 = 0; i0 < PW; i0 += 2) {
+        const int n = i0 + 1 < PW ? 2 : 1;
+        bf16x8 x[2];
+#pragma unroll
+        for (int i = 0; i < n; i++) x[i] = v[(i0 + i) * 64];
+#pragma unroll
+        for (int i = 0; i < n; i++) {
+            const int pc = wave * PW + i0 + i;
+            if (pc >= KB && pc < PIECES) v[(i0 + i) * 64] = keep_keys(x[i], keys_up_to(last - 32 * ((pc - KB) & 1) - 8 * (lane >> 4)));
+        }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+}
 template <int N> __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
 template <int KS, int DT>
@@ -259,7 +278,7 @@ __global__ __launch_bounds__(512, (KS <= 2 && DT <= 4) ? 4 : 2) void latent_pref
     const LatentRows wg(p, seq, qt * 256);
     const int kb = p.kbase[seq];
     const int wg_last = wg.pos0 + min(qt * 256 + 255, wg.n - 1) - wg.k0;
-    const int t0 = wg.key_lo(p) >> 6, n_kt = (wg_last >> 6) + 1;
+    const int t0 = wg.key_lo(p) >> 6, n_kt = (wg_last >> 6) + 1, end = wg.pos0 + wg.n - 1 - wg.k0;
     const int wt0 = w_live ? w.key_lo(p) >> 6 : n_kt, wt1 = w_live ? ((w.last - w.k0) >> 6) + 1 : 0;
     const int full_lo = (p.window > 0 ? w.last - p.window + 1 : 0) - w.k0, full_hi = w.first - w.k0;
     // LDS-DMA: wave w moves pieces w * PW .. of [K: tile t, k-step | V^T: d, 32-key unit]; surplus pieces repeat the last one
@@ -309,6 +328,7 @@ __global__ __launch_bounds__(512, (KS <= 2 && DT <= 4) ? 4 : 2) void latent_pref
     int buf = 0;
     for (int kt = t0; kt < n_kt; kt++) {
         if (kt + 1 < n_kt) wait_vm<PW>(); else wait_vm<0>();      // my pieces of tile kt have landed
+        if (kt + 1 == n_kt && (end >> 6) == kt && (end & 63) != 63) tile_values_up_to<4 * KS, PIECES, PW>(lat_smc + buf * TILE, wave, lane, end & 63);
         __builtin_amdgcn_s_barrier();
         if (kt + 2 < n_kt) { int nb = buf + 2; if (nb >= NBUF) nb -= NBUF; issue(kt + 2, nb); }
         const char* kimg = lat_smc + buf * TILE + lane * 16;
@@ -398,10 +418,11 @@ __global__ __launch_bounds__(256) void latent_prefill_wide_kernel(LatentArgs p) 
 #pragma unroll
         for (int u = 0; u < 2; u++) {
             const bf16x8 pf = latent_pack_p(s[2 * u], s[2 * u + 1]);
+            const u32x4 keep = keys_up_to(j1 - j - 32 * u - 8 * fg);
             lacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pf, lacc, 0, 0, 0);
             const bf16_t* vr = (const bf16_t*)p.vx + (((int64_t)(h * DT) * v_ld + ((kb + j) >> 5) + u) * 64 + lane) * 8;
 #pragma unroll
-            for (int d = 0; d < DT; d++) o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(vr + (int64_t)d * v_ld * 512), pf, o[d], 0, 0, 0);
+            for (int d = 0; d < DT; d++) o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(keep_keys(*(const bf16x8*)(vr + (int64_t)d * v_ld * 512), keep), pf, o[d], 0, 0, 0);
         }
     }
     if (ok) latent_store_o<DT>(p, w.tok0 + r0, h, fg, 1.0f / lacc[0], o);
@@ -553,6 +574,10 @@ __global__ __launch_bounds__(256) void latent_decode_kernel(LatentArgs p) {
     for (int kt = kt0; kt < kt1; kt++) {
         char* img = lat_smc + ((kt - kt0) & 1) * IMG;
         f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (kt * 64 + 63 > pos && kt * 64 + 16 * wave + fq > pos) {      // (common.h keys_up_to)
+#pragma unroll
+            for (int ks = 0; ks < KSN; ks++) a[ks] = bf16x8{};
+        }
 #pragma unroll
         for (int ks = 0; ks < KSN; ks++) {
             s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ks], qf[ks], s, 0, 0, 0);
