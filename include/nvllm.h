@@ -579,8 +579,9 @@ int nvl_bench_gemm(int device, int M, int N, int K, int epi, int force_bnt, int 
  * key 29: milliseconds a tensor-parallel rank waits for its peers inside a P2P all-reduce before the call fails (default 30000).
  * key 30: Mamba2 prefill scan: 1 (default) the chunked SSD form on MFMA, chunks of a sequence in parallel when few (sequence, head)
  * pairs; 2 the chunked form, chunk after chunk only; 0 the sequential recurrence.
- * key 31: MoE decode routing (router logits, softmax, top-k, gate matrix): 1 (default) as one launch, or by the first workgroups of the
- * experts' up projection where streaming every expert costs little beside that launch; 2 always as one launch; 0 router GEMM + gate kernel.
+ * key 31: MoE decode routing (router logits, softmax, top-k, gate matrix): 1 (default) by the first workgroups of the experts' up projection
+ * where streaming every expert costs little beside them, in lists of layers otherwise by the launch of the norm that makes the experts' input
+ * (a norm behind the sublayer, rows of up to 4096), elsewhere as one launch; 2 always as one launch; 0 router GEMM + gate kernel (lists of layers: one launch).
  * key 35: non-temporal K/V loads in the decode attention: 1 (default) when one workgroup serves a kv head's group and the launch
  * fills the chip (>= 160 workgroups) or the batch is one sequence; 0 never; 2 always.
  * key 36: weight tiles per wave of the wide decode projections (FFN-up, LM head): 0 (default) 2 for 17..32 rows and N < 65536, else 4;

@@ -92,9 +92,10 @@ template <typename Rsrc> __device__ __forceinline__ f32x4 delta_rows_get(Rsrc rs
 }
 
 // ------------------------------------------------------------------------------------------
-// prep: grid (heads, workgroups that share its chunks), 8 waves.  Bound by what it moves, 145 KB a chunk of a head of 128 (q, k, v, z in, five operands out): 5.3 TB/s while
-// two workgroups a CU go from chunk to chunk.  They wait for little but stores because a chunk's loads leave when the one before has read its registers, and because
-// pairs are summed one by one inside blocks of 8 tokens only (of 16: 8500 of 46000 cycles a chunk, and two of eight waves had the products as well).
+// prep: grid (heads, workgroups that share its chunks), 8 waves.  Bound by the chain of a chunk, six barriers with little for most waves between some of them, of which two
+// workgroups a CU hide a part: no unit is full.  5 x 300 .. 1900 tokens x 16 heads of 128, 106 us: 147 KB a chunk (q, k, v, z in, five operands out) are 3.9 TB/s, 3.1 of them
+// HBM's (a copy reaches 5.0); vector ALUs 43 % of the time, LDS 32 (12 of it bank conflicts), matrix cores 20.  Loads are no part of the chain because a chunk's leave when the
+// one before has read its registers; pairs are summed one by one inside blocks of 8 tokens only (of 16: 8500 of 46000 cycles a chunk, and two of eight waves had the products as well).
 // us a layer, a workgroup per chunk and blocks of 16 -> here: 5 x 300 .. 1900 tokens x 16 heads 143 -> 109, 10 x 100 .. 900 134 -> 90, 16 x 900 370 -> 290.
 // ------------------------------------------------------------------------------------------
 template <int NK> constexpr int delta_prep_lds_bytes() { return 4 * (3 * DELTA_C * (NK * 16 + 4) + 2 * DELTA_C * 36 + DELTA_C + 512); }

@@ -1383,10 +1383,22 @@ static int g_attn_split = 1;   // nvl_set_tuning key 25: split a decode attentio
 //                                                  1200  958 / 945 (4 x 3), 976 (8 x 2)                                                                       12
 //                                                   900  947 / 956 (4 x 2)  1000  966 / 968 (4 x 2)  1900 1068 / 1048 (8 x 2)                                 16
 //   heads of 128, hybrid-2k, 4 kv heads (requests)  500  713 / 701 (2 x 4)   700  949 / 929 (2 x 6), 932 (4 x 3)  1000 1003 / 971 (2 x 8), 973 (4 x 4)         1
+//                 Llama-3-8B, 8 kv heads            400 3014 / 2948 (2 x 4)  700 3113 / 2957 (2 x 6), 2989 (4 x 3)  1000 3208 / 2966 (2 x 8), 3004 (4 x 4)      1
+//                                                   400 3028 / 2976 (2 x 4), 3012 (4 x 2)   600 3131 / 3012 (2 x 5), 3046 (4 x 3)   800 3250 / 3056 (2 x 7), 3087 (4 x 4)
+//                                                  1000 3300 / 3076 (2 x 8), 3098 (4 x 4)  1500 3495 / 3121 (4 x 6), 3106 (2 x 6)                              4
+//                                                   400 3124 / 3074 (2 x 4), 3099 (4 x 2)   600 3188 / 3108 (2 x 3), 3112 (4 x 3)   700 3221 / 3109 (2 x 3), 3126 (4 x 3)
+//                                                   800 3280 / 3132 (2 x 4), 3139 (4 x 4)   900 3301 / 3139 (2 x 4), 3145 (4 x 4)  1000 3326 / 3150 (2 x 4), 3163 (4 x 4)
+//                                                  1200 3391 / 3220 (4 x 3), 3194 (2 x 4)  1500 3525 / 3249 (4 x 3), 3238 (2 x 3)                              8
+//                 (two waves up to 16 tiles, and up to 24 they would not lose either; six sequences and ragged ones of 1000 / 4 and 900 / 3 alike)
 // Ragged contexts leave room for more parts, since a sequence takes them by its own length and the other workgroups of the grid leave at
-// once: more while those with work stay within 208 (heads of 64, whose parts are smaller: 300, and 280 beyond 85 pairs: 16 of 900 keys, 292 with work, +1.0), the whole grid within 640.  "/ 6": contexts down to a sixth of the longest; without -> with:
+// once: more while those with work stay within 208 (heads of 64, whose parts are smaller, 300, and 280 beyond 85 pairs: below), the whole grid within 640.  "/ 6": contexts down to a sixth of the longest; without -> with:
 //   heads of 64    Granite-3.0-1B 16 of 900 / 6  0.0 -> -1.2 (4 x 2), 12 of 1100 / 6 -0.3 -> -1.6 (4 x 3), Llama-3.2-1B 12 of 1100 / 6 -0.4 -> -1.1,
-//                  14 of 1200 and short ones 0.0 -> -1.3; of 900 / 2  at 227 with work +0.4, so not
+//                  14 of 1200 and short ones 0.0 -> -1.3
+//                  The line is shallow: on either side of it the forms are within a per cent.  Up to 64 pairs it decides between two waves of many parts and four of fewer (15 .. 20 tiles; the
+//                  first against the second at that many with work): 7 of 1000 / 8 of 1000 at 247 / 282 -1.7, -1.2; 6 of 1250, 7 of 1100, 8 of 1040 at 258, 269, 292 -0.5 .. -0.7; 8 of
+//                  1200 / 1.3 at 291 -0.5; 7 of 1180 at 291 +0.4 (Granite-3.0-1B +0.8); 8 of 1200 at 333 +0.9.  Beyond 85 pairs between 4 x 2 or 4 x 3 and whole (15 .. 20 tiles): 12 of
+//                  1200 / 2 and 16 of 1200 / 3 at 211, 247 -2.5, -2.8 against one part fewer; 14 of 1000 at 275 -1.7, 16 of 1000 / 1.7 at 259 -0.6; of 900 / 2 at 232 +0.3 (Granite -0.6,
+//                  GPT-2 -0.1), 15 of 920 at 279 +0.1 .. +0.5; 16 of 900 and of 1000 / 1.3 at 289, 281 +0.9, +0.4
 //   heads of 128   12 of 1500 / 6 -3.6 -> -5.7 (4 x 3), 16 of 1100 / 6 -1.0 -> -2.1 (4 x 3), 12 of 1500 and short ones -5 -> -7.6 (4 x 6); 16 of 1500 and
 //                  short ones -6.4 (4 x 3), -1.9 (4 x 6: a grid of 768); 12 of 900 / 6 in four parts (238 with work) +0.4, 16 of 1500 / 6 in three (251) +0.9
 // Whole sequences of ragged contexts: workgroups start in the grid's order, and a long one that starts in the second round of them runs on alone.
@@ -1672,7 +1684,7 @@ static int g_moe_bm = 0;       // nvl_set_tuning key 17: prefill MoE grouped GEM
 static int g_moe_gather = 1;   // nvl_set_tuning key 16: prefill MoE gathers the token rows into expert order before the grouped GEMM (0 = per-lane gather inside it)
 static int g_moe_defer_down = 1;    // nvl_set_tuning key 33: MoE decode: the last of the K slices' workgroups completes the residual and carries the next norm
                                     // (deferred RMSNorm producer, gemm.h split_finish_wave); 0: slices left to a norm launch
-static int g_moe_fused_route = 1;   // nvl_set_tuning key 31: MoE decode routing (router GEMM + softmax / top-k / gate matrix): 1 one launch, or none (moe_route_beside), 2 always one, 0 two
+static int g_moe_fused_route = 1;   // nvl_set_tuning key 31: MoE decode routing (router GEMM + softmax / top-k / gate matrix): 1 one launch, or none (moe_route_beside, layered.h routes_ahead), 2 always one, 0 two
 static int g_moe_small = 1;    // nvl_set_tuning key 8: fused MoE planning launch + combine folded into the next norm (0 = off)
 static int g_mamba_ssd = 1;    // nvl_set_tuning key 30: chunked (SSD) Mamba2 scan on MFMA for prefill-sized bf16 calls (0 = the sequential scan,
                                // 2 = chunk after chunk only, never the chunk-parallel three-launch form)
